@@ -2,7 +2,9 @@
 
 The library is the only implementation of the operators in this package: there is no
 CPU or PyTorch fallback.  If the shared object is missing or fails to load, importing
-an operator raises; build it with `python -m loongserve_amd.build`.
+an operator raises; build it with `python -m loongserve_amd.build`.  The operators a layer
+calls go through _native.so (csrc/binding.cpp), which fills the same argument blocks without
+the cost of ctypes; what it does not take (it checks, and launches nothing then) comes here.
 """
 from __future__ import annotations
 
@@ -180,6 +182,8 @@ def load():
     if lib.lsattn_version() != LSATTN_VERSION:
         raise ImportError("loongserve_amd: %s has interface version %d, this package is written against %d; rebuild it with "
                           "`python -m loongserve_amd.build`" % (LIB_PATH, lib.lsattn_version(), LSATTN_VERSION))
+    from . import _native  # the native argument pass of the operators calls the same loaded library
+    _native.bind({name: C.cast(getattr(lib, name), C.c_void_p).value for name in EXPORTS})
     _lib = lib
     return lib
 

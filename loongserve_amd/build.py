@@ -1,13 +1,15 @@
 """Build recipe for liblsattn.so (hand-written HIP kernels + C ABI, gfx950 only).
 
 `python -m loongserve_amd.build` compiles loongserve_amd/csrc/*.hip with hipcc into
-loongserve_amd/liblsattn.so.  hipcc cross-compiles without a GPU.
+loongserve_amd/liblsattn.so, and csrc/binding.cpp with g++ into loongserve_amd/_native.so.
+hipcc cross-compiles without a GPU.
 """
 from __future__ import annotations
 
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
@@ -15,6 +17,7 @@ ROOT = os.path.dirname(PKG_DIR)
 CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_PATH = os.path.join(PKG_DIR, "liblsattn.so")
 CEILING_LIB_PATH = os.path.join(PKG_DIR, "libls_ceiling.so")  # measurement aids of bench.py (include/ls_ceiling.h)
+NATIVE_PATH = os.path.join(PKG_DIR, "_native.so")  # the operators' argument pass (csrc/binding.cpp)
 SOURCES = ["prefill.hip", "prefill_small.hip", "decode.hip", "merge_scatter.hip", "elementwise.hip", "pool.hip"]
 # elementwise.hip reproduces the reference's half arithmetic operation by operation: no fused multiply-adds
 # other than the ones it writes
@@ -69,6 +72,24 @@ def build_ceiling(verbose: bool = False, out: str = CEILING_LIB_PATH) -> str:
     return out
 
 
+def build_native(verbose: bool = False, out: str = NATIVE_PATH) -> str:
+    """_native.so: the argument pass of the operators against PyTorch's C++ headers (host code only; it is handed the
+    library's entry points at load time and links neither the library nor a HIP runtime)."""
+    from importlib.util import find_spec
+    torch_dir = os.path.dirname(find_spec("torch").origin)
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
+           "-I" + os.path.join(ROOT, "include"), "-I" + os.path.join(torch_dir, "include"),
+           "-I" + os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"), "-I/opt/rocm/include",
+           "-I" + sysconfig.get_paths()["include"], os.path.join(CSRC, "binding.cpp"), "-o", out,
+           "-L" + os.path.join(torch_dir, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("g++ failed for binding.cpp:\n%s\n%s" % (" ".join(cmd), r.stderr[-6000:]))
+    if verbose:
+        print("built", out)
+    return out
+
+
 C_ABI_EXAMPLES = [os.path.join(ROOT, "tests", "c_abi", n) for n in ("decode_from_c", "prefill_from_c")]
 
 
@@ -88,5 +109,6 @@ def build_c_abi_example(verbose: bool = False):
 
 if __name__ == "__main__":
     build_all(verbose=True, extra_flags=sys.argv[1:])
+    build_native(verbose=True)
     build_ceiling(verbose=True)
     build_c_abi_example(verbose=True)

@@ -7,7 +7,7 @@ import functools
 
 import torch
 
-from . import longserve_cuda_kernels
+from . import _native, longserve_cuda_kernels
 
 
 # The stage functions called on their own (the master path, longserve_transformer_layer_infer.py:272-281 then :360-367)
@@ -82,12 +82,17 @@ def longserve_token_decode_attention_flash_decoding(q, req_to_token_indexs, b_re
                                                     mid_o_logexpsum, batch_size, max_len_in_batch, q_head_num,
                                                     head_dim, cache_k, cache_v, BLOCK_SEQ, out=None,
                                                     o_logexpsum=None):
+    split = _fused_block_seq(BLOCK_SEQ, batch_size, max_len_in_batch, cache_k.shape[1])
+    done = _native.token_decode_attention(q, req_to_token_indexs, b_req_idx, b_seq_len, mid_o, mid_o_logexpsum, batch_size,
+                                          max_len_in_batch, q_head_num, head_dim, cache_k, cache_v, split, out, o_logexpsum,
+                                          longserve_cuda_kernels.FUSED_PARTIALS_BY_REQUEST)
+    if done is not None:
+        return done
     calcu_shape1 = (-1, q_head_num, head_dim)
     # outputs are float32 whatever q is, so that they can be merged again (FDPY:9-10)
     o_tensor = torch.empty_like(q, dtype=torch.float32) if out is None else out
     out_logexpsum = (torch.empty([batch_size, q_head_num], dtype=torch.float32, device=q.device)
                      if o_logexpsum is None else o_logexpsum)
-    split = _fused_block_seq(BLOCK_SEQ, batch_size, max_len_in_batch, cache_k.shape[1])
     longserve_cuda_kernels.flash_decoding(mid_o, mid_o_logexpsum, q.view(calcu_shape1), cache_k, cache_v, req_to_token_indexs,
                                           b_req_idx, b_seq_len, max_len_in_batch, o_tensor.view(calcu_shape1), out_logexpsum,
                                           split)

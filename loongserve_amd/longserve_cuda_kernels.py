@@ -15,7 +15,7 @@ import math
 
 import torch
 
-from . import _lib
+from . import _lib, _native
 from .ops import _DT, _stream
 
 
@@ -77,11 +77,13 @@ def _stage1_args(mid_o, mid_o_logexpsum, q, k, v, req_to_tokens, b_req_idx, b_se
     return a
 
 
-@torch.inference_mode()
 def flash_decoding_stage1(mid_o, mid_o_logexpsum, q, k, v, req_to_tokens, b_req_idx, b_seqlen,
                           max_len_in_batch: int, seq_block_size: int, merge_blocks: int = 1) -> None:
     """ENTRY:103-164, same argument order.  merge_blocks > 1 (not in the reference): one partial per that many consecutive
     blocks, in the row of the first; the rows of the others are marked empty (LSE = -inf)."""
+    if _native.decode_stage1(mid_o, mid_o_logexpsum, q, k, v, req_to_tokens, b_req_idx, b_seqlen, max_len_in_batch, seq_block_size,
+                             merge_blocks):
+        return
     a = _stage1_args(mid_o, mid_o_logexpsum, q, k, v, req_to_tokens, b_req_idx, b_seqlen, max_len_in_batch, seq_block_size,
                      merge_blocks)
     _lib.check(_lib.load().lsattn_decode_stage1(C.byref(a), _stream()), "lsattn_decode_stage1")
@@ -117,23 +119,12 @@ def _stage2_args(o, out_logexpsum, b_seqlen, mid_o, mid_o_logexpsum, block_seq: 
     return a
 
 
-@torch.inference_mode()
 def flash_decoding_stage2(o, out_logexpsum, b_seqlen, mid_o, mid_o_logexpsum, block_seq: int) -> None:
     """ENTRY:166-221, same argument order."""
+    if _native.decode_stage2(o, out_logexpsum, b_seqlen, mid_o, mid_o_logexpsum, block_seq):
+        return
     a = _stage2_args(o, out_logexpsum, b_seqlen, mid_o, mid_o_logexpsum, block_seq)
     _lib.check(_lib.load().lsattn_decode_stage2(C.byref(a), _stream()), "lsattn_decode_stage2")
-
-
-# Argument blocks of the fused call, by the full metadata of its tensors.  A decode step of a serving loop calls with the
-# same buffers every time (the request table, the length vector and the KV pool are updated in place), and the checks and
-# the filling of the two blocks then cost more host time than a small batch's kernels run: a call whose tensors all have
-# the address, shape, strides and dtype of an earlier, validated call reuses that call's blocks.
-_FUSED_CACHE: dict = {}
-_FUSED_CACHE_MAX = 64
-
-
-def _meta(t):
-    return (t.data_ptr(), t.shape, t.stride(), t.dtype, t.device.index)
 
 
 # The fused call keeps the partials of a request side by side in mid_o ([batch, blocks, heads, head_dim] in the same
@@ -146,19 +137,14 @@ def flash_decoding(mid_o, mid_o_logexpsum, q, k, v, req_to_tokens, b_req_idx, b_
                    o, out_logexpsum, block_seq: int) -> None:
     """Stage 1 and stage 2 with the same block size from one library call (what FDPY:12-27 does with two): the checks of
     both, one argument pass, the two launches back to back."""
-    key = (_meta(mid_o), _meta(mid_o_logexpsum), _meta(q), _meta(k), _meta(v), _meta(req_to_tokens), _meta(b_req_idx),
-           _meta(b_seqlen), _meta(o), _meta(out_logexpsum), max_len_in_batch, block_seq, FUSED_PARTIALS_BY_REQUEST)
-    blocks = _FUSED_CACHE.get(key)
-    if blocks is None:
-        a1 = _stage1_args(mid_o, mid_o_logexpsum, q, k, v, req_to_tokens, b_req_idx, b_seqlen, max_len_in_batch, block_seq)
-        a2 = _stage2_args(o, out_logexpsum, b_seqlen, mid_o, mid_o_logexpsum, block_seq)
-        a1.partials_by_request = a2.partials_by_request = 1 if FUSED_PARTIALS_BY_REQUEST else 0
-        if len(_FUSED_CACHE) >= _FUSED_CACHE_MAX:
-            del _FUSED_CACHE[next(iter(_FUSED_CACHE))]  # the oldest entry (a caller that allocates new outputs every call never hits)
-        blocks = _FUSED_CACHE[key] = (a1, a2, C.byref(a1), C.byref(a2), _lib.load().lsattn_decode_attention)
-    rc = blocks[4](blocks[2], blocks[3], _stream())
-    if rc:
-        _lib.check(rc, "lsattn_decode_attention")
+    if mid_o.dim() == 4 and q.dim() == 3 and o.shape == q.shape and _native.token_decode_attention(
+            q, req_to_tokens, b_req_idx, b_seqlen, mid_o, mid_o_logexpsum, q.shape[0], max_len_in_batch, q.shape[1], q.shape[2], k, v,
+            block_seq, o, out_logexpsum, FUSED_PARTIALS_BY_REQUEST):
+        return
+    a1 = _stage1_args(mid_o, mid_o_logexpsum, q, k, v, req_to_tokens, b_req_idx, b_seqlen, max_len_in_batch, block_seq)
+    a2 = _stage2_args(o, out_logexpsum, b_seqlen, mid_o, mid_o_logexpsum, block_seq)
+    a1.partials_by_request = a2.partials_by_request = 1 if FUSED_PARTIALS_BY_REQUEST else 0
+    _lib.check(_lib.load().lsattn_decode_attention(C.byref(a1), C.byref(a2), _stream()), "lsattn_decode_attention")
 
 
 @torch.inference_mode()
@@ -186,9 +172,11 @@ def _half2d(t: torch.Tensor, name: str, dim: int) -> None:
         raise ValueError("%s must be a contiguous %d-d float16 CUDA tensor" % (name, dim))
 
 
-@torch.inference_mode()
 def rms_norm(input: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     """Argument order, checks and result of ENTRY:15-39 (a new [num_tokens, hidden] fp16 tensor)."""
+    done = _native.rms_norm(input, weight, eps)
+    if done is not None:
+        return done
     _half2d(input, "input", 2); _half2d(weight, "weight", 1)
     if input.size(1) != weight.size(0):
         raise ValueError("input.size(1) must equal weight.size(0)")
@@ -198,9 +186,10 @@ def rms_norm(input: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Ten
     return out
 
 
-@torch.inference_mode()
 def silu_and_mul_inplace(io: torch.Tensor) -> None:
     """ENTRY:41-52: io is [num_tokens, 2 * inter]; the first half of every row becomes silu(gate) * up."""
+    if _native.silu_and_mul_inplace(io):
+        return
     _half2d(io, "io", 2)
     if io.size(1) % 2:
         raise ValueError("io.size(1) must be even")
@@ -219,9 +208,10 @@ def _rotary_single(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> Non
                                              _stream()), "lsattn_rotary_emb")
 
 
-@torch.inference_mode()
 def rotary_emb(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> None:
     """ENTRY:54-89: in-place rotary embedding of q and of k (strided views are fine)."""
+    if _native.rotary_emb(q, k, cos, sin):
+        return
     _rotary_single(q, cos, sin)
     _rotary_single(k, cos, sin)
 

@@ -13,12 +13,13 @@ Reference call sites (relative to the reference tree):
 from __future__ import annotations
 
 import ctypes as C
+import functools
 import math
 from typing import List, Optional, Sequence, Tuple
 
 import torch
 
-from . import _lib
+from . import _lib, _native
 from ._lib import LSATTN_BF16, LSATTN_F16, LSATTN_F32
 
 _DT = {torch.float16: LSATTN_F16, torch.bfloat16: LSATTN_BF16, torch.float32: LSATTN_F32}
@@ -208,13 +209,19 @@ def kv_split_count(batch: int, num_q_heads: int, max_q_len: int, kv_rows: int, n
     keys (kv_rows bounds every sequence's chunk: max_kv_len where the caller gives it, else the rows of the k buffer; the
     lengths themselves live on the device).  The launch's size without cuts is counted in 128-row workgroups as the
     kernel forms them: up to four query heads of a KV head side by side (num_kv_heads given), 128 / that many positions each."""
+    return _kv_split_count(int(batch), int(num_q_heads), int(max_q_len), int(kv_rows), num_kv_heads, KV_SPLIT_BELOW_WORKGROUPS,
+                           KV_SPLIT_ROUND, KV_SPLIT_MIN_KEYS)
+
+
+@functools.lru_cache(maxsize=4096)
+def _kv_split_count(batch, num_q_heads, max_q_len, kv_rows, num_kv_heads, below, in_a_round, min_keys):
     pack = 1
     if num_kv_heads:
         group = num_q_heads // num_kv_heads
         while pack < 4 and group % (2 * pack) == 0:
             pack *= 2
     wgs = batch * (num_q_heads // pack) * ((max_q_len + 128 // pack - 1) // (128 // pack))
-    if wgs <= 0 or wgs >= KV_SPLIT_BELOW_WORKGROUPS or kv_rows < KV_SPLIT_MIN_KEYS:
+    if wgs <= 0 or wgs >= below or kv_rows < min_keys:
         return 1
     # rounds(S) / S of the uncut chain is what a CU walks with S cuts.  (measured, GQA 32/8 unless said: 16 rows x 131072 keys
     # 32 cuts 124 us against 134 with 16 and 160 with 64; 100 x 131072 8 cuts 252, 10 cuts 285, 16 cuts 243, 32 cuts 270, MHA 8 cuts 388
@@ -222,7 +229,7 @@ def kv_split_count(batch: int, num_q_heads: int, max_q_len: int, kv_rows: int, n
     best, best_cost = 1, None
     for S in range(1, max(1, min(_lib.LSATTN_MAX_KV_CUTS, kv_rows // 4096)) + 1):
         # (and every cut adds a part to write and to merge: about a thousandth of the uncut chain each in the cases above)
-        cost = (-(-wgs * S // KV_SPLIT_ROUND)) / S + 0.001 * S
+        cost = (-(-wgs * S // in_a_round)) / S + 0.001 * S
         if best_cost is None or cost < best_cost - 1e-9:
             best, best_cost = S, cost
     return best
@@ -233,7 +240,6 @@ def _cut_len(kv_rows: int, S: int) -> int:
     return -(-(-(-kv_rows // S)) // 64) * 64
 
 
-@torch.inference_mode()
 def context_attention_fwd(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first_token_global_idx,
                           kv_b_start_loc, kv_b_seq_len, kv_first_token_global_idx,
                           logical_sp_peers_num: int, max_q_b_seq_len: int, m, l, *, v_f16: Optional[torch.Tensor] = None,
@@ -264,6 +270,26 @@ def context_attention_fwd(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first_token_
     Start from m = -inf, l = 0 (o need not be zeroed).  After k calls o is the
     normalised attention output over all keys seen and ln2*(m + log2 l) their LSE.
     """
+    if v_f16 is None and not v_f16_valid:
+        cuts = kv_rows = 1
+        if workspace is not None and q.shape[-1] == KERNEL_HEAD_DIM:
+            kv_rows = k.shape[0] if max_kv_len is None else max_kv_len
+            cuts = kv_splits if kv_splits is not None else kv_split_count(q_b_seq_len.shape[0], q.shape[1], max_q_b_seq_len, kv_rows,
+                                                                          k.shape[1])
+        if _native.context_attention(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first_token_global_idx, kv_b_start_loc,
+                                     kv_b_seq_len, kv_first_token_global_idx, logical_sp_peers_num, max_q_b_seq_len, m, l,
+                                     0 if total_q_len is None else total_q_len, cuts, kv_rows, workspace, PRECONVERT_BF16_V):
+            return
+    _context_attention_checked(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first_token_global_idx, kv_b_start_loc, kv_b_seq_len,
+                               kv_first_token_global_idx, logical_sp_peers_num, max_q_b_seq_len, m, l, v_f16, v_f16_valid,
+                               workspace, max_kv_len, kv_splits, total_q_len)
+
+
+@torch.inference_mode()
+def _context_attention_checked(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first_token_global_idx, kv_b_start_loc, kv_b_seq_len,
+                               kv_first_token_global_idx, logical_sp_peers_num, max_q_b_seq_len, m, l, v_f16, v_f16_valid,
+                               workspace, max_kv_len, kv_splits, total_q_len) -> None:
+    """context_attention_fwd for arguments the native pass does not take: converts them or raises."""
     if o.dtype != q.dtype:
         raise ValueError("o must have the dtype of q")
     D = q.shape[-1]
@@ -298,7 +324,6 @@ def context_attention_fwd(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first_token_
     _lib.check(_lib.load().lsattn_prefill_step_merge(C.byref(a), _stream()), "lsattn_prefill_step_merge")
 
 
-@torch.inference_mode()
 def prefill_attention_step(q, k, v, q_b_start_loc, q_b_seq_len, q_first_token_global_idx,
                            kv_b_start_loc, kv_b_seq_len, kv_first_token_global_idx,
                            logical_sp_peers_num: int, max_q_b_seq_len: int,
@@ -322,6 +347,29 @@ def prefill_attention_step(q, k, v, q_b_start_loc, q_b_seq_len, q_first_token_gl
     other keys; lse = -inf marks an empty row) in the kernel's epilogue, instead of being written from the empty state;
     rows that see no key in this step keep what they hold.
     """
+    if v_f16 is None and not v_f16_valid:
+        kv_rows = k.shape[0] if max_kv_len is None else max_kv_len
+        cuts = 1
+        if q.shape[-1] == KERNEL_HEAD_DIM:
+            cuts = kv_splits if kv_splits is not None else kv_split_count(q_b_seq_len.shape[0], q.shape[1], max_q_b_seq_len, kv_rows,
+                                                                          k.shape[1])
+        done = _native.prefill_partial(q, k, v, q_b_start_loc, q_b_seq_len, q_first_token_global_idx, kv_b_start_loc, kv_b_seq_len,
+                                       kv_first_token_global_idx, logical_sp_peers_num, max_q_b_seq_len, out, lse, sm_scale,
+                                       accumulate, 0 if total_q_len is None else total_q_len, cuts, kv_rows, kv_split_workspace,
+                                       PRECONVERT_BF16_V)
+        if done is not None:
+            return done
+    return _prefill_attention_step_checked(q, k, v, q_b_start_loc, q_b_seq_len, q_first_token_global_idx, kv_b_start_loc,
+                                           kv_b_seq_len, kv_first_token_global_idx, logical_sp_peers_num, max_q_b_seq_len, out,
+                                           lse, sm_scale, accumulate, v_f16, v_f16_valid, kv_splits, kv_split_workspace,
+                                           max_kv_len, total_q_len)
+
+
+@torch.inference_mode()
+def _prefill_attention_step_checked(q, k, v, q_b_start_loc, q_b_seq_len, q_first_token_global_idx, kv_b_start_loc, kv_b_seq_len,
+                                    kv_first_token_global_idx, logical_sp_peers_num, max_q_b_seq_len, out, lse, sm_scale,
+                                    accumulate, v_f16, v_f16_valid, kv_splits, kv_split_workspace, max_kv_len, total_q_len):
+    """prefill_attention_step for arguments the native pass does not take: converts them or raises."""
     if accumulate and (out is None or lse is None):
         raise ValueError("accumulate=True needs the running out and lse")
     D = q.shape[-1]
@@ -389,13 +437,14 @@ def lse_merge(parts: Sequence[Tuple[torch.Tensor, torch.Tensor]], out: Optional[
     return out, lse
 
 
-@torch.inference_mode()
 def kv_scatter(src: torch.Tensor, dest_index: torch.Tensor, pool: torch.Tensor) -> None:
     """pool[dest_index[i]] = src[i] (bit-exact row scatter into the token-indexed pool).
 
     Semantics of destindex_copy_kv
     (loongserve/common/basemodel/triton_kernel/destindex_copy_kv.py:31-51).
     """
+    if _native.kv_scatter(src, dest_index, pool):
+        return
     _dev(src, "src"); _dev(pool, "pool")
     dest_index = _slots(dest_index, "dest_index", src.shape[0])
     if src.dtype != pool.dtype or src.shape[1:] != pool.shape[1:]:
@@ -445,7 +494,6 @@ def destindex_copy_kv(K: torch.Tensor, DestLoc: torch.Tensor, Out: torch.Tensor)
     kv_scatter(K, DestLoc, Out)
 
 
-@torch.inference_mode()
 def rotary_emb_write_kv(q: torch.Tensor, cache_kv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
                         mem_index: Optional[torch.Tensor] = None, pool: Optional[torch.Tensor] = None,
                         req_to_token_indexs: Optional[torch.Tensor] = None, b_req_idx: Optional[torch.Tensor] = None,
@@ -459,6 +507,18 @@ def rotary_emb_write_kv(q: torch.Tensor, cache_kv: torch.Tensor, cos: torch.Tens
       copy_kv_index_to_req(req_to_token_indexs, b_req_idx, b_seq_len, mem_index)       (decode=True), if the table is given.
     q [T, Hq, D], cache_kv [T, 2*Hkv, D] (K heads then V heads), float16; the results are those of the separate
     operators bit for bit."""
+    if mem_index is not None and (req_to_token_indexs is None or decode or (b_start_loc is not None and max_len_in_batch is not None)):
+        if _native.rotary_kv_write(q, cache_kv, cos, sin, mem_index, pool, req_to_token_indexs, b_req_idx, b_seq_len, b_start_loc,
+                                   max_len_in_batch, decode):
+            return
+    _rotary_emb_write_kv_checked(q, cache_kv, cos, sin, mem_index, pool, req_to_token_indexs, b_req_idx, b_seq_len, b_start_loc,
+                                 max_len_in_batch, decode)
+
+
+@torch.inference_mode()
+def _rotary_emb_write_kv_checked(q, cache_kv, cos, sin, mem_index, pool, req_to_token_indexs, b_req_idx, b_seq_len, b_start_loc,
+                                 max_len_in_batch, decode) -> None:
+    """rotary_emb_write_kv for arguments the native pass does not take: converts them or raises."""
     for t, n in ((q, "q"), (cache_kv, "cache_kv")):
         _dev(t, n)
         if t.dim() != 3 or t.dtype != torch.float16 or t.stride(2) != 1:
@@ -511,12 +571,13 @@ def rotary_emb_write_kv(q: torch.Tensor, cache_kv: torch.Tensor, cos: torch.Tens
     _lib.check(_lib.load().lsattn_rotary_kv_write(C.byref(a), _stream()), "lsattn_rotary_kv_write")
 
 
-@torch.inference_mode()
 def copy_kv_index_to_req(req_to_token_indexs: torch.Tensor, b_req_idx: torch.Tensor, b_seq_len: torch.Tensor,
                          memindex: torch.Tensor) -> None:
     """req_to_token_indexs[b_req_idx[i], b_seq_len[i] - 1] = memindex[i]: registers the slot of each request's new token
     in the decoding stage (loongserve/common/basemodel/triton_kernel/copy_kv_index_to_req.py:22-40, called
     loongserve/models/llama/longserve_model.py:491, :497).  memindex is int32 or, as the allocator returns it, int64."""
+    if _native.register_decode_tokens(req_to_token_indexs, b_req_idx, b_seq_len, memindex):
+        return
     _dev(req_to_token_indexs, "req_to_token_indexs"); _dev(memindex, "memindex")
     B = b_seq_len.shape[0]
     assert b_seq_len.shape[0] == memindex.shape[0] and b_req_idx.shape[0] == b_seq_len.shape[0]  # as the reference
@@ -538,6 +599,9 @@ def init_req_to_token_indexes(req_to_token_indexs, b_req_idx, b_seq_len, alloc_m
 
     Signature of loongserve/common/infer_utils.py:1 plus two optional arguments that avoid
     a host round trip (packed start offsets and the longest length)."""
+    if b_start_loc is not None and max_len_in_batch is not None and _native.register_tokens(
+            req_to_token_indexs, b_req_idx, b_seq_len, alloc_mem_index, b_start_loc, max_len_in_batch):
+        return
     _dev(req_to_token_indexs, "req_to_token_indexs")
     if req_to_token_indexs.dtype != torch.int32 or not req_to_token_indexs.is_contiguous():
         raise ValueError("req_to_token_indexs must be contiguous int32")
