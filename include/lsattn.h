@@ -253,10 +253,9 @@ int lsattn_decode_stage2(const lsattn_decode_stage2_args* a, void* stream);
  * the same mid_o, mid_o_logexpsum, b_seqlen, batch, heads, block count, head_dim, block size and layout of the partials (else
  * LSATTN_ERR_INVALID_ARG); everything else as in the two calls it stands for.
  * mid_o and mid_o_logexpsum are scratch to this call, as they are to the reference's function (FDPY:12-27 hands neither
- * out): the call may cut the contexts otherwise than seq_block_size says.  Launches of eight and more requests with
- * enough tokens deal the blocks of all requests (256 tokens each, or the smallest multiple of that by a power of two
- * whose rows the buffers hold) in equal shares to the waves, whatever the lengths of the requests are, and leave one
- * partial per share and request; (o, out_logexpsum) are the same softmax merged from other pieces.
+ * out): the call may cut the contexts otherwise than seq_block_size says.  Launches of several requests with enough tokens
+ * deal the tokens of all requests (in units of 32) in equal shares to the waves, whatever the lengths of the requests are,
+ * and leave one partial per share and request; (o, out_logexpsum) are the same softmax merged from other pieces.
  */
 int lsattn_decode_attention(const lsattn_decode_stage1_args* s1, const lsattn_decode_stage2_args* s2, void* stream);
 
@@ -270,7 +269,7 @@ int lsattn_decode_attention(const lsattn_decode_stage1_args* s1, const lsattn_de
  * exceed LSATTN_STATIC_SCRATCH_BYTES (else LSATTN_ERR_WORKSPACE); merge_blocks must be 0 or 1.  Results are those of
  * lsattn_decode_attention: the same kernels; bit for bit whenever both calls cut the contexts alike, which they do
  * unless the launch is dealt in equal shares and the array holds fewer rows for the batch than the caller's buffers would
- * (then the shares are counted in larger blocks and the sums are added in another order).  The call allocates and frees nothing.  Each GPU has one such array (held until
+ * (then there are fewer shares and the sums are added in another order).  The call allocates and frees nothing.  Each GPU has one such array (held until
  * the process ends) and every call on that GPU uses it: calls that overlap on one GPU (two streams, two threads) race;
  * calls in stream order on one stream do not.  Nothing needs clearing between calls: stage 2 reads only rows that
  * stage 1 of the same call has written.  The first call on a device looks the array's address up

@@ -37,6 +37,7 @@ struct Stage1Params {
   int32_t blocks_per_wg;  // consecutive blocks walked by one workgroup
   int32_t tasks;          // hkv * (group / GT) wave tasks
   int32_t tasks_on_x;     // grid = (task groups, chunks, batch) instead of (chunks, task groups, batch)
+  int32_t max_shares, share_units;  // equal shares: at most so many, of at least so many units each
 };
 
 constexpr int kTok = 8;  // K/V rows in flight per 16-lane group
@@ -418,9 +419,10 @@ constexpr int kMfmaStage = kMfmaBatch * (kMfmaKRow + kMfmaVRow);  // LDS bytes p
 // fourth batch of its tokens and merge their partials through LDS: four times the waves of the plain shape, each short.
 // One unit of work of a workgroup: request b, task group bid_t, chunk group bid_c (of n_cgroups in the grid; LISTED: the
 // unit comes from a list of the units that exist, and its chunk group is taken as it is).
-// RANGE: the wave's unit is blocks [r_lo, r_hi) of the request instead (r_lo < r_hi <= the request's blocks), computed into
-// one partial, which goes to row r_lo; the rows of the other blocks are left alone (the merge behind it knows which rows
-// hold a partial).
+// RANGE: the wave walks a share of the line of all requests' tokens instead (ShareWalk): batch after batch without a break
+// where one request ends and the next begins (the loads run ahead of the arithmetic across that point: they need only the
+// slot numbers, which come from the table row of whatever request the share has reached), one partial per request it
+// touches, number v + request of the launch (mid_o as [partial, Hq, 128]; the merge behind it knows whose partial that is).
 // The lane's eight 16-byte pieces of a partial's row, 64 bytes apart, each scaled by `inv`.  The stores carry the
 // system-scope bits: such a store goes through to memory as it is issued instead of waiting in the L2 as a dirty line
 // that is written back later, alone, between the reads of a gather that keeps every memory channel busy.  Measured on
@@ -440,10 +442,61 @@ __device__ __forceinline__ void store_partial_row(float* dst, const f32x4 (&acc)
 #undef LSATTN_STORE_ROW_PIECE
 }
 
+__device__ __forceinline__ uint32_t share_units_of(const int len, const int64_t block_seq, const int64_t grid_blocks) {
+  const uint32_t n = len <= 0 ? 0u : ((uint32_t)len + (uint32_t)block_seq - 1u) / (uint32_t)block_seq;
+  return n > (uint32_t)grid_blocks ? (uint32_t)grid_blocks : n;
+}
+// A share of the line of units (kMfmaBatch tokens of a request each): units [x, end) of it, x in request r.
+struct ShareWalk {
+  uint32_t v, x, end;
+  int r;
+  // units of requests 0 .. r, length and table row of request r: lane r's (up to 64 requests) or in LDS and memory
+  bool in_registers;
+  uint32_t incl;
+  int len, req;
+  const uint32_t* first_unit;
+};
+// One request's part of the share: tokens [t, t_end) of request r.
+struct ShareSegment {
+  int r, t, t_end;
+  uint32_t x_end;  // where on the line it ends
+  int req;
+};
+__device__ __forceinline__ ShareSegment share_segment(const Stage1Params& p, const ShareWalk& w, int r, uint32_t x) {
+  uint32_t r0, r1;
+  int len;
+  ShareSegment s;
+  for (;; r++) {  // (requests without units are skipped; x is below the line's end, so one is found)
+    if (w.in_registers) {
+      r1 = __builtin_amdgcn_readlane(w.incl, r);
+      if (r1 > x) {
+        r0 = r > 0 ? __builtin_amdgcn_readlane(w.incl, r - 1) : 0u;
+        len = __builtin_amdgcn_readlane(w.len, r);
+        s.req = __builtin_amdgcn_readlane(w.req, r);
+        break;
+      }
+    } else {
+      r1 = __builtin_amdgcn_readfirstlane(w.first_unit[r + 1]);
+      if (r1 > x) {
+        r0 = __builtin_amdgcn_readfirstlane(w.first_unit[r]);
+        len = p.b_seqlen[r];
+        s.req = p.b_req_idx[r];
+        break;
+      }
+    }
+  }
+  s.r = r;
+  s.x_end = r1 < w.end ? r1 : w.end;
+  s.t = (int)(x - r0) * kMfmaBatch;
+  s.t_end = (int)(s.x_end - r0) * kMfmaBatch;
+  if (s.t_end > len) s.t_end = len;
+  return s;
+}
+
 template <typename T, bool WS, bool LISTED, bool RANGE = false>
 __device__ __forceinline__ void stage1_mfma_unit(const Stage1Params& p, char* lds, const int lane, const int wave, const int64_t b,
                                                  const unsigned bid_t, const unsigned bid_c, const unsigned n_cgroups,
-                                                 const int64_t r_lo = 0, const int64_t r_hi = 0) {
+                                                 const ShareWalk& walk = ShareWalk{}) {
   const int n = lane & 15, g = lane >> 4;  // query head (column) or 16-byte chunk of a row / token group or row of four
   // The waves of a workgroup: tw of them on neighbouring tasks (KV heads: their rows of a token lie side by side in memory
   // and are then fetched at about the same time), the rest on consecutive chunks of tokens.
@@ -457,38 +510,51 @@ __device__ __forceinline__ void stage1_mfma_unit(const Stage1Params& p, char* ld
   const int qh0 = kvh * group + sg * 16;
   const int nh = group - sg * 16 < 16 ? group - sg * 16 : 16;
 
-  const int len = p.b_seqlen[b];
-  int64_t nblk = len <= 0 ? 0 : ((int64_t)len + p.block_seq - 1) / p.block_seq;
-  if (nblk > p.grid_blocks) nblk = p.grid_blocks;
-  if (nblk > (p.num_blocks + p.row_mul - 1) / p.row_mul) nblk = (p.num_blocks + p.row_mul - 1) / p.row_mul;
-  int64_t fine_nblk = len <= 0 ? 0 : ((int64_t)len + p.fine_block_seq - 1) / p.fine_block_seq;
-  if (fine_nblk > p.num_blocks) fine_nblk = p.num_blocks;
-  const unsigned n_chunks = n_cgroups * cw;
-  const unsigned wave_chunk = bid_c * cw + (WS ? 0 : wave >> (tw == 4 ? 2 : tw == 2 ? 1 : 0));
-  const unsigned chunk = LISTED ? wave_chunk : (wave_chunk + (unsigned)b) % n_chunks;  // (rotated by the request, as above)
-  const int64_t blk_begin = RANGE ? r_lo : (int64_t)chunk * p.blocks_per_wg;  // (WS: one block per workgroup)
-  int64_t blk_end = RANGE ? r_hi : blk_begin + p.blocks_per_wg;
-  if (blk_end > nblk) blk_end = nblk;
-  if (blk_begin >= blk_end) return;  // (WS: the same for the four waves, which meet at a barrier below)
-  const int bs = (int)p.block_seq;                    // a multiple of 32 (checked on the host)
   constexpr int kStep = WS ? kMfmaWaves * kMfmaBatch : kMfmaBatch;  // tokens from one of the wave's batches to its next
-  const int t_begin = (int)(blk_begin * bs) + (WS ? wave * kMfmaBatch : 0);
-  const int t_end = blk_end * bs > len ? len : (int)(blk_end * bs);
-  const int t_last = t_end - 1;
-  const int n_batches = t_begin < t_end ? (t_end - t_begin + kStep - 1) / kStep : 0;
+  const int bs = (int)p.block_seq;                    // a multiple of 32 (checked on the host)
+  int64_t fine_nblk = 0, blk_begin = 0;
+  int t_begin, t_end, n_batches;
+  const int32_t* table;
+  ShareSegment sl_seg, co_seg;  // (RANGE) where the slot numbers requested next and the batch computed next stand
+  if constexpr (RANGE) {
+    sl_seg = co_seg = share_segment(p, walk, walk.r, walk.x);
+    t_begin = co_seg.t;
+    t_end = co_seg.t_end;
+    n_batches = (int)(walk.end - walk.x);
+    table = p.req_to_tokens + (int64_t)co_seg.req * p.max_seq_len;
+  } else {
+    const int len = p.b_seqlen[b];
+    int64_t nblk = len <= 0 ? 0 : ((int64_t)len + p.block_seq - 1) / p.block_seq;
+    if (nblk > p.grid_blocks) nblk = p.grid_blocks;
+    if (nblk > (p.num_blocks + p.row_mul - 1) / p.row_mul) nblk = (p.num_blocks + p.row_mul - 1) / p.row_mul;
+    fine_nblk = len <= 0 ? 0 : ((int64_t)len + p.fine_block_seq - 1) / p.fine_block_seq;
+    if (fine_nblk > p.num_blocks) fine_nblk = p.num_blocks;
+    const unsigned n_chunks = n_cgroups * cw;
+    const unsigned wave_chunk = bid_c * cw + (WS ? 0 : wave >> (tw == 4 ? 2 : tw == 2 ? 1 : 0));
+    const unsigned chunk = LISTED ? wave_chunk : (wave_chunk + (unsigned)b) % n_chunks;  // (rotated by the request, as above)
+    blk_begin = (int64_t)chunk * p.blocks_per_wg;  // (WS: one block per workgroup)
+    int64_t blk_end = blk_begin + p.blocks_per_wg;
+    if (blk_end > nblk) blk_end = nblk;
+    if (blk_begin >= blk_end) return;  // (WS: the same for the four waves, which meet at a barrier below)
+    t_begin = (int)(blk_begin * bs) + (WS ? wave * kMfmaBatch : 0);
+    t_end = blk_end * bs > len ? len : (int)(blk_end * bs);
+    n_batches = t_begin < t_end ? (t_end - t_begin + kStep - 1) / kStep : 0;
+    table = p.req_to_tokens + (int64_t)p.b_req_idx[b] * p.max_seq_len;
+  }
+  int t_last = t_end - 1;
 
-  const int32_t* table = p.req_to_tokens + (int64_t)p.b_req_idx[b] * p.max_seq_len;
   const char* kbase = (const char*)p.k + ((int64_t)kvh * p.k_s1) * 2 + n * 16;
   const char* vbase = (const char*)p.v + ((int64_t)kvh * p.v_s1) * 2 + n * 16;
   const int64_t k_row_bytes = p.k_s0 * 2, v_row_bytes = p.v_s0 * 2;
 
   // Q^T as B operands: qb[ks] = Q[head n][32 ks + 8 g .. + 7] (zero for the spare columns)
   u32x4 qb[4];
-  {
-    const char* qrow = (const char*)p.q + ((b * p.hq + qh0 + (n < nh ? n : 0)) * 128 + 8 * g) * 2;
+  auto load_q = [&](const int64_t req) __attribute__((always_inline)) {
+    const char* qrow = (const char*)p.q + ((req * p.hq + qh0 + (n < nh ? n : 0)) * 128 + 8 * g) * 2;
 #pragma unroll
     for (int ks = 0; ks < 4; ks++) qb[ks] = n < nh ? *(const u32x4*)(qrow + ks * 64) : u32x4{0, 0, 0, 0};
-  }
+  };
+  load_q(RANGE ? co_seg.r : b);
   char* lds_k = lds + wave * kMfmaStage;
   char* lds_v = lds_k + kMfmaBatch * kMfmaKRow;
   // the lane writes chunk n of row 4 i + g (one register + 4 i rows as immediate), reads K row n (and 16 + n), chunk
@@ -560,7 +626,7 @@ __device__ __forceinline__ void stage1_mfma_unit(const Stage1Params& p, char* ld
     lt += xlane32(lt);
     if (n < nh) {
       const float inv = 1.f / lt;  // a block holds at least one token
-      const int64_t row = blk * p.row_mul * p.blk_rows + b * p.req_rows + qh0 + n;
+      const int64_t row = RANGE ? ((int64_t)walk.v + co_seg.r) * p.hq + qh0 + n : blk * p.row_mul * p.blk_rows + b * p.req_rows + qh0 + n;
       float* dst = p.mid_o + row * 128 + 4 * g;
       store_partial_row(dst, oacc, inv);
       if (g == 0) p.mid_lse[row] = (m + __builtin_amdgcn_logf(lt)) * kLn2;
@@ -645,8 +711,19 @@ __device__ __forceinline__ void stage1_mfma_unit(const Stage1Params& p, char* ld
   };
   auto finish_batch = [&](int t0) __attribute__((always_inline)) {
     if (WS) return;  // (the block's partial is merged from the four waves after the loop)
-    if (RANGE) {  // (one partial for the whole range)
-      if (t0 + kMfmaBatch >= t_end) flush(blk_begin);
+    if constexpr (RANGE) {
+      co_seg.t += kMfmaBatch;
+      if (co_seg.t >= co_seg.t_end) {  // the share's part of this request is done
+        flush(0);
+        if (co_seg.x_end < walk.end) {
+          reset();
+          co_seg = share_segment(p, walk, co_seg.r + 1, co_seg.x_end);
+          t_end = co_seg.t_end;
+          load_q(co_seg.r);
+          // the query has landed here, not at its first use in the loop, where the wait would be for the rows in flight in every trip
+          asm volatile("" : "+v"(qb[0]), "+v"(qb[1]), "+v"(qb[2]), "+v"(qb[3]));
+        }
+      }
       return;
     }
     if ((t0 + kMfmaBatch - t_begin) % bs == 0 || t0 + kMfmaBatch >= t_end) {
@@ -661,26 +738,44 @@ __device__ __forceinline__ void stage1_mfma_unit(const Stage1Params& p, char* ld
   // oldest group one wait earlier (that vmcnt(24), in front of an issue, is a no-op except in the first trip).
   u32x4 kr0[8], vr0[8], kr1[8], vr1[8];
   Slots s_even, s_odd;
-  load_slots(t_begin, s_even);
-  load_slots(t_begin + kStep, s_odd);
+  // the slot numbers of batch j, j counting up by one from call to call
+  auto next_slots = [&](int j, Slots& sl) __attribute__((always_inline)) {
+    if constexpr (RANGE) {
+      load_slots(sl_seg.t, sl);  // (past the share's end: the last batch again, never used)
+      if (sl_seg.t + kMfmaBatch < sl_seg.t_end) {
+        sl_seg.t += kMfmaBatch;
+      } else if (sl_seg.x_end < walk.end) {
+        sl_seg = share_segment(p, walk, sl_seg.r + 1, sl_seg.x_end);
+        t_last = sl_seg.t_end - 1;
+        table = p.req_to_tokens + (int64_t)sl_seg.req * p.max_seq_len;
+      }
+    } else {
+      load_slots(t_begin + j * kStep, sl);
+    }
+  };
+  next_slots(0, s_even);
+  next_slots(1, s_odd);
   wait_slots(std::integral_constant<int, 8>{}, s_even);
   issue(s_even, kr0, vr0);
   // two batches per trip, so that the register set of a batch is a compile-time choice
   for (int j = 0; j < n_batches; j += 2) {
-    const int t0 = t_begin + j * kStep;
-    load_slots(t0 + 2 * kStep, s_even);                     // slots(j+2): rows(j) have been addressed
+    next_slots(j + 2, s_even);                              // slots(j+2): rows(j) have been addressed
     wait_slots(std::integral_constant<int, 24>{}, s_odd);   // slots(j+1) usable
     issue(s_odd, kr1, vr1);                                 // rows(j+1) (past the end: the last row again, never used)
     wait_rows(kr0, vr0);
-    compute(t0, kr0, vr0);
-    finish_batch(t0);
-    load_slots(t0 + 3 * kStep, s_odd);                      // slots(j+3)
+    {
+      const int t0 = RANGE ? co_seg.t : t_begin + j * kStep;
+      compute(t0, kr0, vr0);
+      finish_batch(t0);
+    }
+    next_slots(j + 3, s_odd);                               // slots(j+3)
     wait_slots(std::integral_constant<int, 24>{}, s_even);  // slots(j+2) usable
     issue(s_even, kr0, vr0);                                // rows(j+2)
     wait_rows(kr1, vr1);
     if (j + 1 < n_batches) {
-      compute(t0 + kStep, kr1, vr1);
-      finish_batch(t0 + kStep);
+      const int t0 = RANGE ? co_seg.t : t_begin + (j + 1) * kStep;
+      compute(t0, kr1, vr1);
+      finish_batch(t0);
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (rows requested past the end land before the registers are given back)
@@ -760,8 +855,12 @@ constexpr int64_t kListedFromWorkgroups = 32768;  // launches of the plain grid 
 constexpr int64_t kListedFromWorkgroupsCoarse = 8192;
 constexpr int64_t kListedCoarseTokens = 1024;
 constexpr int64_t kCUs = 256;                     // compute units of the MI355X
-constexpr int64_t kSharesMinBatch = 8;            // ... and from this many requests on (a few long requests: 4 x 131072 and 1 x 1048576 tokens measured 1 % behind the grids)
-constexpr int64_t kSharesMinBlocks = 4;           // equal shares from this many blocks per worker on (an upper bound from the longest request)
+// Equal shares from eight requests on wherever the plain shape would run, and for two to seven when the launch is large (waves of the plain
+// shape by the longest request): one request is even by itself and 1-3 % faster on the grids (65536 tokens, GQA 32/8: 50.8 us against
+// 52.6), a few long ones of one length 1 % (4 x 131072), a few ragged ones up to 13 % slower (4 of 1000 to 8000 tokens, MHA 32: 62 us
+// against 54; GQA 32/8, 1024 waves: 23.1 against 24.1).
+constexpr int64_t kSharesMinBatch = 8, kSharesMinWavesFew = 2048;
+constexpr int kShareUnits = 4;                    // a share holds at least so many units of kMfmaBatch tokens
 template <typename T>
 __global__ __launch_bounds__(kMfmaWaves * 64, 2) void decode_stage1_mfma_listed_kernel(Stage1Params p) {
   __shared__ __attribute__((aligned(1024))) char lds[kMfmaWaves * kMfmaStage];
@@ -813,74 +912,99 @@ __global__ __launch_bounds__(kMfmaWaves * 64, 2) void decode_stage1_mfma_listed_
   }
 }
 
-// The plain shape with the work dealt in equal shares (the fused call, whose partials are scratch).  All blocks of all
-// requests, request after request, form one line; the workgroups of a task group cut it into as many contiguous shares
-// as they have waves that walk tokens, and a wave computes its share of every request it touches into ONE partial (row
-// = the share's first block of that request).  Every wave gets the same number of blocks to
-// within one whatever the lengths are, a request long or short costs one partial per share it touches instead of one
-// per block (the partials, written while the gather saturates the memory system, cost eight times their bytes), and no
-// split size has to be guessed from the longest request.  Neighbouring workgroups hold the task groups of the same
-// share (all KV heads of a token are fetched at about the same time).  The merge that follows (decode_stage2_kernel with
-// SHARES) works out the same shares from the lengths and visits the rows that hold a partial, nothing else.
+// The plain shape with the work dealt in equal shares (the fused call, whose partials are scratch).  All units of
+// kMfmaBatch tokens of all requests, request after request, form one line, which the workgroups of a task group cut into V
+// contiguous shares, one per wave that walks tokens; a wave computes its share of every request it touches into ONE
+// partial.  Every wave gets the same number of tokens to within one batch whatever the lengths are, a request long or
+// short costs one partial per share it touches instead of one per block (the partials, written while the gather
+// saturates the memory system, cost eight times their bytes), and no split size has to be guessed from the longest request.
+// V is worked out from the tokens that exist: a share per wave that walks tokens of a grid of one workgroup per CU, but none
+// shorter than share_units units.  A launch costs about 7 us of start-up and finish plus its bytes at 6 to 6.6 TB/s; one
+// workgroup per CU (four waves with two batches of rows in flight each, 128 KB) keeps HBM as busy as two do and leaves half as
+// many partials: 24 requests of 200 to 4000 tokens, GQA 32/8, both launches 45.5 -> 39.3 us (56.4 with grids split by the
+// longest request), 64 of 512 to 8192 150 -> 146, 64 of 4000 to 30000 588 -> 582.  Share v of request r leaves partial
+// number v + r (the partials of a request lie side by side, and all of them are below V + batch: mid_o has a row per 256
+// tokens of the longest request and request, which bounds V).
+// Shares are handed to the workgroups first and to the waves of a workgroup that walk tokens second: few shares then sit on
+// as many CUs.  Neighbouring workgroups hold the task groups of the same share (all KV heads of a token are fetched at
+// about the same time).  The merge that follows (decode_merge_shares_kernel) works out the same shares.
+struct Shares {
+  uint32_t total, V;
+  __device__ __forceinline__ Shares(uint32_t total_, uint32_t max_shares, uint32_t share_units) {
+    total = total_;
+    V = total / share_units;
+    V = V > max_shares ? max_shares : V < 1 ? 1 : V;
+  }
+  // quotients of integers below 2^38 by integers below 2^27 are exact through a double: the fraction is 0 or at least 2^-27
+  __device__ __forceinline__ uint32_t begin(uint32_t v) const { return (uint32_t)((double)v * (double)total / (double)V); }
+  __device__ __forceinline__ uint32_t of(uint32_t unit) const { return (uint32_t)(((double)(unit + 1) * (double)V - 1.0) / (double)total); }
+};
 template <typename T>
 __global__ __launch_bounds__(kMfmaWaves * 64, 2) void decode_stage1_mfma_range_kernel(Stage1Params p) {
   __shared__ __attribute__((aligned(1024))) char lds[kMfmaWaves * kMfmaStage];
-  __shared__ uint32_t first_block[kListedMaxBatch + 1];
+  __shared__ uint32_t first_unit[kListedMaxBatch + 1];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int tw = p.tasks_on_x & 7, cw = kMfmaWaves / tw;
+  const int tw = p.tasks_on_x & 7;
   const uint32_t task_groups = (uint32_t)((p.tasks + tw - 1) / tw);
   const int batch = (int)p.batch;  // <= kListedMaxBatch (checked on the host)
-  if (wave == 0) {
-    uint32_t carry = 0;
-    for (int b0 = 0; b0 < batch; b0 += 64) {
-      const int bb = b0 + lane;
-      uint32_t blocks = 0;
-      if (bb < batch) {
-        const int len = p.b_seqlen[bb];
-        int64_t nblk = len <= 0 ? 0 : ((int64_t)len + p.block_seq - 1) / p.block_seq;  // (the same clamps as in the unit)
-        if (nblk > p.grid_blocks) nblk = p.grid_blocks;
-        if (nblk > p.num_blocks) nblk = p.num_blocks;
-        blocks = (uint32_t)nblk;
-      }
-      uint32_t incl = blocks;  // inclusive prefix sum over the 64 lanes
+  // units in front of each request: a wave counts up to 64 requests in its registers, more go through LDS
+  ShareWalk w;
+  w.first_unit = first_unit;
+  w.incl = 0;
+  w.len = w.req = 0;
+  uint32_t total;
+  auto scan64 = [&](int len) __attribute__((always_inline)) {
+    uint32_t s = share_units_of(len, kMfmaBatch, p.grid_blocks);
 #pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t up = __shfl_up(incl, d, 64);
-        if (lane >= d) incl += up;
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t up = __shfl_up(s, d, 64);
+      if (lane >= d) s += up;
+    }
+    return s;
+  };
+  w.in_registers = batch <= 64;
+  if (w.in_registers) {
+    if (lane < batch) {
+      w.len = p.b_seqlen[lane];
+      w.req = p.b_req_idx[lane];
+    }
+    w.incl = scan64(w.len);
+    total = __builtin_amdgcn_readlane(w.incl, 63);
+  } else {
+    if (wave == 0) {
+      uint32_t carry = 0;
+      if (lane == 0) first_unit[0] = 0;
+      for (int b0 = 0; b0 < batch; b0 += 64) {
+        const uint32_t s = scan64(b0 + lane < batch ? p.b_seqlen[b0 + lane] : 0);
+        if (b0 + lane < batch) first_unit[b0 + lane + 1] = carry + s;
+        carry += __builtin_amdgcn_readlane(s, 63);
       }
-      if (bb < batch) first_block[bb] = carry + incl - blocks;
-      carry += __builtin_amdgcn_readlane(incl, 63);
     }
-    if (lane == 0) first_block[batch] = carry;
+    __syncthreads();
+    total = first_unit[batch];
   }
-  __syncthreads();
-  const uint64_t total = first_block[batch];
-  // the wave's share: worker v of V, over the workgroups of its task group and their waves that walk tokens
+  const Shares shares(total, (uint32_t)p.max_shares, (uint32_t)p.share_units);
   const uint32_t tg = blockIdx.x % task_groups;
-  const uint64_t V = (uint64_t)(gridDim.x / task_groups) * cw;
-  const uint64_t v = (uint64_t)(blockIdx.x / task_groups) * cw + (wave / tw);
-  uint32_t x = (uint32_t)(v * total / V);
-  const uint32_t hi_all = (uint32_t)((v + 1) * total / V);
-  if (x >= hi_all) return;
-  // the request that holds block x: first_block[lo] <= x < first_block[hi] throughout (requests without blocks are skipped)
-  int lo = 0, hi = batch;
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    const uint32_t f = __builtin_amdgcn_readfirstlane(first_block[mid]);
-    if (f <= x) lo = mid;
-    else hi = mid;
-  }
-  int r = lo;
-  while (x < hi_all) {
-    const uint32_t r0 = __builtin_amdgcn_readfirstlane(first_block[r]), r1 = __builtin_amdgcn_readfirstlane(first_block[r + 1]);
-    if (r1 > x) {
-      const uint32_t end = r1 < hi_all ? r1 : hi_all;
-      stage1_mfma_unit<T, false, true, true>(p, lds, lane, wave, r, tg, 0, 0, (int64_t)(x - r0), (int64_t)(end - r0));
-      x = end;
+  w.v = (uint32_t)(wave / tw) * (gridDim.x / task_groups) + blockIdx.x / task_groups;
+  if (w.v >= shares.V) return;
+  w.x = __builtin_amdgcn_readfirstlane(shares.begin(w.v));
+  w.end = __builtin_amdgcn_readfirstlane(shares.begin(w.v + 1));
+  if (w.x >= w.end) return;
+  // the request that holds unit x: the last one whose first unit is not past it
+  if (w.in_registers) {
+    w.r = __builtin_popcountll(__builtin_amdgcn_ballot_w64(w.incl <= w.x));
+  } else {
+    int lo = 0, hi = batch;
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      const uint32_t f = __builtin_amdgcn_readfirstlane(first_unit[mid]);
+      if (f <= w.x) lo = mid;
+      else hi = mid;
     }
-    r++;
+    w.r = lo;
   }
+  stage1_mfma_unit<T, false, true, true>(p, lds, lane, wave, 0, tg, 0, 0, w);
 }
 
 // ------------------------------------------------------------------------------------
@@ -897,9 +1021,8 @@ struct Stage2Params {
   const float* mid_lse;
   int64_t batch, heads, num_seq_blocks, block_seq;
   int64_t blk_rows, req_rows;  // rows of mid_o between consecutive blocks / requests
-  int64_t grid_blocks;         // (SHARES) stage 1's bound on a request's blocks, from the longest request
-  int64_t shares_workers;      // (SHARES) the shares stage 1 dealt the blocks of all requests in
-  uint32_t workers_mul, workers_shr;  // (SHARES) n / shares_workers = umulhi(n, mul) >> shr for n < 2^31 (mul = 0: shares_workers = 1)
+  int64_t grid_blocks;         // (SHARES) stage 1's bound on a request's units, from the longest request
+  int64_t max_shares, share_units;  // (SHARES) as in Stage1Params
 };
 
 template <typename OT> __device__ __forceinline__ void store4(void* base, int64_t elem, const f32x4& v);
@@ -913,68 +1036,15 @@ template <> __device__ __forceinline__ void store4<BF16>(void* base, int64_t ele
   *(u32x2*)((uint16_t*)base + elem) = u32x2{pack2<BF16>(v[0], v[1]), pack2<BF16>(v[2], v[3])};
 }
 
-// SHARES: behind decode_stage1_mfma_range_kernel, which dealt the blocks of all requests, request after request, in
-// shares_workers equal shares and left one partial per share and request, at the row of the share's first block of the
-// request.  The workgroup counts the blocks in front of its request and in all (the same clamps as stage 1), lists the
-// shares that begin inside its request, and visits those rows (and row 0, where the share that reaches into the
-// request from the one before it, or begins with it, left its partial).
-template <typename OT, int D, int NT, bool SHARES = false>
+template <typename OT, int D, int NT>
 __global__ __launch_bounds__(NT) void decode_stage2_kernel(Stage2Params p) {
   constexpr int LPR = D / 4;      // lanes per row (float4 each)
   constexpr int SL = NT / LPR;    // slices walking the block axis
   const int64_t b = blockIdx.x / (uint32_t)p.heads, h = blockIdx.x % (uint32_t)p.heads;
   const int slice = threadIdx.x / LPR, c = threadIdx.x % LPR;
-  auto blocks_of = [&](int64_t len) -> int64_t {
-    int64_t nb = len <= 0 ? 0 : (len + p.block_seq - 1) / p.block_seq;
-    if (nb > p.num_seq_blocks) nb = p.num_seq_blocks;
-    if (SHARES && nb > p.grid_blocks) nb = p.grid_blocks;
-    return nb;
-  };
-  int64_t n = blocks_of(p.b_seqlen[b]);
-  // SHARES: entry i of the rows to visit is row 0 for i = 0, else the first block of share v_lo + i - 1 (its distance from
-  // the request's first block); an entry whose share is empty (more shares than blocks) holds nothing
-  uint64_t first = 0, total = 1, v_lo = 0;
-  const uint64_t V = SHARES ? (uint64_t)p.shares_workers : 1;
-  uint64_t per_share = 0;  // total / V ...
-  uint32_t rest = 0;       // ... and total % V: share v begins at block v * per_share + v * rest / V (v * rest < V * V: 32 bits)
-  auto share_begin = [&](uint64_t v) -> uint64_t {
-    const uint32_t t = (uint32_t)v * rest;
-    return v * per_share + (p.workers_mul ? __umulhi(t, p.workers_mul) >> p.workers_shr : t);
-  };
-  if (SHARES) {
-    uint32_t pre = 0, tot = 0;
-    for (int64_t i = threadIdx.x; i < p.batch; i += NT) {
-      const uint32_t nb = (uint32_t)blocks_of(p.b_seqlen[i]);
-      tot += nb;
-      if (i < b) pre += nb;
-    }
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) {
-      pre += __shfl_xor(pre, d, 64);
-      tot += __shfl_xor(tot, d, 64);
-    }
-    __shared__ uint32_t red[2][NT / 64];
-    if ((threadIdx.x & 63) == 0) {
-      red[0][threadIdx.x >> 6] = pre;
-      red[1][threadIdx.x >> 6] = tot;
-    }
-    __syncthreads();
-    pre = tot = 0;
-#pragma unroll
-    for (int w = 0; w < NT / 64; w++) {
-      pre += red[0][w];
-      tot += red[1][w];
-    }
-    first = pre;
-    total = tot > 0 ? tot : 1;
-    per_share = total / V;
-    rest = (uint32_t)(total - per_share * V);
-    if (n > 0) {
-      v_lo = ((first + 1) * V + total - 1) / total;                        // the first share that begins behind block 0 of the request
-      const uint64_t v_end = ((first + (uint64_t)n) * V + total - 1) / total;  // one past the last share that begins inside it
-      n = 1 + (int64_t)(v_end > v_lo ? v_end - v_lo : 0);
-    }
-  }
+  const int len = p.b_seqlen[b];
+  int64_t n = len <= 0 ? 0 : ((int64_t)len + p.block_seq - 1) / p.block_seq;
+  if (n > p.num_seq_blocks) n = p.num_seq_blocks;
   const int64_t row_stride = p.blk_rows;
   const int64_t row0 = b * p.req_rows + h;
   const int64_t out_row = b * p.heads + h;
@@ -1003,15 +1073,8 @@ __global__ __launch_bounds__(NT) void decode_stage2_kernel(Stage2Params p) {
 #pragma unroll
     for (int u = 0; u < U; u++) {
       const int64_t e = i + u * SL < n ? i + u * SL : n - 1;
-      int64_t blk = e;
       holds[u] = i + u * SL < n;
-      if (SHARES && e > 0) {
-        const uint64_t v = v_lo + (uint64_t)e - 1;
-        const uint64_t x = share_begin(v);
-        blk = (int64_t)(x - first);
-        holds[u] = holds[u] && share_begin(v + 1) > x;  // (an empty share left nothing)
-      }
-      const int64_t row = blk * row_stride + row0;
+      const int64_t row = e * row_stride + row0;
       lse[u] = p.mid_lse[row];
       tv[u] = *(const f32x4*)(p.mid_o + row * D + c * 4);
     }
@@ -1042,6 +1105,104 @@ __global__ __launch_bounds__(NT) void decode_stage2_kernel(Stage2Params p) {
     const float inv = Lt > 0.f ? 1.f / Lt : 0.f;
     store4<OT>(p.o, out_row * D + c * 4, a * inv);
     if (c == 0) p.out_lse[out_row] = Lt > 0.f ? Mt + __builtin_amdgcn_logf(Lt) * kLn2 : -INFINITY;
+  }
+}
+
+// The merge behind decode_stage1_mfma_range_kernel: W waves per (request, head), 4 / W pairs per workgroup (heads of one
+// request).  Every wave counts the units in front of its request and in all and knows from them the first and the last
+// share that reach into the request: their partials are consecutive rows.  Half a wave reads a row (16 bytes a lane), eight
+// rows and their log-sum-exps in flight per half wave.  Bound by its chain of dependent loads (the argument block, the lengths, the rows)
+// and, from a few thousand pairs on, by the workgroups' turn-over: with a whole workgroup of eight slices per pair, as in
+// decode_stage2_kernel, 128 requests with 32 heads took 10.2 us for one to three rows each.
+template <typename OT, int W>
+__global__ __launch_bounds__(256) void decode_merge_shares_kernel(Stage2Params p) {
+  constexpr int D = 128, U = 8;
+  constexpr int PAIRS = 4 / W;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint32_t head_groups = ((uint32_t)p.heads + PAIRS - 1) / PAIRS;
+  const int b = blockIdx.x / head_groups;
+  const int h = (int)(blockIdx.x % head_groups) * PAIRS + wave / W;
+  uint32_t pre = 0, tot = 0;
+  for (int i = lane; i < (int)p.batch; i += 64) {
+    const uint32_t u = share_units_of(p.b_seqlen[i], kMfmaBatch, p.grid_blocks);
+    tot += u;
+    pre += i < b ? u : 0u;
+  }
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) {
+    pre += __shfl_xor(pre, d, 64);
+    tot += __shfl_xor(tot, d, 64);
+  }
+  const uint32_t units = share_units_of(p.b_seqlen[b], kMfmaBatch, p.grid_blocks);
+  const bool live = h < (int)p.heads;  // (the last group of heads may be short)
+  int n = 0;
+  int64_t row0 = 0;
+  if (units > 0 && live) {
+    const Shares shares(tot, (uint32_t)p.max_shares, (uint32_t)p.share_units);
+    const uint32_t v0 = shares.of(pre), v1 = shares.of(pre + units - 1);
+    n = (int)(v1 - v0) + 1;
+    row0 = ((int64_t)v0 + b) * p.heads + h;
+  }
+  const int half = lane >> 5, c = lane & 31;
+  const int slice = (wave % W) * 2 + half;
+  float M = -INFINITY, L = 0.f;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < n; i += U * 2 * W) {  // (i and n are the same for the whole wave)
+    float lse[U];
+    f32x4 tv[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int e = i + u * 2 * W + slice;
+      const int64_t row = row0 + (int64_t)(e < n ? e : n - 1) * p.heads;
+      lse[u] = e < n ? p.mid_lse[row] : -INFINITY;
+      tv[u] = *(const f32x4*)(p.mid_o + row * D + c * 4);
+    }
+    float Mn = M;
+#pragma unroll
+    for (int u = 0; u < U; u++) Mn = fmaxf(Mn, lse[u]);
+    const float so = exp2_diff(M * kLog2e, Mn * kLog2e);
+    acc *= so;
+    L *= so;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const float w = exp2_diff(lse[u] * kLog2e, Mn * kLog2e);  // (0 past the last row)
+      acc += tv[u] * w;
+      L += w;
+    }
+    M = Mn;
+  }
+  auto join = [&](float Mo, float Lo, const f32x4& ao) {
+    const float Mn = fmaxf(M, Mo);
+    const float a = exp2_diff(M * kLog2e, Mn * kLog2e), o = exp2_diff(Mo * kLog2e, Mn * kLog2e);
+    acc = acc * a + ao * o;
+    L = L * a + Lo * o;
+    M = Mn;
+  };
+  {
+    f32x4 ao;
+#pragma unroll
+    for (int e = 0; e < 4; e++) ao[e] = __shfl_xor(acc[e], 32, 64);
+    const float Mo = __shfl_xor(M, 32, 64), Lo = __shfl_xor(L, 32, 64);
+    join(Mo, Lo, ao);
+  }
+  if constexpr (W > 1) {
+    __shared__ float sM[W], sL[W];
+    __shared__ f32x4 sAcc[W][32];
+    if (half == 0) sAcc[wave][c] = acc;
+    if (lane == 0) {
+      sM[wave] = M;
+      sL[wave] = L;
+    }
+    __syncthreads();
+    if (wave != 0) return;
+#pragma unroll
+    for (int w = 1; w < W; w++) join(sM[w], sL[w], sAcc[w][c]);
+  }
+  if (half == 0 && live) {
+    const int64_t out_row = (int64_t)b * p.heads + h;
+    const float inv = L > 0.f ? 1.f / L : 0.f;
+    store4<OT>(p.o, out_row * D + c * 4, acc * inv);
+    if (c == 0) p.out_lse[out_row] = L > 0.f ? M + __builtin_amdgcn_logf(L) * kLn2 : -INFINITY;
   }
 }
 
@@ -1111,8 +1272,15 @@ static int launch_stage1(const lsattn_decode_stage1_args* a, hipStream_t st) {
 
 // Large launches: the matrix-pipe kernel, when its conditions hold (blocks a multiple of 32 tokens, enough waves to fill
 // the chip); lsattn_set_tuning forces the choice where the conditions allow it (tuning, tests).
+// What the fused call hands to stage 1 and on to the merge behind it.
+struct SharesPlan {
+  int64_t units;           // in: kMfmaBatch-token units of the longest request
+  int64_t rows;            // in: rows of the partials' buffers per request, as far as the longest request goes
+  int64_t max_shares = 0;  // out: 0 if the launch was none for equal shares
+};
+
 // `shares`: deal the blocks in equal shares (decode_stage1_mfma_range_kernel) or launch nothing (*taken stays false).
-template <typename T> static int launch_stage1_mfma(const lsattn_decode_stage1_args* a, hipStream_t st, bool* taken, int64_t* shares = nullptr) {
+template <typename T> static int launch_stage1_mfma(const lsattn_decode_stage1_args* a, hipStream_t st, bool* taken, SharesPlan* shares = nullptr) {
   *taken = false;
   const int group = (int)(a->num_q_heads / a->num_kv_heads);
   Stage1Params p;
@@ -1166,20 +1334,30 @@ template <typename T> static int launch_stage1_mfma(const lsattn_decode_stage1_a
   if (tn.decode_stage1 == LSATTN_DECODE_STAGE1_MFMA) use = true, split_waves = false;
   if (tn.decode_stage1 == LSATTN_DECODE_STAGE1_SPLIT && can_split) use = false, split_waves = true;
   if (shares) {
-    // only where the plain shape would run, on launches with at least kSharesMinBlocks blocks of 256 tokens and more per
-    // worker to deal (fewer: the grids above, whose workgroups the hardware hands out as they finish)
-    const int tws = p.tasks >= 4 ? 4 : p.tasks >= 2 ? 2 : 1;
-    const int64_t task_groups = (p.tasks + tws - 1) / tws;
-    int64_t per_group = 2 * kCUs / task_groups;  // workgroups per task group: two workgroups per CU in all
+    const int64_t task_groups = (p.tasks + tw - 1) / tw;
     const bool forced = tn.decode_listed == LSATTN_DECODE_LISTED_SHARES;  // (tests: whatever the launch's size)
     if (tn.decode_listed == LSATTN_DECODE_LISTED_OFF || tn.decode_listed == LSATTN_DECODE_LISTED_ON) return LSATTN_OK;
-    if (per_group < 1 || p.row_mul != 1 || a->batch > kListedMaxBatch || nblk * a->batch > 0x7fffffff) return LSATTN_OK;
-    const int64_t workers = per_group * (kMfmaWaves / tws);
-    if (!forced && (!use || split_waves || a->seq_block_size < 256 || a->batch < kSharesMinBatch || nblk * a->batch < kSharesMinBlocks * workers)) return LSATTN_OK;
+        int64_t per_group = kCUs / task_groups;  // workgroups per task group: one workgroup per CU in all
+    if (per_group < 1 || p.row_mul != 1 || a->batch > kListedMaxBatch || shares->units * a->batch > 0x7ffffff) return LSATTN_OK;
+    // partials are numbered below V + batch - 1: the rows of the buffers that the longest request can reach
+    const int64_t by_rows = a->batch * (shares->rows - 1) + 1;
+    int64_t max_shares = per_group * cw;
+    if (max_shares > by_rows) max_shares = by_rows;
+    const int64_t by_tokens = shares->units * a->batch / kShareUnits;
+    if (max_shares > by_tokens) max_shares = by_tokens > 0 ? by_tokens : 1;
+    if (!forced && tn.decode_stage1 != 0) return LSATTN_OK;
+    // (waves of the plain shape at 256 tokens each, whatever the split asked for; the shape whose waves split a block keeps its launches)
+    const int64_t waves256 = (shares->units * kMfmaBatch + 255) / 256 * p.tasks * a->batch;
+    const bool large = waves256 >= (group < 4 ? 768 : p.tasks < 4 ? 3073 : 513);
+    if (!forced && (!large || a->batch < 2 || (a->batch < kSharesMinBatch && waves256 < kSharesMinWavesFew))) return LSATTN_OK;
+    if (per_group > max_shares) per_group = max_shares;
     *taken = true;
-    *shares = workers;
-    p.tasks_on_x = tws;
-    p.blocks_per_wg = 1;
+    shares->max_shares = max_shares;
+    p.max_shares = (int32_t)max_shares;
+    p.share_units = kShareUnits;
+    p.block_seq = p.fine_block_seq = kMfmaBatch;
+    p.grid_blocks = shares->units;
+    p.tasks_on_x = tw;
     LSATTN_LAUNCH_KERNEL((decode_stage1_mfma_range_kernel<T>), dim3((unsigned)(per_group * task_groups)), dim3(kMfmaWaves * 64), 0, st, p);
     return check_launch();
   }
@@ -1215,9 +1393,9 @@ template <typename T> static int launch_stage1_mfma(const lsattn_decode_stage1_a
   return check_launch();
 }
 
-template <typename T> static int dispatch_stage1(const lsattn_decode_stage1_args* a, hipStream_t st, int64_t* shares = nullptr) {
+template <typename T> static int dispatch_stage1(const lsattn_decode_stage1_args* a, hipStream_t st, SharesPlan* shares = nullptr) {
   const int group = (int)(a->num_q_heads / a->num_kv_heads);
-  if (shares) {  // (in equal shares or not at all: *shares is their number, or stays 0)
+  if (shares) {  // (in equal shares or not at all: shares->max_shares stays 0 then)
     bool taken;
     return launch_stage1_mfma<T>(a, st, &taken, shares);
   }
@@ -1239,9 +1417,8 @@ template <typename T> static int dispatch_stage1(const lsattn_decode_stage1_args
 
 using namespace lsattn;
 
-// `shares` (the fused call): launch stage 1 in equal shares if the launch is one for them (*shares: how many) or nothing.
-static int decode_stage1(const lsattn_decode_stage1_args* a, void* stream, int64_t* shares) {
-  if (shares) *shares = 0;
+// `shares` (the fused call): launch stage 1 in equal shares if the launch is one for them (max_shares > 0 then) or nothing.
+static int decode_stage1(const lsattn_decode_stage1_args* a, void* stream, SharesPlan* shares) {
   if (!a || !a->mid_o || !a->mid_o_logexpsum || !a->q || !a->k || !a->v || !a->req_to_tokens || !a->b_req_idx ||
       !a->b_seqlen)
     return LSATTN_ERR_INVALID_ARG;
@@ -1267,12 +1444,11 @@ extern "C" int lsattn_decode_stage1(const lsattn_decode_stage1_args* a, void* st
 // `live_blocks`: an upper bound of the partial rows any request has (the rows of the buffer, or fewer when the caller
 // knows the longest request); it picks the shape of the merge, which decides the order of its additions.
 template <typename OT> static int dispatch_stage2(const Stage2Params& p, int64_t D, dim3 grid, int64_t live_blocks, hipStream_t st) {
-  if (p.shares_workers > 0) {
+  if (p.max_shares > 0) {
     if (D != 128) return LSATTN_ERR_UNSUPPORTED;
-    // (a request's partials: at most one per share and one more, and no more than it has blocks)
-    const int64_t most = live_blocks < p.shares_workers + 1 ? live_blocks : p.shares_workers + 1;
-    if (most >= 64 && (int64_t)grid.x < 2048) LSATTN_LAUNCH_KERNEL((decode_stage2_kernel<OT, 128, 1024, true>), grid, dim3(1024), 0, st, p);
-    else LSATTN_LAUNCH_KERNEL((decode_stage2_kernel<OT, 128, 256, true>), grid, dim3(256), 0, st, p);
+    // four waves per pair while that keeps every pair resident at once (sixteen waves per CU)
+    if ((int64_t)grid.x <= 4 * kCUs) LSATTN_LAUNCH_KERNEL((decode_merge_shares_kernel<OT, 4>), grid, dim3(256), 0, st, p);
+    else LSATTN_LAUNCH_KERNEL((decode_merge_shares_kernel<OT, 1>), dim3((unsigned)(p.batch * ((p.heads + 3) / 4))), dim3(256), 0, st, p);
     return check_launch();
   }
   // few (batch, head) pairs with many partials each (long contexts at small batch): 1024 threads walk the block axis in 32
@@ -1290,7 +1466,7 @@ template <typename OT> static int dispatch_stage2(const Stage2Params& p, int64_t
   return check_launch();
 }
 
-static int decode_stage2(const lsattn_decode_stage2_args* a, int64_t live_blocks, void* stream, int64_t shares_workers = 0, int64_t grid_blocks = 0) {
+static int decode_stage2(const lsattn_decode_stage2_args* a, int64_t live_blocks, void* stream, const SharesPlan* shares = nullptr) {
   if (!a || !a->o || !a->out_logexpsum || !a->b_seqlen || !a->mid_o || !a->mid_o_logexpsum) return LSATTN_ERR_INVALID_ARG;
   if (a->batch < 0 || a->num_heads <= 0 || a->num_seq_blocks < 0 || a->block_seq < 1) return LSATTN_ERR_INVALID_ARG;
   if (((uintptr_t)a->o | (uintptr_t)a->mid_o) & 15) return LSATTN_ERR_INVALID_ARG;
@@ -1300,13 +1476,8 @@ static int decode_stage2(const lsattn_decode_stage2_args* a, int64_t live_blocks
   Stage2Params p{a->o, a->out_logexpsum, a->b_seqlen, a->mid_o, a->mid_o_logexpsum,
                  a->batch, a->num_heads, a->num_seq_blocks, a->block_seq,
                  a->partials_by_request ? a->num_heads : a->batch * a->num_heads,
-                 a->partials_by_request ? a->num_seq_blocks * a->num_heads : a->num_heads, grid_blocks, shares_workers, 0, 0};
-  if (shares_workers > 1) {  // (shares_workers <= 2048: v * rest stays far below 2^31)
-    uint32_t L = 0;
-    while ((1u << L) < (uint32_t)shares_workers) L++;
-    p.workers_mul = (uint32_t)((((uint64_t)1 << (31 + L)) + shares_workers - 1) / shares_workers);
-    p.workers_shr = L - 1;
-  }
+                 a->partials_by_request ? a->num_seq_blocks * a->num_heads : a->num_heads, shares ? shares->units : 0,
+                 shares ? shares->max_shares : 0, kShareUnits};
   dim3 grid((unsigned)(a->batch * a->num_heads));
   hipStream_t st = (hipStream_t)stream;
   switch (a->o_dtype) {
@@ -1328,23 +1499,21 @@ extern "C" int lsattn_decode_attention(const lsattn_decode_stage1_args* s1, cons
       s1->batch != s2->batch || s1->num_q_heads != s2->num_heads || s1->num_blocks != s2->num_seq_blocks ||
       s1->head_dim != s2->head_dim || s1->seq_block_size != s2->block_seq || !s1->partials_by_request != !s2->partials_by_request)
     return LSATTN_ERR_INVALID_ARG;
-  // Large launches deal the tokens in equal shares (decode_stage1_mfma_range_kernel), however coarse the split asked
-  // for: the partials are scratch here, and a share leaves one partial per request it touches whatever the block size.
-  // The blocks the shares are counted in: 256 tokens, or the smallest multiple by a power of two whose rows the buffers hold
-  // (a share's partial goes to the row of its first block).
-  if (s1->merge_blocks <= 1 && s1->seq_block_size >= 256 && s1->max_len_in_batch > 0 && s1->num_blocks > 0) {
-    int64_t g = 256;
-    while ((s1->max_len_in_batch + g - 1) / g > s1->num_blocks) g *= 2;
-    lsattn_decode_stage1_args a1 = *s1;
-    a1.seq_block_size = g;
-    int64_t shares = 0;
-    const int rc1 = decode_stage1(&a1, stream, &shares);
+  // Most launches deal the tokens in equal shares (decode_stage1_mfma_range_kernel), however coarse the split asked for: the
+  // partials are scratch here.  The rows the shares may fill are counted from the longest request, at most one per 256
+  // of its tokens, so that the result does not depend on the height of the buffers where they are tall enough for that.
+  if (s1->merge_blocks <= 1 && s1->seq_block_size >= 256 && s1->max_len_in_batch > 0 && s1->num_blocks > 0 &&
+      s1->max_len_in_batch < 0x7fffff00) {
+    SharesPlan shares;
+    shares.units = (s1->max_len_in_batch + kMfmaBatch - 1) / kMfmaBatch;
+    shares.rows = (s1->max_len_in_batch + 255) / 256;
+    if (shares.rows > s1->num_blocks) shares.rows = s1->num_blocks;
+    const int rc1 = decode_stage1(s1, stream, &shares);
     if (rc1 != LSATTN_OK) return rc1;
-    if (shares > 0) {
+    if (shares.max_shares > 0) {
       lsattn_decode_stage2_args a2 = *s2;
-      a2.block_seq = g;
-      const int64_t rows = (s1->max_len_in_batch + g - 1) / g;
-      return decode_stage2(&a2, rows, stream, shares, rows);
+      a2.block_seq = kMfmaBatch;
+      return decode_stage2(&a2, 0, stream, &shares);
     }
   }
   const int rc = lsattn_decode_stage1(s1, stream);
