@@ -286,6 +286,9 @@ int lsattn_decode_attention_static(const lsattn_decode_stage1_args* s1, const ls
  */
 int lsattn_kv_scatter(const void* src, int64_t src_stride_bytes, void* dst, int64_t dst_stride_bytes,
                       const int32_t* dest_index, int64_t n_rows, int64_t row_bytes, void* stream);
+/* The same with the slots as the allocator hands them out (int64). */
+int lsattn_kv_scatter_i64(const void* src, int64_t src_stride_bytes, void* dst, int64_t dst_stride_bytes,
+                          const int64_t* dest_index, int64_t n_rows, int64_t row_bytes, void* stream);
 
 /*
  * Prefill registration of freshly written slots:
@@ -447,7 +450,7 @@ typedef struct lsattn_rotary_kv_write_args {
   int64_t head_dim;
   void* pool;                   /* [slots, 2*Hkv*D] or NULL */
   int64_t pool_slot_stride;
-  const int32_t* dest_index;    /* [num_tokens] */
+  const void* dest_index;       /* [num_tokens], int32 or int64 (dest_index_is_i64) */
   int32_t* req_to_tokens;       /* [max_req, max_seq_len] */
   int64_t max_seq_len;
   const int32_t* b_req_idx;     /* [batch] */
@@ -456,7 +459,7 @@ typedef struct lsattn_rotary_kv_write_args {
   int64_t batch;
   int64_t max_len_in_batch;     /* register_mode 1: upper bound of b_seq_len[] (sizes the launch) */
   int32_t register_mode;
-  int32_t reserved;
+  int32_t dest_index_is_i64;    /* 0: int32; 1: int64, as the slot allocator hands them out */
 } lsattn_rotary_kv_write_args;
 int lsattn_rotary_kv_write(const lsattn_rotary_kv_write_args* a, void* stream);
 
@@ -483,7 +486,8 @@ int lsattn_pool_find_contiguous(const int32_t* mem_state, int64_t pool_size, int
                                 void* workspace, size_t workspace_bytes, void* stream);
 /*
  * mem_state[index[i]] = old value + delta (delta = +1 or -1) for i < n; a slot listed several times still changes
- * by delta once, as `mem_state[index] += delta` does in torch.  counted (device, int64[2]):
+ * by delta once, as `mem_state[index] += delta` does in torch.  counted (int64[2], device memory or pinned host memory that
+ * the device can write; both words are written once, when they are final):
  *   counted[0] = entries whose slot is non-zero before the update (delta = +1) or after it (delta = -1): the
  *                has_used_tokens / used_tokens of add_refs and decrease_refs (longserve_mem_manager.py:73-88);
  *   counted[1] = entries outside [-pool_size, pool_size), which are skipped (negative entries wrap once).

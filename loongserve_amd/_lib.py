@@ -122,7 +122,7 @@ class RotaryKvWriteArgs(C.Structure):  # mirrors lsattn_rotary_kv_write_args
                 ("cos", _vp), ("sin", _vp), ("num_tokens", _i64), ("head_dim", _i64),
                 ("pool", _vp), ("pool_slot_stride", _i64), ("dest_index", _vp),
                 ("req_to_tokens", _vp), ("max_seq_len", _i64), ("b_req_idx", _vp), ("b_start_loc", _vp), ("b_seq_len", _vp),
-                ("batch", _i64), ("max_len_in_batch", _i64), ("register_mode", _i32), ("reserved", _i32)]
+                ("batch", _i64), ("max_len_in_batch", _i64), ("register_mode", _i32), ("dest_index_is_i64", _i32)]
 
 
 EXPORTS = {
@@ -136,6 +136,7 @@ EXPORTS = {
     "lsattn_decode_attention": (C.c_int, [C.POINTER(DecodeStage1Args), C.POINTER(DecodeStage2Args), _vp]),
     "lsattn_decode_attention_static": (C.c_int, [C.POINTER(DecodeStage1Args), C.POINTER(DecodeStage2Args), _vp]),
     "lsattn_kv_scatter": (C.c_int, [_vp, _i64, _vp, _i64, _vp, _i64, _i64, _vp]),
+    "lsattn_kv_scatter_i64": (C.c_int, [_vp, _i64, _vp, _i64, _vp, _i64, _i64, _vp]),
     "lsattn_register_tokens": (C.c_int, [_vp, _i64, _vp, _vp, _vp, _vp, _i64, _i64, _vp]),
     "lsattn_register_decode_tokens": (C.c_int, [_vp, _i64, _vp, _vp, _vp, C.c_int32, _i64, _vp]),
     "lsattn_kv_ranges": (C.c_int, [_vp, _vp, _vp, C.c_int32, _i64, _vp, _vp, _vp, _vp]),

@@ -4,8 +4,8 @@
 // attribute read per field, a stream object, context managers), more than a small batch's kernels run; here it is about
 // 1 us in front of the launches themselves.
 //
-// Every function takes the common case only and returns None where an argument does not fit it (another type, a failed
-// check, an int64 slot vector where the kernel reads int32, ...), having launched nothing: the Python function then goes
+// Every function takes the common case only and returns None where an argument does not fit it (another type, a
+// failed check), having launched nothing: the Python function then goes
 // through its checked path, which converts or raises.  The library's entry points are handed over as addresses by _lib.load()
 // (bind), so that the same loaded library serves both routes.
 #include <torch/csrc/python_headers.h>
@@ -14,6 +14,9 @@
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
 
+#include <pybind11/pybind11.h>
+
+#include <chrono>
 #include <cmath>
 #include <cstring>
 
@@ -31,12 +34,14 @@ struct Library {
   decltype(&lsattn_decode_stage2) decode_stage2;
   decltype(&lsattn_decode_attention) decode_attention;
   decltype(&lsattn_kv_scatter) kv_scatter;
+  decltype(&lsattn_kv_scatter_i64) kv_scatter_i64;
   decltype(&lsattn_register_tokens) register_tokens;
   decltype(&lsattn_register_decode_tokens) register_decode_tokens;
   decltype(&lsattn_rms_norm) rms_norm;
   decltype(&lsattn_silu_and_mul_inplace) silu_and_mul_inplace;
-  decltype(&lsattn_rotary_emb) rotary_emb;
   decltype(&lsattn_rotary_kv_write) rotary_kv_write;
+  decltype(&lsattn_pool_alloc) pool_alloc;
+  decltype(&lsattn_pool_update_refs) pool_update_refs;
   decltype(&lsattn_strerror) strerror;
 } lib;
 
@@ -51,12 +56,14 @@ PyObject* bind(PyObject*, PyObject* addresses) {
       {"lsattn_decode_stage2", (void**)&lib.decode_stage2},
       {"lsattn_decode_attention", (void**)&lib.decode_attention},
       {"lsattn_kv_scatter", (void**)&lib.kv_scatter},
+      {"lsattn_kv_scatter_i64", (void**)&lib.kv_scatter_i64},
       {"lsattn_register_tokens", (void**)&lib.register_tokens},
       {"lsattn_register_decode_tokens", (void**)&lib.register_decode_tokens},
       {"lsattn_rms_norm", (void**)&lib.rms_norm},
       {"lsattn_silu_and_mul_inplace", (void**)&lib.silu_and_mul_inplace},
-      {"lsattn_rotary_emb", (void**)&lib.rotary_emb},
       {"lsattn_rotary_kv_write", (void**)&lib.rotary_kv_write},
+      {"lsattn_pool_alloc", (void**)&lib.pool_alloc},
+      {"lsattn_pool_update_refs", (void**)&lib.pool_update_refs},
       {"lsattn_strerror", (void**)&lib.strerror},
   };
   for (const auto& e : entries) {
@@ -127,6 +134,8 @@ bool is(const at::Tensor& t, at::ScalarType s) { return t.scalar_type() == s; }
 bool half(const at::Tensor& t) { return is(t, at::kHalf) || is(t, at::kBFloat16); }
 int dtype_of(const at::Tensor& t) { return is(t, at::kHalf) ? LSATTN_F16 : is(t, at::kBFloat16) ? LSATTN_BF16 : LSATTN_F32; }
 bool i32(const at::Tensor& t, int64_t n) { return is(t, at::kInt) && t.size(0) == n && t.is_contiguous(); }
+// one pool slot per row, int32 or as the allocator hands them out
+bool slots(const at::Tensor& t, int64_t n) { return (is(t, at::kInt) || is(t, at::kLong)) && t.size(0) == n && t.is_contiguous(); }
 const int32_t* pi32(const at::Tensor& t) { return (const int32_t*)t.data_ptr(); }
 bool same_shape(const at::Tensor& a, const at::Tensor& b) { return a.sizes() == b.sizes(); }
 at::Tensor empty(at::IntArrayRef sizes, const at::Tensor& like, at::ScalarType s) {
@@ -419,20 +428,23 @@ int64_t row_elements(const at::Tensor& t) {
   return n;
 }
 
-// (src, dest_index int32, pool) -> True or None
+// (src, dest_index int32 or int64, pool) -> True or None
 PyObject* kv_scatter(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   NEED_ARGS(3);
   Args in(args);
   const at::Tensor *src = in.maybe(), &index = in.gpu(1), *pool = in.maybe();
   OR_NONE(in.ok && src && pool && src->dim() >= 1 && src->dim() == pool->dim() && src->scalar_type() == pool->scalar_type());
-  OR_NONE(src->size(0) > 0 && pool->size(0) > 0 && i32(index, src->size(0)));
+  OR_NONE(src->size(0) > 0 && pool->size(0) > 0 && slots(index, src->size(0)));
   OR_NONE(src->sizes().slice(1) == pool->sizes().slice(1));
   const int64_t n = row_elements(*src), es = src->element_size();
   OR_NONE(n > 0 && row_elements(*pool) == n);
-  if (const int rc = lib.kv_scatter(src->data_ptr(), src->stride(0) * es, pool->data_ptr(), pool->stride(0) * es, pi32(index),
-                                    src->size(0), n * es, stream()))
-    return failed(rc, "lsattn_kv_scatter");
+  const int rc = is(index, at::kLong)
+                     ? lib.kv_scatter_i64(src->data_ptr(), src->stride(0) * es, pool->data_ptr(), pool->stride(0) * es,
+                                          (const int64_t*)index.data_ptr(), src->size(0), n * es, stream())
+                     : lib.kv_scatter(src->data_ptr(), src->stride(0) * es, pool->data_ptr(), pool->stride(0) * es, pi32(index),
+                                      src->size(0), n * es, stream());
+  if (rc) return failed(rc, "lsattn_kv_scatter");
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
 }
@@ -517,16 +529,19 @@ PyObject* rotary_emb(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const at::Tensor &q = in.gpu(3), &k = in.gpu(3), &c = in.gpu(2), &s = in.gpu(2);
   OR_NONE(in.ok);
   const int64_t T = q.size(0), D = q.size(2);
-  OR_NONE(rotary_operand(q, T, D) && rotary_operand(k, T, D) && angles(c, s, T, D));
-  void* st = stream();
-  for (const at::Tensor* x : {&q, &k})
-    if (const int rc = lib.rotary_emb(x->data_ptr(), c.data_ptr(), s.data_ptr(), x->stride(0), x->stride(1), T, x->size(1), D, st))
-      return failed(rc, "lsattn_rotary_emb");
+  OR_NONE(T > 0 && q.size(1) > 0 && k.size(1) > 0 && rotary_operand(q, T, D) && rotary_operand(k, T, D) && angles(c, s, T, D));
+  // both in one launch: the write-back of a step without pool and table
+  lsattn_rotary_kv_write_args a;
+  std::memset(&a, 0, sizeof a);
+  a.q = q.data_ptr(), a.q_stride_t = q.stride(0), a.q_stride_h = q.stride(1), a.num_q_heads = q.size(1);
+  a.kv = k.data_ptr(), a.kv_stride_t = k.stride(0), a.kv_stride_h = k.stride(1), a.num_kv_heads = k.size(1);
+  a.cos = c.data_ptr(), a.sin = s.data_ptr(), a.num_tokens = T, a.head_dim = D;
+  if (const int rc = lib.rotary_kv_write(&a, stream())) return failed(rc, "lsattn_rotary_kv_write");
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
 }
 
-// (q, cache_kv, cos, sin, mem_index int32, pool, table, b_req, b_len, b_start_loc, max_len, decode) -> True or None; pool or
+// (q, cache_kv, cos, sin, mem_index int32 or int64, pool, table, b_req, b_len, b_start_loc, max_len, decode) -> True or None; pool or
 // table may be None, b_start_loc with decode
 PyObject* rotary_kv_write(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
@@ -538,12 +553,12 @@ PyObject* rotary_kv_write(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const bool decode = in.integer() != 0;
   OR_NONE(in.ok);
   const int64_t T = q.size(0), D = q.size(2);
-  OR_NONE(rotary_operand(q, T, D) && rotary_operand(kv, T, D) && kv.size(1) % 2 == 0 && angles(c, s, T, D) && i32(mem, T));
+  OR_NONE(rotary_operand(q, T, D) && rotary_operand(kv, T, D) && kv.size(1) % 2 == 0 && angles(c, s, T, D) && slots(mem, T));
   lsattn_rotary_kv_write_args a;
   std::memset(&a, 0, sizeof a);
   a.q = q.data_ptr(), a.q_stride_t = q.stride(0), a.q_stride_h = q.stride(1), a.num_q_heads = q.size(1);
   a.kv = kv.data_ptr(), a.kv_stride_t = kv.stride(0), a.kv_stride_h = kv.stride(1), a.num_kv_heads = kv.size(1) / 2;
-  a.cos = c.data_ptr(), a.sin = s.data_ptr(), a.num_tokens = T, a.head_dim = D, a.dest_index = pi32(mem);
+  a.cos = c.data_ptr(), a.sin = s.data_ptr(), a.num_tokens = T, a.head_dim = D, a.dest_index = mem.data_ptr(), a.dest_index_is_i64 = is(mem, at::kLong);
   if (pool) {
     OR_NONE(pool->dim() == 3 && is(*pool, at::kHalf) && pool->sizes().slice(1) == kv.sizes().slice(1) &&
             row_elements(*pool) == kv.size(1) * D);
@@ -568,12 +583,65 @@ PyObject* rotary_kv_write(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// ------------------------------------------------------------------------------------------------ slot allocator
+// (state int32, need, workspace) -> int64 [need]
+PyObject* pool_alloc(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  NEED_ARGS(3);
+  Args in(args);
+  const at::Tensor& state = in.gpu(1);
+  const int64_t need = in.integer();
+  const at::Tensor& ws = in.gpu(1);
+  if (!in.ok || need < 0) return PyErr_Format(PyExc_ValueError, "pool_alloc: bad arguments");
+  const at::Tensor out = empty({need}, state, at::kLong);
+  if (const int rc = lib.pool_alloc((int32_t*)state.data_ptr(), state.size(0), need, need ? (int64_t*)out.data_ptr() : nullptr,
+                                    ws.data_ptr(), ws.nbytes(), stream()))
+    return failed(rc, "lsattn_pool_alloc");
+  return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
+}
+
+// (state int32, index int64, delta, workspace, cells: pinned int64 [2]) -> (counted, outside).  Waits for the two counts, which
+// the kernel writes to host memory: the caller needs them at once, and a copy of eight bytes behind a synchronisation takes
+// three times as long as looking for them.  Past a few milliseconds of looking (much work queued before this call) the thread waits
+// on the stream instead.
+PyObject* pool_update_refs(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  NEED_ARGS(5);
+  Args in(args);
+  const at::Tensor &state = in.gpu(1), &index = in.gpu(1);
+  const int64_t delta = in.integer();
+  const at::Tensor& ws = in.gpu(1);
+  const at::Tensor* cells = tensor(args[in.i]);
+  if (!in.ok || !is(index, at::kLong) || !index.is_contiguous() || !cells || !is(*cells, at::kLong) || cells->numel() != 2)
+    return PyErr_Format(PyExc_ValueError, "pool_update_refs: bad arguments");
+  volatile int64_t* c = (volatile int64_t*)cells->data_ptr();
+  c[0] = c[1] = -1;
+  const auto st = c10::hip::getCurrentHIPStream();
+  if (const int rc = lib.pool_update_refs((int32_t*)state.data_ptr(), state.size(0), index.numel() ? (const int64_t*)index.data_ptr() : nullptr,
+                                          index.numel(), (int)delta, (int64_t*)c, ws.data_ptr(), ws.nbytes(), st.stream()))
+    return failed(rc, "lsattn_pool_update_refs");
+  {
+    pybind11::gil_scoped_release no_gil;
+    const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(4);
+    while (c[0] < 0 || c[1] < 0) {
+      for (int i = 0; i < 64 && (c[0] < 0 || c[1] < 0); i++) __builtin_ia32_pause();
+      if (std::chrono::steady_clock::now() > until) {
+        st.synchronize();
+        break;
+      }
+    }
+  }
+  return Py_BuildValue("LL", (long long)c[0], (long long)c[1]);
+  END_HANDLE_TH_ERRORS
+}
+
 #define ENTRY(f) {#f, (PyCFunction)(void (*)(void))f, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     {"bind", bind, METH_O, "the library's entry points by name, as addresses"},
     ENTRY(context_attention), ENTRY(prefill_partial), ENTRY(token_decode_attention), ENTRY(decode_stage1), ENTRY(decode_stage2),
     ENTRY(kv_scatter), ENTRY(register_decode_tokens), ENTRY(register_tokens), ENTRY(rms_norm), ENTRY(silu_and_mul_inplace),
-    ENTRY(rotary_emb), ENTRY(rotary_kv_write),
+    ENTRY(rotary_emb), ENTRY(rotary_kv_write), ENTRY(pool_alloc), ENTRY(pool_update_refs),
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", "Native argument pass of loongserve_amd's operators.", -1, methods};
 

@@ -73,6 +73,23 @@ __device__ __forceinline__ float exp2_diff(float a, float b) {
   return (a == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(a - b);
 }
 
+// Division of 0 <= n < 2^31 by a launch constant d >= 1 without the divide sequence (some thirty instructions each, sixty
+// in 64 bits; a prefill workgroup's prologue needs ten): n / d = umulhi(n, mul) >> shr with mul = ceil(2^(31 + L) / d), shr = L - 1,
+// L = ceil(log2 d); d = 1 is mul = 0.
+struct FastDiv {
+  uint32_t mul, shr;
+};
+inline FastDiv fast_div(uint32_t d) {
+  if (d <= 1) return FastDiv{0, 0};
+  uint32_t L = 0;
+  while ((1u << L) < d) L++;
+  return FastDiv{(uint32_t)((((uint64_t)1 << (31 + L)) + d - 1) / d), L - 1};
+}
+__device__ __forceinline__ uint32_t div_by(uint32_t n, const FastDiv& f) { return f.mul ? __umulhi(n, f.mul) >> f.shr : n; }
+
+// Units of work a launch numbers with 31 bits; larger inputs go out in slices of whole tokens.
+constexpr int64_t kMaxUnits = 0x7fffff00;
+
 // The launch choices of lsattn_set_tuning (0 = the library's own); defined in merge_scatter.hip.
 struct Tuning {
   int prefill_rows, prefill_order, prefill_pack, decode_stage1, decode_listed;

@@ -6,13 +6,23 @@
 #include "common.hip.h"
 
 namespace lsattn {
-
+// Streams that are read and written back in place run with non-temporal accesses (NT) once they are larger than the caches:
+// a line that is read, kept in the L2 as dirty and evicted later costs HBM more than one that passes through (activation
+// of 16384 x 11008: 203 -> 177 us, 6.1 TB/s).  Out-of-place streams (the norm, the pool rows) lose by it.
+constexpr int64_t kStreamBytes = 64 << 20;
+template <bool NT, typename V> __device__ __forceinline__ V stream_load(const V* p) { return NT ? __builtin_nontemporal_load(p) : *p; }
+template <bool NT, typename V> __device__ __forceinline__ void stream_store(V* p, const V& v) {
+  if (NT) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
 // ---------------------------------------------------------------------------------------------------
 // rms_norm: out[t, i] = half(float(x[t, i]) * float(w[i]) * inv_rms[t]),  inv_rms = rsqrt(sum x^2 / H + eps),
-// the product in the reference's order (rms_norm.cu:42-45).  One wave per token row; a row of up to
-// 64 * 8 * kRmsChunks elements stays in registers between the two passes, longer rows are read twice.
+// the product in the reference's order (rms_norm.cu:42-45).  One workgroup per token row: a row of up to 8192 elements
+// stays in registers between the two passes (16 bytes of up to four places per lane), longer rows are read twice.  Bound by
+// HBM for many rows and by the chain of its loads for few; a wave per row had a quarter of the loads of a row in flight
+// beside each other: 16384 rows of 4096 49.1 -> 43.7 us (6.1 TB/s), 24 rows 4.9 -> 2.9 us.
 // ---------------------------------------------------------------------------------------------------
-constexpr int kRmsChunks = 16;  // 16-byte pieces per lane held in registers: rows up to 8192 elements
+constexpr int kRmsChunks = 4;  // 16-byte pieces per lane held in registers
 
 __device__ __forceinline__ float wave_sum(float v) {
   v = sum_row16(v);
@@ -22,40 +32,37 @@ __device__ __forceinline__ float wave_sum(float v) {
 }
 
 __global__ __launch_bounds__(256) void rms_norm_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ in,
-                                                       const uint16_t* __restrict__ weight, int64_t num_tokens, int64_t hidden,
-                                                       float eps) {
-  const int lane = threadIdx.x & 63;
-  const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (t >= num_tokens) return;
-  const int64_t pieces = hidden / 8;  // 16-byte pieces in a row
+                                                       const uint16_t* __restrict__ weight, int64_t hidden, float eps) {
+  const int64_t t = blockIdx.x;
+  const int pieces = (int)(hidden / 8);  // 16-byte pieces in a row
   const u32x4* row = (const u32x4*)(in + t * hidden);
   const u32x4* wrow = (const u32x4*)weight;
   u32x4* orow = (u32x4*)(out + t * hidden);
-  const bool cached = pieces <= 64 * kRmsChunks;
+  const bool cached = pieces <= 256 * kRmsChunks;
   u32x4 keep[kRmsChunks];
   float ss = 0.f;
+  auto add_squares = [&](const u32x4& x) {
+    float f[8];
+    unpack8<F16>(x, f);
+#pragma unroll
+    for (int e = 0; e < 8; e++) ss = __builtin_fmaf(f[e], f[e], ss);
+  };
   if (cached) {
 #pragma unroll
     for (int c = 0; c < kRmsChunks; c++) {
-      const int64_t i = lane + 64 * c;
+      const int i = threadIdx.x + 256 * c;
       keep[c] = i < pieces ? row[i] : u32x4{0, 0, 0, 0};
     }
 #pragma unroll
-    for (int c = 0; c < kRmsChunks; c++) {
-      float f[8];
-      unpack8<F16>(keep[c], f);
-#pragma unroll
-      for (int e = 0; e < 8; e++) ss = __builtin_fmaf(f[e], f[e], ss);
-    }
+    for (int c = 0; c < kRmsChunks; c++) add_squares(keep[c]);
   } else {
-    for (int64_t i = lane; i < pieces; i += 64) {
-      float f[8];
-      unpack8<F16>(row[i], f);
-#pragma unroll
-      for (int e = 0; e < 8; e++) ss = __builtin_fmaf(f[e], f[e], ss);
-    }
+    for (int i = threadIdx.x; i < pieces; i += 256) add_squares(row[i]);
   }
   ss = wave_sum(ss);
+  __shared__ float part[4];
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
+  __syncthreads();
+  ss = (part[0] + part[1]) + (part[2] + part[3]);
   const float inv_rms = __builtin_amdgcn_rsqf(ss / (float)hidden + eps);
   auto scale_piece = [&](const u32x4& x, const u32x4& w) {
     float a[8], b[8];
@@ -69,11 +76,11 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(uint16_t* __restrict__ ou
   if (cached) {
 #pragma unroll
     for (int c = 0; c < kRmsChunks; c++) {
-      const int64_t i = lane + 64 * c;
+      const int i = threadIdx.x + 256 * c;
       if (i < pieces) orow[i] = scale_piece(keep[c], wrow[i]);
     }
   } else {
-    for (int64_t i = lane; i < pieces; i += 64) orow[i] = scale_piece(row[i], wrow[i]);
+    for (int i = threadIdx.x; i < pieces; i += 256) orow[i] = scale_piece(row[i], wrow[i]);
   }
 }
 
@@ -81,16 +88,16 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(uint16_t* __restrict__ ou
 // silu_and_mul_inplace: io[t, i] = half(silu(io[t, i])) * io[t, I + i] for i < I, the second half of the row untouched;
 // silu in fp32, rounded to half, then a half multiply (silu_and_mul.cu:14-17, :30-33).
 // ---------------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void silu_and_mul_kernel(uint16_t* __restrict__ io, int64_t num_tokens, int64_t inter) {
-  const int64_t pieces_per_row = inter / 8;
-  const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (gid >= num_tokens * pieces_per_row) return;
-  const int64_t t = gid / pieces_per_row, i = gid % pieces_per_row;
+template <bool NT>
+__global__ __launch_bounds__(256) void silu_and_mul_kernel(uint16_t* __restrict__ io, uint32_t units, int64_t inter, FastDiv by_row) {
+  const uint32_t gid = blockIdx.x * 256 + threadIdx.x;
+  if (gid >= units) return;
+  const uint32_t t = div_by(gid, by_row), i = gid - t * (uint32_t)(inter / 8);
   // (whole rows of eight halves: picking 32-bit words out of an integer vector and bit-casting them to half
   // pairs made this compiler read word 0 every time)
-  f16x8* gate = (f16x8*)(io + t * 2 * inter) + i;
-  const f16x8 g = *gate;
-  const f16x8 u = *((const f16x8*)(io + t * 2 * inter + inter) + i);
+  f16x8* gate = (f16x8*)(io + (int64_t)t * 2 * inter) + i;
+  const f16x8 g = stream_load<NT>(gate);
+  const f16x8 u = stream_load<NT>((const f16x8*)(io + (int64_t)t * 2 * inter + inter) + i);
   f16x8 r;
 #pragma unroll
   for (int e = 0; e < 8; e++) {
@@ -98,7 +105,7 @@ __global__ __launch_bounds__(256) void silu_and_mul_kernel(uint16_t* __restrict_
     const _Float16 sl = (_Float16)(x / (1.f + __builtin_amdgcn_exp2f(-x * kLog2e)));
     r[e] = sl * u[e];  // half multiply, round to nearest even
   }
-  *gate = r;
+  stream_store<NT>(gate, r);
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -106,30 +113,18 @@ __global__ __launch_bounds__(256) void silu_and_mul_kernel(uint16_t* __restrict_
 //   new_x1 = fma(x1, cos, -(x2 * sin)),  new_x2 = fma(x1, sin, x2 * cos)   with x1 = x[..., :D/2], x2 = x[..., D/2:],
 // every product and fma rounded to half once.  A lane owns 8 elements of x1 and the matching 8 of x2.
 // ---------------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void rotary_emb_kernel(uint16_t* __restrict__ x, const uint16_t* __restrict__ cos_t,
-                                                         const uint16_t* __restrict__ sin_t, int64_t stride_t, int64_t stride_h,
-                                                         int64_t num_tokens, int64_t num_heads, int64_t head_dim) {
-  const int64_t pieces = head_dim / 16;  // 16-byte pieces in half a head
-  const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (gid >= num_tokens * num_heads * pieces) return;
-  const int64_t c = gid % pieces;
-  const int64_t h = (gid / pieces) % num_heads;
-  const int64_t t = gid / (pieces * num_heads);
-  uint16_t* base = x + t * stride_t + h * stride_h;
-  f16x8* p1 = (f16x8*)base + c;
-  f16x8* p2 = (f16x8*)(base + head_dim / 2) + c;
-  const f16x8 x1 = *p1, x2 = *p2;
-  const f16x8 co = *((const f16x8*)(cos_t + t * (head_dim / 2)) + c);
-  const f16x8 si = *((const f16x8*)(sin_t + t * (head_dim / 2)) + c);
+// The lane's 16 bytes of x1 and of x2 at p1 and p2, rotated in place; the rotated pieces in n1 and n2.
+template <bool NT>
+__device__ __forceinline__ void rotate_piece(f16x8* p1, f16x8* p2, const f16x8& co, const f16x8& si, f16x8& n1, f16x8& n2) {
+  const f16x8 x1 = stream_load<NT>(p1), x2 = stream_load<NT>(p2);
   const f16x8 t1 = x2 * si, t2 = x2 * co;  // rounded to half (this file is compiled without contraction)
-  f16x8 n1, n2;
 #pragma unroll
   for (int e = 0; e < 8; e++) {
     n1[e] = __builtin_fmaf16(x1[e], co[e], -t1[e]);
     n2[e] = __builtin_fmaf16(x1[e], si[e], t2[e]);
   }
-  *p1 = n1;
-  *p2 = n2;
+  stream_store<NT>(p1, n1);
+  stream_store<NT>(p2, n2);
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -141,54 +136,56 @@ __global__ __launch_bounds__(256) void rotary_emb_kernel(uint16_t* __restrict__ 
 // ---------------------------------------------------------------------------------------------------
 struct RotaryWriteParams {
   uint16_t* q;
-  int64_t q_st, q_sh, hq;
+  int64_t q_st, q_sh;
   uint16_t* kv;
-  int64_t kv_st, kv_sh, hkv;
+  int64_t kv_st, kv_sh;
   const uint16_t* cos_t;
   const uint16_t* sin_t;
-  int64_t num_tokens, head_dim;
   uint16_t* pool;
   int64_t pool_stride;  // elements per slot
-  const int32_t* dest;
+  const void* dest;     // int32 or int64 (dest_i64), of all tokens; this launch begins with token token0
+  int64_t token0;
   int32_t* req_to_tokens;
   int64_t max_seq_len;
   const int32_t* b_req_idx;
   const int32_t* b_start_loc;
   const int32_t* b_seq_len;
-  int64_t batch, data_blocks, reg_blocks_per_req;
+  int64_t batch;
+  uint32_t hq, hkv, head_dim, heads;  // heads: those of a token that are units of this launch (no V heads without a pool)
+  uint32_t units, data_blocks, reg_blocks_per_req;
+  FastDiv by_pieces, by_heads;
   int32_t reg_mode;  // 0 none, 1 every token of every request (prefill), 2 the last token of every request (decode)
+  int32_t dest_i64;
 };
 
-__global__ __launch_bounds__(256) void rotary_kv_write_kernel(RotaryWriteParams p) {
-  if ((int64_t)blockIdx.x >= p.data_blocks) {
-    const int64_t rb = (int64_t)blockIdx.x - p.data_blocks;
+template <bool NT> __global__ __launch_bounds__(256) void rotary_kv_write_kernel(RotaryWriteParams p) {
+  auto slot = [&](int64_t i) -> int64_t { return p.dest_i64 ? ((const int64_t*)p.dest)[i] : (int64_t)((const int32_t*)p.dest)[i]; };
+  if (blockIdx.x >= p.data_blocks) {
+    const uint32_t rb = blockIdx.x - p.data_blocks;
     if (p.reg_mode == 1) {
       const int64_t b = rb / p.reg_blocks_per_req;
-      const int64_t j = (rb % p.reg_blocks_per_req) * 256 + threadIdx.x;
+      const int64_t j = (int64_t)(rb % p.reg_blocks_per_req) * 256 + threadIdx.x;
       if (j >= p.b_seq_len[b] || j >= p.max_seq_len) return;
-      p.req_to_tokens[(int64_t)p.b_req_idx[b] * p.max_seq_len + j] = p.dest[(int64_t)p.b_start_loc[b] + j];
+      p.req_to_tokens[(int64_t)p.b_req_idx[b] * p.max_seq_len + j] = (int32_t)slot((int64_t)p.b_start_loc[b] + j);
     } else {
-      const int64_t i = rb * 256 + threadIdx.x;
+      const int64_t i = (int64_t)rb * 256 + threadIdx.x;
       if (i >= p.batch) return;
       const int64_t pos = (int64_t)p.b_seq_len[i] - 1;
       if (pos < 0 || pos >= p.max_seq_len) return;
-      p.req_to_tokens[(int64_t)p.b_req_idx[i] * p.max_seq_len + pos] = p.dest[i];
+      p.req_to_tokens[(int64_t)p.b_req_idx[i] * p.max_seq_len + pos] = (int32_t)slot(i);
     }
     return;
   }
-  const int64_t pieces = p.head_dim / 16;  // units per head
-  const int64_t heads = p.hq + 2 * p.hkv;
-  const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (gid >= p.num_tokens * heads * pieces) return;
-  const int64_t c = gid % pieces;
-  const int64_t h = (gid / pieces) % heads;
-  const int64_t t = gid / (pieces * heads);
+  const uint32_t gid = blockIdx.x * 256 + threadIdx.x;
+  if (gid >= p.units) return;
+  const uint32_t th = div_by(gid, p.by_pieces), c = gid - th * (p.head_dim / 16);  // unit of its head
+  const int64_t t = div_by(th, p.by_heads);
+  const uint32_t h = th - (uint32_t)t * p.heads;
   if (h >= p.hq + p.hkv) {
     // V head: 32 bytes to the pool
-    if (!p.pool) return;
-    const int64_t hv = h - p.hq;  // head index inside the token's K/V row
+    const uint32_t hv = h - p.hq;  // head index inside the token's K/V row
     const f16x8* src = (const f16x8*)(p.kv + t * p.kv_st + hv * p.kv_sh) + 2 * c;
-    f16x8* dst = (f16x8*)(p.pool + (int64_t)p.dest[t] * p.pool_stride + hv * p.head_dim) + 2 * c;
+    f16x8* dst = (f16x8*)(p.pool + slot(p.token0 + t) * p.pool_stride + (int64_t)hv * p.head_dim) + 2 * c;
     const f16x8 a = src[0], b = src[1];
     dst[0] = a;
     dst[1] = b;
@@ -196,22 +193,12 @@ __global__ __launch_bounds__(256) void rotary_kv_write_kernel(RotaryWriteParams 
   }
   const bool is_k = h >= p.hq;
   uint16_t* base = is_k ? p.kv + t * p.kv_st + (h - p.hq) * p.kv_sh : p.q + t * p.q_st + h * p.q_sh;
-  f16x8* p1 = (f16x8*)base + c;
-  f16x8* p2 = (f16x8*)(base + p.head_dim / 2) + c;
-  const f16x8 x1 = *p1, x2 = *p2;
   const f16x8 co = *((const f16x8*)(p.cos_t + t * (p.head_dim / 2)) + c);
   const f16x8 si = *((const f16x8*)(p.sin_t + t * (p.head_dim / 2)) + c);
-  const f16x8 t1 = x2 * si, t2 = x2 * co;  // rounded to half (this file is compiled without contraction)
   f16x8 n1, n2;
-#pragma unroll
-  for (int e = 0; e < 8; e++) {
-    n1[e] = __builtin_fmaf16(x1[e], co[e], -t1[e]);
-    n2[e] = __builtin_fmaf16(x1[e], si[e], t2[e]);
-  }
-  *p1 = n1;
-  *p2 = n2;
+  rotate_piece<NT>((f16x8*)base + c, (f16x8*)(base + p.head_dim / 2) + c, co, si, n1, n2);
   if (is_k && p.pool) {
-    uint16_t* prow = p.pool + (int64_t)p.dest[t] * p.pool_stride + (h - p.hq) * p.head_dim;
+    uint16_t* prow = p.pool + slot(p.token0 + t) * p.pool_stride + (int64_t)(h - p.hq) * p.head_dim;
     *((f16x8*)prow + c) = n1;
     *((f16x8*)(prow + p.head_dim / 2) + c) = n2;
   }
@@ -222,11 +209,12 @@ __global__ __launch_bounds__(256) void rotary_kv_write_kernel(RotaryWriteParams 
 // for the prefill kernel, whose P V product runs in fp16.  One 16-byte piece per lane.
 // ---------------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void bf16_to_f16_rows_kernel(const uint16_t* __restrict__ src, int64_t src_stride,
-                                                               uint16_t* __restrict__ dst, int64_t dst_stride, int64_t n_rows,
-                                                               int64_t pieces_per_row) {
-  const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (gid >= n_rows * pieces_per_row) return;
-  const int64_t r = gid / pieces_per_row, c = gid % pieces_per_row;
+                                                               uint16_t* __restrict__ dst, int64_t dst_stride, uint32_t pieces,
+                                                               uint32_t pieces_per_row, FastDiv by_row) {
+  const uint32_t gid = blockIdx.x * 256 + threadIdx.x;
+  if (gid >= pieces) return;
+  const int64_t r = div_by(gid, by_row);
+  const uint32_t c = gid - (uint32_t)r * pieces_per_row;
   const u32x4 w = *((const u32x4*)(src + r * src_stride) + c);
   u32x4 o;
 #pragma unroll
@@ -249,10 +237,14 @@ extern "C" int lsattn_bf16_to_f16_rows(const void* src, int64_t src_stride, void
       (((uintptr_t)src | (uintptr_t)dst) & 15))
     return LSATTN_ERR_INVALID_ARG;
   if (n_rows == 0) return LSATTN_OK;
-  const int64_t blocks = (n_rows * (row_elems / 8) + 255) / 256;
-  if (blocks > 0x7fffffff) return LSATTN_ERR_INVALID_ARG;
-  LSATTN_LAUNCH_KERNEL(bf16_to_f16_rows_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, (const uint16_t*)src,
-                     src_stride, (uint16_t*)dst, dst_stride, n_rows, row_elems / 8);
+  const int64_t per_row = row_elems / 8;
+  if (per_row > kMaxUnits) return LSATTN_ERR_INVALID_ARG;
+  for (int64_t r0 = 0, slice = kMaxUnits / per_row; r0 < n_rows; r0 += slice) {
+    const int64_t pieces = (n_rows - r0 < slice ? n_rows - r0 : slice) * per_row;
+    LSATTN_LAUNCH_KERNEL(bf16_to_f16_rows_kernel, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
+                       (const uint16_t*)src + r0 * src_stride, src_stride, (uint16_t*)dst + r0 * dst_stride, dst_stride,
+                       (uint32_t)pieces, (uint32_t)per_row, fast_div((uint32_t)per_row));
+  }
   return check_launch();
 }
 
@@ -261,10 +253,9 @@ extern "C" int lsattn_rms_norm(void* out, const void* in, const void* weight, in
   if (!out || !in || !weight || num_tokens < 0 || hidden_size <= 0) return LSATTN_ERR_INVALID_ARG;
   if (hidden_size % 8 || (((uintptr_t)out | (uintptr_t)in | (uintptr_t)weight) & 15)) return LSATTN_ERR_INVALID_ARG;
   if (num_tokens == 0) return LSATTN_OK;
-  const int64_t blocks = (num_tokens + 3) / 4;
-  if (blocks > 0x7fffffff) return LSATTN_ERR_INVALID_ARG;
-  LSATTN_LAUNCH_KERNEL(rms_norm_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, (uint16_t*)out,
-                     (const uint16_t*)in, (const uint16_t*)weight, num_tokens, hidden_size, eps);
+  if (num_tokens > 0x7fffffff || hidden_size > 0x7fffffff) return LSATTN_ERR_INVALID_ARG;
+  LSATTN_LAUNCH_KERNEL(rms_norm_kernel, dim3((unsigned)num_tokens), dim3(256), 0, (hipStream_t)stream, (uint16_t*)out,
+                     (const uint16_t*)in, (const uint16_t*)weight, hidden_size, eps);
   return check_launch();
 }
 
@@ -272,12 +263,58 @@ extern "C" int lsattn_silu_and_mul_inplace(void* io, int64_t num_tokens, int64_t
   if (!io || num_tokens < 0 || ffn_inter_dim <= 0) return LSATTN_ERR_INVALID_ARG;
   if (ffn_inter_dim % 8 || ((uintptr_t)io & 15)) return LSATTN_ERR_INVALID_ARG;
   if (num_tokens == 0) return LSATTN_OK;
-  const int64_t blocks = (num_tokens * (ffn_inter_dim / 8) + 255) / 256;
-  if (blocks > 0x7fffffff) return LSATTN_ERR_INVALID_ARG;
-  LSATTN_LAUNCH_KERNEL(silu_and_mul_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, (uint16_t*)io, num_tokens,
-                     ffn_inter_dim);
+  const int64_t per_row = ffn_inter_dim / 8;
+  if (per_row > kMaxUnits) return LSATTN_ERR_INVALID_ARG;
+  const bool nt = num_tokens * ffn_inter_dim * 4 >= kStreamBytes;
+  for (int64_t t0 = 0, slice = kMaxUnits / per_row; t0 < num_tokens; t0 += slice) {
+    const int64_t units = (num_tokens - t0 < slice ? num_tokens - t0 : slice) * per_row;
+    uint16_t* rows = (uint16_t*)io + t0 * 2 * ffn_inter_dim;
+    const dim3 grid((unsigned)((units + 255) / 256));
+    if (nt) LSATTN_LAUNCH_KERNEL(silu_and_mul_kernel<true>, grid, dim3(256), 0, (hipStream_t)stream, rows, (uint32_t)units, ffn_inter_dim, fast_div((uint32_t)per_row));
+    else LSATTN_LAUNCH_KERNEL(silu_and_mul_kernel<false>, grid, dim3(256), 0, (hipStream_t)stream, rows, (uint32_t)units, ffn_inter_dim, fast_div((uint32_t)per_row));
+  }
   return check_launch();
 }
+
+namespace lsattn {
+// Launches of rotary_kv_write_kernel over whole tokens, as many as have at most kMaxUnits units; the table is entered with the last one.
+static int launch_rotary(RotaryWriteParams p, int64_t num_tokens, int64_t max_len_in_batch, hipStream_t st) {
+  const int64_t per_token = (int64_t)p.heads * (p.head_dim / 16);
+  if (per_token > kMaxUnits) return LSATTN_ERR_INVALID_ARG;
+  int64_t reg_blocks = 0;
+  if (p.reg_mode == 1) {
+    p.reg_blocks_per_req = (uint32_t)((max_len_in_batch + 255) / 256);
+    reg_blocks = p.reg_blocks_per_req * p.batch;
+  } else if (p.reg_mode == 2) {
+    reg_blocks = (p.batch + 255) / 256;
+  }
+  if (reg_blocks > 0x40000000) return LSATTN_ERR_INVALID_ARG;
+  p.by_pieces = fast_div(p.head_dim / 16);
+  p.by_heads = fast_div(p.heads);
+  const bool nt = num_tokens * (int64_t)(p.hq + p.hkv) * p.head_dim * 2 >= kStreamBytes;
+  const int64_t slice = kMaxUnits / per_token;
+  for (int64_t t0 = 0;; t0 += slice) {
+    const bool last = num_tokens - t0 <= slice;
+    RotaryWriteParams s = p;
+    s.units = (uint32_t)((last ? num_tokens - t0 : slice) * per_token);
+    s.data_blocks = (s.units + 255) / 256;
+    s.q += t0 * p.q_st;
+    s.kv += t0 * p.kv_st;
+    s.cos_t += t0 * (p.head_dim / 2);
+    s.sin_t += t0 * (p.head_dim / 2);
+    if (!last) s.reg_mode = 0;
+    s.token0 = t0;
+    const int64_t blocks = s.data_blocks + (last ? reg_blocks : 0);
+    if (blocks > 0x7fffffff) return LSATTN_ERR_INVALID_ARG;
+    if (blocks > 0) {
+      if (nt) LSATTN_LAUNCH_KERNEL(rotary_kv_write_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, st, s);
+      else LSATTN_LAUNCH_KERNEL(rotary_kv_write_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, st, s);
+    }
+    if (last) break;
+  }
+  return check_launch();
+}
+}  // namespace lsattn
 
 extern "C" int lsattn_rotary_emb(void* x, const void* cos, const void* sin, int64_t x_stride_t, int64_t x_stride_h,
                                  int64_t num_tokens, int64_t num_heads, int64_t head_dim, void* stream) {
@@ -285,11 +322,16 @@ extern "C" int lsattn_rotary_emb(void* x, const void* cos, const void* sin, int6
   if (head_dim % 16 || x_stride_t % 8 || x_stride_h % 8 || (((uintptr_t)x | (uintptr_t)cos | (uintptr_t)sin) & 15))
     return LSATTN_ERR_INVALID_ARG;
   if (num_tokens == 0) return LSATTN_OK;
-  const int64_t blocks = (num_tokens * num_heads * (head_dim / 16) + 255) / 256;
-  if (blocks > 0x7fffffff) return LSATTN_ERR_INVALID_ARG;
-  LSATTN_LAUNCH_KERNEL(rotary_emb_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, (uint16_t*)x,
-                     (const uint16_t*)cos, (const uint16_t*)sin, x_stride_t, x_stride_h, num_tokens, num_heads, head_dim);
-  return check_launch();
+  if (num_heads > kMaxUnits || head_dim > kMaxUnits) return LSATTN_ERR_INVALID_ARG;
+  RotaryWriteParams p = {};
+  p.q = p.kv = (uint16_t*)x;
+  p.q_st = x_stride_t;
+  p.q_sh = x_stride_h;
+  p.cos_t = (const uint16_t*)cos;
+  p.sin_t = (const uint16_t*)sin;
+  p.hq = p.heads = (uint32_t)num_heads;
+  p.head_dim = (uint32_t)head_dim;
+  return launch_rotary(p, num_tokens, 0, (hipStream_t)stream);
 }
 
 extern "C" int lsattn_rotary_kv_write(const lsattn_rotary_kv_write_args* a, void* stream) {
@@ -306,22 +348,26 @@ extern "C" int lsattn_rotary_kv_write(const lsattn_rotary_kv_write_args* a, void
       (!a->req_to_tokens || !a->dest_index || !a->b_req_idx || !a->b_seq_len || a->max_seq_len <= 0 ||
        (a->register_mode == 1 && (!a->b_start_loc || a->max_len_in_batch < 0 || a->max_len_in_batch > a->max_seq_len))))
     return LSATTN_ERR_INVALID_ARG;
-  RotaryWriteParams p;
+  if (a->dest_index_is_i64 != 0 && a->dest_index_is_i64 != 1) return LSATTN_ERR_INVALID_ARG;
+  const int64_t heads = a->num_q_heads + (a->pool ? 2 : 1) * a->num_kv_heads;
+  if (heads > kMaxUnits || a->head_dim > kMaxUnits) return LSATTN_ERR_INVALID_ARG;
+  RotaryWriteParams p = {};
   p.q = (uint16_t*)a->q;
   p.q_st = a->q_stride_t;
   p.q_sh = a->q_stride_h;
-  p.hq = a->num_q_heads;
+  p.hq = (uint32_t)a->num_q_heads;
   p.kv = (uint16_t*)a->kv;
   p.kv_st = a->kv_stride_t;
   p.kv_sh = a->kv_stride_h;
-  p.hkv = a->num_kv_heads;
+  p.hkv = (uint32_t)a->num_kv_heads;
+  p.heads = (uint32_t)heads;
   p.cos_t = (const uint16_t*)a->cos;
   p.sin_t = (const uint16_t*)a->sin;
-  p.num_tokens = a->num_tokens;
-  p.head_dim = a->head_dim;
+  p.head_dim = (uint32_t)a->head_dim;
   p.pool = (uint16_t*)a->pool;
   p.pool_stride = a->pool_slot_stride;
   p.dest = a->dest_index;
+  p.dest_i64 = a->dest_index_is_i64;
   p.req_to_tokens = a->req_to_tokens;
   p.max_seq_len = a->max_seq_len;
   p.b_req_idx = a->b_req_idx;
@@ -329,19 +375,5 @@ extern "C" int lsattn_rotary_kv_write(const lsattn_rotary_kv_write_args* a, void
   p.b_seq_len = a->b_seq_len;
   p.batch = a->batch;
   p.reg_mode = a->register_mode;
-  const int64_t units = a->num_tokens * (a->num_q_heads + 2 * a->num_kv_heads) * (a->head_dim / 16);
-  p.data_blocks = (units + 255) / 256;
-  p.reg_blocks_per_req = 0;
-  int64_t reg_blocks = 0;
-  if (a->register_mode == 1) {
-    p.reg_blocks_per_req = (a->max_len_in_batch + 255) / 256;
-    reg_blocks = p.reg_blocks_per_req * a->batch;
-  } else if (a->register_mode == 2) {
-    reg_blocks = (a->batch + 255) / 256;
-  }
-  const int64_t blocks = p.data_blocks + reg_blocks;
-  if (blocks == 0) return LSATTN_OK;
-  if (blocks > 0x7fffffff) return LSATTN_ERR_INVALID_ARG;
-  LSATTN_LAUNCH_KERNEL(rotary_kv_write_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, p);
-  return check_launch();
+  return launch_rotary(p, a->num_tokens, a->max_len_in_batch, (hipStream_t)stream);
 }

@@ -143,14 +143,15 @@ template <typename OT, int MODE> __global__ __launch_bounds__(256) void merge_cu
 }
 
 // dst[dest_index[i]] = src[i]; 16 bytes per lane, consecutive lanes cover one row
+template <typename IT>
 __global__ __launch_bounds__(256) void kv_scatter_kernel(const char* __restrict__ src, int64_t src_stride,
                                                          char* __restrict__ dst, int64_t dst_stride,
-                                                         const int32_t* __restrict__ dest_index, int64_t n_rows,
-                                                         int32_t chunks_per_row) {
-  const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t row = gid / chunks_per_row;
-  const int c = (int)(gid % chunks_per_row);
-  if (row >= n_rows) return;
+                                                         const IT* __restrict__ dest_index, uint32_t pieces, uint32_t chunks_per_row,
+                                                         FastDiv by_row) {
+  const uint32_t gid = blockIdx.x * 256 + threadIdx.x;
+  if (gid >= pieces) return;
+  const int64_t row = div_by(gid, by_row);
+  const uint32_t c = gid - (uint32_t)row * chunks_per_row;
   const u32x4 w = *(const u32x4*)(src + row * src_stride + (int64_t)c * 16);
   *(u32x4*)(dst + (int64_t)dest_index[row] * dst_stride + (int64_t)c * 16) = w;
 }
@@ -393,18 +394,29 @@ extern "C" int lsattn_prefill_merge_cuts(const lsattn_merge_cuts_args* a, void* 
   return check_launch();
 }
 
-extern "C" int lsattn_kv_scatter(const void* src, int64_t src_stride_bytes, void* dst, int64_t dst_stride_bytes,
-                                 const int32_t* dest_index, int64_t n_rows, int64_t row_bytes, void* stream) {
+template <typename IT>
+static int kv_scatter(const void* src, int64_t src_stride_bytes, void* dst, int64_t dst_stride_bytes, const IT* dest_index,
+                      int64_t n_rows, int64_t row_bytes, hipStream_t st) {
   if (!src || !dst || !dest_index || n_rows < 0 || row_bytes <= 0) return LSATTN_ERR_INVALID_ARG;
   if (row_bytes % 16 || src_stride_bytes % 16 || dst_stride_bytes % 16 || (((uintptr_t)src | (uintptr_t)dst) & 15))
     return LSATTN_ERR_INVALID_ARG;
-  if (n_rows == 0) return LSATTN_OK;
   const int64_t cpr = row_bytes / 16;
-  const int64_t blocks = (n_rows * cpr + 255) / 256;
-  if (blocks > 0x7fffffff || cpr > 0x7fffffff) return LSATTN_ERR_INVALID_ARG;
-  LSATTN_LAUNCH_KERNEL(kv_scatter_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, (const char*)src,
-                     src_stride_bytes, (char*)dst, dst_stride_bytes, dest_index, n_rows, (int32_t)cpr);
-  return check_launch();
+  if (cpr > kMaxUnits) return LSATTN_ERR_INVALID_ARG;
+  for (int64_t r0 = 0, slice = kMaxUnits / cpr; r0 < n_rows; r0 += slice) {
+    const int64_t pieces = (n_rows - r0 < slice ? n_rows - r0 : slice) * cpr;
+    LSATTN_LAUNCH_KERNEL(kv_scatter_kernel<IT>, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, st,
+                       (const char*)src + r0 * src_stride_bytes, src_stride_bytes, (char*)dst, dst_stride_bytes, dest_index + r0,
+                       (uint32_t)pieces, (uint32_t)cpr, fast_div((uint32_t)cpr));
+  }
+  return n_rows > 0 ? check_launch() : LSATTN_OK;
+}
+extern "C" int lsattn_kv_scatter(const void* src, int64_t src_stride_bytes, void* dst, int64_t dst_stride_bytes,
+                                 const int32_t* dest_index, int64_t n_rows, int64_t row_bytes, void* stream) {
+  return kv_scatter(src, src_stride_bytes, dst, dst_stride_bytes, dest_index, n_rows, row_bytes, (hipStream_t)stream);
+}
+extern "C" int lsattn_kv_scatter_i64(const void* src, int64_t src_stride_bytes, void* dst, int64_t dst_stride_bytes,
+                                     const int64_t* dest_index, int64_t n_rows, int64_t row_bytes, void* stream) {
+  return kv_scatter(src, src_stride_bytes, dst, dst_stride_bytes, dest_index, n_rows, row_bytes, (hipStream_t)stream);
 }
 
 extern "C" int lsattn_register_tokens(int32_t* req_to_tokens, int64_t max_seq_len, const int32_t* b_req_idx,

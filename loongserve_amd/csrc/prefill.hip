@@ -41,20 +41,6 @@
 
 namespace lsattn {
 
-// Division of 0 <= n < 2^31 by a launch constant d >= 1 without the divide sequence (some thirty instructions each, and
-// the prologue of a workgroup needs ten): n / d = umulhi(n, mul) >> shr with mul = ceil(2^(31 + L) / d), shr = L - 1,
-// L = ceil(log2 d); d = 1 is mul = 0.
-struct FastDiv {
-  uint32_t mul, shr;
-};
-static FastDiv fast_div(uint32_t d) {
-  if (d <= 1) return FastDiv{0, 0};
-  uint32_t L = 0;
-  while ((1u << L) < d) L++;
-  return FastDiv{(uint32_t)((((uint64_t)1 << (31 + L)) + d - 1) / d), L - 1};
-}
-__device__ __forceinline__ uint32_t div_by(uint32_t n, const FastDiv& f) { return f.mul ? __umulhi(n, f.mul) >> f.shr : n; }
-
 struct PrefillParams {
   const void* q;
   const void* k;

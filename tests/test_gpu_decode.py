@@ -645,3 +645,28 @@ def test_random_decode_shapes_on_both_stage1_kernels(lsa, tuning, seed):
             assert torch.equal(torch.isnan(ml_d.cpu()), untouched), "rows written, " + what
             assert_o_close(o_d, o_ref, "o, " + what)
             assert_lse_close(l_d, l_ref, "lse, " + what)
+
+
+@pytest.mark.parametrize("Hq,Hkv,B", [(32, 8, 64), (32, 8, 65), (4, 4, 8), (24, 3, 130), (5, 5, 9)])
+def test_equal_shares_at_the_edges_of_their_launches(lsa, tuning, Hq, Hkv, B):
+    """Shares forced on batches that are counted in registers (up to 64 requests) and in LDS, merged with one wave and with four
+    per (request, head) (up to 1024 pairs), heads that do not fill the merge's groups of four: lengths around the unit of 32
+    tokens, empty requests first and last, one request that holds most of the tokens."""
+    import random
+    rng = random.Random(B)
+    tuning(decode_listed="shares")
+    lens = [rng.choice([0, 1, 31, 32, 33, 64, 127, 128, 129, 300]) for _ in range(B)]
+    lens[0] = lens[-1] = 0
+    lens[B // 2] = 5000
+    D = 128
+    q, kv, table, b_req, b_len = decode_case(300 + B, B, Hq, Hkv, D, lens, sum(lens) + 100, torch.float16)
+    o_ref, l_ref = orc.decode_full(q, kv[:, :Hkv], kv[:, Hkv:], table, b_req, b_len)
+    kvd = kv.to(DEV)
+    nblk = (max(lens) + 255) // 256
+    mo_d = torch.full((nblk, B, Hq, D), float("nan"), device=DEV)
+    ml_d = torch.full((nblk, B, Hq), float("nan"), device=DEV)
+    o_d, l_d = lsa.longserve_token_decode_attention_flash_decoding(q.to(DEV), table.to(DEV), b_req.to(DEV), b_len.to(DEV), mo_d, ml_d, B,
+                                                                   max(lens), Hq, D, kvd[:, :Hkv], kvd[:, Hkv:], 256)
+    torch.cuda.synchronize()
+    assert_o_close(o_d, o_ref, "o")
+    assert_lse_close(l_d, l_ref, "lse")

@@ -165,3 +165,43 @@ def test_argument_checks(lsa):
         k.silu_and_mul_inplace(torch.zeros(2, 8, dtype=torch.float16))  # CPU tensor
     with pytest.raises(RuntimeError):
         k.rms_norm(torch.zeros(2, 12, dtype=torch.float16, device=DEV), torch.zeros(12, dtype=torch.float16, device=DEV), 1e-5)  # 12 % 8 != 0
+
+
+@pytest.mark.parametrize("T", [1, 9, 3000])
+def test_int64_slots_go_to_the_kernels_as_they_are(lsa, T):
+    """The scatter and the fused write-back with the slots as the allocator hands them out against the same with int32 slots,
+    with and without the non-temporal route of large streams (3000 tokens of 64 + 16 heads: 61 MB and more)."""
+    g = torch.Generator(device=DEV).manual_seed(T)
+    Hq, Hkv, D = 96, 8, 128
+    q, kv = (torch.randn((T, h, D), generator=g, device=DEV).half() for h in (Hq, 2 * Hkv))
+    cos, sin = (torch.randn((T, D // 2), generator=g, device=DEV).half() for _ in range(2))
+    slots = torch.randperm(2 * T, generator=g, device=DEV)[:T]
+    table = [torch.zeros((T, 5), dtype=torch.int32, device=DEV) for _ in range(2)]
+    req, length = torch.arange(T, dtype=torch.int32, device=DEV), torch.full((T,), 3, dtype=torch.int32, device=DEV)
+    pools = [torch.zeros((2 * T, 2 * Hkv, D), dtype=torch.float16, device=DEV) for _ in range(2)]
+    qs, kvs = [q.clone(), q.clone()], [kv.clone(), kv.clone()]
+    for i, s in enumerate((slots, slots.int())):
+        lsa.rotary_emb_write_kv(qs[i], kvs[i], cos, sin, s, pools[i], table[i], req, length, decode=True)
+    assert torch.equal(qs[0], qs[1]) and torch.equal(kvs[0], kvs[1]) and torch.equal(pools[0], pools[1]) and torch.equal(table[0], table[1])
+    assert torch.equal(table[0][:, 2], slots.int()) and torch.equal(pools[0][slots], kvs[0])
+    qc, kc = q[:9].cpu().numpy().copy(), kv[:9, :Hkv].cpu().numpy().copy()
+    for x in (qc, kc):
+        ew.rotary_emb(x, cos[:9].cpu().numpy(), sin[:9].cpu().numpy())
+    assert torch.equal(qs[0][:9].cpu(), torch.from_numpy(qc)) and torch.equal(kvs[0][:9, :Hkv].cpu(), torch.from_numpy(kc))
+    pool = torch.zeros_like(pools[0])
+    lsa.destindex_copy_kv(kv, slots, pool)
+    assert torch.equal(pool[slots], kv) and int((pool != 0).any(-1).any(-1).sum()) == T
+
+
+@pytest.mark.parametrize("T,I", [(1600, 11008), (3, 11008)])
+def test_silu_and_mul_on_both_sides_of_the_streaming_rule(lsa, T, I):
+    """From 64 MB on the activation runs with non-temporal accesses: the same halves either way."""
+    g = torch.Generator(device=DEV).manual_seed(T)
+    io = torch.randn((T, 2 * I), generator=g, device=DEV).half()
+    want = io[-3:].cpu().numpy().copy()
+    ew.silu_and_mul_inplace(want)
+    up = io[:, I:].clone()
+    lsa.longserve_cuda_kernels.silu_and_mul_inplace(io)
+    torch.cuda.synchronize()
+    assert torch.equal(io[:, I:], up)
+    assert _ulp(io[-3:].cpu().numpy(), want).max() <= 2
