@@ -4,7 +4,8 @@
 //   find the first run of `need` consecutive free slots           (alloc_contiguous, :50-55)
 //   add / drop one reference on a list of slots and count          (add_refs :73-79, decrease_refs :82-88)
 // `mem_state` is int32 per slot, 0 = free.  All of it is integer work on a few MB, bound by launch latency and
-// by one pass over the state array; three short launches replace the reference's nonzero / slice / compare chains.
+// by one pass over the state array; two short launches replace the reference's nonzero / slice / compare chains (three for
+// pools of more than 8 million slots), one for the reference counts of up to 4096 slots.
 #include "common.hip.h"
 
 namespace lsattn {
@@ -61,7 +62,9 @@ __device__ __forceinline__ int64_t wave_incl_max(int64_t v) {
 // ---------------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(kPoolThreads) void pool_summarise_kernel(const int32_t* __restrict__ state, int64_t size,
                                                                       int32_t* __restrict__ blk_free,
-                                                                      int64_t* __restrict__ blk_last_used) {
+                                                                      int64_t* __restrict__ blk_last_used,
+                                                                      int64_t* __restrict__ first_fit) {
+  if (first_fit && blockIdx.x == 0 && threadIdx.x == 0) *first_fit = -1;  // "no run", until pass 3 finds one
   __shared__ int sh_cnt[kPoolWaves];
   __shared__ int64_t sh_last[kPoolWaves];
   PoolTile t;
@@ -99,17 +102,16 @@ __global__ __launch_bounds__(kPoolThreads) void pool_summarise_kernel(const int3
 }
 
 // ---------------------------------------------------------------------------------------------------
-// Pass 2 (one workgroup): exclusive prefix sum of the free counts and exclusive prefix maximum of the last-used
-// positions over the workgroups of pass 1.  cells[0] = total free; *first_fit (when given) is preset to -1 = "no run".
-// When fewer than `need` slots are free, out_index[total .. need) is filled with -1 so the result is defined.
+// Pass 2 (one workgroup), for pools of more than kPoolDirectBlocks workgroups of pass 1: exclusive prefix sum of their
+// free counts and exclusive prefix maximum of their last-used positions.  Smaller pools do without it: there each workgroup of
+// pass 3 adds up the summaries in front of it itself (at most eight per thread, from the L2), which costs less than
+// a launch: alloc of 64 slots of 2.5 million 10 -> 6 us on the device.
 // ---------------------------------------------------------------------------------------------------
+constexpr int64_t kPoolDirectBlocks = 2048;
 __global__ __launch_bounds__(1024) void pool_scan_summaries_kernel(const int32_t* __restrict__ blk_free,
                                                                    const int64_t* __restrict__ blk_last_used, int64_t nb,
                                                                    int64_t* __restrict__ free_before,
-                                                                   int64_t* __restrict__ last_used_before,
-                                                                   int64_t* __restrict__ cells, int64_t need,
-                                                                   int64_t* __restrict__ out_index,
-                                                                   int64_t* __restrict__ first_fit) {
+                                                                   int64_t* __restrict__ last_used_before) {
   __shared__ int64_t sh_sum[1024];
   __shared__ int64_t sh_max[1024];
   const int64_t per = (nb + 1023) / 1024;
@@ -142,27 +144,49 @@ __global__ __launch_bounds__(1024) void pool_scan_summaries_kernel(const int32_t
     run_sum += blk_free[b];
     run_max = blk_last_used[b] > run_max ? blk_last_used[b] : run_max;
   }
-  const int64_t total = sh_sum[1023];
-  if (threadIdx.x == 0) {
-    cells[0] = total;
-    if (first_fit) *first_fit = -1;
+}
+
+// The sum of blk_free (MAX: the maximum of blk_last_used) over the workgroups in front of this one, by all its threads.
+template <bool MAX>
+__device__ __forceinline__ int64_t pool_before(const int32_t* __restrict__ blk_free, const int64_t* __restrict__ blk_last_used) {
+  __shared__ int64_t sh[kPoolWaves];
+  int64_t v = MAX ? -1 : 0;
+  for (int64_t b = threadIdx.x; b < blockIdx.x; b += kPoolThreads) {
+    if (MAX) v = blk_last_used[b] > v ? blk_last_used[b] : v;
+    else v += blk_free[b];
   }
-  if (out_index)
-    for (int64_t i = total + threadIdx.x; i < need; i += 1024) out_index[i] = -1;
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) {
+    const int64_t o = __shfl_xor(v, d);
+    v = MAX ? (o > v ? o : v) : v + o;
+  }
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+  __syncthreads();
+  v = sh[0];
+#pragma unroll
+  for (int w = 1; w < kPoolWaves; w++) v = MAX ? (sh[w] > v ? sh[w] : v) : v + sh[w];
+  return v;
 }
 
 // ---------------------------------------------------------------------------------------------------
 // Pass 3 of alloc: the free slot with rank r < need (ranks count free slots in ascending slot order) is written to
-// out_index[r] and marked in use.  Workgroups whose first rank is already >= need leave at once.
+// out_index[r] and marked in use.  Workgroups whose first rank is already >= need leave at once.  When fewer than `need` slots
+// are free, the last workgroup fills the rest of out_index with -1, so the result is defined.
 // ---------------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(kPoolThreads) void pool_take_kernel(int32_t* __restrict__ state, int64_t size,
-                                                                 const int64_t* __restrict__ free_before, int64_t need,
-                                                                 int64_t* __restrict__ out_index) {
+                                                                 const int64_t* __restrict__ free_before,
+                                                                 const int32_t* __restrict__ blk_free, int64_t need,
+                                                                 int64_t* __restrict__ out_index, int64_t* __restrict__ cells) {
   __shared__ int sh[kPoolPieces][kPoolWaves];
-  const int64_t first_rank = free_before[blockIdx.x];
-  if (first_rank >= need) return;
   PoolTile t;
-  t.load(state, size);
+  t.load(state, size);  // (asked for beside the summaries)
+  const int64_t first_rank = free_before ? free_before[blockIdx.x] : pool_before<false>(blk_free, nullptr);
+  if (blockIdx.x == gridDim.x - 1) {
+    const int64_t total = first_rank + blk_free[blockIdx.x];
+    if (threadIdx.x == 0) cells[0] = total;
+    for (int64_t i = total + threadIdx.x; i < need; i += kPoolThreads) out_index[i] = -1;
+  }
+  if (first_rank >= need) return;
   const int wave = threadIdx.x >> 6;
   int incl[kPoolPieces], mine[kPoolPieces];
 #pragma unroll
@@ -211,10 +235,12 @@ __global__ __launch_bounds__(kPoolThreads) void pool_take_kernel(int32_t* __rest
 // ---------------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(kPoolThreads) void pool_first_fit_kernel(const int32_t* __restrict__ state, int64_t size,
                                                                       const int64_t* __restrict__ last_used_before,
+                                                                      const int64_t* __restrict__ blk_last_used,
                                                                       int64_t need, int64_t* __restrict__ first_fit) {
   __shared__ int64_t sh[kPoolPieces][kPoolWaves];
   PoolTile t;
   t.load(state, size);
+  const int64_t u_before = last_used_before ? last_used_before[blockIdx.x] : pool_before<true>(nullptr, blk_last_used);
   const int wave = threadIdx.x >> 6;
   int64_t own[kPoolPieces], incl[kPoolPieces];
 #pragma unroll
@@ -230,7 +256,7 @@ __global__ __launch_bounds__(kPoolThreads) void pool_first_fit_kernel(const int3
   int64_t best = INT64_MAX;
 #pragma unroll
   for (int j = 0; j < kPoolPieces; j++) {
-    int64_t u = last_used_before[blockIdx.x];
+    int64_t u = u_before;
     for (int jj = 0; jj < kPoolPieces; jj++)
       for (int w = 0; w < kPoolWaves; w++)
         if (jj < j || (jj == j && w < wave)) u = sh[jj][w] > u ? sh[jj][w] : u;
@@ -256,6 +282,64 @@ __global__ __launch_bounds__(kPoolThreads) void pool_first_fit_kernel(const int3
 // (-1: used_tokens, :85) the update; counted[1] = entries outside the pool (skipped).  Negative entries wrap
 // once, as in torch indexing.
 // ---------------------------------------------------------------------------------------------------
+// The counts may be asked for in pinned host memory, where the caller looks for them while the kernel ends: whole words, written
+// through to the system.
+__device__ __forceinline__ void put_counts(int64_t* counted, int64_t used, int64_t bad) {
+  __hip_atomic_store(counted, used, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(counted + 1, bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Up to kRefsOneGroup entries by one workgroup: every old value is in a register before the barrier, every new one is
+// written behind it.  (bound by its three dependent loads and a store: 3 us, where the two launches below take 4 and a gap)
+constexpr int kRefsPer = 4;
+constexpr int64_t kRefsOneGroup = 1024 * kRefsPer;
+__global__ __launch_bounds__(1024) void pool_refs_small_kernel(int32_t* __restrict__ state, int64_t size,
+                                                               const int64_t* __restrict__ index, int64_t n, int delta,
+                                                               int64_t* __restrict__ counted) {
+  __shared__ int sh[2][16];
+  int64_t slot[kRefsPer];
+  int32_t old[kRefsPer];
+#pragma unroll
+  for (int k = 0; k < kRefsPer; k++) {
+    const int64_t i = threadIdx.x + 1024 * k;
+    slot[k] = i < n ? index[i] : 0;
+  }
+  int used = 0, bad = 0;
+#pragma unroll
+  for (int k = 0; k < kRefsPer; k++) {
+    const bool listed = threadIdx.x + 1024 * k < n;
+    if (slot[k] < 0) slot[k] += size;
+    const bool inside = slot[k] >= 0 && slot[k] < size;
+    bad += listed && !inside;
+    if (!listed || !inside) slot[k] = -1;
+    old[k] = slot[k] >= 0 ? state[slot[k]] : 0;
+  }
+#pragma unroll
+  for (int k = 0; k < kRefsPer; k++) used += slot[k] >= 0 && (delta > 0 ? old[k] : old[k] + delta) != 0;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < kRefsPer; k++)
+    if (slot[k] >= 0) state[slot[k]] = old[k] + delta;
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) {
+    used += __shfl_xor(used, d);
+    bad += __shfl_xor(bad, d);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    sh[0][threadIdx.x >> 6] = used;
+    sh[1][threadIdx.x >> 6] = bad;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    used = bad = 0;
+    for (int w = 0; w < 16; w++) {
+      used += sh[0][w];
+      bad += sh[1][w];
+    }
+    put_counts(counted, used, bad);
+  }
+}
+
 __global__ __launch_bounds__(256) void pool_refs_gather_kernel(const int32_t* __restrict__ state, int64_t size,
                                                                const int64_t* __restrict__ index, int64_t n, int delta,
                                                                int32_t* __restrict__ old_state, int64_t* __restrict__ blk_counts) {
@@ -318,13 +402,12 @@ __global__ __launch_bounds__(256) void pool_refs_apply_kernel(int32_t* __restric
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-      counted[0] = sh[0][0] + sh[0][1] + sh[0][2] + sh[0][3];
-      counted[1] = sh[1][0] + sh[1][1] + sh[1][2] + sh[1][3];
+      put_counts(counted, sh[0][0] + sh[0][1] + sh[0][2] + sh[0][3], sh[1][0] + sh[1][1] + sh[1][2] + sh[1][3]);
     }
   }
 }
 
-// Workspace layout of the searches: int64 cells[2] (cells[0] = free slots in the pool at the time of the call) | int64 free_before[nb] | int64 last_used_before[nb] |
+// Workspace layout of the searches: int64 cells[2] (cells[0] = free slots in the pool at the time of an alloc) | int64 free_before[nb] | int64 last_used_before[nb] |
 // int64 blk_last_used[nb] | int32 blk_free[nb]
 struct PoolWorkspace {
   int64_t nb;
@@ -363,6 +446,16 @@ static int pool_search_checks(const void* mem_state, int64_t size, int64_t need,
   return LSATTN_OK;
 }
 
+// Passes 1 and, for a large pool, 2; true if pass 2 has run.
+static bool pool_summarise(const PoolWorkspace& w, const int32_t* mem_state, int64_t pool_size, int64_t* first_fit, hipStream_t st) {
+  LSATTN_LAUNCH_KERNEL(pool_summarise_kernel, dim3((unsigned)w.nb), dim3(kPoolThreads), 0, st, mem_state, pool_size, w.blk_free,
+                     w.blk_last_used, first_fit);
+  if (w.nb <= kPoolDirectBlocks) return false;
+  LSATTN_LAUNCH_KERNEL(pool_scan_summaries_kernel, dim3(1), dim3(1024), 0, st, w.blk_free, w.blk_last_used, w.nb, w.free_before,
+                     w.last_used_before);
+  return true;
+}
+
 extern "C" int lsattn_pool_alloc(int32_t* mem_state, int64_t pool_size, int64_t need, int64_t* out_index, void* workspace,
                                  size_t workspace_bytes, void* stream) {
   const int rc = pool_search_checks(mem_state, pool_size, need, workspace, workspace_bytes);
@@ -370,13 +463,9 @@ extern "C" int lsattn_pool_alloc(int32_t* mem_state, int64_t pool_size, int64_t 
   if (need > 0 && !out_index) return LSATTN_ERR_INVALID_ARG;
   hipStream_t st = (hipStream_t)stream;
   const PoolWorkspace w = pool_carve(workspace, pool_size);
-  LSATTN_LAUNCH_KERNEL(pool_summarise_kernel, dim3((unsigned)w.nb), dim3(kPoolThreads), 0, st, mem_state, pool_size, w.blk_free,
-                     w.blk_last_used);
-  LSATTN_LAUNCH_KERNEL(pool_scan_summaries_kernel, dim3(1), dim3(1024), 0, st, w.blk_free, w.blk_last_used, w.nb, w.free_before,
-                     w.last_used_before, w.cells, need, out_index, (int64_t*)nullptr);
-  if (need > 0)
-    LSATTN_LAUNCH_KERNEL(pool_take_kernel, dim3((unsigned)w.nb), dim3(kPoolThreads), 0, st, mem_state, pool_size, w.free_before,
-                       need, out_index);
+  const bool scan = pool_summarise(w, mem_state, pool_size, nullptr, st);
+  LSATTN_LAUNCH_KERNEL(pool_take_kernel, dim3((unsigned)w.nb), dim3(kPoolThreads), 0, st, mem_state, pool_size,
+                     scan ? w.free_before : nullptr, w.blk_free, need, out_index, w.cells);
   return check_launch();
 }
 
@@ -387,12 +476,9 @@ extern "C" int lsattn_pool_find_contiguous(const int32_t* mem_state, int64_t poo
   if (!out_start || need <= 0) return LSATTN_ERR_INVALID_ARG;
   hipStream_t st = (hipStream_t)stream;
   const PoolWorkspace w = pool_carve(workspace, pool_size);
-  LSATTN_LAUNCH_KERNEL(pool_summarise_kernel, dim3((unsigned)w.nb), dim3(kPoolThreads), 0, st, mem_state, pool_size, w.blk_free,
-                     w.blk_last_used);
-  LSATTN_LAUNCH_KERNEL(pool_scan_summaries_kernel, dim3(1), dim3(1024), 0, st, w.blk_free, w.blk_last_used, w.nb, w.free_before,
-                     w.last_used_before, w.cells, (int64_t)0, (int64_t*)nullptr, out_start);
+  const bool scan = pool_summarise(w, mem_state, pool_size, out_start, st);
   LSATTN_LAUNCH_KERNEL(pool_first_fit_kernel, dim3((unsigned)w.nb), dim3(kPoolThreads), 0, st, mem_state, pool_size,
-                     w.last_used_before, need, out_start);
+                     scan ? w.last_used_before : nullptr, w.blk_last_used, need, out_start);
   return check_launch();
 }
 
@@ -407,11 +493,13 @@ extern "C" int lsattn_pool_update_refs(int32_t* mem_state, int64_t pool_size, co
   hipStream_t st = (hipStream_t)stream;
   int64_t* blk_counts = (int64_t*)workspace;
   int32_t* old_state = (int32_t*)(blk_counts + 2 * nblk);
-  if (n > 0)
-    LSATTN_LAUNCH_KERNEL(pool_refs_gather_kernel, dim3((unsigned)nblk), dim3(256), 0, st, mem_state, pool_size, index, n, delta,
-                       old_state, blk_counts);
-  // with n == 0 one workgroup still runs, to write counted = {0, 0}
-  LSATTN_LAUNCH_KERNEL(pool_refs_apply_kernel, dim3((unsigned)(nblk > 0 ? nblk : 1)), dim3(256), 0, st, mem_state, pool_size, index,
+  if (n <= kRefsOneGroup) {  // (n = 0 too: counted = {0, 0})
+    LSATTN_LAUNCH_KERNEL(pool_refs_small_kernel, dim3(1), dim3(1024), 0, st, mem_state, pool_size, index, n, delta, counted);
+    return check_launch();
+  }
+  LSATTN_LAUNCH_KERNEL(pool_refs_gather_kernel, dim3((unsigned)nblk), dim3(256), 0, st, mem_state, pool_size, index, n, delta,
+                     old_state, blk_counts);
+  LSATTN_LAUNCH_KERNEL(pool_refs_apply_kernel, dim3((unsigned)nblk), dim3(256), 0, st, mem_state, pool_size, index,
                      n, delta, old_state, blk_counts, nblk, counted);
   return check_launch();
 }

@@ -206,3 +206,36 @@ def test_request_manager_and_int64_slots_in_the_kv_operators(lsa):
     assert rm.can_use_req_size == 8 and mm.can_use_mem_size == 4096
     mm.resize_mem(100)
     assert mm.mem_state.numel() == 100 and mm.kv_buffer.shape[1] == 100 and mm.alloc(100).cpu().tolist() == list(range(100))
+
+
+@pytest.mark.parametrize("n", [0, 1, 1023, 1024, 1025, 4096, 4097])
+def test_reference_counts_at_the_edges_of_the_one_launch_kernel(lsa, n):
+    """Up to 4096 entries are counted by one workgroup (four per thread), more by two launches: entries listed twice,
+    slots that fall to zero, negative entries that wrap."""
+    rng = np.random.default_rng(n)
+    size = 6000
+    m, o = _pair(lsa, rng.integers(0, 3, size).astype(np.int32))
+    index = rng.integers(0, size, n).astype(np.int64)
+    index[1::7] = index[0] if n else 0
+    m.add_refs(torch.from_numpy(index).to(DEV))
+    o.add_refs(index)
+    _same(m, o)
+    index[2::5] -= size
+    m.decrease_refs(torch.from_numpy(index).to(DEV))
+    o.decrease_refs(index)
+    _same(m, o)
+
+
+def test_alloc_and_first_fit_in_a_pool_that_takes_the_scan_launch(lsa):
+    """More than 2048 workgroups of 4096 slots: the summaries are scanned by a launch of their own."""
+    size = 2049 * 4096 + 77
+    state = torch.ones(size, dtype=torch.int32)
+    free = [3, 4095, 4096, 1024 * 4096 + 5, size - 78, size - 2, size - 1]
+    state[free] = 0
+    m = _manager(lsa, size)
+    m.mem_state.copy_(state)
+    m.can_use_mem_size = len(free)
+    got = m.alloc_contiguous(2)
+    assert got is not None and got[1:] == (4095, 4097)
+    assert m.alloc(5).cpu().tolist() == [3, 1024 * 4096 + 5, size - 78, size - 2, size - 1]
+    assert int((m.mem_state == 0).sum()) == 0 and m.can_use_mem_size == 0
