@@ -1,18 +1,23 @@
 // The prefill attention step for head sizes 16, 32 and 64 (the reference's Triton kernel takes them beside 128:
 // loongserve/models/llama/triton_kernel/ring_context_flashattention_nopad.py:248-250), gfx950, wave64.
 //
-// Same arithmetic as the 128-wide kernel of prefill.hip in a plain form: no LLaMA-family model the reference serves has
-// such heads, so this kernel is built to be exact and free of hidden copies, not tuned tile by tile.
-//   * a workgroup of eight waves owns 128 consecutive query positions of one query head, a wave 16 of them; K and V
-//     tiles of 64 keys are staged through LDS by all threads (global -> registers -> LDS, the next tile requested
-//     before the present one is worked on; bfloat16 V converted to fp16 on the way), one barrier per tile;
+// What bounds it is vector work: a 32 x 32 block of scores takes a wave 16 exponentials, 16 multiply-adds, 16 additions and
+// some 15 conversions and checks against 16 (D = 64) to 6 (D = 16) MFMAs, and the time falls only a third from D = 64 to 16.
+// Hence no work beside those in the common path, and four waves per SIMD whose phases mix freely:
+//   * a workgroup of four waves; a wave owns 32 (small launches: 16) query positions of one head.  With grouped-query
+//     heads up to four heads of a KV head sit side by side in a workgroup, which then ends sooner on the diagonal;
+//   * K and V tiles of 64 keys go to LDS by direct loads, two stages, one barrier per tile, chunks XOR-swizzled (bfloat16 V
+//     passes through registers and becomes fp16 there);
 //   * scores transposed, S^T = K Q^T with v_mfma_f32_16x16x32 (a head of 16 fills half of the contraction with
-//     zeros), 32 keys per step, so a lane owns one query column: running max and sum are in-lane work plus an exchange
-//     between the four lanes of a column, and the fp32 scores turn into the B operand of O^T += V^T P^T in place (P and
-//     V as fp16, as in the 128-wide kernel); V^T operands through ds_read_b64_tr_b16; a wave skips the steps none of
-//     its rows sees;
+//     zeros), 32 keys per step, so a lane owns one query column: the fp32 scores turn into the B operand of O^T += V^T P^T in
+//     place (P and V as fp16, sums of P in fp32), V^T operands through ds_read_b64_tr_b16; a wave skips the steps none of its
+//     rows sees;
+//   * the running maximum of a row is raised only when a P of 2 or more shows up; no exchange between lanes otherwise;
 //   * the three epilogues of the 128-wide kernel: 0 the step's fp32 partial (O, LSE), 1 the reference's in-place
 //     (o, m, l) update (ring_context_flashattention_nopad.py:171-188), 2 the LSE merge into a running fp32 (O, LSE).
+// Against 16 positions per wave, eight waves, tiles staged through registers and the maximum exchanged in every step
+// (fp16, causal): D = 64, 8 x 2048 tokens GQA 32/8 380 -> 183 us (0.75 PFLOP/s), 1 x 8192 MHA 640 -> 310, 16 x 512 73 -> 47,
+// 1 x 100 7.4 -> 6.0; D = 32, 8 x 2048 283 -> 135; D = 16 278 -> 121.
 #include <type_traits>
 
 #include "common.hip.h"
@@ -76,7 +81,10 @@ struct SmallParams {
   const int32_t* kv_len;
   const int32_t* kv_first;
   const int32_t* o_start;
-  int32_t hq, heads_per_kv, peers, v_f16;
+  int32_t hq, hkv, heads_per_kv, peers;
+  int32_t group, pack_shift;  // groups of 1 << pack_shift heads side by side per KV head
+  int32_t last_tile;          // of query positions, the first one of the launch
+  FastDiv d_hkv, d_peers;
   float scale_log2;
   void* o;
   int64_t o_st, o_sh;
@@ -86,51 +94,78 @@ struct SmallParams {
   int64_t ml_st, ml_sh;
 };
 
-constexpr int kWaves = 8;   // waves per workgroup
-constexpr int kQB = 1;      // blocks of 16 query positions per wave: 128 positions of one head per workgroup (two blocks,
-                            // which share every K and V operand read, measured no faster: the waves wait on their own chains of
-                            // dependent steps, and there are half as many of them to fill the gaps)
-constexpr int kRows = kWaves * kQB * 16;
+constexpr int kWaves = 4;   // waves per workgroup
 constexpr int kTile = 64;   // keys per LDS tile
+constexpr uint32_t kOnes = 0x3C003C00u;  // two ones in fp16
+constexpr int64_t kCUs = 256;
+constexpr int64_t kMaxTiles = 65535;  // tiles of one launch (the third index of a grid)
 
-template <typename T, int D, int MODE>
-__global__ __launch_bounds__(kWaves * 64) void prefill_small_kernel(SmallParams p) {
+// s_waitcnt vmcnt(0) (expcnt / lgkmcnt fields left at their maximum)
+__device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+
+// 16 bytes per lane from tile + off into LDS at dst (wave-uniform) + 16 * lane.  From inline assembly, or the compiler would
+// wait for the load before every later LDS read; the s_nop is the wait state between a write of m0 and its use.
+__device__ __forceinline__ void load_to_lds(int dst, const char* tile, uint32_t off) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(tile) : "m0", "memory");
+}
+__device__ __forceinline__ const char* uniform_ptr(const char* ptr) {
+  const uint64_t u = (uint64_t)ptr;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)u), hi = __builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
+  return (const char*)(((uint64_t)hi << 32) | lo);
+}
+
+// DV: the V tiles are fp16 in memory and go straight into LDS as the K tiles do; otherwise (bfloat16 V) they pass through
+// registers and are converted on the way.  QB: blocks of 16 query positions per wave.
+template <typename T, int D, int MODE, bool DV, int QB>
+__global__ __launch_bounds__(kWaves * 64, QB == 2 && D == 64 && !DV ? 3 : 4) void prefill_small_kernel(SmallParams p) {
   constexpr int KS = D >= 32 ? D / 32 : 1;  // contraction steps of Q K^T (32 elements each; D = 16 fills half of one)
   constexpr int NDB = D / 16;               // 16-wide blocks of the head
   constexpr int CPR = D / 8;                // 16-byte chunks per K or V row
-  constexpr int NCH = kTile * CPR;          // chunks per tile: at most one per thread (512 for D = 64)
-  constexpr int RB = D * 2 + 16;            // bytes per row in LDS (padded: neighbouring rows start in different banks)
+  constexpr int RB = D * 2;                 // bytes per row in LDS
   constexpr int TB = kTile * RB;            // bytes per tile
-  static_assert(NCH <= kWaves * 64, "one chunk per thread and tile");
-  // two stages of (K tile, V tile): the next tile is written while the present one is read
-  __shared__ __attribute__((aligned(16))) char lds[2 * 2 * TB];
+  constexpr int RPI = 64 / CPR;             // rows per load instruction (a wave's 64 lanes, 16 bytes each)
+  constexpr int NI = (kTile + kWaves * RPI - 1) / (kWaves * RPI);  // load instructions per wave and tile: two for D = 64, else one
+  constexpr int RPB = 256 / RB;             // rows that pass all 64 LDS banks once
+  // two stages of (K tile, V tile): the next tile is written while the present one is read.  Rows are not padded (a load to
+  // LDS writes 1 KB in a row); instead the 16-byte chunks of a row are XORed with a function of the row: K so that a
+  // column of chunks of sixteen rows, which one read takes, lies in sixteen different sets of four banks, V so that 32 bytes of
+  // each of eight rows (half a transposing read) cover the banks once.  Rows sixteen apart share their XOR.
+  __shared__ __attribute__((aligned(1024))) char lds[2 * 2 * TB];
+  auto swz_k = [](int row) { return (row / RPB) & (CPR - 1); };
+  auto swz_v = [](int row) { return ((row / RPB) & (CPR / 2 - 1)) << 1; };
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
-  const int b = blockIdx.z, h = blockIdx.y;
+  // grid: (KV head, heads side by side), request, tile from the last one down: the heaviest tiles of all requests start
+  // first, and with a multiple of eight KV heads the workgroups of one run on one XCD (ids are dealt round-robin)
+  const int gq = (int)div_by(blockIdx.x, p.d_hkv), kvh = (int)blockIdx.x - gq * p.hkv;
+  const int b = blockIdx.y;
+  const int rows_wg = (kWaves * QB * 16) >> p.pack_shift;  // query positions of this workgroup
+  const int m_wg = (p.last_tile - (int)blockIdx.z) * rows_wg;
   const int q_len = p.q_len[b];
-  const int m_wg = (int)blockIdx.x * kRows;
   if (m_wg >= q_len) return;  // (the whole workgroup: the loop below holds barriers)
-  const int m0 = m_wg + wave * (kQB * 16);  // the wave's first position
+  const int wph_shift = 2 - p.pack_shift;  // log2 of the waves per head
+  const int h = kvh * p.heads_per_kv + (gq << p.pack_shift) + (wave >> wph_shift);
+  const int m0 = m_wg + (wave & ((1 << wph_shift) - 1)) * (QB * 16);  // the wave's first position
   const int kv_len = p.kv_len[b], qf = p.q_first[b], kf = p.kv_first[b], P = p.peers;
   const int64_t q_start = p.q_start[b], kv_start = p.kv_start[b];
   const int64_t o_start = p.o_start ? (int64_t)p.o_start[b] : q_start;
-  const int kvh = h / p.heads_per_kv;
 
   // keys of this KV chunk visible to global query position qpos (ring_context_flashattention_nopad.py:156-159)
   auto visible_keys = [&](int qpos) -> int {
     const int dq = qpos - kf;
-    const int n = dq >= 0 ? dq / P + 1 : 0;
+    const int n = dq >= 0 ? (int)div_by((uint32_t)dq, p.d_peers) + 1 : 0;
     return n > kv_len ? kv_len : n;
   };
   // per block qb of 16 positions: the lane's position m0 + 16 qb + c, whether it exists, the keys it sees
-  bool in_range[kQB];
-  int cnt[kQB];
-  u32x4 qreg[kQB][KS];  // Q^T as B operands: qreg[qb][ks] = Q[position][32 ks + 8 g .. + 7]
-  f32x4 oacc[kQB][NDB]; // O^T: oacc[qb][db][j] = O[position][16 db + 4 g + j]
-  float m_run[kQB], l_run[kQB];  // log2-domain running max of the column; the lane's share of its running sum
+  bool in_range[QB];
+  int cnt[QB];
+  u32x4 qreg[QB][KS];  // Q^T as B operands: qreg[qb][ks] = Q[position][32 ks + 8 g .. + 7]
+  f32x4 oacc[QB][NDB]; // O^T: oacc[qb][db][j] = O[position][16 db + 4 g + j]
+  float m_run[QB], l_run[QB];  // log2-domain running max of the column; the lane's share of its running sum
+  f32x4 l_pv[QB];  // the column's sum of the fp16 values that multiply V (all four elements)
 #pragma unroll
-  for (int qb = 0; qb < kQB; qb++) {
+  for (int qb = 0; qb < QB; qb++) {
     const int m = m0 + 16 * qb + c;
     in_range[qb] = m < q_len;
     cnt[qb] = in_range[qb] ? visible_keys(qf + m * P) : 0;
@@ -144,126 +179,196 @@ __global__ __launch_bounds__(kWaves * 64) void prefill_small_kernel(SmallParams 
     for (int db = 0; db < NDB; db++) oacc[qb][db] = f32x4{0.f, 0.f, 0.f, 0.f};
     m_run[qb] = -INFINITY;
     l_run[qb] = 0.f;
+    l_pv[qb] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   // (positions ascend: a later row sees at least as many keys)
   auto last_seen = [&](int first, int rows) -> int {  // keys the last existing position of [first, first + rows) sees; 0 if none exists
     return first < q_len ? visible_keys(qf + (first + rows - 1 < q_len ? first + rows - 1 : q_len - 1) * P) : 0;
   };
-  const int cnt_wave = last_seen(m0, kQB * 16);
-  const int cnt_first = m0 < q_len ? visible_keys(qf + m0 * P) : 0;
-  const int cnt_wg = last_seen(m_wg, kRows);
+  const int cnt_wave = __builtin_amdgcn_readfirstlane(last_seen(m0, QB * 16));
+  // (rows past the end see nothing: a wave that holds some masks everywhere only where it has to, in their own columns,
+  // which nothing reads; its first row sees the fewest keys of the others)
+  const int cnt_first = __builtin_amdgcn_readfirstlane(m0 < q_len ? visible_keys(qf + m0 * P) : 0);
+  const int cnt_wg = __builtin_amdgcn_readfirstlane(last_seen(m_wg, rows_wg));
 
   const char* kbase = (const char*)p.k + (kv_start * p.k_st + (int64_t)kvh * p.k_sh) * 2;
   const char* vbase = (const char*)p.v + (kv_start * p.v_st + (int64_t)kvh * p.v_sh) * 2;
-  const int last_key = kv_len - 1;
-  // staging: thread `tid` carries chunk `tid` of the K tile and of the V tile (row tid / CPR, 16 bytes at 8 (tid % CPR))
-  const bool stager = tid < NCH;
-  const int st_row = tid / CPR, st_cc = tid % CPR;
-  const int st_at = st_row * RB + st_cc * 16;
-  u32x4 kst = {0u, 0u, 0u, 0u}, vst = {0u, 0u, 0u, 0u};
-  auto request = [&](int t) __attribute__((always_inline)) {
-    if (stager) {
-      const int key = t * kTile + st_row < last_key ? t * kTile + st_row : last_key;  // (rows past the end repeat the last one and are masked)
-      kst = *(const u32x4*)(kbase + ((int64_t)key * p.k_st + 8 * st_cc) * 2);
-      vst = *(const u32x4*)(vbase + ((int64_t)key * p.v_st + 8 * st_cc) * 2);
+  // staging: instruction i of a wave carries rows (wave + 4 i) * RPI .. of the K tile and of the V tile.  Tiles that lie inside the
+  // chunk take a scalar tile address and the lane's 32-bit offset, no vector arithmetic.
+  const bool stager = NI * kWaves * RPI == kTile || wave * RPI < kTile;  // (D = 16: two waves)
+  const int st_row = wave * RPI + lane / CPR;
+  const uint32_t k_row = (uint32_t)p.k_st * 2, v_row = (uint32_t)p.v_st * 2;  // (a tile's rows span less than 2^31 bytes)
+  const uint32_t k_off = st_row * k_row + ((lane % CPR) ^ swz_k(st_row)) * 16, v_off = st_row * v_row + ((lane % CPR) ^ swz_v(st_row)) * 16;
+  const int lds_base = (int)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+  u32x4 vst[NI];
+  auto request = [&](int stage, int t) __attribute__((always_inline)) {
+    if (!stager) return;
+    const char* kt = uniform_ptr(kbase + (int64_t)t * kTile * k_row);
+    const char* vt = uniform_ptr(vbase + (int64_t)t * kTile * v_row);
+    const int dst = __builtin_amdgcn_readfirstlane(lds_base + stage * 2 * TB + wave * 1024);
+    const int last = kv_len - 1 - t * kTile;
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+      constexpr int STEP = kWaves * RPI;
+      uint32_t ko = k_off, vo = v_off;
+      if (last < kTile - 1) {  // (wave-uniform; rows past the end repeat the last one and are masked)
+        int r0 = st_row;
+        asm volatile("" : "+v"(r0));  // (worked out here and not kept in registers over the loop)
+        int back = r0 + i * STEP - last;
+        back = back < 0 ? 0 : back;
+        ko -= (uint32_t)back * k_row;
+        vo -= (uint32_t)back * v_row;
+      }
+      load_to_lds(dst + i * kWaves * 1024, kt, ko + (uint32_t)(i * STEP) * k_row);
+      if (DV) load_to_lds(dst + TB + i * kWaves * 1024, vt, vo + (uint32_t)(i * STEP) * v_row);
+      else vst[i] = *(const u32x4*)(vt + (vo + (uint32_t)(i * STEP) * v_row));
     }
   };
+  // the tile that was requested, complete in LDS for this wave
   auto deposit = [&](int stage) __attribute__((always_inline)) {
-    if (stager) {
-      *(u32x4*)(lds + stage * 2 * TB + st_at) = kst;
-      *(u32x4*)(lds + stage * 2 * TB + TB + st_at) = (std::is_same<T, BF16>::value && !p.v_f16) ? bf16_to_f16(vst) : vst;
+    if (!DV && stager) {
+#pragma unroll
+      for (int i = 0; i < NI; i++) *(u32x4*)(lds + stage * 2 * TB + TB + (wave + i * kWaves) * 1024 + lane * 16) = bf16_to_f16(vst[i]);
     }
+    wait_loads();
   };
   // transposing read: lane c of a 16-lane group points at row c >> 2, columns 4 (c & 3) .. + 3 of a 4 x 16 block and
   // receives column c of it; group g takes rows 4 g .. 4 g + 3 and, sixteen rows on, 16 + 4 g .. + 3: the eight keys
   // whose scores the lane holds
-  const int vread0 = (4 * g + (c >> 2)) * RB + 4 * (c & 3) * 2;
-  const int kread0 = c * RB + 8 * g * 2;
-
-  const int nt = (cnt_wg + kTile - 1) / kTile;  // the same for every wave of the workgroup
-  if (nt > 0) {
-    request(0);
-    deposit(0);
-    __syncthreads();
+  int kaddr[KS], vaddr[NDB];
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++) kaddr[ks] = lds_base + c * RB + (((4 * ks + g) & (CPR - 1)) ^ swz_k(c)) * 16;
+#pragma unroll
+  for (int db = 0; db < NDB; db++) {
+    const int row = 4 * g + (c >> 2);
+    vaddr[db] = lds_base + TB + row * RB + ((2 * db + ((c & 3) >> 1)) ^ swz_v(row)) * 16 + (c & 1) * 8;
   }
-  for (int t = 0; t < nt; t++) {
-    if (t + 1 < nt) request(t + 1);
-    const char* kl = lds + (t & 1) * 2 * TB;
-    const char* vl = kl + TB;
+  const float scale = p.scale_log2;
+  const int nt = (cnt_wg + kTile - 1) / kTile;  // the same for every wave of the workgroup
+
+  u32x4 ka[2][KS];  // K operands of the next 32 keys
+  auto load_ka = [&](int at) __attribute__((always_inline)) {
+#pragma unroll
+    for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) {
+        ka[kb][ks] = *(const __attribute__((address_space(3))) u32x4*)(kaddr[ks] + at + kb * 16 * RB);
+        if (D == 16 && g >= 2) ka[kb][ks] = u32x4{0u, 0u, 0u, 0u};
+      }
+  };
+  auto tile = [&](auto stage_tag, int t) __attribute__((always_inline)) {
+    constexpr int S = decltype(stage_tag)::value;
+    if (t + 1 < nt) request(S ^ 1, t + 1);
+    if (t * kTile < cnt_wave) load_ka(S * 2 * TB);
 #pragma unroll
     for (int half = 0; half < 2; half++) {
       const int k0 = t * kTile + 32 * half;
-      if (k0 >= cnt_wave) continue;  // (wave-uniform: none of the wave's rows sees these keys)
-      // S^T = K Q^T: s[qb][kb][j] = score of key k0 + 16 kb + 4 g + j for the lane's query of block qb; a K operand
-      // serves both blocks
-      f32x4 s[kQB][2];
+      if (k0 < cnt_wave) {  // (wave-uniform: else none of the wave's rows sees these keys)
+        // S^T = K Q^T: s[qb][kb][j] = score of key k0 + 16 kb + 4 g + j for the lane's query of block qb; a K operand
+        // serves all blocks
+        f32x4 s[QB][2];
 #pragma unroll
-      for (int kb = 0; kb < 2; kb++) {
-#pragma unroll
-        for (int qb = 0; qb < kQB; qb++) s[qb][kb] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-          const int d0 = 32 * ks + 8 * g;
-          const u32x4 ka = d0 < D ? *(const u32x4*)(kl + (32 * half + 16 * kb) * RB + kread0 + 64 * ks) : u32x4{0u, 0u, 0u, 0u};
-#pragma unroll
-          for (int qb = 0; qb < kQB; qb++) s[qb][kb] = MfmaS<T>::run(ka, qreg[qb][ks], s[qb][kb]);
-        }
-      }
-      u32x4 pk[kQB];  // P^T as B operands: the lane's eight keys are contraction slots 8 g .. 8 g + 7, the order the V^T operand uses
-#pragma unroll
-      for (int qb = 0; qb < kQB; qb++) {
-        if (k0 + 32 > cnt_first) {  // (wave-uniform: the wave's first row, which sees the fewest keys, does not see the whole step)
+        for (int ks = 0; ks < KS; ks++)
 #pragma unroll
           for (int kb = 0; kb < 2; kb++)
 #pragma unroll
-            for (int j = 0; j < 4; j++) s[qb][kb][j] = k0 + 16 * kb + 4 * g + j < cnt[qb] ? s[qb][kb][j] : -INFINITY;
-        }
-        const float mx = fmaxf(fmaxf(fmaxf(s[qb][0][0], s[qb][0][1]), fmaxf(s[qb][0][2], s[qb][0][3])),
-                               fmaxf(fmaxf(s[qb][1][0], s[qb][1][1]), fmaxf(s[qb][1][2], s[qb][1][3])));
-        const float m_new = fmaxf(m_run[qb], col_max(mx) * p.scale_log2);  // (the scale is positive)
-        if (__builtin_amdgcn_ballot_w64(m_new != m_run[qb]) != 0) {
-          const float alpha = exp2_diff(m_run[qb], m_new);
-          l_run[qb] *= alpha;
+            for (int qb = 0; qb < QB; qb++) s[qb][kb] = MfmaS<T>::run(ka[kb][ks], qreg[qb][ks], ks == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : s[qb][kb]);
+        if (k0 + 32 > cnt_first) {  // (wave-uniform: the wave's first row, which sees the fewest keys, does not see the whole step)
 #pragma unroll
-          for (int db = 0; db < NDB; db++) oacc[qb][db] *= alpha;
-          m_run[qb] = m_new;
-        }
-        const float neg_m = m_run[qb] == -INFINITY ? 0.f : -m_run[qb];  // (a row that has seen no key yet: every P below is 0)
-        float pv[8], ps = 0.f;
+          for (int qb = 0; qb < QB; qb++) {
+            const int rel = cnt[qb] - k0 - 4 * g;
 #pragma unroll
-        for (int kb = 0; kb < 2; kb++)
+            for (int kb = 0; kb < 2; kb++)
 #pragma unroll
-          for (int j = 0; j < 4; j++) {
-            pv[4 * kb + j] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[qb][kb][j], p.scale_log2, neg_m));
-            ps += pv[4 * kb + j];
+              for (int j = 0; j < 4; j++) s[qb][kb][j] = 16 * kb + j < rel ? s[qb][kb][j] : -INFINITY;
           }
-        l_run[qb] += ps;
+        }
+        // P = exp2(S * scale - m) with the running maxima as they are; they are raised, and the step done again, only if some
+        // P comes out as 2 or more (or as inf or NaN, as for a row that has seen no key yet: m = -inf), which is bit 14 of
+        // its fp16 form.  No exchange between lanes, no chain through the maximum in the common case.
+        u32x4 pk[QB];  // P^T as B operands: the lane's eight keys are contraction slots 8 g .. 8 g + 7, the order the V^T operand uses
+        float ps[QB];
+        auto compute_p = [&](int qb, float neg_m) __attribute__((always_inline)) {
+          float pv[8];
 #pragma unroll
-        for (int e = 0; e < 4; e++) pk[qb][e] = pack2<F16>(pv[2 * e], pv[2 * e + 1]);
-      }
+          for (int e = 0; e < 8; e++) pv[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[qb][e / 4][e % 4], scale, neg_m));
+          ps[qb] = ((pv[0] + pv[1]) + (pv[2] + pv[3])) + ((pv[4] + pv[5]) + (pv[6] + pv[7]));
 #pragma unroll
-      for (int db = 0; db < NDB; db++) {
-        const int at = (int)(uintptr_t)(const __attribute__((address_space(3))) char*)vl + 32 * half * RB + vread0 + db * 32;
-        const i16x4 xa = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_ptr)at);
-        const i16x4 xb = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_ptr)(at + 16 * RB));
-        const u32x2 wa = __builtin_bit_cast(u32x2, xa), wb = __builtin_bit_cast(u32x2, xb);
-        const u32x4 va = u32x4{wa[0], wa[1], wb[0], wb[1]};
+          for (int e = 0; e < 4; e++) pk[qb][e] = pack2<F16>(pv[2 * e], pv[2 * e + 1]);
+        };
+        uint32_t any = 0;
 #pragma unroll
-        for (int qb = 0; qb < kQB; qb++) oacc[qb][db] = MfmaS<F16>::run(va, pk[qb], oacc[qb][db]);
+        for (int qb = 0; qb < QB; qb++) {
+          compute_p(qb, -m_run[qb]);
+          any |= (pk[qb][0] | pk[qb][1]) | (pk[qb][2] | pk[qb][3]);
+        }
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64((any & 0x40004000u) != 0) != 0, 0)) {
+#pragma unroll
+          for (int qb = 0; qb < QB; qb++) {
+            const float mx = fmaxf(fmaxf(fmaxf(s[qb][0][0], s[qb][0][1]), fmaxf(s[qb][0][2], s[qb][0][3])),
+                                   fmaxf(fmaxf(s[qb][1][0], s[qb][1][1]), fmaxf(s[qb][1][2], s[qb][1][3])));
+            const float m_new = fmaxf(m_run[qb], col_max(mx) * scale);  // (the scale is positive)
+            const float alpha = exp2_diff(m_run[qb], m_new);
+            l_run[qb] *= alpha;
+            l_pv[qb] *= alpha;
+#pragma unroll
+            for (int db = 0; db < NDB; db++) oacc[qb][db] *= alpha;
+            m_run[qb] = m_new;
+            compute_p(qb, m_new == -INFINITY ? 0.f : -m_new);  // (a row that has seen no key: every P is 0)
+          }
+        }
+#pragma unroll
+        for (int qb = 0; qb < QB; qb++) l_run[qb] += ps[qb];
+        // (the scores' registers are free now and take the next K operands; asked for any earlier, these or the V operands
+        // below spill: 64-wide heads, 8 x 2048 tokens, 217 us instead of 168 (without l_pv) with the V operands read before the softmax)
+        __builtin_amdgcn_sched_barrier(0);
+        u32x4 va[NDB];
+#pragma unroll
+        for (int db = 0; db < NDB; db++) {
+          const int at = vaddr[db] + S * 2 * TB + 32 * half * RB;
+          const i16x4 xa = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_ptr)at);
+          const i16x4 xb = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_ptr)(at + 16 * RB));
+          const u32x2 wa = __builtin_bit_cast(u32x2, xa), wb = __builtin_bit_cast(u32x2, xb);
+          va[db] = u32x4{wa[0], wa[1], wb[0], wb[1]};
+        }
+        if (half == 0) load_ka(S * 2 * TB + 32 * RB);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int db = 0; db < NDB; db++)
+#pragma unroll
+          for (int qb = 0; qb < QB; qb++) oacc[qb][db] = MfmaS<F16>::run(va[db], pk[qb], oacc[qb][db]);
+#pragma unroll
+        for (int qb = 0; qb < QB; qb++) l_pv[qb] = MfmaS<F16>::run(u32x4{kOnes, kOnes, kOnes, kOnes}, pk[qb], l_pv[qb]);
       }
     }
-    // the next tile into the other stage (last read one barrier ago), then everyone meets: that tile is complete and
-    // this one is done with
-    if (t + 1 < nt) deposit((t + 1) & 1);
+    // the next tile is in the other stage (last read one barrier ago), then everyone meets: that tile is complete and this
+    // one is done with
+    if (t + 1 < nt) deposit(S ^ 1);
     __syncthreads();
+  };
+  if (nt > 0) {
+    request(0, 0);
+    deposit(0);
+    __syncthreads();
+  }
+  for (int t = 0; t < nt; t += 2) {  // (the stage is a constant of the code)
+    tile(std::integral_constant<int, 0>{}, t);
+    if (t + 1 < nt) tile(std::integral_constant<int, 1>{}, t + 1);
   }
 
   // ---- epilogues (the 128-wide kernel's), block by block of 16 positions ----
 #pragma unroll
-  for (int qb = 0; qb < kQB; qb++) {
+  for (int qb = 0; qb < QB; qb++) {
     const int mb = m0 + 16 * qb;
     if (mb >= q_len) break;  // (wave-uniform: a block without positions; it only helped to stage)
     const float l_tot = col_sum(l_run[qb]);
+    // O becomes a mean with the very weights it was summed with: a rounding that a row's weights share (one key that outweighs
+    // the others) falls out of it, which makes up for maxima that lag (a P of 1 is exact in fp16, one of 1.4 is not).
+    // Against 64 bits the fp32 partial of N(0, 1) * 0.5 inputs is off by 1.70e-4 to 1.72e-4 at 1000 to 3000 tokens of 64-wide heads,
+    // 1.74e-4 to 1.75e-4 with maxima that never lag and 1.76e-4 with neither.  The sum that (m, l) and the LSE state stays the fp32 one.
+    const float fix = l_pv[qb][0] > 0.f ? l_tot / l_pv[qb][0] : 0.f;
+#pragma unroll
+    for (int db = 0; db < NDB; db++) oacc[qb][db] *= fix;
     const bool here = in_range[qb];
     const int64_t tok = o_start + (here ? mb + c : mb);
     if (MODE == 0) {
@@ -333,28 +438,46 @@ __global__ __launch_bounds__(kWaves * 64) void prefill_small_kernel(SmallParams 
   }
 }
 
-template <typename T, int D, int MODE> int launch(const SmallParams& p, const lsattn_prefill_args* a, hipStream_t st) {
-  const int64_t tiles = (a->max_q_len + kRows - 1) / kRows;  // workgroups per head and request
-  if (tiles > 0x7fffffff || a->num_q_heads > 65535 || a->batch > 65535) return LSATTN_ERR_INVALID_ARG;
-  LSATTN_LAUNCH_KERNEL((prefill_small_kernel<T, D, MODE>), dim3((unsigned)tiles, (unsigned)a->num_q_heads, (unsigned)a->batch),
-                     dim3(kWaves * 64), 0, st, p);
-  return check_launch();
+template <typename T, int D, int MODE, bool DV, int QB> int launch_rows(SmallParams p, const lsattn_prefill_args* a, hipStream_t st) {
+  const int64_t rows_wg = (kWaves * QB * 16) >> p.pack_shift;
+  for (int64_t tiles = (a->max_q_len + rows_wg - 1) / rows_wg; tiles > 0; tiles -= kMaxTiles) {
+    p.last_tile = (int32_t)(tiles - 1);
+    LSATTN_LAUNCH_KERNEL((prefill_small_kernel<T, D, MODE, DV, QB>),
+                         dim3((unsigned)(p.hkv * p.group), (unsigned)a->batch, (unsigned)(tiles < kMaxTiles ? tiles : kMaxTiles)),
+                         dim3(kWaves * 64), 0, st, p);
+    const int rc = check_launch();
+    if (rc != LSATTN_OK) return rc;
+  }
+  return LSATTN_OK;
 }
 
-template <typename T, int MODE> int launch_d(const SmallParams& p, const lsattn_prefill_args* a, hipStream_t st) {
+// 32 positions per wave serve twice the rows with each K and V operand read, 16 make twice as many, shorter waves: these from
+// three workgroups of the larger shape per CU down, where the launch is as long as its longest wave.  Measured at 64-wide heads
+// (32 | 16 positions, without the sum of the fp16 weights, which costs both 4 to 8 %): 256 workgroups 21.5 | 16.2 us, 512 24.9 | 20.4 and 40.3 | 32.6, 768 30.4 | 31.4, 1024 36.6 | 35.7 and
+// 92.8 | 99.3, 2048 43.9 | 48.6, 4096 170 | 200.
+template <typename T, int D, int MODE, bool DV> int launch(const SmallParams& p, const lsattn_prefill_args* a, hipStream_t st) {
+  if (a->num_q_heads > 65535 || a->batch > 65535) return LSATTN_ERR_INVALID_ARG;
+  const int64_t rows2 = (kWaves * 2 * 16) >> p.pack_shift;
+  const int64_t by_longest = a->batch * ((a->max_q_len + rows2 - 1) / rows2);
+  const int64_t by_total = a->total_q_rows > 0 ? (a->total_q_rows + rows2 - 1) / rows2 + a->batch : by_longest;
+  const int64_t wgs = (by_total < by_longest ? by_total : by_longest) * p.hkv * p.group;
+  return wgs < 3 * kCUs ? launch_rows<T, D, MODE, DV, 1>(p, a, st) : launch_rows<T, D, MODE, DV, 2>(p, a, st);
+}
+
+template <typename T, int MODE, bool DV> int launch_d(const SmallParams& p, const lsattn_prefill_args* a, hipStream_t st) {
   switch (a->head_dim) {
-    case 16: return launch<T, 16, MODE>(p, a, st);
-    case 32: return launch<T, 32, MODE>(p, a, st);
-    case 64: return launch<T, 64, MODE>(p, a, st);
+    case 16: return launch<T, 16, MODE, DV>(p, a, st);
+    case 32: return launch<T, 32, MODE, DV>(p, a, st);
+    case 64: return launch<T, 64, MODE, DV>(p, a, st);
     default: return LSATTN_ERR_UNSUPPORTED;
   }
 }
 
-template <typename T> int launch_mode(const SmallParams& p, const lsattn_prefill_args* a, int mode, hipStream_t st) {
+template <typename T, bool DV> int launch_mode(const SmallParams& p, const lsattn_prefill_args* a, int mode, hipStream_t st) {
   switch (mode) {
-    case 0: return launch_d<T, 0>(p, a, st);
-    case 1: return launch_d<T, 1>(p, a, st);
-    case 2: return launch_d<T, 2>(p, a, st);
+    case 0: return launch_d<T, 0, DV>(p, a, st);
+    case 1: return launch_d<T, 1, DV>(p, a, st);
+    case 2: return launch_d<T, 2, DV>(p, a, st);
     default: return LSATTN_ERR_INVALID_ARG;
   }
 }
@@ -381,9 +504,14 @@ int launch_prefill_small(const lsattn_prefill_args* a, int mode, hipStream_t st)
   p.kv_first = a->kv_first_token_global_idx;
   p.o_start = a->o_b_start_loc;
   p.hq = (int32_t)a->num_q_heads;
+  p.hkv = (int32_t)a->num_kv_heads;
   p.heads_per_kv = (int32_t)(a->num_q_heads / a->num_kv_heads);
   p.peers = (int32_t)a->sp_peers;
-  p.v_f16 = a->v_is_f16;
+  // query heads of a KV head side by side in a workgroup: as many (1, 2 or 4) as the group divides by
+  p.pack_shift = p.heads_per_kv % 4 == 0 ? 2 : p.heads_per_kv % 2 == 0 ? 1 : 0;
+  p.group = p.heads_per_kv >> p.pack_shift;
+  p.d_hkv = fast_div((uint32_t)p.hkv);
+  p.d_peers = fast_div((uint32_t)p.peers);
   p.scale_log2 = a->sm_scale * kLog2e;
   p.o = a->o;
   p.o_st = a->o_stride_t;
@@ -393,7 +521,8 @@ int launch_prefill_small(const lsattn_prefill_args* a, int mode, hipStream_t st)
   p.l = a->l;
   p.ml_st = a->ml_stride_t;
   p.ml_sh = a->ml_stride_h;
-  return a->dtype == LSATTN_F16 ? launch_mode<F16>(p, a, mode, st) : launch_mode<BF16>(p, a, mode, st);
+  if (a->dtype == LSATTN_F16) return launch_mode<F16, true>(p, a, mode, st);
+  return a->v_is_f16 ? launch_mode<BF16, true>(p, a, mode, st) : launch_mode<BF16, false>(p, a, mode, st);
 }
 
 }  // namespace lsattn

@@ -742,3 +742,25 @@ def test_launch_geometry_with_divisors_that_are_not_powers_of_two(lsa, Hq, Hkv, 
     torch.cuda.synchronize()
     assert_o_close(o, o_ref, "O")
     assert_lse_close(lse, lse_ref, "LSE")
+
+
+@pytest.mark.parametrize("D", [16, 32, 64])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("copies,Hq,Hkv", [(1, 8, 2), (6, 16, 4), (6, 6, 6)])
+def test_small_heads_at_the_edges_of_their_tiles(lsa, D, dtype, copies, Hq, Hkv):
+    """16 positions per wave (the small launch) and 32 (the other two: more than 768 workgroups of that shape), four heads
+    side by side in a workgroup and one: lengths around the waves' rows and the 64-key tiles, keys behind a cached context, scores
+    that grow along the keys so that the running maxima are raised again and again."""
+    print("case D", D, dtype, copies, Hq, Hkv, flush=True)
+    lens = [0, 1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 128, 129, 430] * copies
+    ctx = [i % 3 * 61 for i in range(len(lens))]
+    klens = [n + c for n, c in zip(lens, ctx)]
+    T, TK = sum(lens), sum(klens)
+    q, k, v = rand_t((T, Hq, D), 51, dtype), rand_t((TK, Hkv, D), 52, dtype), rand_t((TK, Hkv, D), 53, dtype)
+    ramp = torch.cat([torch.arange(n) for n in klens]).float() / 40 + 1
+    k = (k.float() * ramp[:, None, None]).to(dtype)
+    qm, km = meta(lens, ctx), meta(klens)
+    o, lse = _run_step(lsa, q, k, v, qm, km, 1, max(lens))
+    o_ref, lse_ref = orc.attn_step(q, k, v, *qm, *km, 1)
+    assert_o_close(o, o_ref, "O")
+    assert_lse_close(lse, lse_ref, "LSE")
