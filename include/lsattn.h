@@ -487,12 +487,14 @@ int lsattn_pool_find_contiguous(const int32_t* mem_state, int64_t pool_size, int
 /*
  * mem_state[index[i]] = old value + delta (delta = +1 or -1) for i < n; a slot listed several times still changes
  * by delta once, as `mem_state[index] += delta` does in torch.  counted (int64[2], device memory or pinned host memory that
- * the device can write; both words are written once, when they are final):
+ * the device can write; both words are written once, when they are final; for n <= LSATTN_POOL_REFS_ORDERED after the new state is
+ * visible to the device, else possibly before the last of it):
  *   counted[0] = entries whose slot is non-zero before the update (delta = +1) or after it (delta = -1): the
  *                has_used_tokens / used_tokens of add_refs and decrease_refs (longserve_mem_manager.py:73-88);
  *   counted[1] = entries outside [-pool_size, pool_size), which are skipped (negative entries wrap once).
  * workspace: lsattn_pool_refs_workspace_bytes(n) bytes, 16-byte aligned.
  */
+#define LSATTN_POOL_REFS_ORDERED 4096
 size_t lsattn_pool_refs_workspace_bytes(int64_t n);
 int lsattn_pool_update_refs(int32_t* mem_state, int64_t pool_size, const int64_t* index, int64_t n, int delta,
                             int64_t* counted, void* workspace, size_t workspace_bytes, void* stream);

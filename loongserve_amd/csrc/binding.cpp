@@ -623,6 +623,9 @@ PyObject* pool_update_refs(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     return failed(rc, "lsattn_pool_update_refs");
   {
     pybind11::gil_scoped_release no_gil;
+    // Up to 4096 entries the counts are written behind the state; of a longer list (two launches) they may be there before
+    // it: the caller, who may go on to another stream, waits for the launch.
+    if (index.numel() > LSATTN_POOL_REFS_ORDERED) st.synchronize();
     const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(4);
     while (c[0] < 0 || c[1] < 0) {
       for (int i = 0; i < 64 && (c[0] < 0 || c[1] < 0); i++) __builtin_ia32_pause();

@@ -290,9 +290,10 @@ __device__ __forceinline__ void put_counts(int64_t* counted, int64_t used, int64
 }
 
 // Up to kRefsOneGroup entries by one workgroup: every old value is in a register before the barrier, every new one is
-// written behind it.  (bound by its three dependent loads and a store: 3 us, where the two launches below take 4 and a gap)
+// written behind it.  (bound by its three dependent loads and two stores: 3 us, where the two launches below take 4 and a gap)
 constexpr int kRefsPer = 4;
 constexpr int64_t kRefsOneGroup = 1024 * kRefsPer;
+static_assert(kRefsOneGroup == LSATTN_POOL_REFS_ORDERED, "counts behind the state: the one-workgroup launch");
 __global__ __launch_bounds__(1024) void pool_refs_small_kernel(int32_t* __restrict__ state, int64_t size,
                                                                const int64_t* __restrict__ index, int64_t n, int delta,
                                                                int64_t* __restrict__ counted) {
@@ -320,6 +321,7 @@ __global__ __launch_bounds__(1024) void pool_refs_small_kernel(int32_t* __restri
 #pragma unroll
   for (int k = 0; k < kRefsPer; k++)
     if (slot[k] >= 0) state[slot[k]] = old[k] + delta;
+  __threadfence_system();  // whoever sees the counts (the host, which may go on to another stream) finds the state written
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) {
     used += __shfl_xor(used, d);

@@ -239,3 +239,20 @@ def test_alloc_and_first_fit_in_a_pool_that_takes_the_scan_launch(lsa):
     assert got is not None and got[1:] == (4095, 4097)
     assert m.alloc(5).cpu().tolist() == [3, 1024 * 4096 + 5, size - 78, size - 2, size - 1]
     assert int((m.mem_state == 0).sum()) == 0 and m.can_use_mem_size == 0
+
+
+@pytest.mark.parametrize("n", [64, 4096, 20000])
+def test_freed_slots_are_seen_from_another_stream(lsa, n):
+    """free() has read its counts when it returns, and the state behind them is written by then: an allocation that follows on
+    another stream, without an event between the two, finds the slots."""
+    m = _manager(lsa, n)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    for i in range(20):
+        with torch.cuda.stream(streams[0]):
+            held = m.alloc(n)
+            m.free(held)
+        with torch.cuda.stream(streams[1]):
+            again = m.alloc(n)
+            m.free(again)
+        assert again.cpu().tolist() == list(range(n))
