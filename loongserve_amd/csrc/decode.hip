@@ -860,6 +860,15 @@ constexpr int64_t kCUs = 256;                     // compute units of the MI355X
 // 52.6), a few long ones of one length 1 % (4 x 131072), a few ragged ones up to 13 % slower (4 of 1000 to 8000 tokens, MHA 32: 62 us
 // against 54; GQA 32/8, 1024 waves: 23.1 against 24.1).
 constexpr int64_t kSharesMinBatch = 8, kSharesMinWavesFew = 2048;
+// Not where the rows of the partials' buffers hold less than half of the shares the chip has waves for: 256 requests of 256 tokens,
+// GQA 32/8, are one share (2.9 ms) or a grid (57 us).  And not in place of a grid that one round of workgroups, one per CU, walks,
+// if the rows hold fewer shares than the chip has waves for (24 requests of 1024 tokens, GQA 32/8, 73 shares: 30.1 us against 22.6; 33 of
+// 512: 32.2 against 20.6), or if the requests are few and the longest one's blocks about equal (8 of 8000 GQA 32/8: 48.4 against 45.7, 32 of
+// 384 MHA 32: 38.9 against 35.4, ragged 27.9 against 27.1; with unequal blocks shares win, 16 ragged ones up to 1500 in blocks of 1024, MHA 32:
+// 45.7 against 55.7, and so they do for 128 ragged requests up to 1024: 56.7 against 65.1).  Past one round the shares win also where the
+// rows cut them (65 requests of 257 tokens, GQA 32/8, 66 shares: 26.5 against 32.1; of 512 between 5 % slower and 2 % faster,
+// ragged 27.6 against 31.2).
+constexpr int64_t kSharesOneRoundBatch = 32;
 constexpr int kShareUnits = 4;                    // a share holds at least so many units of kMfmaBatch tokens
 template <typename T>
 __global__ __launch_bounds__(kMfmaWaves * 64, 2) void decode_stage1_mfma_listed_kernel(Stage1Params p) {
@@ -1337,19 +1346,25 @@ template <typename T> static int launch_stage1_mfma(const lsattn_decode_stage1_a
     const int64_t task_groups = (p.tasks + tw - 1) / tw;
     const bool forced = tn.decode_listed == LSATTN_DECODE_LISTED_SHARES;  // (tests: whatever the launch's size)
     if (tn.decode_listed == LSATTN_DECODE_LISTED_OFF || tn.decode_listed == LSATTN_DECODE_LISTED_ON) return LSATTN_OK;
-        int64_t per_group = kCUs / task_groups;  // workgroups per task group: one workgroup per CU in all
+    int64_t per_group = kCUs / task_groups;  // workgroups per task group: one workgroup per CU in all
     if (per_group < 1 || p.row_mul != 1 || a->batch > kListedMaxBatch || shares->units * a->batch > 0x7ffffff) return LSATTN_OK;
-    // partials are numbered below V + batch - 1: the rows of the buffers that the longest request can reach
-    const int64_t by_rows = a->batch * (shares->rows - 1) + 1;
     int64_t max_shares = per_group * cw;
-    if (max_shares > by_rows) max_shares = by_rows;
     const int64_t by_tokens = shares->units * a->batch / kShareUnits;
     if (max_shares > by_tokens) max_shares = by_tokens > 0 ? by_tokens : 1;
+    // partials are numbered below V + batch - 1: the rows of the buffers that the longest request can reach
+    const int64_t wanted = max_shares, by_rows = a->batch * (shares->rows - 1) + 1;
+    if (max_shares > by_rows) max_shares = by_rows;
     if (!forced && tn.decode_stage1 != 0) return LSATTN_OK;
     // (waves of the plain shape at 256 tokens each, whatever the split asked for; the shape whose waves split a block keeps its launches)
     const int64_t waves256 = (shares->units * kMfmaBatch + 255) / 256 * p.tasks * a->batch;
     const bool large = waves256 >= (group < 4 ? 768 : p.tasks < 4 ? 3073 : 513);
     if (!forced && (!large || a->batch < 2 || (a->batch < kSharesMinBatch && waves256 < kSharesMinWavesFew))) return LSATTN_OK;
+    // Short contexts, whose rows hold too few shares (a longest request of up to 256 tokens one share, whatever the batch),
+    // and grids of one round of workgroups, see kSharesOneRoundBatch.
+    const int64_t wgs = wgs_x * wgs_y * a->batch;
+    const bool one_round = wgs > kCUs / 2 && wgs <= kCUs;
+    const bool even = nblk == 1 || a->max_len_in_batch * 8 >= nblk * p.block_seq * 7;
+    if (!forced && (by_rows * 2 < wanted || (one_round && (by_rows < wanted || (even && a->batch <= kSharesOneRoundBatch))))) return LSATTN_OK;
     if (per_group > max_shares) per_group = max_shares;
     *taken = true;
     shares->max_shares = max_shares;

@@ -670,3 +670,43 @@ def test_equal_shares_at_the_edges_of_their_launches(lsa, tuning, Hq, Hkv, B):
     torch.cuda.synchronize()
     assert_o_close(o_d, o_ref, "o")
     assert_lse_close(l_d, l_ref, "lse")
+
+
+@pytest.mark.parametrize("Hq,Hkv,B,longest,BS", [(32, 8, 128, 200, 256), (32, 8, 256, 256, 256), (32, 32, 65, 130, 256), (32, 8, 128, 1000, 1024)])
+def test_batches_of_short_contexts_fill_the_chip(lsa, Hq, Hkv, B, longest, BS):
+    """One row of partials per request: right, and in the fused call no slower than three times the two stages called one after
+    the other (a few dozen us; dealt as the one share that the rows leave room for, such a batch takes ten to fifty times that)."""
+    print("case", Hq, Hkv, B, longest, BS, flush=True)
+    D = 128
+    lens = [longest - i % 90 for i in range(B)]
+    q, kv, table, b_req, b_len = decode_case(700 + B, B, Hq, Hkv, D, lens, sum(lens) + 100, torch.float16)
+    o_ref, l_ref = orc.decode_full(q, kv[:, :Hkv], kv[:, Hkv:], table, b_req, b_len)
+    qd, kvd, td, rd, ld = q.to(DEV), kv.to(DEV), table.to(DEV), b_req.to(DEV), b_len.to(DEV)
+    mo, ml = torch.empty((1, B, Hq, D), device=DEV), torch.empty((1, B, Hq), device=DEV)
+    o, l = torch.empty((B, Hq, D), device=DEV), torch.empty((B, Hq), device=DEV)
+
+    def fused():
+        lsa.longserve_token_decode_attention_flash_decoding(qd, td, rd, ld, mo, ml, B, longest, Hq, D, kvd[:, :Hkv], kvd[:, Hkv:], BS, o, l)
+
+    def staged():
+        lsa.longserve_flash_decode_stage1(qd, kvd[:, :Hkv], kvd[:, Hkv:], td, rd, ld, longest, mo, ml, BS)
+        lsa.longserve_flash_decode_stage2(mo, ml, ld, o, l, BS)
+
+    def time_of(call):
+        best = math.inf
+        for _ in range(4):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(4):
+                call()
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+
+    staged_ms = time_of(staged)
+    o.fill_(float("nan"))
+    fused_ms = time_of(fused)
+    assert_o_close(o, o_ref, "o")
+    assert_lse_close(l, l_ref, "lse")
+    assert fused_ms < 3 * staged_ms, "%.3f ms fused, %.3f ms in two stages" % (fused_ms, staged_ms)
