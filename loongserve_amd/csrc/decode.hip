@@ -1283,7 +1283,7 @@ static int launch_stage1(const lsattn_decode_stage1_args* a, hipStream_t st) {
 // the chip); lsattn_set_tuning forces the choice where the conditions allow it (tuning, tests).
 // What the fused call hands to stage 1 and on to the merge behind it.
 struct SharesPlan {
-  int64_t units;           // in: kMfmaBatch-token units of the longest request
+  int64_t units;           // in: kMfmaBatch-token units of the longest request, in whole blocks of 256 tokens
   int64_t rows;            // in: rows of the partials' buffers per request, as far as the longest request goes
   int64_t max_shares = 0;  // out: 0 if the launch was none for equal shares
 };
@@ -1520,8 +1520,9 @@ extern "C" int lsattn_decode_attention(const lsattn_decode_stage1_args* s1, cons
   if (s1->merge_blocks <= 1 && s1->seq_block_size >= 256 && s1->max_len_in_batch > 0 && s1->num_blocks > 0 &&
       s1->max_len_in_batch < 0x7fffff00) {
     SharesPlan shares;
-    shares.units = (s1->max_len_in_batch + kMfmaBatch - 1) / kMfmaBatch;
+    // (in whole blocks of 256 tokens, as the grids count: a request a little longer than the bound is attended to the end)
     shares.rows = (s1->max_len_in_batch + 255) / 256;
+    shares.units = shares.rows * (256 / kMfmaBatch);
     if (shares.rows > s1->num_blocks) shares.rows = s1->num_blocks;
     const int rc1 = decode_stage1(s1, stream, &shares);
     if (rc1 != LSATTN_OK) return rc1;

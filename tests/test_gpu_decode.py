@@ -710,3 +710,20 @@ def test_batches_of_short_contexts_fill_the_chip(lsa, Hq, Hkv, B, longest, BS):
     assert_o_close(o, o_ref, "o")
     assert_lse_close(l, l_ref, "lse")
     assert fused_ms < 3 * staged_ms, "%.3f ms fused, %.3f ms in two stages" % (fused_ms, staged_ms)
+
+
+@pytest.mark.parametrize("shares", [True, False])
+def test_fused_call_counts_the_bound_on_lengths_in_whole_blocks(lsa, tuning, shares):
+    """max_len_in_batch sizes the launch; a request that is longer within the same 256 tokens is attended to its end, in equal shares
+    as on the grids."""
+    tuning(decode_listed=None if shares else "off")
+    B, Hq, Hkv, D = 24, 32, 8, 128
+    lens = [3990, 3905] + [200 + 37 * i for i in range(B - 2)]
+    q, kv, table, b_req, b_len = decode_case(41, B, Hq, Hkv, D, lens, sum(lens) + 100, torch.float16)
+    o_ref, l_ref = orc.decode_full(q, kv[:, :Hkv], kv[:, Hkv:], table, b_req, b_len)
+    kvd = kv.to(DEV)
+    mo, ml = torch.empty((16, B, Hq, D), device=DEV), torch.empty((16, B, Hq), device=DEV)
+    o, l = lsa.longserve_token_decode_attention_flash_decoding(q.to(DEV), table.to(DEV), b_req.to(DEV), b_len.to(DEV), mo, ml, B, 3900, Hq, D,
+                                                               kvd[:, :Hkv], kvd[:, Hkv:], 256)
+    assert_o_close(o, o_ref, "o")
+    assert_lse_close(l, l_ref, "lse")
