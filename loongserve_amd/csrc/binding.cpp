@@ -19,6 +19,8 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <utility>
+#include <vector>
 
 #include "lsattn.h"
 
@@ -42,6 +44,7 @@ struct Library {
   decltype(&lsattn_rotary_kv_write) rotary_kv_write;
   decltype(&lsattn_pool_alloc) pool_alloc;
   decltype(&lsattn_pool_update_refs) pool_update_refs;
+  decltype(&lsattn_pool_refs_workspace_bytes) pool_refs_workspace_bytes;
   decltype(&lsattn_strerror) strerror;
 } lib;
 
@@ -64,6 +67,7 @@ PyObject* bind(PyObject*, PyObject* addresses) {
       {"lsattn_rotary_kv_write", (void**)&lib.rotary_kv_write},
       {"lsattn_pool_alloc", (void**)&lib.pool_alloc},
       {"lsattn_pool_update_refs", (void**)&lib.pool_update_refs},
+      {"lsattn_pool_refs_workspace_bytes", (void**)&lib.pool_refs_workspace_bytes},
       {"lsattn_strerror", (void**)&lib.strerror},
   };
   for (const auto& e : entries) {
@@ -601,31 +605,62 @@ PyObject* pool_alloc(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
-// (state int32, index int64, delta, workspace, cells: pinned int64 [2]) -> (counted, outside).  Waits for the two counts, which
-// the kernel writes to host memory: the caller needs them at once, and a copy of eight bytes behind a synchronisation takes
-// three times as long as looking for them.  Past a few milliseconds of looking (much work queued before this call) the thread waits
-// on the stream instead.
+// Two words of pinned host memory that a kernel writes its counts to: a pair for every call in flight, taken and given back under
+// the GIL, so that threads never share one.  Idle pairs are kept (kMaxIdle at most, the rest goes back to PyTorch's allocator) and
+// outlive the interpreter: their memory must not be freed behind a HIP runtime that is already gone.
+class Cells {
+  static constexpr size_t kMaxIdle = 64;
+  static std::vector<at::Tensor>& idle() {
+    static auto* pairs = new std::vector<at::Tensor>;
+    return *pairs;
+  }
+  at::Tensor pair;
+
+ public:
+  volatile int64_t* words;
+  Cells() {
+    if (idle().empty()) {
+      pair = at::empty({2}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
+    } else {
+      pair = std::move(idle().back());
+      idle().pop_back();
+    }
+    words = (volatile int64_t*)pair.data_ptr();
+    words[0] = words[1] = -1;
+  }
+  void give_back() {  // (the kernel is done with it)
+    if (idle().size() < kMaxIdle) idle().push_back(std::move(pair));
+  }
+};
+
+// (state int32, index int64, delta, workspace for lists of up to LSATTN_POOL_REFS_ORDERED entries) -> (counted, outside).  Waits for the
+// two counts, which the kernel writes to host memory: the caller needs them at once, and a copy of eight bytes behind a
+// synchronisation takes three times as long as looking for them.  Past a few milliseconds of looking (much work queued before this
+// call) the thread waits on the stream instead.
 PyObject* pool_update_refs(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
-  NEED_ARGS(5);
+  NEED_ARGS(4);
   Args in(args);
   const at::Tensor &state = in.gpu(1), &index = in.gpu(1);
   const int64_t delta = in.integer();
-  const at::Tensor& ws = in.gpu(1);
-  const at::Tensor* cells = tensor(args[in.i]);
-  if (!in.ok || !is(index, at::kLong) || !index.is_contiguous() || !cells || !is(*cells, at::kLong) || cells->numel() != 2)
-    return PyErr_Format(PyExc_ValueError, "pool_update_refs: bad arguments");
-  volatile int64_t* c = (volatile int64_t*)cells->data_ptr();
-  c[0] = c[1] = -1;
+  const at::Tensor& small_ws = in.gpu(1);
+  if (!in.ok || !is(index, at::kLong) || !index.is_contiguous()) return PyErr_Format(PyExc_ValueError, "pool_update_refs: bad arguments");
+  const int64_t n = index.numel();
+  // a longer list takes two launches that hand the old states on: a workspace of this call's own, which no other thread or stream uses
+  const bool ordered = n <= LSATTN_POOL_REFS_ORDERED;
+  const at::Tensor ws = ordered ? small_ws : empty({(int64_t)lib.pool_refs_workspace_bytes(n)}, state, at::kByte);
+  Cells cells;
   const auto st = c10::hip::getCurrentHIPStream();
-  if (const int rc = lib.pool_update_refs((int32_t*)state.data_ptr(), state.size(0), index.numel() ? (const int64_t*)index.data_ptr() : nullptr,
-                                          index.numel(), (int)delta, (int64_t*)c, ws.data_ptr(), ws.nbytes(), st.stream()))
+  if (const int rc = lib.pool_update_refs((int32_t*)state.data_ptr(), state.size(0), n ? (const int64_t*)index.data_ptr() : nullptr, n, (int)delta,
+                                          (int64_t*)cells.words, ws.data_ptr(), ws.nbytes(), st.stream()))
     return failed(rc, "lsattn_pool_update_refs");
+  int64_t counted, outside;
   {
     pybind11::gil_scoped_release no_gil;
     // Up to 4096 entries the counts are written behind the state; of a longer list (two launches) they may be there before
     // it: the caller, who may go on to another stream, waits for the launch.
-    if (index.numel() > LSATTN_POOL_REFS_ORDERED) st.synchronize();
+    if (!ordered) st.synchronize();
+    const volatile int64_t* c = cells.words;
     const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(4);
     while (c[0] < 0 || c[1] < 0) {
       for (int i = 0; i < 64 && (c[0] < 0 || c[1] < 0); i++) __builtin_ia32_pause();
@@ -634,8 +669,11 @@ PyObject* pool_update_refs(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         break;
       }
     }
+    counted = c[0], outside = c[1];
   }
-  return Py_BuildValue("LL", (long long)c[0], (long long)c[1]);
+  if (counted < 0 || outside < 0) return PyErr_Format(PyExc_RuntimeError, "pool_update_refs: the launch left no counts");
+  cells.give_back();
+  return Py_BuildValue("LL", (long long)counted, (long long)outside);
   END_HANDLE_TH_ERRORS
 }
 

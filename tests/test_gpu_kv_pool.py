@@ -256,3 +256,46 @@ def test_freed_slots_are_seen_from_another_stream(lsa, n):
             again = m.alloc(n)
             m.free(again)
         assert again.cpu().tolist() == list(range(n))
+
+
+@pytest.mark.parametrize("n", [50, 6000])
+def test_reference_counts_of_threads_that_share_a_manager(lsa, n):
+    """Two threads count on slots of their own, one on free and one on used ones: each gets its own counts, whatever the other does
+    meanwhile (one workgroup, and the two launches of a longer list)."""
+    import threading
+    m = _manager(lsa, 4 * n)
+    m.mem_state[2 * n:] = 1
+    lists = [torch.arange(n, device=DEV), torch.arange(2 * n, 3 * n + 1, device=DEV)]
+    torch.cuda.synchronize()
+    wrong = []
+
+    def count(index, before):
+        try:
+            for _ in range(400):
+                up, down = m._slots.update_refs(index, 1), m._slots.update_refs(index, -1)
+                if (up, down) != (before, before):
+                    wrong.append((up, down, before))
+        except Exception as e:  # (an assertion in a thread would go unseen)
+            wrong.append(e)
+
+    threads = [threading.Thread(target=count, args=a) for a in zip(lists, (0, n + 1))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong, wrong[:4]
+    assert torch.equal(m.mem_state.cpu(), (torch.arange(4 * n) >= 2 * n).int())
+
+
+def test_a_copied_manager_counts(lsa):
+    """copy.deepcopy copies the tensors a manager holds, pinned ones into pageable memory: none of them is written to from the device
+    as host memory."""
+    import copy
+    m = copy.deepcopy(_manager(lsa, 300))
+    assert all(t.is_cuda for t in vars(m._slots).values() if isinstance(t, torch.Tensor))
+    held = m.alloc(7)
+    m.add_refs(held)
+    m.free(held)
+    assert m.can_use_mem_size == 293
+    m.free(held)
+    assert m.can_use_mem_size == 300 and int(m.mem_state.sum()) == 0
