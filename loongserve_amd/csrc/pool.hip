@@ -323,7 +323,8 @@ __global__ __launch_bounds__(1024) void pool_refs_small_kernel(int32_t* __restri
     if (slot[k] >= 0) __hip_atomic_store(state + slot[k], old[k] + delta, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   // Whoever sees the counts (the host, which may go on to another stream) finds the state written: the stores go through to
   // memory and have arrived in front of the barrier below (a fence of the device writes the whole L2 back, 3 us more).
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  // (from inline assembly that names memory: no store may be moved past it, as past the builtin, which names none)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) {
     used += __shfl_xor(used, d);

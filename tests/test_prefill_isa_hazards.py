@@ -420,3 +420,27 @@ def test_inline_assembly_stores_of_a_partial_keep_their_data_registers_for_two_c
                 m = re.match(r"s_nop (\d+)", nxt)
                 assert m and int(m.group(1)) >= 1, "%s line %d: %s is followed by %s" % (src, i + 1, ins, nxt)
         assert seen >= 8, (src, seen)
+
+
+@pytest.mark.skipif(shutil.which(HIPCC) is None, reason="hipcc not available")
+def test_reference_counts_are_written_behind_a_wait_for_the_slot_states():
+    """pool_refs_small_kernel promises whoever sees its counts that the slot states are in memory: every store of a state (a word with
+    the system-scope bits) runs into the inline-assembly wait for all of them, which the compiler moves no store past, and a barrier lies
+    between that wait and the stores of the counts (double words)."""
+    lines = _device_asm("pool.hip").split("\n")
+    at = next(i for i, ln in enumerate(lines) if re.match(r"^_ZN6lsattn22pool_refs_small_kernel\w+:", ln))
+    end = next(i for i in range(at, len(lines)) if lines[i].startswith(".Lfunc_end"))
+    labels = {m.group(1): i for i in range(at, end) if (m := re.match(r"^(\.LBB\d+_\d+):", lines[i]))}
+    waits = [i for i in range(at, end) if lines[i].strip() == "s_waitcnt vmcnt(0)" and "#ASMSTART" in lines[i - 1]]
+    assert len(waits) == 1, waits
+    states = [i for i in range(at, end) if re.match(r"\s+global_store_dword v.* sc0 sc1", lines[i])]
+    counts = [i for i in range(at, end) if re.match(r"\s+global_store_dwordx2 .* sc0 sc1", lines[i])]
+    barriers = [i for i in range(at, end) if lines[i].strip() == "s_barrier"]
+    assert len(states) == 4 and len(counts) == 2 and len(barriers) == 2, (states, counts, barriers)
+    assert barriers[0] < waits[0] < barriers[1] < min(counts)
+    for i in states:  # a store in front of the wait falls into it; one that was moved out of line branches back to a place in front of it
+        if i > waits[0]:
+            back = next(m for ln in lines[i:end] if (m := re.match(r"\s+s_c?branch\w*\s+(\.LBB\d+_\d+)", ln)))
+            assert labels[back.group(1)] <= waits[0] and barriers[0] < labels[back.group(1)], lines[i]
+        else:
+            assert i > barriers[0], lines[i]
