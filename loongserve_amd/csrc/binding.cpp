@@ -14,11 +14,10 @@
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
 
-#include <pybind11/pybind11.h>
-
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <utility>
 #include <vector>
 
@@ -81,6 +80,24 @@ PyObject* bind(PyObject*, PyObject* addresses) {
 
 PyObject* failed(int rc, const char* what) {
   return PyErr_Format(PyExc_RuntimeError, "%s failed: %s (code %d)", what, lib.strerror(rc), rc);
+}
+
+struct NoGil {
+  PyThreadState* const state = PyEval_SaveThread();
+  ~NoGil() { PyEval_RestoreThread(state); }
+};
+// A call of the library without the GIL: a launch waits where the stream's queue is full, and the other threads of the program
+// go on meanwhile.
+template <typename F, typename... A> auto call(F f, A... a) {
+  NoGil others_run;
+  return f(a...);
+}
+// The allocator's launches of one call belong together (the second reads what the first counted): no other thread's in between.
+std::mutex pool_launches;
+template <typename F, typename... A> int call_pool(F f, A... a) {
+  NoGil others_run;
+  std::lock_guard<std::mutex> alone(pool_launches);
+  return f(a...);
 }
 
 void* stream() { return c10::hip::getCurrentHIPStream().stream(); }
@@ -195,7 +212,7 @@ struct Step {
     const int64_t T = v->size(0), H = v->size(1), D = v->size(2);
     v16 = empty({T, H, D}, *v, at::kHalf);
     p.v = v16.data_ptr(), p.v_stride_t = H * D, p.v_stride_h = D, p.v_is_f16 = 1;
-    return T ? lib.bf16_to_f16_rows(v->data_ptr(), v->stride(0), v16.data_ptr(), H * D, T, H * D, st) : LSATTN_OK;
+    return T ? call(lib.bf16_to_f16_rows, v->data_ptr(), v->stride(0), v16.data_ptr(), H * D, T, H * D, st) : LSATTN_OK;
   }
   // one launch over S cuts of the keys into `parts` (o parts, then their log-sum-exps)
   int cut(int64_t S, int64_t kv_rows, float* parts, void* st) {
@@ -205,7 +222,7 @@ struct Step {
     c.lse = parts + S * Tq * Hq * D;
     c.kv_cuts = (int32_t)S, c.kv_cut_len = (int32_t)(((kv_rows + S - 1) / S + 63) / 64 * 64), c.o_cut_rows = Tq;
     c.total_q_rows = 0;
-    return lib.prefill_step(&c, st);
+    return call(lib.prefill_step, &c, st);
   }
   lsattn_merge_cuts_args merge(int64_t S, const float* parts, int mode) const {
     lsattn_merge_cuts_args m;
@@ -253,11 +270,11 @@ PyObject* context_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
     float* parts = (float*)ws->data_ptr();
     if (const int rc = s.cut(S, kv_rows, parts, st)) return failed(rc, "lsattn_prefill_step");
     const lsattn_merge_cuts_args a = s.merge(S, parts, 1);
-    if (const int rc = lib.prefill_merge_cuts(&a, st)) return failed(rc, "lsattn_prefill_merge_cuts");
+    if (const int rc = call(lib.prefill_merge_cuts, &a, st)) return failed(rc, "lsattn_prefill_merge_cuts");
     Py_RETURN_TRUE;
   }
   s.p.total_q_rows = total;
-  if (const int rc = lib.prefill_step_merge(&s.p, st)) return failed(rc, "lsattn_prefill_step_merge");
+  if (const int rc = call(lib.prefill_step_merge, &s.p, st)) return failed(rc, "lsattn_prefill_step_merge");
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
 }
@@ -302,13 +319,13 @@ PyObject* prefill_partial(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     float* parts = (float*)(ws ? *ws : own).data_ptr();
     if (const int rc = s.cut(S, kv_rows, parts, st)) return failed(rc, "lsattn_prefill_step");
     const lsattn_merge_cuts_args a = s.merge(S, parts, accumulate ? 2 : 0);
-    if (const int rc = lib.prefill_merge_cuts(&a, st)) return failed(rc, "lsattn_prefill_merge_cuts");
+    if (const int rc = call(lib.prefill_merge_cuts, &a, st)) return failed(rc, "lsattn_prefill_merge_cuts");
   } else {
     s.p.total_q_rows = total;
     if (accumulate) {
-      if (const int rc = lib.prefill_step_accumulate(&s.p, st)) return failed(rc, "lsattn_prefill_step_accumulate");
+      if (const int rc = call(lib.prefill_step_accumulate, &s.p, st)) return failed(rc, "lsattn_prefill_step_accumulate");
     } else {
-      if (const int rc = lib.prefill_step(&s.p, st)) return failed(rc, "lsattn_prefill_step");
+      if (const int rc = call(lib.prefill_step, &s.p, st)) return failed(rc, "lsattn_prefill_step");
     }
   }
   PyObject* o1 = out_in ? (Py_INCREF(py_out), py_out) : THPVariable_Wrap(out);
@@ -381,7 +398,7 @@ PyObject* token_decode_attention(PyObject*, PyObject* const* args, Py_ssize_t na
   const at::Tensor lse = lse_in ? *lse_in : empty({batch, Hq}, *q, at::kFloat);
   OR_NONE(d.stage2(out, lse, b_len, mid_o, mid_lse, split));
   d.s1.partials_by_request = d.s2.partials_by_request = by_request;
-  if (const int rc = lib.decode_attention(&d.s1, &d.s2, stream())) return failed(rc, "lsattn_decode_attention");
+  if (const int rc = call(lib.decode_attention, &d.s1, &d.s2, stream())) return failed(rc, "lsattn_decode_attention");
   PyObject* o1 = out_in ? (Py_INCREF(py_out), py_out) : THPVariable_Wrap(out);
   PyObject* o2 = lse_in ? (Py_INCREF(py_lse), py_lse) : THPVariable_Wrap(lse);
   return Py_BuildValue("(NN)", o1, o2);
@@ -400,7 +417,7 @@ PyObject* decode_stage1(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   Decode d;
   OR_NONE(d.stage1(mid_o, mid_lse, q, k, v, table, b_req, b_len, max_len, block, merge));
   OR_NONE(q.size(0) == mid_o.size(1) && q.size(1) == mid_o.size(2) && q.size(2) == mid_o.size(3));
-  if (const int rc = lib.decode_stage1(&d.s1, stream())) return failed(rc, "lsattn_decode_stage1");
+  if (const int rc = call(lib.decode_stage1, &d.s1, stream())) return failed(rc, "lsattn_decode_stage1");
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
 }
@@ -416,7 +433,7 @@ PyObject* decode_stage2(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   Decode d;
   OR_NONE(d.stage2(o, lse, b_len, mid_o, mid_lse, block));
   OR_NONE(o.size(0) == mid_o.size(1) && o.size(1) == mid_o.size(2) && o.size(2) == mid_o.size(3));
-  if (const int rc = lib.decode_stage2(&d.s2, stream())) return failed(rc, "lsattn_decode_stage2");
+  if (const int rc = call(lib.decode_stage2, &d.s2, stream())) return failed(rc, "lsattn_decode_stage2");
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
 }
@@ -444,9 +461,9 @@ PyObject* kv_scatter(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const int64_t n = row_elements(*src), es = src->element_size();
   OR_NONE(n > 0 && row_elements(*pool) == n);
   const int rc = is(index, at::kLong)
-                     ? lib.kv_scatter_i64(src->data_ptr(), src->stride(0) * es, pool->data_ptr(), pool->stride(0) * es,
+                     ? call(lib.kv_scatter_i64, src->data_ptr(), src->stride(0) * es, pool->data_ptr(), pool->stride(0) * es,
                                           (const int64_t*)index.data_ptr(), src->size(0), n * es, stream())
-                     : lib.kv_scatter(src->data_ptr(), src->stride(0) * es, pool->data_ptr(), pool->stride(0) * es, pi32(index),
+                     : call(lib.kv_scatter, src->data_ptr(), src->stride(0) * es, pool->data_ptr(), pool->stride(0) * es, pi32(index),
                                       src->size(0), n * es, stream());
   if (rc) return failed(rc, "lsattn_kv_scatter");
   Py_RETURN_TRUE;
@@ -463,7 +480,7 @@ PyObject* register_decode_tokens(PyObject*, PyObject* const* args, Py_ssize_t na
   const int64_t B = b_len.size(0);
   OR_NONE(is(table, at::kInt) && table.is_contiguous() && i32(b_req, B) && i32(b_len, B));
   OR_NONE((is(mem, at::kInt) || is(mem, at::kLong)) && mem.is_contiguous() && mem.size(0) == B);
-  if (const int rc = lib.register_decode_tokens((int32_t*)table.data_ptr(), table.size(1), pi32(b_req), pi32(b_len), mem.data_ptr(),
+  if (const int rc = call(lib.register_decode_tokens, (int32_t*)table.data_ptr(), table.size(1), pi32(b_req), pi32(b_len), mem.data_ptr(),
                                                 is(mem, at::kLong), B, stream()))
     return failed(rc, "lsattn_register_decode_tokens");
   Py_RETURN_TRUE;
@@ -480,7 +497,7 @@ PyObject* register_tokens(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   OR_NONE(in.ok);
   const int64_t B = b_req.size(0);
   OR_NONE(is(table, at::kInt) && table.is_contiguous() && i32(b_req, B) && i32(b_len, B) && i32(start, B) && i32(mem, mem.size(0)));
-  if (const int rc = lib.register_tokens((int32_t*)table.data_ptr(), table.size(1), pi32(b_req), pi32(start), pi32(b_len), pi32(mem), B,
+  if (const int rc = call(lib.register_tokens, (int32_t*)table.data_ptr(), table.size(1), pi32(b_req), pi32(start), pi32(b_len), pi32(mem), B,
                                          max_len, stream()))
     return failed(rc, "lsattn_register_tokens");
   Py_RETURN_TRUE;
@@ -499,7 +516,7 @@ PyObject* rms_norm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const double eps = in.real();
   OR_NONE(in.ok && half_contiguous(x) && half_contiguous(w) && x.size(1) == w.size(0));
   const at::Tensor out = empty(x.sizes(), x, at::kHalf);
-  if (const int rc = lib.rms_norm(out.data_ptr(), x.data_ptr(), w.data_ptr(), x.size(0), x.size(1), (float)eps, stream()))
+  if (const int rc = call(lib.rms_norm, out.data_ptr(), x.data_ptr(), w.data_ptr(), x.size(0), x.size(1), (float)eps, stream()))
     return failed(rc, "lsattn_rms_norm");
   return THPVariable_Wrap(out);
   END_HANDLE_TH_ERRORS
@@ -512,7 +529,7 @@ PyObject* silu_and_mul_inplace(PyObject*, PyObject* const* args, Py_ssize_t narg
   Args in(args);
   const at::Tensor& io = in.gpu(2);
   OR_NONE(in.ok && half_contiguous(io) && io.size(1) % 2 == 0);
-  if (const int rc = lib.silu_and_mul_inplace(io.data_ptr(), io.size(0), io.size(1) / 2, stream()))
+  if (const int rc = call(lib.silu_and_mul_inplace, io.data_ptr(), io.size(0), io.size(1) / 2, stream()))
     return failed(rc, "lsattn_silu_and_mul_inplace");
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
@@ -540,7 +557,7 @@ PyObject* rotary_emb(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   a.q = q.data_ptr(), a.q_stride_t = q.stride(0), a.q_stride_h = q.stride(1), a.num_q_heads = q.size(1);
   a.kv = k.data_ptr(), a.kv_stride_t = k.stride(0), a.kv_stride_h = k.stride(1), a.num_kv_heads = k.size(1);
   a.cos = c.data_ptr(), a.sin = s.data_ptr(), a.num_tokens = T, a.head_dim = D;
-  if (const int rc = lib.rotary_kv_write(&a, stream())) return failed(rc, "lsattn_rotary_kv_write");
+  if (const int rc = call(lib.rotary_kv_write, &a, stream())) return failed(rc, "lsattn_rotary_kv_write");
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
 }
@@ -582,7 +599,7 @@ PyObject* rotary_kv_write(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       a.b_start_loc = pi32(*start), a.max_len_in_batch = max_len, a.register_mode = 1;
     }
   }
-  if (const int rc = lib.rotary_kv_write(&a, stream())) return failed(rc, "lsattn_rotary_kv_write");
+  if (const int rc = call(lib.rotary_kv_write, &a, stream())) return failed(rc, "lsattn_rotary_kv_write");
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
 }
@@ -598,7 +615,7 @@ PyObject* pool_alloc(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const at::Tensor& ws = in.gpu(1);
   if (!in.ok || need < 0) return PyErr_Format(PyExc_ValueError, "pool_alloc: bad arguments");
   const at::Tensor out = empty({need}, state, at::kLong);
-  if (const int rc = lib.pool_alloc((int32_t*)state.data_ptr(), state.size(0), need, need ? (int64_t*)out.data_ptr() : nullptr,
+  if (const int rc = call_pool(lib.pool_alloc, (int32_t*)state.data_ptr(), state.size(0), need, need ? (int64_t*)out.data_ptr() : nullptr,
                                     ws.data_ptr(), ws.nbytes(), stream()))
     return failed(rc, "lsattn_pool_alloc");
   return THPVariable_Wrap(out);
@@ -651,12 +668,12 @@ PyObject* pool_update_refs(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const at::Tensor ws = ordered ? small_ws : empty({(int64_t)lib.pool_refs_workspace_bytes(n)}, state, at::kByte);
   Cells cells;
   const auto st = c10::hip::getCurrentHIPStream();
-  if (const int rc = lib.pool_update_refs((int32_t*)state.data_ptr(), state.size(0), n ? (const int64_t*)index.data_ptr() : nullptr, n, (int)delta,
+  if (const int rc = call_pool(lib.pool_update_refs, (int32_t*)state.data_ptr(), state.size(0), n ? (const int64_t*)index.data_ptr() : nullptr, n, (int)delta,
                                           (int64_t*)cells.words, ws.data_ptr(), ws.nbytes(), st.stream()))
     return failed(rc, "lsattn_pool_update_refs");
   int64_t counted, outside;
   {
-    pybind11::gil_scoped_release no_gil;
+    NoGil others_run;
     // Up to 4096 entries the counts are written behind the state; of a longer list (two launches) they may be there before
     // it: the caller, who may go on to another stream, waits for the launch.
     if (!ordered) st.synchronize();

@@ -97,3 +97,35 @@ def test_an_error_left_behind_by_the_host_program_is_not_reported_as_a_launch_fa
             d = lsa.longserve_token_decode_attention_flash_decoding(dq, table, b_req, b_len, mo, ml, 2, 500, Hq, D, dkv[:, :Hkv], dkv[:, Hkv:], BS)
             torch.cuda.synchronize()
             assert torch.equal(d[0], d_ok[0]) and torch.equal(d[1], d_ok[1])
+
+
+def test_other_threads_run_while_a_launch_waits(lsa):
+    """A launch that waits (a full queue; here poll(2) in the place of the library's entry point, which takes the same words: no
+    descriptors and 300 milliseconds) holds up its own thread only."""
+    import ctypes
+    import time
+
+    from loongserve_amd import _lib, _native
+    addresses = {name: ctypes.cast(getattr(_lib.load(), name), ctypes.c_void_p).value for name in _lib.EXPORTS}
+    waits = ctypes.cast(ctypes.CDLL(None).poll, ctypes.c_void_p).value
+    io = torch.empty((0, 600), dtype=torch.float16, device=DEV)
+    ticks, done = [], threading.Event()
+
+    def tick():
+        while not done.is_set():
+            ticks.append(time.monotonic())
+            time.sleep(0.01)
+
+    other = threading.Thread(target=tick)
+    _native.bind({**addresses, "lsattn_silu_and_mul_inplace": waits})
+    try:
+        other.start()
+        begin = time.monotonic()
+        assert _native.silu_and_mul_inplace(io)
+        end = time.monotonic()
+    finally:
+        done.set()
+        _native.bind(addresses)
+        other.join()
+    assert end - begin > 0.25
+    assert sum(begin + 0.02 < t < end - 0.02 for t in ticks) >= 5, len(ticks)
