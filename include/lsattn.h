@@ -543,8 +543,10 @@ const char* lsattn_strerror(int code);
  * carry no size field, so a caller must be compiled against the header of the library it loads: check
  * lsattn_version() == LSATTN_VERSION once after loading and refuse to run otherwise.
  * 2 = o_b_start_loc in lsattn_prefill_args, partials_by_request in both decode argument blocks; 3 = lsattn_set_tuning,
- * kv_cuts / kv_cut_len / o_cut_rows / total_q_rows in lsattn_prefill_args, lsattn_prefill_merge_cuts. */
-#define LSATTN_VERSION 3
+ * kv_cuts / kv_cut_len / o_cut_rows / total_q_rows in lsattn_prefill_args, lsattn_prefill_merge_cuts; 4 = dest_index of
+ * lsattn_rotary_kv_write_args untyped, its slots int32 or int64 by dest_index_is_i64 (a reserved word before), lsattn_kv_scatter_i64,
+ * the counts of lsattn_pool_update_refs also in pinned host memory and, past LSATTN_POOL_REFS_ORDERED entries, not behind the state. */
+#define LSATTN_VERSION 4
 int lsattn_version(void);
 
 #ifdef __cplusplus

@@ -95,7 +95,7 @@ TUNING_VALUES = {
     "decode_stage1": {None: 0, "lane": 1, "mfma": 2, "split": 3},
     "decode_listed": {None: 0, "off": 1, "on": 2, "shares": 3},
 }
-LSATTN_VERSION = 3  # of include/lsattn.h, which the argument blocks above mirror
+LSATTN_VERSION = 4  # of include/lsattn.h, which the argument blocks above mirror
 
 
 # every symbol include/lsattn.h declares: name -> (restype, argtypes)
@@ -185,6 +185,9 @@ def load():
         raise ImportError("loongserve_amd: %s has interface version %d, this package is written against %d; rebuild it with "
                           "`python -m loongserve_amd.build`" % (LIB_PATH, lib.lsattn_version(), LSATTN_VERSION))
     from . import _native  # the native argument pass of the operators calls the same loaded library
+    if getattr(_native, "LSATTN_VERSION", None) != LSATTN_VERSION:  # (it fills the same argument blocks)
+        raise ImportError("loongserve_amd: %s was built for another interface version than %d; rebuild it with "
+                          "`python -m loongserve_amd.build`" % (_native.__file__, LSATTN_VERSION))
     _native.bind({name: C.cast(getattr(lib, name), C.c_void_p).value for name in EXPORTS})
     _lib = lib
     return lib

@@ -705,4 +705,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", "Native argument pass of
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__native(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__native(void) {
+  PyObject* m = PyModule_Create(&module);
+  // the interface whose argument blocks are compiled in here; _lib.load() compares it with the library's
+  if (m && PyModule_AddIntConstant(m, "LSATTN_VERSION", LSATTN_VERSION) < 0) Py_CLEAR(m);
+  return m;
+}

@@ -57,6 +57,19 @@ def test_library_exports_every_declared_symbol():
     assert b"invalid" in lib.lsattn_strerror(-1)
 
 
+def test_native_argument_pass_is_built_for_the_same_interface(monkeypatch):
+    """_native.so holds the argument blocks too: one that was built against another header is refused, as such a library is."""
+    from loongserve_amd import _lib, _native
+    header = open(os.path.join(ROOT, "include", "lsattn.h")).read()
+    assert _native.LSATTN_VERSION == int(re.search(r"#define LSATTN_VERSION (\d+)", header).group(1))
+    assert "int32_t dest_index_is_i64;" in header and _native.LSATTN_VERSION >= 4  # (version 3 had a reserved word there)
+    monkeypatch.setattr(_lib, "_lib", None)
+    for other in (_native.LSATTN_VERSION - 1, None):
+        monkeypatch.setattr(_native, "LSATTN_VERSION", other)
+        with pytest.raises(ImportError, match="interface version"):
+            _lib.load()
+
+
 def test_struct_layout_matches_header():
     # compile a tiny C program against the header and compare sizeof / offsetof with ctypes
     import subprocess
