@@ -292,6 +292,7 @@ static int launch_rotary(RotaryWriteParams p, int64_t num_tokens, int64_t max_le
   p.by_pieces = fast_div(p.head_dim / 16);
   p.by_heads = fast_div(p.heads);
   const bool nt = num_tokens * (int64_t)(p.hq + p.hkv) * p.head_dim * 2 >= kStreamBytes;
+  if (num_tokens == 0 && reg_blocks == 0) return LSATTN_OK;  // (no launch whose outcome there is to report)
   const int64_t slice = kMaxUnits / per_token;
   for (int64_t t0 = 0;; t0 += slice) {
     const bool last = num_tokens - t0 <= slice;

@@ -129,3 +129,23 @@ def test_other_threads_run_while_a_launch_waits(lsa):
         other.join()
     assert end - begin > 0.25
     assert sum(begin + 0.02 < t < end - 0.02 for t in ticks) >= 5, len(ticks)
+
+
+def test_a_write_back_of_no_tokens_reports_no_error_of_others(lsa):
+    """lsattn_rotary_kv_write without tokens and without registration launches nothing, and what the host program left in the
+    thread's last-error slot is not its to report."""
+    import ctypes
+
+    from loongserve_amd import _lib
+    loaded = sorted({ln.split()[-1] for ln in open("/proc/self/maps") if "libamdhip64" in ln})
+    hip = ctypes.CDLL(loaded[0])
+    hip.hipSetDevice.argtypes = [ctypes.c_int]
+    x = torch.zeros((4, 2, 128), dtype=torch.float16, device=DEV)
+    c = torch.zeros((4, 64), dtype=torch.float16, device=DEV)
+    a = _lib.RotaryKvWriteArgs(q=x.data_ptr(), q_stride_t=256, q_stride_h=128, num_q_heads=2, kv=x.data_ptr(), kv_stride_t=256, kv_stride_h=128,
+                               num_kv_heads=1, cos=c.data_ptr(), sin=c.data_ptr(), num_tokens=0, head_dim=128)
+    torch.cuda.synchronize()
+    assert hip.hipSetDevice(12345) != 0  # fails, changes nothing, and stays behind as the thread's last error
+    rc = _lib.load().lsattn_rotary_kv_write(ctypes.byref(a), torch.cuda.current_stream().cuda_stream)
+    hip.hipGetLastError()
+    assert rc == 0
