@@ -542,6 +542,17 @@ bool angles(const at::Tensor& c, const at::Tensor& s, int64_t T, int64_t D) {
   return half_contiguous(c) && half_contiguous(s) && same_shape(c, s) && c.size(0) == T && c.size(1) == D / 2;
 }
 
+// Rows [T, H, D] of a and b that surely share no element: the two lie apart, or the rows of one lie between those of the other
+// (views of one packed buffer).  False also for what this does not see (heads of the two in turn).
+bool apart(const at::Tensor& a, const at::Tensor& b) {
+  const int64_t T = a.size(0), st = a.stride(0);
+  const int64_t row_a = (a.size(1) - 1) * a.stride(1) + a.size(2), row_b = (b.size(1) - 1) * b.stride(1) + b.size(2);
+  const int64_t d = ((const char*)b.data_ptr() - (const char*)a.data_ptr()) / a.element_size();  // (both 16-byte aligned, or refused)
+  if (d >= (T - 1) * st + row_a || -d >= (T - 1) * b.stride(0) + row_b) return true;
+  const int64_t r = st > 0 ? (d % st + st) % st : 0;
+  return st == b.stride(0) && row_a <= r && r + row_b <= st;
+}
+
 // (q, k, cos, sin) -> True or None
 PyObject* rotary_emb(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
@@ -551,6 +562,7 @@ PyObject* rotary_emb(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   OR_NONE(in.ok);
   const int64_t T = q.size(0), D = q.size(2);
   OR_NONE(T > 0 && q.size(1) > 0 && k.size(1) > 0 && rotary_operand(q, T, D) && rotary_operand(k, T, D) && angles(c, s, T, D));
+  OR_NONE(apart(q, k));  // (else one after the other)
   // both in one launch: the write-back of a step without pool and table
   lsattn_rotary_kv_write_args a;
   std::memset(&a, 0, sizeof a);

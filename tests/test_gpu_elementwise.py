@@ -205,3 +205,23 @@ def test_silu_and_mul_on_both_sides_of_the_streaming_rule(lsa, T, I):
     torch.cuda.synchronize()
     assert torch.equal(io[:, I:], up)
     assert _ulp(io[-3:].cpu().numpy(), want).max() <= 2
+
+
+@pytest.mark.parametrize("heads", [4, 2, 1])
+def test_rotary_emb_of_operands_that_share_memory(lsa, heads):
+    """q and k are rotated one after the other: heads that belong to both are rotated twice, as with the reference's two launches.
+    Views of one packed buffer that only lie between each other are rotated once."""
+    g = torch.Generator(device=DEV).manual_seed(heads)
+    T, D = 3000, 128
+    x = torch.randn((T, 4 + 2 * heads, D), generator=g, device=DEV).half()
+    ang = torch.rand((T, D // 2), generator=g, device=DEV)
+    cos, sin = ang.cos().half(), ang.sin().half()
+    want = x.clone()
+    for part in (want[:, :4], want[:, 4 - heads:4 + heads]):  # (one tensor a call)
+        lsa.longserve_cuda_kernels._rotary_single(part, cos, sin)
+    lsa.longserve_cuda_kernels.rotary_emb(x[:, :4], x[:, 4 - heads:4 + heads], cos, sin)
+    assert torch.equal(x, want)
+    for part in (want[:, :4], want[:, 4:4 + heads]):
+        lsa.longserve_cuda_kernels._rotary_single(part, cos, sin)
+    lsa.longserve_cuda_kernels.rotary_emb(x[:, :4], x[:, 4:4 + heads], cos, sin)
+    assert torch.equal(x, want)
