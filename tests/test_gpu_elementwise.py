@@ -225,3 +225,17 @@ def test_rotary_emb_of_operands_that_share_memory(lsa, heads):
         lsa.longserve_cuda_kernels._rotary_single(part, cos, sin)
     lsa.longserve_cuda_kernels.rotary_emb(x[:, :4], x[:, 4:4 + heads], cos, sin)
     assert torch.equal(x, want)
+
+
+def test_rms_norm_of_more_rows_than_one_launch_has_workgroups(lsa):
+    """2^24 + 100 rows: a launch of a workgroup per row would have more than 2^32 threads."""
+    T, H = (1 << 24) + 100, 8
+    g = torch.Generator(device=DEV).manual_seed(5)
+    x = torch.randn((T, H), generator=g, device=DEV).half()
+    w = torch.randn((H,), generator=g, device=DEV).half()
+    out = lsa.longserve_cuda_kernels.rms_norm(x, w, 1e-5)
+    for at in (slice(0, 5), slice((1 << 24) - 5, (1 << 24) + 5), slice(T - 5, T)):  # (both ends of both launches)
+        assert _ulp(out[at].cpu().numpy(), ew.rms_norm(x[at].cpu().numpy(), w.cpu().numpy(), 1e-5)).max() <= 1
+    xf = x.float()
+    want = (xf * w.float() * torch.rsqrt((xf * xf).mean(-1, keepdim=True) + 1e-5)).half()
+    assert bool(((out.float() - want.float()).abs() <= 2e-3 * want.float().abs() + 1e-7).all())  # (two steps of a half: 2 * 2^-11 and a little)
