@@ -17,13 +17,17 @@ template <bool NT, typename V> __device__ __forceinline__ void stream_store(V* p
 }
 // ---------------------------------------------------------------------------------------------------
 // rms_norm: out[t, i] = half(float(x[t, i]) * float(w[i]) * inv_rms[t]),  inv_rms = rsqrt(sum x^2 / H + eps),
-// the product in the reference's order (rms_norm.cu:42-45).  One workgroup per token row: a row of up to 8192 elements
-// stays in registers between the two passes (16 bytes of up to four places per lane), longer rows are read twice.  Bound by
-// HBM for many rows and by the chain of its loads for few; a wave per row had a quarter of the loads of a row in flight
-// beside each other: 16384 rows of 4096 49.1 -> 43.7 us (6.1 TB/s), 24 rows 4.9 -> 2.9 us.
+// the product in the reference's order (rms_norm.cu:42-45).  A row is a workgroup's (WPR = 4 waves) or, where it is
+// narrow, a wave's (WPR = 1, four rows per workgroup).  Rows of up to WPR * 64 * CHUNKS pieces of 16 bytes stay in registers
+// between the two passes, longer rows are read twice.  Bound by HBM for many rows and by the chain of its loads for few;
+// in a wave per row there is a quarter of the loads of a row in flight beside each other (16384 rows of 4096 49.1 us against
+// 43.7, 24 rows 4.9 against 2.9), but in a workgroup per row a narrow one leaves lanes idle and meets at a barrier for little: 262144 rows of
+// 128 174 us against 64, of 512 199 against 96, of 1024 265 against 177 (5.9 to 6.1 TB/s from 512 on; below that the turn-over of the
+// workgroups bounds it).  A wave per row up to 512 wide, and up to 1024 from 1024 rows on (fewer take 2.5 us instead of 2.4); at 1536
+// the wave wins from 4096 rows on (87.8 against 78.9 at 65536) and loses 15 % below, at 2048 it loses throughout.
 // ---------------------------------------------------------------------------------------------------
-constexpr int kRmsChunks = 4;  // 16-byte pieces per lane held in registers
-constexpr int64_t kMaxGroups = (1 << 24) - 1;  // workgroups of 256 threads in one launch
+constexpr int64_t kRmsNarrow = 512, kRmsNarrowRows = 1024;
+constexpr int64_t kMaxGroups = (1 << 24) - 1;  // workgroups of 256 threads in one launch (fewer than 2^32 threads)
 
 __device__ __forceinline__ float wave_sum(float v) {
   v = sum_row16(v);
@@ -32,15 +36,19 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
+template <int WPR, int CHUNKS>
 __global__ __launch_bounds__(256) void rms_norm_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ in,
-                                                       const uint16_t* __restrict__ weight, int64_t hidden, float eps) {
-  const int64_t t = blockIdx.x;
+                                                       const uint16_t* __restrict__ weight, int64_t rows, int64_t hidden, float eps) {
+  constexpr int LANES = 64 * WPR;  // of a row
+  const int64_t t = (int64_t)blockIdx.x * (4 / WPR) + threadIdx.x / LANES;
+  if (WPR == 1 && t >= rows) return;  // (no barrier below then)
+  const int lane = threadIdx.x % LANES;
   const int pieces = (int)(hidden / 8);  // 16-byte pieces in a row
   const u32x4* row = (const u32x4*)(in + t * hidden);
   const u32x4* wrow = (const u32x4*)weight;
   u32x4* orow = (u32x4*)(out + t * hidden);
-  const bool cached = pieces <= 256 * kRmsChunks;
-  u32x4 keep[kRmsChunks];
+  const bool cached = pieces <= LANES * CHUNKS;
+  u32x4 keep[CHUNKS];
   float ss = 0.f;
   auto add_squares = [&](const u32x4& x) {
     float f[8];
@@ -50,20 +58,22 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(uint16_t* __restrict__ ou
   };
   if (cached) {
 #pragma unroll
-    for (int c = 0; c < kRmsChunks; c++) {
-      const int i = threadIdx.x + 256 * c;
+    for (int c = 0; c < CHUNKS; c++) {
+      const int i = lane + LANES * c;
       keep[c] = i < pieces ? row[i] : u32x4{0, 0, 0, 0};
     }
 #pragma unroll
-    for (int c = 0; c < kRmsChunks; c++) add_squares(keep[c]);
+    for (int c = 0; c < CHUNKS; c++) add_squares(keep[c]);
   } else {
-    for (int i = threadIdx.x; i < pieces; i += 256) add_squares(row[i]);
+    for (int i = lane; i < pieces; i += LANES) add_squares(row[i]);
   }
   ss = wave_sum(ss);
-  __shared__ float part[4];
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
-  __syncthreads();
-  ss = (part[0] + part[1]) + (part[2] + part[3]);
+  if constexpr (WPR > 1) {
+    __shared__ float part[4];
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    ss = (part[0] + part[1]) + (part[2] + part[3]);
+  }
   const float inv_rms = __builtin_amdgcn_rsqf(ss / (float)hidden + eps);
   auto scale_piece = [&](const u32x4& x, const u32x4& w) {
     float a[8], b[8];
@@ -76,13 +86,27 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(uint16_t* __restrict__ ou
   };
   if (cached) {
 #pragma unroll
-    for (int c = 0; c < kRmsChunks; c++) {
-      const int i = threadIdx.x + 256 * c;
+    for (int c = 0; c < CHUNKS; c++) {
+      const int i = lane + LANES * c;
       if (i < pieces) orow[i] = scale_piece(keep[c], wrow[i]);
     }
   } else {
-    for (int i = threadIdx.x; i < pieces; i += 256) orow[i] = scale_piece(row[i], wrow[i]);
+    for (int i = lane; i < pieces; i += LANES) orow[i] = scale_piece(row[i], wrow[i]);
   }
+}
+
+// WPR waves per row, in slices of as many rows as a launch has workgroups for.
+template <int WPR, int CHUNKS>
+static int launch_rms_norm(uint16_t* out, const uint16_t* in, const uint16_t* weight, int64_t rows, int64_t hidden, float eps, hipStream_t st) {
+  constexpr int64_t PER_WG = 4 / WPR;
+  for (int64_t t0 = 0; t0 < rows; t0 += kMaxGroups * PER_WG) {
+    const int64_t n = rows - t0 < kMaxGroups * PER_WG ? rows - t0 : kMaxGroups * PER_WG;
+    LSATTN_LAUNCH_KERNEL((rms_norm_kernel<WPR, CHUNKS>), dim3((unsigned)((n + PER_WG - 1) / PER_WG)), dim3(256), 0, st, out + t0 * hidden,
+                       in + t0 * hidden, weight, n, hidden, eps);
+    const int rc = check_launch();
+    if (rc != LSATTN_OK) return rc;
+  }
+  return LSATTN_OK;
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -255,15 +279,12 @@ extern "C" int lsattn_rms_norm(void* out, const void* in, const void* weight, in
   if (hidden_size % 8 || (((uintptr_t)out | (uintptr_t)in | (uintptr_t)weight) & 15)) return LSATTN_ERR_INVALID_ARG;
   if (num_tokens == 0) return LSATTN_OK;
   if (hidden_size > 0x7fffffff) return LSATTN_ERR_INVALID_ARG;
-  // (a launch has fewer than 2^32 threads)
-  for (int64_t t0 = 0; t0 < num_tokens; t0 += kMaxGroups) {
-    LSATTN_LAUNCH_KERNEL(rms_norm_kernel, dim3((unsigned)(num_tokens - t0 < kMaxGroups ? num_tokens - t0 : kMaxGroups)), dim3(256), 0,
-                       (hipStream_t)stream, (uint16_t*)out + t0 * hidden_size, (const uint16_t*)in + t0 * hidden_size,
-                       (const uint16_t*)weight, hidden_size, eps);
-    const int rc = check_launch();
-    if (rc != LSATTN_OK) return rc;
-  }
-  return LSATTN_OK;
+  uint16_t* o = (uint16_t*)out;
+  const uint16_t *x = (const uint16_t*)in, *w = (const uint16_t*)weight;
+  hipStream_t st = (hipStream_t)stream;
+  if (hidden_size <= kRmsNarrow || (hidden_size <= 2 * kRmsNarrow && num_tokens >= kRmsNarrowRows))
+    return launch_rms_norm<1, 2>(o, x, w, num_tokens, hidden_size, eps, st);
+  return launch_rms_norm<4, 4>(o, x, w, num_tokens, hidden_size, eps, st);
 }
 
 extern "C" int lsattn_silu_and_mul_inplace(void* io, int64_t num_tokens, int64_t ffn_inter_dim, void* stream) {

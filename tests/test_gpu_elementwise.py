@@ -239,3 +239,16 @@ def test_rms_norm_of_more_rows_than_one_launch_has_workgroups(lsa):
     xf = x.float()
     want = (xf * w.float() * torch.rsqrt((xf * xf).mean(-1, keepdim=True) + 1e-5)).half()
     assert bool(((out.float() - want.float()).abs() <= 2e-3 * want.float().abs() + 1e-7).all())  # (two steps of a half: 2 * 2^-11 and a little)
+
+
+@pytest.mark.parametrize("H", [8, 504, 512, 520, 1016, 1024, 1032, 8192, 8200])
+@pytest.mark.parametrize("T", [1, 3, 1023, 1024, 1025, 4097])
+def test_rms_norm_on_both_sides_of_the_narrow_rows_rule(lsa, T, H):
+    """A wave per row (up to 512 wide, up to 1024 from 1024 rows on; four rows to a workgroup, the last one's missing) and a workgroup
+    per row, in registers and read twice."""
+    rng = np.random.default_rng(T + H)
+    x = (rng.standard_normal((T, H)) * 1.5).astype(np.float16)
+    w = (1 + 0.2 * rng.standard_normal(H)).astype(np.float16)
+    got = lsa.longserve_cuda_kernels.rms_norm(torch.from_numpy(x).to(DEV), torch.from_numpy(w).to(DEV), 1e-5).cpu().numpy()
+    d = _ulp(got, ew.rms_norm(x, w, 1e-5))
+    assert d.max() <= 1 and (d > 0).mean() < 2e-2, (d.max(), (d > 0).mean())
