@@ -179,7 +179,7 @@ __global__ __launch_bounds__(kPoolThreads) void pool_take_kernel(int32_t* __rest
                                                                  int64_t* __restrict__ out_index, int64_t* __restrict__ cells) {
   __shared__ int sh[kPoolPieces][kPoolWaves];
   PoolTile t;
-  t.load(state, size);  // (asked for beside the summaries)
+  if (!free_before) t.load(state, size);  // (asked for beside the summaries)
   const int64_t first_rank = free_before ? free_before[blockIdx.x] : pool_before<false>(blk_free, nullptr);
   if (blockIdx.x == gridDim.x - 1) {
     const int64_t total = first_rank + blk_free[blockIdx.x];
@@ -187,6 +187,8 @@ __global__ __launch_bounds__(kPoolThreads) void pool_take_kernel(int32_t* __rest
     for (int64_t i = total + threadIdx.x; i < need; i += kPoolThreads) out_index[i] = -1;
   }
   if (first_rank >= need) return;
+  // (behind pass 2 by those that take something only: 64 of 42 million slots, with the free after it, 86 us when all read, 66 so)
+  if (free_before) t.load(state, size);
   const int wave = threadIdx.x >> 6;
   int incl[kPoolPieces], mine[kPoolPieces];
 #pragma unroll
