@@ -269,7 +269,7 @@ int lsattn_decode_attention(const lsattn_decode_stage1_args* s1, const lsattn_de
  * exceed LSATTN_STATIC_SCRATCH_BYTES (else LSATTN_ERR_WORKSPACE); merge_blocks must be 0 or 1.  Results are those of
  * lsattn_decode_attention: the same kernels; bit for bit whenever both calls cut the contexts alike, which they do
  * unless the launch is dealt in equal shares and the array holds fewer rows for the batch than the caller's buffers would
- * (then there are fewer shares and the sums are added in another order).  The call allocates and frees nothing.  Each GPU has one such array (held until
+ * (then there are fewer shares, or the launch runs undealt, and the sums are added in another order).  The call allocates and frees nothing.  Each GPU has one such array (held until
  * the process ends) and every call on that GPU uses it: calls that overlap on one GPU (two streams, two threads) race;
  * calls in stream order on one stream do not.  Nothing needs clearing between calls: stage 2 reads only rows that
  * stage 1 of the same call has written.  The first call on a device looks the array's address up
@@ -527,7 +527,7 @@ int lsattn_bf16_to_f16_rows(const void* src, int64_t src_stride, void* dst, int6
 #define LSATTN_DECODE_STAGE1_SPLIT 3 /* the matrix-pipe kernel, the four waves of a workgroup on one block          */
 #define LSATTN_DECODE_LISTED_OFF 1   /* stage 1's grid sized by the longest request                                */
 #define LSATTN_DECODE_LISTED_ON 2    /* a fixed grid walks the list of units that exist                            */
-#define LSATTN_DECODE_LISTED_SHARES 3 /* lsattn_decode_attention deals the blocks in equal shares whatever the size   */
+#define LSATTN_DECODE_LISTED_SHARES 3 /* lsattn_decode_attention deals the tokens in equal shares whatever the size   */
 typedef struct lsattn_tuning {
   int32_t prefill_rows;
   int32_t prefill_order;

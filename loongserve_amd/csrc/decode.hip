@@ -1588,8 +1588,8 @@ extern "C" int lsattn_decode_attention_static(const lsattn_decode_stage1_args* s
   const int64_t per_row = s1->batch * s1->num_q_heads;  // (request, head) pairs per block row
   if (per_row > 0 && rows > (int64_t)LSATTN_STATIC_SCRATCH_BYTES / 4 / 129 / per_row) return LSATTN_ERR_WORKSPACE;
   if ((uint64_t)(rows * per_row * 129) * 4 > (uint64_t)LSATTN_STATIC_SCRATCH_BYTES) return LSATTN_ERR_WORKSPACE;
-  // The array is laid out for as many rows as it holds for this batch, up to one per 256 tokens of the longest request:
-  // the fused call below counts its equal shares in the smallest blocks whose rows it is given.
+  // The array is laid out for as many rows as it holds for this batch, up to one per 256 tokens of the longest request: the
+  // rows bound the number of equal shares in the fused call below.
   int64_t rows_laid = (s1->max_len_in_batch + 255) / 256;
   if (per_row > 0 && rows_laid > (int64_t)LSATTN_STATIC_SCRATCH_BYTES / 4 / 129 / per_row) rows_laid = (int64_t)LSATTN_STATIC_SCRATCH_BYTES / 4 / 129 / per_row;
   if (rows_laid < rows) rows_laid = rows;

@@ -154,7 +154,7 @@ __device__ __forceinline__ void rotate_piece(f16x8* p1, f16x8* p2, const f16x8& 
 
 // ---------------------------------------------------------------------------------------------------
 // The write-back of a step's new tokens in one launch: rotary embedding of q and of the K heads in place (the arithmetic
-// of rotary_emb_kernel), every token's rotated K heads and its V heads copied to the token's slot of the KV pool, and the
+// of rotate_piece), every token's rotated K heads and its V heads copied to the token's slot of the KV pool, and the
 // slots entered in the request table.  A unit is 32 bytes of one (token, head): the two 16-byte halves a rotary lane
 // owns, or two consecutive 16-byte pieces of a V head.  Blocks past the data units do the registration, one table entry
 // per lane.

@@ -87,7 +87,7 @@ def _v_as_f16(v: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tens
     return out
 
 
-KERNEL_HEAD_DIM = 128  # the tuned kernel's head size (and the only one whose KV chunks are cut); 16, 32 and 64 take the plain kernel
+KERNEL_HEAD_DIM = 128  # the tuned kernel's head size (and the only one whose KV chunks are cut); 16, 32 and 64 take prefill_small_kernel
 
 
 def _prefill_args(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first, kv_b_start_loc, kv_b_seq_len, kv_first,

@@ -170,7 +170,8 @@ def test_argument_checks(lsa):
 @pytest.mark.parametrize("T", [1, 9, 3000])
 def test_int64_slots_go_to_the_kernels_as_they_are(lsa, T):
     """The scatter and the fused write-back with the slots as the allocator hands them out against the same with int32 slots,
-    with and without the non-temporal route of large streams (3000 tokens of 64 + 16 heads: 61 MB and more)."""
+    with and without the non-temporal route of large streams (3000 tokens of 96 + 8 rotated heads of 256 bytes:
+    79.9 MB, from 67.1 on)."""
     g = torch.Generator(device=DEV).manual_seed(T)
     Hq, Hkv, D = 96, 8, 128
     q, kv = (torch.randn((T, h, D), generator=g, device=DEV).half() for h in (Hq, 2 * Hkv))
