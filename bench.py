@@ -37,7 +37,7 @@ if ROOT not in sys.path:
 TRAFFIC_SOURCE = "profiles/bench_default_hbm_traffic.txt (rocprofv3 --pmc, scaled by a 1 GiB copy); constants of bench.py, not measured in this run"
 TRAFFIC_BYTES = {
     "config2": 1305.9e6,    # per launch, averaged over the four launches of a ring step (one diagonal + three full)
-    "config3": 5186.9e6,    # the fused call: stage 1 in equal shares (5180.2) + the merge behind it (6.7)
+    "config3": 5194.3e6,    # the fused call: stage 1 in equal shares (5189.8) + the merge behind it (4.5)
     "config1": 92.6e6,
     "config4": 8614.1e6,    # stage 1 over one instance's 4 x 131072 tokens
     "config5": 104980.5e6,    # the attention launch (K/V re-fetched from HBM about 25 times)
@@ -990,7 +990,7 @@ def main():
         # is reported beside it.
         ach = gbs
         plain = d.bytes / (s1["median_ms"] * 1e-3) / 1e9
-        droof = {"decode_kernel": "decode_stage1_mfma_range_kernel<F16> (+ decode_stage2_kernel<float,128,256,true>: the fused call's two launches, timed together)",
+        droof = {"decode_kernel": "decode_stage1_mfma_range_kernel<F16> (+ decode_merge_shares_kernel<float,1>: the fused call's two launches, timed together)",
                  "decode_achieved_gbs": ach, "decode_frac": ach / PEAK_HBM_GBS,
                  "decode_per_launch_ms": st["median_ms"], "decode_traffic": TRAFFIC_BYTES["config3"], "decode_algorithmic_gb": d.bytes / 1e9,
                  "decode_sustained_peak_gbs": read_peak, "decode_frac_of_sustained": ach / read_peak,
@@ -999,14 +999,14 @@ def main():
                  # 256 tokens in this gather): ordinary stores / stores written through as they are issued (the kernel's)
                  "decode_read_with_partial_stores_gbs": read_stores_plain, "decode_read_with_partial_stores_written_through_gbs": read_stores_through}
         summary["config3"] = {"value": _r(gbs, 1), "unit": "GB/s", "frac": _r(gbs / PEAK_HBM_GBS), "ms": _r(st["median_ms"]),
-                              "p10_ms": _r(st["p10_ms"]), "p90_ms": _r(st["p90_ms"]), "kernel": "decode_stage1_mfma_range_kernel<F16> + decode_stage2_kernel",
+                              "p10_ms": _r(st["p10_ms"]), "p90_ms": _r(st["p90_ms"]), "kernel": "decode_stage1_mfma_range_kernel<F16> + decode_merge_shares_kernel",
                               "frac_of_sustained": _r(gbs / read_peak), "plain_grid_stage1_frac": _r(plain / PEAK_HBM_GBS),
                               "two_stages_reference_buffers_ms": _r(sep["median_ms"]),
                               "two_stages_reference_buffers_frac": _r(d.bytes / (sep["median_ms"] * 1e-3) / 1e9 / PEAK_HBM_GBS),
                               "two_stages_merged_blocks_frac": _r(d.bytes / (sepm["median_ms"] * 1e-3) / 1e9 / PEAK_HBM_GBS),
                               "two_stages_frac_of_read_with_as_many_stores": _r(d.bytes / (sep["median_ms"] * 1e-3) / 1e9 / read_stores_through),
                               "workload": "config 3: batch 64, ctx U[4096,32768], GQA 32/8, fp16, 2.5M-slot scattered pool; fused call, BLOCK_SEQ %d, "
-                                          "stage 1 in equal shares of 256-token blocks" % d.BS}
+                                          "stage 1 in equal shares of 32-token units" % d.BS}
         if only == "decode":
             line.update({"value": gbs, "unit": "GB/s", "ms_per_step": st["median_ms"], "steps": 50, "warmup": 10,
                          "config": {"workload": summary["config3"]["workload"]}})
