@@ -108,7 +108,17 @@ typedef struct lsattn_prefill_args {
    * the bound the launch may be sized by the query tiles that can exist instead, each workgroup finding its request from
    * q_b_seq_len.  A bound below the real sum leaves the rows beyond it uncomputed. */
   int64_t total_q_rows;
+  /* Optional (0: unknown); no counterpart in the reference.  An upper bound of the sum of kv_b_seq_len over the batch (the
+   * rows of a packed k).  With it and with total_q_rows the library can tell a batch of short prompts from short chunks
+   * behind long contexts, and takes a kernel of shorter workgroups for the former.  It only steers that choice: a wrong
+   * bound costs time, not results. */
+  int64_t total_kv_rows;
 } lsattn_prefill_args;
+
+/* 1 if the step these arguments describe (v_is_f16 = 0) converts a bfloat16 V on its way into LDS at no cost, as the kernels
+ * for head sizes below 128 and for batches of short prompts do; 0 if the caller should make an fp16 copy of V first
+ * (lsattn_bf16_to_f16_rows).  Looks at the numbers in the block only, not through its pointers. */
+int lsattn_prefill_converts_v(const lsattn_prefill_args* a);
 
 /* Partial of one step from the empty state: o = normalised fp32 output, lse = natural-log
  * log-sum-exp; rows that see no key get o = 0, lse = -inf.  Uses o (F32), lse. */
@@ -545,8 +555,9 @@ const char* lsattn_strerror(int code);
  * 2 = o_b_start_loc in lsattn_prefill_args, partials_by_request in both decode argument blocks; 3 = lsattn_set_tuning,
  * kv_cuts / kv_cut_len / o_cut_rows / total_q_rows in lsattn_prefill_args, lsattn_prefill_merge_cuts; 4 = dest_index of
  * lsattn_rotary_kv_write_args untyped, its slots int32 or int64 by dest_index_is_i64 (a reserved word before), lsattn_kv_scatter_i64,
- * the counts of lsattn_pool_update_refs also in pinned host memory and, past LSATTN_POOL_REFS_ORDERED entries, not behind the state. */
-#define LSATTN_VERSION 4
+ * the counts of lsattn_pool_update_refs also in pinned host memory and, past LSATTN_POOL_REFS_ORDERED entries, not behind the state; 5 = total_kv_rows in lsattn_prefill_args,
+ * lsattn_prefill_converts_v. */
+#define LSATTN_VERSION 5
 int lsattn_version(void);
 
 #ifdef __cplusplus

@@ -30,6 +30,7 @@ struct Library {
   decltype(&lsattn_prefill_step_merge) prefill_step_merge;
   decltype(&lsattn_prefill_step_accumulate) prefill_step_accumulate;
   decltype(&lsattn_prefill_merge_cuts) prefill_merge_cuts;
+  decltype(&lsattn_prefill_converts_v) prefill_converts_v;
   decltype(&lsattn_bf16_to_f16_rows) bf16_to_f16_rows;
   decltype(&lsattn_decode_stage1) decode_stage1;
   decltype(&lsattn_decode_stage2) decode_stage2;
@@ -53,6 +54,7 @@ PyObject* bind(PyObject*, PyObject* addresses) {
       {"lsattn_prefill_step_merge", (void**)&lib.prefill_step_merge},
       {"lsattn_prefill_step_accumulate", (void**)&lib.prefill_step_accumulate},
       {"lsattn_prefill_merge_cuts", (void**)&lib.prefill_merge_cuts},
+      {"lsattn_prefill_converts_v", (void**)&lib.prefill_converts_v},
       {"lsattn_bf16_to_f16_rows", (void**)&lib.bf16_to_f16_rows},
       {"lsattn_decode_stage1", (void**)&lib.decode_stage1},
       {"lsattn_decode_stage2", (void**)&lib.decode_stage2},
@@ -199,6 +201,7 @@ struct Step {
     p.dtype = dtype_of(*q);
     p.sp_peers = (int32_t)peers, p.max_q_len = (int32_t)max_q;
     p.sm_scale = (float)(1.0 / std::sqrt((double)D));
+    p.total_kv_rows = k->size(0);
     return true;
   }
   bool state(const at::Tensor& o) {  // where the result goes
@@ -206,8 +209,10 @@ struct Step {
     p.o = o.data_ptr(), p.o_stride_t = o.stride(0), p.o_stride_h = o.stride(1), p.o_dtype = dtype_of(o);
     return true;
   }
-  // a bfloat16 V of the 128-wide kernel is rewritten as fp16 in front of the launch
-  bool copies_v(bool preconvert) const { return preconvert && p.dtype == LSATTN_BF16 && p.head_dim == 128; }
+  // a bfloat16 V is rewritten as fp16 in front of a launch that does not convert it at no cost itself (cuts: the step is cut along the keys)
+  bool copies_v(bool preconvert, bool cuts) const {
+    return preconvert && p.dtype == LSATTN_BF16 && p.head_dim == 128 && (cuts || !lib.prefill_converts_v(&p));
+  }
   int convert(void* st) {
     const int64_t T = v->size(0), H = v->size(1), D = v->size(2);
     v16 = empty({T, H, D}, *v, at::kHalf);
@@ -261,7 +266,8 @@ PyObject* context_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
     if (per_cut > 0) S = std::min<int64_t>(S, ws->numel() / per_cut);
     S = std::min<int64_t>(S, LSATTN_MAX_KV_CUTS);
   }
-  const bool copy = s.copies_v(preconvert);
+  s.p.total_q_rows = total;
+  const bool copy = s.copies_v(preconvert, S > 1);
   OR_NONE(!copy || v.stride(1) == v.size(2));
   void* st = stream();
   if (copy)
@@ -273,7 +279,6 @@ PyObject* context_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
     if (const int rc = call(lib.prefill_merge_cuts, &a, st)) return failed(rc, "lsattn_prefill_merge_cuts");
     Py_RETURN_TRUE;
   }
-  s.p.total_q_rows = total;
   if (const int rc = call(lib.prefill_step_merge, &s.p, st)) return failed(rc, "lsattn_prefill_step_merge");
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
@@ -299,7 +304,8 @@ PyObject* prefill_partial(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const bool preconvert = in.integer() != 0;
   OR_NONE(in.ok && total >= 0 && S <= LSATTN_MAX_KV_CUTS);
   OR_NONE(!accumulate || (out_in && lse_in));
-  const bool copy = s.copies_v(preconvert);
+  s.p.total_q_rows = total;
+  const bool copy = s.copies_v(preconvert, S > 1);
   OR_NONE(!copy || v.stride(1) == v.size(2));
   const int64_t Tq = q.size(0), Hq = q.size(1), D = q.size(2);
   const int64_t need = S * Tq * Hq * (D + 1);
@@ -321,7 +327,6 @@ PyObject* prefill_partial(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const lsattn_merge_cuts_args a = s.merge(S, parts, accumulate ? 2 : 0);
     if (const int rc = call(lib.prefill_merge_cuts, &a, st)) return failed(rc, "lsattn_prefill_merge_cuts");
   } else {
-    s.p.total_q_rows = total;
     if (accumulate) {
       if (const int rc = call(lib.prefill_step_accumulate, &s.p, st)) return failed(rc, "lsattn_prefill_step_accumulate");
     } else {

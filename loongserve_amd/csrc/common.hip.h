@@ -96,9 +96,11 @@ struct Tuning {
 };
 Tuning tuning();
 
-// The prefill step for head sizes 16, 32 and 64 (prefill_small.hip); `mode`: 0 fp32 partial, 1 in-place (o, m, l), 2 merge into a
+// The prefill step for head sizes 16, 32 and 64, and for short prompts of 128-wide heads (prefill_small.hip); `mode`: 0 fp32 partial, 1 in-place (o, m, l), 2 merge into a
 // running fp32 partial.  Arguments validated by the caller.
 int launch_prefill_small(const lsattn_prefill_args* a, int mode, hipStream_t st);
+// Blocks of 16 query positions per wave (1 or 2) with which that kernel takes this step of 128-wide heads; 0: it does not.
+int prefill_short_blocks(const lsattn_prefill_args* a);
 
 // check_launch reports what the launch in front of it left in the host thread's last-error slot, so every launch first
 // empties that slot: an earlier runtime call of the host program may have left something there that is not this

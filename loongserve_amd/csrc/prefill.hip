@@ -1352,7 +1352,7 @@ extern "C" int lsattn_prefill_step(const lsattn_prefill_args* a, void* stream) {
   const int rc = validate(a, 0);
   if (rc != LSATTN_OK) return rc;
   if (a->batch == 0 || a->max_q_len == 0) return LSATTN_OK;
-  if (a->head_dim != 128) return launch_prefill_small(a, 0, (hipStream_t)stream);
+  if (a->head_dim != 128 || prefill_short_blocks(a)) return launch_prefill_small(a, 0, (hipStream_t)stream);
   if (a->dtype == LSATTN_F16) return launch_prefill<F16, 0, true>(a, (hipStream_t)stream);
   return a->v_is_f16 ? launch_prefill<BF16, 0, true>(a, (hipStream_t)stream) : launch_prefill<BF16, 0, false>(a, (hipStream_t)stream);
 }
@@ -1361,7 +1361,7 @@ extern "C" int lsattn_prefill_step_merge(const lsattn_prefill_args* a, void* str
   const int rc = validate(a, 1);
   if (rc != LSATTN_OK) return rc;
   if (a->batch == 0 || a->max_q_len == 0) return LSATTN_OK;
-  if (a->head_dim != 128) return launch_prefill_small(a, 1, (hipStream_t)stream);
+  if (a->head_dim != 128 || prefill_short_blocks(a)) return launch_prefill_small(a, 1, (hipStream_t)stream);
   if (a->dtype == LSATTN_F16) return launch_prefill<F16, 1, true>(a, (hipStream_t)stream);
   return a->v_is_f16 ? launch_prefill<BF16, 1, true>(a, (hipStream_t)stream) : launch_prefill<BF16, 1, false>(a, (hipStream_t)stream);
 }
@@ -1370,7 +1370,7 @@ extern "C" int lsattn_prefill_step_accumulate(const lsattn_prefill_args* a, void
   const int rc = validate(a, 2);
   if (rc != LSATTN_OK) return rc;
   if (a->batch == 0 || a->max_q_len == 0) return LSATTN_OK;
-  if (a->head_dim != 128) return launch_prefill_small(a, 2, (hipStream_t)stream);
+  if (a->head_dim != 128 || prefill_short_blocks(a)) return launch_prefill_small(a, 2, (hipStream_t)stream);
   if (a->dtype == LSATTN_F16) return launch_prefill<F16, 2, true>(a, (hipStream_t)stream);
   return a->v_is_f16 ? launch_prefill<BF16, 2, true>(a, (hipStream_t)stream) : launch_prefill<BF16, 2, false>(a, (hipStream_t)stream);
 }

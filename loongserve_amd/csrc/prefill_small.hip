@@ -1,5 +1,6 @@
 // The prefill attention step for head sizes 16, 32 and 64 (the reference's Triton kernel takes them beside 128:
-// loongserve/models/llama/triton_kernel/ring_context_flashattention_nopad.py:248-250), gfx950, wave64.
+// loongserve/models/llama/triton_kernel/ring_context_flashattention_nopad.py:248-250) and, for batches of short prompts, 128
+// (prefill_short_blocks), gfx950, wave64.
 //
 // What bounds it is vector work: a 32 x 32 block of scores takes a wave 16 exponentials, 16 multiply-adds, 16 additions and
 // some 15 conversions and checks against 16 (D = 64) to 6 (D = 16) MFMAs, and the time falls only a third from D = 64 to 16.
@@ -98,6 +99,8 @@ constexpr int kWaves = 4;   // waves per workgroup
 constexpr int kTile = 64;   // keys per LDS tile
 constexpr uint32_t kOnes = 0x3C003C00u;  // two ones in fp16
 constexpr int64_t kCUs = 256;
+constexpr int32_t kShortMaxRows = 768;    // 128-wide heads: the longest query chunk this kernel takes
+constexpr int64_t kShortMeanKeys = 1024;  // and the keys per request up to which it does
 constexpr int64_t kMaxTiles = 65535;  // tiles of one launch (the third index of a grid)
 
 // s_waitcnt vmcnt(0) (expcnt / lgkmcnt fields left at their maximum)
@@ -117,7 +120,7 @@ __device__ __forceinline__ const char* uniform_ptr(const char* ptr) {
 // DV: the V tiles are fp16 in memory and go straight into LDS as the K tiles do; otherwise (bfloat16 V) they pass through
 // registers and are converted on the way.  QB: blocks of 16 query positions per wave.
 template <typename T, int D, int MODE, bool DV, int QB>
-__global__ __launch_bounds__(kWaves * 64, QB == 2 && D == 64 && !DV ? 3 : 4) void prefill_small_kernel(SmallParams p) {
+__global__ __launch_bounds__(kWaves * 64, D == 128 ? 2 : QB == 2 && D == 64 && !DV ? 3 : 4) void prefill_small_kernel(SmallParams p) {
   constexpr int KS = D >= 32 ? D / 32 : 1;  // contraction steps of Q K^T (32 elements each; D = 16 fills half of one)
   constexpr int NDB = D / 16;               // 16-wide blocks of the head
   constexpr int CPR = D / 8;                // 16-byte chunks per K or V row
@@ -451,17 +454,31 @@ template <typename T, int D, int MODE, bool DV, int QB> int launch_rows(SmallPar
   return LSATTN_OK;
 }
 
+// query heads of a KV head side by side in a workgroup: as many (1, 2 or 4; the power of two) as the group divides by
+int pack_shift_of(const lsattn_prefill_args* a) {
+  const int32_t heads = a->num_q_heads / a->num_kv_heads;
+  return heads % 4 == 0 ? 2 : heads % 2 == 0 ? 1 : 0;
+}
+// Workgroups that find rows, with `blocks` blocks of 16 positions per wave: the longest request's times the batch, or fewer if
+// the caller bounds the rows of all requests together.
+int64_t workgroups(const lsattn_prefill_args* a, int pack_shift, int blocks) {
+  const int64_t rows = (kWaves * blocks * 16) >> pack_shift;
+  const int64_t by_longest = a->batch * ((a->max_q_len + rows - 1) / rows);
+  const int64_t by_total = a->total_q_rows > 0 ? (a->total_q_rows + rows - 1) / rows + a->batch : by_longest;
+  return (by_total < by_longest ? by_total : by_longest) * (a->num_q_heads >> pack_shift);
+}
+
 // 32 positions per wave serve twice the rows with each K and V operand read, 16 make twice as many, shorter waves: these from
 // three workgroups of the larger shape per CU down, where the launch is as long as its longest wave.  Measured at 64-wide heads
 // (32 | 16 positions, without the sum of the fp16 weights, which costs both 4 to 8 %): 256 workgroups 21.5 | 16.2 us, 512 24.9 | 20.4 and 40.3 | 32.6, 768 30.4 | 31.4, 1024 36.6 | 35.7 and
 // 92.8 | 99.3, 2048 43.9 | 48.6, 4096 170 | 200.
 template <typename T, int D, int MODE, bool DV> int launch(const SmallParams& p, const lsattn_prefill_args* a, hipStream_t st) {
   if (a->num_q_heads > 65535 || a->batch > 65535) return LSATTN_ERR_INVALID_ARG;
-  const int64_t rows2 = (kWaves * 2 * 16) >> p.pack_shift;
-  const int64_t by_longest = a->batch * ((a->max_q_len + rows2 - 1) / rows2);
-  const int64_t by_total = a->total_q_rows > 0 ? (a->total_q_rows + rows2 - 1) / rows2 + a->batch : by_longest;
-  const int64_t wgs = (by_total < by_longest ? by_total : by_longest) * p.hkv * p.group;
-  return wgs < 3 * kCUs ? launch_rows<T, D, MODE, DV, 1>(p, a, st) : launch_rows<T, D, MODE, DV, 2>(p, a, st);
+  return workgroups(a, p.pack_shift, 2) < 3 * kCUs ? launch_rows<T, D, MODE, DV, 1>(p, a, st) : launch_rows<T, D, MODE, DV, 2>(p, a, st);
+}
+
+template <typename T, int MODE, bool DV> int launch_128(const SmallParams& p, const lsattn_prefill_args* a, hipStream_t st) {
+  return prefill_short_blocks(a) == 1 ? launch_rows<T, 128, MODE, DV, 1>(p, a, st) : launch_rows<T, 128, MODE, DV, 2>(p, a, st);
 }
 
 template <typename T, int MODE, bool DV> int launch_d(const SmallParams& p, const lsattn_prefill_args* a, hipStream_t st) {
@@ -469,6 +486,7 @@ template <typename T, int MODE, bool DV> int launch_d(const SmallParams& p, cons
     case 16: return launch<T, 16, MODE, DV>(p, a, st);
     case 32: return launch<T, 32, MODE, DV>(p, a, st);
     case 64: return launch<T, 64, MODE, DV>(p, a, st);
+    case 128: return launch_128<T, MODE, DV>(p, a, st);
     default: return LSATTN_ERR_UNSUPPORTED;
   }
 }
@@ -483,6 +501,32 @@ template <typename T, bool DV> int launch_mode(const SmallParams& p, const lsatt
 }
 
 }  // namespace
+
+// Short prompts of 128-wide heads: the kernel of prefill.hip spends 9 us on starting and ending whatever it computes (eight
+// waves of 256 registers that fill 128 KB of rings and some 40 KB of code before the first product); this one has a
+// quarter of the code, workgroups of 64 rows (128) and two of them per CU, converts a bfloat16 V on the way (no launch in front
+// that copies it), but reads LDS four times (twice) as much per product, which bounds a full chip.  Measured over 472 launches (1 to
+// 32 prompts of 32 to 2048 tokens, equal or log-uniform over a factor of 8, 32/32, 32/8, 64/8 and 8/1 heads; both epilogues;
+// microseconds, the kernel of prefill.hip | 16 positions per wave | 32; bf16 with its copy of V):
+//   1 x 100 MHA f16 10.9 | 5.5 | 7.8        1 x 512 32/8 f16 15.6 | 12.3 | 16.5    16 x 128 MHA f16 25.6 | 19.6 | 17.7
+//   1 x 30 32/8 bf16 12.4 | 4.9 | 6.4       7 x 67..269 32/8 13.5 | 9.3 | 10.8      16 x 256 MHA f16 37.4 | 45.1 | 36.7
+//   8 x 512 32/8 f16 36.6 | 43.6 | 37.9     1 x 1024 32/8 f16 20.8 | 21.5 | 26.9    (neither is taken)
+// 16 positions per wave win up to two and a half workgroups per CU (with one head per workgroup, which leaves the other kernel
+// four times the rows to mask, up to six, for prompts of up to 512 tokens), 32 up to six and 256 tokens; the geometric
+// mean over the launches the rule takes is 25 to 35 % below the other kernel, the worst is 5 % above it.
+// The keys: a tile of 64 costs a wave 0.95 us here (bf16 V 1.15) against 0.86, so short chunks behind a long context, which the
+// host cannot tell from prompts by the query lengths alone, stay with the other kernel: total_kv_rows has to be known.
+int prefill_short_blocks(const lsattn_prefill_args* a) {
+  if (a->head_dim != 128 || a->kv_cuts > 1 || a->o_b_start_loc || a->max_q_len > kShortMaxRows || a->total_kv_rows <= 0 || a->batch <= 0 ||
+      a->total_kv_rows > (int64_t)a->batch * kShortMeanKeys || a->num_kv_heads <= 0)
+    return 0;
+  const Tuning tn = tuning();
+  if (tn.prefill_rows || tn.prefill_order || tn.prefill_pack) return 0;  // (choices among the 128-wide kernel's shapes)
+  const int pack = pack_shift_of(a);
+  const int64_t one = workgroups(a, pack, 1), two = workgroups(a, pack, 2);
+  if (one <= 5 * kCUs / 2 || (pack == 0 && a->max_q_len <= 512 && one <= 6 * kCUs)) return 1;
+  return a->max_q_len <= 256 && two <= 6 * kCUs ? 2 : 0;
+}
 
 // One prefill step with head_dim 16, 32 or 64 (arguments already validated; epilogue `mode` as in the 128-wide kernel).
 int launch_prefill_small(const lsattn_prefill_args* a, int mode, hipStream_t st) {
@@ -507,8 +551,7 @@ int launch_prefill_small(const lsattn_prefill_args* a, int mode, hipStream_t st)
   p.hkv = (int32_t)a->num_kv_heads;
   p.heads_per_kv = (int32_t)(a->num_q_heads / a->num_kv_heads);
   p.peers = (int32_t)a->sp_peers;
-  // query heads of a KV head side by side in a workgroup: as many (1, 2 or 4) as the group divides by
-  p.pack_shift = p.heads_per_kv % 4 == 0 ? 2 : p.heads_per_kv % 2 == 0 ? 1 : 0;
+  p.pack_shift = pack_shift_of(a);
   p.group = p.heads_per_kv >> p.pack_shift;
   p.d_hkv = fast_div((uint32_t)p.hkv);
   p.d_peers = fast_div((uint32_t)p.peers);
@@ -526,3 +569,11 @@ int launch_prefill_small(const lsattn_prefill_args* a, int mode, hipStream_t st)
 }
 
 }  // namespace lsattn
+
+extern "C" int lsattn_prefill_converts_v(const lsattn_prefill_args* a) {
+  if (!a || a->dtype != LSATTN_BF16) return 0;
+  if (a->head_dim != 128) return 1;
+  // (a V that the tile loads cannot read as it lies is copied: the copy lies straight)
+  if (((uintptr_t)a->v & 15) || a->v_stride_t % 8 || a->v_stride_h % 8 || a->v_stride_t <= 0 || a->v_stride_t > (1 << 24)) return 0;
+  return lsattn::prefill_short_blocks(a) != 0;
+}

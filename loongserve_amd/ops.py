@@ -87,7 +87,7 @@ def _v_as_f16(v: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tens
     return out
 
 
-KERNEL_HEAD_DIM = 128  # the tuned kernel's head size (and the only one whose KV chunks are cut); 16, 32 and 64 take prefill_small_kernel
+KERNEL_HEAD_DIM = 128  # the tuned kernel's head size (and the only one whose KV chunks are cut); 16, 32 and 64, and short prompts, take prefill_small_kernel
 
 
 def _prefill_args(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first, kv_b_start_loc, kv_b_seq_len, kv_first,
@@ -119,16 +119,6 @@ def _prefill_args(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first, kv_b_start_lo
                  (kv_b_start_loc, "kv_b_start_loc"), (kv_b_seq_len, "kv_b_seq_len"), (kv_first, "kv_first_token_global_idx")):
         _i32vec(t, n, B)
     a = _lib.PrefillArgs()
-    # (the kernel for head sizes below 128 converts V as it stages it, at no cost: no copy unless the caller brings one)
-    if q.dtype == torch.bfloat16 and ((PRECONVERT_BF16_V and Lq == KERNEL_HEAD_DIM) or v_f16 is not None):
-        if v_f16_valid:
-            if v_f16 is None or v_f16.dtype != torch.float16 or v_f16.shape != v.shape or v_f16.stride(2) != 1:
-                raise ValueError("v_f16_valid needs v_f16, the float16 copy of v")
-            v = v_f16
-        else:
-            v = _v_as_f16(v, v_f16)
-        a.v_is_f16 = 1
-        a._v_f16 = v  # keeps the copy alive as long as the argument block
     a.q, a.k, a.v = q.data_ptr(), k.data_ptr(), v.data_ptr()
     a.q_stride_t, a.q_stride_h = q.stride(0), q.stride(1)
     a.k_stride_t, a.k_stride_h = k.stride(0), k.stride(1)
@@ -152,6 +142,19 @@ def _prefill_args(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first, kv_b_start_lo
         if int(total_q_len) < 0:
             raise ValueError("total_q_len must be >= 0")
         a.total_q_rows = int(total_q_len)
+    a.total_kv_rows = k.shape[0]
+    # (where the kernel converts V as it stages it, at no cost, there is no copy unless the caller brings one)
+    if q.dtype == torch.bfloat16 and (v_f16 is not None or (PRECONVERT_BF16_V and Lq == KERNEL_HEAD_DIM
+                                                            and not _lib.load().lsattn_prefill_converts_v(C.byref(a)))):
+        if v_f16_valid:
+            if v_f16 is None or v_f16.dtype != torch.float16 or v_f16.shape != v.shape or v_f16.stride(2) != 1:
+                raise ValueError("v_f16_valid needs v_f16, the float16 copy of v")
+            v = v_f16
+        else:
+            v = _v_as_f16(v, v_f16)
+        a.v, a.v_stride_t, a.v_stride_h = v.data_ptr(), v.stride(0), v.stride(1)
+        a.v_is_f16 = 1
+        a._v_f16 = v  # keeps the copy alive as long as the argument block
     return a
 
 

@@ -764,3 +764,58 @@ def test_small_heads_at_the_edges_of_their_tiles(lsa, D, dtype, copies, Hq, Hkv)
     o_ref, lse_ref = orc.attn_step(q, k, v, *qm, *km, 1)
     assert_o_close(o, o_ref, "O")
     assert_lse_close(lse, lse_ref, "LSE")
+
+
+@pytest.mark.parametrize("mode", ["partial", "accumulate", "in_place"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Hq,Hkv,lens,ctx,P", [
+    (8, 2, [0, 1, 15, 16, 17, 33, 63, 64, 65, 129], [0, 61, 122], 1),  # 16 positions per wave, four heads side by side
+    (6, 3, [768, 1, 127, 128], [0, 5], 1),                             # the longest prompt that is taken, two heads
+    (3, 3, [31, 257, 64], [3], 4),                                     # one head per workgroup, a striped ring of four
+    (32, 32, [128, 100, 7, 256, 65, 33] * 5, [0, 40], 1),              # 32 positions per wave
+    (4, 4, [769], [0], 1),                                             # one row past it: the kernel of 128-row workgroups
+])
+def test_short_prompts_of_128_wide_heads(lsa, mode, dtype, Hq, Hkv, lens, ctx, P):
+    """Prompts around the waves' rows and the 64-key tiles, keys behind a cached context, scores that grow along the keys, K and
+    V interleaved; every epilogue, the folding ones over two halves of the keys."""
+    print("case", mode, dtype, Hq, Hkv, lens[:6], P, flush=True)
+    D = 128
+    ctx = [ctx[i % len(ctx)] for i in range(len(lens))]
+    klens = [n + c for n, c in zip(lens, ctx)]
+    T, TK = sum(lens), sum(klens)
+    q, kv = rand_t((T, Hq, D), 61, dtype), rand_t((TK, 2 * Hkv, D), 62, dtype)
+    ramp = torch.cat([torch.arange(n) for n in klens]).float() / 80 + 1
+    kv[:, :Hkv] = (kv[:, :Hkv].float() * ramp[:, None, None]).to(dtype)
+    k, v = kv[:, :Hkv], kv[:, Hkv:]
+    qf = [P - 1 + c * P for c in ctx]
+    qm, km = meta(lens, qf), meta(klens)
+    o_ref, lse_ref = orc.attn_step(q, k.contiguous(), v.contiguous(), *qm, *km, P)
+    qd, kvd = q.to(DEV), kv.to(DEV)
+    if mode == "partial":
+        o, lse = lsa.prefill_attention_step(qd, kvd[:, :Hkv], kvd[:, Hkv:], *_dev(*qm), *_dev(*km), P, max(lens), total_q_len=T)
+        torch.cuda.synchronize()
+        assert_o_close(o, o_ref, "O")
+        assert_lse_close(lse, lse_ref, "LSE")
+        return
+    first = [n // 2 for n in klens]
+    begin = (torch.cumsum(torch.tensor(klens), 0) - torch.tensor(klens)).to(torch.int32)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32)
+    steps = [(begin, i32(first), i32([0] * len(lens))),
+             (begin + i32(first), i32([n - f for n, f in zip(klens, first)]), i32([f * P for f in first]))]
+    if mode == "accumulate":
+        o, lse = torch.full((T, Hq, D), 7.0, device=DEV), torch.full((T, Hq), float("-inf"), device=DEV)
+        for s in steps:
+            lsa.prefill_attention_step(qd, kvd[:, :Hkv], kvd[:, Hkv:], *_dev(*qm), *_dev(*s), P, max(lens), o, lse, accumulate=True, total_q_len=T)
+        torch.cuda.synchronize()
+        assert_o_close(o, o_ref, "O")
+        assert_lse_close(lse, lse_ref, "LSE")
+        return
+    o = torch.full((T, Hq, D), 7.0, dtype=dtype, device=DEV)
+    m, l = torch.full((T, Hq), float("-inf"), device=DEV), torch.zeros((T, Hq), device=DEV)
+    o_st, m_st, l_st = torch.zeros((T, Hq, D), dtype=dtype), torch.full((T, Hq), float("-inf")), torch.zeros(T, Hq)
+    for s in steps:
+        lsa.context_attention_fwd(qd, kvd[:, :Hkv], kvd[:, Hkv:], o, *_dev(*qm), *_dev(*s), P, max(lens), m, l, total_q_len=T)
+        orc.context_attention_fwd(q, k.contiguous(), v.contiguous(), o_st, *qm, *s, P, max(lens), m_st, l_st)
+    torch.cuda.synchronize()
+    assert_inplace_o_close(o.cpu(), o_st, o_ref, "o")
+    assert_lse_close(orc.state_lse(m.cpu(), l.cpu()).float(), lse_ref, "state LSE")
