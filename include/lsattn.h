@@ -113,6 +113,11 @@ typedef struct lsattn_prefill_args {
    * behind long contexts, and takes a kernel of shorter workgroups for the former.  It only steers that choice: a wrong
    * bound costs time, not results. */
   int64_t total_kv_rows;
+  /* With kv_cuts = S > 1.  0: cut c of a sequence is [c * kv_cut_len, (c + 1) * kv_cut_len), as above.  1: the S cuts of a sequence
+   * are equal, ceil(kv_b_seq_len / S) keys rounded up to a multiple of 64 but at most kv_cut_len, so that every cut of a short
+   * sequence has keys too (the host knows the longest chunk a batch can hold, not the lengths). */
+  int32_t kv_cut_even;
+  int32_t reserved;
 } lsattn_prefill_args;
 
 /* 1 if the step these arguments describe (v_is_f16 = 0) converts a bfloat16 V on its way into LDS at no cost, as the kernels
@@ -555,7 +560,7 @@ const char* lsattn_strerror(int code);
  * 2 = o_b_start_loc in lsattn_prefill_args, partials_by_request in both decode argument blocks; 3 = lsattn_set_tuning,
  * kv_cuts / kv_cut_len / o_cut_rows / total_q_rows in lsattn_prefill_args, lsattn_prefill_merge_cuts; 4 = dest_index of
  * lsattn_rotary_kv_write_args untyped, its slots int32 or int64 by dest_index_is_i64 (a reserved word before), lsattn_kv_scatter_i64,
- * the counts of lsattn_pool_update_refs also in pinned host memory and, past LSATTN_POOL_REFS_ORDERED entries, not behind the state; 5 = total_kv_rows in lsattn_prefill_args,
+ * the counts of lsattn_pool_update_refs also in pinned host memory and, past LSATTN_POOL_REFS_ORDERED entries, not behind the state; 5 = total_kv_rows and kv_cut_even in lsattn_prefill_args,
  * lsattn_prefill_converts_v. */
 #define LSATTN_VERSION 5
 int lsattn_version(void);

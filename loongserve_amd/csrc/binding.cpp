@@ -225,7 +225,7 @@ struct Step {
     lsattn_prefill_args c = p;
     c.o = parts, c.o_stride_t = Hq * D, c.o_stride_h = D, c.o_dtype = LSATTN_F32;
     c.lse = parts + S * Tq * Hq * D;
-    c.kv_cuts = (int32_t)S, c.kv_cut_len = (int32_t)(((kv_rows + S - 1) / S + 63) / 64 * 64), c.o_cut_rows = Tq;
+    c.kv_cuts = (int32_t)S, c.kv_cut_len = (int32_t)(((kv_rows + S - 1) / S + 63) / 64 * 64), c.o_cut_rows = Tq, c.kv_cut_even = 1;
     c.total_q_rows = 0;
     return call(lib.prefill_step, &c, st);
   }

@@ -70,6 +70,8 @@ struct PrefillParams {
   float* m;
   float* l;
   int64_t ml_st, ml_sh;
+  int32_t spread;    // how many XCDs further the units of the next (sequence, cut) start
+  int32_t cut_mask;  // 0: the cuts of a sequence share its own length, at most kv_cut_len keys each; else all bits: kv_cut_len keys
 };
 
 constexpr int BM = 256;   // query rows per workgroup (32 per wave)
@@ -245,7 +247,7 @@ __global__ __launch_bounds__(HALF ? NWAVE * 32 : NWAVE * 64, HALF ? 2 : 1) void 
   // workgroups sharing a KV head's K/V meet in few L2s and every XCD has work whatever the head count.
   const int group = p.group;
   uint32_t j = blockIdx.x >> 3;
-  const int xcd = blockIdx.x & 7;
+  int xcd = blockIdx.x & 7;
   // A launch of the four-wave shape that fits the chip at once (two workgroups per CU) is paired up by the hardware:
   // workgroup id and id + 256 share a CU.  The second 256 then run from the lightest tile upwards, so that the heaviest
   // meets the lightest and every CU gets the same work.
@@ -300,6 +302,9 @@ __global__ __launch_bounds__(HALF ? NWAVE * 32 : NWAVE * 64, HALF ? 2 : 1) void 
     up = p.tile_major ? r2 : r1;
     slot = p.tile_major ? r1 : r2;
     // (sequence, cut of its KV chunk): j < batch * kv_cuts for every workgroup of the grid
+    // (where a KV head's units are dealt to several XCDs, the units left over from whole rounds of them land on other XCDs from one
+    // (sequence, cut) to the next: a launch of 4 units x 48 cuts on one KV head used half the chip)
+    xcd = (xcd + (int)j * p.spread) & 7;
     b = (int)div_by(j, p.d_cuts);
     cut = (int)j - b * p.kv_cuts;
   }
@@ -310,9 +315,13 @@ __global__ __launch_bounds__(HALF ? NWAVE * 32 : NWAVE * 64, HALF ? 2 : 1) void 
   const int o_start32 = p.o_start ? p.o_start[b] : q_start32;
   asm volatile("" ::"s"(q_len), "s"(kv_len_all), "s"(qf), "s"(kf_all), "s"(q_start32), "s"(kv_start32), "s"(o_start32));
   // the cut's share of the chunk: keys [cut, cut + 1) * kv_cut_len, key n of the chunk at global position kv_first + n * peers
-  const int key0 = cut * p.kv_cut_len;
+  // (or the sequence's own length over the cuts, in whole tiles; no branch here, where the parameters' loads are on their way:
+  // with one, launches without cuts took 0.3 us longer to start)
+  const int even = (((int)(__umulhi((uint32_t)((kv_len_all > 1 ? kv_len_all : 1) - 1), p.d_cuts.mul) >> p.d_cuts.shr) + BN) & -BN) | p.cut_mask;
+  const int cut_len = even < p.kv_cut_len ? even : p.kv_cut_len;
+  const int key0 = cut * cut_len;
   const int kv_rest = kv_len_all - key0;
-  const int kv_len = kv_rest < 0 ? 0 : (kv_rest < p.kv_cut_len ? kv_rest : p.kv_cut_len);
+  const int kv_len = kv_rest < 0 ? 0 : (kv_rest < cut_len ? kv_rest : cut_len);
   const int kf = kf_all + key0 * p.peers;
   const int64_t q_start = q_start32, kv_start = (int64_t)kv_start32 + key0, o_start = o_start32 + (int64_t)cut * p.o_cut_rows;
   const int vh = xcd + 8 * slot;  // (KV head, slice) pair: always < hkv * slices
@@ -1197,10 +1206,12 @@ static int launch_prefill_rows(const lsattn_prefill_args* a, bool tile_major, co
   p.heads_per_kv = a->num_q_heads / a->num_kv_heads;
   const int group = p.heads_per_kv >> p.pack_shift;  // workgroups side by side over the heads of a KV head
   p.group = group;
+  p.spread = (int32_t)((int64_t)group * p.nz % p.slices);
   p.units_per_slice = (int32_t)(((int64_t)group * p.nz + p.slices - 1) / p.slices);
   p.d_group = fast_div((uint32_t)group);
   p.d_slices = fast_div((uint32_t)p.slices);
   p.kv_cuts = a->kv_cuts > 1 ? a->kv_cuts : 1;
+  p.cut_mask = a->kv_cuts > 1 && a->kv_cut_even ? 0 : 0x7fffffff;
   p.kv_cut_len = a->kv_cuts > 1 ? a->kv_cut_len : 0x7fffffff;
   p.o_cut_rows = a->kv_cuts > 1 ? a->o_cut_rows : 0;
   p.d_cuts = fast_div((uint32_t)p.kv_cuts);
@@ -1326,6 +1337,7 @@ static int validate(const lsattn_prefill_args* a, int mode) {
   // the chunk cut along the keys: a multiple of the 64-key tile per cut, the cuts' outputs apart (fp32 partials only),
   // and key positions that stay within 31 bits
   if (a->kv_cuts < 0 || a->kv_cuts > LSATTN_MAX_KV_CUTS) return LSATTN_ERR_INVALID_ARG;
+  if (a->kv_cut_even != 0 && a->kv_cut_even != 1) return LSATTN_ERR_INVALID_ARG;
   if (a->kv_cuts > 1 && (mode != 0 || a->kv_cut_len < 64 || a->kv_cut_len % 64 || a->o_cut_rows <= 0 ||
                          (int64_t)a->kv_cut_len * a->kv_cuts > 0x7fffffff))
     return LSATTN_ERR_INVALID_ARG;

@@ -138,6 +138,7 @@ def _prefill_args(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first, kv_b_start_lo
         a.o_b_start_loc = o_b_start_loc.data_ptr()
     if cuts is not None:
         a.kv_cuts, a.kv_cut_len, a.o_cut_rows = int(cuts[0]), int(cuts[1]), int(cuts[2])
+        a.kv_cut_even = 1
     if total_q_len is not None:
         if int(total_q_len) < 0:
             raise ValueError("total_q_len must be >= 0")
@@ -199,7 +200,7 @@ def _merge_cuts(po, pl, S: int, Tq: int, q_b_start_loc, q_b_seq_len, max_q_len: 
     _lib.check(_lib.load().lsattn_prefill_merge_cuts(C.byref(a), _stream()), "lsattn_prefill_merge_cuts")
 
 
-# Launches below this many 128-row workgroups (batch x query heads x ceil(max_q / 128)) are cut along the keys when the
+# kv_split_count: launches below this many 128-row workgroups (batch x query heads x ceil(max_q / 128)) are cut along the keys when the
 # KV chunks may hold at least KV_SPLIT_MIN_KEYS keys: 256 CUs run one workgroup each.
 KV_SPLIT_BELOW_WORKGROUPS = 192
 KV_SPLIT_ROUND = 256  # workgroups of a cut launch that run at once: one per CU
@@ -207,10 +208,11 @@ KV_SPLIT_MIN_KEYS = 8192
 
 
 def kv_split_count(batch: int, num_q_heads: int, max_q_len: int, kv_rows: int, num_kv_heads: Optional[int] = None) -> int:
-    """KV cuts the prefill operators use by themselves: the count that leaves the longest chain of tiles on a CU shortest
+    """KV cuts to size a workspace for: the count that leaves the longest chain of tiles on a CU shortest
     when the launch's workgroups run in rounds of 256 (one per CU), the smaller count on ties, with cuts of at least 4096
-    keys (kv_rows bounds every sequence's chunk: max_kv_len where the caller gives it, else the rows of the k buffer; the
-    lengths themselves live on the device).  The launch's size without cuts is counted in 128-row workgroups as the
+    keys; the operators use as many as their workspace holds where shorter cuts are faster still (_choose_cuts).  kv_rows bounds
+    every sequence's chunk (max_kv_len where the caller gives it, else the rows of the k buffer; the lengths themselves live on
+    the device).  The launch's size without cuts is counted in 128-row workgroups as the
     kernel forms them: up to four query heads of a KV head side by side (num_kv_heads given), 128 / that many positions each."""
     return _kv_split_count(int(batch), int(num_q_heads), int(max_q_len), int(kv_rows), num_kv_heads, KV_SPLIT_BELOW_WORKGROUPS,
                            KV_SPLIT_ROUND, KV_SPLIT_MIN_KEYS)
@@ -238,6 +240,58 @@ def _kv_split_count(batch, num_q_heads, max_q_len, kv_rows, num_kv_heads, below,
     return best
 
 
+@functools.lru_cache(maxsize=4096)
+def _cuts_for(batch: int, num_q_heads: int, max_q_len: int, keys: int, num_kv_heads: int, most: int) -> int:
+    """KV cuts of a step over `keys` keys a sequence, at most `most` (what the memory for the parts holds): the count with the
+    least predicted time, the smallest within 3 % of it.  A launch of W workgroups without cuts runs W * S with S of them, in rounds of one per CU, each of them
+    a sequence's share of the tiles and a fixed start and end; every cut adds a part to write and to merge; and K and V cannot pass
+    faster than the workgroups' CUs draw them.  The constants, in us: 0.88 per 64-key tile and 13 around it for the
+    128-row shape, 1.57 and 9 for the 256-row one (chosen here as lsattn_prefill_step chooses), 6 + 0.2 per part for the merge and its
+    rows at 4 TB/s, K/V at 5.3 TB/s.  Over 77 shapes (64 to 1024 rows behind 8192 to 100000 keys, one sequence and two;
+    32/32, 32/8, 64/8, 8/1 heads), each timed with 1 to 64 cuts, the pick is 1 % behind the best count in the geometric mean and kv_split_count's
+    13 %: 64 rows x 8192 keys 32/8 51 -> 30 us, 200 x 9000 8/1 56 -> 28, 500 x 65000 32/8 439 -> 415."""
+    group = num_q_heads // num_kv_heads
+
+    def packed(limit):  # query heads side by side in a workgroup
+        p = 1
+        while p < limit and group % (2 * p) == 0:
+            p *= 2
+        return p
+
+    p8, p4 = packed(8), packed(4)
+    tiles256, tiles128 = -(-max_q_len * p8 // 256), -(-max_q_len * p4 // 128)
+    w256, w128 = batch * (num_q_heads // p8) * tiles256, batch * (num_q_heads // p4) * tiles128
+    if w128 <= 0 or w128 >= 2 * KV_SPLIT_ROUND or most <= 1:
+        return 1
+    padded = (tiles128 * 128 // p4) * 5 <= (tiles256 * 256 // p8) * 4
+    part_us = batch * max_q_len * num_q_heads * 1032 / 4e6
+    times = []
+    for S in range(1, max(1, min(_lib.LSATTN_MAX_KV_CUTS, most, batch * keys // 512)) + 1):
+        split = padded or S * w256 <= KV_SPLIT_ROUND // 2 or (S * w256 <= KV_SPLIT_ROUND and max_q_len > 1024)
+        live = S * (w128 if split else w256)
+        per_tile, around = (0.88, 13.0) if split else (1.57, 9.0)
+        walk = -(-live // KV_SPLIT_ROUND) * (-(-keys / S // 64) * per_tile + around)
+        merge = 6.0 + S * (0.2 + part_us) if S > 1 else 0.0
+        draw = batch * keys * num_kv_heads * 512 / 5.3e6 * max(1.0, KV_SPLIT_ROUND / live) + around
+        times.append(max(walk, draw) + merge)
+    return next(S for S, t in enumerate(times, 1) if t <= 1.03 * min(times))
+
+
+def _choose_cuts(q, k, batch: int, max_q_len: int, max_kv_len: Optional[int], workspace) -> int:
+    """KV cuts an operator uses where the caller names none: as many as are fastest and `workspace` holds, but kv_split_count
+    where that is the caller's measure of it (a pair of tensors, or one tensor that holds fewer)."""
+    kv_rows = k.shape[0] if max_kv_len is None else int(max_kv_len)
+    if kv_rows < KV_SPLIT_MIN_KEYS or batch <= 0 or k.shape[1] == 0 or q.shape[1] % k.shape[1]:
+        return 1
+    most = _workspace_cuts(workspace, q.shape[0], q.shape[1], q.shape[-1])
+    if workspace is not None:
+        sized = kv_split_count(batch, q.shape[1], max_q_len, kv_rows, k.shape[1])
+        if isinstance(workspace, (tuple, list)) or most < sized:
+            return sized
+    keys = kv_rows if max_kv_len is not None else max(1, kv_rows // batch)  # (the rows of the buffer are those of all sequences)
+    return _cuts_for(batch, q.shape[1], int(max_q_len), keys, k.shape[1], min(most, _lib.LSATTN_MAX_KV_CUTS))
+
+
 def _cut_len(kv_rows: int, S: int) -> int:
     """Keys per cut: kv_rows over S cuts, rounded up to the kernel's 64-key tile."""
     return -(-(-(-kv_rows // S)) // 64) * 64
@@ -259,7 +313,7 @@ def context_attention_fwd(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first_token_
     one workgroup per 128 query rows and head, too few for the chip.  With workspace (a contiguous float32 tensor the caller
     owns, S * Tq * Hq * (D + 1) elements for S cuts; or a pair of tensors [S*Tq,Hq,D], [S*Tq,Hq]) the KV chunks are cut
     into S slices inside one launch that writes S fp32 partials per row to the workspace, and a second launch folds
-    them into (o, m, l) by the same update (RING:171-188).  S follows kv_split_count (from shapes alone; max_kv_len, an
+    them into (o, m, l) by the same update (RING:171-188).  S follows from shapes alone (_choose_cuts; max_kv_len, an
     upper bound of every chunk's length, replaces the rows of the k buffer there: in the layer k is a view of a buffer
     sized for the longest batch), capped by what the workspace holds; kv_splits forces it.  Without a workspace the call
     is the reference's: one launch, no scratch.  (m, l) stay opaque: a step folded this way enters as (its LSE, 1).
@@ -277,8 +331,7 @@ def context_attention_fwd(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first_token_
         cuts = kv_rows = 1
         if workspace is not None and q.shape[-1] == KERNEL_HEAD_DIM:
             kv_rows = k.shape[0] if max_kv_len is None else max_kv_len
-            cuts = kv_splits if kv_splits is not None else kv_split_count(q_b_seq_len.shape[0], q.shape[1], max_q_b_seq_len, kv_rows,
-                                                                          k.shape[1])
+            cuts = kv_splits if kv_splits is not None else _choose_cuts(q, k, q_b_seq_len.shape[0], max_q_b_seq_len, max_kv_len, workspace)
         if _native.context_attention(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first_token_global_idx, kv_b_start_loc,
                                      kv_b_seq_len, kv_first_token_global_idx, logical_sp_peers_num, max_q_b_seq_len, m, l,
                                      0 if total_q_len is None else total_q_len, cuts, kv_rows, workspace, PRECONVERT_BF16_V):
@@ -305,7 +358,7 @@ def _context_attention_checked(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first_t
     S = 1
     if workspace is not None and D == KERNEL_HEAD_DIM and q.dim() == 3:
         kv_rows = k.shape[0] if max_kv_len is None else int(max_kv_len)
-        S = kv_split_count(q_b_seq_len.shape[0], q.shape[1], int(max_q_b_seq_len), kv_rows, k.shape[1]) if kv_splits is None else int(kv_splits)
+        S = _choose_cuts(q, k, q_b_seq_len.shape[0], max_q_b_seq_len, max_kv_len, workspace) if kv_splits is None else int(kv_splits)
         S = min(S, _workspace_cuts(workspace, q.shape[0], q.shape[1], D), _lib.LSATTN_MAX_KV_CUTS)
     if S > 1:
         Tq = q.shape[0]
@@ -340,7 +393,7 @@ def prefill_attention_step(q, k, v, q_b_start_loc, q_b_seq_len, q_first_token_gl
     kv_splits: short query chunks against a long KV chunk give the launch too few workgroups for the chip (one per 128
     query rows and head); with kv_splits = S > 1 every sequence's KV chunk is cut into S slices inside one launch, which
     computes the S partials of every row (lsattn_prefill_args.kv_cuts), and lsattn_prefill_merge_cuts joins them for the
-    rows of the sequences.  None chooses S from the shapes (kv_split_count over max_kv_len, an upper bound of every
+    rows of the sequences.  None chooses S from the shapes (_choose_cuts over max_kv_len, an upper bound of every
     chunk's length; the rows of the k buffer if not given), 1 switches it off.  The partials take S times the size of
     (out, lse): kv_split_workspace passes the caller's memory for them (as context_attention_fwd's workspace).
 
@@ -354,8 +407,9 @@ def prefill_attention_step(q, k, v, q_b_start_loc, q_b_seq_len, q_first_token_gl
         kv_rows = k.shape[0] if max_kv_len is None else max_kv_len
         cuts = 1
         if q.shape[-1] == KERNEL_HEAD_DIM:
-            cuts = kv_splits if kv_splits is not None else kv_split_count(q_b_seq_len.shape[0], q.shape[1], max_q_b_seq_len, kv_rows,
-                                                                          k.shape[1])
+            cuts = kv_splits
+            if cuts is None:
+                cuts = _choose_cuts(q, k, q_b_seq_len.shape[0], max_q_b_seq_len, max_kv_len, kv_split_workspace)
         done = _native.prefill_partial(q, k, v, q_b_start_loc, q_b_seq_len, q_first_token_global_idx, kv_b_start_loc, kv_b_seq_len,
                                        kv_first_token_global_idx, logical_sp_peers_num, max_q_b_seq_len, out, lse, sm_scale,
                                        accumulate, 0 if total_q_len is None else total_q_len, cuts, kv_rows, kv_split_workspace,
@@ -383,7 +437,11 @@ def _prefill_attention_step_checked(q, k, v, q_b_start_loc, q_b_seq_len, q_first
     if out.dtype != torch.float32 or lse.dtype != torch.float32 or not lse.is_contiguous():
         raise ValueError("out and lse must be float32, lse contiguous")
     kv_rows = k.shape[0] if max_kv_len is None else int(max_kv_len)
-    S = kv_split_count(q_b_seq_len.shape[0], q.shape[1], int(max_q_b_seq_len), kv_rows, k.shape[1]) if kv_splits is None else int(kv_splits)
+    S = 1
+    if kv_splits is not None:
+        S = int(kv_splits)
+    elif D == KERNEL_HEAD_DIM:
+        S = _choose_cuts(q, k, q_b_seq_len.shape[0], max_q_b_seq_len, max_kv_len, kv_split_workspace)
     if D != KERNEL_HEAD_DIM:
         S = 1  # (the cut along the keys is the 128-wide kernel's)
     if S > 1:

@@ -321,3 +321,23 @@ def test_kv_split_count_from_shapes():
     assert kv_split_count(1, 100, 128, 100000) == 5          # 100 workgroups: two rounds of five cuts walk less than one round of two
     assert kv_split_count(1, 32, 100, 4096) == 1             # short KV
     assert kv_split_count(0, 32, 100, 100000) == 1
+
+
+def test_cuts_are_bounded_by_the_memory_for_their_parts():
+    """What the operators choose by themselves: never more parts than the caller's workspace holds, kv_split_count where it is a
+    pair of tensors or holds fewer than that (the operators cap or refuse it then), one for short chunks."""
+    torch = pytest.importorskip("torch")
+    from loongserve_amd.ops import _choose_cuts, kv_split_count
+    q = torch.empty((64, 8, 128), dtype=torch.float16, device="meta")
+    for rows in (8192, 20000, 100000):
+        k = torch.empty((rows, 1, 128), dtype=torch.float16, device="meta")
+        sized = kv_split_count(1, 8, 64, rows, 1)
+        free = _choose_cuts(q, k, 1, 64, None, None)
+        assert 1 < sized <= free <= 64 and rows // free >= 512
+        for held in (1, sized - 1, sized, sized + 1, 64):
+            got = _choose_cuts(q, k, 1, 64, None, torch.empty(held * 64 * 8 * 129, device="meta"))
+            assert got == sized if held < sized else got <= held
+        assert _choose_cuts(q, k, 1, 64, None, (None, None)) == sized
+        assert _choose_cuts(q, k, 1, 64, 8191, None) == 1
+        assert _choose_cuts(q, k, 0, 64, None, None) == 1
+    assert _choose_cuts(torch.empty((4096, 32, 128), device="meta"), k, 8, 4096, None, None) == 1

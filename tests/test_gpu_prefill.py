@@ -819,3 +819,32 @@ def test_short_prompts_of_128_wide_heads(lsa, mode, dtype, Hq, Hkv, lens, ctx, P
     torch.cuda.synchronize()
     assert_inplace_o_close(o.cpu(), o_st, o_ref, "o")
     assert_lse_close(orc.state_lse(m.cpu(), l.cpu()).float(), lse_ref, "state LSE")
+
+
+@pytest.mark.parametrize("even", [1, 0])
+@pytest.mark.parametrize("Hq,Hkv,S", [(8, 1, 5), (8, 1, 64), (4, 2, 16), (6, 3, 2), (12, 4, 33)])
+def test_kv_cuts_on_fewer_heads_than_xcds(lsa, Hq, Hkv, S, even):
+    """The cuts of a sequence as shares of its own length or of a length for all, on launches whose units start on another XCD
+    from one cut to the next: ragged chunks (none, fewer keys than cuts, one tile and one key more), every row once."""
+    import ctypes as C
+    from loongserve_amd import _lib, ops
+    print("case", Hq, Hkv, S, even, flush=True)
+    D, P = 128, 2
+    qlens, klens = [40, 7, 130, 1, 33], [0, 3, 1000, 65, 64 * S]
+    longest = max(klens)
+    q = rand_t((sum(qlens), Hq, D), 71, torch.float16)
+    kv = rand_t((sum(klens), 2 * Hkv, D), 72, torch.float16)
+    k, v = kv[:, :Hkv], kv[:, Hkv:]
+    qm, km = meta(qlens, [0, 5, 700, 200, 64 * S * P]), meta(klens, [0, 1, 0, 0, 0])
+    o_ref, lse_ref = orc.attn_step(q, k.contiguous(), v.contiguous(), *qm, *km, P)
+    T, qd, kvd, qmd, kmd = sum(qlens), q.to(DEV), kv.to(DEV), _dev(*qm), _dev(*km)
+    po, pl = torch.full((S * T, Hq, D), 7.0, device=DEV), torch.full((S * T, Hq), 7.0, device=DEV)
+    a = ops._prefill_args(qd, kvd[:, :Hkv], kvd[:, Hkv:], po, *qmd, *kmd, P, max(qlens), None, cuts=(S, ops._cut_len(longest, S), T))
+    a.lse, a.kv_cut_even = pl.data_ptr(), even
+    st = torch.cuda.current_stream().cuda_stream
+    _lib.check(_lib.load().lsattn_prefill_step(C.byref(a), C.c_void_p(st)), "lsattn_prefill_step")
+    o, lse = torch.empty((T, Hq, D), device=DEV), torch.empty((T, Hq), device=DEV)
+    ops._merge_cuts(po, pl, S, T, qmd[0], qmd[1], max(qlens), 0, o, lse=lse)
+    torch.cuda.synchronize()
+    assert_o_close(o, o_ref, "O")
+    assert_lse_close(lse, lse_ref, "LSE")
