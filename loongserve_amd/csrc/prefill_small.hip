@@ -93,6 +93,8 @@ struct SmallParams {
   float* m;
   float* l;
   int64_t ml_st, ml_sh;
+  int32_t batch;  // (TURN: a request's place among the ids moves on by one from tile to tile)
+  FastDiv d_batch;
 };
 
 constexpr int kWaves = 4;   // waves per workgroup
@@ -119,7 +121,7 @@ __device__ __forceinline__ const char* uniform_ptr(const char* ptr) {
 
 // DV: the V tiles are fp16 in memory and go straight into LDS as the K tiles do; otherwise (bfloat16 V) they pass through
 // registers and are converted on the way.  QB: blocks of 16 query positions per wave.
-template <typename T, int D, int MODE, bool DV, int QB>
+template <typename T, int D, int MODE, bool DV, int QB, bool TURN = false>
 __global__ __launch_bounds__(kWaves * 64, D == 128 ? 2 : QB == 2 && D == 64 && !DV ? 3 : 4) void prefill_small_kernel(SmallParams p) {
   constexpr int KS = D >= 32 ? D / 32 : 1;  // contraction steps of Q K^T (32 elements each; D = 16 fills half of one)
   constexpr int NDB = D / 16;               // 16-wide blocks of the head
@@ -142,7 +144,11 @@ __global__ __launch_bounds__(kWaves * 64, D == 128 ? 2 : QB == 2 && D == 64 && !
   // grid: (KV head, heads side by side), request, tile from the last one down: the heaviest tiles of all requests start
   // first, and with a multiple of eight KV heads the workgroups of one run on one XCD (ids are dealt round-robin)
   const int gq = (int)div_by(blockIdx.x, p.d_hkv), kvh = (int)blockIdx.x - gq * p.hkv;
-  const int b = blockIdx.y;
+  int b = blockIdx.y;
+  if constexpr (TURN) {  // (requests_take_turns; a kernel of its own, so that the others stay as they are)
+    const uint32_t place = blockIdx.y + blockIdx.z;
+    b = (int)(place - div_by(place, p.d_batch) * (uint32_t)p.batch);
+  }
   const int rows_wg = (kWaves * QB * 16) >> p.pack_shift;  // query positions of this workgroup
   const int m_wg = (p.last_tile - (int)blockIdx.z) * rows_wg;
   const int q_len = p.q_len[b];
@@ -441,11 +447,24 @@ __global__ __launch_bounds__(kWaves * 64, D == 128 ? 2 : QB == 2 && D == 64 && !
   }
 }
 
-template <typename T, int D, int MODE, bool DV, int QB> int launch_rows(SmallParams p, const lsattn_prefill_args* a, hipStream_t st) {
+// Whether a request's place among the ids moves on from tile to tile (TURN).  Ids go to the eight XCDs in turn and within one to its four
+// shader engines.  If the ids of two tiles of a request are a multiple of 32 apart, all its workgroups share one shader engine of an
+// XCD, and while only the longest requests have a tile left to start, the others idle: 8 sequences of 1000 to 3000 tokens, 32/8 heads
+// of 64, had 2 workgroups on a CU until half of the launch was over, some 4 and some 1, where 8 x 2048 keep 3.9.  Turning places
+// fill them evenly.  Measured over 60 ragged launches (2 to 32 sequences, 300 to 6000 tokens; microseconds, fixed | turning):
+//   8 x 1000..3000 32/8 183 | 165   2 x 1206..3618 64/8 144 | 123   4 x 120..3615 64/8 bf16 87.9 | 61.8   4 x 688..2064 32/32 53.2 | 47.3
+//   4 x 2582..5165 32/8 bf16 344 | 314   8 x 1304..2608 12/12 88.8 | 79.5   16 x 31..959 64/8 57.3 | 53.5
+// At other distances (11 x 388..1166 32/8 44.8 | 47.1; distance 6 of the eights 9 % better to 4 % worse), with fewer than 16 tiles
+// (8 x 280..842 32/32 31.5 | 33.3) and with equal lengths turning gains nothing: those keep the kernel without it.
+bool requests_take_turns(const lsattn_prefill_args* a, int64_t ids_per_tile, int64_t tiles) {
+  return ids_per_tile * a->batch % 32 == 0 && tiles >= 16 && a->total_q_rows > 0 && a->total_q_rows * 10 <= (int64_t)a->batch * a->max_q_len * 9;
+}
+
+template <typename T, int D, int MODE, bool DV, int QB, bool TURN = false> int launch_rows(SmallParams p, const lsattn_prefill_args* a, hipStream_t st) {
   const int64_t rows_wg = (kWaves * QB * 16) >> p.pack_shift;
   for (int64_t tiles = (a->max_q_len + rows_wg - 1) / rows_wg; tiles > 0; tiles -= kMaxTiles) {
     p.last_tile = (int32_t)(tiles - 1);
-    LSATTN_LAUNCH_KERNEL((prefill_small_kernel<T, D, MODE, DV, QB>),
+    LSATTN_LAUNCH_KERNEL((prefill_small_kernel<T, D, MODE, DV, QB, TURN>),
                          dim3((unsigned)(p.hkv * p.group), (unsigned)a->batch, (unsigned)(tiles < kMaxTiles ? tiles : kMaxTiles)),
                          dim3(kWaves * 64), 0, st, p);
     const int rc = check_launch();
@@ -474,7 +493,10 @@ int64_t workgroups(const lsattn_prefill_args* a, int pack_shift, int blocks) {
 // 92.8 | 99.3, 2048 43.9 | 48.6, 4096 170 | 200.
 template <typename T, int D, int MODE, bool DV> int launch(const SmallParams& p, const lsattn_prefill_args* a, hipStream_t st) {
   if (a->num_q_heads > 65535 || a->batch > 65535) return LSATTN_ERR_INVALID_ARG;
-  return workgroups(a, p.pack_shift, 2) < 3 * kCUs ? launch_rows<T, D, MODE, DV, 1>(p, a, st) : launch_rows<T, D, MODE, DV, 2>(p, a, st);
+  if (workgroups(a, p.pack_shift, 2) < 3 * kCUs) return launch_rows<T, D, MODE, DV, 1>(p, a, st);  // (all at once on the chip)
+  const int64_t rows_wg = (kWaves * 2 * 16) >> p.pack_shift;
+  return requests_take_turns(a, (int64_t)p.hkv * p.group, (a->max_q_len + rows_wg - 1) / rows_wg)
+             ? launch_rows<T, D, MODE, DV, 2, true>(p, a, st) : launch_rows<T, D, MODE, DV, 2>(p, a, st);
 }
 
 template <typename T, int MODE, bool DV> int launch_128(const SmallParams& p, const lsattn_prefill_args* a, hipStream_t st) {
@@ -555,6 +577,8 @@ int launch_prefill_small(const lsattn_prefill_args* a, int mode, hipStream_t st)
   p.group = p.heads_per_kv >> p.pack_shift;
   p.d_hkv = fast_div((uint32_t)p.hkv);
   p.d_peers = fast_div((uint32_t)p.peers);
+  p.batch = (int32_t)a->batch;
+  p.d_batch = fast_div((uint32_t)p.batch);
   p.scale_log2 = a->sm_scale * kLog2e;
   p.o = a->o;
   p.o_st = a->o_stride_t;

@@ -766,6 +766,27 @@ def test_small_heads_at_the_edges_of_their_tiles(lsa, D, dtype, copies, Hq, Hkv)
     assert_lse_close(lse, lse_ref, "LSE")
 
 
+@pytest.mark.parametrize("D,dtype", [(64, torch.float16), (64, torch.bfloat16), (16, torch.float16)])
+@pytest.mark.parametrize("lens", [[1500, 700, 1, 0, 33, 1201, 64, 500], [31, 2600, 0, 1297], [5000, 2]])
+def test_small_heads_in_a_ragged_batch_of_many_tiles(lsa, D, dtype, lens):
+    """Some 2000 workgroups whose requests are shorter than the longest by far, the total known, the ids of a request's tiles a
+    multiple of 32 apart: the requests take turns in the grid, and every row is computed just as without the bound."""
+    print("case D", D, dtype, lens, flush=True)
+    T, Hq, Hkv = sum(lens), 64, 8
+    q, k, v = rand_t((T, Hq, D), 61, dtype), rand_t((T, Hkv, D), 62, dtype), rand_t((T, Hkv, D), 63, dtype)
+    m = meta(lens)
+    md = _dev(*m)
+    o, lse = lsa.prefill_attention_step(*_dev(q, k, v), *md, *md, 1, max(lens), total_q_len=T)
+    torch.cuda.synchronize()
+    # (the oracle over one query head of every KV head; all rows are compared with the launch that knows no total)
+    first = q[:, ::Hq // Hkv].contiguous()
+    o_ref, lse_ref = orc.attn_step(first, k, v, *m, *m, 1)
+    assert_o_close(o[:, ::Hq // Hkv], o_ref, "O")
+    assert_lse_close(lse[:, ::Hq // Hkv], lse_ref, "LSE")
+    o_all, lse_all = lsa.prefill_attention_step(*_dev(q, k, v), *md, *md, 1, max(lens))
+    assert torch.equal(o, o_all) and torch.equal(lse, lse_all)
+
+
 @pytest.mark.parametrize("mode", ["partial", "accumulate", "in_place"])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("Hq,Hkv,lens,ctx,P", [
