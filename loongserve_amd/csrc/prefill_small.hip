@@ -371,22 +371,25 @@ __global__ __launch_bounds__(kWaves * 64, D == 128 ? 2 : QB == 2 && D == 64 && !
     const int mb = m0 + 16 * qb;
     if (mb >= q_len) break;  // (wave-uniform: a block without positions; it only helped to stage)
     const float l_tot = col_sum(l_run[qb]);
+    // (0 exactly if the row saw no key.  A NaN score makes the sum NaN: it counts as a key, so that the row's outputs and its running
+    // state become NaN, as they do in the reference, and no step before or after hides it)
+    const bool seen = !(l_tot == 0.f);
     // O becomes a mean with the very weights it was summed with: a rounding that a row's weights share (one key that outweighs
     // the others) falls out of it, which makes up for maxima that lag (a P of 1 is exact in fp16, one of 1.4 is not).
     // Against 64 bits the fp32 partial of N(0, 1) * 0.5 inputs is off by 1.70e-4 to 1.72e-4 at 1000 to 3000 tokens of 64-wide heads,
     // 1.74e-4 to 1.75e-4 with maxima that never lag and 1.76e-4 with neither.  The sum that (m, l) and the LSE state stays the fp32 one.
-    const float fix = l_pv[qb][0] > 0.f ? l_tot / l_pv[qb][0] : 0.f;
+    const float fix = l_pv[qb][0] == 0.f ? 0.f : l_tot / l_pv[qb][0];
 #pragma unroll
     for (int db = 0; db < NDB; db++) oacc[qb][db] *= fix;
     const bool here = in_range[qb];
     const int64_t tok = o_start + (here ? mb + c : mb);
     if (MODE == 0) {
       if (here) {
-        const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+        const float inv = seen ? 1.f / l_tot : 0.f;
         float* orow = (float*)p.o + tok * p.o_st + (int64_t)h * p.o_sh;
 #pragma unroll
         for (int db = 0; db < NDB; db++) *(f32x4*)(orow + db * 16 + 4 * g) = oacc[qb][db] * inv;
-        if (g == 0) p.lse[tok * p.hq + h] = l_tot > 0.f ? (m_run[qb] + __builtin_amdgcn_logf(l_tot)) * kLn2 : -INFINITY;
+        if (g == 0) p.lse[tok * p.hq + h] = seen ? (m_run[qb] + __builtin_amdgcn_logf(l_tot)) * kLn2 : -INFINITY;
       }
     }
     if (MODE == 1) {
@@ -394,7 +397,7 @@ __global__ __launch_bounds__(kWaves * 64, D == 128 ? 2 : QB == 2 && D == 64 && !
       const int64_t at = tok * p.ml_st + (int64_t)h * p.ml_sh;
       const float m_old = p.m[at], l_old = p.l[at];
       const float M = fmaxf(m_run[qb], m_old);
-      const bool upd = here && M != -INFINITY && l_tot > 0.f;
+      const bool upd = here && seen;  // (a row that saw a key has a maximum, unless all its scores are NaN)
       float L = 0.f;
       if (upd) {
         const float w_old = l_old * exp2_diff(m_old, M);
@@ -423,7 +426,7 @@ __global__ __launch_bounds__(kWaves * 64, D == 128 ? 2 : QB == 2 && D == 64 && !
     }
     if (MODE == 2) {
       // fold the step's partial into the running fp32 (O, LSE); a row that saw no key stays as it is
-      const bool upd = here && l_tot > 0.f;
+      const bool upd = here && seen;
       const float a_old = p.lse[tok * p.hq + h] * kLog2e;
       float new_lse = 0.f;
       if (upd) {

@@ -1,0 +1,57 @@
+"""GPU parity of prefill_small_kernel beyond the shapes of test_gpu_prefill.py, which forces the 128-wide kernel's shapes in turn: here the
+library chooses."""
+import pytest
+import torch
+
+from oracle import attn_oracle as orc
+from tests.helpers import assert_inplace_o_close, assert_lse_close, assert_o_close, meta, rand_t
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _dev(*ts):
+    return [t.to(DEV) for t in ts]
+
+
+@pytest.mark.parametrize("mode", ["partial", "accumulate", "in_place"])
+@pytest.mark.parametrize("D,dtype", [(128, torch.float16), (128, torch.bfloat16), (64, torch.float16), (16, torch.bfloat16)])
+def test_nan_scores_reach_the_rows_that_see_them(lsa, mode, D, dtype):
+    """A NaN in a K row and in a Q row (short prompts of 128-wide heads, small heads): the rows that meet one become NaN, outputs and
+    running state, stay NaN through a second step, and no other row changes by more than its rounding."""
+    print("case", mode, D, dtype, flush=True)
+    lens, Hq, Hkv = [100, 33], 4, 2
+    T = sum(lens)
+    q, k, v = rand_t((T, Hq, D), 81, dtype), rand_t((T, Hkv, D), 82, dtype), rand_t((T, Hkv, D), 83, dtype)
+    m = meta(lens)
+    o_ref, lse_ref = orc.attn_step(q, k, v, *m, *m, 1)
+    qn, kn = q.clone(), k.clone()
+    kn[10, 0, 3] = float("nan")   # key 10 of the first request, heads 0 and 1
+    qn[105, 2, 0] = float("nan")  # row 5 of the second request, head 2
+    hit = torch.zeros((T, Hq), dtype=torch.bool)
+    hit[10:100, :2] = True
+    hit[105, 2] = True
+    qd, kd, vd, md = *_dev(qn, kn, v), _dev(*m)
+    if mode == "in_place":
+        o = torch.full((T, Hq, D), 7.0, dtype=dtype, device=DEV)
+        ms, ls = torch.full((T, Hq), float("-inf"), device=DEV), torch.zeros((T, Hq), device=DEV)
+        step = lambda K: lsa.context_attention_fwd(qd, K, vd, o, *md, *md, 1, max(lens), ms, ls, total_q_len=T)
+        lse_of = lambda: orc.state_lse(ms.cpu(), ls.cpu()).float()
+    else:
+        o, lse = torch.full((T, Hq, D), 7.0, device=DEV), torch.full((T, Hq), float("-inf"), device=DEV)
+        step = lambda K: lsa.prefill_attention_step(qd, K, vd, *md, *md, 1, max(lens), o, lse, accumulate=mode == "accumulate", total_q_len=T)
+        lse_of = lambda: lse.cpu()
+    step(kd)
+    torch.cuda.synchronize()
+    got, got_lse = o.float().cpu(), lse_of()
+    assert torch.equal(got.isnan().all(-1), hit) and torch.equal(got.isnan().any(-1), hit) and torch.equal(got_lse.isnan(), hit)
+    got[hit], got_lse[hit] = o_ref.float()[hit], lse_ref.float()[hit]
+    if mode == "in_place":
+        assert_inplace_o_close(got.to(dtype), o_ref.to(dtype), o_ref, "o")
+    else:
+        assert_o_close(got, o_ref, "O")
+    assert_lse_close(got_lse, lse_ref, "LSE")
+    if mode != "partial":  # the same keys once more, without the NaN in K: the rows stay NaN
+        step(k.to(DEV))
+        torch.cuda.synchronize()
+        assert torch.equal(o.float().cpu().isnan().all(-1), hit) and torch.equal(lse_of().isnan(), hit)
