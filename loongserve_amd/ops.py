@@ -144,15 +144,13 @@ def _prefill_args(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first, kv_b_start_lo
             raise ValueError("total_q_len must be >= 0")
         a.total_q_rows = int(total_q_len)
     a.total_kv_rows = k.shape[0]
-    # (where the kernel converts V as it stages it, at no cost, there is no copy unless the caller brings one)
-    if q.dtype == torch.bfloat16 and (v_f16 is not None or (PRECONVERT_BF16_V and Lq == KERNEL_HEAD_DIM
-                                                            and not _lib.load().lsattn_prefill_converts_v(C.byref(a)))):
-        if v_f16_valid:
-            if v_f16 is None or v_f16.dtype != torch.float16 or v_f16.shape != v.shape or v_f16.stride(2) != 1:
-                raise ValueError("v_f16_valid needs v_f16, the float16 copy of v")
-            v = v_f16
-        else:
-            v = _v_as_f16(v, v_f16)
+    if q.dtype == torch.bfloat16 and (v_f16 is not None or (PRECONVERT_BF16_V and Lq == KERNEL_HEAD_DIM)):
+        if v_f16_valid and (v_f16 is None or v_f16.dtype != torch.float16 or v_f16.shape != v.shape or v_f16.stride(2) != 1):
+            raise ValueError("v_f16_valid needs v_f16, the float16 copy of v")
+        # (where the kernel converts V as it stages it, at no cost, there is no copy unless the caller brings one)
+        if v_f16 is None and _lib.load().lsattn_prefill_converts_v(C.byref(a)):
+            return a
+        v = v_f16 if v_f16_valid else _v_as_f16(v, v_f16)
         a.v, a.v_stride_t, a.v_stride_h = v.data_ptr(), v.stride(0), v.stride(1)
         a.v_is_f16 = 1
         a._v_f16 = v  # keeps the copy alive as long as the argument block

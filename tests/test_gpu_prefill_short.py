@@ -55,3 +55,23 @@ def test_nan_scores_reach_the_rows_that_see_them(lsa, mode, D, dtype):
         step(k.to(DEV))
         torch.cuda.synchronize()
         assert torch.equal(o.float().cpu().isnan().all(-1), hit) and torch.equal(lse_of().isnan(), hit)
+
+
+@pytest.mark.parametrize("rows", [100, 2000])
+def test_v_f16_valid_needs_the_copy_whatever_kernel_runs(lsa, rows):
+    """Short prompts (whose kernel converts a bfloat16 V itself) and longer ones: the flag without the buffer, or with one that cannot be
+    the copy, is refused by both operators."""
+    q, k, v = (torch.zeros((rows, 2, 128), dtype=torch.bfloat16, device=DEV) for _ in range(3))
+    md = _dev(*meta([rows]))
+    o, m, l = torch.zeros_like(q), torch.zeros((rows, 2), device=DEV), torch.zeros((rows, 2), device=DEV)
+    for held in (None, v, torch.zeros((rows, 1, 128), dtype=torch.float16, device=DEV)):
+        with pytest.raises(ValueError, match="v_f16_valid needs v_f16"):
+            lsa.prefill_attention_step(q, k, v, *md, *md, 1, rows, v_f16=held, v_f16_valid=True)
+        with pytest.raises(ValueError, match="v_f16_valid needs v_f16"):
+            lsa.context_attention_fwd(q, k, v, o, *md, *md, 1, rows, m, l, v_f16=held, v_f16_valid=True)
+    for t in (q, k, v):
+        t.normal_().mul_(8).round_().div_(8)  # (exact in fp16 too)
+    want = lsa.prefill_attention_step(q, k, v, *md, *md, 1, rows)
+    got = lsa.prefill_attention_step(q, k, v, *md, *md, 1, rows, v_f16=v.half(), v_f16_valid=True)
+    torch.cuda.synchronize()
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
