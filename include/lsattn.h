@@ -109,7 +109,7 @@ typedef struct lsattn_prefill_args {
    * q_b_seq_len.  A bound below the real sum leaves the rows beyond it uncomputed. */
   int64_t total_q_rows;
   /* Optional (0: unknown); no counterpart in the reference.  An upper bound of the sum of kv_b_seq_len over the batch (the
-   * rows of a packed k).  With it and with total_q_rows the library can tell a batch of short prompts from short chunks
+   * rows of a packed k).  With it, total_q_rows and max_kv_len the library can tell a batch of short prompts from short chunks
    * behind long contexts, and takes a kernel of shorter workgroups for the former.  It only steers that choice: a wrong
    * bound costs time, not results. */
   int64_t total_kv_rows;
@@ -117,8 +117,24 @@ typedef struct lsattn_prefill_args {
    * are equal, ceil(kv_b_seq_len / S) keys rounded up to a multiple of 64 but at most kv_cut_len, so that every cut of a short
    * sequence has keys too (the host knows the longest chunk a batch can hold, not the lengths). */
   int32_t kv_cut_even;
-  int32_t reserved;
+  /* Optional (0 or less: unknown).  An upper bound of every kv_b_seq_len; steers the same choice as total_kv_rows, and like it
+   * costs time at most. */
+  int32_t max_kv_len;
 } lsattn_prefill_args;
+
+/* Which kernel the step these arguments describe runs (by the numbers in the block and the tuning block; nothing is launched and
+ * no pointer followed).  Meant for tests and for reading profiles: the routes and where they change are the library's own. */
+enum {
+  LSATTN_ROUTE_INVALID = 0,      /* no such step */
+  LSATTN_ROUTE_SMALL_16 = 1,     /* heads of 16 to 64 and short prompts of 128-wide ones: 16 query positions per wave, */
+  LSATTN_ROUTE_SMALL_32 = 2,     /* 32, */
+  LSATTN_ROUTE_SMALL_TURNS = 3,  /* 32, the requests' places in the grid turning from tile to tile */
+  LSATTN_ROUTE_ROWS_256 = 4,     /* the 128-wide kernel: 256 query rows per workgroup, */
+  LSATTN_ROUTE_ROWS_128 = 5,     /* 128 over two waves per 32 rows, */
+  LSATTN_ROUTE_HALF = 6,         /* 128 in four waves, */
+  LSATTN_ROUTE_HALF_FOLDED = 7   /* the same, the second half of the grid backwards */
+};
+int lsattn_prefill_route(const lsattn_prefill_args* a);
 
 /* 1 if the step these arguments describe (v_is_f16 = 0) converts a bfloat16 V on its way into LDS at no cost, as the kernels
  * for head sizes below 128 and for batches of short prompts do; 0 if the caller should make an fp16 copy of V first
@@ -561,8 +577,8 @@ const char* lsattn_strerror(int code);
  * kv_cuts / kv_cut_len / o_cut_rows / total_q_rows in lsattn_prefill_args, lsattn_prefill_merge_cuts; 4 = dest_index of
  * lsattn_rotary_kv_write_args untyped, its slots int32 or int64 by dest_index_is_i64 (a reserved word before), lsattn_kv_scatter_i64,
  * the counts of lsattn_pool_update_refs also in pinned host memory and, past LSATTN_POOL_REFS_ORDERED entries, not behind the state; 5 = total_kv_rows and kv_cut_even in lsattn_prefill_args,
- * lsattn_prefill_converts_v. */
-#define LSATTN_VERSION 5
+ * lsattn_prefill_converts_v; 6 = max_kv_len there (a reserved word before), lsattn_prefill_route. */
+#define LSATTN_VERSION 6
 int lsattn_version(void);
 
 #ifdef __cplusplus

@@ -40,7 +40,7 @@ class PrefillArgs(C.Structure):
         ("ml_stride_t", _i64), ("ml_stride_h", _i64),
         ("o_b_start_loc", _vp),
         ("kv_cuts", _i32), ("kv_cut_len", _i32), ("o_cut_rows", _i64), ("total_q_rows", _i64),
-        ("total_kv_rows", _i64), ("kv_cut_even", _i32), ("reserved", _i32),
+        ("total_kv_rows", _i64), ("kv_cut_even", _i32), ("max_kv_len", _i32),
     ]
 
 
@@ -96,7 +96,7 @@ TUNING_VALUES = {
     "decode_stage1": {None: 0, "lane": 1, "mfma": 2, "split": 3},
     "decode_listed": {None: 0, "off": 1, "on": 2, "shares": 3},
 }
-LSATTN_VERSION = 5  # of include/lsattn.h, which the argument blocks above mirror
+LSATTN_VERSION = 6  # of include/lsattn.h, which the argument blocks above mirror
 
 
 # every symbol include/lsattn.h declares: name -> (restype, argtypes)
@@ -155,6 +155,7 @@ EXPORTS = {
     "lsattn_pool_refs_workspace_bytes": (C.c_size_t, [_i64]),
     "lsattn_pool_update_refs": (C.c_int, [_vp, _i64, _vp, _i64, C.c_int, _vp, _vp, C.c_size_t, _vp]),
     "lsattn_prefill_converts_v": (C.c_int, [C.POINTER(PrefillArgs)]),
+    "lsattn_prefill_route": (C.c_int, [C.POINTER(PrefillArgs)]),
     "lsattn_bf16_to_f16_rows": (C.c_int, [_vp, _i64, _vp, _i64, _i64, _i64, _vp]),
     "lsattn_set_tuning": (C.c_int, [C.POINTER(Tuning)]),
     "lsattn_strerror": (C.c_char_p, [C.c_int]),

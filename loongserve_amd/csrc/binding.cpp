@@ -14,6 +14,7 @@
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
 
+#include <algorithm>
 #include <chrono>
 #include <cmath>
 #include <cstring>
@@ -204,6 +205,7 @@ struct Step {
     p.total_kv_rows = k->size(0);
     return true;
   }
+  void keys_up_to(int64_t n) { p.max_kv_len = (int32_t)std::clamp<int64_t>(n, 0, INT32_MAX); }  // (0: the caller gave no bound)
   bool state(const at::Tensor& o) {  // where the result goes
     if (o.stride(2) != 1) return false;
     p.o = o.data_ptr(), p.o_stride_t = o.stride(0), p.o_stride_h = o.stride(1), p.o_dtype = dtype_of(o);
@@ -242,10 +244,10 @@ struct Step {
   }
 };
 
-// (q, k, v, o, six vectors, peers, max_q, m, l, total_q, cuts, kv_rows, workspace, preconvert) -> True or None
+// (q, k, v, o, six vectors, peers, max_q, m, l, total_q, cuts, kv_rows, workspace, preconvert, max_kv) -> True or None
 PyObject* context_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
-  NEED_ARGS(19);
+  NEED_ARGS(20);
   Args in(args);
   const at::Tensor &q = in.gpu(3), &k = in.gpu(3), &v = in.gpu(3), &o = in.gpu(3);
   OR_NONE(in.ok);
@@ -257,6 +259,7 @@ PyObject* context_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
   const int64_t kv_rows = in.integer();
   const at::Tensor* ws = in.maybe();
   const bool preconvert = in.integer() != 0;
+  s.keys_up_to(in.integer());
   OR_NONE(in.ok && total >= 0 && is(m, at::kFloat) && is(l, at::kFloat) && m.strides() == l.strides() && same_shape(m, l));
   OR_NONE(m.size(0) == q.size(0) && m.size(1) == q.size(1));
   s.p.m = (float*)m.data_ptr(), s.p.l = (float*)l.data_ptr(), s.p.ml_stride_t = m.stride(0), s.p.ml_stride_h = m.stride(1);
@@ -284,11 +287,11 @@ PyObject* context_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
   END_HANDLE_TH_ERRORS
 }
 
-// (q, k, v, six vectors, peers, max_q, out, lse, sm_scale or None, accumulate, total_q, cuts, kv_rows, workspace, preconvert)
+// (q, k, v, six vectors, peers, max_q, out, lse, sm_scale or None, accumulate, total_q, cuts, kv_rows, workspace, preconvert, max_kv)
 // -> (out, lse) or None
 PyObject* prefill_partial(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
-  NEED_ARGS(20);
+  NEED_ARGS(21);
   Args in(args);
   const at::Tensor &q = in.gpu(3), &k = in.gpu(3), &v = in.gpu(3);
   OR_NONE(in.ok);
@@ -302,6 +305,7 @@ PyObject* prefill_partial(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const int64_t total = in.integer(), S = in.integer(), kv_rows = in.integer();
   const at::Tensor* ws = in.maybe();
   const bool preconvert = in.integer() != 0;
+  s.keys_up_to(in.integer());
   OR_NONE(in.ok && total >= 0 && S <= LSATTN_MAX_KV_CUTS);
   OR_NONE(!accumulate || (out_in && lse_in));
   s.p.total_q_rows = total;

@@ -101,6 +101,8 @@ Tuning tuning();
 int launch_prefill_small(const lsattn_prefill_args* a, int mode, hipStream_t st);
 // Blocks of 16 query positions per wave (1 or 2) with which that kernel takes this step of 128-wide heads; 0: it does not.
 int prefill_short_blocks(const lsattn_prefill_args* a);
+// LSATTN_ROUTE_SMALL_* of a step that runs it.
+int prefill_small_route(const lsattn_prefill_args* a);
 
 // check_launch reports what the launch in front of it left in the host thread's last-error slot, so every launch first
 // empties that slot: an earlier runtime call of the host program may have left something there that is not this

@@ -1264,8 +1264,11 @@ static int launch_prefill_rows(const lsattn_prefill_args* a, bool tile_major, co
 // and 4096 tokens the head-by-head order leaves a CU with tiles 9 and 16 of 16 and takes 160 us where the other takes 128.
 // lsattn_set_tuning overrides both choices (tuning and tests).  The size counts workgroups as they are launched: with the query heads of a KV head side by side
 // (pack_shift_for) a workgroup covers 256 >> pack_shift positions of 1 << pack_shift heads.
-template <typename T, int MODE, bool DV> static int launch_prefill(const lsattn_prefill_args* a, hipStream_t st) {
-  const Tuning tn = tuning();
+struct Shape {
+  int route;  // LSATTN_ROUTE_*
+  bool tile_major;
+};
+static Shape choose_shape(const lsattn_prefill_args* a, bool dv, const Tuning& tn) {
   const int64_t nz256 = (a->max_q_len + BM - 1) / BM;
   const int ps = pack_shift_for(a, false, tn);  // (the workgroups of several heads are shorter: less padding past a short chunk)
   const int64_t cuts = a->kv_cuts > 1 ? a->kv_cuts : 1;
@@ -1280,46 +1283,54 @@ template <typename T, int MODE, bool DV> static int launch_prefill(const lsattn_
   bool tile_major = wgs256 < kTileMajorBelowWorkgroups;
   if (tn.prefill_order == LSATTN_PREFILL_ORDER_TILE) tile_major = true;
   if (tn.prefill_order == LSATTN_PREFILL_ORDER_HEAD) tile_major = false;
-  if constexpr (!DV) {
-    return launch_prefill_rows<T, MODE, false, false>(a, tile_major, tn, st);
-  } else {
-    bool split = wgs256 <= kCUs / 2 || (wgs256 <= kCUs && nz256 >= 5);
-    // Short chunks that a 256-row workgroup pads much further than a 128-row one (100 rows of one head: 256 against 128): the
-    // 128-row shapes walk the same tiles for at most four fifths of the rows (100 rows x 131072 keys in 15 cuts, MHA 32:
-    // 507 -> 376 us).  Per row and tile they are 5 to 10 % behind the 256-row shape, hence the margin.
-    {
-      // (query positions the longest chunk is padded to; the heads side by side in a workgroup cancel out)
-      const int64_t padded256 = ((a->max_q_len + (BM >> ps) - 1) / (BM >> ps)) * (BM >> ps);
-      const int ph0 = pack_shift_for(a, true, tn);
-      const int64_t padded128 = ((a->max_q_len + (BM / 2 >> ph0) - 1) / (BM / 2 >> ph0)) * (BM / 2 >> ph0);
-      if (padded128 * 5 <= padded256 * 4) split = true;
-    }
-    // The four-wave shape (two workgroups per CU) for chunks of up to 1024 rows (1536 with one head per workgroup),
-    // whose workgroups walk a few tiles each and spend as long starting and ending as working, from three workgroups
-    // per CU on: 3 to 17 % shorter launches on batches of 4 to 32 requests of 128 to 1536 tokens.  Smaller launches keep
-    // the shapes above: with at most a pair of these workgroups per CU a launch of short chunks would gain as much, but
-    // one of short chunks against long K/V (which the host cannot tell apart) would run on half the CUs.  Not for
-    // launches that write their rows elsewhere either (the step cut along the keys: few, long workgroups).
-    const int ph = pack_shift_for(a, true, tn);
-    const int64_t wgs128 = cuts * (a->num_q_heads >> ph) * tiles_of(BM / 2 >> ph);
-    bool half = a->max_q_len <= (ph ? 1024 : 1536) && !a->o_b_start_loc && a->kv_cuts <= 1 && wgs128 >= 3 * kCUs;
-    if (tn.prefill_rows == LSATTN_PREFILL_ROWS_128) split = true, half = false;
-    if (tn.prefill_rows == LSATTN_PREFILL_ROWS_256) split = false, half = false;
-    if (tn.prefill_rows == LSATTN_PREFILL_ROWS_HALF) half = true;
-    // One request whose four-wave workgroups all fit the chip at once, more than one and at most two per CU (a single
-    // sequence of up to 2048 tokens: 32 heads x sixteen 128-row tiles): the four-wave shape with the second half of the
-    // grid running backwards (see the kernel), each CU one heavy and one light workgroup side by side, instead of the
-    // split shape's two rounds.  Longer chunks keep the rules above (the pairs' work is then long against what a
-    // workgroup costs besides its tiles, and the shape's rings of two tiles are the slower ones per tile).
-    // (measured, one sequence, MHA 32: 2048 tokens = 512 workgroups 45.7 us against 47.1 split and 47.3 unfolded; 1792 tokens
-    // = 448 39.6 against 40.5; 1536 = 384 34.2 against 33.5 and 1280 = 320 29.7 against 27.4: the fold pays from seven
-    // eighths of two workgroups per CU on, below that the split shape's two rounds do)
-    const bool fold = a->batch == 1 && cuts == 1 && !a->o_b_start_loc && a->max_q_len <= 2048 && wgs128 * 8 >= 7 * 2 * kCUs &&
-                      wgs128 <= 2 * kCUs && tn.prefill_rows == 0;
-    if (fold) return launch_prefill_rows<T, MODE, true, false, true>(a, true, tn, st, true);
-    if (half) return launch_prefill_rows<T, MODE, true, false, true>(a, true, tn, st);
-    return split ? launch_prefill_rows<T, MODE, true, true>(a, true, tn, st) : launch_prefill_rows<T, MODE, true, false>(a, tile_major, tn, st);
+  if (!dv) return {LSATTN_ROUTE_ROWS_256, tile_major};
+  bool split = wgs256 <= kCUs / 2 || (wgs256 <= kCUs && nz256 >= 5);
+  // Short chunks that a 256-row workgroup pads much further than a 128-row one (100 rows of one head: 256 against 128): the
+  // 128-row shapes walk the same tiles for at most four fifths of the rows (100 rows x 131072 keys in 15 cuts, MHA 32:
+  // 507 -> 376 us).  Per row and tile they are 5 to 10 % behind the 256-row shape, hence the margin.
+  {
+    // (query positions the longest chunk is padded to; the heads side by side in a workgroup cancel out)
+    const int64_t padded256 = ((a->max_q_len + (BM >> ps) - 1) / (BM >> ps)) * (BM >> ps);
+    const int ph0 = pack_shift_for(a, true, tn);
+    const int64_t padded128 = ((a->max_q_len + (BM / 2 >> ph0) - 1) / (BM / 2 >> ph0)) * (BM / 2 >> ph0);
+    if (padded128 * 5 <= padded256 * 4) split = true;
   }
+  // The four-wave shape (two workgroups per CU) for chunks of up to 1024 rows (1536 with one head per workgroup),
+  // whose workgroups walk a few tiles each and spend as long starting and ending as working, from three workgroups
+  // per CU on: 3 to 17 % shorter launches on batches of 4 to 32 requests of 128 to 1536 tokens.  Smaller launches keep
+  // the shapes above: with at most a pair of these workgroups per CU a launch of short chunks would gain as much, but
+  // one of short chunks against long K/V (which the host cannot tell apart) would run on half the CUs.  Not for
+  // launches that write their rows elsewhere either (the step cut along the keys: few, long workgroups).
+  const int ph = pack_shift_for(a, true, tn);
+  const int64_t wgs128 = cuts * (a->num_q_heads >> ph) * tiles_of(BM / 2 >> ph);
+  bool half = a->max_q_len <= (ph ? 1024 : 1536) && !a->o_b_start_loc && a->kv_cuts <= 1 && wgs128 >= 3 * kCUs;
+  if (tn.prefill_rows == LSATTN_PREFILL_ROWS_128) split = true, half = false;
+  if (tn.prefill_rows == LSATTN_PREFILL_ROWS_256) split = false, half = false;
+  if (tn.prefill_rows == LSATTN_PREFILL_ROWS_HALF) half = true;
+  // One request whose four-wave workgroups all fit the chip at once, more than one and at most two per CU (a single
+  // sequence of up to 2048 tokens: 32 heads x sixteen 128-row tiles): the four-wave shape with the second half of the
+  // grid running backwards (see the kernel), each CU one heavy and one light workgroup side by side, instead of the
+  // split shape's two rounds.  Longer chunks keep the rules above (the pairs' work is then long against what a
+  // workgroup costs besides its tiles, and the shape's rings of two tiles are the slower ones per tile).
+  // (measured, one sequence, MHA 32: 2048 tokens = 512 workgroups 45.7 us against 47.1 split and 47.3 unfolded; 1792 tokens
+  // = 448 39.6 against 40.5; 1536 = 384 34.2 against 33.5 and 1280 = 320 29.7 against 27.4: the fold pays from seven
+  // eighths of two workgroups per CU on, below that the split shape's two rounds do)
+  const bool fold = a->batch == 1 && cuts == 1 && !a->o_b_start_loc && a->max_q_len <= 2048 && wgs128 * 8 >= 7 * 2 * kCUs &&
+                    wgs128 <= 2 * kCUs && tn.prefill_rows == 0;
+  if (fold) return {LSATTN_ROUTE_HALF_FOLDED, true};
+  if (half) return {LSATTN_ROUTE_HALF, true};
+  return split ? Shape{LSATTN_ROUTE_ROWS_128, true} : Shape{LSATTN_ROUTE_ROWS_256, tile_major};
+}
+
+template <typename T, int MODE, bool DV> static int launch_prefill(const lsattn_prefill_args* a, hipStream_t st) {
+  const Tuning tn = tuning();
+  const Shape shape = choose_shape(a, DV, tn);
+  if constexpr (DV) {
+    if (shape.route == LSATTN_ROUTE_HALF_FOLDED) return launch_prefill_rows<T, MODE, true, false, true>(a, true, tn, st, true);
+    if (shape.route == LSATTN_ROUTE_HALF) return launch_prefill_rows<T, MODE, true, false, true>(a, true, tn, st);
+    if (shape.route == LSATTN_ROUTE_ROWS_128) return launch_prefill_rows<T, MODE, true, true>(a, true, tn, st);
+  }
+  return launch_prefill_rows<T, MODE, DV, false>(a, shape.tile_major, tn, st);
 }
 
 static int validate(const lsattn_prefill_args* a, int mode) {
@@ -1385,4 +1396,11 @@ extern "C" int lsattn_prefill_step_accumulate(const lsattn_prefill_args* a, void
   if (a->head_dim != 128 || prefill_short_blocks(a)) return launch_prefill_small(a, 2, (hipStream_t)stream);
   if (a->dtype == LSATTN_F16) return launch_prefill<F16, 2, true>(a, (hipStream_t)stream);
   return a->v_is_f16 ? launch_prefill<BF16, 2, true>(a, (hipStream_t)stream) : launch_prefill<BF16, 2, false>(a, (hipStream_t)stream);
+}
+
+extern "C" int lsattn_prefill_route(const lsattn_prefill_args* a) {
+  if (!a || a->num_q_heads <= 0 || a->num_kv_heads <= 0 || a->num_q_heads % a->num_kv_heads || a->batch <= 0 || a->max_q_len <= 0) return LSATTN_ROUTE_INVALID;
+  if (a->head_dim != 128 && a->head_dim != 64 && a->head_dim != 32 && a->head_dim != 16) return LSATTN_ROUTE_INVALID;
+  if (a->head_dim != 128 || prefill_short_blocks(a)) return prefill_small_route(a);
+  return choose_shape(a, a->dtype == LSATTN_F16 || a->v_is_f16, tuning()).route;
 }

@@ -102,7 +102,7 @@ constexpr int kTile = 64;   // keys per LDS tile
 constexpr uint32_t kOnes = 0x3C003C00u;  // two ones in fp16
 constexpr int64_t kCUs = 256;
 constexpr int32_t kShortMaxRows = 768;    // 128-wide heads: the longest query chunk this kernel takes
-constexpr int64_t kShortMeanKeys = 1024;  // and the keys per request up to which it does
+constexpr int64_t kShortMaxKeys = 1024;   // and the keys up to which it does, of the longest request
 constexpr int64_t kMaxTiles = 65535;  // tiles of one launch (the third index of a grid)
 
 // s_waitcnt vmcnt(0) (expcnt / lgkmcnt fields left at their maximum)
@@ -496,14 +496,15 @@ int64_t workgroups(const lsattn_prefill_args* a, int pack_shift, int blocks) {
 // 92.8 | 99.3, 2048 43.9 | 48.6, 4096 170 | 200.
 template <typename T, int D, int MODE, bool DV> int launch(const SmallParams& p, const lsattn_prefill_args* a, hipStream_t st) {
   if (a->num_q_heads > 65535 || a->batch > 65535) return LSATTN_ERR_INVALID_ARG;
-  if (workgroups(a, p.pack_shift, 2) < 3 * kCUs) return launch_rows<T, D, MODE, DV, 1>(p, a, st);  // (all at once on the chip)
-  const int64_t rows_wg = (kWaves * 2 * 16) >> p.pack_shift;
-  return requests_take_turns(a, (int64_t)p.hkv * p.group, (a->max_q_len + rows_wg - 1) / rows_wg)
-             ? launch_rows<T, D, MODE, DV, 2, true>(p, a, st) : launch_rows<T, D, MODE, DV, 2>(p, a, st);
+  switch (prefill_small_route(a)) {
+    case LSATTN_ROUTE_SMALL_16: return launch_rows<T, D, MODE, DV, 1>(p, a, st);
+    case LSATTN_ROUTE_SMALL_TURNS: return launch_rows<T, D, MODE, DV, 2, true>(p, a, st);
+    default: return launch_rows<T, D, MODE, DV, 2>(p, a, st);
+  }
 }
 
 template <typename T, int MODE, bool DV> int launch_128(const SmallParams& p, const lsattn_prefill_args* a, hipStream_t st) {
-  return prefill_short_blocks(a) == 1 ? launch_rows<T, 128, MODE, DV, 1>(p, a, st) : launch_rows<T, 128, MODE, DV, 2>(p, a, st);
+  return prefill_small_route(a) == LSATTN_ROUTE_SMALL_16 ? launch_rows<T, 128, MODE, DV, 1>(p, a, st) : launch_rows<T, 128, MODE, DV, 2>(p, a, st);
 }
 
 template <typename T, int MODE, bool DV> int launch_d(const SmallParams& p, const lsattn_prefill_args* a, hipStream_t st) {
@@ -539,12 +540,25 @@ template <typename T, bool DV> int launch_mode(const SmallParams& p, const lsatt
 // 16 positions per wave win up to two and a half workgroups per CU (with one head per workgroup, which leaves the other kernel
 // four times the rows to mask, up to six, for prompts of up to 512 tokens), 32 up to six and 256 tokens; the geometric
 // mean over the launches the rule takes is 25 to 35 % below the other kernel, the worst is 5 % above it.
-// The keys: a tile of 64 costs a wave 0.95 us here (bf16 V 1.15) against 0.86, so short chunks behind a long context, which the
-// host cannot tell from prompts by the query lengths alone, stay with the other kernel: total_kv_rows has to be known.
+// The keys: a tile of 64 costs a wave 0.95 us here (bf16 V 1.5) against 0.56 in the 128-row shape, which a launch with one long
+// context waits for, so the longest request decides (whole call, 32/8 heads, the other kernel | this one, f16, then bf16):
+//   8 x 64 rows behind 600 keys each 20.8 | 15.7, 28.0 | 18.7      4 x 100 behind 1000 each 24.9 | 21.7, 30.5 | 25.9      1 x 200 behind 1024 22.1 | 19.8, 25.2 | 24.0
+//   2 x 100, one behind 1900 30.6 | 31.8, 34.5 | 39.8      8 x 64, one behind 7500 79.8 | 108.8, 88 | 169      16 x 64, one behind 15000 145 | 264, 155 | 352
+// The host knows no lengths, only bounds: what total_kv_rows holds beyond the query rows may all belong to one request.
 int prefill_short_blocks(const lsattn_prefill_args* a) {
-  if (a->head_dim != 128 || a->kv_cuts > 1 || a->o_b_start_loc || a->max_q_len > kShortMaxRows || a->total_kv_rows <= 0 || a->batch <= 0 ||
-      a->total_kv_rows > (int64_t)a->batch * kShortMeanKeys || a->num_kv_heads <= 0)
+  if (a->head_dim != 128 || a->kv_cuts > 1 || a->o_b_start_loc || a->max_q_len <= 0 || a->max_q_len > kShortMaxRows || a->batch <= 0 || a->num_kv_heads <= 0)
     return 0;
+  int64_t longest = kShortMaxKeys + 1;
+  if (a->total_kv_rows > 0) {
+    longest = a->total_kv_rows;
+    if (a->total_q_rows > 0) {
+      const int64_t most = (int64_t)a->batch * a->max_q_len, rows = a->total_q_rows < most ? a->total_q_rows : most;
+      const int64_t beyond = a->total_kv_rows > rows ? a->total_kv_rows - rows : 0;
+      if (a->max_q_len + beyond < longest) longest = a->max_q_len + beyond;
+    }
+  }
+  if (a->max_kv_len > 0 && a->max_kv_len < longest) longest = a->max_kv_len;
+  if (longest > kShortMaxKeys) return 0;
   const Tuning tn = tuning();
   if (tn.prefill_rows || tn.prefill_order || tn.prefill_pack) return 0;  // (choices among the 128-wide kernel's shapes)
   const int pack = pack_shift_of(a);
@@ -553,7 +567,15 @@ int prefill_short_blocks(const lsattn_prefill_args* a) {
   return a->max_q_len <= 256 && two <= 6 * kCUs ? 2 : 0;
 }
 
-// One prefill step with head_dim 16, 32 or 64 (arguments already validated; epilogue `mode` as in the 128-wide kernel).
+int prefill_small_route(const lsattn_prefill_args* a) {
+  if (a->head_dim == 128) return prefill_short_blocks(a) == 1 ? LSATTN_ROUTE_SMALL_16 : LSATTN_ROUTE_SMALL_32;
+  const int pack = pack_shift_of(a);
+  if (workgroups(a, pack, 2) < 3 * kCUs) return LSATTN_ROUTE_SMALL_16;
+  const int64_t rows_wg = (kWaves * 2 * 16) >> pack;
+  return requests_take_turns(a, a->num_q_heads >> pack, (a->max_q_len + rows_wg - 1) / rows_wg) ? LSATTN_ROUTE_SMALL_TURNS : LSATTN_ROUTE_SMALL_32;
+}
+
+// One prefill step with head_dim 16, 32 or 64, or a short one with 128 (arguments already validated; epilogue `mode` as in the 128-wide kernel).
 int launch_prefill_small(const lsattn_prefill_args* a, int mode, hipStream_t st) {
   SmallParams p;
   p.q = a->q;

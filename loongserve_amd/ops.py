@@ -90,10 +90,15 @@ def _v_as_f16(v: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tens
 KERNEL_HEAD_DIM = 128  # the tuned kernel's head size (and the only one whose KV chunks are cut); 16, 32 and 64, and short prompts, take prefill_small_kernel
 
 
+def _keys_up_to(max_kv_len: Optional[int]) -> int:
+    return 0 if max_kv_len is None else min(max(int(max_kv_len), 0), 2 ** 31 - 1)
+
+
 def _prefill_args(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first, kv_b_start_loc, kv_b_seq_len, kv_first,
                   peers: int, max_q_len: int, sm_scale: Optional[float], v_f16: Optional[torch.Tensor] = None,
                   v_f16_valid: bool = False, o_b_start_loc: Optional[torch.Tensor] = None,
-                  cuts: Optional[Tuple[int, int, int]] = None, total_q_len: Optional[int] = None) -> _lib.PrefillArgs:
+                  cuts: Optional[Tuple[int, int, int]] = None, total_q_len: Optional[int] = None,
+                  max_kv_len: Optional[int] = None) -> _lib.PrefillArgs:
     for t, n in ((q, "q"), (k, "k"), (v, "v"), (o, "o")):
         _dev(t, n)
         if t.dim() != 3:
@@ -144,6 +149,7 @@ def _prefill_args(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first, kv_b_start_lo
             raise ValueError("total_q_len must be >= 0")
         a.total_q_rows = int(total_q_len)
     a.total_kv_rows = k.shape[0]
+    a.max_kv_len = _keys_up_to(max_kv_len)
     if q.dtype == torch.bfloat16 and (v_f16 is not None or (PRECONVERT_BF16_V and Lq == KERNEL_HEAD_DIM)):
         if v_f16_valid and (v_f16 is None or v_f16.dtype != torch.float16 or v_f16.shape != v.shape or v_f16.stride(2) != 1):
             raise ValueError("v_f16_valid needs v_f16, the float16 copy of v")
@@ -316,6 +322,9 @@ def context_attention_fwd(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first_token_
     sized for the longest batch), capped by what the workspace holds; kv_splits forces it.  Without a workspace the call
     is the reference's: one launch, no scratch.  (m, l) stay opaque: a step folded this way enters as (its LSE, 1).
 
+    Keyword-only: max_kv_len also tells a batch of short chunks behind short contexts from one with a long context among them; up to
+    1024 keys a kernel of shorter workgroups runs (without it only where the rows of k and total_q_len, or the rows of k alone, prove as much).
+
     Keyword-only, for batches that mix long and short requests: total_q_len, an upper bound of the sum of q_b_seq_len
     (q.shape[0] when q is packed and no two sequences share rows).  The launch is sized by max_q_b_seq_len times the batch
     (RING:262), all the host knows; with the bound it is sized by the query tiles that can exist when those are at most half
@@ -332,7 +341,8 @@ def context_attention_fwd(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first_token_
             cuts = kv_splits if kv_splits is not None else _choose_cuts(q, k, q_b_seq_len.shape[0], max_q_b_seq_len, max_kv_len, workspace)
         if _native.context_attention(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first_token_global_idx, kv_b_start_loc,
                                      kv_b_seq_len, kv_first_token_global_idx, logical_sp_peers_num, max_q_b_seq_len, m, l,
-                                     0 if total_q_len is None else total_q_len, cuts, kv_rows, workspace, PRECONVERT_BF16_V):
+                                     0 if total_q_len is None else total_q_len, cuts, kv_rows, workspace, PRECONVERT_BF16_V,
+                                     _keys_up_to(max_kv_len)):
             return
     _context_attention_checked(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first_token_global_idx, kv_b_start_loc, kv_b_seq_len,
                                kv_first_token_global_idx, logical_sp_peers_num, max_q_b_seq_len, m, l, v_f16, v_f16_valid,
@@ -372,7 +382,7 @@ def _context_attention_checked(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first_t
         return
     a = _prefill_args(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first_token_global_idx, kv_b_start_loc,
                       kv_b_seq_len, kv_first_token_global_idx, logical_sp_peers_num, max_q_b_seq_len,
-                      1.0 / (D ** 0.5), v_f16, v_f16_valid, total_q_len=total_q_len)
+                      1.0 / (D ** 0.5), v_f16, v_f16_valid, total_q_len=total_q_len, max_kv_len=max_kv_len)
     a.m, a.l = m.data_ptr(), l.data_ptr()
     a.ml_stride_t, a.ml_stride_h = m.stride(0), m.stride(1)
     _lib.check(_lib.load().lsattn_prefill_step_merge(C.byref(a), _stream()), "lsattn_prefill_step_merge")
@@ -411,7 +421,7 @@ def prefill_attention_step(q, k, v, q_b_start_loc, q_b_seq_len, q_first_token_gl
         done = _native.prefill_partial(q, k, v, q_b_start_loc, q_b_seq_len, q_first_token_global_idx, kv_b_start_loc, kv_b_seq_len,
                                        kv_first_token_global_idx, logical_sp_peers_num, max_q_b_seq_len, out, lse, sm_scale,
                                        accumulate, 0 if total_q_len is None else total_q_len, cuts, kv_rows, kv_split_workspace,
-                                       PRECONVERT_BF16_V)
+                                       PRECONVERT_BF16_V, _keys_up_to(max_kv_len))
         if done is not None:
             return done
     return _prefill_attention_step_checked(q, k, v, q_b_start_loc, q_b_seq_len, q_first_token_global_idx, kv_b_start_loc,
@@ -458,7 +468,7 @@ def _prefill_attention_step_checked(q, k, v, q_b_start_loc, q_b_seq_len, q_first
         return out, lse
     a = _prefill_args(q, k, v, out, q_b_start_loc, q_b_seq_len, q_first_token_global_idx, kv_b_start_loc,
                       kv_b_seq_len, kv_first_token_global_idx, logical_sp_peers_num, max_q_b_seq_len, sm_scale,
-                      v_f16, v_f16_valid, total_q_len=total_q_len)
+                      v_f16, v_f16_valid, total_q_len=total_q_len, max_kv_len=max_kv_len)
     a.lse = lse.data_ptr()
     if accumulate:
         _lib.check(_lib.load().lsattn_prefill_step_accumulate(C.byref(a), _stream()), "lsattn_prefill_step_accumulate")

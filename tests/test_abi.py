@@ -341,3 +341,46 @@ def test_cuts_are_bounded_by_the_memory_for_their_parts():
         assert _choose_cuts(q, k, 1, 64, 8191, None) == 1
         assert _choose_cuts(q, k, 0, 64, None, None) == 1
     assert _choose_cuts(torch.empty((4096, 32, 128), device="meta"), k, 8, 4096, None, None) == 1
+
+
+def _route(batch, max_q, heads, head_dim=128, total_q=0, total_kv=0, max_kv=0, dtype=0, v_is_f16=0, cuts=0):
+    from loongserve_amd import _lib
+    a = _lib.PrefillArgs()
+    a.batch, a.max_q_len, a.head_dim, a.dtype, a.v_is_f16, a.kv_cuts = batch, max_q, head_dim, dtype, v_is_f16, cuts
+    a.num_q_heads, a.num_kv_heads = heads
+    a.total_q_rows, a.total_kv_rows, a.max_kv_len = total_q, total_kv, max_kv
+    return _lib.load().lsattn_prefill_route(C.byref(a))
+
+
+SMALL_16, SMALL_32, SMALL_TURNS, ROWS_256, ROWS_128, HALF, HALF_FOLDED = range(1, 8)
+
+
+def test_short_prompts_kernel_goes_by_the_longest_request():
+    """The kernel of short prompts runs where no request can have more than 1024 keys: what the K buffer holds beyond the query rows may
+    all belong to one request, unless the caller bounds the lengths (16 requests of 64 rows, one behind 15000 keys: 145 -> 264 us in it)."""
+    heads = (32, 8)
+    assert _route(1, 100, (32, 32), total_q=100, total_kv=100) == SMALL_16
+    assert _route(16, 64, heads, total_q=1024, total_kv=1024) == SMALL_16
+    assert _route(16, 64, heads, total_q=1024, total_kv=15960) == ROWS_128
+    assert _route(8, 64, heads, total_q=512, total_kv=448 + 7500) == ROWS_128
+    assert _route(2, 100, heads, total_q=200, total_kv=2000) == ROWS_128  # (one of them behind 1900)
+    assert _route(2, 100, heads, total_q=4096, total_kv=2000) == ROWS_128  # (a loose bound of the rows proves nothing)
+    assert _route(8, 64, heads, total_q=512, total_kv=4800) == ROWS_128
+    assert _route(8, 64, heads, total_q=512, total_kv=4800, max_kv=600) == SMALL_16
+    assert _route(8, 64, heads, total_q=512, max_kv=1024) == SMALL_16
+    assert _route(8, 64, heads, total_q=512, max_kv=1025) == ROWS_128
+    assert _route(8, 64, heads, total_kv=1024) == SMALL_16 and _route(8, 64, heads, total_kv=1025) == ROWS_128
+    assert _route(8, 64, heads) == _route(8, 64, heads, total_q=512) == ROWS_128  # (nothing known of the keys)
+    assert _route(1, 768, heads, total_q=768, total_kv=1024) == SMALL_16 and _route(1, 768, heads, total_q=768, total_kv=1025) == ROWS_128
+    assert _route(1, 769, heads, total_q=769, total_kv=769) == ROWS_128
+
+
+def test_prefill_route_names_a_kernel_for_every_step_and_none_for_others():
+    assert _route(24, 256, (32, 32), total_q=1800, total_kv=1800) == SMALL_32
+    assert _route(8, 3000, (32, 8), 64, total_q=16000, total_kv=16000) == SMALL_TURNS
+    assert _route(8, 3000, (32, 8), 64, total_q=24000) == _route(8, 3000, (32, 8), 64) == SMALL_32
+    assert _route(1, 100, (32, 32), 16) == SMALL_16
+    assert _route(1, 2048, (32, 32)) == HALF_FOLDED and _route(16, 1024, (32, 8)) == HALF
+    assert _route(1, 16384, (32, 32)) == ROWS_256 and _route(1, 500, (32, 8), cuts=2) == ROWS_128 and _route(1, 500, (32, 8), cuts=3) == ROWS_256
+    assert _route(1, 100, (32, 8), dtype=1) == ROWS_256 and _route(1, 100, (32, 8), dtype=1, v_is_f16=1) == ROWS_128
+    assert _route(0, 100, (32, 8)) == _route(1, 0, (32, 8)) == _route(1, 100, (32, 0)) == _route(1, 100, (32, 5)) == _route(1, 100, (32, 8), 80) == 0

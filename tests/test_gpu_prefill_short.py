@@ -75,3 +75,22 @@ def test_v_f16_valid_needs_the_copy_whatever_kernel_runs(lsa, rows):
     got = lsa.prefill_attention_step(q, k, v, *md, *md, 1, rows, v_f16=v.half(), v_f16_valid=True)
     torch.cuda.synchronize()
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_short_rows_behind_one_long_context_and_bounded_ones(lsa, dtype):
+    """A batch of short chunks of which one has a long context (the 128-wide kernel) and one whose contexts the caller bounds (the
+    kernel of short prompts), through the native pass and the checked one."""
+    for lens, ctx, bound in [([64, 33, 64, 1], [0, 2500, 0, 7], None), ([64, 33, 64, 1], [700, 900, 0, 960], 961)]:
+        klens = [n + c for n, c in zip(lens, ctx)]
+        T = sum(lens)
+        q, kv = rand_t((T, 8, 128), 91, dtype), rand_t((sum(klens), 4, 128), 92, dtype)
+        qm, km = meta(lens, ctx), meta(klens)
+        o_ref, lse_ref = orc.attn_step(q, kv[:, :2].contiguous(), kv[:, 2:].contiguous(), *qm, *km, 1)
+        qd, kvd = q.to(DEV), kv.to(DEV)
+        k, v = kvd[:, :2], kvd[:, 2:]
+        for given in (bound, None if bound is None else torch.tensor(bound)):  # (a tensor goes through the checked pass)
+            o, lse = lsa.prefill_attention_step(qd, k, v, *_dev(*qm), *_dev(*km), 1, max(lens), total_q_len=T, max_kv_len=given)
+            torch.cuda.synchronize()
+            assert_o_close(o, o_ref, "O")
+            assert_lse_close(lse, lse_ref, "LSE")
