@@ -70,7 +70,8 @@ struct PrefillParams {
   float* m;
   float* l;
   int64_t ml_st, ml_sh;
-  int32_t spread;    // how many XCDs further the units of the next (sequence, cut) start
+  int32_t dense, head_bits;  // (cut launches) the grid numbers the units without gaps; log2 of the KV heads
+  int32_t spread;    // (cut launches with gaps) how many XCDs further the units of the next (sequence, cut) start
   int32_t cut_mask;  // 0: the cuts of a sequence share its own length, at most kv_cut_len keys each; else all bits: kv_cut_len keys
 };
 
@@ -222,6 +223,7 @@ __device__ __forceinline__ const char* uniform_ptr(const char* ptr) {
 // HALF: four waves and 128 query rows, 32 per wave and every key, with rings of two tiles (64 KB of LDS): two such
 // workgroups fit a CU, and one's start-up, finish and turn-over run beside the other's tiles.  For launches whose
 // workgroups are short (a few tiles each): there a workgroup that fills the CU spends as long starting and ending as working.
+// CUTS: a step cut along the keys (epilogue 0 only).
 // A 16-byte store that goes through to memory as it is issued (system-scope bits) instead of waiting in the L2 as a dirty
 // line until the end of the launch.  From inline assembly (the compiler has no such store that is not atomic); the
 // s_nop keeps vector instructions off the data registers for the two cycles a store of more than 64 bits needs.
@@ -229,7 +231,7 @@ __device__ __forceinline__ void store16_through(float* addr, const f32x4 v) {
   asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" : : "v"(addr), "v"(v) : "memory");
 }
 
-template <typename T, int MODE, bool DV, bool SPLIT, bool HALF = false>
+template <typename T, int MODE, bool DV, bool SPLIT, bool HALF, bool CUTS>
 __global__ __launch_bounds__(HALF ? NWAVE * 32 : NWAVE * 64, HALF ? 2 : 1) void prefill_kernel(PrefillParams p) {
   static_assert(DV || !SPLIT, "the split variant takes fp16 V tiles only");
   static_assert(!HALF || (DV && !SPLIT), "the four-wave variant takes fp16 V tiles only and is not split");
@@ -296,17 +298,34 @@ __global__ __launch_bounds__(HALF ? NWAVE * 32 : NWAVE * 64, HALF ? 2 : 1) void 
     }
     if (b < 0) return;  // past the last unit that exists
     cut = 0;
+  } else if (CUTS && p.dense) {
+    // A step cut along the keys is often one round of workgroups, and on 1, 2 or 4 KV heads the ids below leave gaps (units of a KV
+    // head that its slices do not divide evenly): workgroups that end at once but take their turn among the XCDs and, within one,
+    // among its four shader engines, so that some of these get a ninth workgroup for eight CUs and the launch a second round
+    // (300 rows x 40000 keys, 8/1 heads, 12 cuts, 240 units: 91 us with gaps, 58 without; 2 x 300 x 100000, 6 cuts: 359, 228).  Here every id has a unit; the heads
+    // run fastest, so a head stays on its XCDs.
+    const uint32_t n = blockIdx.x >> p.head_bits;
+    j = div_by(n, p.d_second);
+    const int unit = (int)(n - j * p.n_second);
+    up = unit >> (3 - p.head_bits);
+    xcd = (int)(blockIdx.x & ((1u << p.head_bits) - 1)) * p.slices + (unit & (p.slices - 1));
+    slot = 0;
+    b = (int)div_by(j, p.d_cuts);
+    cut = (int)j - b * p.kv_cuts;
   } else {
     j = div_by(j1, p.d_second);
     const int r2 = (int)(j1 - j * p.n_second);
     up = p.tile_major ? r2 : r1;
     slot = p.tile_major ? r1 : r2;
-    // (sequence, cut of its KV chunk): j < batch * kv_cuts for every workgroup of the grid
-    // (where a KV head's units are dealt to several XCDs, the units left over from whole rounds of them land on other XCDs from one
-    // (sequence, cut) to the next: a launch of 4 units x 48 cuts on one KV head used half the chip)
-    xcd = (xcd + (int)j * p.spread) & 7;
-    b = (int)div_by(j, p.d_cuts);
-    cut = (int)j - b * p.kv_cuts;
+    b = (int)j;  // (j < batch * kv_cuts for every workgroup of the grid)
+    cut = 0;
+    if (CUTS) {
+      // (where a KV head's units are dealt to several XCDs, the units left over from whole rounds of them land on other XCDs from one
+      // (sequence, cut) to the next)
+      xcd = (xcd + (int)j * p.spread) & 7;
+      b = (int)div_by(j, p.d_cuts);
+      cut = (int)j - b * p.kv_cuts;
+    }
   }
   // The request's six numbers, all requested before the first of them is used (one memory latency instead of three on
   // the way to the first tile load; a workgroup's start-up is what a short launch is made of).
@@ -314,14 +333,17 @@ __global__ __launch_bounds__(HALF ? NWAVE * 32 : NWAVE * 64, HALF ? 2 : 1) void 
   const int q_start32 = p.q_start[b], kv_start32 = p.kv_start[b];
   const int o_start32 = p.o_start ? p.o_start[b] : q_start32;
   asm volatile("" ::"s"(q_len), "s"(kv_len_all), "s"(qf), "s"(kf_all), "s"(q_start32), "s"(kv_start32), "s"(o_start32));
-  // the cut's share of the chunk: keys [cut, cut + 1) * kv_cut_len, key n of the chunk at global position kv_first + n * peers
-  // (or the sequence's own length over the cuts, in whole tiles; no branch here, where the parameters' loads are on their way:
-  // with one, launches without cuts took 0.3 us longer to start)
-  const int even = (((int)(__umulhi((uint32_t)((kv_len_all > 1 ? kv_len_all : 1) - 1), p.d_cuts.mul) >> p.d_cuts.shr) + BN) & -BN) | p.cut_mask;
-  const int cut_len = even < p.kv_cut_len ? even : p.kv_cut_len;
-  const int key0 = cut * cut_len;
-  const int kv_rest = kv_len_all - key0;
-  const int kv_len = kv_rest < 0 ? 0 : (kv_rest < cut_len ? kv_rest : cut_len);
+  // the cut's share of the chunk: keys [cut, cut + 1) * kv_cut_len, or as many of the sequence's own length over the cuts, in whole
+  // tiles; key n of the chunk is at global position kv_first + n * peers
+  int key0 = 0, kv_len = kv_len_all;
+  if (CUTS) {
+    const int even = (((int)(__umulhi((uint32_t)((kv_len_all > 1 ? kv_len_all : 1) - 1), p.d_cuts.mul) >> p.d_cuts.shr) + BN) & -BN) | p.cut_mask;
+    const int cut_len = even < p.kv_cut_len ? even : p.kv_cut_len;
+    key0 = cut * cut_len;
+    const int kv_rest = kv_len_all - key0;
+    kv_len = kv_rest < cut_len ? kv_rest : cut_len;
+  }
+  kv_len = kv_len < 0 ? 0 : kv_len;
   const int kf = kf_all + key0 * p.peers;
   const int64_t q_start = q_start32, kv_start = (int64_t)kv_start32 + key0, o_start = o_start32 + (int64_t)cut * p.o_cut_rows;
   const int vh = xcd + 8 * slot;  // (KV head, slice) pair: always < hkv * slices
@@ -1161,7 +1183,7 @@ static int pack_shift_for(const lsattn_prefill_args* a, bool split, const Tuning
   return s;
 }
 
-template <typename T, int MODE, bool DV, bool SPLIT, bool HALF = false>
+template <typename T, int MODE, bool DV, bool SPLIT, bool HALF, bool CUTS>
 static int launch_prefill_rows(const lsattn_prefill_args* a, bool tile_major, const Tuning& tn, hipStream_t st, bool fold = false) {
   constexpr int BMW = SPLIT || HALF ? BM / 2 : BM;
   PrefillParams p;
@@ -1206,7 +1228,6 @@ static int launch_prefill_rows(const lsattn_prefill_args* a, bool tile_major, co
   p.heads_per_kv = a->num_q_heads / a->num_kv_heads;
   const int group = p.heads_per_kv >> p.pack_shift;  // workgroups side by side over the heads of a KV head
   p.group = group;
-  p.spread = (int32_t)((int64_t)group * p.nz % p.slices);
   p.units_per_slice = (int32_t)(((int64_t)group * p.nz + p.slices - 1) / p.slices);
   p.d_group = fast_div((uint32_t)group);
   p.d_slices = fast_div((uint32_t)p.slices);
@@ -1225,10 +1246,22 @@ static int launch_prefill_rows(const lsattn_prefill_args* a, bool tile_major, co
   p.fold_from = p.fold_sum = 0;
   p.listed = 0;
   p.rows_shift = (SPLIT || HALF ? 7 : 8) - p.pack_shift;
+  // (1, 2 or 4 KV heads: all slots are one, and the slices a power of two.  Heads on eight XCDs leave no gaps; those that do otherwise, 3
+  // or 6 say, at least start elsewhere from one cut to the next)
+  const int64_t units = (int64_t)group * p.nz;
+  p.spread = CUTS ? (int32_t)(units % p.slices) : 0;
+  p.dense = CUTS && p.kv_slots == 1 && p.slices > 1;
+  p.head_bits = 0;
+  while (p.dense && (1 << p.head_bits) < a->num_kv_heads) p.head_bits++;
   // A grid of the units that can exist instead of one sized by the longest request (see the kernel), when the caller
   // bounds the rows of all requests together and that grid is at most half of the other: a skewed batch.  (One KV head
   // or slot per XCD index only, and no cuts along the keys.)
   int64_t wgs_launch = wgs;
+  if (p.dense) {
+    p.n_second = (int32_t)units;
+    p.d_second = fast_div((uint32_t)units);
+    wgs_launch = units * a->num_kv_heads * a->batch * p.kv_cuts;
+  }
   if (a->total_q_rows > 0 && p.slices == 1 && p.kv_cuts == 1 && a->batch <= kListedMaxBatch && wgs >= kListedFromWorkgroups) {
     const int64_t rows_wg = BMW >> p.pack_shift;
     const int64_t units_max = (int64_t)group * ((a->total_q_rows + rows_wg - 1) / rows_wg + a->batch);
@@ -1247,7 +1280,7 @@ static int launch_prefill_rows(const lsattn_prefill_args* a, bool tile_major, co
   // (a round: two four-wave workgroups per CU, one of the others.  Two rounds still gain: 16 x 256 tokens 38.0 -> 36.8 us,
   // 1 x 4096 129.0 -> 127.7; six rounds lose 1-3 %, sixteen 5 %.)
   p.store_through = MODE == 0 && wgs_launch <= 2 * (HALF ? 2 * kCUs : kCUs);
-  LSATTN_LAUNCH_KERNEL((prefill_kernel<T, MODE, DV, SPLIT, HALF>), dim3((unsigned)wgs_launch), dim3(HALF ? NWAVE * 32 : NWAVE * 64), 0, st, p);
+  LSATTN_LAUNCH_KERNEL((prefill_kernel<T, MODE, DV, SPLIT, HALF, CUTS>), dim3((unsigned)wgs_launch), dim3(HALF ? NWAVE * 32 : NWAVE * 64), 0, st, p);
   return check_launch();
 }
 
@@ -1322,15 +1355,23 @@ static Shape choose_shape(const lsattn_prefill_args* a, bool dv, const Tuning& t
   return split ? Shape{LSATTN_ROUTE_ROWS_128, true} : Shape{LSATTN_ROUTE_ROWS_256, tile_major};
 }
 
-template <typename T, int MODE, bool DV> static int launch_prefill(const lsattn_prefill_args* a, hipStream_t st) {
+template <typename T, int MODE, bool DV, bool CUTS> static int launch_prefill_shape(const lsattn_prefill_args* a, hipStream_t st) {
   const Tuning tn = tuning();
   const Shape shape = choose_shape(a, DV, tn);
   if constexpr (DV) {
-    if (shape.route == LSATTN_ROUTE_HALF_FOLDED) return launch_prefill_rows<T, MODE, true, false, true>(a, true, tn, st, true);
-    if (shape.route == LSATTN_ROUTE_HALF) return launch_prefill_rows<T, MODE, true, false, true>(a, true, tn, st);
-    if (shape.route == LSATTN_ROUTE_ROWS_128) return launch_prefill_rows<T, MODE, true, true>(a, true, tn, st);
+    if (shape.route == LSATTN_ROUTE_HALF_FOLDED) return launch_prefill_rows<T, MODE, true, false, true, CUTS>(a, true, tn, st, true);
+    if (shape.route == LSATTN_ROUTE_HALF) return launch_prefill_rows<T, MODE, true, false, true, CUTS>(a, true, tn, st);
+    if (shape.route == LSATTN_ROUTE_ROWS_128) return launch_prefill_rows<T, MODE, true, true, false, CUTS>(a, true, tn, st);
   }
-  return launch_prefill_rows<T, MODE, DV, false>(a, shape.tile_major, tn, st);
+  return launch_prefill_rows<T, MODE, DV, false, false, CUTS>(a, shape.tile_major, tn, st);
+}
+
+// (the cut along the keys in kernels of its own: its few scalar instructions lie in front of the first load, and cost launches without
+// cuts 0.1 to 0.2 us)
+template <typename T, int MODE, bool DV> static int launch_prefill(const lsattn_prefill_args* a, hipStream_t st) {
+  if constexpr (MODE == 0)
+    if (a->kv_cuts > 1) return launch_prefill_shape<T, 0, DV, true>(a, st);
+  return launch_prefill_shape<T, MODE, DV, false>(a, st);
 }
 
 static int validate(const lsattn_prefill_args* a, int mode) {
