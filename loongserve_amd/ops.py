@@ -283,15 +283,19 @@ def _cuts_for(batch: int, num_q_heads: int, max_q_len: int, keys: int, num_kv_he
 
 def _choose_cuts(q, k, batch: int, max_q_len: int, max_kv_len: Optional[int], workspace) -> int:
     """KV cuts an operator uses where the caller names none: as many as are fastest and `workspace` holds, but kv_split_count
-    where that is the caller's measure of it (a pair of tensors, or one tensor that holds fewer)."""
+    where that is the caller's measure of it (a pair of tensors, or one tensor that holds fewer), and none where that says
+    none: a launch of 192 workgroups and more gains little (1 x 1024 x 20000 keys, MHA 32, 280 -> 271 us with two cuts; 1 x 1500 x 8192
+    185 -> 192 with four), takes memory for its parts, and loses by much where the K buffer is larger than what is in it (1 x 1024
+    against as many keys of a 32768-row buffer: 21.9 -> 34.2 us with two)."""
     kv_rows = k.shape[0] if max_kv_len is None else int(max_kv_len)
     if kv_rows < KV_SPLIT_MIN_KEYS or batch <= 0 or k.shape[1] == 0 or q.shape[1] % k.shape[1]:
         return 1
+    sized = kv_split_count(batch, q.shape[1], max_q_len, kv_rows, k.shape[1])
+    if sized == 1:
+        return 1
     most = _workspace_cuts(workspace, q.shape[0], q.shape[1], q.shape[-1])
-    if workspace is not None:
-        sized = kv_split_count(batch, q.shape[1], max_q_len, kv_rows, k.shape[1])
-        if isinstance(workspace, (tuple, list)) or most < sized:
-            return sized
+    if workspace is not None and (isinstance(workspace, (tuple, list)) or most < sized):
+        return sized
     keys = kv_rows if max_kv_len is not None else max(1, kv_rows // batch)  # (the rows of the buffer are those of all sequences)
     return _cuts_for(batch, q.shape[1], int(max_q_len), keys, k.shape[1], min(most, _lib.LSATTN_MAX_KV_CUTS))
 

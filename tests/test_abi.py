@@ -343,6 +343,28 @@ def test_cuts_are_bounded_by_the_memory_for_their_parts():
     assert _choose_cuts(torch.empty((4096, 32, 128), device="meta"), k, 8, 4096, None, None) == 1
 
 
+def test_operators_cut_no_launch_that_kv_split_count_leaves_whole():
+    """A launch that is not cut takes no memory for parts; the ones that are stay near the 64 MB that kv_split_count's own cuts take."""
+    torch = pytest.importorskip("torch")
+    from loongserve_amd.ops import _choose_cuts, kv_split_count
+    most, whole = 0, 0
+    for batch in (1, 2, 3, 4, 8):
+        for rows in (1, 64, 200, 500, 896, 1024, 1100, 1792, 2047):
+            for keys in (8191, 8192, 9000, 20000, 100000):
+                for Hq, Hkv in ((32, 32), (32, 8), (64, 8), (8, 1)):
+                    q = torch.empty((batch * rows, Hq, 128), dtype=torch.float16, device="meta")
+                    k = torch.empty((keys, Hkv, 128), dtype=torch.float16, device="meta")
+                    for held in (None, torch.empty(64 * q.numel() * 2, device="meta")):
+                        for given in (None, keys):
+                            got = _choose_cuts(q, k, batch, rows, given, held)
+                            if kv_split_count(batch, Hq, rows, keys, Hkv) == 1:
+                                assert got == 1, (batch, rows, keys, Hq, Hkv)
+                                whole += 1
+                            else:
+                                most = max(most, got * batch * rows * Hq * 129 * 4)
+    assert whole and most <= 96 << 20, most
+
+
 def _route(batch, max_q, heads, head_dim=128, total_q=0, total_kv=0, max_kv=0, dtype=0, v_is_f16=0, cuts=0):
     from loongserve_amd import _lib
     a = _lib.PrefillArgs()
