@@ -136,6 +136,10 @@ enum {
 };
 int lsattn_prefill_route(const lsattn_prefill_args* a);
 
+/* Cuts along the keys (kv_cuts) with the least predicted time for a step of 128-wide heads over `keys` keys a sequence, at most `most`
+ * (what the memory for the parts holds); 1: leave it whole.  For launches of fewer than 192 workgroups, where it was measured. */
+int lsattn_prefill_cut_count(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads, int32_t max_q_len, int64_t keys, int32_t most);
+
 /* 1 if the step these arguments describe (v_is_f16 = 0) converts a bfloat16 V on its way into LDS at no cost, as the kernels
  * for head sizes below 128 and for batches of short prompts do; 0 if the caller should make an fp16 copy of V first
  * (lsattn_bf16_to_f16_rows).  Looks at the numbers in the block only, not through its pointers. */
@@ -577,7 +581,8 @@ const char* lsattn_strerror(int code);
  * kv_cuts / kv_cut_len / o_cut_rows / total_q_rows in lsattn_prefill_args, lsattn_prefill_merge_cuts; 4 = dest_index of
  * lsattn_rotary_kv_write_args untyped, its slots int32 or int64 by dest_index_is_i64 (a reserved word before), lsattn_kv_scatter_i64,
  * the counts of lsattn_pool_update_refs also in pinned host memory and, past LSATTN_POOL_REFS_ORDERED entries, not behind the state; 5 = total_kv_rows and kv_cut_even in lsattn_prefill_args,
- * lsattn_prefill_converts_v; 6 = max_kv_len there (a reserved word before), lsattn_prefill_route. */
+ * lsattn_prefill_converts_v; 6 = max_kv_len there (a reserved word before), lsattn_prefill_route,
+ * lsattn_prefill_cut_count. */
 #define LSATTN_VERSION 6
 int lsattn_version(void);
 

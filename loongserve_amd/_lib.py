@@ -156,6 +156,7 @@ EXPORTS = {
     "lsattn_pool_update_refs": (C.c_int, [_vp, _i64, _vp, _i64, C.c_int, _vp, _vp, C.c_size_t, _vp]),
     "lsattn_prefill_converts_v": (C.c_int, [C.POINTER(PrefillArgs)]),
     "lsattn_prefill_route": (C.c_int, [C.POINTER(PrefillArgs)]),
+    "lsattn_prefill_cut_count": (C.c_int, [_i32, _i32, _i32, _i32, _i64, _i32]),
     "lsattn_bf16_to_f16_rows": (C.c_int, [_vp, _i64, _vp, _i64, _i64, _i64, _vp]),
     "lsattn_set_tuning": (C.c_int, [C.POINTER(Tuning)]),
     "lsattn_strerror": (C.c_char_p, [C.c_int]),

@@ -1445,3 +1445,44 @@ extern "C" int lsattn_prefill_route(const lsattn_prefill_args* a) {
   if (a->head_dim != 128 || prefill_short_blocks(a)) return prefill_small_route(a);
   return choose_shape(a, a->dtype == LSATTN_F16 || a->v_is_f16, tuning()).route;
 }
+
+// The count of cuts with the least predicted time, the smallest within 3 % of it.  A launch of W workgroups without cuts runs W * S with S of
+// them, in rounds of one per CU, each of them a sequence's share of the tiles and a fixed start and end; every cut adds a part to write and
+// to merge; and K and V cannot pass faster than the workgroups' CUs draw them.  The constants, in us: 0.88 per 64-key tile and 13 around
+// it for the 128-row shape, 1.57 and 9 for the 256-row one, 6 + 0.2 per part for the merge and its rows at 4 TB/s, K/V at 5.3 TB/s.
+// Over 88 launches that kv_split_count (ops.py) cuts (64 to 2000 rows behind 8192 to 65000 keys, 1 to 8 sequences; 32/32, 32/8, 64/8, 8/1
+// heads), each timed with 1 to 64 cuts, the pick is 0 to 3 % behind the best count in the geometric mean and kv_split_count's 4 to 22 %
+// (64 rows x 8192 keys 32/8 51 -> 30 us, 200 x 9000 8/1 56 -> 28, 500 x 65000 32/8 439 -> 415); the worst against the latter is 200 x 20000
+// 32/8 with 73.4 -> 76.8.
+extern "C" int lsattn_prefill_cut_count(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads, int32_t max_q_len, int64_t keys, int32_t most) {
+  if (batch <= 0 || num_q_heads <= 0 || num_kv_heads <= 0 || num_q_heads % num_kv_heads || max_q_len <= 0 || keys <= 0) return 1;
+  constexpr double kTile128 = 0.88, kAround128 = 13.0, kTile256 = 1.57, kAround256 = 9.0, kMerge = 6.0, kMergePart = 0.2;
+  constexpr double kPartBytesPerUs = 4e6, kDrawBytesPerUs = 5.3e6;
+  lsattn_prefill_args a = {};
+  a.batch = batch, a.num_q_heads = num_q_heads, a.num_kv_heads = num_kv_heads, a.head_dim = 128, a.max_q_len = max_q_len;
+  const Tuning tn = tuning();
+  auto workgroups = [&](bool rows128) {
+    const int64_t rows = (rows128 ? BM / 2 : BM) >> pack_shift_for(&a, rows128, tn);
+    return (int64_t)batch * (num_q_heads >> pack_shift_for(&a, rows128, tn)) * ((max_q_len + rows - 1) / rows);
+  };
+  const int64_t wgs256 = workgroups(false), wgs128 = workgroups(true);
+  const double part_us = (double)batch * max_q_len * num_q_heads * 2 * (128 + 1) * 4 / kPartBytesPerUs;  // (written and read)
+  const double kv_us = (double)batch * keys * num_kv_heads * 2 * 128 * 2 / kDrawBytesPerUs;
+  int64_t last = (int64_t)batch * keys / 512;
+  last = last < most ? last : most;
+  last = last < LSATTN_MAX_KV_CUTS ? last : LSATTN_MAX_KV_CUTS;
+  double times[LSATTN_MAX_KV_CUTS + 1], least = 0;
+  for (int S = 1; S <= last; S++) {
+    a.kv_cuts = S;
+    const bool rows128 = choose_shape(&a, true, tn).route != LSATTN_ROUTE_ROWS_256;
+    const int64_t live = S * (rows128 ? wgs128 : wgs256), tiles = ((keys + S - 1) / S + 63) / 64;
+    const double per_tile = rows128 ? kTile128 : kTile256, around = rows128 ? kAround128 : kAround256;
+    const double walk = (double)((live + kCUs - 1) / kCUs) * (tiles * per_tile + around);
+    const double draw = kv_us * (live < kCUs ? (double)kCUs / live : 1.0) + around;
+    times[S] = (walk > draw ? walk : draw) + (S > 1 ? kMerge + S * (kMergePart + part_us) : 0.0);
+    if (S == 1 || times[S] < least) least = times[S];
+  }
+  for (int S = 1; S <= last; S++)
+    if (times[S] <= 1.03 * least) return S;
+  return 1;
+}

@@ -212,7 +212,7 @@ KV_SPLIT_MIN_KEYS = 8192
 
 
 def kv_split_count(batch: int, num_q_heads: int, max_q_len: int, kv_rows: int, num_kv_heads: Optional[int] = None) -> int:
-    """KV cuts to size a workspace for: the count that leaves the longest chain of tiles on a CU shortest
+    """KV cuts to size a workspace for: launches of 192 workgroups and more stay whole; else the count that leaves the longest chain of tiles on a CU shortest
     when the launch's workgroups run in rounds of 256 (one per CU), the smaller count on ties, with cuts of at least 4096
     keys; the operators use as many as their workspace holds where shorter cuts are faster still (_choose_cuts).  kv_rows bounds
     every sequence's chunk (max_kv_len where the caller gives it, else the rows of the k buffer; the lengths themselves live on
@@ -244,43 +244,6 @@ def _kv_split_count(batch, num_q_heads, max_q_len, kv_rows, num_kv_heads, below,
     return best
 
 
-@functools.lru_cache(maxsize=4096)
-def _cuts_for(batch: int, num_q_heads: int, max_q_len: int, keys: int, num_kv_heads: int, most: int) -> int:
-    """KV cuts of a step over `keys` keys a sequence, at most `most` (what the memory for the parts holds): the count with the
-    least predicted time, the smallest within 3 % of it.  A launch of W workgroups without cuts runs W * S with S of them, in rounds of one per CU, each of them
-    a sequence's share of the tiles and a fixed start and end; every cut adds a part to write and to merge; and K and V cannot pass
-    faster than the workgroups' CUs draw them.  The constants, in us: 0.88 per 64-key tile and 13 around it for the
-    128-row shape, 1.57 and 9 for the 256-row one (chosen here as lsattn_prefill_step chooses), 6 + 0.2 per part for the merge and its
-    rows at 4 TB/s, K/V at 5.3 TB/s.  Over 77 shapes (64 to 1024 rows behind 8192 to 100000 keys, one sequence and two;
-    32/32, 32/8, 64/8, 8/1 heads), each timed with 1 to 64 cuts, the pick is 1 % behind the best count in the geometric mean and kv_split_count's
-    13 %: 64 rows x 8192 keys 32/8 51 -> 30 us, 200 x 9000 8/1 56 -> 28, 500 x 65000 32/8 439 -> 415."""
-    group = num_q_heads // num_kv_heads
-
-    def packed(limit):  # query heads side by side in a workgroup
-        p = 1
-        while p < limit and group % (2 * p) == 0:
-            p *= 2
-        return p
-
-    p8, p4 = packed(8), packed(4)
-    tiles256, tiles128 = -(-max_q_len * p8 // 256), -(-max_q_len * p4 // 128)
-    w256, w128 = batch * (num_q_heads // p8) * tiles256, batch * (num_q_heads // p4) * tiles128
-    if w128 <= 0 or w128 >= 2 * KV_SPLIT_ROUND or most <= 1:
-        return 1
-    padded = (tiles128 * 128 // p4) * 5 <= (tiles256 * 256 // p8) * 4
-    part_us = batch * max_q_len * num_q_heads * 1032 / 4e6
-    times = []
-    for S in range(1, max(1, min(_lib.LSATTN_MAX_KV_CUTS, most, batch * keys // 512)) + 1):
-        split = padded or S * w256 <= KV_SPLIT_ROUND // 2 or (S * w256 <= KV_SPLIT_ROUND and max_q_len > 1024)
-        live = S * (w128 if split else w256)
-        per_tile, around = (0.88, 13.0) if split else (1.57, 9.0)
-        walk = -(-live // KV_SPLIT_ROUND) * (-(-keys / S // 64) * per_tile + around)
-        merge = 6.0 + S * (0.2 + part_us) if S > 1 else 0.0
-        draw = batch * keys * num_kv_heads * 512 / 5.3e6 * max(1.0, KV_SPLIT_ROUND / live) + around
-        times.append(max(walk, draw) + merge)
-    return next(S for S, t in enumerate(times, 1) if t <= 1.03 * min(times))
-
-
 def _choose_cuts(q, k, batch: int, max_q_len: int, max_kv_len: Optional[int], workspace) -> int:
     """KV cuts an operator uses where the caller names none: as many as are fastest and `workspace` holds, but kv_split_count
     where that is the caller's measure of it (a pair of tensors, or one tensor that holds fewer), and none where that says
@@ -297,7 +260,7 @@ def _choose_cuts(q, k, batch: int, max_q_len: int, max_kv_len: Optional[int], wo
     if workspace is not None and (isinstance(workspace, (tuple, list)) or most < sized):
         return sized
     keys = kv_rows if max_kv_len is not None else max(1, kv_rows // batch)  # (the rows of the buffer are those of all sequences)
-    return _cuts_for(batch, q.shape[1], int(max_q_len), keys, k.shape[1], min(most, _lib.LSATTN_MAX_KV_CUTS))
+    return _lib.load().lsattn_prefill_cut_count(batch, q.shape[1], k.shape[1], int(max_q_len), keys, min(most, _lib.LSATTN_MAX_KV_CUTS))
 
 
 def _cut_len(kv_rows: int, S: int) -> int:
@@ -406,8 +369,9 @@ def prefill_attention_step(q, k, v, q_b_start_loc, q_b_seq_len, q_first_token_gl
     query rows and head); with kv_splits = S > 1 every sequence's KV chunk is cut into S slices inside one launch, which
     computes the S partials of every row (lsattn_prefill_args.kv_cuts), and lsattn_prefill_merge_cuts joins them for the
     rows of the sequences.  None chooses S from the shapes (_choose_cuts over max_kv_len, an upper bound of every
-    chunk's length; the rows of the k buffer if not given), 1 switches it off.  The partials take S times the size of
-    (out, lse): kv_split_workspace passes the caller's memory for them (as context_attention_fwd's workspace).
+    chunk's length; the rows of the k buffer if not given: give it where k is larger than what is in it, or short chunks take
+    the parts of long ones), 1 switches it off.  The partials take S times the size of (out, lse), up to some 200 MB with S from
+    the shapes: kv_split_workspace passes the caller's memory for them (as context_attention_fwd's workspace), else torch allocates it.
 
     Same inputs as context_attention_fwd; rows that see no key get O = 0, LSE = -inf.
     total_q_len: as in context_attention_fwd (an upper bound of the rows of all sequences together, for skewed batches).

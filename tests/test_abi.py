@@ -344,10 +344,11 @@ def test_cuts_are_bounded_by_the_memory_for_their_parts():
 
 
 def test_operators_cut_no_launch_that_kv_split_count_leaves_whole():
-    """A launch that is not cut takes no memory for parts; the ones that are stay near the 64 MB that kv_split_count's own cuts take."""
+    """A launch that is not cut takes no memory for parts; the ones that are take no more, over these shapes, than kv_split_count's
+    counts may take."""
     torch = pytest.importorskip("torch")
     from loongserve_amd.ops import _choose_cuts, kv_split_count
-    most, whole = 0, 0
+    most, most_sized, whole = 0, 0, 0
     for batch in (1, 2, 3, 4, 8):
         for rows in (1, 64, 200, 500, 896, 1024, 1100, 1792, 2047):
             for keys in (8191, 8192, 9000, 20000, 100000):
@@ -357,12 +358,29 @@ def test_operators_cut_no_launch_that_kv_split_count_leaves_whole():
                     for held in (None, torch.empty(64 * q.numel() * 2, device="meta")):
                         for given in (None, keys):
                             got = _choose_cuts(q, k, batch, rows, given, held)
-                            if kv_split_count(batch, Hq, rows, keys, Hkv) == 1:
+                            sized, part = kv_split_count(batch, Hq, rows, keys, Hkv), batch * rows * Hq * 129 * 4
+                            if sized == 1:
                                 assert got == 1, (batch, rows, keys, Hq, Hkv)
                                 whole += 1
                             else:
-                                most = max(most, got * batch * rows * Hq * 129 * 4)
-    assert whole and most <= 96 << 20, most
+                                most, most_sized = max(most, got * part), max(most_sized, sized * part)
+    assert whole and 0 < most <= most_sized < 256 << 20, (most, most_sized)
+
+
+def test_cut_count_of_a_step():
+    """The library's count: within what the memory holds, a cut no shorter than 512 keys, one where the arguments describe no step; the
+    counts that were measured at some lengths."""
+    from loongserve_amd import _lib
+    count = _lib.load().lsattn_prefill_cut_count
+    assert count(1, 32, 8, 64, 8192, 64) == 10 and count(1, 32, 8, 500, 65000, 64) == 4 and count(1, 32, 8, 500, 65000, 2) == 2
+    assert count(1, 8, 1, 64, 17467, 64) in range(16, 25) and count(1, 8, 1, 209, 26261, 64) == 16
+    for args in ((0, 32, 8, 64, 8192, 64), (1, 32, 0, 64, 8192, 64), (1, 32, 5, 64, 8192, 64), (1, 32, 8, 0, 8192, 64), (1, 32, 8, 64, 0, 64),
+                 (1, 32, 8, 64, 8192, 0), (1, 32, 8, 64, 8192, -3), (1, 32, 8, 64, 1023, 64)):
+        assert count(*args) == 1, args
+    for rows in (1, 64, 500, 2047):
+        for keys in (1024, 8192, 100000, 2 ** 31 - 1):
+            for most in (1, 3, 64, 1000):
+                assert 1 <= count(1, 8, 1, rows, keys, most) <= min(most, keys // 512, 64)
 
 
 def _route(batch, max_q, heads, head_dim=128, total_q=0, total_kv=0, max_kv=0, dtype=0, v_is_f16=0, cuts=0):
