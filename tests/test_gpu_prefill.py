@@ -793,7 +793,7 @@ def test_small_heads_in_a_ragged_batch_of_many_tiles(lsa, D, dtype, lens):
     (8, 2, [0, 1, 15, 16, 17, 33, 63, 64, 65, 129], [0, 61, 122], 1),  # 16 positions per wave, four heads side by side
     (6, 3, [768, 1, 127, 128], [0, 5], 1),                             # the longest prompt that is taken, two heads
     (3, 3, [31, 257, 64], [3], 4),                                     # one head per workgroup, a striped ring of four
-    (32, 32, [128, 100, 7, 256, 65, 33] * 5, [0, 40], 1),              # 32 positions per wave
+    (32, 32, [128, 100, 7, 256, 65, 33] * 5, [0, 40], 1),              # more workgroups than it takes (32 positions per wave: test_gpu_prefill_short.py)
     (4, 4, [769], [0], 1),                                             # one row past it: the kernel of 128-row workgroups
 ])
 def test_short_prompts_of_128_wide_heads(lsa, mode, dtype, Hq, Hkv, lens, ctx, P):

@@ -1,5 +1,7 @@
 """GPU parity of prefill_small_kernel beyond the shapes of test_gpu_prefill.py, which forces the 128-wide kernel's shapes in turn: here the
 library chooses."""
+import ctypes as C
+
 import pytest
 import torch
 
@@ -94,3 +96,68 @@ def test_short_rows_behind_one_long_context_and_bounded_ones(lsa, dtype):
             torch.cuda.synchronize()
             assert_o_close(o, o_ref, "O")
             assert_lse_close(lse, lse_ref, "LSE")
+
+
+SMALL_16, SMALL_32, SMALL_TURNS = 1, 2, 3  # LSATTN_ROUTE_* of include/lsattn.h
+
+
+def _every_epilogue_on(route, lsa, mode, V, D, Hq, Hkv, lens, ctx):
+    """One step (the partial) or two over halves of the keys (the folding epilogues) against the oracle, each of them on `route`.
+    V: "f16", "bf16" (converted by the kernel) or "bf16 copied" (the caller's buffer for the fp16 copy)."""
+    from loongserve_amd import _lib, ops
+    dtype = torch.float16 if V == "f16" else torch.bfloat16
+    klens = [n + c for n, c in zip(lens, ctx)]
+    T, TK = sum(lens), sum(klens)
+    q, k, v = rand_t((T, Hq, D), 71, dtype), rand_t((TK, Hkv, D), 72, dtype), rand_t((TK, Hkv, D), 73, dtype)
+    ramp = torch.cat([torch.arange(n) % 400 for n in klens]).float() / 80 + 1  # (the running maxima are raised again and again)
+    k = (k.float() * ramp[:, None, None]).to(dtype)
+    qm, km = meta(lens, ctx), meta(klens)
+    o_ref, lse_ref = orc.attn_step(q, k, v, *qm, *km, 1)
+    half = [n // 2 for n in klens]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32)
+    steps = [(km[0], i32(half), i32([0] * len(lens))), (km[0] + i32(half), i32([n - f for n, f in zip(klens, half)]), i32(half))]
+    qd, kd, vd, qmd = *_dev(q, k, v), _dev(*qm)
+    kw = dict(v_f16=torch.empty(v.shape, dtype=torch.float16, device=DEV)) if V == "bf16 copied" else {}
+
+    def on_route(o, s):
+        a = ops._prefill_args(qd, kd, vd, o, *qmd, *s, 1, max(lens), None, total_q_len=T, **kw)
+        assert _lib.load().lsattn_prefill_route(C.byref(a)) == route and a.v_is_f16 == (V == "bf16 copied")
+        return s
+
+    if mode == "in_place":
+        o = torch.full((T, Hq, D), 7.0, dtype=dtype, device=DEV)
+        m, l = torch.full((T, Hq), float("-inf"), device=DEV), torch.zeros((T, Hq), device=DEV)
+        o_st, m_st, l_st = torch.zeros((T, Hq, D), dtype=dtype), torch.full((T, Hq), float("-inf")), torch.zeros(T, Hq)
+        for s in steps:
+            lsa.context_attention_fwd(qd, kd, vd, o, *qmd, *on_route(o, _dev(*s)), 1, max(lens), m, l, total_q_len=T, **kw)
+            orc.context_attention_fwd(q, k, v, o_st, *qm, *s, 1, max(lens), m_st, l_st)
+        torch.cuda.synchronize()
+        assert_inplace_o_close(o.cpu(), o_st, o_ref, "o")
+        assert_lse_close(orc.state_lse(m.cpu(), l.cpu()).float(), lse_ref, "state LSE")
+        return
+    o, lse = torch.full((T, Hq, D), 7.0, device=DEV), torch.full((T, Hq), float("-inf"), device=DEV)
+    for s in steps if mode == "accumulate" else [km]:
+        lsa.prefill_attention_step(qd, kd, vd, *qmd, *on_route(o, _dev(*s)), 1, max(lens), o, lse, accumulate=mode == "accumulate",
+                                   total_q_len=T, **kw)
+    torch.cuda.synchronize()
+    assert_o_close(o, o_ref, "O")
+    assert_lse_close(lse, lse_ref, "LSE")
+
+
+@pytest.mark.parametrize("mode", ["partial", "accumulate", "in_place"])
+@pytest.mark.parametrize("V", ["f16", "bf16", "bf16 copied"])
+@pytest.mark.parametrize("Hq,Hkv", [(32, 32), (16, 8), (16, 4)])
+def test_short_prompts_with_32_positions_per_wave(lsa, mode, V, Hq, Hkv):
+    """128-wide heads, more workgroups than the 16-position shape takes: one, two and four heads side by side, prompts around the waves'
+    32 rows and the 64-key tiles, some behind a context."""
+    print("case", mode, V, Hq, Hkv, flush=True)
+    _every_epilogue_on(SMALL_32, lsa, mode, V, 128, Hq, Hkv, [128, 100, 7, 256, 65, 33] * 4, [0, 40] * 12)
+
+
+@pytest.mark.parametrize("mode", ["partial", "accumulate", "in_place"])
+@pytest.mark.parametrize("V", ["f16", "bf16", "bf16 copied"])
+@pytest.mark.parametrize("D", [64, 32, 16])
+def test_requests_that_take_turns_in_the_grid(lsa, mode, V, D):
+    """Heads of 16 to 64 in a ragged batch whose places in the grid turn from tile to tile."""
+    print("case", mode, V, D, flush=True)
+    _every_epilogue_on(SMALL_TURNS, lsa, mode, V, D, 16, 4, [1500, 1200, 1, 33, 1000, 64, 1301, 900], [0] * 8)
