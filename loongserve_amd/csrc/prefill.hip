@@ -1367,7 +1367,7 @@ template <typename T, int MODE, bool DV, bool CUTS> static int launch_prefill_sh
 }
 
 // (the cut along the keys in kernels of its own: its few scalar instructions lie in front of the first load, and cost launches without
-// cuts 0.1 to 0.2 us)
+// cuts 0.1 us)
 template <typename T, int MODE, bool DV> static int launch_prefill(const lsattn_prefill_args* a, hipStream_t st) {
   if constexpr (MODE == 0)
     if (a->kv_cuts > 1) return launch_prefill_shape<T, 0, DV, true>(a, st);

@@ -129,7 +129,7 @@ __global__ __launch_bounds__(kWaves * 64, D == 128 ? 2 : QB == 2 && D == 64 && !
   constexpr int RB = D * 2;                 // bytes per row in LDS
   constexpr int TB = kTile * RB;            // bytes per tile
   constexpr int RPI = 64 / CPR;             // rows per load instruction (a wave's 64 lanes, 16 bytes each)
-  constexpr int NI = (kTile + kWaves * RPI - 1) / (kWaves * RPI);  // load instructions per wave and tile: two for D = 64, else one
+  constexpr int NI = (kTile + kWaves * RPI - 1) / (kWaves * RPI);  // load instructions per wave and tile: four for D = 128, two for 64, else one
   constexpr int RPB = 256 / RB;             // rows that pass all 64 LDS banks once
   // two stages of (K tile, V tile): the next tile is written while the present one is read.  Rows are not padded (a load to
   // LDS writes 1 KB in a row); instead the 16-byte chunks of a row are XORed with a function of the row: K so that a
@@ -531,7 +531,7 @@ template <typename T, bool DV> int launch_mode(const SmallParams& p, const lsatt
 // Short prompts of 128-wide heads: the kernel of prefill.hip spends 9 us on starting and ending whatever it computes (eight
 // waves of 256 registers that fill 128 KB of rings and some 40 KB of code before the first product); this one has a
 // quarter of the code, workgroups of 64 rows (128) and two of them per CU, converts a bfloat16 V on the way (no launch in front
-// that copies it), but reads LDS four times (twice) as much per product, which bounds a full chip.  Measured over 472 launches (1 to
+// that copies it), but reads LDS four times (twice) as much per product, and a tile takes longer (below).  Measured over 472 launches (1 to
 // 32 prompts of 32 to 2048 tokens, equal or log-uniform over a factor of 8, 32/32, 32/8, 64/8 and 8/1 heads; both epilogues;
 // microseconds, the kernel of prefill.hip | 16 positions per wave | 32; bf16 with its copy of V):
 //   1 x 100 MHA f16 10.9 | 5.5 | 7.8        1 x 512 32/8 f16 15.6 | 12.3 | 16.5    16 x 128 MHA f16 25.6 | 19.6 | 17.7
