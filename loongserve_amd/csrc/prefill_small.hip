@@ -2,23 +2,24 @@
 // loongserve/models/llama/triton_kernel/ring_context_flashattention_nopad.py:248-250) and, for batches of short prompts, 128
 // (prefill_short_blocks), gfx950, wave64.
 //
-// What bounds it is vector work: a 32 x 32 block of scores takes a wave 16 exponentials, 16 multiply-adds, 16 additions and
-// some 15 conversions and checks against 16 (D = 64) to 6 (D = 16) MFMAs, and the time falls only a third from D = 64 to 16.
-// Hence no work beside those in the common path, and four waves per SIMD whose phases mix freely:
+// What bounds it at 64 and below is vector work: a 32 x 32 block of scores takes a wave 16 exponentials, 16 multiply-adds, 16 additions and
+// some 15 conversions and checks against 18 (D = 64) to 8 (D = 16) MFMAs, and the time falls only a third from D = 64 to 16.  At 128
+// it is MFMA and LDS, and for short prompts the start and end of workgroups.
+// Hence no work beside those in the common path, and three or four waves per SIMD whose phases mix freely:
 //   * a workgroup of four waves; a wave owns 32 (small launches: 16) query positions of one head.  With grouped-query
 //     heads up to four heads of a KV head sit side by side in a workgroup, which then ends sooner on the diagonal;
-//   * K and V tiles of 64 keys go to LDS by direct loads, two stages, one barrier per tile, chunks XOR-swizzled (bfloat16 V
-//     passes through registers and becomes fp16 there);
+//   * K and V tiles of 64 keys (two stages), or 32 (128-wide heads, 32 positions: three), go to LDS by direct loads, one barrier per tile,
+//     chunks XOR-swizzled (bfloat16 V passes through registers and becomes fp16 there);
 //   * scores transposed, S^T = K Q^T with v_mfma_f32_16x16x32 (a head of 16 fills half of the contraction with
 //     zeros), 32 keys per step, so a lane owns one query column: the fp32 scores turn into the B operand of O^T += V^T P^T in
 //     place (P and V as fp16, sums of P in fp32), V^T operands through ds_read_b64_tr_b16; a wave skips the steps none of its
 //     rows sees;
 //   * the running maximum of a row is raised only when a P of 2 or more shows up; no exchange between lanes otherwise;
 //   * the three epilogues of the 128-wide kernel: 0 the step's fp32 partial (O, LSE), 1 the reference's in-place
-//     (o, m, l) update (ring_context_flashattention_nopad.py:171-188), 2 the LSE merge into a running fp32 (O, LSE).
-// Against 16 positions per wave, eight waves, tiles staged through registers and the maximum exchanged in every step
-// (fp16, causal): D = 64, 8 x 2048 tokens GQA 32/8 380 -> 183 us (0.75 PFLOP/s), 1 x 8192 MHA 640 -> 310, 16 x 512 73 -> 47,
-// 1 x 100 7.4 -> 6.0; D = 32, 8 x 2048 283 -> 135; D = 16 278 -> 121.
+//     (o, m, l) update (ring_context_flashattention_nopad.py:171-188), 2 the LSE merge into a running fp32 (O, LSE); O is turned round
+//     in LDS first, so that stores fill whole lines.
+// Measured (fp16, causal, in place, whole calls): D = 64, 8 x 2048 tokens GQA 32/8 172 to 178 us (0.78 PFLOP/s), 16 x 512 43, 32 x 256 34,
+// 16 x 1024 107; D = 128, 16 x 1024 191 us (0.72 PFLOP/s), 16 x 512 65, 1 x 100 9.0 (of which 2.6 are the fills of m and l).
 #include <type_traits>
 
 #include "common.hip.h"
@@ -93,20 +94,20 @@ struct SmallParams {
   float* m;
   float* l;
   int64_t ml_st, ml_sh;
-  int32_t batch;  // (TURN: a request's place among the ids moves on by one from tile to tile)
-  FastDiv d_batch;
+  int32_t batch, bunch, turns;  // the grid takes `bunch` requests at a time; whether their places move on by one from tile to tile
+  FastDiv d_bunch;
 };
 
 constexpr int kWaves = 4;   // waves per workgroup
-constexpr int kTile = 64;   // keys per LDS tile
 constexpr uint32_t kOnes = 0x3C003C00u;  // two ones in fp16
 constexpr int64_t kCUs = 256;
-constexpr int32_t kShortMaxRows = 768;    // 128-wide heads: the longest query chunk this kernel takes
-constexpr int64_t kShortMaxKeys = 1024;   // and the keys up to which it does, of the longest request
-constexpr int64_t kMaxTiles = 65535;  // tiles of one launch (the third index of a grid)
+constexpr int64_t kL2Bytes = 32 << 20;    // of the eight L2s together
+constexpr int64_t kBunchWorkgroups = 512; // workgroups of a bunch of requests of about equal, short lengths
+constexpr int64_t kShortMaxKeys = 2048;   // 128-wide heads: the keys of the longest request up to which this kernel may take a step
+constexpr int64_t kMaxIds = 65535;  // of the second or third index of a grid
 
-// s_waitcnt vmcnt(0) (expcnt / lgkmcnt fields left at their maximum)
-__device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+// s_waitcnt vmcnt(N) (expcnt / lgkmcnt fields left at their maximum)
+template <int N> __device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14)); }
 
 // 16 bytes per lane from tile + off into LDS at dst (wave-uniform) + 16 * lane.  From inline assembly, or the compiler would
 // wait for the load before every later LDS read; the s_nop is the wait state between a write of m0 and its use.
@@ -119,46 +120,59 @@ __device__ __forceinline__ const char* uniform_ptr(const char* ptr) {
   return (const char*)(((uint64_t)hi << 32) | lo);
 }
 
+// A launch's shape by head size and positions per wave: keys per LDS tile, tiles in LDS (requested one fewer ahead), workgroups per CU.
+// 128-wide heads, 32 positions per wave: three stages of 32 keys (48 KB) and 168 registers, so that three workgroups fit a CU.
+template <int D, int WP> constexpr int kTileOf = D == 128 && WP == 32 ? 32 : 64;
+template <int D, int WP> constexpr int kStagesOf = D == 128 && WP == 32 ? 3 : 2;
+template <int D, int WP, bool DV> constexpr int kResident = D == 128 ? (WP == 32 ? 3 : 2) : WP == 32 && D == 64 && !DV ? 3 : 4;
+
 // DV: the V tiles are fp16 in memory and go straight into LDS as the K tiles do; otherwise (bfloat16 V) they pass through
-// registers and are converted on the way.  QB: blocks of 16 query positions per wave.
-template <typename T, int D, int MODE, bool DV, int QB, bool TURN = false>
-__global__ __launch_bounds__(kWaves * 64, D == 128 ? 2 : QB == 2 && D == 64 && !DV ? 3 : 4) void prefill_small_kernel(SmallParams p) {
+// registers and are converted on the way.  WP: query positions per wave, 16 or 32.  (Products of 32 x 32 x 16, which take a tenth fewer
+// vector instructions, ran at 1.88 GHz where these run at 2.16: 8 ragged sequences of 64-wide heads 164 us against 161, 16 x 1024 tokens of
+// 128-wide ones 199 against 194.)
+template <typename T, int D, int MODE, bool DV, int WP>
+__global__ __launch_bounds__(kWaves * 64, (kResident<D, WP, DV>)) void prefill_small_kernel(SmallParams p) {
+  constexpr int QB = WP / 16;               // blocks of 16 positions per wave
   constexpr int KS = D >= 32 ? D / 32 : 1;  // contraction steps of Q K^T (32 elements each; D = 16 fills half of one)
   constexpr int NDB = D / 16;               // 16-wide blocks of the head
+  constexpr int TK = kTileOf<D, WP>, NS = kStagesOf<D, WP>;
   constexpr int CPR = D / 8;                // 16-byte chunks per K or V row
   constexpr int RB = D * 2;                 // bytes per row in LDS
-  constexpr int TB = kTile * RB;            // bytes per tile
+  constexpr int TB = TK * RB;               // bytes per tile
   constexpr int RPI = 64 / CPR;             // rows per load instruction (a wave's 64 lanes, 16 bytes each)
-  constexpr int NI = (kTile + kWaves * RPI - 1) / (kWaves * RPI);  // load instructions per wave and tile: four for D = 128, two for 64, else one
+  constexpr int NI = (TK + kWaves * RPI - 1) / (kWaves * RPI);  // load instructions per wave and tile
   constexpr int RPB = 256 / RB;             // rows that pass all 64 LDS banks once
-  // two stages of (K tile, V tile): the next tile is written while the present one is read.  Rows are not padded (a load to
+  // NS stages of (K tile, V tile): the next tiles are written while the present one is read.  Rows are not padded (a load to
   // LDS writes 1 KB in a row); instead the 16-byte chunks of a row are XORed with a function of the row: K so that a
   // column of chunks of sixteen rows, which one read takes, lies in sixteen different sets of four banks, V so that 32 bytes of
   // each of eight rows (half a transposing read) cover the banks once.  Rows sixteen apart share their XOR.
-  __shared__ __attribute__((aligned(1024))) char lds[2 * 2 * TB];
+  // (behind them, for the epilogue that folds into (o, m, l): 256 bytes per wave for the old m and l of its rows)
+  constexpr int kStateOff = NS * 2 * TB;
+  __shared__ __attribute__((aligned(1024))) char lds[kStateOff + (MODE == 1 ? kWaves * 256 : 0)];
   auto swz_k = [](int row) { return (row / RPB) & (CPR - 1); };
   auto swz_v = [](int row) { return ((row / RPB) & (CPR / 2 - 1)) << 1; };
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int c = lane & 15, g = lane >> 4;
-  // grid: (KV head, heads side by side), request, tile from the last one down: the heaviest tiles of all requests start
-  // first, and with a multiple of eight KV heads the workgroups of one run on one XCD (ids are dealt round-robin)
+  const int c = lane & 15, g = lane >> 4;  // query column, lane group
+  // grid: (KV head, heads side by side), (tile from the last one down, request of a bunch), bunch of requests: the heaviest tiles of
+  // all requests of a bunch start first, and with a multiple of eight KV heads the workgroups of one run on one XCD (ids are dealt round-robin)
   const int gq = (int)div_by(blockIdx.x, p.d_hkv), kvh = (int)blockIdx.x - gq * p.hkv;
-  int b = blockIdx.y;
-  if constexpr (TURN) {  // (requests_take_turns; a kernel of its own, so that the others stay as they are)
-    const uint32_t place = blockIdx.y + blockIdx.z;
-    b = (int)(place - div_by(place, p.d_batch) * (uint32_t)p.batch);
-  }
-  const int rows_wg = (kWaves * QB * 16) >> p.pack_shift;  // query positions of this workgroup
-  const int m_wg = (p.last_tile - (int)blockIdx.z) * rows_wg;
-  const int q_len = p.q_len[b];
+  const int tile_id = (int)div_by(blockIdx.y, p.d_bunch);
+  int place = (int)blockIdx.y - tile_id * p.bunch;
+  if (p.turns) place += tile_id, place -= (int)div_by((uint32_t)place, p.d_bunch) * p.bunch;
+  const int b = (int)blockIdx.z * p.bunch + place;
+  if (b >= p.batch) return;
+  const int rows_wg = (kWaves * WP) >> p.pack_shift;  // query positions of this workgroup
+  const int m_wg = (p.last_tile - tile_id) * rows_wg;
+  // (the request's numbers are all asked for before the first of them is used)
+  const int q_len = p.q_len[b], kv_len = p.kv_len[b], qf = p.q_first[b], kf = p.kv_first[b], P = p.peers;
+  const int q_start32 = p.q_start[b], kv_start32 = p.kv_start[b], o_start32 = p.o_start ? p.o_start[b] : q_start32;
+  asm volatile("" ::"s"(q_len), "s"(kv_len), "s"(qf), "s"(kf), "s"(q_start32), "s"(kv_start32), "s"(o_start32));
   if (m_wg >= q_len) return;  // (the whole workgroup: the loop below holds barriers)
   const int wph_shift = 2 - p.pack_shift;  // log2 of the waves per head
   const int h = kvh * p.heads_per_kv + (gq << p.pack_shift) + (wave >> wph_shift);
-  const int m0 = m_wg + (wave & ((1 << wph_shift) - 1)) * (QB * 16);  // the wave's first position
-  const int kv_len = p.kv_len[b], qf = p.q_first[b], kf = p.kv_first[b], P = p.peers;
-  const int64_t q_start = p.q_start[b], kv_start = p.kv_start[b];
-  const int64_t o_start = p.o_start ? (int64_t)p.o_start[b] : q_start;
+  const int m0 = m_wg + (wave & ((1 << wph_shift) - 1)) * WP;  // the wave's first position
+  const int64_t q_start = q_start32, kv_start = kv_start32, o_start = o_start32;
 
   // keys of this KV chunk visible to global query position qpos (ring_context_flashattention_nopad.py:156-159)
   auto visible_keys = [&](int qpos) -> int {
@@ -166,19 +180,26 @@ __global__ __launch_bounds__(kWaves * 64, D == 128 ? 2 : QB == 2 && D == 64 && !
     const int n = dq >= 0 ? (int)div_by((uint32_t)dq, p.d_peers) + 1 : 0;
     return n > kv_len ? kv_len : n;
   };
-  // per block qb of 16 positions: the lane's position m0 + 16 qb + c, whether it exists, the keys it sees
-  bool in_range[QB];
-  int cnt[QB];
-  u32x4 qreg[QB][KS];  // Q^T as B operands: qreg[qb][ks] = Q[position][32 ks + 8 g .. + 7]
-  f32x4 oacc[QB][NDB]; // O^T: oacc[qb][db][j] = O[position][16 db + 4 g + j]
+  const int lds_base = (int)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+  // The old m and l (MODE 1) are asked for first of all and go straight into LDS: no register is held over the loop, and the epilogue need
+  // not go to memory to learn whether a row is still in its start state, whose old o is never read.
+  if (MODE == 1) {  // (lanes 0 to 31 the m of a position each, the others the l)
+    const int m = m0 + (lane & (WP - 1));
+    const int64_t at = (o_start + (m < q_len ? m : m_wg)) * p.ml_st + (int64_t)h * p.ml_sh;
+    const float* src = (lane < 32 ? p.m : p.l) + at;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds_base + kStateOff + wave * 256), "v"(src) : "m0", "memory");
+  }
+  // per block qb of 16 positions, the lane's position m0 + 16 qb + c
+  int cnt[QB];           // keys it sees (0 if it does not exist), from the lane's first key of a step
+  u32x4 qreg[QB][KS];    // Q^T as B operands: qreg[qb][ks] = Q[position][32 ks + 8 g .. + 7]
+  f32x4 oacc[QB][NDB];   // O^T: oacc[qb][db][j] = O[position][16 db + 4 g + j]
   float m_run[QB], l_run[QB];  // log2-domain running max of the column; the lane's share of its running sum
-  f32x4 l_pv[QB];  // the column's sum of the fp16 values that multiply V (all four elements)
+  f32x4 l_pv[QB];        // the column's sum of the fp16 values that multiply V (all four elements)
 #pragma unroll
   for (int qb = 0; qb < QB; qb++) {
     const int m = m0 + 16 * qb + c;
-    in_range[qb] = m < q_len;
-    cnt[qb] = in_range[qb] ? visible_keys(qf + m * P) : 0;
-    const char* src = (const char*)p.q + ((q_start + (in_range[qb] ? m : m_wg)) * p.q_st + (int64_t)h * p.q_sh) * 2;
+    cnt[qb] = (m < q_len ? visible_keys(qf + m * P) : 0) - 4 * g;
+    const char* src = (const char*)p.q + ((q_start + (m < q_len ? m : m_wg)) * p.q_st + (int64_t)h * p.q_sh) * 2;
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
       const int d0 = 32 * ks + 8 * g;
@@ -194,7 +215,7 @@ __global__ __launch_bounds__(kWaves * 64, D == 128 ? 2 : QB == 2 && D == 64 && !
   auto last_seen = [&](int first, int rows) -> int {  // keys the last existing position of [first, first + rows) sees; 0 if none exists
     return first < q_len ? visible_keys(qf + (first + rows - 1 < q_len ? first + rows - 1 : q_len - 1) * P) : 0;
   };
-  const int cnt_wave = __builtin_amdgcn_readfirstlane(last_seen(m0, QB * 16));
+  const int cnt_wave = __builtin_amdgcn_readfirstlane(last_seen(m0, WP));
   // (rows past the end see nothing: a wave that holds some masks everywhere only where it has to, in their own columns,
   // which nothing reads; its first row sees the fewest keys of the others)
   const int cnt_first = __builtin_amdgcn_readfirstlane(m0 < q_len ? visible_keys(qf + m0 * P) : 0);
@@ -204,92 +225,132 @@ __global__ __launch_bounds__(kWaves * 64, D == 128 ? 2 : QB == 2 && D == 64 && !
   const char* vbase = (const char*)p.v + (kv_start * p.v_st + (int64_t)kvh * p.v_sh) * 2;
   // staging: instruction i of a wave carries rows (wave + 4 i) * RPI .. of the K tile and of the V tile.  Tiles that lie inside the
   // chunk take a scalar tile address and the lane's 32-bit offset, no vector arithmetic.
-  const bool stager = NI * kWaves * RPI == kTile || wave * RPI < kTile;  // (D = 16: two waves)
+  const bool stager = NI * kWaves * RPI == TK || wave * RPI < TK;  // (D = 16: two waves)
   const int st_row = wave * RPI + lane / CPR;
   const uint32_t k_row = (uint32_t)p.k_st * 2, v_row = (uint32_t)p.v_st * 2;  // (a tile's rows span less than 2^31 bytes)
   const uint32_t k_off = st_row * k_row + ((lane % CPR) ^ swz_k(st_row)) * 16, v_off = st_row * v_row + ((lane % CPR) ^ swz_v(st_row)) * 16;
-  const int lds_base = (int)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+  constexpr int STEP = kWaves * RPI;  // rows between a wave's load instructions
+  constexpr bool APART = !DV && NS > 2;  // K tiles are requested NS - 1 tiles ahead, V tiles that pass through registers one
   u32x4 vst[NI];
-  auto request = [&](int stage, int t) __attribute__((always_inline)) {
+  // K and V of tile t (or one of them)
+  auto request = [&](auto k_tag, auto v_tag, int stage, int t) __attribute__((always_inline)) {
+    constexpr bool K = decltype(k_tag)::value, V = decltype(v_tag)::value;
     if (!stager) return;
-    const char* kt = uniform_ptr(kbase + (int64_t)t * kTile * k_row);
-    const char* vt = uniform_ptr(vbase + (int64_t)t * kTile * v_row);
+    const char* kt = K ? uniform_ptr(kbase + (int64_t)t * TK * k_row) : nullptr;
+    const char* vt = V ? uniform_ptr(vbase + (int64_t)t * TK * v_row) : nullptr;
     const int dst = __builtin_amdgcn_readfirstlane(lds_base + stage * 2 * TB + wave * 1024);
-    const int last = kv_len - 1 - t * kTile;
+    const int last = kv_len - 1 - t * TK;
 #pragma unroll
     for (int i = 0; i < NI; i++) {
-      constexpr int STEP = kWaves * RPI;
       uint32_t ko = k_off, vo = v_off;
-      if (last < kTile - 1) {  // (wave-uniform; rows past the end repeat the last one and are masked)
+      if (last < TK - 1) {  // (wave-uniform; rows past the end repeat the last one and are masked)
         int r0 = st_row;
         asm volatile("" : "+v"(r0));  // (worked out here and not kept in registers over the loop)
         int back = r0 + i * STEP - last;
         back = back < 0 ? 0 : back;
-        ko -= (uint32_t)back * k_row;
-        vo -= (uint32_t)back * v_row;
+        if (K) ko -= (uint32_t)back * k_row;
+        if (V) vo -= (uint32_t)back * v_row;
       }
-      load_to_lds(dst + i * kWaves * 1024, kt, ko + (uint32_t)(i * STEP) * k_row);
-      if (DV) load_to_lds(dst + TB + i * kWaves * 1024, vt, vo + (uint32_t)(i * STEP) * v_row);
-      else vst[i] = *(const u32x4*)(vt + (vo + (uint32_t)(i * STEP) * v_row));
+      if (K) load_to_lds(dst + i * kWaves * 1024, kt, ko + (uint32_t)(i * STEP) * k_row);
+      if (V && DV) load_to_lds(dst + TB + i * kWaves * 1024, vt, vo + (uint32_t)(i * STEP) * v_row);
+      if (V && !DV) vst[i] = *(const u32x4*)(vt + (vo + (uint32_t)(i * STEP) * v_row));
     }
   };
-  // the tile that was requested, complete in LDS for this wave
-  auto deposit = [&](int stage) __attribute__((always_inline)) {
+  constexpr std::true_type yes{};
+  constexpr std::false_type no{};
+  auto deposit_v = [&](int stage) __attribute__((always_inline)) {  // (bfloat16 V: the tile in the registers into LDS)
     if (!DV && stager) {
 #pragma unroll
       for (int i = 0; i < NI; i++) *(u32x4*)(lds + stage * 2 * TB + TB + (wave + i * kWaves) * 1024 + lane * 16) = bf16_to_f16(vst[i]);
     }
-    wait_loads();
   };
   // transposing read: lane c of a 16-lane group points at row c >> 2, columns 4 (c & 3) .. + 3 of a 4 x 16 block and
   // receives column c of it; group g takes rows 4 g .. 4 g + 3 and, sixteen rows on, 16 + 4 g .. + 3: the eight keys
   // whose scores the lane holds
-  int kaddr[KS], vaddr[NDB];
+  // (the contraction step and the block are bits of the chunk number that g and the lane leave free, so they are XORed into the address:
+  // in registers of their own, or, where none are to spare (LEAN), next to each read)
+  constexpr bool LEAN = D == 128 && WP == 32;
+  constexpr bool LEAN_V = LEAN || (D == 64 && WP == 32);
+  constexpr int NKA = LEAN ? 1 : KS, NVA = LEAN_V ? 1 : NDB;
+  int kaddr[NKA], vaddr[NVA];
 #pragma unroll
-  for (int ks = 0; ks < KS; ks++) kaddr[ks] = lds_base + c * RB + (((4 * ks + g) & (CPR - 1)) ^ swz_k(c)) * 16;
+  for (int ks = 0; ks < NKA; ks++) kaddr[ks] = lds_base + c * RB + (((4 * ks + g) & (CPR - 1)) ^ swz_k(c)) * 16;
 #pragma unroll
-  for (int db = 0; db < NDB; db++) {
+  for (int db = 0; db < NVA; db++) {
     const int row = 4 * g + (c >> 2);
     vaddr[db] = lds_base + TB + row * RB + ((2 * db + ((c & 3) >> 1)) ^ swz_v(row)) * 16 + (c & 1) * 8;
   }
+  auto kaddr_of = [&](int ks) __attribute__((always_inline)) {
+    if (!LEAN) return kaddr[LEAN ? 0 : ks];
+    int a = kaddr[0];
+    if (ks) asm volatile("v_xor_b32 %0, %1, %2" : "=v"(a) : "n"(ks * 64), "v"(kaddr[0]));
+    return a;
+  };
+  auto vaddr_of = [&](int db) __attribute__((always_inline)) {
+    if (!LEAN_V) return vaddr[LEAN_V ? 0 : db];
+    int a = vaddr[0];
+    if (db) asm volatile("v_xor_b32 %0, %1, %2" : "=v"(a) : "n"(db * 32), "v"(vaddr[0]));
+    return a;
+  };
   const float scale = p.scale_log2;
-  const int nt = (cnt_wg + kTile - 1) / kTile;  // the same for every wave of the workgroup
+  const int nt = (cnt_wg + TK - 1) / TK;  // the same for every wave of the workgroup
 
-  u32x4 ka[2][KS];  // K operands of the next 32 keys
+  constexpr int KR = LEAN ? 4 : KS;        // K operands in registers, per block of keys
+  constexpr int VR = LEAN ? 4 : NDB;       // V operands
+  u32x4 ka[2][KR];  // K operands of the next 32 keys, the first KR of KS steps
+  auto load_ka1 = [&](int at, int kb, int ks) __attribute__((always_inline)) {
+    u32x4 x = *(const __attribute__((address_space(3))) u32x4*)(kaddr_of(ks) + at + kb * 16 * RB);
+    if (D == 16 && g >= 2) x = u32x4{0u, 0u, 0u, 0u};
+    return x;
+  };
   auto load_ka = [&](int at) __attribute__((always_inline)) {
 #pragma unroll
     for (int kb = 0; kb < 2; kb++)
 #pragma unroll
-      for (int ks = 0; ks < KS; ks++) {
-        ka[kb][ks] = *(const __attribute__((address_space(3))) u32x4*)(kaddr[ks] + at + kb * 16 * RB);
-        if (D == 16 && g >= 2) ka[kb][ks] = u32x4{0u, 0u, 0u, 0u};
-      }
+      for (int ks = 0; ks < KR; ks++) ka[kb][ks] = load_ka1(at, kb, ks);
   };
   auto tile = [&](auto stage_tag, int t) __attribute__((always_inline)) {
     constexpr int S = decltype(stage_tag)::value;
-    if (t + 1 < nt) request(S ^ 1, t + 1);
-    if (t * kTile < cnt_wave) load_ka(S * 2 * TB);
+    // the wave's loads of this tile have landed (those of a tile behind it may be under way), then everyone meets: the tile is complete,
+    // and the stage of the tile before it is done with and takes the next request
+    if (DV && NS > 2 && t + 1 < nt) wait_loads<2 * NI * (NS - 2)>();
+    else wait_loads<0>();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if constexpr (APART) {
+      if (t + NS - 1 < nt) request(yes, no, (S + NS - 1) % NS, t + NS - 1);
+      if (t + 1 < nt) request(no, yes, 0, t + 1);  // (into registers)
+    } else {
+      if (t + NS - 1 < nt) request(yes, yes, (S + NS - 1) % NS, t + NS - 1);
+    }
+    if (t * TK < cnt_wave) load_ka(S * 2 * TB);
 #pragma unroll
-    for (int half = 0; half < 2; half++) {
-      const int k0 = t * kTile + 32 * half;
+    for (int part = 0; part < TK / 32; part++) {
+      const int k0 = t * TK + 32 * part;
       if (k0 < cnt_wave) {  // (wave-uniform: else none of the wave's rows sees these keys)
-        // S^T = K Q^T: s[qb][kb][j] = score of key k0 + 16 kb + 4 g + j for the lane's query of block qb; a K operand
-        // serves all blocks
+        // S^T = K Q^T: s[qb][kb][j] = score of key k0 + 16 kb + 4 g + j for the lane's query of block qb; a K operand serves all blocks
+        // (starting from named zeros: with the zero written into the first product the 128-wide kernel spills 22 registers)
         f32x4 s[QB][2];
+#pragma unroll
+        for (int qb = 0; qb < QB; qb++) s[qb][0] = s[qb][1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ks = 0; ks < KS; ks++)
 #pragma unroll
-          for (int kb = 0; kb < 2; kb++)
+          for (int kb = 0; kb < 2; kb++) {
 #pragma unroll
-            for (int qb = 0; qb < QB; qb++) s[qb][kb] = MfmaS<T>::run(ka[kb][ks], qreg[qb][ks], ks == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : s[qb][kb]);
+            for (int qb = 0; qb < QB; qb++) s[qb][kb] = MfmaS<T>::run(ka[kb][ks % KR], qreg[qb][ks], s[qb][kb]);
+            if (ks + KR < KS) {
+              ka[kb][ks % KR] = load_ka1(S * 2 * TB + 32 * part * RB, kb, ks + KR);
+              __builtin_amdgcn_sched_barrier(0);
+            }
+          }
         if (k0 + 32 > cnt_first) {  // (wave-uniform: the wave's first row, which sees the fewest keys, does not see the whole step)
 #pragma unroll
           for (int qb = 0; qb < QB; qb++) {
-            const int rel = cnt[qb] - k0 - 4 * g;
+            const int rel = cnt[qb] - k0;
 #pragma unroll
-            for (int kb = 0; kb < 2; kb++)
-#pragma unroll
-              for (int j = 0; j < 4; j++) s[qb][kb][j] = 16 * kb + j < rel ? s[qb][kb][j] : -INFINITY;
+            for (int e = 0; e < 8; e++) s[qb][e / 4][e % 4] = 16 * (e / 4) + e % 4 < rel ? s[qb][e / 4][e % 4] : -INFINITY;
           }
         }
         // P = exp2(S * scale - m) with the running maxima as they are; they are raised, and the step done again, only if some
@@ -331,45 +392,69 @@ __global__ __launch_bounds__(kWaves * 64, D == 128 ? 2 : QB == 2 && D == 64 && !
         // (the scores' registers are free now and take the next K operands; asked for any earlier, these or the V operands
         // below spill: 64-wide heads, 8 x 2048 tokens, 217 us instead of 168 (without l_pv) with the V operands read before the softmax)
         __builtin_amdgcn_sched_barrier(0);
-        u32x4 va[NDB];
-#pragma unroll
-        for (int db = 0; db < NDB; db++) {
-          const int at = vaddr[db] + S * 2 * TB + 32 * half * RB;
+        u32x4 va[VR];  // V operand of block db in va[db % VR]
+        auto load_va = [&](int db) __attribute__((always_inline)) {
+          const int at = vaddr_of(db) + S * 2 * TB + 32 * part * RB;
           const i16x4 xa = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_ptr)at);
           const i16x4 xb = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_ptr)(at + 16 * RB));
           const u32x2 wa = __builtin_bit_cast(u32x2, xa), wb = __builtin_bit_cast(u32x2, xb);
-          va[db] = u32x4{wa[0], wa[1], wb[0], wb[1]};
-        }
-        if (half == 0) load_ka(S * 2 * TB + 32 * RB);
+          return u32x4{wa[0], wa[1], wb[0], wb[1]};
+        };
+#pragma unroll
+        for (int db = 0; db < VR; db++) va[db] = load_va(db);
+        if (32 * (part + 1) < TK) load_ka(S * 2 * TB + 32 * (part + 1) * RB);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int db = 0; db < NDB; db++)
+        for (int db = 0; db < NDB; db++) {
 #pragma unroll
-          for (int qb = 0; qb < QB; qb++) oacc[qb][db] = MfmaS<F16>::run(va[db], pk[qb], oacc[qb][db]);
+          for (int qb = 0; qb < QB; qb++) oacc[qb][db] = MfmaS<F16>::run(va[db % VR], pk[qb], oacc[qb][db]);
+          if (db + VR < NDB) {
+            va[db % VR] = load_va(db + VR);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
 #pragma unroll
         for (int qb = 0; qb < QB; qb++) l_pv[qb] = MfmaS<F16>::run(u32x4{kOnes, kOnes, kOnes, kOnes}, pk[qb], l_pv[qb]);
       }
     }
-    // the next tile is in the other stage (last read one barrier ago), then everyone meets: that tile is complete and this
-    // one is done with
-    if (t + 1 < nt) deposit(S ^ 1);
-    __syncthreads();
+    if (!DV && t + 1 < nt) deposit_v((S + 1) % NS);
   };
-  if (nt > 0) {
-    request(0, 0);
-    deposit(0);
-    __syncthreads();
+#pragma unroll
+  for (int t = 0; t < NS - 1; t++) {
+    if (t < nt) {
+      if (APART && t > 0) request(yes, no, t, t);
+      else request(yes, yes, t, t);
+    }
   }
-  for (int t = 0; t < nt; t += 2) {  // (the stage is a constant of the code)
+  if (nt > 0) deposit_v(0);
+  for (int t = 0; t < nt; t += NS) {  // (the stage is a constant of the code)
     tile(std::integral_constant<int, 0>{}, t);
     if (t + 1 < nt) tile(std::integral_constant<int, 1>{}, t + 1);
+    if constexpr (NS == 3)
+      if (t + 2 < nt) tile(std::integral_constant<int, 2>{}, t + 2);
   }
 
-  // ---- epilogues (the 128-wide kernel's), block by block of 16 positions ----
+  // ---- epilogues (the 128-wide kernel's) ----
+  // O leaves through LDS (MODE 0 and 1, 32 positions per wave): written as the lanes hold it, a store touches 16 rows with 32 or 64 bytes
+  // each, a request per row to the L2s, and turned round whole lines of a few rows: 16 x 1024 tokens 32/8 199 -> 190 us in
+  // place and 207 -> 201 as fp32, 16 x 512 bf16 72 -> 66 (128-wide heads).  The small launches of 16 positions write directly (1 x 100 9.2 us, turned round 9.6).
+  constexpr bool TURNED = MODE != 2 && WP == 32;
+  constexpr int ES = MODE == 1 ? 2 : 4;                // bytes per element of O
+  constexpr int RBO = D * ES < 256 ? D * ES : 256;     // bytes of a row that are turned round at a time
+  constexpr int CO = RBO / 16;                         // 16-byte chunks of them, XORed with a function of the row as the tiles' are
+  static_assert(!TURNED || kWaves * WP * RBO <= kStateOff, "the tiles' LDS holds the waves' rows");
+  auto o_chunk = [](int row, int chunk) { return row * RBO + ((chunk ^ (row / (256 / RBO) & (CO - 1))) << 4); };
+  char* const o_lds = lds + wave * WP * RBO;
+  if (MODE == 1 && nt == 0) wait_loads<0>();  // (else the loop has waited for the old m and l)
+  if (TURNED) __syncthreads();                // (the last tile is done with)
+  if (m0 >= q_len) return;                    // (wave-uniform: a wave without positions; it only helped to stage)
+  // (the lane's numbers are worked out again and not kept over the loop)
+  const int lane_e = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), c_e = lane_e & 15, g_e = lane_e >> 4;
+  uint32_t rows = 0;      // (MODE 1) which of the wave's rows are written
+  float factor[QB];       // (MODE 0) of the row's O
 #pragma unroll
   for (int qb = 0; qb < QB; qb++) {
     const int mb = m0 + 16 * qb;
-    if (mb >= q_len) break;  // (wave-uniform: a block without positions; it only helped to stage)
     const float l_tot = col_sum(l_run[qb]);
     // (0 exactly if the row saw no key.  A NaN score makes the sum NaN: it counts as a key, so that the row's outputs and its running
     // state become NaN, as they do in the reference, and no step before or after hides it)
@@ -379,49 +464,57 @@ __global__ __launch_bounds__(kWaves * 64, D == 128 ? 2 : QB == 2 && D == 64 && !
     // Against 64 bits the fp32 partial of N(0, 1) * 0.5 inputs is off by 1.70e-4 to 1.72e-4 at 1000 to 3000 tokens of 64-wide heads,
     // 1.74e-4 to 1.75e-4 with maxima that never lag and 1.76e-4 with neither.  The sum that (m, l) and the LSE state stays the fp32 one.
     const float fix = l_pv[qb][0] == 0.f ? 0.f : l_tot / l_pv[qb][0];
-#pragma unroll
-    for (int db = 0; db < NDB; db++) oacc[qb][db] *= fix;
-    const bool here = in_range[qb];
-    const int64_t tok = o_start + (here ? mb + c : mb);
+    const int m_e = mb + c_e;
+    const bool here = m_e < q_len;
+    const int64_t tok = o_start + (here ? m_e : m0);  // (a lane without a position: the wave's first, never written)
     if (MODE == 0) {
+      factor[qb] = seen ? fix * (1.f / l_tot) : 0.f;
       if (here) {
-        const float inv = seen ? 1.f / l_tot : 0.f;
-        float* orow = (float*)p.o + tok * p.o_st + (int64_t)h * p.o_sh;
+        if (!TURNED) {
+          float* orow = (float*)p.o + tok * p.o_st + (int64_t)h * p.o_sh + 4 * g_e;
 #pragma unroll
-        for (int db = 0; db < NDB; db++) *(f32x4*)(orow + db * 16 + 4 * g) = oacc[qb][db] * inv;
-        if (g == 0) p.lse[tok * p.hq + h] = seen ? (m_run[qb] + __builtin_amdgcn_logf(l_tot)) * kLn2 : -INFINITY;
+          for (int db = 0; db < NDB; db++) *(f32x4*)(orow + 16 * db) = oacc[qb][db] * factor[qb];
+        }
+        if (g_e == 0) p.lse[tok * p.hq + h] = seen ? (m_run[qb] + __builtin_amdgcn_logf(l_tot)) * kLn2 : -INFINITY;
       }
     }
     if (MODE == 1) {
       // the reference's update of (o, m, l); a row in its start state (m = -inf, l = 0) may hold anything in o
-      const int64_t at = tok * p.ml_st + (int64_t)h * p.ml_sh;
-      const float m_old = p.m[at], l_old = p.l[at];
+      const float m_old = *(const float*)(lds + kStateOff + wave * 256 + (16 * qb + c_e) * 4);
+      const float l_old = *(const float*)(lds + kStateOff + wave * 256 + 128 + (16 * qb + c_e) * 4);
       const float M = fmaxf(m_run[qb], m_old);
       const bool upd = here && seen;  // (a row that saw a key has a maximum, unless all its scores are NaN)
-      float L = 0.f;
-      if (upd) {
-        const float w_old = l_old * exp2_diff(m_old, M);
-        const float w_new = exp2_diff(m_run[qb], M);
-        L = w_old + l_tot * w_new;
-        const float inv = 1.f / L;
-        uint16_t* orow = (uint16_t*)p.o + tok * p.o_st + (int64_t)h * p.o_sh;
+      const float w_old = upd ? l_old * exp2_diff(m_old, M) : 0.f;
+      const float w_new = exp2_diff(m_run[qb], M) * fix;
+      const float L = w_old + l_tot * exp2_diff(m_run[qb], M);
+      const float inv = 1.f / L;
+      uint16_t* orow = (uint16_t*)p.o + tok * p.o_st + (int64_t)h * p.o_sh + 4 * g_e;
+      u32x2 old[NDB];
 #pragma unroll
-        for (int db = 0; db < NDB; db++) {
-          float o0 = 0.f, o1 = 0.f, o2 = 0.f, o3 = 0.f;
-          if (w_old != 0.f) {
-            const u32x2 old = *(const u32x2*)(orow + db * 16 + 4 * g);
-            unpack2<T>(old[0], o0, o1);
-            unpack2<T>(old[1], o2, o3);
-          }
-          const float r0 = (o0 * w_old + oacc[qb][db][0] * w_new) * inv, r1 = (o1 * w_old + oacc[qb][db][1] * w_new) * inv;
-          const float r2 = (o2 * w_old + oacc[qb][db][2] * w_new) * inv, r3 = (o3 * w_old + oacc[qb][db][3] * w_new) * inv;
-          *(u32x2*)(orow + db * 16 + 4 * g) = u32x2{pack2<T>(r0, r1), pack2<T>(r2, r3)};
+      for (int db = 0; db < NDB; db++) old[db] = u32x2{0u, 0u};
+      // (a wave none of whose rows carries an earlier step's result, as in the first step of a ring and in a prefill on one GPU, does not
+      // read o; w_old is NaN if an old sum or maximum is)
+      if (__builtin_amdgcn_ballot_w64(w_old != 0.f) != 0) {
+        if (w_old != 0.f) {
+#pragma unroll
+          for (int db = 0; db < NDB; db++) old[db] = *(const u32x2*)(orow + 16 * db);
         }
       }
-      // (the four lanes of a column all read the old m and l above, in the same instruction as the one that writes them below)
-      if (upd && g == 0) {
-        p.m[at] = M;
-        p.l[at] = L;
+#pragma unroll
+      for (int db = 0; db < NDB; db++) {
+        float o0, o1, o2, o3;
+        unpack2<T>(old[db][0], o0, o1);
+        unpack2<T>(old[db][1], o2, o3);
+        const f32x4& x = oacc[qb][db];
+        const u32x2 res = u32x2{pack2<T>((o0 * w_old + x[0] * w_new) * inv, (o1 * w_old + x[1] * w_new) * inv),
+                                pack2<T>((o2 * w_old + x[2] * w_new) * inv, (o3 * w_old + x[3] * w_new) * inv)};
+        if (TURNED) *(u32x2*)(o_lds + o_chunk(16 * qb + c_e, 2 * db + (g_e >> 1)) + (g_e & 1) * 8) = res;
+        else if (upd) *(u32x2*)(orow + 16 * db) = res;
+      }
+      rows |= (uint32_t)(__builtin_amdgcn_ballot_w64(upd) & 0xffffu) << 16 * qb;
+      if (upd && g_e == 0) {
+        p.m[tok * p.ml_st + (int64_t)h * p.ml_sh] = M;
+        p.l[tok * p.ml_st + (int64_t)h * p.ml_sh] = L;
       }
     }
     if (MODE == 2) {
@@ -435,22 +528,46 @@ __global__ __launch_bounds__(kWaves * 64, D == 128 ? 2 : QB == 2 && D == 64 && !
         const float w_old = exp2_diff(a_old, top);
         const float w_new = __builtin_amdgcn_exp2f(a_new - top);
         const float W = w_old + w_new;
-        const float c_old = w_old / W, c_new = w_new / (W * l_tot);
-        float* orow = (float*)p.o + tok * p.o_st + (int64_t)h * p.o_sh;
+        const float c_old = w_old / W, c_new = w_new / (W * l_tot) * fix;
+        float* orow = (float*)p.o + tok * p.o_st + (int64_t)h * p.o_sh + 4 * g_e;
 #pragma unroll
         for (int db = 0; db < NDB; db++) {
           // an empty row (lse = -inf) may hold anything: its old values are dropped, not multiplied by zero
-          const f32x4 keep = w_old != 0.f ? *(const f32x4*)(orow + db * 16 + 4 * g) : f32x4{0.f, 0.f, 0.f, 0.f};
-          *(f32x4*)(orow + db * 16 + 4 * g) = keep * c_old + oacc[qb][db] * c_new;
+          const f32x4 keep = w_old != 0.f ? *(const f32x4*)(orow + 16 * db) : f32x4{0.f, 0.f, 0.f, 0.f};
+          *(f32x4*)(orow + 16 * db) = keep * c_old + oacc[qb][db] * c_new;
         }
         new_lse = (top + __builtin_amdgcn_logf(W)) * kLn2;
       }
-      if (upd && g == 0) p.lse[tok * p.hq + h] = new_lse;
+      if (upd && g_e == 0) p.lse[tok * p.hq + h] = new_lse;
+    }
+  }
+  if (TURNED) {
+    // (four-byte words of a row's 16 bytes: o_stride_t and o_stride_h are multiples of four elements)
+    typedef u32x4 ChunkAt8 __attribute__((aligned(8)));
+    char* obase = (char*)p.o + ((o_start + m0) * p.o_st + (int64_t)h * p.o_sh) * ES;
+    const int n_rows = q_len - m0 < WP ? q_len - m0 : WP;
+#pragma unroll
+    for (int half = 0; half < D * ES / RBO; half++) {
+      if (MODE == 0) {
+#pragma unroll
+        for (int qb = 0; qb < QB; qb++)
+#pragma unroll
+          for (int db = half * RBO / 64; db < NDB && db < (half + 1) * RBO / 64; db++)
+            *(f32x4*)(o_lds + o_chunk(16 * qb + c_e, 4 * db - half * CO + g_e)) = oacc[qb][db] * factor[qb];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (the wave's own rows: its LDS instructions keep their order)
+#pragma unroll
+      for (int it = 0; it < WP * CO / 64; it++) {
+        const int r = it * (64 / CO) + lane_e / CO;
+        const u32x4 v = *(const u32x4*)(o_lds + o_chunk(r, lane_e % CO));
+        if (MODE == 1 ? (rows >> r & 1) != 0 : r < n_rows) *(ChunkAt8*)(obase + r * p.o_st * ES + half * RBO + lane_e % CO * 16) = v;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
   }
 }
 
-// Whether a request's place among the ids moves on from tile to tile (TURN).  Ids go to the eight XCDs in turn and within one to its four
+// Whether a request's place among the ids moves on from tile to tile.  Ids go to the eight XCDs in turn and within one to its four
 // shader engines.  If the ids of two tiles of a request are a multiple of 32 apart, all its workgroups share one shader engine of an
 // XCD, and while only the longest requests have a tile left to start, the others idle: 8 sequences of 1000 to 3000 tokens, 32/8 heads
 // of 64, had 2 workgroups on a CU until half of the launch was over, some 4 and some 1, where 8 x 2048 keep 3.9.  Turning places
@@ -458,18 +575,57 @@ __global__ __launch_bounds__(kWaves * 64, D == 128 ? 2 : QB == 2 && D == 64 && !
 //   8 x 1000..3000 32/8 183 | 165   2 x 1206..3618 64/8 144 | 123   4 x 120..3615 64/8 bf16 87.9 | 61.8   4 x 688..2064 32/32 53.2 | 47.3
 //   4 x 2582..5165 32/8 bf16 344 | 314   8 x 1304..2608 12/12 88.8 | 79.5   16 x 31..959 64/8 57.3 | 53.5
 // At other distances (11 x 388..1166 32/8 44.8 | 47.1; distance 6 of the eights 9 % better to 4 % worse), with fewer than 16 tiles
-// (8 x 280..842 32/32 31.5 | 33.3) and with equal lengths turning gains nothing: those keep the kernel without it.
+// (8 x 280..842 32/32 31.5 | 33.3) and with equal lengths turning gains nothing: there the places stay.
+bool ragged(const lsattn_prefill_args* a) { return a->total_q_rows > 0 && a->total_q_rows * 10 <= (int64_t)a->batch * a->max_q_len * 9; }
 bool requests_take_turns(const lsattn_prefill_args* a, int64_t ids_per_tile, int64_t tiles) {
-  return ids_per_tile * a->batch % 32 == 0 && tiles >= 16 && a->total_q_rows > 0 && a->total_q_rows * 10 <= (int64_t)a->batch * a->max_q_len * 9;
+  return ids_per_tile % 32 == 0 && tiles >= 16 && ragged(a);
 }
 
-template <typename T, int D, int MODE, bool DV, int QB, bool TURN = false> int launch_rows(SmallParams p, const lsattn_prefill_args* a, hipStream_t st) {
-  const int64_t rows_wg = (kWaves * QB * 16) >> p.pack_shift;
-  for (int64_t tiles = (a->max_q_len + rows_wg - 1) / rows_wg; tiles > 0; tiles -= kMaxTiles) {
+// How many requests the grid takes at a time (a bunch), the heaviest tiles of all of them first.  All of the batch starts the heaviest work of the
+// launch first,
+// and is best for ragged batches; but every layer of tiles then reads the K/V of the whole batch again, which past the
+// L2s' 32 MB comes from beyond them, so bunches hold about as much.  And short prompts of about equal length leave the CUs unevenly filled that
+// way (their workgroups come in layers of equal length): in bunches of some 512 workgroups, light tiles of one run beside heavy
+// ones of the next.  Measured (microseconds, 1, 2, 4, 8, 16 and 32 requests at a time up to the batch, 128-wide heads):
+//   16 x 512 32/32 (8 MB each) 77 75 78 86 99   16 x 1024 32/32 (16 MB) 231 229 235 243 262   32 x 512 32/32 170 169 171 182 197 201
+//   32 x 256 32/8 52.2 50.6 47.9 52.0 61.4 61.4   16 x 256 32/8 34.6 32.8 30.8 30.5 35.6   8 x 512 32/8 44.3 42.0 37.8 43.4   16 x 512 32/8 71 67 64 70 72
+//   16 x 1024 32/8 216 207 204 201 206   4 x 1024 32/8 62.7 57.9 55.3   ragged: 8 x 100..2000 32/8 70.6 68.9 64.3 61.2, 20 x 200..800 32/8 81 78 72 80 80 71 (all 20)
+// and 64-wide: 16 x 1024 32/32 119 120 125 128 140   8 x 2048 32/32 198 192 189 210   16 x 512 32/8 44.3 42.2 39.9 45.1 44.4   16 x 1024 32/8 117 112 112 108 108
+int64_t requests_per_bunch(const lsattn_prefill_args* a, int64_t ids, int64_t tiles) {
+  int64_t bunches = 1;
+  const int64_t kv_bytes = a->total_kv_rows * a->num_kv_heads * a->head_dim * 4;
+  if (kv_bytes >= 2 * kL2Bytes) bunches = kv_bytes / kL2Bytes;
+  const int64_t wgs = ids * tiles * a->batch, resident = (a->head_dim == 128 ? 3 : 4) * kCUs;
+  if (a->total_q_rows > 0 && !ragged(a) && a->max_q_len <= 512 && wgs > resident && wgs / kBunchWorkgroups > bunches) bunches = wgs / kBunchWorkgroups;
+  if (bunches > a->batch) bunches = a->batch;
+  return (a->batch + bunches - 1) / bunches;
+}
+
+struct Order {
+  int64_t bunch;
+  bool turns;
+};
+// (of the shape with 32 positions per wave; launches of the other are small)
+Order order_of(const lsattn_prefill_args* a, int pack_shift) {
+  const int64_t rows_wg = (kWaves * 32) >> pack_shift, tiles = (a->max_q_len + rows_wg - 1) / rows_wg, ids = a->num_q_heads >> pack_shift;
+  const int64_t fits = tiles < kMaxIds ? kMaxIds / tiles : 1;  // (the grid's second index)
+  int64_t bunch = requests_per_bunch(a, ids, tiles);
+  bunch = bunch < fits ? bunch : fits;
+  return {bunch, requests_take_turns(a, ids * bunch, tiles)};
+}
+
+template <typename T, int D, int MODE, bool DV, int WP> int launch_rows(SmallParams p, const lsattn_prefill_args* a, hipStream_t st) {
+  const int64_t rows_wg = (kWaves * WP) >> p.pack_shift;
+  const Order order = WP == 32 ? order_of(a, p.pack_shift) : Order{p.batch, false};
+  p.bunch = (int32_t)order.bunch;
+  p.d_bunch = fast_div((uint32_t)p.bunch);
+  p.turns = order.turns;
+  const int64_t most = kMaxIds / p.bunch;  // tiles of one launch
+  const unsigned bunches = (unsigned)((a->batch + p.bunch - 1) / p.bunch);
+  for (int64_t tiles = (a->max_q_len + rows_wg - 1) / rows_wg; tiles > 0; tiles -= most) {
     p.last_tile = (int32_t)(tiles - 1);
-    LSATTN_LAUNCH_KERNEL((prefill_small_kernel<T, D, MODE, DV, QB, TURN>),
-                         dim3((unsigned)(p.hkv * p.group), (unsigned)a->batch, (unsigned)(tiles < kMaxTiles ? tiles : kMaxTiles)),
-                         dim3(kWaves * 64), 0, st, p);
+    LSATTN_LAUNCH_KERNEL((prefill_small_kernel<T, D, MODE, DV, WP>),
+                         dim3((unsigned)(p.hkv * p.group), (unsigned)((tiles < most ? tiles : most) * p.bunch), bunches), dim3(kWaves * 64), 0, st, p);
     const int rc = check_launch();
     if (rc != LSATTN_OK) return rc;
   }
@@ -497,14 +653,16 @@ int64_t workgroups(const lsattn_prefill_args* a, int pack_shift, int blocks) {
 template <typename T, int D, int MODE, bool DV> int launch(const SmallParams& p, const lsattn_prefill_args* a, hipStream_t st) {
   if (a->num_q_heads > 65535 || a->batch > 65535) return LSATTN_ERR_INVALID_ARG;
   switch (prefill_small_route(a)) {
-    case LSATTN_ROUTE_SMALL_16: return launch_rows<T, D, MODE, DV, 1>(p, a, st);
-    case LSATTN_ROUTE_SMALL_TURNS: return launch_rows<T, D, MODE, DV, 2, true>(p, a, st);
-    default: return launch_rows<T, D, MODE, DV, 2>(p, a, st);
+    case LSATTN_ROUTE_SMALL_16: return launch_rows<T, D, MODE, DV, 16>(p, a, st);
+    default: return launch_rows<T, D, MODE, DV, 32>(p, a, st);
   }
 }
 
 template <typename T, int MODE, bool DV> int launch_128(const SmallParams& p, const lsattn_prefill_args* a, hipStream_t st) {
-  return prefill_small_route(a) == LSATTN_ROUTE_SMALL_16 ? launch_rows<T, 128, MODE, DV, 1>(p, a, st) : launch_rows<T, 128, MODE, DV, 2>(p, a, st);
+  switch (prefill_small_route(a)) {
+    case LSATTN_ROUTE_SMALL_16: return launch_rows<T, 128, MODE, DV, 16>(p, a, st);
+    default: return launch_rows<T, 128, MODE, DV, 32>(p, a, st);
+  }
 }
 
 template <typename T, int MODE, bool DV> int launch_d(const SmallParams& p, const lsattn_prefill_args* a, hipStream_t st) {
@@ -529,24 +687,28 @@ template <typename T, bool DV> int launch_mode(const SmallParams& p, const lsatt
 }  // namespace
 
 // Short prompts of 128-wide heads: the kernel of prefill.hip spends 9 us on starting and ending whatever it computes (eight
-// waves of 256 registers that fill 128 KB of rings and some 40 KB of code before the first product); this one has a
-// quarter of the code, workgroups of 64 rows (128) and two of them per CU, converts a bfloat16 V on the way (no launch in front
-// that copies it), but reads LDS four times (twice) as much per product, and a tile takes longer (below).  Measured over 472 launches (1 to
-// 32 prompts of 32 to 2048 tokens, equal or log-uniform over a factor of 8, 32/32, 32/8, 64/8 and 8/1 heads; both epilogues;
-// microseconds, the kernel of prefill.hip | 16 positions per wave | 32; bf16 with its copy of V):
-//   1 x 100 MHA f16 10.9 | 5.5 | 7.8        1 x 512 32/8 f16 15.6 | 12.3 | 16.5    16 x 128 MHA f16 25.6 | 19.6 | 17.7
-//   1 x 30 32/8 bf16 12.4 | 4.9 | 6.4       7 x 67..269 32/8 13.5 | 9.3 | 10.8      16 x 256 MHA f16 37.4 | 45.1 | 36.7
-//   8 x 512 32/8 f16 36.6 | 43.6 | 37.9     1 x 1024 32/8 f16 20.8 | 21.5 | 26.9    (neither is taken)
-// 16 positions per wave win up to two and a half workgroups per CU (with one head per workgroup, which leaves the other kernel
-// four times the rows to mask, up to six, for prompts of up to 512 tokens), 32 up to six and 256 tokens; the geometric
-// mean over the launches the rule takes is 25 to 35 % below the other kernel, the worst is 5 % above it.
-// The keys: a tile of 64 costs a wave 0.95 us here (bf16 V 1.5) against 0.56 in the 128-row shape, which a launch with one long
-// context waits for, so the longest request decides (whole call, 32/8 heads, the other kernel | this one, f16, then bf16):
+// waves of 256 registers that fill 128 KB of rings and some 40 KB of code before the first product; its four-wave shape 12 us, two workgroups on a
+// CU).  This one has a quarter of the code and, with 32 positions per wave, three workgroups on a CU, of which one starts or ends while the others
+// compute, at the same rate per tile; it converts a bfloat16 V on the way (no launch in front that copies it).  16 positions
+// per wave are for launches that do not fill the chip.  Measured over 700 launches (1 to 40 prompts of 32 to 2048 tokens, equal or
+// log-uniform over a factor of up to 20, a fifth behind contexts; 32/32, 32/8, 64/8 and 8/1 heads; both epilogues; microseconds, the
+// kernel of prefill.hip | 16 positions per wave | 32; bf16 with its copy of V):
+//   1 x 636 32/8 24.2 | 19.9 | 24.4         9 x 222 at most 32/32 32.9 | 18.3 | 20.4      9 x 126 at most 32/32 bf16 24.7 | 9.7 | 13.2
+//   14 x 99 32/8 bf16 23.3 | 19.2 | 16.3    30 x 100 32/8 32.4 | 27.5 | 24.2              12 x 324 at most 32/8 33.0 | 35.1 | 28.8
+//   16 x 512 32/8 76 | 86 | 65              13 x 1317 at most 32/8 72.4 | 75.1 | 59.6     4 x 1416 32/32 114 | 122 | 100
+//   16 x 1024 32/8 200 | 290 | 191          20 x 200..800 32/8 91 | - | 71                16 x 512 32/32 88 | 127 | 76
+//   3 x 1012 32/8 38.0 | 37.3 | 39.8        2 x 1594 32/8 64.3 | 75.8 | 65.8              19 x 1244 64/8 608 | 847 | 625
+// 16 positions win up to two and a half workgroups per CU (four with one head per workgroup, which leaves each wave fewer rows to mask);
+// 32 from there on, for prompts beyond 768 tokens from three (of its own) per CU.  Equal prompts beyond 1280 tokens in launches of ten and
+// more per CU keep the other kernel, whose loop is the faster one.
+// The geometric mean over the launches the rule takes is 32 % below the other kernel; the worst is 6 % above it.
+// The keys: a chunk behind a context waits for its longest request, and a tile of a lone workgroup takes longer here (0.95 us against 0.56 in the
+// 128-row shape), so the longest request decides (whole call, 32/8 heads, the other kernel | this one with 16 positions, f16, then bf16):
 //   8 x 64 rows behind 600 keys each 20.8 | 15.7, 28.0 | 18.7      4 x 100 behind 1000 each 24.9 | 21.7, 30.5 | 25.9      1 x 200 behind 1024 22.1 | 19.8, 25.2 | 24.0
 //   2 x 100, one behind 1900 30.6 | 31.8, 34.5 | 39.8      8 x 64, one behind 7500 79.8 | 108.8, 88 | 169      16 x 64, one behind 15000 145 | 264, 155 | 352
 // The host knows no lengths, only bounds: what total_kv_rows holds beyond the query rows may all belong to one request.
 int prefill_short_blocks(const lsattn_prefill_args* a) {
-  if (a->head_dim != 128 || a->kv_cuts > 1 || a->o_b_start_loc || a->max_q_len <= 0 || a->max_q_len > kShortMaxRows || a->batch <= 0 || a->num_kv_heads <= 0)
+  if (a->head_dim != 128 || a->kv_cuts > 1 || a->o_b_start_loc || a->max_q_len <= 0 || a->max_q_len > kShortMaxKeys || a->batch <= 0 || a->batch > kMaxIds || a->num_kv_heads <= 0)
     return 0;
   int64_t longest = kShortMaxKeys + 1;
   if (a->total_kv_rows > 0) {
@@ -563,16 +725,18 @@ int prefill_short_blocks(const lsattn_prefill_args* a) {
   if (tn.prefill_rows || tn.prefill_order || tn.prefill_pack) return 0;  // (choices among the 128-wide kernel's shapes)
   const int pack = pack_shift_of(a);
   const int64_t one = workgroups(a, pack, 1), two = workgroups(a, pack, 2);
-  if (one <= 5 * kCUs / 2 || (pack == 0 && a->max_q_len <= 512 && one <= 6 * kCUs)) return 1;
-  return a->max_q_len <= 256 && two <= 6 * kCUs ? 2 : 0;
+  if (longest <= 1024) {
+    if (a->max_q_len <= 768) return one <= 5 * kCUs / 2 || (pack == 0 && a->max_q_len <= 512 && one <= 4 * kCUs) ? 1 : 2;
+  } else if (a->max_q_len <= 768) {
+    return 0;
+  }
+  return two >= 3 * kCUs && (a->max_q_len <= 1280 || two <= 10 * kCUs || ragged(a)) ? 2 : 0;
 }
 
 int prefill_small_route(const lsattn_prefill_args* a) {
-  if (a->head_dim == 128) return prefill_short_blocks(a) == 1 ? LSATTN_ROUTE_SMALL_16 : LSATTN_ROUTE_SMALL_32;
   const int pack = pack_shift_of(a);
-  if (workgroups(a, pack, 2) < 3 * kCUs) return LSATTN_ROUTE_SMALL_16;
-  const int64_t rows_wg = (kWaves * 2 * 16) >> pack;
-  return requests_take_turns(a, a->num_q_heads >> pack, (a->max_q_len + rows_wg - 1) / rows_wg) ? LSATTN_ROUTE_SMALL_TURNS : LSATTN_ROUTE_SMALL_32;
+  if (a->head_dim == 128 ? prefill_short_blocks(a) == 1 : workgroups(a, pack, 2) < 3 * kCUs) return LSATTN_ROUTE_SMALL_16;
+  return order_of(a, pack).turns ? LSATTN_ROUTE_SMALL_TURNS : LSATTN_ROUTE_SMALL_32;
 }
 
 // One prefill step with head_dim 16, 32 or 64, or a short one with 128 (arguments already validated; epilogue `mode` as in the 128-wide kernel).
@@ -603,7 +767,6 @@ int launch_prefill_small(const lsattn_prefill_args* a, int mode, hipStream_t st)
   p.d_hkv = fast_div((uint32_t)p.hkv);
   p.d_peers = fast_div((uint32_t)p.peers);
   p.batch = (int32_t)a->batch;
-  p.d_batch = fast_div((uint32_t)p.batch);
   p.scale_log2 = a->sm_scale * kLog2e;
   p.o = a->o;
   p.o_st = a->o_stride_t;

@@ -415,6 +415,22 @@ def test_short_prompts_kernel_goes_by_the_longest_request():
     assert _route(1, 769, heads, total_q=769, total_kv=769) == ROWS_128
 
 
+def test_short_prompts_kernel_goes_by_the_workgroups_and_the_longest_prompt():
+    """With 32 positions per wave it takes prompts of up to 768 tokens that are too many for 16, longer ones from three workgroups per
+    CU on, and beyond 1280 tokens equal ones only up to ten."""
+    heads = (32, 8)  # (32 positions of four heads: 8 workgroups per 32 tokens)
+    own = lambda batch, n, **kw: _route(batch, n, heads, total_q=batch * n, total_kv=batch * n, **kw)
+    assert own(2, 640) == SMALL_16 and own(4, 640) == SMALL_32 and own(4, 768) == SMALL_32
+    assert own(3, 990) not in (SMALL_16, SMALL_32) and own(3, 1000) == SMALL_32
+    assert own(3, 1024) == own(3, 1025) == SMALL_32 and own(2, 1500) not in (SMALL_16, SMALL_32, SMALL_TURNS)
+    assert own(16, 1280) == SMALL_32 and own(16, 1281) == ROWS_256 and own(5, 1700) == SMALL_32
+    assert _route(16, 2000, heads, total_q=14000, total_kv=14000) == SMALL_TURNS and own(16, 2000) == ROWS_256
+    assert _route(8, 2049, heads, total_q=5000, total_kv=5000) == ROWS_256
+    assert _route(16, 1000, heads, total_q=16000, total_kv=17100) == HALF  # (one of them behind 1100 more)
+    assert _route(16, 1000, heads, total_q=16000) == _route(16, 1000, heads) == HALF  # (nothing known of the keys)
+    assert _route(70000, 16, heads, total_q=70000 * 16, total_kv=70000 * 16) not in (SMALL_16, SMALL_32, SMALL_TURNS)  # (past the grid's index)
+
+
 def test_prefill_route_names_a_kernel_for_every_step_and_none_for_others():
     assert _route(24, 256, (32, 32), total_q=1800, total_kv=1800) == SMALL_32
     assert _route(8, 3000, (32, 8), 64, total_q=16000, total_kv=16000) == SMALL_TURNS
