@@ -5,7 +5,7 @@
 //   add / drop one reference on a list of slots and count          (add_refs :73-79, decrease_refs :82-88)
 // `mem_state` is int32 per slot, 0 = free.  All of it is integer work on a few MB, bound by launch latency and
 // by one pass over the state array; two short launches replace the reference's nonzero / slice / compare chains (three for
-// pools of more than 8 million slots), one for the reference counts of up to 4096 slots.
+// pools of more than 8 million slots, one for an alloc from up to 65536), one for the reference counts of up to 4096 slots.
 #include "common.hip.h"
 
 namespace lsattn {
@@ -230,6 +230,112 @@ __global__ __launch_bounds__(kPoolThreads) void pool_take_kernel(int32_t* __rest
 }
 
 // ---------------------------------------------------------------------------------------------------
+// alloc of a pool of up to kPoolOneGroup slots in one launch: one workgroup walks it from the front, kScanSlots at a time with the next
+// two lots under way, and stops behind the last slot it takes.  Every wave has 1024 slots in a row of a lot, so that ranks need one count
+// per wave.  Bound by the latency of its first load and, past that, by issue: 0.8 us for a lot without a free slot, 1.5 for one that has some.
+// 24 slots of 65536, device time, the two launches above | this one: half of the pool free 6.1 | 4.0, the last slots only 7.1 | 6.9, scattered
+// over the whole pool 7.0 | 7.8 (256 of them 7.3 | 10.5); and the host has one launch less, 2 us of a decode layer's pass.  Larger pools
+// that are full up to their end would pay more than that, so they keep the two launches, which read the pool on all CUs.
+// ---------------------------------------------------------------------------------------------------
+constexpr int64_t kPoolOneGroup = 65536;
+constexpr int kScanPieces = 4, kScanSlots = 1024 * 4 * kScanPieces;
+__global__ __launch_bounds__(1024) void pool_alloc_one_group_kernel(int32_t* __restrict__ state, int size, int64_t need, int64_t* __restrict__ out_index,
+                                                                    int64_t* __restrict__ cells) {
+  __shared__ __attribute__((aligned(16))) int sh[2][16];  // (two sets in turn: one barrier per lot)
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  struct Lot {
+    i32x4 s[kScanPieces];
+  };
+  auto pos = [&](int base, int j) { return base + wave * (256 * kScanPieces) + j * 256 + lane * 4; };
+  auto load = [&](int base) {  // (slots past the end read as in use)
+    Lot l;
+#pragma unroll
+    for (int j = 0; j < kScanPieces; j++) {
+      const int p = pos(base, j);
+      if (p + 3 < size) {
+        l.s[j] = *(const i32x4*)(state + p);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++) l.s[j][e] = p + e < size ? state[p + e] : 1;
+      }
+    }
+    return l;
+  };
+  const int wanted = need < size ? (int)need : size;
+  int taken = 0;  // free slots in front of the lot: the rank of its first one
+  int set = 0;
+  // takes what is free of the lot at `base`; true if the walk goes on
+  auto take = [&](const Lot& cur, int base) __attribute__((always_inline)) {
+    set ^= 1;
+    int mine = 0;  // of this wave
+#pragma unroll
+    for (int j = 0; j < kScanPieces; j++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) mine += __builtin_popcountll(__builtin_amdgcn_ballot_w64(cur.s[j][e] == 0));
+    if (lane == 0) sh[set][wave] = mine;
+    __syncthreads();
+    int before = 0, all = 0;  // of the waves in front, of all
+#pragma unroll
+    for (int w = 0; w < 16; w += 4) {
+      const i32x4 n = *(const i32x4*)&sh[set][w];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        before += w + e < wave ? n[e] : 0;
+        all += n[e];
+      }
+    }
+    int first = taken + __builtin_amdgcn_readfirstlane(before);  // the rank of the wave's first free slot
+    taken += __builtin_amdgcn_readfirstlane(all);
+    if (mine > 0 && first < wanted) {  // (wave-uniform)
+#pragma unroll
+      for (int j = 0; j < kScanPieces; j++) {
+        int below = 0, piece = 0;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const uint64_t lanes = __builtin_amdgcn_ballot_w64(cur.s[j][e] == 0);
+          below += __builtin_amdgcn_mbcnt_hi((uint32_t)(lanes >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)lanes, 0u));
+          piece += __builtin_popcountll(lanes);
+        }
+        int rank = first + below;
+        first += piece;
+        if (piece == 0) continue;
+        i32x4 ns = cur.s[j];
+        bool any = false;
+        const int p = pos(base, j);
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          if (cur.s[j][e] == 0 && rank < wanted) {
+            out_index[rank++] = p + e;
+            ns[e] = 1;
+            any = true;
+          }
+        if (any) {
+          if (p + 3 < size) {
+            *(i32x4*)(state + p) = ns;
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+              if (p + e < size) state[p + e] = ns[e];
+          }
+        }
+      }
+    }
+    return taken < wanted && base + kScanSlots < size;
+  };
+  Lot a = load(0), b = load(kScanSlots), c = load(2 * kScanSlots);
+  for (int base = 0; need > 0; base += 3 * kScanSlots) {
+    if (!take(a, base)) break;
+    a = load(base + 3 * kScanSlots);
+    if (!take(b, base + kScanSlots)) break;
+    b = load(base + 4 * kScanSlots);
+    if (!take(c, base + 2 * kScanSlots)) break;
+    c = load(base + 5 * kScanSlots);
+  }
+  for (int64_t i = (int64_t)taken + threadIdx.x; i < need; i += 1024) out_index[i] = -1;
+  if (threadIdx.x == 0) cells[0] = taken;
+}
+
+// ---------------------------------------------------------------------------------------------------
 // Pass 3 of alloc_contiguous: with u(p) = position of the last slot in use at or before p, a run of free slots
 // reaches length `need` exactly at the one p with p - u(p) == need, and starts at p - need + 1.  The smallest
 // such start over the pool is the reference's can_use_index[...][0] (longserve_mem_manager.py:52-55).  The minimum is
@@ -414,7 +520,7 @@ __global__ __launch_bounds__(256) void pool_refs_apply_kernel(int32_t* __restric
   }
 }
 
-// Workspace layout of the searches: int64 cells[2] (cells[0] = free slots in the pool at the time of an alloc) | int64 free_before[nb] | int64 last_used_before[nb] |
+// Workspace layout of the searches: int64 cells[2] (cells[0] = free slots an alloc has come across: all of the pool unless the one-workgroup launch had enough before its end) | int64 free_before[nb] | int64 last_used_before[nb] |
 // int64 blk_last_used[nb] | int32 blk_free[nb]
 struct PoolWorkspace {
   int64_t nb;
@@ -470,6 +576,10 @@ extern "C" int lsattn_pool_alloc(int32_t* mem_state, int64_t pool_size, int64_t 
   if (need > 0 && !out_index) return LSATTN_ERR_INVALID_ARG;
   hipStream_t st = (hipStream_t)stream;
   const PoolWorkspace w = pool_carve(workspace, pool_size);
+  if (pool_size <= kPoolOneGroup) {
+    LSATTN_LAUNCH_KERNEL(pool_alloc_one_group_kernel, dim3(1), dim3(1024), 0, st, mem_state, (int)pool_size, need, out_index, w.cells);
+    return check_launch();
+  }
   const bool scan = pool_summarise(w, mem_state, pool_size, nullptr, st);
   LSATTN_LAUNCH_KERNEL(pool_take_kernel, dim3((unsigned)w.nb), dim3(kPoolThreads), 0, st, mem_state, pool_size,
                      scan ? w.free_before : nullptr, w.blk_free, need, out_index, w.cells);

@@ -51,6 +51,21 @@ def test_alloc_takes_the_first_free_slots(lsa, size):
     _same(m, o)
 
 
+@pytest.mark.parametrize("size", [16383, 16384, 16385, 49151, 49152, 49153, 65535, 65536, 65537])
+def test_alloc_walks_the_pool_in_lots(lsa, size):
+    """Around the lots of 16384 slots that one workgroup walks, three of them in registers, and the size from which all CUs read the pool:
+    free slots at the far end, one around every multiple of a wave's 1024, and a dense stretch across two lots."""
+    patterns = [[size - 1], list(range(size - 5, size)), sorted({p for k in range(0, size, 1024) for p in (k - 1, k, k + 1) if 0 <= p < size}),
+                list(range(16000, min(size, 17000)))]
+    for free in patterns:
+        state = np.ones(size, dtype=np.int32)
+        state[free] = 0
+        m, o = _pair(lsa, state)
+        for need in (1, len(free) // 2, len(free) - 1 - len(free) // 2):
+            assert m.alloc(need).cpu().tolist() == o.alloc(need).tolist()
+            _same(m, o)
+
+
 def test_alloc_through_the_c_abi_pads_with_minus_one_when_the_pool_runs_out(lsa):
     from loongserve_amd import _lib
     lib = _lib.load()
