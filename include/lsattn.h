@@ -290,7 +290,9 @@ int lsattn_decode_stage2(const lsattn_decode_stage2_args* a, void* stream);
  * mid_o and mid_o_logexpsum are scratch to this call, as they are to the reference's function (FDPY:12-27 hands neither
  * out): the call may cut the contexts otherwise than seq_block_size says.  Launches of several requests with enough tokens
  * deal the tokens of all requests (in units of 32) in equal shares to the waves, whatever the lengths of the requests are,
- * and leave one partial per share and request; (o, out_logexpsum) are the same softmax merged from other pieces.
+ * and leave one partial per share and request; (o, out_logexpsum) are the same softmax merged from other pieces.  Short contexts are one
+ * launch, which writes the result itself and leaves the scratch as it was.  o and out_logexpsum may lie over q, b_seqlen and b_req_idx (such
+ * a call is two launches, unless o is q row for row); over the pool's rows or the table they may not.
  */
 int lsattn_decode_attention(const lsattn_decode_stage1_args* s1, const lsattn_decode_stage2_args* s2, void* stream);
 

@@ -13,6 +13,7 @@
 //     result is deterministic;
 //   * a workgroup walks several consecutive blocks, so the launch is sized for the chip
 //     and not for block_seq.
+// Short contexts in the fused call are one launch without partials (decode_direct_kernel).
 #include <atomic>
 #include <type_traits>
 
@@ -38,6 +39,8 @@ struct Stage1Params {
   int32_t tasks;          // hkv * (group / GT) wave tasks
   int32_t tasks_on_x;     // grid = (task groups, chunks, batch) instead of (chunks, task groups, batch)
   int32_t max_shares, share_units;  // equal shares: at most so many, of at least so many units each
+  void* o;                          // (DIRECT) the result [batch, hq, 128] and its log-sum-exps
+  float* out_lse;
 };
 
 constexpr int kTok = 8;  // K/V rows in flight per 16-lane group
@@ -493,10 +496,25 @@ __device__ __forceinline__ ShareSegment share_segment(const Stage1Params& p, con
   return s;
 }
 
-template <typename T, bool WS, bool LISTED, bool RANGE = false>
+template <typename OT> __device__ __forceinline__ void store4(void* base, int64_t elem, const f32x4& v);
+template <> __device__ __forceinline__ void store4<float>(void* base, int64_t elem, const f32x4& v) {
+  *(f32x4*)((float*)base + elem) = v;
+}
+template <> __device__ __forceinline__ void store4<F16>(void* base, int64_t elem, const f32x4& v) {
+  *(u32x2*)((uint16_t*)base + elem) = u32x2{pack2<F16>(v[0], v[1]), pack2<F16>(v[2], v[3])};
+}
+template <> __device__ __forceinline__ void store4<BF16>(void* base, int64_t elem, const f32x4& v) {
+  *(u32x2*)((uint16_t*)base + elem) = u32x2{pack2<BF16>(v[0], v[1]), pack2<BF16>(v[2], v[3])};
+}
+
+// OT (WS): the workgroup takes all tokens of its request and writes the result, in this type; void: partials.
+template <typename T, bool WS, bool LISTED, bool RANGE = false, typename OT = void>
 __device__ __forceinline__ void stage1_mfma_unit(const Stage1Params& p, char* lds, const int lane, const int wave, const int64_t b,
                                                  const unsigned bid_t, const unsigned bid_c, const unsigned n_cgroups,
                                                  const ShareWalk& walk = ShareWalk{}) {
+  constexpr bool DIRECT = !std::is_same<OT, void>::value;
+  static_assert(!DIRECT || WS, "the waves of a workgroup share the request");
+  constexpr float kUp = DIRECT && std::is_same<T, F16>::value ? 16384.f : 1.f;  // the weights in O are so many times those in l
   const int n = lane & 15, g = lane >> 4;  // query head (column) or 16-byte chunk of a row / token group or row of four
   // The waves of a workgroup: tw of them on neighbouring tasks (KV heads: their rows of a token lie side by side in memory
   // and are then fetched at about the same time), the rest on consecutive chunks of tokens.
@@ -523,7 +541,7 @@ __device__ __forceinline__ void stage1_mfma_unit(const Stage1Params& p, char* ld
     n_batches = (int)(walk.end - walk.x);
     table = p.req_to_tokens + (int64_t)co_seg.req * p.max_seq_len;
   } else {
-    const int len = p.b_seqlen[b];
+    const int len = p.b_seqlen[b], req = p.b_req_idx[b];  // (both before anything is stored: scalar loads)
     int64_t nblk = len <= 0 ? 0 : ((int64_t)len + p.block_seq - 1) / p.block_seq;
     if (nblk > p.grid_blocks) nblk = p.grid_blocks;
     if (nblk > (p.num_blocks + p.row_mul - 1) / p.row_mul) nblk = (p.num_blocks + p.row_mul - 1) / p.row_mul;
@@ -532,14 +550,21 @@ __device__ __forceinline__ void stage1_mfma_unit(const Stage1Params& p, char* ld
     const unsigned n_chunks = n_cgroups * cw;
     const unsigned wave_chunk = bid_c * cw + (WS ? 0 : wave >> (tw == 4 ? 2 : tw == 2 ? 1 : 0));
     const unsigned chunk = LISTED ? wave_chunk : (wave_chunk + (unsigned)b) % n_chunks;  // (rotated by the request, as above)
-    blk_begin = (int64_t)chunk * p.blocks_per_wg;  // (WS: one block per workgroup)
+    blk_begin = DIRECT ? 0 : (int64_t)chunk * p.blocks_per_wg;  // (WS: one block per workgroup)
     int64_t blk_end = blk_begin + p.blocks_per_wg;
-    if (blk_end > nblk) blk_end = nblk;
-    if (blk_begin >= blk_end) return;  // (WS: the same for the four waves, which meet at a barrier below)
+    if (DIRECT || blk_end > nblk) blk_end = nblk;
+    if constexpr (DIRECT) {
+      if (nblk <= 0) {  // a request without tokens (the same for all waves)
+        for (int i = wave * 64 + lane; i < nh * 32; i += kMfmaWaves * 64) store4<OT>(p.o, (b * p.hq + qh0) * 128 + i * 4, f32x4{0.f, 0.f, 0.f, 0.f});
+        if (wave == 0 && lane < nh) p.out_lse[b * p.hq + qh0 + lane] = -INFINITY;
+        return;
+      }
+    }
+    if (blk_begin >= blk_end) return;  // (WS: the same for the waves, which meet at a barrier below)
     t_begin = (int)(blk_begin * bs) + (WS ? wave * kMfmaBatch : 0);
     t_end = blk_end * bs > len ? len : (int)(blk_end * bs);
     n_batches = t_begin < t_end ? (t_end - t_begin + kStep - 1) / kStep : 0;
-    table = p.req_to_tokens + (int64_t)p.b_req_idx[b] * p.max_seq_len;
+    table = p.req_to_tokens + (int64_t)req * p.max_seq_len;
   }
   int t_last = t_end - 1;
 
@@ -675,21 +700,52 @@ __device__ __forceinline__ void stage1_mfma_unit(const Stage1Params& p, char* ld
       l *= alpha;
     }
     m = m_new;
+    const float m_ref = DIRECT && m_new == -INFINITY ? 0.f : m_new;  // (scores of -inf weigh nothing, as in the lane kernel)
     float pv[8];
     float ps = 0.f;
 #pragma unroll
     for (int h = 0; h < 2; h++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        pv[4 * h + r] = __builtin_amdgcn_exp2f(s[h][r] - m_new);
+        pv[4 * h + r] = __builtin_amdgcn_exp2f(s[h][r] - m_ref);
         ps += pv[4 * h + r];
       }
     l += ps;
     // P^T as B operand: the lane's eight tokens are the contraction slots 8 g .. 8 g + 7, the order the V^T operand uses
-    u32x4 phi, plo;
-    if (std::is_same<T, F16>::value) {
+    u32x4 phi, plo, prest;
+    if (DIRECT && std::is_same<T, F16>::value) {
+      // P in two parts of eleven bits, 2^14 times as large (which the result is divided by), so that a small weight keeps its bits too.
+      // The parts are cut off and so none is below zero; nor is one zero (2^-38 of the largest weight), or an infinite V would turn into
+      // a NaN at it.
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const float x0 = pv[2 * e] * kUp, x1 = pv[2 * e + 1] * kUp;
+        phi[e] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x0, x1));
+        float h0, h1;
+        unpack2<F16>(phi[e], h0, h1);
+        plo[e] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(fmaxf(x0 - h0, 0x1p-24f), fmaxf(x1 - h1, 0x1p-24f)));
+      }
+    } else if (std::is_same<T, F16>::value) {
 #pragma unroll
       for (int e = 0; e < 4; e++) phi[e] = pack2<F16>(pv[2 * e], pv[2 * e + 1]);
+    } else if (DIRECT) {
+      // P in full, as the lane kernel has it for the launches that were its own: three parts of eight bits, cut off likewise
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        uint32_t hi[2], lo[2];
+        float rest[2];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+          const float x = pv[2 * e + i];
+          hi[i] = __builtin_bit_cast(uint32_t, x) & 0xffff0000u;
+          const float x1 = fmaxf(x - __builtin_bit_cast(float, hi[i]), 0x1p-126f);
+          lo[i] = __builtin_bit_cast(uint32_t, x1) & 0xffff0000u;
+          rest[i] = fmaxf(x1 - __builtin_bit_cast(float, lo[i]), 0x1p-126f);
+        }
+        phi[e] = (hi[0] >> 16) | hi[1];
+        plo[e] = (lo[0] >> 16) | lo[1];
+        prest[e] = pack2<BF16>(rest[0], rest[1]);
+      }
     } else {
 #pragma unroll
       for (int e = 0; e < 4; e++) {
@@ -706,7 +762,8 @@ __device__ __forceinline__ void stage1_mfma_unit(const Stage1Params& p, char* ld
       const u32x2 wa = __builtin_bit_cast(u32x2, xa), wb = __builtin_bit_cast(u32x2, xb);
       const u32x4 va = u32x4{wa[0], wa[1], wb[0], wb[1]};
       oacc[db] = Mfma16<T>::run(va, phi, oacc[db]);
-      if (!std::is_same<T, F16>::value) oacc[db] = Mfma16<T>::run(va, plo, oacc[db]);
+      if (DIRECT || !std::is_same<T, F16>::value) oacc[db] = Mfma16<T>::run(va, plo, oacc[db]);
+      if (DIRECT && !std::is_same<T, F16>::value) oacc[db] = Mfma16<T>::run(va, prest, oacc[db]);
     }
   };
   auto finish_batch = [&](int t0) __attribute__((always_inline)) {
@@ -807,21 +864,23 @@ __device__ __forceinline__ void stage1_mfma_unit(const Stage1Params& p, char* ld
       L += li[w] * mi[w];
     }
     if (n < nh) {
-      const float inv = 1.f / L;  // a block holds at least one token
-      const int64_t row = blk_begin * p.row_mul * p.blk_rows + b * p.req_rows + qh0 + n;
-      float* dst = p.mid_o + row * 128 + 4 * g;
+      const float inv = DIRECT && L == 0.f ? 0.f : 1.f / L * (1.f / kUp);  // a block holds at least one token (whose score may be -inf)
+      const int64_t row = DIRECT ? b * p.hq + qh0 + n : blk_begin * p.row_mul * p.blk_rows + b * p.req_rows + qh0 + n;
 #pragma unroll
       for (int d = 0; d < 2; d++) {
         const int db = 2 * wave + d;
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int w = 0; w < kMfmaWaves; w++) acc += ((const f32x4*)(lds + w * kMfmaStage))[db * 64 + lane] * mi[w];
-        *(f32x4*)(dst + 16 * db) = acc * inv;
+        if constexpr (DIRECT) store4<OT>(p.o, row * 128 + 16 * db + 4 * g, acc * inv);
+        else *(f32x4*)(p.mid_o + row * 128 + 16 * db + 4 * g) = acc * inv;
       }
       if (wave == 0) {
-        if (g == 0) p.mid_lse[row] = (M + __builtin_amdgcn_logf(L)) * kLn2;
-        for (int r = 1 + g; r < p.row_mul; r += 4)
-          if (blk_begin * p.row_mul + r < fine_nblk) p.mid_lse[(blk_begin * p.row_mul + r) * p.blk_rows + b * p.req_rows + qh0 + n] = -INFINITY;
+        float* lse = DIRECT ? p.out_lse : p.mid_lse;
+        if (g == 0) lse[row] = (M + __builtin_amdgcn_logf(L)) * kLn2;
+        if (!DIRECT)
+          for (int r = 1 + g; r < p.row_mul; r += 4)
+            if (blk_begin * p.row_mul + r < fine_nblk) p.mid_lse[(blk_begin * p.row_mul + r) * p.blk_rows + b * p.req_rows + qh0 + n] = -INFINITY;
       }
     }
   }
@@ -835,6 +894,19 @@ __global__ __launch_bounds__(kMfmaWaves * 64, 2) void decode_stage1_mfma_kernel(
   const bool tasks_first = !WS && (p.tasks_on_x & 8) != 0;  // grid = (task groups, chunk groups, batch): a chunk's task groups are dispatched together
   stage1_mfma_unit<T, WS, false>(p, lds, lane, wave, blockIdx.z, tasks_first ? blockIdx.x : blockIdx.y, tasks_first ? blockIdx.y : blockIdx.x,
                                  tasks_first ? gridDim.y : gridDim.x);
+}
+
+// Short contexts in one launch: a workgroup takes all tokens of a (request, task), as the shape whose waves split a block does with a
+// block's, and writes the result itself; no partials, no merge behind.  Bound by latency: request, slot numbers, rows, the four waves' parts,
+// each behind the other; 128 tokens take 5.9 us, where two launches take 8.8 (4.4 each, whatever they do; replayed from a graph).
+// The weights go to the matrix pipe in two (f16) or three (bf16) parts, as good as fp32: the error against 64 bits of the fp32 result
+// is 1e-7 to 5e-7, where one f16 part leaves 2e-4, and two bf16 parts 5e-6.  The parts cost no time that shows: loads are waited for.
+template <typename T, typename OT>
+__global__ __launch_bounds__(kMfmaWaves * 64, 2) void decode_direct_kernel(Stage1Params p) {
+  __shared__ __attribute__((aligned(1024))) char lds[kMfmaWaves * kMfmaStage];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  stage1_mfma_unit<T, true, false, false, OT>(p, lds, lane, wave, blockIdx.y, blockIdx.x, 0, 1);
 }
 
 // The plain shape over a list of the units that exist.  The grid above has a workgroup for every (chunk group, task group)
@@ -1033,17 +1105,6 @@ struct Stage2Params {
   int64_t grid_blocks;         // (SHARES) stage 1's bound on a request's units, from the longest request
   int64_t max_shares, share_units;  // (SHARES) as in Stage1Params
 };
-
-template <typename OT> __device__ __forceinline__ void store4(void* base, int64_t elem, const f32x4& v);
-template <> __device__ __forceinline__ void store4<float>(void* base, int64_t elem, const f32x4& v) {
-  *(f32x4*)((float*)base + elem) = v;
-}
-template <> __device__ __forceinline__ void store4<F16>(void* base, int64_t elem, const f32x4& v) {
-  *(u32x2*)((uint16_t*)base + elem) = u32x2{pack2<F16>(v[0], v[1]), pack2<F16>(v[2], v[3])};
-}
-template <> __device__ __forceinline__ void store4<BF16>(void* base, int64_t elem, const f32x4& v) {
-  *(u32x2*)((uint16_t*)base + elem) = u32x2{pack2<BF16>(v[0], v[1]), pack2<BF16>(v[2], v[3])};
-}
 
 template <typename OT, int D, int NT>
 __global__ __launch_bounds__(NT) void decode_stage2_kernel(Stage2Params p) {
@@ -1408,6 +1469,69 @@ template <typename T> static int launch_stage1_mfma(const lsattn_decode_stage1_a
   return check_launch();
 }
 
+// Which launches of the fused call are one (decode_direct_kernel).  A workgroup walks its request in turns of 128 tokens, some 0.8 us each;
+// two launches take some 4 us more than one for their starts and ends, and the longer the request the more workgroups share it.  Measured over
+// 660 launches (32 to 1400 tokens, 1 to 256 requests, ten head counts, f16 and bf16; two launches | one, us, replayed from a graph):
+//   1 x 128 32/8 8.8 | 5.9    1 x 256 32/8 9.5 | 6.6    1 x 512 32/8 9.8 | 8.9    1 x 1024 32/8 9.9 | 13.0    64 x 64..500 32/8 23.2 | 18.3
+//   32 x 300 32/8 15.8 | 11.6    256 x 64..200 32/8 40.7 | 36.0    32 x 1000 32/8 28.1 | 25.5    16 x 100..1000 32/8 13.9 | 16.9
+//   64 x 256 8/1 9.8 | 6.8    8 x 200..300 32/32 12.5 | 9.5    1 x 377 32/32 8.9 | 9.0    36 x 816 24/8 27.4 | 28.0
+// So up to 512 tokens, and up to 1024 where one round of one to two workgroups per CU is full either way (0.75 to 1.00 of two launches);
+// with two or three query heads per KV head (most of an MFMA's columns idle) below four workgroups per CU, 0.99 at worst (past that 1.09);
+// with one, where the lane kernel stands against it, up to 320 tokens and below two per CU.  The launches that it takes: 0.68 in the mean.
+static bool decode_is_direct(const lsattn_decode_stage1_args* a, const lsattn_decode_stage2_args* s2) {
+  const Tuning tn = tuning();
+  if (tn.decode_stage1 != 0 || tn.decode_listed != 0) return false;  // (choices among the shapes of two launches)
+  if (a->merge_blocks > 1 || a->batch > 65535 || a->k_stride_0 >= (1 << 30) || a->v_stride_0 >= (1 << 30)) return false;
+  const int64_t group = a->num_q_heads / a->num_kv_heads, wgs = a->batch * a->num_kv_heads * ((group + 15) / 16), longest = a->max_len_in_batch;
+  if (group == 1 ? longest > 320 || wgs >= 2 * kCUs
+      : group < 4 ? longest > 512 || wgs >= 4 * kCUs
+                  : longest > 1024 || (longest > 512 && (wgs < kCUs || wgs > 2 * kCUs)))
+    return false;
+  // The result is written while other workgroups still read the queries: not where it lies over them, unless row by row (each
+  // workgroup reads its own first), or over the lengths and rows of the requests.
+  const int64_t pairs = a->batch * a->num_q_heads;
+  auto apart = [](const void* x, int64_t nx, const void* y, int64_t ny) { return (const char*)x + nx <= (const char*)y || (const char*)y + ny <= (const char*)x; };
+  const int64_t o_bytes = pairs * 128 * (s2->o_dtype == LSATTN_F32 ? 4 : 2), q_bytes = pairs * 256;
+  const bool rows_match = s2->o == a->q && o_bytes == q_bytes;
+  return (rows_match || apart(s2->o, o_bytes, a->q, q_bytes)) && apart(s2->out_logexpsum, pairs * 4, a->q, q_bytes) &&
+         apart(s2->o, o_bytes, a->b_seqlen, a->batch * 4) && apart(s2->o, o_bytes, a->b_req_idx, a->batch * 4) &&
+         apart(s2->out_logexpsum, pairs * 4, a->b_seqlen, a->batch * 4) && apart(s2->out_logexpsum, pairs * 4, a->b_req_idx, a->batch * 4);
+}
+template <typename T> static int launch_direct(const lsattn_decode_stage1_args* a, const lsattn_decode_stage2_args* s2, hipStream_t st) {
+  Stage1Params p = {};
+  p.q = a->q;
+  p.k = a->k;
+  p.v = a->v;
+  p.k_s0 = a->k_stride_0;
+  p.k_s1 = a->k_stride_1;
+  p.v_s0 = a->v_stride_0;
+  p.v_s1 = a->v_stride_1;
+  p.scale_log2 = a->sm_scale * kLog2e;
+  p.req_to_tokens = a->req_to_tokens;
+  p.b_req_idx = a->b_req_idx;
+  p.b_seqlen = a->b_seqlen;
+  p.batch = a->batch;
+  p.hq = a->num_q_heads;
+  p.hkv = a->num_kv_heads;
+  p.num_blocks = a->num_blocks;  // (the tokens attended to are those that blocks and rows of partials would have covered)
+  p.max_seq_len = a->max_seq_len;
+  p.row_mul = 1;
+  p.fine_block_seq = p.block_seq = a->seq_block_size;
+  p.grid_blocks = (a->max_len_in_batch + p.block_seq - 1) / p.block_seq;
+  p.tasks = (int)(a->num_kv_heads * ((a->num_q_heads / a->num_kv_heads + 15) / 16));
+  p.tasks_on_x = 1;
+  p.o = s2->o;
+  p.out_lse = s2->out_logexpsum;
+  const dim3 grid((unsigned)p.tasks, (unsigned)a->batch), block(kMfmaWaves * 64);
+  switch (s2->o_dtype) {
+    case LSATTN_F32: LSATTN_LAUNCH_KERNEL((decode_direct_kernel<T, float>), grid, block, 0, st, p); break;
+    case LSATTN_F16: LSATTN_LAUNCH_KERNEL((decode_direct_kernel<T, F16>), grid, block, 0, st, p); break;
+    case LSATTN_BF16: LSATTN_LAUNCH_KERNEL((decode_direct_kernel<T, BF16>), grid, block, 0, st, p); break;
+    default: return LSATTN_ERR_UNSUPPORTED;
+  }
+  return check_launch();
+}
+
 template <typename T> static int dispatch_stage1(const lsattn_decode_stage1_args* a, hipStream_t st, SharesPlan* shares = nullptr) {
   const int group = (int)(a->num_q_heads / a->num_kv_heads);
   if (shares) {  // (in equal shares or not at all: shares->max_shares stays 0 then)
@@ -1432,8 +1556,7 @@ template <typename T> static int dispatch_stage1(const lsattn_decode_stage1_args
 
 using namespace lsattn;
 
-// `shares` (the fused call): launch stage 1 in equal shares if the launch is one for them (max_shares > 0 then) or nothing.
-static int decode_stage1(const lsattn_decode_stage1_args* a, void* stream, SharesPlan* shares) {
+static int validate_stage1(const lsattn_decode_stage1_args* a) {
   if (!a || !a->mid_o || !a->mid_o_logexpsum || !a->q || !a->k || !a->v || !a->req_to_tokens || !a->b_req_idx ||
       !a->b_seqlen)
     return LSATTN_ERR_INVALID_ARG;
@@ -1447,6 +1570,13 @@ static int decode_stage1(const lsattn_decode_stage1_args* a, void* stream, Share
   if (a->k_stride_0 % 8 || a->k_stride_1 % 8 || a->v_stride_0 % 8 || a->v_stride_1 % 8) return LSATTN_ERR_INVALID_ARG;
   if (((uintptr_t)a->k | (uintptr_t)a->v | (uintptr_t)a->q | (uintptr_t)a->mid_o) & 15) return LSATTN_ERR_INVALID_ARG;
   if (a->head_dim != 128) return LSATTN_ERR_UNSUPPORTED;  // as flash_decoding_stage1.cu:210
+  return LSATTN_OK;
+}
+
+// `shares` (the fused call): launch stage 1 in equal shares if the launch is one for them (max_shares > 0 then) or nothing.
+static int decode_stage1(const lsattn_decode_stage1_args* a, void* stream, SharesPlan* shares) {
+  const int rc = validate_stage1(a);
+  if (rc != LSATTN_OK) return rc;
   if (a->batch == 0 || a->num_blocks == 0 || a->max_len_in_batch == 0) return LSATTN_OK;
   hipStream_t st = (hipStream_t)stream;
   if (a->dtype == LSATTN_F16) return dispatch_stage1<F16>(a, st, shares);
@@ -1481,13 +1611,18 @@ template <typename OT> static int dispatch_stage2(const Stage2Params& p, int64_t
   return check_launch();
 }
 
-static int decode_stage2(const lsattn_decode_stage2_args* a, int64_t live_blocks, void* stream, const SharesPlan* shares = nullptr) {
+static int validate_stage2(const lsattn_decode_stage2_args* a) {
   if (!a || !a->o || !a->out_logexpsum || !a->b_seqlen || !a->mid_o || !a->mid_o_logexpsum) return LSATTN_ERR_INVALID_ARG;
   if (a->batch < 0 || a->num_heads <= 0 || a->num_seq_blocks < 0 || a->block_seq < 1) return LSATTN_ERR_INVALID_ARG;
   if (((uintptr_t)a->o | (uintptr_t)a->mid_o) & 15) return LSATTN_ERR_INVALID_ARG;
   if (a->head_dim != 32 && a->head_dim != 64 && a->head_dim != 128) return LSATTN_ERR_UNSUPPORTED;
+  return a->batch * a->num_heads > 0x7fffffff ? LSATTN_ERR_INVALID_ARG : LSATTN_OK;
+}
+
+static int decode_stage2(const lsattn_decode_stage2_args* a, int64_t live_blocks, void* stream, const SharesPlan* shares = nullptr) {
+  const int rc = validate_stage2(a);
+  if (rc != LSATTN_OK) return rc;
   if (a->batch == 0) return LSATTN_OK;
-  if (a->batch * a->num_heads > 0x7fffffff) return LSATTN_ERR_INVALID_ARG;
   Stage2Params p{a->o, a->out_logexpsum, a->b_seqlen, a->mid_o, a->mid_o_logexpsum,
                  a->batch, a->num_heads, a->num_seq_blocks, a->block_seq,
                  a->partials_by_request ? a->num_heads : a->batch * a->num_heads,
@@ -1514,6 +1649,11 @@ extern "C" int lsattn_decode_attention(const lsattn_decode_stage1_args* s1, cons
       s1->batch != s2->batch || s1->num_q_heads != s2->num_heads || s1->num_blocks != s2->num_seq_blocks ||
       s1->head_dim != s2->head_dim || s1->seq_block_size != s2->block_seq || !s1->partials_by_request != !s2->partials_by_request)
     return LSATTN_ERR_INVALID_ARG;
+  // (anything that either stage would refuse goes the way of two launches, which refuses it)
+  if (validate_stage1(s1) == LSATTN_OK && validate_stage2(s2) == LSATTN_OK && s1->batch > 0 && s1->num_blocks > 0 && s1->max_len_in_batch > 0 &&
+      (s1->dtype == LSATTN_F16 || s1->dtype == LSATTN_BF16) && (s2->o_dtype == LSATTN_F32 || s2->o_dtype == LSATTN_F16 || s2->o_dtype == LSATTN_BF16) &&
+      decode_is_direct(s1, s2))
+    return s1->dtype == LSATTN_F16 ? launch_direct<F16>(s1, s2, (hipStream_t)stream) : launch_direct<BF16>(s1, s2, (hipStream_t)stream);
   // Most launches deal the tokens in equal shares (decode_stage1_mfma_range_kernel), however coarse the split asked for: the
   // partials are scratch here.  The rows the shares may fill are counted from the longest request, at most one per 256
   // of its tokens, so that the result does not depend on the height of the buffers where they are tall enough for that.

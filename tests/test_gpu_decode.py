@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from oracle import attn_oracle as orc
-from tests.helpers import assert_lse_close, assert_o_close, decode_case
+from tests.helpers import O_MAX_ABS, O_REL, assert_lse_close, assert_o_close, decode_case
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -727,3 +727,93 @@ def test_fused_call_counts_the_bound_on_lengths_in_whole_blocks(lsa, tuning, sha
                                                                kvd[:, :Hkv], kvd[:, Hkv:], 256)
     assert_o_close(o, o_ref, "o")
     assert_lse_close(l, l_ref, "lse")
+
+
+def _direct_case(lsa, seed, B, Hq, Hkv, lens, dtype, o_dtype=torch.float32, in_place=False):
+    """The fused call and whether it left its partials alone, as the launch does that writes the result itself."""
+    D = 128
+    q, kv, table, b_req, b_len = decode_case(seed, B, Hq, Hkv, D, lens, sum(lens) + 100, dtype)
+    o_ref, l_ref = orc.decode_full(q, kv[:, :Hkv], kv[:, Hkv:], table, b_req, b_len)
+    qd, kvd, rows = q.to(DEV), kv.to(DEV), (max(lens) + 255) // 256
+    mo, ml = torch.full((rows, B, Hq, D), float("nan"), device=DEV), torch.full((rows, B, Hq), float("nan"), device=DEV)
+    o = qd if in_place else torch.full((B, Hq, D), float("nan"), dtype=o_dtype, device=DEV)
+    l = torch.full((B, Hq), float("nan"), device=DEV)
+    lsa.longserve_token_decode_attention_flash_decoding(qd, table.to(DEV), b_req.to(DEV), b_len.to(DEV), mo, ml, B, max(lens), Hq, D,
+                                                        kvd[:, :Hkv], kvd[:, Hkv:], 256, o, l)
+    torch.cuda.synchronize()
+    # (a result in 16 bits: half a last place of values below 4 on top)
+    eps = {torch.float32: 0.0, torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}[o.dtype]
+    assert_o_close(o, o_ref, "o", max_abs=O_MAX_ABS + eps, rel=O_REL + eps / 2)
+    assert_lse_close(l, l_ref, "lse")
+    return bool(torch.isnan(mo).all() and torch.isnan(ml).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("out", ["float32", "same", "other", "in place"])
+@pytest.mark.parametrize("Hq,Hkv", [(4, 4), (8, 4), (9, 3), (32, 8), (17, 1), (5, 1)])
+def test_short_contexts_in_one_launch(lsa, dtype, out, Hq, Hkv):
+    """Lengths around a batch (32), a turn of the four waves (128) and the ends of the range, none among them."""
+    print("case", dtype, out, Hq, Hkv, flush=True)
+    lens = [0, 1, 31, 32, 33, 0, 127, 128, 129, 160, 161, 255, 256, 257, 319, 320] + ([383, 384, 511, 512] if Hq > Hkv else [])
+    other = torch.bfloat16 if dtype == torch.float16 else torch.float16
+    assert _direct_case(lsa, 61, len(lens), Hq, Hkv, lens, dtype, {"float32": torch.float32, "other": other}.get(out, dtype), out == "in place")
+
+
+@pytest.mark.parametrize("Hq,Hkv,B,longest,direct", [
+    (4, 4, 1, 320, True), (4, 4, 1, 321, False), (4, 4, 127, 20, True), (4, 4, 128, 20, False), (8, 4, 255, 30, True), (8, 4, 256, 30, False),
+    (8, 4, 1, 512, True), (8, 4, 1, 513, False), (8, 4, 64, 600, False), (32, 8, 300, 40, True), (32, 8, 31, 513, False), (32, 8, 32, 513, True), (8, 1, 256, 1024, True),
+    (8, 1, 257, 1025, False), (32, 8, 64, 600, True), (32, 8, 65, 600, False)])
+def test_which_short_contexts_take_one_launch(lsa, Hq, Hkv, B, longest, direct):
+    print("case", Hq, Hkv, B, longest, flush=True)
+    assert _direct_case(lsa, 67, B, Hq, Hkv, [longest] + [1 + (7 * i) % min(longest, 60) for i in range(B - 1)], torch.bfloat16) == direct
+
+
+def test_result_over_the_queries_takes_two_launches(lsa):
+    """A result that lies over the queries row for row is written in one launch; shifted against them it waits for the last read."""
+    B, Hq, Hkv, D = 6, 8, 2, 128
+    lens = [100, 1, 300, 64, 256, 31]
+    q, kv, table, b_req, b_len = decode_case(71, B, Hq, Hkv, D, lens, 1000, torch.float16)
+    o_ref, l_ref = orc.decode_full(q, kv[:, :Hkv], kv[:, Hkv:], table, b_req, b_len)
+    kvd = kv.to(DEV)
+    for shift, direct in ((0, True), (D, False), (B * Hq * D, True)):
+        room = torch.zeros(2 * B * Hq * D, dtype=torch.float16, device=DEV)
+        qd, o = room[shift:shift + B * Hq * D].view(B, Hq, D), room[:B * Hq * D].view(B, Hq, D)
+        qd.copy_(q)
+        mo, ml = torch.full((2, B, Hq, D), float("nan"), device=DEV), torch.empty((2, B, Hq), device=DEV)
+        l = torch.empty((B, Hq), device=DEV)
+        lsa.longserve_token_decode_attention_flash_decoding(qd, table.to(DEV), b_req.to(DEV), b_len.to(DEV), mo, ml, B, 300, Hq, D,
+                                                            kvd[:, :Hkv], kvd[:, Hkv:], 256, o, l)
+        assert bool(torch.isnan(mo).all()) == direct
+        assert_o_close(o, o_ref, "o", max_abs=O_MAX_ABS + 2.0 ** -10, rel=O_REL + 2.0 ** -11)
+        assert_lse_close(l, l_ref, "lse")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_one_launch_and_infinite_keys_and_values(lsa, tuning, dtype):
+    """Scores of minus infinity weigh nothing (a request of nothing else has the result of an empty one) and infinite values stay
+    infinite, as in the lane kernel's two launches."""
+    B, H, D = 5, 4, 128
+    lens = [32, 40, 200, 129, 64]
+    q, kv, table, b_req, b_len = decode_case(73, B, H, H, D, lens, 600, dtype)
+    q = q.abs() + 0.125
+    slot = [table[int(b_req[b])] for b in range(B)]
+    kv[slot[0][:32].long(), :H] = float("-inf")                # nothing but -inf
+    kv[slot[1][:32].long(), :H] = float("-inf")                # the first batch
+    kv[slot[2][130:200].long(), :H] = float("-inf")            # whole waves at the end
+    kv[slot[3][7].long(), H:, 5] = float("inf")
+    kv[slot[3][90].long(), H:, 6] = float("-inf")
+    qd, kvd = q.to(DEV), kv.to(DEV)
+    got = []
+    for kernel in (None, "lane"):
+        tuning(decode_stage1=kernel)
+        mo, ml = torch.full((1, B, H, D), float("nan"), device=DEV), torch.full((1, B, H), float("nan"), device=DEV)
+        o, l = lsa.longserve_token_decode_attention_flash_decoding(qd, table.to(DEV), b_req.to(DEV), b_len.to(DEV), mo, ml, B, 200, H, D,
+                                                                   kvd[:, :H], kvd[:, H:], 256)
+        torch.cuda.synchronize()
+        assert bool(torch.isnan(mo).all()) == (kernel is None)
+        got.append((o.cpu(), l.cpu()))
+    (o, l), (o2, l2) = got
+    assert torch.equal(o.isinf() * o.sign(), o2.isinf() * o2.sign()) and torch.equal(o.isnan(), o2.isnan())
+    fin = o2.isfinite()
+    assert_o_close(o[fin], o2[fin], "o")
+    assert_lse_close(l, l2, "lse")

@@ -400,6 +400,15 @@ def test_decode_matrix_pipe_kernel_touches_no_register_of_a_load_in_flight():
 
 
 @pytest.mark.skipif(shutil.which(HIPCC) is None, reason="hipcc not available")
+def test_decode_kernel_of_one_launch_touches_no_register_of_a_load_in_flight():
+    res = loads_in_flight_violations(_decode_asm(), "decode_direct_")
+    assert len(res) == 6, list(res)                       # fp16 and bf16, each with a result of three types
+    for name, (n, bad) in res.items():
+        assert n >= 3 * 8 + 3 * 16, (name, n)
+        assert not bad, name + "\n" + "\n".join(bad[:20])
+
+
+@pytest.mark.skipif(shutil.which(HIPCC) is None, reason="hipcc not available")
 def test_inline_assembly_stores_of_a_partial_keep_their_data_registers_for_two_cycles():
     """The matrix-pipe decode kernel stores a partial's row from inline assembly (the compiler has no plain store with the
     system-scope bits).  A vector instruction may not overwrite the data registers of a store of more than 64 bits in
