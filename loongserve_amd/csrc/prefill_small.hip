@@ -699,7 +699,14 @@ template <typename T, bool DV> int launch_mode(const SmallParams& p, const lsatt
 //   16 x 1024 32/8 200 | 290 | 191          20 x 200..800 32/8 91 | - | 71                16 x 512 32/32 88 | 127 | 76
 //   3 x 1012 32/8 38.0 | 37.3 | 39.8        2 x 1594 32/8 64.3 | 75.8 | 65.8              19 x 1244 64/8 608 | 847 | 625
 // 16 positions win up to two and a half workgroups per CU (four with one head per workgroup, which leaves each wave fewer rows to mask);
-// 32 from there on, for prompts beyond 768 tokens from three (of its own) per CU.  Equal prompts beyond 1280 tokens in launches of ten and
+// 32 from there on, for prompts beyond 768 tokens from three (of its own) per CU.  Those take 16 positions where the other kernel's workgroups of
+// 128 rows, one to a CU, would fill half the chip, or a second round with a few of them (with 16 positions: up to one workgroup per CU, and
+// the third; there prompts beyond 1024 tokens only into the in-place epilogue, which lasts longer in the other kernel, and in bf16 with
+// one head per workgroup: the others came to between 0.86 and 1.12 of it).  Over 128 such launches, prompts and steps of a ring alike,
+// 15 % below the other kernel, the worst 3 % below it (in place, other kernel | 16 positions):
+//   1 x 925 40/40 38.9 | 28.2    1 x 1125 32/32 32.8 | 28.2    1 x 1093 32/8 bf16 34.6 | 32.9 (not taken)    1 x 1133 32/8 bf16 partial 27.8 | 31.1 (not taken)
+//   four ring steps of 1120 32/32 186 | 167, 32/8 184 | 169, 8/1 105 | 90    three striped of 1500 32/32 125 | 109, 32/8 122 | 110
+// Equal prompts beyond 1280 tokens in launches of ten and
 // more per CU keep the other kernel, whose loop is the faster one.
 // The geometric mean over the launches the rule takes is 32 % below the other kernel; the worst is 6 % above it.
 // The keys: a chunk behind a context waits for its longest request, and a tile of a lone workgroup takes longer here (0.95 us against 0.56 in the
@@ -729,6 +736,13 @@ int prefill_short_blocks(const lsattn_prefill_args* a) {
     if (a->max_q_len <= 768) return one <= 5 * kCUs / 2 || (pack == 0 && a->max_q_len <= 512 && one <= 4 * kCUs) ? 1 : 2;
   } else if (a->max_q_len <= 768) {
     return 0;
+  }
+  const bool f16 = a->dtype == LSATTN_F16;
+  if (one <= kCUs) {
+    if (longest <= (f16 ? 1280 : 1024)) return 1;
+  } else if (one > 2 * kCUs && one <= 3 * kCUs) {
+    // (m: of the three steps only the in-place one has it.  bf16 does not look at it: whether V is to be copied is asked before)
+    if (longest <= 1024 || (f16 ? a->m && longest <= 1536 : pack == 0 && longest <= 1280)) return 1;
   }
   return two >= 3 * kCUs && (a->max_q_len <= 1280 || two <= 10 * kCUs || ragged(a)) ? 2 : 0;
 }

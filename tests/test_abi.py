@@ -383,12 +383,12 @@ def test_cut_count_of_a_step():
                 assert 1 <= count(1, 8, 1, rows, keys, most) <= min(most, keys // 512, 64)
 
 
-def _route(batch, max_q, heads, head_dim=128, total_q=0, total_kv=0, max_kv=0, dtype=0, v_is_f16=0, cuts=0):
+def _route(batch, max_q, heads, head_dim=128, total_q=0, total_kv=0, max_kv=0, dtype=0, v_is_f16=0, cuts=0, m=None):
     from loongserve_amd import _lib
     a = _lib.PrefillArgs()
     a.batch, a.max_q_len, a.head_dim, a.dtype, a.v_is_f16, a.kv_cuts = batch, max_q, head_dim, dtype, v_is_f16, cuts
     a.num_q_heads, a.num_kv_heads = heads
-    a.total_q_rows, a.total_kv_rows, a.max_kv_len = total_q, total_kv, max_kv
+    a.total_q_rows, a.total_kv_rows, a.max_kv_len, a.m = total_q, total_kv, max_kv, m
     return _lib.load().lsattn_prefill_route(C.byref(a))
 
 
@@ -429,6 +429,25 @@ def test_short_prompts_kernel_goes_by_the_workgroups_and_the_longest_prompt():
     assert _route(16, 1000, heads, total_q=16000, total_kv=17100) == HALF  # (one of them behind 1100 more)
     assert _route(16, 1000, heads, total_q=16000) == _route(16, 1000, heads) == HALF  # (nothing known of the keys)
     assert _route(70000, 16, heads, total_q=70000 * 16, total_kv=70000 * 16) not in (SMALL_16, SMALL_32, SMALL_TURNS)  # (past the grid's index)
+
+
+def test_longer_prompts_in_few_workgroups_of_16_positions():
+    """Beyond 768 tokens where 128-row workgroups would fill half the chip, or start a second round of few."""
+    small = (SMALL_16, SMALL_32, SMALL_TURNS)
+    one = lambda n, heads, dtype=0, **kw: _route(1, n, heads, total_q=n, total_kv=kw.pop("total_kv", n), dtype=dtype, **kw)
+    assert one(769, (8, 1)) == one(1280, (8, 1)) == SMALL_16 and one(1281, (8, 1)) not in small          # one workgroup per CU and less
+    assert one(1024, (8, 1), 1) == SMALL_16 and one(1025, (8, 1), 1) not in small
+    assert one(1024, (16, 16)) == SMALL_16 and one(1025, (16, 16)) not in small                          # 256 and 272 workgroups
+    place = dict(m=256)  # (an in-place step has one; no pointer is followed)
+    assert one(1000, (40, 40)) == one(1024, (40, 40), 1) == SMALL_16                                     # 640 workgroups, any epilogue
+    assert one(1024, (32, 32), **place) not in small and one(1025, (32, 32), **place) == SMALL_16        # 512 and 544
+    assert one(1025, (32, 32)) not in small and one(1025, (32, 32), 1) == SMALL_16
+    assert one(1536, (32, 8), **place) == SMALL_16 and one(1537, (32, 8), **place) not in small          # 768 and 776
+    assert one(1280, (32, 32), 1) == SMALL_16 and one(1281, (32, 32), 1, **place) not in small
+    assert one(1040, (32, 8), 1, **place) not in small
+    assert _route(1, 1120, (32, 32), total_q=1120, total_kv=1536, **place) == SMALL_16                   # (keys beyond the rows)
+    assert _route(1, 1120, (32, 32), total_q=1120, total_kv=1537, **place) not in small
+    assert _route(1, 1120, (32, 32), total_q=1120, **place) not in small
 
 
 def test_prefill_route_names_a_kernel_for_every_step_and_none_for_others():

@@ -184,3 +184,11 @@ def test_short_prompts_in_three_stages_and_the_grids_orders(lsa, mode, V, what):
         _every_epilogue_on(SMALL_32, lsa, mode, V, 64, 8, 8, [130] * 72 + [1], [0] * 73)
     else:
         _every_epilogue_on(SMALL_32, lsa, mode, V, 64, 32, 8, [700, 33, 650, 64, 1, 600, 400, 20, 300, 512, 129], [0] * 11, spare=1 << 16)
+
+
+@pytest.mark.parametrize("mode", ["partial", "accumulate", "in_place"])
+@pytest.mark.parametrize("V", ["f16", "bf16", "bf16 copied"])
+@pytest.mark.parametrize("Hq,Hkv,lens", [(20, 20, [1024, 993]), (8, 2, [897, 30, 800])])
+def test_longer_prompts_with_16_positions_per_wave(lsa, mode, V, Hq, Hkv, lens):
+    print("case", mode, V, Hq, Hkv, flush=True)
+    _every_epilogue_on(SMALL_16, lsa, mode, V, 128, Hq, Hkv, lens, [0] * len(lens))
