@@ -698,7 +698,8 @@ template <typename T, bool DV> int launch_mode(const SmallParams& p, const lsatt
 //   16 x 512 32/8 76 | 86 | 65              13 x 1317 at most 32/8 72.4 | 75.1 | 59.6     4 x 1416 32/32 114 | 122 | 100
 //   16 x 1024 32/8 200 | 290 | 191          20 x 200..800 32/8 91 | - | 71                16 x 512 32/32 88 | 127 | 76
 //   3 x 1012 32/8 38.0 | 37.3 | 39.8        2 x 1594 32/8 64.3 | 75.8 | 65.8              19 x 1244 64/8 608 | 847 | 625
-// 16 positions win up to two and a half workgroups per CU (four with one head per workgroup, which leaves each wave fewer rows to mask);
+// 16 positions win up to two and a half workgroups per CU (four with one head per workgroup, which leaves each wave fewer rows to mask; three
+// for equal prompts beyond 640 tokens; with 32 and with 16: 4 x 753 16/16 36.7 | 29.7, 2 x 764 32/4 31.5 | 24.8, 1 x 696 64/8 bf16 34.7 | 28.9);
 // 32 from there on, for prompts beyond 768 tokens from three (of its own) per CU.  Those take 16 positions where the other kernel's workgroups of
 // 128 rows, one to a CU, would fill half the chip, or a second round with a few of them (with 16 positions: up to one workgroup per CU, and
 // the third; there prompts beyond 1024 tokens only into the in-place epilogue, which lasts longer in the other kernel, and in bf16 with
@@ -733,7 +734,7 @@ int prefill_short_blocks(const lsattn_prefill_args* a) {
   const int pack = pack_shift_of(a);
   const int64_t one = workgroups(a, pack, 1), two = workgroups(a, pack, 2);
   if (longest <= 1024) {
-    if (a->max_q_len <= 768) return one <= 5 * kCUs / 2 || (pack == 0 && a->max_q_len <= 512 && one <= 4 * kCUs) ? 1 : 2;
+    if (a->max_q_len <= 768) return one <= (pack == 0 ? 4 * kCUs : a->max_q_len > 640 && !ragged(a) ? 3 * kCUs : 5 * kCUs / 2) ? 1 : 2;
   } else if (a->max_q_len <= 768) {
     return 0;
   }
