@@ -434,6 +434,15 @@ def test_short_prompts_kernel_goes_by_the_workgroups_and_the_longest_prompt():
     assert _route(70000, 16, heads, total_q=70000 * 16, total_kv=70000 * 16) not in (SMALL_16, SMALL_32, SMALL_TURNS)  # (past the grid's index)
 
 
+def test_one_prompt_in_a_few_four_wave_workgroups_more_than_two_per_cu():
+    one = lambda n, heads, **kw: _route(1, n, heads, total_q=n, **{"total_kv": n, **kw})
+    assert [one(n, (32, 32)) for n in (2049, 2816, 2817, 4097)] == [HALF, HALF, ROWS_256, ROWS_256]
+    assert [one(n, (32, 8)) for n in (2049, 2304, 2305, 4097)] == [HALF, HALF, ROWS_256, ROWS_256]
+    assert one(6144, (11, 11)) == HALF and one(6145, (11, 11)) == ROWS_256
+    assert one(2561, (32, 32), total_kv=2562) == one(2561, (32, 32), total_kv=0) == one(2561, (32, 32), cuts=2) == ROWS_256
+    assert _route(2, 1100, (32, 32), total_q=2200, total_kv=2200) != HALF
+
+
 def test_longer_prompts_in_few_workgroups_of_16_positions():
     """Beyond 768 tokens where 128-row workgroups would fill half the chip, or start a second round of few."""
     small = (SMALL_16, SMALL_32, SMALL_TURNS)
