@@ -422,7 +422,7 @@ def test_short_prompts_kernel_goes_by_the_workgroups_and_the_longest_prompt():
     own = lambda batch, n, **kw: _route(batch, n, heads, total_q=batch * n, total_kv=batch * n, **kw)
     assert own(2, 640) == SMALL_16 and own(4, 640) == SMALL_32 and own(4, 768) == SMALL_32
     assert own(2, 704) == SMALL_16 and own(3, 704) == SMALL_32 and own(3, 640) == SMALL_32               # (704, 1056 and 960 workgroups of 16)
-    assert _route(4, 700, heads, total_q=1400, total_kv=1400) == SMALL_32                                 # (736, of which some are short)
+    assert _route(4, 700, heads, total_q=1400, total_kv=1400) == SMALL_TURNS                               # (736, of which some are short)
     assert _route(2, 768, (40, 40), total_q=1536, total_kv=1536) == SMALL_16 and _route(3, 768, (32, 32), total_q=2304, total_kv=2304) == SMALL_32
     assert own(3, 990) not in (SMALL_16, SMALL_32) and own(3, 1000) == SMALL_32
     assert own(3, 1024) == own(3, 1025) == SMALL_32 and own(2, 1500) not in (SMALL_16, SMALL_32, SMALL_TURNS)
