@@ -715,8 +715,8 @@ __device__ __forceinline__ void stage1_mfma_unit(const Stage1Params& p, char* ld
     u32x4 phi, plo, prest;
     if (DIRECT && std::is_same<T, F16>::value) {
       // P in two parts of eleven bits, 2^14 times as large (which the result is divided by), so that a small weight keeps its bits too.
-      // The parts are cut off and so none is below zero; nor is one zero (2^-38 of the largest weight), or an infinite V would turn into
-      // a NaN at it.
+      // The parts are cut off and so none is below zero; nor is the second one zero (2^-38 of the largest weight), or an infinite V would
+      // turn into a NaN at it.  (Weights below 2^-38 have no first part, as those below 2^-25 have none in the kernels of two launches.)
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         const float x0 = pv[2 * e] * kUp, x1 = pv[2 * e + 1] * kUp;
