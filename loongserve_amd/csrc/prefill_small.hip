@@ -103,7 +103,7 @@ constexpr uint32_t kOnes = 0x3C003C00u;  // two ones in fp16
 constexpr int64_t kCUs = 256;
 constexpr int64_t kL2Bytes = 32 << 20;    // of the eight L2s together
 constexpr int64_t kBunchWorkgroups = 512; // workgroups of a bunch of requests of about equal, short lengths
-constexpr int64_t kShortMaxKeys = 2048;   // 128-wide heads: the keys of the longest request up to which this kernel may take a step
+constexpr int64_t kShortMaxKeys = 1280;   // 128-wide heads: the keys of the longest request up to which this kernel may take a step
 constexpr int64_t kMaxIds = 65535;  // of the second or third index of a grid
 
 // s_waitcnt vmcnt(N) (expcnt / lgkmcnt fields left at their maximum)
@@ -690,26 +690,25 @@ template <typename T, bool DV> int launch_mode(const SmallParams& p, const lsatt
 // waves of 256 registers that fill 128 KB of rings and some 40 KB of code before the first product; its four-wave shape 12 us, two workgroups on a
 // CU).  This one has a quarter of the code and, with 32 positions per wave, three workgroups on a CU, of which one starts or ends while the others
 // compute, at the same rate per tile; it converts a bfloat16 V on the way (no launch in front that copies it).  16 positions
-// per wave are for launches that do not fill the chip.  Measured over 700 launches (1 to 40 prompts of 32 to 2048 tokens, equal or
-// log-uniform over a factor of up to 20, a fifth behind contexts; 32/32, 32/8, 64/8 and 8/1 heads; both epilogues; microseconds, the
-// kernel of prefill.hip | 16 positions per wave | 32; bf16 with its copy of V):
-//   1 x 636 32/8 24.2 | 19.9 | 24.4         9 x 222 at most 32/32 32.9 | 18.3 | 20.4      9 x 126 at most 32/32 bf16 24.7 | 9.7 | 13.2
-//   14 x 99 32/8 bf16 23.3 | 19.2 | 16.3    30 x 100 32/8 32.4 | 27.5 | 24.2              12 x 324 at most 32/8 33.0 | 35.1 | 28.8
-//   16 x 512 32/8 76 | 86 | 65              13 x 1317 at most 32/8 72.4 | 75.1 | 59.6     4 x 1416 32/32 114 | 122 | 100
-//   16 x 1024 32/8 200 | 290 | 191          20 x 200..800 32/8 91 | - | 71                16 x 512 32/32 88 | 127 | 76
-//   3 x 1012 32/8 38.0 | 37.3 | 39.8        2 x 1594 32/8 64.3 | 75.8 | 65.8              19 x 1244 64/8 608 | 847 | 625
-// 16 positions win up to two and a half workgroups per CU (four with one head per workgroup, which leaves each wave fewer rows to mask; three
-// for equal prompts beyond 640 tokens; with 32 and with 16: 4 x 753 16/16 36.7 | 29.7, 2 x 764 32/4 31.5 | 24.8, 1 x 696 64/8 bf16 34.7 | 28.9);
-// 32 from there on, for prompts beyond 768 tokens from three (of its own) per CU.  Those take 16 positions where the other kernel's workgroups of
-// 128 rows, one to a CU, would fill half the chip, or a second round with a few of them (with 16 positions: up to one workgroup per CU, and
-// the third; there prompts beyond 1024 tokens only into the in-place epilogue, which lasts longer in the other kernel, and in bf16 with
-// one head per workgroup: the others came to between 0.86 and 1.12 of it).  Over 128 such launches, prompts and steps of a ring alike,
-// 15 % below the other kernel, the worst 3 % below it (in place, other kernel | 16 positions):
-//   1 x 925 40/40 38.9 | 28.2    1 x 1125 32/32 32.8 | 28.2    1 x 1093 32/8 bf16 34.6 | 32.9 (not taken)    1 x 1133 32/8 bf16 partial 27.8 | 31.1 (not taken)
-//   four ring steps of 1120 32/32 186 | 167, 32/8 184 | 169, 8/1 105 | 90    three striped of 1500 32/32 125 | 109, 32/8 122 | 110
-// Equal prompts beyond 1280 tokens in launches of ten and
-// more per CU keep the other kernel, whose loop is the faster one.
-// The geometric mean over the launches the rule takes is 32 % below the other kernel; the worst is 6 % above it.
+// per wave are for launches that do not fill the chip.  Measured over 10600 launches (1 to 40 prompts of 200 to 2048 tokens, equal or log-uniform
+// over a factor of up to 20, some behind contexts; 32/32, 32/8, 64/8, 8/1, 16/16, 40/40, 24/8 and 16/8 heads; the three epilogues; calls with
+// the fills of m and l; microseconds, the kernel of prefill.hip | 16 positions per wave | 32; bf16 with its copy of V):
+//   3 x 560 32/32 bf16 45.6 | 28.1 | 29.0     10 x 306 32/8 35.3 | 32.6 | 26.9       19 x 566 32/8 bf16 104.4 | 118.4 | 83.8   3 x 386 at most 64/8 25.0 | 20.0 | 21.1
+//   2 x 819 32/8 34.0 | 27.4 | 31.6           7 x 821 at most 32/8 bf16 52.6 | 51.4 | 39.9   6 x 999 64/8 141 | 164 | 127            16 x 853 at most 32/8 72.6 | 88.4 | 59.3
+//   1 x 1113 32/8 29.0 | 26.9 | 35.9          6 x 1072 at most 64/8 81.7 | 89.5 | 63.9       3 x 1012 32/8 49.0 | 50.6 | 45.5, partial 41.1 | 44.8 | 41.2
+//   2 x 1594 32/8 partial 49.0 | 62.9 | 59.1 (not taken)     19 x 1244 64/8 partial 594 | 846 | 621 (not taken)    2 x 1793 at most 32/8 partial 47.9 | 74.0 | 62.5 (not taken)
+// A full step of a ring (all keys of the chunk seen by all rows, as in a ring over contiguous shards) gains less: twice the tiles for the same
+// start and end.  The host cannot tell it from a batch of prompts, whose numbers are the same.  The launches taken come, in the geometric mean (95 of
+// 100 stay below the figure in brackets), to so much of the time before this kernel, prompts, then full steps:
+//   up to 768 rows 0.79 (0.97), 0.91 (1.16)     769 to 1024 0.85 (0.99), 1.03 (1.25)     1025 to 1280 0.88 (1.02), 1.01 (1.12)
+// so the rule goes by the prompts up to 1024 rows and from there on takes what a ring's shards bear too; past 1280 that is nothing.
+//   16 positions: up to three workgroups per CU (two and a half of a ragged batch; with one head per workgroup, which leaves each wave fewer
+// rows to mask, four and six), past 768 rows up to one, and the third, where workgroups of 128 rows would run a second round with a few of them (a ragged batch
+// only with one head per workgroup: a lone long request between short ones came to up to 1.6 of the other kernel's time).  Past 1024 rows
+// these only for one prompt, or for equal ones in the in-place epilogue, which lasts longer in the other kernel, and in bf16 with one
+// head per workgroup.  (Four ring steps of 1120 rows 32/32 186 | 167, 32/8 184 | 169, 8/1 105 | 90.)
+//   32 from there on: past 768 rows from three (ragged: three and a half) of its own per CU, past 1024 from four (five), where the other
+// kernel's four-wave shape has more than one round; equal prompts past 1024 rows in more than ten per CU are for that kernel's faster loop.
 // The keys: a chunk behind a context waits for its longest request, and a tile of a lone workgroup takes longer here (0.95 us against 0.56 in the
 // 128-row shape), so the longest request decides (whole call, 32/8 heads, the other kernel | this one with 16 positions, f16, then bf16):
 //   8 x 64 rows behind 600 keys each 20.8 | 15.7, 28.0 | 18.7      4 x 100 behind 1000 each 24.9 | 21.7, 30.5 | 25.9      1 x 200 behind 1024 22.1 | 19.8, 25.2 | 24.0
@@ -733,19 +732,14 @@ int prefill_short_blocks(const lsattn_prefill_args* a) {
   if (tn.prefill_rows || tn.prefill_order || tn.prefill_pack) return 0;  // (choices among the 128-wide kernel's shapes)
   const int pack = pack_shift_of(a);
   const int64_t one = workgroups(a, pack, 1), two = workgroups(a, pack, 2);
-  if (longest <= 1024) {
-    if (a->max_q_len <= 768) return one <= (pack == 0 ? 4 * kCUs : a->max_q_len > 640 && !ragged(a) ? 3 * kCUs : 5 * kCUs / 2) ? 1 : 2;
-  } else if (a->max_q_len <= 768) {
-    return 0;
-  }
-  const bool f16 = a->dtype == LSATTN_F16;
-  if (one <= kCUs) {
-    if (longest <= (f16 ? 1280 : 1024)) return 1;
-  } else if (one > 2 * kCUs && one <= 3 * kCUs) {
-    // (m: of the three steps only the in-place one has it.  bf16 does not look at it: whether V is to be copied is asked before)
-    if (longest <= 1024 || (f16 ? a->m && longest <= 1536 : pack == 0 && longest <= 1280)) return 1;
-  }
-  return two >= 3 * kCUs && (a->max_q_len <= 1280 || two <= 10 * kCUs || ragged(a)) ? 2 : 0;
+  const bool f16 = a->dtype == LSATTN_F16, rag = ragged(a);
+  if (a->max_q_len <= 768) return longest > 1024 ? 0 : 2 * one <= (pack ? rag ? 5 : 6 : rag ? 12 : 8) * kCUs ? 1 : 2;
+  const bool past = longest > 1024;
+  if (one <= kCUs) return !past || (f16 && a->batch == 1) ? 1 : 0;
+  // (m: of the three steps only the in-place one has it.  bf16 does not look at it: whether V is to be copied is asked before)
+  if (one > 2 * kCUs && one <= 3 * kCUs && (past ? !rag && (f16 ? a->m != nullptr : pack == 0) : !rag || pack == 0)) return 1;
+  if (past) return two > (rag ? 5 : 4) * kCUs && (rag || two <= 10 * kCUs) ? 2 : 0;
+  return 2 * two >= (rag ? 7 : 6) * kCUs ? 2 : 0;
 }
 
 int prefill_small_route(const lsattn_prefill_args* a) {

@@ -416,22 +416,38 @@ def test_short_prompts_kernel_goes_by_the_longest_request():
 
 
 def test_short_prompts_kernel_goes_by_the_workgroups_and_the_longest_prompt():
-    """With 32 positions per wave it takes prompts of up to 768 tokens that are too many for 16, longer ones from three workgroups per
-    CU on, and beyond 1280 tokens equal ones only up to ten."""
+    """With 32 positions per wave it takes prompts of up to 768 tokens that are too many for 16, up to 1024 from three workgroups per CU
+    on, up to 1280 from four to ten; ragged batches from a half, then a whole one more."""
+    small = (SMALL_16, SMALL_32, SMALL_TURNS)
     heads = (32, 8)  # (32 positions of four heads: 8 workgroups per 32 tokens)
-    own = lambda batch, n, **kw: _route(batch, n, heads, total_q=batch * n, total_kv=batch * n, **kw)
-    assert own(2, 640) == SMALL_16 and own(4, 640) == SMALL_32 and own(4, 768) == SMALL_32
-    assert own(2, 704) == SMALL_16 and own(3, 704) == SMALL_32 and own(3, 640) == SMALL_32               # (704, 1056 and 960 workgroups of 16)
-    assert _route(4, 700, heads, total_q=1400, total_kv=1400) == SMALL_TURNS                               # (736, of which some are short)
-    assert _route(2, 768, (40, 40), total_q=1536, total_kv=1536) == SMALL_16 and _route(3, 768, (32, 32), total_q=2304, total_kv=2304) == SMALL_32
-    assert own(3, 990) not in (SMALL_16, SMALL_32) and own(3, 1000) == SMALL_32
-    assert own(3, 1024) == own(3, 1025) == SMALL_32 and own(2, 1500) not in (SMALL_16, SMALL_32, SMALL_TURNS)
-    assert own(16, 1280) == SMALL_32 and own(16, 1281) == ROWS_256 and own(5, 1700) == SMALL_32
-    assert _route(16, 2000, heads, total_q=14000, total_kv=14000) == SMALL_TURNS and own(16, 2000) == ROWS_256
+    own = lambda batch, n, heads=heads, **kw: _route(batch, n, heads, total_q=batch * n, total_kv=batch * n, **kw)
+    mixed = lambda batch, n, total, heads=heads: _route(batch, n, heads, total_q=total, total_kv=total)
+    assert own(2, 640) == own(2, 704) == own(2, 768) == SMALL_16 and own(3, 640) == own(3, 704) == own(4, 768) == SMALL_32  # 640, 704, 768 | 960 ..
+    assert mixed(4, 700, 1216) == SMALL_16 and mixed(4, 700, 1217) == SMALL_TURNS                          # 640 and 648, of which some are short
+    assert own(2, 768, (40, 40)) == SMALL_16 and own(3, 768, (32, 32)) == SMALL_32                       # 960 and 1152
+    assert mixed(4, 768, 2000, (32, 32)) == SMALL_16                                                     # 1152
+    assert own(3, 992) not in small and own(3, 1024) == SMALL_32                                         # 744 and 768 of 32
+    assert mixed(8, 1024, 3296) not in small and mixed(8, 1024, 3297) in small                           # 888 and 896
+    assert own(4, 1025) == SMALL_32 and own(3, 1025) not in small                                        # 1056 and 792
+    assert own(8, 1280) == SMALL_32 and own(9, 1280) not in small and own(8, 1281) not in small          # 2560 and 2880
+    assert mixed(12, 1280, 4736) not in small and mixed(12, 1280, 4737) in small and mixed(16, 1280, 16000) in small  # 1280, 1288 and 4128
     assert _route(8, 2049, heads, total_q=5000, total_kv=5000) == ROWS_256
     assert _route(16, 1000, heads, total_q=16000, total_kv=17100) == HALF  # (one of them behind 1100 more)
     assert _route(16, 1000, heads, total_q=16000) == _route(16, 1000, heads) == HALF  # (nothing known of the keys)
-    assert _route(70000, 16, heads, total_q=70000 * 16, total_kv=70000 * 16) not in (SMALL_16, SMALL_32, SMALL_TURNS)  # (past the grid's index)
+    assert _route(70000, 16, heads, total_q=70000 * 16, total_kv=70000 * 16) not in small  # (past the grid's index)
+
+
+def test_prompts_that_lasted_longer_in_the_short_kernel_are_left_to_the_other():
+    """Launches that took 2 to 31 % longer in it than in the 128-wide kernel (microseconds, that kernel | this one): 2 x 1594 32/8 partial 49.0 | 59.1, 19 x 1244 64/8 594 | 621, 2 x 1793 at most 47.9 | 62.5, and, as full steps of a ring, 5 x 1000 at most 32/8 up to twice as long
+    with 16 positions per wave; and ragged batches that took longer with 32 positions than with 16 (15 x 356 at most 24/8 16.2 | 19.4)."""
+    small = (SMALL_16, SMALL_32, SMALL_TURNS)
+    for batch, n, heads in ((2, 1594, (32, 8)), (19, 1244, (64, 8)), (5, 1700, (32, 8)), (16, 2000, (32, 8))):
+        for dtype in (0, 1):
+            for m in (None, 256):
+                assert _route(batch, n, heads, total_q=batch * n, total_kv=batch * n, dtype=dtype, m=m) not in small, (batch, n, heads)
+    assert _route(2, 1793, (32, 8), total_q=3029, total_kv=3029) not in small and _route(16, 2000, (32, 8), total_q=14000, total_kv=14000) not in small
+    assert _route(5, 1000, (32, 8), total_q=1400, total_kv=1400, m=256) not in small                     # 3 per CU of 16, one long prompt
+    assert _route(15, 356, (24, 8), total_q=1785, total_kv=1785, dtype=1) == SMALL_16
 
 
 def test_one_prompt_in_a_few_four_wave_workgroups_more_than_two_per_cu():
@@ -454,11 +470,13 @@ def test_longer_prompts_in_few_workgroups_of_16_positions():
     assert one(1000, (40, 40)) == one(1024, (40, 40), 1) == SMALL_16                                     # 640 workgroups, any epilogue
     assert one(1024, (32, 32), **place) not in small and one(1025, (32, 32), **place) == SMALL_16        # 512 and 544
     assert one(1025, (32, 32)) not in small and one(1025, (32, 32), 1) == SMALL_16
-    assert one(1536, (32, 8), **place) == SMALL_16 and one(1537, (32, 8), **place) not in small          # 768 and 776
+    assert one(1280, (32, 8), **place) == SMALL_16 and one(1281, (32, 8), **place) not in small          # 640 and 648
     assert one(1280, (32, 32), 1) == SMALL_16 and one(1281, (32, 32), 1, **place) not in small
+    assert _route(2, 1000, (20, 20), total_q=1900, total_kv=1900) == _route(3, 1000, (20, 20), total_q=1900, total_kv=1900) == SMALL_16
+    assert _route(3, 1000, (32, 8), total_q=1200, total_kv=1200) not in small                            # 624, ragged, four heads side by side
     assert one(1040, (32, 8), 1, **place) not in small
-    assert _route(1, 1120, (32, 32), total_q=1120, total_kv=1536, **place) == SMALL_16                   # (keys beyond the rows)
-    assert _route(1, 1120, (32, 32), total_q=1120, total_kv=1537, **place) not in small
+    assert _route(1, 1120, (32, 32), total_q=1120, total_kv=1280, **place) == SMALL_16                   # (keys beyond the rows)
+    assert _route(1, 1120, (32, 32), total_q=1120, total_kv=1281, **place) not in small
     assert _route(1, 1120, (32, 32), total_q=1120, **place) not in small
 
 
