@@ -1470,22 +1470,25 @@ template <typename T> static int launch_stage1_mfma(const lsattn_decode_stage1_a
 }
 
 // Which launches of the fused call are one (decode_direct_kernel).  A workgroup walks its request in turns of 128 tokens, some 0.8 us each;
-// two launches take some 4 us more than one for their starts and ends, and the longer the request the more workgroups share it.  Measured over
-// 660 launches (32 to 1400 tokens, 1 to 256 requests, ten head counts, f16 and bf16; two launches | one, us, replayed from a graph):
-//   1 x 128 32/8 8.8 | 5.9    1 x 256 32/8 9.5 | 6.6    1 x 512 32/8 9.8 | 8.9    1 x 1024 32/8 9.9 | 13.0    64 x 64..500 32/8 23.2 | 18.3
-//   32 x 300 32/8 15.8 | 11.6    256 x 64..200 32/8 40.7 | 36.0    32 x 1000 32/8 28.1 | 25.5    16 x 100..1000 32/8 13.9 | 16.9
-//   64 x 256 8/1 9.8 | 6.8    8 x 200..300 32/32 12.5 | 9.5    1 x 377 32/32 8.9 | 9.0    36 x 816 24/8 27.4 | 28.0
-// So up to 512 tokens, and up to 1024 where one round of one to two workgroups per CU is full either way (0.75 to 1.00 of two launches);
-// with two or three query heads per KV head (most of an MFMA's columns idle) below four workgroups per CU, 0.99 at worst (past that 1.09);
-// with one, where the lane kernel stands against it, up to 320 tokens and below two per CU.  The launches that it takes: 0.68 in the mean.
+// two launches take some 4 us more than one for their starts and ends, and the longer the request the more workgroups share it.  The launch
+// lasts as long as its longest request, whatever the others are, so the rule takes what is no slower with one long request among short
+// ones, with a mild spread and with equal lengths.  Measured over 2700 launches (the longest 192 to 768 tokens, the others as long, a quarter or
+// 16; 16 to 4096 workgroups; 32/8, 8/1, 64/8, 64/4, 24/8, 16/8 and 32/32 heads, f16 and bf16; two launches | one, us, replayed from a graph):
+//   8 x 320 32/8 10.1 | 9.4    16 x 384 8/1 9.4 | 8.8      16 x 512 32/8 12.8 | 13.7 (not taken)   32, one of 640, the others 160, 32/8 17.5 | 13.7
+//   64 x 640 64/8 37.6 | 32.6  256 x 512 32/8 100 | 95     48 x 512 16/8 22.5 | 24.3 (not taken)   48, one of 1024, the others 128, 32/8 15.0 | 20.3 (not taken)
+//   4 x 320 32/32 9.6 | 9.7    2048 of 80 8/1 49.6 | 29.3  512, one of 320, the others 16, 32/8 36.8 | 39.5 (not taken)
+// So up to 384 tokens, and up to 640 where there is a workgroup per CU (the two launches too walk more than a turn each then); with groups of
+// four to seven query heads up to eight workgroups per CU, of more without a bound (at 16 per CU 0.49 to 0.95); with two or three (most of an
+// MFMA's columns idle) up to 384 tokens below four per CU; with one, where the lane kernel stands against it, up to 320 below two.  The launches
+// taken: 0.71 in the mean, 1.02 at most.
 static bool decode_is_direct(const lsattn_decode_stage1_args* a, const lsattn_decode_stage2_args* s2) {
   const Tuning tn = tuning();
   if (tn.decode_stage1 != 0 || tn.decode_listed != 0) return false;  // (choices among the shapes of two launches)
   if (a->merge_blocks > 1 || a->batch > 65535 || a->k_stride_0 >= (1 << 30) || a->v_stride_0 >= (1 << 30)) return false;
   const int64_t group = a->num_q_heads / a->num_kv_heads, wgs = a->batch * a->num_kv_heads * ((group + 15) / 16), longest = a->max_len_in_batch;
   if (group == 1 ? longest > 320 || wgs >= 2 * kCUs
-      : group < 4 ? longest > 512 || wgs >= 4 * kCUs
-                  : longest > 1024 || (longest > 512 && (wgs < kCUs || wgs > 2 * kCUs)))
+      : group < 4 ? longest > 384 || wgs >= 4 * kCUs
+                  : longest > (wgs < kCUs ? 384 : 640) || (group < 8 && wgs > 8 * kCUs))
     return false;
   // The result is written while other workgroups still read the queries: not where it lies over them, unless row by row (each
   // workgroup reads its own first), or over the lengths and rows of the requests.

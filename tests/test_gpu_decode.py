@@ -754,16 +754,19 @@ def _direct_case(lsa, seed, B, Hq, Hkv, lens, dtype, o_dtype=torch.float32, in_p
 def test_short_contexts_in_one_launch(lsa, dtype, out, Hq, Hkv):
     """Lengths around a batch (32), a turn of the four waves (128) and the ends of the range, none among them."""
     print("case", dtype, out, Hq, Hkv, flush=True)
-    lens = [0, 1, 31, 32, 33, 0, 127, 128, 129, 160, 161, 255, 256, 257, 319, 320] + ([383, 384, 511, 512] if Hq > Hkv else [])
+    lens = [0, 1, 31, 32, 33, 0, 127, 128, 129, 160, 161, 255, 256, 257, 319, 320] + ([383, 384] if Hq > Hkv else [])
     other = torch.bfloat16 if dtype == torch.float16 else torch.float16
     assert _direct_case(lsa, 61, len(lens), Hq, Hkv, lens, dtype, {"float32": torch.float32, "other": other}.get(out, dtype), out == "in place")
 
 
 @pytest.mark.parametrize("Hq,Hkv,B,longest,direct", [
     (4, 4, 1, 320, True), (4, 4, 1, 321, False), (4, 4, 127, 20, True), (4, 4, 128, 20, False), (8, 4, 255, 30, True), (8, 4, 256, 30, False),
-    (8, 4, 1, 512, True), (8, 4, 1, 513, False), (8, 4, 64, 600, False), (32, 8, 300, 40, True), (32, 8, 31, 513, False), (32, 8, 32, 513, True), (8, 1, 256, 1024, True),
-    (8, 1, 257, 1025, False), (32, 8, 64, 600, True), (32, 8, 65, 600, False)])
+    (8, 4, 1, 384, True), (8, 4, 1, 385, False), (8, 4, 64, 385, False), (32, 8, 300, 40, False), (32, 8, 256, 40, True), (32, 8, 31, 385, False),
+    (32, 8, 31, 384, True), (32, 8, 32, 640, True), (32, 8, 32, 641, False), (8, 1, 256, 640, True), (8, 1, 2049, 30, True),
+    (8, 1, 256, 1024, False), (32, 8, 48, 1024, False), (32, 8, 64, 800, False), (32, 8, 16, 512, False), (16, 8, 48, 512, False)])
 def test_which_short_contexts_take_one_launch(lsa, Hq, Hkv, B, longest, direct):
+    """One long request among short ones, for which one launch is no faster than a walk of the long one: past 640 tokens, and past 384 on part
+    of the CUs, two launches share it (48 requests on 32/8 heads, one of 1024 tokens, 15.0 us in two, 20.3 in one)."""
     print("case", Hq, Hkv, B, longest, flush=True)
     assert _direct_case(lsa, 67, B, Hq, Hkv, [longest] + [1 + (7 * i) % min(longest, 60) for i in range(B - 1)], torch.bfloat16) == direct
 
