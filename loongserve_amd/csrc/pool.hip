@@ -5,7 +5,7 @@
 //   add / drop one reference on a list of slots and count          (add_refs :73-79, decrease_refs :82-88)
 // `mem_state` is int32 per slot, 0 = free.  All of it is integer work on a few MB, bound by launch latency and
 // by one pass over the state array; two short launches replace the reference's nonzero / slice / compare chains (three for
-// pools of more than 8 million slots, one for an alloc from up to 65536), one for the reference counts of up to 4096 slots.
+// pools of more than 8 million slots, one for small allocs from up to 65536), one for the reference counts of up to 4096 slots.
 #include "common.hip.h"
 
 namespace lsattn {
@@ -230,15 +230,21 @@ __global__ __launch_bounds__(kPoolThreads) void pool_take_kernel(int32_t* __rest
 }
 
 // ---------------------------------------------------------------------------------------------------
-// alloc of a pool of up to kPoolOneGroup slots in one launch: one workgroup walks it from the front, kScanSlots at a time with the next
+// alloc of a few slots of a pool of up to 65536 in one launch (pool_is_one_group): one workgroup walks it from the front, kScanSlots at a time with the next
 // two lots under way, and stops behind the last slot it takes.  Every wave has 1024 slots in a row of a lot, so that ranks need one count
 // per wave.  Bound by the latency of its first load and, past that, by issue: 0.8 us for a lot without a free slot, 1.5 for one that has some.
-// 24 slots of 65536, device time, the two launches above | this one: half of the pool free 6.1 | 4.0, the last slots only 7.1 | 6.9, scattered
-// over the whole pool 7.0 | 7.8 (256 of them 7.3 | 10.5); and the host has one launch less, 2 us of a decode layer's pass.  Larger pools
-// that are full up to their end would pay more than that, so they keep the two launches, which read the pool on all CUs.
+// The host has one launch less, 3.4 us of a call (15.6 -> 12.2 with a fill in front).  Device time, the two launches above | this one, by where the free slots
+// lie (at the front, every second one, as many as are asked for and scattered over the whole pool, those at its end):
+//   24 of 65536 6.8 | 4.9, 6.2 | 4.3, 7.1 | 8.6, 7.2 | 7.1     64 of 65536 6.7 | 4.9, 6.4 | 4.4, 7.2 | 9.5, 7.2 | 7.1    256 of 65536 6.6 | 4.9, 6.4 | 4.4, 7.3 | 11.7, 7.2 | 7.1
+//   64 of 32768 6.5 | 4.0, 6.2 | 4.6, 7.2 | 6.8, 7.2 | 5.2     256 of 32768 6.5 | 4.1, 6.3 | 4.6, 7.3 | 7.8, 7.3 | 5.3   1024 of 32768 6.6 | 4.7, 6.5 | 4.8, 7.5 | 9.1, 7.2 | 5.9
+//   64 of 16384 6.3 | 3.9, 6.2 | 4.4, 6.9 | 4.8, 6.8 | 4.1     1024 of 16384 6.4 | 4.5, 6.5 | 4.7, 7.2 | 6.0, 7.0 | 4.7  4096 of 16384 7.2 | 4.6, 7.0 | 4.8, 7.2 | 6.0, 7.2 | 4.8
+// So pools of one lot whatever is asked for (all 16384 of 16384 7.3 | 7.7), of two for up to 256 slots, and of four for up to 64: a full pool's few
+// scattered slots then cost the device 2.3 us more at most, less than the host saves, and the other states up to 2.5 less.  Past four lots
+// the walk to the end alone takes as long as the two launches, which read the pool on all CUs.
+// (All lots read and counted before the first is taken from, so that no store stands between them: slower everywhere, 4.3 -> 7.1 and 8.6 -> 10.2.)
 // ---------------------------------------------------------------------------------------------------
-constexpr int64_t kPoolOneGroup = 65536;
 constexpr int kScanPieces = 4, kScanSlots = 1024 * 4 * kScanPieces;
+constexpr bool pool_is_one_group(int64_t size, int64_t need) { return size <= kScanSlots || (size <= 2 * kScanSlots ? need <= 256 : size <= 4 * kScanSlots && need <= 64); }
 __global__ __launch_bounds__(1024) void pool_alloc_one_group_kernel(int32_t* __restrict__ state, int size, int64_t need, int64_t* __restrict__ out_index,
                                                                     int64_t* __restrict__ cells) {
   __shared__ __attribute__((aligned(16))) int sh[2][16];  // (two sets in turn: one barrier per lot)
@@ -576,7 +582,7 @@ extern "C" int lsattn_pool_alloc(int32_t* mem_state, int64_t pool_size, int64_t 
   if (need > 0 && !out_index) return LSATTN_ERR_INVALID_ARG;
   hipStream_t st = (hipStream_t)stream;
   const PoolWorkspace w = pool_carve(workspace, pool_size);
-  if (pool_size <= kPoolOneGroup) {
+  if (pool_is_one_group(pool_size, need)) {
     LSATTN_LAUNCH_KERNEL(pool_alloc_one_group_kernel, dim3(1), dim3(1024), 0, st, mem_state, (int)pool_size, need, out_index, w.cells);
     return check_launch();
   }

@@ -66,6 +66,21 @@ def test_alloc_walks_the_pool_in_lots(lsa, size):
             _same(m, o)
 
 
+@pytest.mark.parametrize("size,need,one", [(16384, 16384, True), (16385, 256, True), (32768, 256, True), (32768, 257, False), (32769, 64, True),
+                                           (65536, 64, True), (65536, 65, False), (65537, 1, False)])
+def test_one_workgroup_allocates_few_slots_of_small_pools(lsa, size, need, one):
+    """Free slots scattered over a pool that is full otherwise: 256 of 65536 took one workgroup 11.7 us, where the launches over all CUs, which
+    leave their counts in the workspace, take 7.3."""
+    rng = np.random.default_rng(need)
+    state = np.ones(size, dtype=np.int32)
+    state[rng.permutation(size)[:need]] = 0
+    m, o = _pair(lsa, state)
+    m._slots._search_ws.fill_(0xAB)
+    assert m.alloc(need).cpu().tolist() == o.alloc(need).tolist()
+    _same(m, o)
+    assert bool((m._slots._search_ws[16:] == 0xAB).all()) == one
+
+
 def test_alloc_through_the_c_abi_pads_with_minus_one_when_the_pool_runs_out(lsa):
     from loongserve_amd import _lib
     lib = _lib.load()
