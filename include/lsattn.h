@@ -110,14 +110,14 @@ typedef struct lsattn_prefill_args {
   int64_t total_q_rows;
   /* Optional (0: unknown); no counterpart in the reference.  An upper bound of the sum of kv_b_seq_len over the batch (the
    * rows of a packed k).  With it, total_q_rows and max_kv_len the library can tell a batch of short prompts from short chunks
-   * behind long contexts, and takes a kernel of shorter workgroups for the former.  It only steers that choice: a wrong
-   * bound costs time, not results. */
+   * behind long contexts, and takes a kernel of shorter workgroups for the former; and where the K/V read exceeds the L2s that
+   * kernel takes the requests a few at a time.  It only steers these choices: a wrong bound costs time, not results. */
   int64_t total_kv_rows;
   /* With kv_cuts = S > 1.  0: cut c of a sequence is [c * kv_cut_len, (c + 1) * kv_cut_len), as above.  1: the S cuts of a sequence
    * are equal, ceil(kv_b_seq_len / S) keys rounded up to a multiple of 64 but at most kv_cut_len, so that every cut of a short
    * sequence has keys too (the host knows the longest chunk a batch can hold, not the lengths). */
   int32_t kv_cut_even;
-  /* Optional (0 or less: unknown).  An upper bound of every kv_b_seq_len; steers the same choice as total_kv_rows, and like it
+  /* Optional (0 or less: unknown).  An upper bound of every kv_b_seq_len; steers the same choices as total_kv_rows, and like it
    * costs time at most. */
   int32_t max_kv_len;
 } lsattn_prefill_args;

@@ -480,6 +480,19 @@ def test_longer_prompts_in_few_workgroups_of_16_positions():
     assert _route(1, 1120, (32, 32), total_q=1120, **place) not in small
 
 
+def test_spare_rows_of_the_k_buffer_leave_the_order_of_the_grid_alone():
+    """64-wide heads, ragged requests that take turns (ids of a tile a multiple of 32, which a bunch of one request is not): against a K buffer of
+    many more rows than the requests have as against their own, with the bound on the rows and with one on the keys; behind contexts
+    that the caller bounds, the K/V read counts."""
+    ragged = dict(total_q=9000)
+    assert _route(8, 2000, (32, 8), 64, total_kv=9000, **ragged) == SMALL_TURNS
+    for spare in (1 << 17, 1 << 20):
+        assert _route(8, 2000, (32, 8), 64, total_kv=spare, **ragged) == SMALL_TURNS
+        assert _route(8, 2000, (32, 8), 64, total_kv=spare, max_kv=2000, **ragged) == SMALL_TURNS
+        assert _route(8, 2000, (32, 8), 64, total_kv=spare, max_kv=40000, **ragged) == SMALL_32
+    assert _route(8, 30000, (32, 8), 64, total_q=130000, total_kv=130000) == SMALL_32                  # (266 MB, bunches of one)
+
+
 def test_prefill_route_names_a_kernel_for_every_step_and_none_for_others():
     assert _route(24, 256, (32, 32), total_q=1800, total_kv=1800) == SMALL_32
     assert _route(8, 3000, (32, 8), 64, total_q=16000, total_kv=16000) == SMALL_TURNS
