@@ -567,16 +567,20 @@ __global__ __launch_bounds__(kWaves * 64, (kResident<D, WP, DV>)) void prefill_s
   }
 }
 
-// Whether a request's place among the ids moves on from tile to tile.  Ids go to the eight XCDs in turn and within one to its four
-// shader engines.  If the ids of two tiles of a request are a multiple of 32 apart, all its workgroups share one shader engine of an
-// XCD, and while only the longest requests have a tile left to start, the others idle: 8 sequences of 1000 to 3000 tokens, 32/8 heads
-// of 64, had 2 workgroups on a CU until half of the launch was over, some 4 and some 1, where 8 x 2048 keep 3.9.  Turning places
-// fill them evenly.  Measured over 60 ragged launches (2 to 32 sequences, 300 to 6000 tokens; microseconds, fixed | turning):
-//   8 x 1000..3000 32/8 183 | 165   2 x 1206..3618 64/8 144 | 123   4 x 120..3615 64/8 bf16 87.9 | 61.8   4 x 688..2064 32/32 53.2 | 47.3
-//   4 x 2582..5165 32/8 bf16 344 | 314   8 x 1304..2608 12/12 88.8 | 79.5   16 x 31..959 64/8 57.3 | 53.5
-// At other distances (11 x 388..1166 32/8 44.8 | 47.1; distance 6 of the eights 9 % better to 4 % worse), with fewer than 16 tiles
-// (8 x 280..842 32/32 31.5 | 33.3) and with equal lengths turning gains nothing: there the places stay.
-bool ragged(const lsattn_prefill_args* a) { return a->total_q_rows > 0 && a->total_q_rows * 10 <= (int64_t)a->batch * a->max_q_len * 9; }
+// query heads of a KV head side by side in a workgroup: as many (1, 2 or 4; the power of two) as the group divides by
+int pack_shift_of(const lsattn_prefill_args* a) {
+  const int32_t heads = a->num_q_heads / a->num_kv_heads;
+  return heads % 4 == 0 ? 2 : heads % 2 == 0 ? 1 : 0;
+}
+// Workgroups that find rows, with `blocks` blocks of 16 positions per wave: the longest request's times the batch, or fewer if
+// the caller bounds the rows of all requests together.
+int64_t workgroups(const lsattn_prefill_args* a, int pack_shift, int blocks) {
+  const int64_t rows = (kWaves * blocks * 16) >> pack_shift;
+  const int64_t by_longest = a->batch * ((a->max_q_len + rows - 1) / rows);
+  const int64_t by_total = a->total_q_rows > 0 ? (a->total_q_rows + rows - 1) / rows + a->batch : by_longest;
+  return (by_total < by_longest ? by_total : by_longest) * (a->num_q_heads >> pack_shift);
+}
+
 // Rows of K that the requests read, as far as the host can tell: those of the prompts, and of contexts where the caller bounds them.  The K
 // buffer may have more (a view with spare rows).
 int64_t kv_rows_read(const lsattn_prefill_args* a) {
@@ -587,13 +591,23 @@ int64_t kv_rows_read(const lsattn_prefill_args* a) {
   if (a->max_kv_len > 0 && (int64_t)a->batch * a->max_kv_len < rows) rows = (int64_t)a->batch * a->max_kv_len;
   return rows;
 }
+
+// Whether a request's place among the ids moves on from tile to tile.  Ids go to the eight XCDs in turn and within one to its four
+// shader engines.  If the ids of two tiles of a request are a multiple of 32 apart, all its workgroups share one shader engine of an
+// XCD, and while only the longest requests have a tile left to start, the others idle: 8 sequences of 1000 to 3000 tokens, 32/8 heads
+// of 64, had 2 workgroups on a CU until half of the launch was over, some 4 and some 1, where 8 x 2048 keep 3.9.  Turning places
+// fill them evenly.  Measured over 60 ragged launches (2 to 32 sequences, 300 to 6000 tokens; microseconds, fixed | turning):
+//   8 x 1000..3000 32/8 183 | 165   2 x 1206..3618 64/8 144 | 123   4 x 120..3615 64/8 bf16 87.9 | 61.8   4 x 688..2064 32/32 53.2 | 47.3
+//   4 x 2582..5165 32/8 bf16 344 | 314   8 x 1304..2608 12/12 88.8 | 79.5   16 x 31..959 64/8 57.3 | 53.5
+// At other distances (11 x 388..1166 32/8 44.8 | 47.1; distance 6 of the eights 9 % better to 4 % worse), with fewer than 16 tiles
+// (8 x 280..842 32/32 31.5 | 33.3) and with equal lengths turning gains nothing: there the places stay.
+bool ragged(const lsattn_prefill_args* a) { return a->total_q_rows > 0 && a->total_q_rows * 10 <= (int64_t)a->batch * a->max_q_len * 9; }
 bool requests_take_turns(const lsattn_prefill_args* a, int64_t ids_per_tile, int64_t tiles) {
   return ids_per_tile % 32 == 0 && tiles >= 16 && ragged(a);
 }
 
 // How many requests the grid takes at a time (a bunch), the heaviest tiles of all of them first.  All of the batch starts the heaviest work of the
-// launch first,
-// and is best for ragged batches; but every layer of tiles then reads the K/V of the whole batch again, which past the
+// launch first, and is best for ragged batches; but every layer of tiles then reads the K/V of the whole batch again, which past the
 // L2s' 32 MB comes from beyond them, so bunches hold about as much.  And short prompts of about equal length leave the CUs unevenly filled that
 // way (their workgroups come in layers of equal length): in bunches of some 512 workgroups, light tiles of one run beside heavy
 // ones of the next.  Measured (microseconds, 1, 2, 4, 8, 16 and 32 requests at a time up to the batch, 128-wide heads):
@@ -603,13 +617,17 @@ bool requests_take_turns(const lsattn_prefill_args* a, int64_t ids_per_tile, int
 // and 64-wide: 16 x 1024 32/32 119 120 125 128 140   8 x 2048 32/32 198 192 189 210   16 x 512 32/8 44.3 42.2 39.9 45.1 44.4   16 x 1024 32/8 117 112 112 108 108
 // The K/V bytes are those that the requests read (kv_rows_read), not those of the buffer: in bunches of one or two for a larger buffer's sake, requests
 // of 16- to 64-wide heads took up to a third longer (14 x 1300 at most 16/16 against 65536 rows; 250 ragged batches 1.035 in the mean).  Ragged batches
-// gain by bytes too, though they lose the heaviest-first order of the whole batch: 375 of 300 to 6000 tokens whose K/V is 64 MB and more, 16- to
-// 64-wide heads, 0.955 in the mean (0.73 to 1.14), 192 of 128-wide ones 0.973; equal lengths 0.936 (121 launches) and 0.948 (85).
+// gain by bytes too, though they lose the heaviest-first order of the whole batch, but not where a bunch is about one round of workgroups, which then
+// ends with the longest request's alone (16- to 64-wide heads, where one has 1024; 11 x 5345 at most 16/16 146 us whole, 193 in two).  Over launches of 300 to
+// 6000 tokens whose K/V is 64 MB and more, of the time before the bunches (all at once | by bytes | by bytes from two rounds per bunch on; the mean, the worst):
+//   16 to 64 wide, 540 ragged 0.944 1.05 | 0.899 1.33 | 0.910 1.05, 188 equal 0.950 1.06 | 0.888 1.19 | 0.913 1.06;  128 wide, 305 ragged 0.880 1.29 | 0.849 1.10, 143 equal 0.957 1.55 | 0.894 1.10
+// (128-wide heads fill a bunch of 32 MB with half a round, and fare best so.)
 int64_t requests_per_bunch(const lsattn_prefill_args* a, int64_t ids, int64_t tiles) {
   int64_t bunches = 1;
   const int64_t kv_bytes = kv_rows_read(a) * a->num_kv_heads * a->head_dim * 4;
-  if (kv_bytes >= 2 * kL2Bytes) bunches = kv_bytes / kL2Bytes;
   const int64_t wgs = ids * tiles * a->batch, resident = (a->head_dim == 128 ? 3 : 4) * kCUs;
+  const int64_t by_kv = kv_bytes / kL2Bytes < a->batch ? kv_bytes / kL2Bytes : a->batch;
+  if (by_kv > 1 && (a->head_dim == 128 || workgroups(a, pack_shift_of(a), 2) >= 2 * resident * by_kv)) bunches = by_kv;
   if (a->total_q_rows > 0 && !ragged(a) && a->max_q_len <= 512 && wgs > resident && wgs / kBunchWorkgroups > bunches) bunches = wgs / kBunchWorkgroups;
   if (bunches > a->batch) bunches = a->batch;
   return (a->batch + bunches - 1) / bunches;
@@ -644,20 +662,6 @@ template <typename T, int D, int MODE, bool DV, int WP> int launch_rows(SmallPar
     if (rc != LSATTN_OK) return rc;
   }
   return LSATTN_OK;
-}
-
-// query heads of a KV head side by side in a workgroup: as many (1, 2 or 4; the power of two) as the group divides by
-int pack_shift_of(const lsattn_prefill_args* a) {
-  const int32_t heads = a->num_q_heads / a->num_kv_heads;
-  return heads % 4 == 0 ? 2 : heads % 2 == 0 ? 1 : 0;
-}
-// Workgroups that find rows, with `blocks` blocks of 16 positions per wave: the longest request's times the batch, or fewer if
-// the caller bounds the rows of all requests together.
-int64_t workgroups(const lsattn_prefill_args* a, int pack_shift, int blocks) {
-  const int64_t rows = (kWaves * blocks * 16) >> pack_shift;
-  const int64_t by_longest = a->batch * ((a->max_q_len + rows - 1) / rows);
-  const int64_t by_total = a->total_q_rows > 0 ? (a->total_q_rows + rows - 1) / rows + a->batch : by_longest;
-  return (by_total < by_longest ? by_total : by_longest) * (a->num_q_heads >> pack_shift);
 }
 
 // 32 positions per wave serve twice the rows with each K and V operand read, 16 make twice as many, shorter waves: these from

@@ -481,16 +481,22 @@ def test_longer_prompts_in_few_workgroups_of_16_positions():
 
 
 def test_spare_rows_of_the_k_buffer_leave_the_order_of_the_grid_alone():
-    """64-wide heads, ragged requests that take turns (ids of a tile a multiple of 32, which a bunch of one request is not): against a K buffer of
-    many more rows than the requests have as against their own, with the bound on the rows and with one on the keys; behind contexts
-    that the caller bounds, the K/V read counts."""
-    ragged = dict(total_q=9000)
-    assert _route(8, 2000, (32, 8), 64, total_kv=9000, **ragged) == SMALL_TURNS
-    for spare in (1 << 17, 1 << 20):
-        assert _route(8, 2000, (32, 8), 64, total_kv=spare, **ragged) == SMALL_TURNS
-        assert _route(8, 2000, (32, 8), 64, total_kv=spare, max_kv=2000, **ragged) == SMALL_TURNS
-        assert _route(8, 2000, (32, 8), 64, total_kv=spare, max_kv=40000, **ragged) == SMALL_32
-    assert _route(8, 30000, (32, 8), 64, total_q=130000, total_kv=130000) == SMALL_32                  # (266 MB, bunches of one)
+    """64-wide heads, ragged requests that take turns (ids of a tile a multiple of 32, which those of a bunch of one request are not): against a K
+    buffer of many more rows than the requests have as against their own, with the bound on the rows and with one on the keys; behind
+    contexts that the caller bounds, the K/V read counts."""
+    for spare in (0, 1 << 17, 1 << 20):
+        assert _route(8, 2000, (32, 8), 64, total_q=9000, total_kv=9000 + spare) == SMALL_TURNS
+        assert _route(8, 2000, (32, 8), 64, total_q=9000, total_kv=9000 + spare, max_kv=2000) == SMALL_TURNS
+    # (184 MB read, bunches of one request; 41 MB)
+    assert _route(8, 20000, (32, 8), 64, total_q=90000, total_kv=1 << 20, max_kv=20000) == SMALL_32
+    assert _route(8, 8000, (32, 8), 64, total_q=20000, total_kv=1 << 20, max_kv=8000) == SMALL_TURNS
+
+
+def test_bunches_by_the_kv_that_is_read_have_two_rounds_of_workgroups():
+    """64-wide heads, ragged, 16/16 heads, K/V of 73 MB: two bunches would be about a round of workgroups each, of which one ends with the longest
+    request's alone (11 requests of at most 5345 tokens 193 us, whole 146); 266 MB on 32/8 are eight bunches of four rounds."""
+    assert _route(6, 5345, (16, 16), 64, total_q=18652, total_kv=18652) == SMALL_TURNS    # (6 x 16 ids a tile are a multiple of 32, 3 x 16 are not)
+    assert _route(8, 30000, (32, 8), 64, total_q=130000, total_kv=130000) == SMALL_32     # (8 x 8 are, 8 are not)
 
 
 def test_prefill_route_names_a_kernel_for_every_step_and_none_for_others():

@@ -101,10 +101,10 @@ def test_short_rows_behind_one_long_context_and_bounded_ones(lsa, dtype):
 SMALL_16, SMALL_32, SMALL_TURNS = 1, 2, 3  # LSATTN_ROUTE_* of include/lsattn.h
 
 
-def _every_epilogue_on(route, lsa, mode, V, D, Hq, Hkv, lens, ctx, spare=0, max_kv=None):
+def _every_epilogue_on(route, lsa, mode, V, D, Hq, Hkv, lens, ctx, spare=0):
     """One step (the partial) or two over halves of the keys (the folding epilogues) against the oracle, each of them on `route`.
     V: "f16", "bf16" (converted by the kernel) or "bf16 copied" (the caller's buffer for the fp16 copy).  spare: rows of the K/V
-    buffers behind the last request's.  max_kv: a bound of the keys, if the caller has one."""
+    buffers behind the last request's."""
     from loongserve_amd import _lib, ops
     dtype = torch.float16 if V == "f16" else torch.bfloat16
     klens = [n + c for n, c in zip(lens, ctx)]
@@ -120,7 +120,7 @@ def _every_epilogue_on(route, lsa, mode, V, D, Hq, Hkv, lens, ctx, spare=0, max_
     qd, kd, vd, qmd = *_dev(q, k, v), _dev(*qm)
     if spare:
         kd, vd = (torch.cat([x, x.new_full((spare, Hkv, D), float("nan"))]) for x in (kd, vd))
-    kw = dict(max_kv_len=max_kv, **(dict(v_f16=torch.empty(vd.shape, dtype=torch.float16, device=DEV)) if V == "bf16 copied" else {}))
+    kw = dict(v_f16=torch.empty(vd.shape, dtype=torch.float16, device=DEV)) if V == "bf16 copied" else {}
 
     def on_route(o, s):
         a = ops._prefill_args(qd, kd, vd, o, *qmd, *s, 1, max(lens), None, total_q_len=T, **kw)
@@ -172,7 +172,7 @@ def test_requests_that_take_turns_in_the_grid(lsa, mode, V, D):
 def test_short_prompts_in_three_stages_and_the_grids_orders(lsa, mode, V, what):
     """128-wide heads with 32 positions per wave: prompts around multiples of the 32-key tiles and their three stages; a ragged batch whose
     requests take turns; and grids that take a few requests at a time, by the count of workgroups (a last bunch that is short) and,
-    where the K/V that the requests may read is larger than the L2s, by that."""
+    where the K/V that the requests read is larger than the L2s, by that."""
     print("case", mode, V, what, flush=True)
     if what == "stages":
         _every_epilogue_on(SMALL_32, lsa, mode, V, 128, 16, 4, [31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 159, 161, 191, 193] * 2, [0, 31, 1, 0] * 8)
@@ -183,7 +183,7 @@ def test_short_prompts_in_three_stages_and_the_grids_orders(lsa, mode, V, what):
     elif what == "bunches of 64":
         _every_epilogue_on(SMALL_32, lsa, mode, V, 64, 8, 8, [130] * 72 + [1], [0] * 73)
     else:
-        _every_epilogue_on(SMALL_32, lsa, mode, V, 64, 32, 8, [700, 33, 650, 64, 1, 600, 400, 20, 300, 512, 129], [0] * 11, spare=1 << 16, max_kv=20000)
+        _every_epilogue_on(SMALL_32, lsa, mode, V, 128, 32, 32, [700, 33, 650, 64, 1, 600, 400, 20, 768, 512, 129, 300, 300], [0] * 13, spare=64)
 
 
 @pytest.mark.parametrize("mode", ["partial", "accumulate", "in_place"])
