@@ -614,7 +614,11 @@ bool requests_take_turns(const lsattn_prefill_args* a, int64_t ids_per_tile, int
 //   16 x 512 32/32 (8 MB each) 77 75 78 86 99   16 x 1024 32/32 (16 MB) 231 229 235 243 262   32 x 512 32/32 170 169 171 182 197 201
 //   32 x 256 32/8 52.2 50.6 47.9 52.0 61.4 61.4   16 x 256 32/8 34.6 32.8 30.8 30.5 35.6   8 x 512 32/8 44.3 42.0 37.8 43.4   16 x 512 32/8 71 67 64 70 72
 //   16 x 1024 32/8 216 207 204 201 206   4 x 1024 32/8 62.7 57.9 55.3   ragged: 8 x 100..2000 32/8 70.6 68.9 64.3 61.2, 20 x 200..800 32/8 81 78 72 80 80 71 (all 20)
-// and 64-wide: 16 x 1024 32/32 119 120 125 128 140   8 x 2048 32/32 198 192 189 210   16 x 512 32/8 44.3 42.2 39.9 45.1 44.4   16 x 1024 32/8 117 112 112 108 108
+// and 64-wide: 16 x 1024 32/32 119 120 125 128 140   8 x 2048 32/32 198 192 189 210   16 x 1024 32/8 117 112 112 108 108
+// Short equal prompts over 3000 launches (2 to 60 of 60 to 512 tokens), in bunches of some 512 workgroups, of the time of all at once (the mean; 95 of 100
+// stay below): 128-wide 0.97 (1.03); narrower heads, one per workgroup, from two rounds of the chip on 0.86 (0.99), below 0.99 (1.07); several
+// side by side, whose prompts have up to four times the tiles, 1.02 (1.12), the worst 1.28 (11 x 333 64/8 16-wide 17.9 | 20.7).  Narrower heads thus
+// only the first of these.
 // The K/V bytes are those that the requests read (kv_rows_read), not those of the buffer: in bunches of one or two for a larger buffer's sake, requests
 // of 16- to 64-wide heads took up to a third longer (14 x 1300 at most 16/16 against 65536 rows; 250 ragged batches 1.035 in the mean).  Ragged batches
 // gain by bytes too, though they lose the heaviest-first order of the whole batch, but not where a bunch is about one round of workgroups, which then
@@ -628,7 +632,8 @@ int64_t requests_per_bunch(const lsattn_prefill_args* a, int64_t ids, int64_t ti
   const int64_t wgs = ids * tiles * a->batch, resident = (a->head_dim == 128 ? 3 : 4) * kCUs;
   const int64_t by_kv = kv_bytes / kL2Bytes < a->batch ? kv_bytes / kL2Bytes : a->batch;
   if (by_kv > 1 && (a->head_dim == 128 || workgroups(a, pack_shift_of(a), 2) >= 2 * resident * by_kv)) bunches = by_kv;
-  if (a->total_q_rows > 0 && !ragged(a) && a->max_q_len <= 512 && wgs > resident && wgs / kBunchWorkgroups > bunches) bunches = wgs / kBunchWorkgroups;
+  const bool layers = a->head_dim == 128 ? wgs > resident : pack_shift_of(a) == 0 && wgs >= 2 * resident;
+  if (a->total_q_rows > 0 && !ragged(a) && a->max_q_len <= 512 && layers && wgs / kBunchWorkgroups > bunches) bunches = wgs / kBunchWorkgroups;
   if (bunches > a->batch) bunches = a->batch;
   return (a->batch + bunches - 1) / bunches;
 }

@@ -181,7 +181,7 @@ def test_short_prompts_in_three_stages_and_the_grids_orders(lsa, mode, V, what):
     elif what == "bunches":
         _every_epilogue_on(SMALL_32, lsa, mode, V, 128, 16, 8, [130] * 19 + [97], [0] * 20)
     elif what == "bunches of 64":
-        _every_epilogue_on(SMALL_32, lsa, mode, V, 64, 8, 8, [130] * 72 + [1], [0] * 73)
+        _every_epilogue_on(SMALL_32, lsa, mode, V, 64, 16, 16, [130] * 72 + [1], [0] * 73)
     else:
         _every_epilogue_on(SMALL_32, lsa, mode, V, 128, 32, 32, [700, 33, 650, 64, 1, 600, 400, 20, 768, 512, 129, 300, 300], [0] * 13, spare=64)
 
