@@ -715,15 +715,16 @@ __device__ __forceinline__ void stage1_mfma_unit(const Stage1Params& p, char* ld
     u32x4 phi, plo, prest;
     if (DIRECT && std::is_same<T, F16>::value) {
       // P in two parts of eleven bits, 2^14 times as large (which the result is divided by), so that a small weight keeps its bits too.
-      // The parts are cut off and so none is below zero; nor is the second one zero (2^-38 of the largest weight), or an infinite V would
-      // turn into a NaN at it.  (Weights below 2^-38 have no first part, as those below 2^-25 have none in the kernels of two launches.)
+      // The parts are cut off and so none is below zero; nor is the second one zero beside a first one (but at least 2^-38 of the largest weight), or an
+      // infinite V would turn into a NaN at it.  A weight of zero has no parts.  (Weights below 2^-38 have no first part, as those below
+      // 2^-25 have none in the kernels of two launches.)
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         const float x0 = pv[2 * e] * kUp, x1 = pv[2 * e + 1] * kUp;
         phi[e] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x0, x1));
         float h0, h1;
         unpack2<F16>(phi[e], h0, h1);
-        plo[e] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(fmaxf(x0 - h0, 0x1p-24f), fmaxf(x1 - h1, 0x1p-24f)));
+        plo[e] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(fmaxf(x0 - h0, fminf(x0, 0x1p-24f)), fmaxf(x1 - h1, fminf(x1, 0x1p-24f))));
       }
     } else if (std::is_same<T, F16>::value) {
 #pragma unroll
@@ -738,9 +739,9 @@ __device__ __forceinline__ void stage1_mfma_unit(const Stage1Params& p, char* ld
         for (int i = 0; i < 2; i++) {
           const float x = pv[2 * e + i];
           hi[i] = __builtin_bit_cast(uint32_t, x) & 0xffff0000u;
-          const float x1 = fmaxf(x - __builtin_bit_cast(float, hi[i]), 0x1p-126f);
+          const float least = fminf(x, 0x1p-126f), x1 = fmaxf(x - __builtin_bit_cast(float, hi[i]), least);
           lo[i] = __builtin_bit_cast(uint32_t, x1) & 0xffff0000u;
-          rest[i] = fmaxf(x1 - __builtin_bit_cast(float, lo[i]), 0x1p-126f);
+          rest[i] = fmaxf(x1 - __builtin_bit_cast(float, lo[i]), least);
         }
         phi[e] = (hi[0] >> 16) | hi[1];
         plo[e] = (lo[0] >> 16) | lo[1];

@@ -820,3 +820,29 @@ def test_one_launch_and_infinite_keys_and_values(lsa, tuning, dtype):
     fin = o2.isfinite()
     assert_o_close(o[fin], o2[fin], "o")
     assert_lse_close(l, l2, "lse")
+
+
+@pytest.mark.parametrize("dtype,huge", [(torch.float16, 65504.0), (torch.bfloat16, 3e38)])
+@pytest.mark.parametrize("Hq,Hkv", [(4, 4), (8, 2)])
+def test_one_launch_and_huge_values_that_weigh_nothing(lsa, dtype, huge, Hq, Hkv):
+    """Tokens with scores of minus infinity and values at the end of the type's range, among them the last one, which the places past a request's end
+    repeat: the sum over the others, small by comparison, is as if they were not there."""
+    print("case", dtype, Hq, Hkv, flush=True)
+    D, lens = 128, [33, 40, 200, 129, 1 + 128 + 31]
+    q, kv, table, b_req, b_len = decode_case(79, len(lens), Hq, Hkv, D, lens, 700, dtype)
+    q = q.abs() + 0.125
+    kv[:, Hkv:] = kv[:, Hkv:] * 2.0 ** -10
+    for b, n in enumerate(lens):
+        gone = table[int(b_req[b])][[0, n // 2, n - 1]].long()
+        kv[gone, :Hkv] = float("-inf")
+        kv[gone, Hkv:] = huge
+    o_ref, l_ref = orc.decode_full(q, kv[:, :Hkv], kv[:, Hkv:], table, b_req, b_len)
+    kvd = kv.to(DEV)
+    mo, ml = torch.full((1, len(lens), Hq, D), float("nan"), device=DEV), torch.full((1, len(lens), Hq), float("nan"), device=DEV)
+    o, l = lsa.longserve_token_decode_attention_flash_decoding(q.to(DEV), table.to(DEV), b_req.to(DEV), b_len.to(DEV), mo, ml, len(lens), max(lens), Hq, D,
+                                                               kvd[:, :Hkv], kvd[:, Hkv:], 256)
+    torch.cuda.synchronize()
+    assert bool(torch.isnan(mo).all())  # (one launch)
+    # (2^-10 of what the sums of values around 1 are held to)
+    assert_o_close(o * 2.0 ** 10, o_ref * 2.0 ** 10, "o")
+    assert_lse_close(l, l_ref, "lse")
