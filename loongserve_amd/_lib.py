@@ -76,7 +76,7 @@ class DecodeStage1Args(C.Structure):
 
 class DecodeStage2Args(C.Structure):
     _fields_ = [
-        ("o", _vp), ("o_dtype", _i32), ("reserved", _i32), ("out_logexpsum", _vp), ("b_seqlen", _vp),
+        ("o", _vp), ("o_dtype", _i32), ("o_is_apart", _i32), ("out_logexpsum", _vp), ("b_seqlen", _vp),
         ("mid_o", _vp), ("mid_o_logexpsum", _vp),
         ("batch", _i64), ("num_heads", _i64), ("num_seq_blocks", _i64), ("head_dim", _i64), ("block_seq", _i64),
         ("partials_by_request", _i64),
@@ -96,7 +96,7 @@ TUNING_VALUES = {
     "decode_stage1": {None: 0, "lane": 1, "mfma": 2, "split": 3},
     "decode_listed": {None: 0, "off": 1, "on": 2, "shares": 3},
 }
-LSATTN_VERSION = 6  # of include/lsattn.h, which the argument blocks above mirror
+LSATTN_VERSION = 7  # of include/lsattn.h, which the argument blocks above mirror
 
 
 # every symbol include/lsattn.h declares: name -> (restype, argtypes)

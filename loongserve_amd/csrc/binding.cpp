@@ -386,6 +386,16 @@ struct Decode {
   }
 };
 
+// whether two tensors share no address from the first to the last element of each
+bool no_overlap(const at::Tensor& x, const at::Tensor& y) {
+  auto end = [](const at::Tensor& t) {
+    int64_t last = 0;
+    for (int64_t d = 0; d < t.dim(); d++) last += (t.size(d) - 1) * t.stride(d);
+    return (const char*)t.data_ptr() + (t.numel() ? (last + 1) * (int64_t)t.element_size() : 0);
+  };
+  return end(x) <= (const char*)y.data_ptr() || end(y) <= (const char*)x.data_ptr();
+}
+
 // (q, table, b_req, b_len, mid_o, mid_lse, batch, max_len, q_heads, head_dim, k, v, split, out, out_lse, by_request)
 // -> (out, out_lse) or None
 PyObject* token_decode_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
@@ -407,6 +417,8 @@ PyObject* token_decode_attention(PyObject*, PyObject* const* args, Py_ssize_t na
   const at::Tensor lse = lse_in ? *lse_in : empty({batch, Hq}, *q, at::kFloat);
   OR_NONE(d.stage2(out, lse, b_len, mid_o, mid_lse, split));
   d.s1.partials_by_request = d.s2.partials_by_request = by_request;
+  d.s2.o_is_apart = (!out_in || (no_overlap(out, k) && no_overlap(out, v) && no_overlap(out, table))) &&
+                    (!lse_in || (no_overlap(lse, k) && no_overlap(lse, v) && no_overlap(lse, table)));
   if (const int rc = call(lib.decode_attention, &d.s1, &d.s2, stream())) return failed(rc, "lsattn_decode_attention");
   PyObject* o1 = out_in ? (Py_INCREF(py_out), py_out) : THPVariable_Wrap(out);
   PyObject* o2 = lse_in ? (Py_INCREF(py_lse), py_lse) : THPVariable_Wrap(lse);

@@ -1491,8 +1491,10 @@ static bool decode_is_direct(const lsattn_decode_stage1_args* a, const lsattn_de
       : group < 4 ? longest > 384 || wgs >= 4 * kCUs
                   : longest > (wgs < kCUs ? 384 : 640) || (group < 8 && wgs > 8 * kCUs))
     return false;
-  // The result is written while other workgroups still read the queries: not where it lies over them, unless row by row (each
-  // workgroup reads its own first), or over the lengths and rows of the requests.
+  // The result is written while other workgroups still read.  Whether it lies over the pool's rows or the table only the caller knows (their
+  // extents are not in the arguments).  Not where it lies over the queries, unless row by row (each workgroup reads its own first),
+  // or over the lengths and rows of the requests.
+  if (s2->o_is_apart != 1) return false;
   const int64_t pairs = a->batch * a->num_q_heads;
   auto apart = [](const void* x, int64_t nx, const void* y, int64_t ny) { return (const char*)x + nx <= (const char*)y || (const char*)y + ny <= (const char*)x; };
   const int64_t o_bytes = pairs * 128 * (s2->o_dtype == LSATTN_F32 ? 4 : 2), q_bytes = pairs * 256;

@@ -133,6 +133,14 @@ def flash_decoding_stage2(o, out_logexpsum, b_seqlen, mid_o, mid_o_logexpsum, bl
 FUSED_PARTIALS_BY_REQUEST = True
 
 
+def _apart(x: torch.Tensor, y: torch.Tensor) -> bool:
+    """Whether two tensors share no address from the first to the last element of each."""
+    def end(t):
+        last = sum((n - 1) * s for n, s in zip(t.shape, t.stride()))
+        return t.data_ptr() + ((last + 1) * t.element_size() if t.numel() else 0)
+    return end(x) <= y.data_ptr() or end(y) <= x.data_ptr()
+
+
 def flash_decoding(mid_o, mid_o_logexpsum, q, k, v, req_to_tokens, b_req_idx, b_seqlen, max_len_in_batch: int,
                    o, out_logexpsum, block_seq: int) -> None:
     """Stage 1 and stage 2 with the same block size from one library call (what FDPY:12-27 does with two): the checks of
@@ -144,6 +152,7 @@ def flash_decoding(mid_o, mid_o_logexpsum, q, k, v, req_to_tokens, b_req_idx, b_
     a1 = _stage1_args(mid_o, mid_o_logexpsum, q, k, v, req_to_tokens, b_req_idx, b_seqlen, max_len_in_batch, block_seq)
     a2 = _stage2_args(o, out_logexpsum, b_seqlen, mid_o, mid_o_logexpsum, block_seq)
     a1.partials_by_request = a2.partials_by_request = 1 if FUSED_PARTIALS_BY_REQUEST else 0
+    a2.o_is_apart = all(_apart(x, y) for x in (o, out_logexpsum) for y in (k, v, req_to_tokens))
     _lib.check(_lib.load().lsattn_decode_attention(C.byref(a1), C.byref(a2), _stream()), "lsattn_decode_attention")
 
 
@@ -163,6 +172,7 @@ def flash_decoding_static(q, k, v, req_to_tokens, b_req_idx, b_seqlen, max_len_i
     a1 = _stage1_args(mid_o, mid_lse, q, k, v, req_to_tokens, b_req_idx, b_seqlen, max_len_in_batch, block_seq,
                       partials_in_library=True)
     a2 = _stage2_args(o, out_logexpsum, b_seqlen, mid_o, mid_lse, block_seq, partials_in_library=True)
+    a2.o_is_apart = all(_apart(x, y) for x in (o, out_logexpsum) for y in (k, v, req_to_tokens))
     _lib.check(_lib.load().lsattn_decode_attention_static(C.byref(a1), C.byref(a2), _stream()),
                "lsattn_decode_attention_static")
 

@@ -791,6 +791,37 @@ def test_result_over_the_queries_takes_two_launches(lsa):
         assert_lse_close(l, l_ref, "lse")
 
 
+@pytest.mark.parametrize("call", ["native", "checked", "static"])
+@pytest.mark.parametrize("where", ["apart", "o over K", "o over V", "o over the table", "lse over K", "lse over the table"])
+def test_result_over_the_pool_or_the_table_is_written_behind_the_last_read(lsa, monkeypatch, call, where):
+    """Short contexts whose result lies over rows of the pool, or of the table, that requests still read: two launches, as for calls of the C ABI that do
+    not say that it lies apart."""
+    print("case", call, where, flush=True)
+    ck, D, B, Hq, Hkv, lens = lsa.longserve_cuda_kernels, 128, 8, 8, 2, [100, 1, 300, 64, 256, 31, 200, 128]
+    if call == "checked":
+        monkeypatch.setattr(ck._native, "token_decode_attention", lambda *a: None)
+    q, kv, table, b_req, b_len = decode_case(83, B, Hq, Hkv, D, lens, 2000, torch.float16, pad_seq=200)
+    o_ref, l_ref = orc.decode_full(q, kv[:, :Hkv], kv[:, Hkv:], table, b_req, b_len)
+    qd, rd, ld, td = q.to(DEV), b_req.to(DEV), b_len.to(DEV), table.to(DEV).contiguous()
+    pool = torch.cat([kv[:, :Hkv].reshape(-1), kv[:, Hkv:].reshape(-1)]).to(DEV)  # (K and V apart, so that either can be met alone)
+    k, v = pool[:pool.numel() // 2].view(-1, Hkv, D), pool[pool.numel() // 2:].view(-1, Hkv, D)
+    n = B * Hq * D
+    o = {"o over K": k.reshape(-1)[:n], "o over V": v.reshape(-1)[n:2 * n], "o over the table": td.view(-1)[:n // 2].view(torch.float16)}.get(
+        where, torch.zeros(n, dtype=torch.float16, device=DEV))
+    l = {"lse over K": k.reshape(-1)[:2 * B * Hq].view(torch.float32), "lse over the table": td.view(-1)[:B * Hq].view(torch.float32)}.get(
+        where, torch.zeros(B * Hq, device=DEV))
+    o, l = o.view(B, Hq, D), l.view(B, Hq)
+    mo, ml = torch.full((2, B, Hq, D), float("nan"), device=DEV), torch.full((2, B, Hq), float("nan"), device=DEV)
+    if call == "static":
+        ck.flash_decoding_static(qd, k, v, td, rd, ld, max(lens), o, l, 256)
+    else:
+        ck.flash_decoding(mo, ml, qd, k, v, td, rd, ld, max(lens), o, l, 256)
+        assert bool(torch.isnan(mo).all()) == (where == "apart")
+    torch.cuda.synchronize()
+    assert_o_close(o, o_ref, "o", max_abs=O_MAX_ABS + 2.0 ** -10, rel=O_REL + 2.0 ** -11)
+    assert_lse_close(l, l_ref, "lse")
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_one_launch_and_infinite_keys_and_values(lsa, tuning, dtype):
     """Scores of minus infinity weigh nothing (a request of nothing else has the result of an empty one) and infinite values stay
