@@ -295,19 +295,17 @@ __global__ __launch_bounds__(kWaves * 64, (kResident<D, WP, DV>)) void prefill_s
   const float scale = p.scale_log2;
   const int nt = (cnt_wg + TK - 1) / TK;  // the same for every wave of the workgroup
 
-  constexpr int KR = LEAN ? 4 : KS;        // K operands in registers, per block of keys
   constexpr int VR = LEAN ? 4 : NDB;       // V operands
-  u32x4 ka[2][KR];  // K operands of the next 32 keys, the first KR of KS steps
-  auto load_ka1 = [&](int at, int kb, int ks) __attribute__((always_inline)) {
-    u32x4 x = *(const __attribute__((address_space(3))) u32x4*)(kaddr_of(ks) + at + kb * 16 * RB);
-    if (D == 16 && g >= 2) x = u32x4{0u, 0u, 0u, 0u};
-    return x;
-  };
+  u32x4 ka[2][KS];  // K operands of the next 32 keys
   auto load_ka = [&](int at) __attribute__((always_inline)) {
 #pragma unroll
     for (int kb = 0; kb < 2; kb++)
 #pragma unroll
-      for (int ks = 0; ks < KR; ks++) ka[kb][ks] = load_ka1(at, kb, ks);
+      for (int ks = 0; ks < KS; ks++) {
+        u32x4 x = *(const __attribute__((address_space(3))) u32x4*)(kaddr_of(ks) + at + kb * 16 * RB);
+        if (D == 16 && g >= 2) x = u32x4{0u, 0u, 0u, 0u};
+        ka[kb][ks] = x;
+      }
   };
   auto tile = [&](auto stage_tag, int t) __attribute__((always_inline)) {
     constexpr int S = decltype(stage_tag)::value;
@@ -337,14 +335,9 @@ __global__ __launch_bounds__(kWaves * 64, (kResident<D, WP, DV>)) void prefill_s
 #pragma unroll
         for (int ks = 0; ks < KS; ks++)
 #pragma unroll
-          for (int kb = 0; kb < 2; kb++) {
+          for (int kb = 0; kb < 2; kb++)
 #pragma unroll
-            for (int qb = 0; qb < QB; qb++) s[qb][kb] = MfmaS<T>::run(ka[kb][ks % KR], qreg[qb][ks], s[qb][kb]);
-            if (ks + KR < KS) {
-              ka[kb][ks % KR] = load_ka1(S * 2 * TB + 32 * part * RB, kb, ks + KR);
-              __builtin_amdgcn_sched_barrier(0);
-            }
-          }
+            for (int qb = 0; qb < QB; qb++) s[qb][kb] = MfmaS<T>::run(ka[kb][ks], qreg[qb][ks], s[qb][kb]);
         if (k0 + 32 > cnt_first) {  // (wave-uniform: the wave's first row, which sees the fewest keys, does not see the whole step)
 #pragma unroll
           for (int qb = 0; qb < QB; qb++) {
