@@ -529,7 +529,7 @@ __device__ __forceinline__ void stage1_mfma_unit(const Stage1Params& p, char* ld
   const int nh = group - sg * 16 < 16 ? group - sg * 16 : 16;
 
   constexpr int kStep = WS ? kMfmaWaves * kMfmaBatch : kMfmaBatch;  // tokens from one of the wave's batches to its next
-  const int bs = (int)p.block_seq;                    // a multiple of 32 (checked on the host)
+  const int bs = (int)p.block_seq;  // a multiple of 32 where blocks end within the walk (checked on the host); DIRECT walks a request whole, whatever it is
   int64_t fine_nblk = 0, blk_begin = 0;
   int t_begin, t_end, n_batches;
   const int32_t* table;

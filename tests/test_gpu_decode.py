@@ -759,6 +759,38 @@ def test_short_contexts_in_one_launch(lsa, dtype, out, Hq, Hkv):
     assert _direct_case(lsa, 61, len(lens), Hq, Hkv, lens, dtype, {"float32": torch.float32, "other": other}.get(out, dtype), out == "in place")
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("BS", [1, 16, 48, 100, 256, 1000])
+@pytest.mark.parametrize("rows", [None, 1, 3])
+def test_one_launch_attends_the_tokens_that_the_blocks_cover(lsa, tuning, dtype, BS, rows):
+    """Any block size, and fewer rows of partials than the longest request fills: the tokens attended are those of the blocks that have a row, as in
+    two launches (the fused call's own split kept out by the entry point)."""
+    print("case", dtype, BS, rows, flush=True)
+    ck, D, B, Hq, Hkv, lens = lsa.longserve_cuda_kernels, 128, 5, 8, 2, [300, 47, 48, 16, 0]
+    q, kv, table, b_req, b_len = decode_case(87, B, Hq, Hkv, D, lens, 600, dtype)
+    qd, kvd, td, rd, ld = q.to(DEV), kv.to(DEV), table.to(DEV), b_req.to(DEV), b_len.to(DEV)
+    n = min(rows or 300, (300 + BS - 1) // BS)
+    got = []
+    for kernel in (None, "lane"):
+        tuning(decode_stage1=kernel)
+        mo, ml = torch.full((n, B, Hq, D), float("nan"), device=DEV), torch.full((n, B, Hq), float("nan"), device=DEV)
+        o, l = torch.full((B, Hq, D), float("nan"), device=DEV), torch.full((B, Hq), float("nan"), device=DEV)
+        if kernel:  # two launches; the merge reads the rows there are
+            ck.flash_decoding_stage1(mo, ml, qd, kvd[:, :Hkv], kvd[:, Hkv:], td, rd, ld, 300, BS)
+            ck.flash_decoding_stage2(o, l, torch.clamp(ld, max=n * BS), mo, ml, BS)
+        else:
+            ck.flash_decoding(mo, ml, qd, kvd[:, :Hkv], kvd[:, Hkv:], td, rd, ld, 300, o, l, BS)
+        torch.cuda.synchronize()
+        assert bool(torch.isnan(mo).all()) == (kernel is None)
+        got.append((o.cpu(), l.cpu()))
+    (o, l), (o2, l2) = got
+    o_ref, l_ref = orc.decode_full(q, kv[:, :Hkv], kv[:, Hkv:], table, b_req, torch.clamp(b_len, max=n * BS))
+    for x, y, what in ((o, o2, "o against two launches"), (o, o_ref, "o")):
+        assert_o_close(x, y, what)
+    assert_lse_close(l, l2, "lse against two launches")
+    assert_lse_close(l, l_ref, "lse")
+
+
 @pytest.mark.parametrize("Hq,Hkv,B,longest,direct", [
     (4, 4, 1, 320, True), (4, 4, 1, 321, False), (4, 4, 127, 20, True), (4, 4, 128, 20, False), (8, 4, 255, 30, True), (8, 4, 256, 30, False),
     (8, 4, 1, 384, True), (8, 4, 1, 385, False), (8, 4, 64, 385, False), (32, 8, 300, 40, False), (32, 8, 256, 40, True), (32, 8, 31, 385, False),

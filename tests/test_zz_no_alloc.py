@@ -29,6 +29,7 @@ def _both(lsa, seed, B, Hq, Hkv, lens, BS, dtype=torch.float16, spare_rows=0):
     l = torch.full((B, Hq), float("nan"), device=dev)
     ck.flash_decoding_static(q, k, v, table, b_req, b_len, max_len, o, l, BS)
     torch.cuda.synchronize()
+    assert not bool(torch.isnan(mid_l).all())  # (two launches: one that writes the result itself would leave partials out of it)
     return (o, l), (o_ref, l_ref), (q, kv, table, b_req, b_len)
 
 
@@ -44,7 +45,7 @@ def test_static_scratch_decode_matches_caller_scratch_twice(lsa):
     assert_lse_close(l, ll, "static decode LSE")
     # second call, smaller in every dimension (fewer requests, heads, rows, shorter blocks): the array still holds
     # the first call's partials
-    lens2 = [300, 65, 129]
+    lens2 = [700, 65, 129]
     (o, l), (o_ref, l_ref), inp = _both(lsa, 42, len(lens2), 8, 2, lens2, 64, torch.bfloat16)
     assert torch.equal(o, o_ref) and torch.equal(l, l_ref)
     q, kv, table, b_req, b_len = (t.cpu() for t in inp)
