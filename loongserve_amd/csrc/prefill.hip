@@ -1339,9 +1339,9 @@ static Shape choose_shape(const lsattn_prefill_args* a, bool dv, const Tuning& t
   bool half = a->max_q_len <= (ph ? 1024 : 1536) && !a->o_b_start_loc && a->kv_cuts <= 1 && wgs128 >= 3 * kCUs;
   // One prompt, or a chunk against one as long (a ring's step), whose 128-row workgroups are a few more than two per CU: the
   // shapes of one workgroup per CU end in a round of a few of them, this one in a round of lone ones, twice as fast as a pair.  Up to
-  // 11/4 per CU with one head per workgroup (66 launches of 1400 to 6100 rows: 7 % below, the worst 1.00 of them), 9/4 with several
-  // (20: 6 %, 0.97); past that it is even, and so it is a few more than four per CU (0.94 to 1.06), for several requests (0.89
-  // to 1.15) and behind longer contexts (0.90 to 1.12).
+  // 11/4 per CU with one head per workgroup, 9/4 with several: over 1900 launches of 1100 to 6100 rows, prompts and full ring steps, the three epilogues,
+  // 8 % below the other shapes, the worst 1.03 of them (folded into a running partial).  Past that it is even, and so it is a few more than four per CU
+  // (0.94 to 1.10), for several requests (0.89 to 1.15) and behind longer contexts (0.90 to 1.12).
   //   (other shapes | this: two ring steps of 2561 rows 32/32 217 | 198, bf16 226 | 209; 1 x 2266 tokens 32/8 57.5 | 54.6)
   if (a->batch == 1 && a->max_q_len <= 6144 && a->total_kv_rows > 0 && a->total_kv_rows <= a->max_q_len && !a->o_b_start_loc && a->kv_cuts <= 1 &&
       (wgs128 > 2 * kCUs && wgs128 <= (ph ? 9 : 11) * kCUs / 4))

@@ -19,7 +19,7 @@
 //     (o, m, l) update (ring_context_flashattention_nopad.py:171-188), 2 the LSE merge into a running fp32 (O, LSE); O is turned round
 //     in LDS first, so that stores fill whole lines.
 // Measured (fp16, causal, in place, whole calls): D = 64, 8 x 2048 tokens GQA 32/8 172 to 178 us (0.78 PFLOP/s), 16 x 512 43, 32 x 256 34,
-// 16 x 1024 107; D = 128, 16 x 1024 191 us (0.72 PFLOP/s), 16 x 512 65, 1 x 100 9.0 (of which 2.6 are the fills of m and l).
+// 16 x 1024 107; D = 128, 16 x 1024 191 us (0.72 PFLOP/s), 16 x 512 65, 1 x 100 8.7 replayed from a graph (of which 3.6 are the fills of m and l; 4.9 as a partial).
 #include <type_traits>
 
 #include "common.hip.h"
@@ -121,7 +121,8 @@ __device__ __forceinline__ const char* uniform_ptr(const char* ptr) {
 }
 
 // A launch's shape by head size and positions per wave: keys per LDS tile, tiles in LDS (requested one fewer ahead), workgroups per CU.
-// 128-wide heads, 32 positions per wave: three stages of 32 keys (48 KB) and 168 registers, so that three workgroups fit a CU.
+// 128-wide heads, 32 positions per wave: three stages of 32 keys (48 KB) and at most 168 registers (158; 168 where V is bfloat16), so that three
+// workgroups fit a CU.
 template <int D, int WP> constexpr int kTileOf = D == 128 && WP == 32 ? 32 : 64;
 template <int D, int WP> constexpr int kStagesOf = D == 128 && WP == 32 ? 3 : 2;
 template <int D, int WP, bool DV> constexpr int kResident = D == 128 ? (WP == 32 ? 3 : 2) : WP == 32 && D == 64 && !DV ? 3 : 4;
@@ -430,7 +431,7 @@ __global__ __launch_bounds__(kWaves * 64, (kResident<D, WP, DV>)) void prefill_s
   // ---- epilogues (the 128-wide kernel's) ----
   // O leaves through LDS (MODE 0 and 1, 32 positions per wave): written as the lanes hold it, a store touches 16 rows with 32 or 64 bytes
   // each, a request per row to the L2s, and turned round whole lines of a few rows: 16 x 1024 tokens 32/8 199 -> 190 us in
-  // place and 207 -> 201 as fp32, 16 x 512 bf16 72 -> 66 (128-wide heads).  The small launches of 16 positions write directly (1 x 100 9.2 us, turned round 9.6).
+  // place and 207 -> 201 as fp32, 16 x 512 bf16 72 -> 66 (128-wide heads).  The small launches of 16 positions write directly (turned round, 1 x 100 took 0.4 us more).
   constexpr bool TURNED = MODE != 2 && WP == 32;
   constexpr int ES = MODE == 1 ? 2 : 4;                // bytes per element of O
   constexpr int RBO = D * ES < 256 ? D * ES : 256;     // bytes of a row that are turned round at a time
