@@ -270,7 +270,9 @@ typedef struct lsattn_decode_stage2_args {
   int32_t o_dtype;         /* LSATTN_F16 / BF16 / F32  */
   int32_t o_is_apart;      /* read by the fused calls below.  1: neither o nor out_logexpsum shares memory with the pool's rows or the
                               table, so that short contexts may be one launch, which writes the result while others still read;
-                              0: not known (the call's two launches write it behind the last read) */
+                              0: not known (the call's two launches write it behind the last read).  2: as 1, and o lies in memory that
+                              the GPU of the launch has allocated (not the host's, not another GPU's) and nobody else uses during
+                              the call, so that workgroups may count in it with 64-bit atomics before the result is written there */
   float* out_logexpsum;    /* [batch, H] */
   const int32_t* b_seqlen; /* [batch]    */
   const float* mid_o;            /* [num_seq_blocks, batch, H, D] */
@@ -293,7 +295,8 @@ int lsattn_decode_stage2(const lsattn_decode_stage2_args* a, void* stream);
  * out): the call may cut the contexts otherwise than seq_block_size says.  Launches of several requests with enough tokens
  * deal the tokens of all requests (in units of 32) in equal shares to the waves, whatever the lengths of the requests are,
  * and leave one partial per share and request; (o, out_logexpsum) are the same softmax merged from other pieces.  Short contexts are one
- * launch, which writes the result itself and leaves the scratch as it was, if o_is_apart says that it may.  o and out_logexpsum may lie over q,
+ * launch, which writes the result itself and leaves the scratch as it was, if o_is_apart says that it may; with o_is_apart = 2 requests of a few
+ * partials each are one launch too, whose last workgroup on a request merges them.  o and out_logexpsum may lie over q,
  * b_seqlen and b_req_idx (such a call is two launches, unless o is q row for row), and with o_is_apart = 0 over anything but the scratch.
  */
 int lsattn_decode_attention(const lsattn_decode_stage1_args* s1, const lsattn_decode_stage2_args* s2, void* stream);
@@ -586,8 +589,8 @@ const char* lsattn_strerror(int code);
  * lsattn_rotary_kv_write_args untyped, its slots int32 or int64 by dest_index_is_i64 (a reserved word before), lsattn_kv_scatter_i64,
  * the counts of lsattn_pool_update_refs also in pinned host memory and, past LSATTN_POOL_REFS_ORDERED entries, not behind the state; 5 = total_kv_rows and kv_cut_even in lsattn_prefill_args,
  * lsattn_prefill_converts_v; 6 = max_kv_len there (a reserved word before), lsattn_prefill_route,
- * lsattn_prefill_cut_count; 7 = o_is_apart in lsattn_decode_stage2_args (a reserved word before). */
-#define LSATTN_VERSION 7
+ * lsattn_prefill_cut_count; 7 = o_is_apart in lsattn_decode_stage2_args (a reserved word before); 8 = o_is_apart of 2. */
+#define LSATTN_VERSION 8
 int lsattn_version(void);
 
 #ifdef __cplusplus

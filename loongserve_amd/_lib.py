@@ -96,7 +96,7 @@ TUNING_VALUES = {
     "decode_stage1": {None: 0, "lane": 1, "mfma": 2, "split": 3},
     "decode_listed": {None: 0, "off": 1, "on": 2, "shares": 3},
 }
-LSATTN_VERSION = 7  # of include/lsattn.h, which the argument blocks above mirror
+LSATTN_VERSION = 8  # of include/lsattn.h, which the argument blocks above mirror
 
 
 # every symbol include/lsattn.h declares: name -> (restype, argtypes)

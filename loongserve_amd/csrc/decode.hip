@@ -15,6 +15,7 @@
 //     and not for block_seq.
 // Short contexts in the fused call are one launch without partials (decode_direct_kernel).
 #include <atomic>
+#include <chrono>
 #include <type_traits>
 
 #include "common.hip.h"
@@ -39,8 +40,10 @@ struct Stage1Params {
   int32_t tasks;          // hkv * (group / GT) wave tasks
   int32_t tasks_on_x;     // grid = (task groups, chunks, batch) instead of (chunks, task groups, batch)
   int32_t max_shares, share_units;  // equal shares: at most so many, of at least so many units each
-  void* o;                          // (DIRECT) the result [batch, hq, 128] and its log-sum-exps
+  void* o;                          // (DIRECT, JOIN) the result [batch, hq, 128] and its log-sum-exps
   float* out_lse;
+  int32_t o_dtype;                  // (JOIN)
+  uint64_t arrivals;                // (JOIN) where this launch's counts of arrivals start
 };
 
 constexpr int kTok = 8;  // K/V rows in flight per 16-lane group
@@ -50,6 +53,120 @@ template <int N, typename F> __device__ __forceinline__ void static_for(F&& f) {
   if constexpr (N > 0) {
     static_for<N - 1>(f);
     f(std::integral_constant<int, N - 1>{});
+  }
+}
+
+template <typename OT> __device__ __forceinline__ void store4(void* base, int64_t elem, const f32x4& v);
+template <> __device__ __forceinline__ void store4<float>(void* base, int64_t elem, const f32x4& v) {
+  *(f32x4*)((float*)base + elem) = v;
+}
+template <> __device__ __forceinline__ void store4<F16>(void* base, int64_t elem, const f32x4& v) {
+  *(u32x2*)((uint16_t*)base + elem) = u32x2{pack2<F16>(v[0], v[1]), pack2<F16>(v[2], v[3])};
+}
+template <> __device__ __forceinline__ void store4<BF16>(void* base, int64_t elem, const f32x4& v) {
+  *(u32x2*)((uint16_t*)base + elem) = u32x2{pack2<BF16>(v[0], v[1]), pack2<BF16>(v[2], v[3])};
+}
+
+// ------------------------------------------------------------------------------------
+// Stage 1 and the merge in one launch (JOIN): the workgroup, or wave, of a (request, task) that is the last to have stored its partial
+// merges all of them into the result.  Nobody waits for anybody.  What it takes is a count of arrivals in memory that the caller
+// does not clear: the first eight bytes of the task's rows of the result, which the merge overwrites.  They hold anything at first.
+// Whoever finds no count of this launch there puts the launch's start in (one of them succeeds), before it counts itself; the start
+// is 64 bits that no other launch has, so nothing else is taken for a count, and a replay from a graph finds the last replay's result.
+// Partials go through to memory and are read past the L2s (each XCD has its own).
+// ------------------------------------------------------------------------------------
+constexpr int64_t kJoinMaxPartials = 64;
+constexpr int64_t kCUs = 256;  // compute units of the MI355X
+__device__ __forceinline__ void store_through(float* dst, const f32x4& v) {
+  asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" : : "v"(dst), "v"(v) : "memory");  // (the s_nop: as in store_partial_row)
+}
+template <typename V> __device__ __forceinline__ V load_past_l2(const V* src) {
+  return __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t* arrivals_of(const Stage1Params& p, int64_t out_row0) {
+  return (uint64_t*)((char*)p.o + out_row0 * 128 * (p.o_dtype == LSATTN_F32 ? 4 : 2));
+}
+__device__ __forceinline__ void store_result(const Stage1Params& p, int64_t elem, const f32x4& v) {
+  if (p.o_dtype == LSATTN_F32) store4<float>(p.o, elem, v);
+  else if (p.o_dtype == LSATTN_F16) store4<F16>(p.o, elem, v);
+  else store4<BF16>(p.o, elem, v);
+}
+// `seen`: what the word held when the workgroup (wave) started; n: partials, one of them each.
+__device__ __forceinline__ void start_arrivals(uint64_t* word, uint64_t seen, uint64_t start, int n) {
+  if (seen - start > (uint64_t)n) __hip_atomic_compare_exchange_strong(word, &seen, start, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ bool arrive(uint64_t* word, uint64_t start, int n) {  // (behind a wait for the stores of the partial)
+  return __hip_atomic_fetch_add(word, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - start == (uint64_t)(n - 1);
+}
+// The merge of `n` <= kJoinMaxPartials partials of up to 16 query heads, by the four waves of a workgroup.
+// Half a wave reads a row, 16 bytes a lane; a head's rows are dealt to S half waves, which meet in LDS.  Sixteen rows of a
+// half wave are asked for at once, beside the log-sum-exps, of which lane e holds those of partials e and 32 + e.
+__device__ __forceinline__ void join_partials(const Stage1Params& p, char* lds, const int lane, const int wave, const int64_t out_row0, const int nh,
+                                              const int64_t row0, const int n) {
+  const int c = lane & 31, half = wave * 2 + (lane >> 5);
+  const int S = nh == 1 ? 8 : nh == 2 ? 4 : nh <= 4 ? 2 : 1, slice = half & (S - 1);
+  const int rows_here = (n + S - 1) / S;  // (the same for all half waves; positions past the last partial repeat it and weigh nothing)
+  const float* const lse_at = p.mid_lse + row0;
+  const float* const rows_at = p.mid_o + row0 * 128;
+  const uint32_t blk_rows = (uint32_t)p.blk_rows;  // (offsets below 2^31 bytes, checked on the host)
+  for (int h0 = 0; h0 < nh; h0 += 8 / S) {
+    const int h = h0 + half / S;
+    const bool live = h < nh;
+    const uint32_t hh = live ? h : nh - 1;
+    float lse0 = -INFINITY, lse1 = -INFINITY;
+    if (c < n) lse0 = load_past_l2(lse_at + (hh + c * blk_rows));
+    if (32 + c < n) lse1 = load_past_l2(lse_at + (hh + (32 + c) * blk_rows));
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    float M = 0.f, L = 0.f, w0 = 0.f, w1 = 0.f;
+    for (int i = 0; i < rows_here; i += 16) {
+      f32x4 row[16];
+#pragma unroll
+      for (int q = 0; q < 16; q += 4) {
+        if (i + q < rows_here) {
+#pragma unroll
+          for (int u = q; u < q + 4; u++) {
+            const int e = (i + u) * S + slice;
+            const uint32_t at = (hh + (e < n ? e : n - 1) * blk_rows) * 512u + c * 16u;
+            asm volatile("global_load_dwordx4 %0, %1, %2 sc1" : "=v"(row[u]) : "v"(at), "s"(rows_at) : "memory");
+          }
+        }
+      }
+      if (i == 0) {
+        M = fmaxf(lse0, lse1);
+#pragma unroll
+        for (int d = 16; d > 0; d >>= 1) M = fmaxf(M, __shfl_xor(M, d, 64));
+        w0 = exp2_diff(lse0 * kLog2e, M * kLog2e);  // (0 past the last partial)
+        w1 = exp2_diff(lse1 * kLog2e, M * kLog2e);
+        L = w0 + w1;
+#pragma unroll
+        for (int d = 16; d > 0; d >>= 1) L += __shfl_xor(L, d, 64);
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int q = 0; q < 16; q += 4) {
+        if (i + q < rows_here) {
+#pragma unroll
+          for (int u = q; u < q + 4; u++) {
+            asm volatile("" : "+v"(row[u]));
+            const int e = (i + u) * S + slice;
+            const float w = e < n ? __shfl(e < 32 ? w0 : w1, (lane & 32) | (e & 31), 64) : 0.f;
+            if (w != 0.f) acc += row[u] * w;  // (what has no weight may be infinite)
+          }
+        }
+      }
+    }
+    if (S > 1) {
+      f32x4* part = (f32x4*)(lds + 16);
+      part[half * 32 + c] = acc;
+      __syncthreads();
+      if (slice == 0)
+        for (int w = 1; w < S; w++) acc += part[(half + w) * 32 + c];
+    }
+    if (slice == 0 && live) {
+      const float inv = L > 0.f ? 1.f / L : 0.f;
+      store_result(p, (out_row0 + h) * 128 + c * 4, acc * inv);
+      if (c == 0) p.out_lse[out_row0 + h] = L > 0.f ? M + __builtin_amdgcn_logf(L) * kLn2 : -INFINITY;
+    }
   }
 }
 
@@ -78,8 +195,9 @@ template <> struct Dot<BF16> {
 // ONCE: every K/V row is read by one wave only (at most GT query heads per KV head), so the rows are loaded
 // non-temporally; otherwise the waves that take the other query heads of the group read them again and ordinary loads let
 // those find the rows in L2.
-template <typename T, int GT, int NW, bool SPLIT, bool ONCE, int HR>
-__global__ __launch_bounds__(NW * 64) void decode_stage1_kernel(Stage1Params p) {
+template <typename T, int GT, int NW, bool SPLIT, bool ONCE, int HR, bool JOIN = false>
+__global__ __launch_bounds__(NW * 64, JOIN ? (GT == 1 ? 4 : 3) : 1) void decode_stage1_kernel(Stage1Params p) {
+  static_assert(!JOIN || (SPLIT && NW == 4), "join_partials takes the four waves of a workgroup");
   constexpr int GH = GT * HR;  // query heads per task
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -115,7 +233,16 @@ __global__ __launch_bounds__(NW * 64) void decode_stage1_kernel(Stage1Params p) 
   const int64_t blk_begin = (int64_t)chunk * p.blocks_per_wg;
   int64_t blk_end = blk_begin + p.blocks_per_wg;
   if (blk_end > nblk) blk_end = nblk;
+  if (JOIN && nblk <= 0 && blk_begin == 0) {  // a request without tokens
+    for (int i = wave * 64 + lane; i < nh * 32; i += NW * 64) store_result(p, (b * p.hq + qh0) * 128 + i * 4, f32x4{0.f, 0.f, 0.f, 0.f});
+    if (wave == 0 && lane < nh) p.out_lse[b * p.hq + qh0 + lane] = -INFINITY;
+  }
   if (blk_begin >= blk_end) return;
+  // (JOIN) workgroups that store partials of this request and task, of one block each or of several
+  const int arrivals = JOIN ? (int)((nblk + p.blocks_per_wg - 1) / p.blocks_per_wg) : 0;
+  uint64_t* const word = JOIN ? arrivals_of(p, b * p.hq + qh0) : nullptr;
+  uint64_t seen = 0;
+  if (JOIN) seen = load_past_l2(word);  // (by every wave: no branch, and so no wait here)
 
   const int32_t* table = p.req_to_tokens + (int64_t)p.b_req_idx[b] * p.max_seq_len;
   const char* kbase = (const char*)p.k + ((int64_t)kvh * p.k_s1 + sub * 8) * 2;
@@ -313,6 +440,15 @@ __global__ __launch_bounds__(NW * 64) void decode_stage1_kernel(Stage1Params p) 
     auto write_partial = [&](int h, float M, float L, const float (&ov)[8]) {
       if (h >= nh) return;
       const float inv = 1.f / L;
+      if constexpr (JOIN) {
+        const f32x4 lo = f32x4{ov[0] * inv, ov[1] * inv, ov[2] * inv, ov[3] * inv}, hi = f32x4{ov[4] * inv, ov[5] * inv, ov[6] * inv, ov[7] * inv};
+        const float lse = (M + __builtin_amdgcn_logf(L)) * kLn2;
+        const int64_t row = blk * p.blk_rows + b * p.req_rows + qh0 + h;
+        store_through(p.mid_o + row * 128 + sub * 8, lo);
+        store_through(p.mid_o + row * 128 + sub * 8 + 4, hi);
+        if (sub == 0) __hip_atomic_store(p.mid_lse + row, lse, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        return;
+      }
       const int64_t row = blk * p.row_mul * p.blk_rows + b * p.req_rows + qh0 + h;
       f32x4* dst = (f32x4*)(p.mid_o + row * 128 + sub * 8);
       dst[0] = f32x4{ov[0] * inv, ov[1] * inv, ov[2] * inv, ov[3] * inv};
@@ -372,6 +508,16 @@ __global__ __launch_bounds__(NW * 64) void decode_stage1_kernel(Stage1Params p) 
       }
       __syncthreads();  // the next block of this workgroup writes the same LDS
     }
+  }
+  if constexpr (JOIN) {
+    __shared__ __attribute__((aligned(16))) char meet[16 + 8 * 32 * 16];
+    if (wave == 0 && lane == 0) {
+      start_arrivals(word, seen, p.arrivals, arrivals);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (wave 0 has stored the partials)
+      *(uint32_t*)meet = arrive(word, p.arrivals, arrivals);
+    }
+    __syncthreads();
+    if (*(const uint32_t*)meet) join_partials(p, meet, lane, wave, b * p.hq + qh0, nh, b * p.req_rows + qh0, (int)nblk);
   }
 }
 
@@ -496,24 +642,14 @@ __device__ __forceinline__ ShareSegment share_segment(const Stage1Params& p, con
   return s;
 }
 
-template <typename OT> __device__ __forceinline__ void store4(void* base, int64_t elem, const f32x4& v);
-template <> __device__ __forceinline__ void store4<float>(void* base, int64_t elem, const f32x4& v) {
-  *(f32x4*)((float*)base + elem) = v;
-}
-template <> __device__ __forceinline__ void store4<F16>(void* base, int64_t elem, const f32x4& v) {
-  *(u32x2*)((uint16_t*)base + elem) = u32x2{pack2<F16>(v[0], v[1]), pack2<F16>(v[2], v[3])};
-}
-template <> __device__ __forceinline__ void store4<BF16>(void* base, int64_t elem, const f32x4& v) {
-  *(u32x2*)((uint16_t*)base + elem) = u32x2{pack2<BF16>(v[0], v[1]), pack2<BF16>(v[2], v[3])};
-}
-
 // OT (WS): the workgroup takes all tokens of its request and writes the result, in this type; void: partials.
-template <typename T, bool WS, bool LISTED, bool RANGE = false, typename OT = void>
+// JOIN (WS): partials, and the workgroup of a (request, task) that is the last to have written its own merges them into the result.
+template <typename T, bool WS, bool LISTED, bool RANGE = false, typename OT = void, bool JOIN = false>
 __device__ __forceinline__ void stage1_mfma_unit(const Stage1Params& p, char* lds, const int lane, const int wave, const int64_t b,
                                                  const unsigned bid_t, const unsigned bid_c, const unsigned n_cgroups,
                                                  const ShareWalk& walk = ShareWalk{}) {
   constexpr bool DIRECT = !std::is_same<OT, void>::value;
-  static_assert(!DIRECT || WS, "the waves of a workgroup share the request");
+  static_assert(!(DIRECT || JOIN) || (WS && DIRECT != JOIN), "the waves of a workgroup share the request");
   constexpr float kUp = DIRECT && std::is_same<T, F16>::value ? 16384.f : 1.f;  // the weights in O are so many times those in l
   const int n = lane & 15, g = lane >> 4;  // query head (column) or 16-byte chunk of a row / token group or row of four
   // The waves of a workgroup: tw of them on neighbouring tasks (KV heads: their rows of a token lie side by side in memory
@@ -532,6 +668,7 @@ __device__ __forceinline__ void stage1_mfma_unit(const Stage1Params& p, char* ld
   const int bs = (int)p.block_seq;  // a multiple of 32 where blocks end within the walk (checked on the host); DIRECT walks a request whole, whatever it is
   int64_t fine_nblk = 0, blk_begin = 0;
   int t_begin, t_end, n_batches;
+  int join_n = 0;  // (JOIN) partials of the request
   const int32_t* table;
   ShareSegment sl_seg, co_seg;  // (RANGE) where the slot numbers requested next and the batch computed next stand
   if constexpr (RANGE) {
@@ -553,9 +690,14 @@ __device__ __forceinline__ void stage1_mfma_unit(const Stage1Params& p, char* ld
     blk_begin = DIRECT ? 0 : (int64_t)chunk * p.blocks_per_wg;  // (WS: one block per workgroup)
     int64_t blk_end = blk_begin + p.blocks_per_wg;
     if (DIRECT || blk_end > nblk) blk_end = nblk;
-    if constexpr (DIRECT) {
-      if (nblk <= 0) {  // a request without tokens (the same for all waves)
-        for (int i = wave * 64 + lane; i < nh * 32; i += kMfmaWaves * 64) store4<OT>(p.o, (b * p.hq + qh0) * 128 + i * 4, f32x4{0.f, 0.f, 0.f, 0.f});
+    join_n = (int)nblk;
+    if constexpr (DIRECT || JOIN) {
+      if (nblk <= 0 && blk_begin == 0) {  // a request without tokens (the same for all waves)
+        for (int i = wave * 64 + lane; i < nh * 32; i += kMfmaWaves * 64) {
+          const int64_t elem = (b * p.hq + qh0) * 128 + i * 4;
+          if constexpr (DIRECT) store4<OT>(p.o, elem, f32x4{0.f, 0.f, 0.f, 0.f});
+          else store_result(p, elem, f32x4{0.f, 0.f, 0.f, 0.f});
+        }
         if (wave == 0 && lane < nh) p.out_lse[b * p.hq + qh0 + lane] = -INFINITY;
         return;
       }
@@ -811,6 +953,9 @@ __device__ __forceinline__ void stage1_mfma_unit(const Stage1Params& p, char* ld
       load_slots(t_begin + j * kStep, sl);
     }
   };
+  uint64_t* const word = JOIN ? arrivals_of(p, b * p.hq + qh0) : nullptr;
+  uint64_t seen = 0;
+  if (JOIN) seen = load_past_l2(word);
   next_slots(0, s_even);
   next_slots(1, s_odd);
   wait_slots(std::integral_constant<int, 8>{}, s_even);
@@ -837,6 +982,7 @@ __device__ __forceinline__ void stage1_mfma_unit(const Stage1Params& p, char* ld
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (rows requested past the end land before the registers are given back)
+  if (JOIN && wave == 0 && lane == 0) start_arrivals(word, seen, p.arrivals, join_n);
   if constexpr (WS) {
     // The four partials of the block meet in LDS (each wave's own 17.5 KB: its last batch's operands have been consumed);
     // every wave then finishes two of the eight d-blocks.  A wave without a batch of its own brings m = -inf, l = 0.
@@ -874,15 +1020,26 @@ __device__ __forceinline__ void stage1_mfma_unit(const Stage1Params& p, char* ld
 #pragma unroll
         for (int w = 0; w < kMfmaWaves; w++) acc += ((const f32x4*)(lds + w * kMfmaStage))[db * 64 + lane] * mi[w];
         if constexpr (DIRECT) store4<OT>(p.o, row * 128 + 16 * db + 4 * g, acc * inv);
+        else if (JOIN) store_through(p.mid_o + row * 128 + 16 * db + 4 * g, acc * inv);
         else *(f32x4*)(p.mid_o + row * 128 + 16 * db + 4 * g) = acc * inv;
       }
       if (wave == 0) {
         float* lse = DIRECT ? p.out_lse : p.mid_lse;
-        if (g == 0) lse[row] = (M + __builtin_amdgcn_logf(L)) * kLn2;
-        if (!DIRECT)
+        const float value = (M + __builtin_amdgcn_logf(L)) * kLn2;
+        if (JOIN && g == 0) __hip_atomic_store(lse + row, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        else if (g == 0) lse[row] = value;
+        if (!DIRECT && !JOIN)
           for (int r = 1 + g; r < p.row_mul; r += 4)
             if (blk_begin * p.row_mul + r < fine_nblk) p.mid_lse[(blk_begin * p.row_mul + r) * p.blk_rows + b * p.req_rows + qh0 + n] = -INFINITY;
       }
+    }
+    if constexpr (JOIN) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's part of the partial is in memory
+      __syncthreads();                                  // ... and so are the others'
+      uint32_t* const last = (uint32_t*)lds;
+      if (wave == 0 && lane == 0) *last = arrive(word, p.arrivals, join_n);
+      __syncthreads();
+      if (*last) join_partials(p, lds, lane, wave, b * p.hq + qh0, nh, b * p.req_rows + qh0, join_n);
     }
   }
 }
@@ -910,6 +1067,15 @@ __global__ __launch_bounds__(kMfmaWaves * 64, 2) void decode_direct_kernel(Stage
   stage1_mfma_unit<T, true, false, false, OT>(p, lds, lane, wave, blockIdx.y, blockIdx.x, 0, 1);
 }
 
+// The shape whose waves split a block, with the merge in the launch (JOIN).
+template <typename T>
+__global__ __launch_bounds__(kMfmaWaves * 64, 2) void decode_joined_kernel(Stage1Params p) {
+  __shared__ __attribute__((aligned(1024))) char lds[kMfmaWaves * kMfmaStage];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  stage1_mfma_unit<T, true, false, false, void, true>(p, lds, lane, wave, blockIdx.z, blockIdx.y, blockIdx.x, gridDim.x);
+}
+
 // The plain shape over a list of the units that exist.  The grid above has a workgroup for every (chunk group, task group)
 // of the longest request times the batch, and the host does not know the lengths: a batch of one long request and many
 // short ones is mostly workgroups that find nothing to do (one request of 131072 tokens with 255 of 512, 256 tokens per
@@ -927,7 +1093,6 @@ constexpr int64_t kListedFromWorkgroups = 32768;  // launches of the plain grid 
 // list costs an even batch more than that (config 3, 16384 workgroups: 947 -> 962 us) and stays with the larger grids.
 constexpr int64_t kListedFromWorkgroupsCoarse = 8192;
 constexpr int64_t kListedCoarseTokens = 1024;
-constexpr int64_t kCUs = 256;                     // compute units of the MI355X
 // Equal shares from eight requests on wherever the plain shape would run, and for two to seven when the launch is large (waves of the plain
 // shape by the longest request): one request is even by itself and 1-3 % faster on the grids (65536 tokens, GQA 32/8: 50.8 us against
 // 52.6), a few long ones of one length 1 % (4 x 131072), a few ragged ones up to 13 % slower (4 of 1000 to 8000 tokens, MHA 32: 62 us
@@ -1277,8 +1442,41 @@ __global__ __launch_bounds__(256) void decode_merge_shares_kernel(Stage2Params p
   }
 }
 
+// What the fused call allows stage 1 to do beside it: merge its partials itself (JOIN), which leaves `done` set.
+struct JoinPlan {
+  const lsattn_decode_stage2_args* s2;
+  bool done = false;
+};
+// Where a launch's counts of arrivals start: 64 bits that another launch does not have, far from any other's in all likelihood.
+static uint64_t next_arrivals() {
+  static std::atomic<uint64_t> launches{(uint64_t)std::chrono::steady_clock::now().time_since_epoch().count()};
+  uint64_t x = launches.fetch_add(1, std::memory_order_relaxed) * 0x9e3779b97f4a7c15ull;  // (splitmix64, Steele et al. 2014)
+  x = (x ^ (x >> 30)) * 0xbf58476d1ce4e5b9ull;
+  x = (x ^ (x >> 27)) * 0x94d049bb133111ebull;
+  return x ^ (x >> 31);
+}
+// Which launches merge their own partials.  `partials` per request at most, of `heads` query heads per task; workgroups of the grid.  The last
+// workgroup reads the partials alone, at some 50 GB/s: up to max_rows of them (one memory latency, 2 to 2.5 us behind the kernel's
+// work, where a second launch takes 3.5 and more), half of that where two workgroups per CU are busy with rows of their own.
+// Measured over 108 launches (two launches | one, us a call, eager; and replayed from a graph), GQA 32/8:
+//   1 x 2048 11.9 | 10.9 (9.5 | 9.3)   4 x 1500 12.7 | 10.6 (11.2 | 10.2)   6 of 87..700 12.5 | 11.2 (10.7 | 10.0)   16 x 900 18.4 | 16.7 (17.9 | 17.2)
+//   1 x 8192, 32 partials, 13.4 | 12.3 (13.1 | 12.5)   1 x 16384, 64, 20.3 | 20.3 (20.3 | 21.0, not taken)   2 x 8000 19.0 | 18.6 (18.7 | 19.0, not taken)
+// eight heads per task: 1 x 2048 8/1 10.5 | 9.6   1 x 3000 8/1, 96 rows, 11.1 | 10.8 (10.4 | 10.6, not taken)   1 x 8000 8/1, 256, 11.4 | 13.0 (not taken)
+// the lane kernel: 1 x 2048 32/32 10.6 | 9.5   10 x 400 24/8 14.0 | 13.1   4 x 5000 24/8, 60 rows, 640 workgroups, 24.8 | 25.4 (not taken)
+// sixteen heads: 1 x 1500 64/4, 96 rows in two turns, 12.0 | 12.8 (not taken).
+static bool join_takes(JoinPlan* join, Stage1Params& p, int64_t partials, int64_t heads, int64_t max_rows, int64_t workgroups) {
+  if (workgroups >= 2 * kCUs) max_rows /= 2;
+  if (!join || p.row_mul != 1 || partials > kJoinMaxPartials || heads > 8 || partials * heads > max_rows || (partials * p.blk_rows + heads) * 512 > 0x7fffffff) return false;
+  join->done = true;
+  p.o = join->s2->o;
+  p.out_lse = join->s2->out_logexpsum;
+  p.o_dtype = join->s2->o_dtype;
+  p.arrivals = next_arrivals();
+  return true;
+}
+
 template <typename T, int GT, int HR>
-static int launch_stage1(const lsattn_decode_stage1_args* a, hipStream_t st) {
+static int launch_stage1(const lsattn_decode_stage1_args* a, hipStream_t st, JoinPlan* join) {
   constexpr int NW = 4;  // waves (tasks) per workgroup; 8 measured no faster
   Stage1Params p;
   p.mid_o = a->mid_o;
@@ -1329,6 +1527,12 @@ static int launch_stage1(const lsattn_decode_stage1_args* a, hipStream_t st) {
     p.tasks_on_x = chunks <= 65535;
     dim3 grid = p.tasks_on_x ? dim3((unsigned)p.tasks, (unsigned)chunks, (unsigned)a->batch)
                              : dim3((unsigned)chunks, (unsigned)p.tasks, (unsigned)a->batch);
+    if constexpr (HR == 1) {
+      if (once && join_takes(join, p, nblk, group, 64, chunks * p.tasks * a->batch)) {
+        LSATTN_LAUNCH_KERNEL((decode_stage1_kernel<T, GT, NW, true, true, 1, true>), grid, dim3(NW * 64), 0, st, p);
+        return check_launch();
+      }
+    }
     if (once) LSATTN_LAUNCH_KERNEL((decode_stage1_kernel<T, GT, NW, true, true, HR>), grid, dim3(NW * 64), 0, st, p);
     else LSATTN_LAUNCH_KERNEL((decode_stage1_kernel<T, GT, NW, true, false, HR>), grid, dim3(NW * 64), 0, st, p);
     return check_launch();
@@ -1351,7 +1555,8 @@ struct SharesPlan {
 };
 
 // `shares`: deal the blocks in equal shares (decode_stage1_mfma_range_kernel) or launch nothing (*taken stays false).
-template <typename T> static int launch_stage1_mfma(const lsattn_decode_stage1_args* a, hipStream_t st, bool* taken, SharesPlan* shares = nullptr) {
+template <typename T> static int launch_stage1_mfma(const lsattn_decode_stage1_args* a, hipStream_t st, bool* taken, SharesPlan* shares = nullptr,
+                                                    JoinPlan* join = nullptr) {
   *taken = false;
   const int group = (int)(a->num_q_heads / a->num_kv_heads);
   Stage1Params p;
@@ -1442,6 +1647,10 @@ template <typename T> static int launch_stage1_mfma(const lsattn_decode_stage1_a
     *taken = true;
     p.blocks_per_wg = 1;
     p.tasks_on_x = 1;
+    if (join_takes(join, p, nblk, group, group <= 4 ? 128 : 64, nblk * p.tasks * a->batch)) {
+      LSATTN_LAUNCH_KERNEL((decode_joined_kernel<T>), dim3((unsigned)nblk, (unsigned)p.tasks, (unsigned)a->batch), dim3(kMfmaWaves * 64), 0, st, p);
+      return check_launch();
+    }
     LSATTN_LAUNCH_KERNEL((decode_stage1_mfma_kernel<T, true>), dim3((unsigned)nblk, (unsigned)p.tasks, (unsigned)a->batch), dim3(kMfmaWaves * 64),
                        0, st, p);
     return check_launch();
@@ -1470,6 +1679,20 @@ template <typename T> static int launch_stage1_mfma(const lsattn_decode_stage1_a
   return check_launch();
 }
 
+// The result is written while other workgroups still read.  Whether it lies over the pool's rows or the table only the caller knows (their
+// extents are not in the arguments).  Not where it lies over the queries, unless row by row and each workgroup reads its own first
+// (`rows_may_match`), or over the lengths and rows of the requests.
+static bool result_is_apart(const lsattn_decode_stage1_args* a, const lsattn_decode_stage2_args* s2, bool rows_may_match) {
+  if (s2->o_is_apart != 1 && s2->o_is_apart != 2) return false;
+  const int64_t pairs = a->batch * a->num_q_heads;
+  auto apart = [](const void* x, int64_t nx, const void* y, int64_t ny) { return (const char*)x + nx <= (const char*)y || (const char*)y + ny <= (const char*)x; };
+  const int64_t o_bytes = pairs * 128 * (s2->o_dtype == LSATTN_F32 ? 4 : 2), q_bytes = pairs * 256;
+  const bool rows_match = rows_may_match && s2->o == a->q && o_bytes == q_bytes;
+  return (rows_match || apart(s2->o, o_bytes, a->q, q_bytes)) && apart(s2->out_logexpsum, pairs * 4, a->q, q_bytes) &&
+         apart(s2->o, o_bytes, a->b_seqlen, a->batch * 4) && apart(s2->o, o_bytes, a->b_req_idx, a->batch * 4) &&
+         apart(s2->out_logexpsum, pairs * 4, a->b_seqlen, a->batch * 4) && apart(s2->out_logexpsum, pairs * 4, a->b_req_idx, a->batch * 4);
+}
+
 // Which launches of the fused call are one (decode_direct_kernel).  A workgroup walks its request in turns of 128 tokens, some 0.8 us each;
 // two launches take some 4 us more than one for their starts and ends, and the longer the request the more workgroups share it.  The launch
 // lasts as long as its longest request, whatever the others are, so the rule takes what is no slower with one long request among short
@@ -1491,17 +1714,7 @@ static bool decode_is_direct(const lsattn_decode_stage1_args* a, const lsattn_de
       : group < 4 ? longest > 384 || wgs >= 4 * kCUs
                   : longest > (wgs < kCUs ? 384 : 640) || (group < 8 && wgs > 8 * kCUs))
     return false;
-  // The result is written while other workgroups still read.  Whether it lies over the pool's rows or the table only the caller knows (their
-  // extents are not in the arguments).  Not where it lies over the queries, unless row by row (each workgroup reads its own first),
-  // or over the lengths and rows of the requests.
-  if (s2->o_is_apart != 1) return false;
-  const int64_t pairs = a->batch * a->num_q_heads;
-  auto apart = [](const void* x, int64_t nx, const void* y, int64_t ny) { return (const char*)x + nx <= (const char*)y || (const char*)y + ny <= (const char*)x; };
-  const int64_t o_bytes = pairs * 128 * (s2->o_dtype == LSATTN_F32 ? 4 : 2), q_bytes = pairs * 256;
-  const bool rows_match = s2->o == a->q && o_bytes == q_bytes;
-  return (rows_match || apart(s2->o, o_bytes, a->q, q_bytes)) && apart(s2->out_logexpsum, pairs * 4, a->q, q_bytes) &&
-         apart(s2->o, o_bytes, a->b_seqlen, a->batch * 4) && apart(s2->o, o_bytes, a->b_req_idx, a->batch * 4) &&
-         apart(s2->out_logexpsum, pairs * 4, a->b_seqlen, a->batch * 4) && apart(s2->out_logexpsum, pairs * 4, a->b_req_idx, a->batch * 4);
+  return result_is_apart(a, s2, true);
 }
 template <typename T> static int launch_direct(const lsattn_decode_stage1_args* a, const lsattn_decode_stage2_args* s2, hipStream_t st) {
   Stage1Params p = {};
@@ -1538,7 +1751,7 @@ template <typename T> static int launch_direct(const lsattn_decode_stage1_args* 
   return check_launch();
 }
 
-template <typename T> static int dispatch_stage1(const lsattn_decode_stage1_args* a, hipStream_t st, SharesPlan* shares = nullptr) {
+template <typename T> static int dispatch_stage1(const lsattn_decode_stage1_args* a, hipStream_t st, SharesPlan* shares = nullptr, JoinPlan* join = nullptr) {
   const int group = (int)(a->num_q_heads / a->num_kv_heads);
   if (shares) {  // (in equal shares or not at all: shares->max_shares stays 0 then)
     bool taken;
@@ -1546,16 +1759,16 @@ template <typename T> static int dispatch_stage1(const lsattn_decode_stage1_args
   }
   {
     bool taken;
-    const int rc = launch_stage1_mfma<T>(a, st, &taken);
+    const int rc = launch_stage1_mfma<T>(a, st, &taken, nullptr, join);
     if (taken) return rc;
   }
   // groups of 3 and 4 take four query heads per task (3: one spare): fetching a K/V row once per group matters more than
   // the spare accumulators cost
   // groups of more than four: eight query heads per task in two rounds of four over the same rows
-  if (group >= 5) return launch_stage1<T, 4, 2>(a, st);
-  if (group >= 3) return launch_stage1<T, 4, 1>(a, st);
-  if (group == 2) return launch_stage1<T, 2, 1>(a, st);
-  return launch_stage1<T, 1, 1>(a, st);
+  if (group >= 5) return launch_stage1<T, 4, 2>(a, st, join);
+  if (group >= 3) return launch_stage1<T, 4, 1>(a, st, join);
+  if (group == 2) return launch_stage1<T, 2, 1>(a, st, join);
+  return launch_stage1<T, 1, 1>(a, st, join);
 }
 
 }  // namespace lsattn
@@ -1580,13 +1793,13 @@ static int validate_stage1(const lsattn_decode_stage1_args* a) {
 }
 
 // `shares` (the fused call): launch stage 1 in equal shares if the launch is one for them (max_shares > 0 then) or nothing.
-static int decode_stage1(const lsattn_decode_stage1_args* a, void* stream, SharesPlan* shares) {
+static int decode_stage1(const lsattn_decode_stage1_args* a, void* stream, SharesPlan* shares, JoinPlan* join = nullptr) {
   const int rc = validate_stage1(a);
   if (rc != LSATTN_OK) return rc;
   if (a->batch == 0 || a->num_blocks == 0 || a->max_len_in_batch == 0) return LSATTN_OK;
   hipStream_t st = (hipStream_t)stream;
-  if (a->dtype == LSATTN_F16) return dispatch_stage1<F16>(a, st, shares);
-  if (a->dtype == LSATTN_BF16) return dispatch_stage1<BF16>(a, st, shares);
+  if (a->dtype == LSATTN_F16) return dispatch_stage1<F16>(a, st, shares, join);
+  if (a->dtype == LSATTN_BF16) return dispatch_stage1<BF16>(a, st, shares, join);
   return LSATTN_ERR_UNSUPPORTED;
 }
 
@@ -1678,8 +1891,13 @@ extern "C" int lsattn_decode_attention(const lsattn_decode_stage1_args* s1, cons
       return decode_stage2(&a2, 0, stream, &shares);
     }
   }
-  const int rc = lsattn_decode_stage1(s1, stream);
-  if (rc != LSATTN_OK) return rc;
+  // (the merge in stage 1's launch counts in o, which only memory of this GPU's own is sure to take; launches of forced shapes are two)
+  JoinPlan join{s2};
+  const Tuning tn = tuning();
+  const bool may_join = s2->o_is_apart == 2 && tn.decode_stage1 == 0 && tn.decode_listed == 0 && validate_stage2(s2) == LSATTN_OK && (s2->o_dtype == LSATTN_F32 || s2->o_dtype == LSATTN_F16 || s2->o_dtype == LSATTN_BF16) &&
+                        result_is_apart(s1, s2, false);
+  const int rc = decode_stage1(s1, stream, nullptr, may_join ? &join : nullptr);
+  if (rc != LSATTN_OK || join.done) return rc;
   // the merge's shape from the rows the longest request can reach, not from the rows the buffer happens to have: the
   // same call gives the same bits whatever the buffer's height (lsattn_decode_attention_static passes its own)
   int64_t live = s1->seq_block_size > 0 ? (s1->max_len_in_batch + s1->seq_block_size - 1) / s1->seq_block_size : 0;

@@ -141,6 +141,13 @@ def _apart(x: torch.Tensor, y: torch.Tensor) -> bool:
     return end(x) <= y.data_ptr() or end(y) <= x.data_ptr()
 
 
+def _o_is_apart(o, out_logexpsum, q, k, v, req_to_tokens) -> int:
+    """o_is_apart of lsattn_decode_stage2_args."""
+    if not all(_apart(x, y) for x in (o, out_logexpsum) for y in (k, v, req_to_tokens)):
+        return 0
+    return 2 if o.is_cuda and o.device == q.device else 1
+
+
 def flash_decoding(mid_o, mid_o_logexpsum, q, k, v, req_to_tokens, b_req_idx, b_seqlen, max_len_in_batch: int,
                    o, out_logexpsum, block_seq: int) -> None:
     """Stage 1 and stage 2 with the same block size from one library call (what FDPY:12-27 does with two): the checks of
@@ -152,7 +159,7 @@ def flash_decoding(mid_o, mid_o_logexpsum, q, k, v, req_to_tokens, b_req_idx, b_
     a1 = _stage1_args(mid_o, mid_o_logexpsum, q, k, v, req_to_tokens, b_req_idx, b_seqlen, max_len_in_batch, block_seq)
     a2 = _stage2_args(o, out_logexpsum, b_seqlen, mid_o, mid_o_logexpsum, block_seq)
     a1.partials_by_request = a2.partials_by_request = 1 if FUSED_PARTIALS_BY_REQUEST else 0
-    a2.o_is_apart = all(_apart(x, y) for x in (o, out_logexpsum) for y in (k, v, req_to_tokens))
+    a2.o_is_apart = _o_is_apart(o, out_logexpsum, q, k, v, req_to_tokens)
     _lib.check(_lib.load().lsattn_decode_attention(C.byref(a1), C.byref(a2), _stream()), "lsattn_decode_attention")
 
 
@@ -172,7 +179,7 @@ def flash_decoding_static(q, k, v, req_to_tokens, b_req_idx, b_seqlen, max_len_i
     a1 = _stage1_args(mid_o, mid_lse, q, k, v, req_to_tokens, b_req_idx, b_seqlen, max_len_in_batch, block_seq,
                       partials_in_library=True)
     a2 = _stage2_args(o, out_logexpsum, b_seqlen, mid_o, mid_lse, block_seq, partials_in_library=True)
-    a2.o_is_apart = all(_apart(x, y) for x in (o, out_logexpsum) for y in (k, v, req_to_tokens))
+    a2.o_is_apart = _o_is_apart(o, out_logexpsum, q, k, v, req_to_tokens)
     _lib.check(_lib.load().lsattn_decode_attention_static(C.byref(a1), C.byref(a2), _stream()),
                "lsattn_decode_attention_static")
 

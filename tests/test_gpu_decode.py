@@ -791,6 +791,70 @@ def test_one_launch_attends_the_tokens_that_the_blocks_cover(lsa, tuning, dtype,
     assert_lse_close(l, l_ref, "lse")
 
 
+def _kernel_nodes(graph):
+    """How many nodes a captured graph has."""
+    import ctypes
+    n = ctypes.c_size_t()
+    hip = ctypes.CDLL("libamdhip64.so")
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(int(graph.raw_cuda_graph())), None, ctypes.byref(n)) == 0
+    return n.value
+
+
+# per request at most 3 partials; the most that one of four, eight, five heads, of one, two and three in the lane kernel take (128 and 64 rows); one more
+@pytest.mark.parametrize("Hq,Hkv,lens,joined", [
+    (32, 8, [0, 1, 255, 256, 257, 0, 511, 513, 700, 768], True), (8, 2, [8192], True), (8, 2, [8193], False), (8, 1, [2048, 300, 5], True), (8, 1, [2049], False),
+    (5, 1, [3072, 1, 0], True), (4, 4, [16384], True), (4, 4, [16385], False), (8, 4, [8192, 256, 257], True), (8, 4, [8193], False),
+    (9, 3, [5376, 31, 129], True), (3, 1, [5377], False), (9, 1, [600], False), (17, 1, [600], False), (16, 8, [385, 0, 2000], True),
+    (32, 8, [2048] * 8, True), (32, 8, [8192, 700], False)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("out", ["float32", "same", "other"])
+def test_partials_merged_in_the_launch_that_wrote_them(lsa, Hq, Hkv, lens, joined, dtype, out):
+    """The last workgroup on a request merges its partials, whatever the result's memory held before (where the workgroups count each
+    other); replayed from a graph among other calls over the same memory it counts anew every time."""
+    print("case", Hq, Hkv, lens[:3], dtype, out, flush=True)
+    B, D = len(lens), 128
+    q, kv, table, b_req, b_len = decode_case(93, B, Hq, Hkv, D, lens, sum(lens) + 100, dtype)
+    o_ref, l_ref = orc.decode_full(q, kv[:, :Hkv], kv[:, Hkv:], table, b_req, b_len)
+    qd, kvd, td, rd, ld, rows = q.to(DEV), kv.to(DEV), table.to(DEV), b_req.to(DEV), b_len.to(DEV), (max(lens) + 255) // 256
+    mo, ml = torch.full((rows, B, Hq, D), float("nan"), device=DEV), torch.full((rows, B, Hq), float("nan"), device=DEV)
+    other = torch.bfloat16 if dtype == torch.float16 else torch.float16
+    o = torch.empty((B, Hq, D), dtype={"float32": torch.float32, "other": other}.get(out, dtype), device=DEV)
+    l = torch.empty((B, Hq), device=DEV)
+    words = o.view(torch.int64)
+
+    def call():
+        lsa.longserve_token_decode_attention_flash_decoding(qd, td, rd, ld, mo, ml, B, max(lens), Hq, D, kvd[:, :Hkv], kvd[:, Hkv:], 256, o, l)
+
+    # (a result in 16 bits: half a last place of values below 4 on top)
+    eps = {torch.float32: 0.0, torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}[o.dtype]
+    first = None
+    for held in (0, -1, 1, 2, 0x7fffffffffffffff, -2 ** 63, None):  # (None: the last call's result)
+        if held is not None:
+            words.fill_(held)
+        call()
+        torch.cuda.synchronize()
+        if first is None:
+            first = (o.clone(), l.clone())
+            assert_o_close(o, o_ref, "o", max_abs=O_MAX_ABS + eps, rel=O_REL + eps / 2)
+            assert_lse_close(l, l_ref, "lse")
+        assert torch.equal(o, first[0]) and torch.equal(l, first[1]), held
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        call()
+    assert (_kernel_nodes(graph) == 1) == joined
+    q2 = torch.roll(qd, 1, 1)
+    for turn in range(4):
+        o.view(torch.uint8).random_(0, 256)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(o, first[0]) and torch.equal(l, first[1]), turn
+        if turn == 1:  # other eager work over the same result and partials
+            keep = qd.clone()
+            qd.copy_(q2)
+            call()
+            qd.copy_(keep)
+
+
 @pytest.mark.parametrize("Hq,Hkv,B,longest,direct", [
     (4, 4, 1, 320, True), (4, 4, 1, 321, False), (4, 4, 127, 20, True), (4, 4, 128, 20, False), (8, 4, 255, 30, True), (8, 4, 256, 30, False),
     (8, 4, 1, 384, True), (8, 4, 1, 385, False), (8, 4, 64, 385, False), (32, 8, 300, 40, False), (32, 8, 256, 40, True), (32, 8, 31, 385, False),

@@ -409,6 +409,19 @@ def test_decode_kernel_of_one_launch_touches_no_register_of_a_load_in_flight():
 
 
 @pytest.mark.skipif(shutil.which(HIPCC) is None, reason="hipcc not available")
+def test_kernels_that_merge_their_own_partials_touch_no_register_of_a_load_in_flight():
+    asm = _decode_asm()
+    res = loads_in_flight_violations(asm, "decode_joined_")
+    assert len(res) == 2, list(res)                       # fp16 and bf16
+    # the lane kernel with one, two and four heads per task, whose only such loads are the merge's sixteen rows
+    lane = {n: r for n, r in loads_in_flight_violations(asm, "decode_stage1_kernel").items() if r[0]}
+    assert len(lane) == 6, list(lane)
+    for name, (n, bad) in {**res, **lane}.items():
+        assert n == (16 if name in lane else 4 * 8 + 3 * 16 + 16), (name, n)
+        assert not bad, name + "\n" + "\n".join(bad[:20])
+
+
+@pytest.mark.skipif(shutil.which(HIPCC) is None, reason="hipcc not available")
 def test_inline_assembly_stores_of_a_partial_keep_their_data_registers_for_two_cycles():
     """The matrix-pipe decode kernel stores a partial's row from inline assembly (the compiler has no plain store with the
     system-scope bits).  A vector instruction may not overwrite the data registers of a store of more than 64 bits in
