@@ -262,7 +262,7 @@ int lsattn_decode_stage1(const lsattn_decode_stage1_args* a, void* stream);
 /*
  * Flash-decoding stage 2: LSE-weighted merge over the block axis.  Replaces
  * LongServe::flash_decoding_stage2 (S2H:7-19, S2CU:116-132) behind ENTRY:166-221.
- * n_b = b_seqlen[b] <= 0 ? 0 : ceil(b_seqlen[b]/block_seq) rows are merged (S2CU:30);
+ * n_b = lead_rows + (b_seqlen[b] <= 0 ? 0 : ceil(b_seqlen[b]/block_seq)) rows are merged (S2CU:30, where lead_rows is 0);
  * n_b = 0 writes o = 0, out_logexpsum = -inf.
  */
 typedef struct lsattn_decode_stage2_args {
@@ -283,6 +283,8 @@ typedef struct lsattn_decode_stage2_args {
   int64_t head_dim;        /* 32, 64 or 128 */
   int64_t block_seq;
   int64_t partials_by_request; /* as in lsattn_decode_stage1_args: 1 reads mid_o as [batch, num_seq_blocks, H, D] */
+  int64_t lead_rows;       /* rows in front of a request's blocks that are merged with them whatever its length is (its peers' partials, on the
+                              instance that merges them); 0 for the fused calls below */
 } lsattn_decode_stage2_args;
 int lsattn_decode_stage2(const lsattn_decode_stage2_args* a, void* stream);
 
@@ -589,8 +591,9 @@ const char* lsattn_strerror(int code);
  * lsattn_rotary_kv_write_args untyped, its slots int32 or int64 by dest_index_is_i64 (a reserved word before), lsattn_kv_scatter_i64,
  * the counts of lsattn_pool_update_refs also in pinned host memory and, past LSATTN_POOL_REFS_ORDERED entries, not behind the state; 5 = total_kv_rows and kv_cut_even in lsattn_prefill_args,
  * lsattn_prefill_converts_v; 6 = max_kv_len there (a reserved word before), lsattn_prefill_route,
- * lsattn_prefill_cut_count; 7 = o_is_apart in lsattn_decode_stage2_args (a reserved word before); 8 = o_is_apart of 2. */
-#define LSATTN_VERSION 8
+ * lsattn_prefill_cut_count; 7 = o_is_apart in lsattn_decode_stage2_args (a reserved word before); 8 = o_is_apart of 2;
+ * 9 = lead_rows in lsattn_decode_stage2_args. */
+#define LSATTN_VERSION 9
 int lsattn_version(void);
 
 #ifdef __cplusplus

@@ -79,7 +79,7 @@ class DecodeStage2Args(C.Structure):
         ("o", _vp), ("o_dtype", _i32), ("o_is_apart", _i32), ("out_logexpsum", _vp), ("b_seqlen", _vp),
         ("mid_o", _vp), ("mid_o_logexpsum", _vp),
         ("batch", _i64), ("num_heads", _i64), ("num_seq_blocks", _i64), ("head_dim", _i64), ("block_seq", _i64),
-        ("partials_by_request", _i64),
+        ("partials_by_request", _i64), ("lead_rows", _i64),
     ]
 
 
@@ -96,7 +96,7 @@ TUNING_VALUES = {
     "decode_stage1": {None: 0, "lane": 1, "mfma": 2, "split": 3},
     "decode_listed": {None: 0, "off": 1, "on": 2, "shares": 3},
 }
-LSATTN_VERSION = 8  # of include/lsattn.h, which the argument blocks above mirror
+LSATTN_VERSION = 9  # of include/lsattn.h, which the argument blocks above mirror
 
 
 # every symbol include/lsattn.h declares: name -> (restype, argtypes)

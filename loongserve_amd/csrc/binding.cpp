@@ -444,16 +444,17 @@ PyObject* decode_stage1(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
-// (o, out_lse, b_len, mid_o, mid_lse, block) -> True or None
+// (o, out_lse, b_len, mid_o, mid_lse, block, lead_rows) -> True or None
 PyObject* decode_stage2(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
-  NEED_ARGS(6);
+  NEED_ARGS(7);
   Args in(args);
   const at::Tensor &o = in.gpu(3), &lse = in.gpu(2), &b_len = in.gpu(1), &mid_o = in.gpu(4), &mid_lse = in.gpu(3);
-  const int64_t block = in.integer();
-  OR_NONE(in.ok);
+  const int64_t block = in.integer(), lead_rows = in.integer();
+  OR_NONE(in.ok && lead_rows >= 0);
   Decode d;
   OR_NONE(d.stage2(o, lse, b_len, mid_o, mid_lse, block));
+  d.s2.lead_rows = lead_rows;
   OR_NONE(o.size(0) == mid_o.size(1) && o.size(1) == mid_o.size(2) && o.size(2) == mid_o.size(3));
   if (const int rc = call(lib.decode_stage2, &d.s2, stream())) return failed(rc, "lsattn_decode_stage2");
   Py_RETURN_TRUE;

@@ -1270,6 +1270,7 @@ struct Stage2Params {
   int64_t blk_rows, req_rows;  // rows of mid_o between consecutive blocks / requests
   int64_t grid_blocks;         // (SHARES) stage 1's bound on a request's units, from the longest request
   int64_t max_shares, share_units;  // (SHARES) as in Stage1Params
+  int64_t lead_rows;                // rows in front of every request's blocks
 };
 
 template <typename OT, int D, int NT>
@@ -1279,7 +1280,7 @@ __global__ __launch_bounds__(NT) void decode_stage2_kernel(Stage2Params p) {
   const int64_t b = blockIdx.x / (uint32_t)p.heads, h = blockIdx.x % (uint32_t)p.heads;
   const int slice = threadIdx.x / LPR, c = threadIdx.x % LPR;
   const int len = p.b_seqlen[b];
-  int64_t n = len <= 0 ? 0 : ((int64_t)len + p.block_seq - 1) / p.block_seq;
+  int64_t n = p.lead_rows + (len <= 0 ? 0 : ((int64_t)len + p.block_seq - 1) / p.block_seq);
   if (n > p.num_seq_blocks) n = p.num_seq_blocks;
   const int64_t row_stride = p.blk_rows;
   const int64_t row0 = b * p.req_rows + h;
@@ -1832,7 +1833,7 @@ template <typename OT> static int dispatch_stage2(const Stage2Params& p, int64_t
 
 static int validate_stage2(const lsattn_decode_stage2_args* a) {
   if (!a || !a->o || !a->out_logexpsum || !a->b_seqlen || !a->mid_o || !a->mid_o_logexpsum) return LSATTN_ERR_INVALID_ARG;
-  if (a->batch < 0 || a->num_heads <= 0 || a->num_seq_blocks < 0 || a->block_seq < 1) return LSATTN_ERR_INVALID_ARG;
+  if (a->batch < 0 || a->num_heads <= 0 || a->num_seq_blocks < 0 || a->block_seq < 1 || a->lead_rows < 0) return LSATTN_ERR_INVALID_ARG;
   if (((uintptr_t)a->o | (uintptr_t)a->mid_o) & 15) return LSATTN_ERR_INVALID_ARG;
   if (a->head_dim != 32 && a->head_dim != 64 && a->head_dim != 128) return LSATTN_ERR_UNSUPPORTED;
   return a->batch * a->num_heads > 0x7fffffff ? LSATTN_ERR_INVALID_ARG : LSATTN_OK;
@@ -1846,7 +1847,7 @@ static int decode_stage2(const lsattn_decode_stage2_args* a, int64_t live_blocks
                  a->batch, a->num_heads, a->num_seq_blocks, a->block_seq,
                  a->partials_by_request ? a->num_heads : a->batch * a->num_heads,
                  a->partials_by_request ? a->num_seq_blocks * a->num_heads : a->num_heads, shares ? shares->units : 0,
-                 shares ? shares->max_shares : 0, kShareUnits};
+                 shares ? shares->max_shares : 0, kShareUnits, a->lead_rows};
   dim3 grid((unsigned)(a->batch * a->num_heads));
   hipStream_t st = (hipStream_t)stream;
   switch (a->o_dtype) {
@@ -1866,7 +1867,7 @@ extern "C" int lsattn_decode_attention(const lsattn_decode_stage1_args* s1, cons
   // the two stages must describe the same partials
   if (s1->mid_o != s2->mid_o || s1->mid_o_logexpsum != s2->mid_o_logexpsum || s1->b_seqlen != s2->b_seqlen ||
       s1->batch != s2->batch || s1->num_q_heads != s2->num_heads || s1->num_blocks != s2->num_seq_blocks ||
-      s1->head_dim != s2->head_dim || s1->seq_block_size != s2->block_seq || !s1->partials_by_request != !s2->partials_by_request)
+      s1->head_dim != s2->head_dim || s1->seq_block_size != s2->block_seq || s2->lead_rows != 0 || !s1->partials_by_request != !s2->partials_by_request)
     return LSATTN_ERR_INVALID_ARG;
   // (anything that either stage would refuse goes the way of two launches, which refuses it)
   if (validate_stage1(s1) == LSATTN_OK && validate_stage2(s2) == LSATTN_OK && s1->batch > 0 && s1->num_blocks > 0 && s1->max_len_in_batch > 0 &&
@@ -1939,7 +1940,7 @@ extern "C" int lsattn_decode_attention_static(const lsattn_decode_stage1_args* s
   // the partials are the library's here: the caller names none
   if (s1->mid_o || s1->mid_o_logexpsum || s2->mid_o || s2->mid_o_logexpsum) return LSATTN_ERR_INVALID_ARG;
   if (s1->b_seqlen != s2->b_seqlen || s1->batch != s2->batch || s1->num_q_heads != s2->num_heads ||
-      s1->num_blocks != s2->num_seq_blocks || s1->head_dim != s2->head_dim || s1->seq_block_size != s2->block_seq)
+      s1->num_blocks != s2->num_seq_blocks || s1->head_dim != s2->head_dim || s1->seq_block_size != s2->block_seq || s2->lead_rows != 0)
     return LSATTN_ERR_INVALID_ARG;
   if (s1->batch < 0 || s1->num_q_heads <= 0 || s1->num_blocks < 0 || s1->seq_block_size < 1 || s1->max_len_in_batch < 0 ||
       s1->merge_blocks > 1)

@@ -119,11 +119,13 @@ def _stage2_args(o, out_logexpsum, b_seqlen, mid_o, mid_o_logexpsum, block_seq: 
     return a
 
 
-def flash_decoding_stage2(o, out_logexpsum, b_seqlen, mid_o, mid_o_logexpsum, block_seq: int) -> None:
-    """ENTRY:166-221, same argument order."""
-    if _native.decode_stage2(o, out_logexpsum, b_seqlen, mid_o, mid_o_logexpsum, block_seq):
+def flash_decoding_stage2(o, out_logexpsum, b_seqlen, mid_o, mid_o_logexpsum, block_seq: int, lead_rows: int = 0) -> None:
+    """ENTRY:166-221, same argument order; lead_rows: rows in front of a request's blocks that are merged with them."""
+    if _native.decode_stage2(o, out_logexpsum, b_seqlen, mid_o, mid_o_logexpsum, block_seq, lead_rows):
         return
+    _req(lead_rows >= 0, "lead_rows >= 0")
     a = _stage2_args(o, out_logexpsum, b_seqlen, mid_o, mid_o_logexpsum, block_seq)
+    a.lead_rows = int(lead_rows)
     _lib.check(_lib.load().lsattn_decode_stage2(C.byref(a), _stream()), "lsattn_decode_stage2")
 
 

@@ -156,8 +156,6 @@ def multi_instance_decode(q, instances: Sequence[DecodeInstance], num_kv_heads: 
     global_mid_o = buf("global_mid_o", (P - 1 + num_seq_block, B, Hq, D))
     global_mid_lse = buf("global_mid_o_logexpsum", (P - 1 + num_seq_block, B, Hq))
     global_out_lse = buf("global_out_logexpsum", (B, Hq))
-    # MODEL:516
-    merge_len = ((P - 1) + (master.b_seq_len + (BS - 1)) // BS).to(torch.int32).contiguous()
 
     # peers: stage1 + stage2 over what they hold, fp32 partial straight into the master's rows 0..P-2
     for r, inst in enumerate(instances[1:]):
@@ -173,6 +171,7 @@ def multi_instance_decode(q, instances: Sequence[DecodeInstance], num_kv_heads: 
                                   master.req_to_token, master.b_req_idx, master.b_seq_len, master.max_len_in_batch,
                                   global_mid_o[P - 1:], global_mid_lse[P - 1:], BS)
     o = torch.empty_like(q) if out is None else out
-    # LI:360-367
-    longserve_flash_decode_stage2(global_mid_o, global_mid_lse, merge_len, o.view(-1, Hq, D), global_out_lse, 1)
+    # LI:360-367: the peers' rows and the master's blocks of each request.  (MODEL:516 works their number out on the GPU once for all layers, as
+    # lengths to a merge of block_seq 1; here the merge does, from the lengths it has: three small launches less, 4.5 us each.)
+    longserve_flash_decode_stage2(global_mid_o, global_mid_lse, master.b_seq_len, o.view(-1, Hq, D), global_out_lse, BS, P - 1)
     return o, global_out_lse

@@ -353,6 +353,27 @@ def test_stage2_empty_request_defined(lsa):
     assert_lse_close(l[1], l_ref, "lse", rel=1e-5)
 
 
+@pytest.mark.parametrize("lead", [0, 1, 3, 70])
+@pytest.mark.parametrize("own", [1, 5, 66])
+def test_stage2_with_rows_of_peers_in_front(lsa, lead, own):
+    """The peers' rows and a request's own blocks, whose number follows from its length: as the merge of so many rows of one token each."""
+    print("case", lead, own, flush=True)
+    B, H, D, BS = 5, 3, 128, 16
+    g = torch.Generator().manual_seed(lead * 100 + own)
+    mo, ml = torch.randn(lead + own, B, H, D, generator=g).to(DEV), torch.randn(lead + own, B, H, generator=g).to(DEV)
+    lens = torch.tensor([own * BS, 0, 1, (own * BS) // 2 + 1, 3 * own * BS], dtype=torch.int32)  # (the last one: no more rows than there are)
+    rows = torch.tensor([own, 0, 1, -(-((own * BS) // 2 + 1) // BS), own], dtype=torch.int32) + lead
+    got = []
+    for args in ((lens, BS, lead), (rows, 1)):
+        o, l = torch.full((B, H, D), 9.0, device=DEV), torch.full((B, H), 9.0, device=DEV)
+        lsa.longserve_flash_decode_stage2(mo, ml, args[0].to(DEV), o, l, *args[1:])
+        got.append((o, l))
+    torch.cuda.synchronize()
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    with pytest.raises(ValueError):
+        lsa.longserve_flash_decode_stage2(mo, ml, lens.to(DEV), o, l, BS, -1)
+
+
 @pytest.mark.parametrize("nblk", [1, 7, 31, 64, 65, 300, 1029])
 def test_stage2_alone_over_few_and_many_partials(lsa, nblk):
     """The merge on its own, on random partials: every count of blocks around the points where the kernel changes its
