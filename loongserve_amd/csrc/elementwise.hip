@@ -8,7 +8,7 @@
 namespace lsattn {
 // Streams that are read and written back in place run with non-temporal accesses (NT) once they are larger than the caches:
 // a line that is read, kept in the L2 as dirty and evicted later costs HBM more than one that passes through (activation
-// of 16384 x 11008: 203 -> 177 us, 6.1 TB/s).  Out-of-place streams (the norm, the pool rows) lose by it.
+// of 16384 x 11008: 203 -> 177 us, 6.1 TB/s).  Out-of-place streams of that size (the norm, the pool rows) lose by it.
 constexpr int64_t kStreamBytes = 64 << 20;
 template <bool NT, typename V> __device__ __forceinline__ V stream_load(const V* p) { return NT ? __builtin_nontemporal_load(p) : *p; }
 template <bool NT, typename V> __device__ __forceinline__ void stream_store(V* p, const V& v) {
@@ -26,7 +26,12 @@ template <bool NT, typename V> __device__ __forceinline__ void stream_store(V* p
 // workgroups bounds it).  A wave per row up to 512 wide, and up to 1024 from 1024 rows on (fewer take 2.5 us instead of 2.4); at 1536
 // the wave wins from 4096 rows on (87.8 against 78.9 at 65536) and loses 15 % below, at 2048 it loses throughout.
 // ---------------------------------------------------------------------------------------------------
-constexpr int64_t kRmsNarrow = 512, kRmsNarrowRows = 1024;
+// The weights are asked for beside the row, not behind the barrier (24 rows of 4096 2.65 -> 2.56 us, one 2.55 -> 2.46).
+// The result is stored non-temporally (NT) where it is no larger than the L2s are together: it does not wait there as dirty lines for the
+// next kernel's reads (1000 rows of 4096 5.3 -> 4.7 us, 4000 13.9 -> 11.3; with a kernel that reads the result behind it 12.0 -> 11.1 and 24.7 -> 23.8,
+// with a product by 4096 x 1024 31.6 -> 31.1 and 58.6 -> 58.1).  Past that the norm itself may gain, but whoever reads the result loses more: 8000 rows and
+// the product 96 -> 98, 16384 rows and it 160 -> 165, and an addition 80 -> 86.
+constexpr int64_t kRmsNarrow = 512, kRmsNarrowRows = 1024, kRmsStreamedBytes = 32 << 20;
 constexpr int64_t kMaxGroups = (1 << 24) - 1;  // workgroups of 256 threads in one launch (fewer than 2^32 threads)
 
 __device__ __forceinline__ float wave_sum(float v) {
@@ -36,7 +41,7 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
-template <int WPR, int CHUNKS>
+template <int WPR, int CHUNKS, bool NT>
 __global__ __launch_bounds__(256) void rms_norm_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ in,
                                                        const uint16_t* __restrict__ weight, int64_t rows, int64_t hidden, float eps) {
   constexpr int LANES = 64 * WPR;  // of a row
@@ -48,7 +53,7 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(uint16_t* __restrict__ ou
   const u32x4* wrow = (const u32x4*)weight;
   u32x4* orow = (u32x4*)(out + t * hidden);
   const bool cached = pieces <= LANES * CHUNKS;
-  u32x4 keep[CHUNKS];
+  u32x4 keep[CHUNKS], weights[CHUNKS];
   float ss = 0.f;
   auto add_squares = [&](const u32x4& x) {
     float f[8];
@@ -61,9 +66,12 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(uint16_t* __restrict__ ou
     for (int c = 0; c < CHUNKS; c++) {
       const int i = lane + LANES * c;
       keep[c] = i < pieces ? row[i] : u32x4{0, 0, 0, 0};
+      weights[c] = i < pieces ? wrow[i] : u32x4{0, 0, 0, 0};
     }
 #pragma unroll
     for (int c = 0; c < CHUNKS; c++) add_squares(keep[c]);
+#pragma unroll
+    for (int c = 0; c < CHUNKS; c++) asm volatile("" : "+v"(weights[c]));  // (or the compiler moves their loads behind the barrier)
   } else {
     for (int i = lane; i < pieces; i += LANES) add_squares(row[i]);
   }
@@ -88,10 +96,10 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(uint16_t* __restrict__ ou
 #pragma unroll
     for (int c = 0; c < CHUNKS; c++) {
       const int i = lane + LANES * c;
-      if (i < pieces) orow[i] = scale_piece(keep[c], wrow[i]);
+      if (i < pieces) stream_store<NT>(orow + i, scale_piece(keep[c], weights[c]));
     }
   } else {
-    for (int i = lane; i < pieces; i += LANES) orow[i] = scale_piece(row[i], wrow[i]);
+    for (int i = lane; i < pieces; i += LANES) stream_store<NT>(orow + i, scale_piece(row[i], wrow[i]));
   }
 }
 
@@ -99,10 +107,12 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(uint16_t* __restrict__ ou
 template <int WPR, int CHUNKS>
 static int launch_rms_norm(uint16_t* out, const uint16_t* in, const uint16_t* weight, int64_t rows, int64_t hidden, float eps, hipStream_t st) {
   constexpr int64_t PER_WG = 4 / WPR;
+  const bool nt = rows <= kRmsStreamedBytes / 2 / hidden;
   for (int64_t t0 = 0; t0 < rows; t0 += kMaxGroups * PER_WG) {
     const int64_t n = rows - t0 < kMaxGroups * PER_WG ? rows - t0 : kMaxGroups * PER_WG;
-    LSATTN_LAUNCH_KERNEL((rms_norm_kernel<WPR, CHUNKS>), dim3((unsigned)((n + PER_WG - 1) / PER_WG)), dim3(256), 0, st, out + t0 * hidden,
-                       in + t0 * hidden, weight, n, hidden, eps);
+    const dim3 grid((unsigned)((n + PER_WG - 1) / PER_WG));
+    if (nt) LSATTN_LAUNCH_KERNEL((rms_norm_kernel<WPR, CHUNKS, true>), grid, dim3(256), 0, st, out + t0 * hidden, in + t0 * hidden, weight, n, hidden, eps);
+    else LSATTN_LAUNCH_KERNEL((rms_norm_kernel<WPR, CHUNKS, false>), grid, dim3(256), 0, st, out + t0 * hidden, in + t0 * hidden, weight, n, hidden, eps);
     const int rc = check_launch();
     if (rc != LSATTN_OK) return rc;
   }

@@ -253,3 +253,16 @@ def test_rms_norm_on_both_sides_of_the_narrow_rows_rule(lsa, T, H):
     got = lsa.longserve_cuda_kernels.rms_norm(torch.from_numpy(x).to(DEV), torch.from_numpy(w).to(DEV), 1e-5).cpu().numpy()
     d = _ulp(got, ew.rms_norm(x, w, 1e-5))
     assert d.max() <= 1 and (d > 0).mean() < 2e-2, (d.max(), (d > 0).mean())
+
+
+@pytest.mark.parametrize("T,H", [(2048, 8192), (2049, 8192), (1024, 16384), (1025, 16384)])
+def test_rms_norm_on_both_sides_of_the_streamed_result_rule(lsa, T, H):
+    """Results of 32 MB, the most that is stored non-temporally, and one row more; rows held in registers and rows read twice."""
+    g = torch.Generator(device=DEV).manual_seed(T + H)
+    x = torch.empty((T, H), dtype=torch.float16, device=DEV).normal_(0.0, 1.0, generator=g)
+    w = torch.empty((H,), dtype=torch.float16, device=DEV).normal_(0.0, 1.0, generator=g)
+    out = lsa.longserve_cuda_kernels.rms_norm(x, w, 1e-5)
+    at = torch.tensor([0, 1, T // 2, T - 2, T - 1], device=DEV)
+    assert _ulp(out[at].cpu().numpy(), ew.rms_norm(x[at].cpu().numpy(), w.cpu().numpy(), 1e-5)).max() <= 1
+    # (every row is the same function of its own values)
+    assert torch.equal(out, torch.cat([lsa.longserve_cuda_kernels.rms_norm(x[i:i + 700], w, 1e-5) for i in range(0, T, 700)]))
