@@ -1343,9 +1343,19 @@ static Shape choose_shape(const lsattn_prefill_args* a, bool dv, const Tuning& t
   // 8 % below the other shapes, the worst 1.03 of them (folded into a running partial).  Past that it is even, and so it is a few more than four per CU
   // (0.94 to 1.10), for several requests (0.89 to 1.15) and behind longer contexts (0.90 to 1.12).
   //   (other shapes | this: two ring steps of 2561 rows 32/32 217 | 198, bf16 226 | 209; 1 x 2266 tokens 32/8 57.5 | 54.6)
-  if (a->batch == 1 && a->max_q_len <= 6144 && a->total_kv_rows > 0 && a->total_kv_rows <= a->max_q_len && !a->o_b_start_loc && a->kv_cuts <= 1 &&
-      (wgs128 > 2 * kCUs && wgs128 <= (ph ? 9 : 11) * kCUs / 4))
-    half = true;
+  // Folded in place, which the 256-row shape takes longer for, up to 23/8 and 11/4 (several heads from 1537 rows on; below 0.87 to 1.04): over 90 such launches
+  // 0.95 of the others, 1.02 at most; and past 6144 rows (few heads), up to 21/8, three rounds of the split shape beat two of the 256-row one: 0.81 to 1.01
+  // of it over 60 launches (to 11/4 up to 1.04).
+  //   (256 rows | this: a ring step of 2500 rows 32/8 134 | 121, the prompt 67.8 | 63.7; of 9000 rows 8/1 396 | 349, the prompt 187 | 171)
+  const bool as_long = a->batch == 1 && a->total_kv_rows > 0 && a->total_kv_rows <= a->max_q_len && !a->o_b_start_loc && a->kv_cuts <= 1;
+  if (as_long && wgs128 > 2 * kCUs) {
+    const bool several = ph > 0 && a->max_q_len <= 1536;
+    if (a->max_q_len > 6144) split = split || (a->m && wgs128 <= 21 * kCUs / 8);
+    else if (wgs128 <= (a->m && !several ? ph ? 22 : 23 : ph ? 18 : 22) * kCUs / 8) half = true;
+  }
+  // ... and where they are between three halves and seven quarters of a CU's and short (from there on the folded grid below): the split shape's second
+  // round is one of a few too (36 to 48 heads, 1040 to 1400 rows: prompts 0.83 to 1.01, full steps 0.84 to 0.93; 32 heads, 1600 rows: 0.94 to 1.05, not taken).
+  if (as_long && a->max_q_len <= 1408 && 2 * wgs128 > 3 * kCUs && 4 * wgs128 < 7 * kCUs) half = true;
   if (tn.prefill_rows == LSATTN_PREFILL_ROWS_128) split = true, half = false;
   if (tn.prefill_rows == LSATTN_PREFILL_ROWS_256) split = false, half = false;
   if (tn.prefill_rows == LSATTN_PREFILL_ROWS_HALF) half = true;

@@ -103,7 +103,8 @@ constexpr uint32_t kOnes = 0x3C003C00u;  // two ones in fp16
 constexpr int64_t kCUs = 256;
 constexpr int64_t kL2Bytes = 32 << 20;    // of the eight L2s together
 constexpr int64_t kBunchWorkgroups = 512; // workgroups of a bunch of requests of about equal, short lengths
-constexpr int64_t kShortMaxKeys = 1280;   // 128-wide heads: the keys of the longest request up to which this kernel may take a step
+constexpr int64_t kShortMaxKeys = 1280;   // 128-wide heads: the keys of the longest request up to which this kernel may take a step,
+constexpr int64_t kLoneMaxKeys = 1472;    // of a lone prompt folded in place
 constexpr int64_t kMaxIds = 65535;  // of the second or third index of a grid
 
 // s_waitcnt vmcnt(N) (expcnt / lgkmcnt fields left at their maximum)
@@ -718,7 +719,10 @@ template <typename T, bool DV> int launch_mode(const SmallParams& p, const lsatt
 // start and end.  The host cannot tell it from a batch of prompts, whose numbers are the same.  The launches taken come, in the geometric mean (95 of
 // 100 stay below the figure in brackets), to so much of the time before this kernel, prompts, then full steps:
 //   up to 768 rows 0.79 (0.97), 0.91 (1.16)     769 to 1024 0.85 (0.99), 1.03 (1.25)     1025 to 1280 0.88 (1.02), 1.01 (1.12)
-// so the rule goes by the prompts up to 1024 rows and from there on takes what a ring's shards bear too; past 1280 that is nothing.
+// so the rule goes by the prompts up to 1024 rows and from there on takes what a ring's shards bear too; past 1280 that is one f16 prompt, up to
+// 1472 rows, in the in-place epilogue, with 16 positions: with one head per workgroup the third workgroup per CU, 0.78 to 0.91 and full steps 0.97 to 1.08
+// (1410 tokens 32/32 37.9 -> 31.3 us); up to one per CU 0.92 to 0.95 and 0.90 to 0.95.  (1536 rows 0.89 to 0.95 and 1.06 to 1.12, the partial 0.87 to 1.01 and
+// 1.06 to 1.12: not taken.)
 //   16 positions: up to three workgroups per CU (two and a half of a ragged batch; with one head per workgroup, which leaves each wave fewer
 // rows to mask, four and six), past 768 rows up to one, and the third, where workgroups of 128 rows would run a second round with a few of them (a ragged batch
 // only with one head per workgroup: a lone long request between short ones came to up to 1.6 of the other kernel's time).  Past 1024 rows
@@ -732,9 +736,9 @@ template <typename T, bool DV> int launch_mode(const SmallParams& p, const lsatt
 //   2 x 100, one behind 1900 30.6 | 31.8, 34.5 | 39.8      8 x 64, one behind 7500 79.8 | 108.8, 88 | 169      16 x 64, one behind 15000 145 | 264, 155 | 352
 // The host knows no lengths, only bounds: what total_kv_rows holds beyond the query rows may all belong to one request.
 int prefill_short_blocks(const lsattn_prefill_args* a) {
-  if (a->head_dim != 128 || a->kv_cuts > 1 || a->o_b_start_loc || a->max_q_len <= 0 || a->max_q_len > kShortMaxKeys || a->batch <= 0 || a->batch > kMaxIds || a->num_kv_heads <= 0)
+  if (a->head_dim != 128 || a->kv_cuts > 1 || a->o_b_start_loc || a->max_q_len <= 0 || a->max_q_len > kLoneMaxKeys || a->batch <= 0 || a->batch > kMaxIds || a->num_kv_heads <= 0)
     return 0;
-  int64_t longest = kShortMaxKeys + 1;
+  int64_t longest = kLoneMaxKeys + 1;
   if (a->total_kv_rows > 0) {
     longest = a->total_kv_rows;
     if (a->total_q_rows > 0) {
@@ -744,13 +748,17 @@ int prefill_short_blocks(const lsattn_prefill_args* a) {
     }
   }
   if (a->max_kv_len > 0 && a->max_kv_len < longest) longest = a->max_kv_len;
-  if (longest > kShortMaxKeys) return 0;
+  if (longest > kLoneMaxKeys) return 0;
   const Tuning tn = tuning();
   if (tn.prefill_rows || tn.prefill_order || tn.prefill_pack) return 0;  // (choices among the 128-wide kernel's shapes)
   const int pack = pack_shift_of(a);
   const int64_t one = workgroups(a, pack, 1), two = workgroups(a, pack, 2);
   const bool f16 = a->dtype == LSATTN_F16, rag = ragged(a);
   if (a->max_q_len <= 768) return longest > 1024 ? 0 : 2 * one <= (pack ? rag ? 5 : 6 : rag ? 12 : 8) * kCUs ? 1 : 2;
+  if (longest > kShortMaxKeys || a->max_q_len > kShortMaxKeys) {
+    if (a->batch > 1 || a->max_q_len != longest) return 0;
+    return f16 && a->m && (one <= kCUs || (pack == 0 && one > 2 * kCUs && one <= 3 * kCUs));
+  }
   const bool past = longest > 1024;
   if (one <= kCUs) return !past || (f16 && a->batch == 1) ? 1 : 0;
   // (m: of the three steps only the in-place one has it.  bf16 does not look at it: whether V is to be copied is asked before)

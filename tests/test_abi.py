@@ -508,3 +508,29 @@ def test_prefill_route_names_a_kernel_for_every_step_and_none_for_others():
     assert _route(1, 16384, (32, 32)) == ROWS_256 and _route(1, 500, (32, 8), cuts=2) == ROWS_128 and _route(1, 500, (32, 8), cuts=3) == ROWS_256
     assert _route(1, 100, (32, 8), dtype=1) == ROWS_256 and _route(1, 100, (32, 8), dtype=1, v_is_f16=1) == ROWS_128
     assert _route(0, 100, (32, 8)) == _route(1, 0, (32, 8)) == _route(1, 100, (32, 0)) == _route(1, 100, (32, 5)) == _route(1, 100, (32, 8), 80) == 0
+
+
+def test_lone_prompts_past_1280_rows_fold_in_the_short_prompts_kernel():
+    """One f16 prompt of up to 1472 rows in the in-place epilogue, up to one workgroup of 64 rows per CU or, with a head each, in the third.
+    Not behind a context, against fewer keys, or beside another request."""
+    lone = lambda n, heads, kv=None, **kw: _route(1, n, heads, total_q=n, total_kv=kv or n, **kw)
+    for n in (1281, 1410, 1472):
+        assert lone(n, (8, 1), m=256) == lone(n, (32, 32), m=256) == SMALL_16
+        assert lone(n, (32, 32)) == lone(n, (8, 1)) == ROWS_128 and lone(n, (8, 1), dtype=1, v_is_f16=1, m=256) == ROWS_128
+        assert lone(n, (32, 32), dtype=1, v_is_f16=1, m=256) == lone(n, (32, 8), m=256) == ROWS_128
+        assert lone(n, (32, 32), kv=n + 1, m=256) == lone(n, (32, 32), kv=1000, m=256) == ROWS_128
+        assert _route(2, n, (32, 32), total_q=2 * n, total_kv=2 * n, m=256) not in (SMALL_16, SMALL_32)
+    assert lone(1473, (32, 32), m=256) == lone(1473, (8, 1), m=256) == ROWS_128
+    assert lone(1300, (20, 20), m=256) == ROWS_128  # (1.6 workgroups of 64 rows per CU)
+
+
+def test_lone_prompts_of_a_few_workgroups_past_two_per_cu():
+    """Folded in place, where 256-row workgroups end in a round of a few: two of four waves per CU, or three rounds of the split shape past 6144 rows."""
+    lone = lambda n, heads, m=256: _route(1, n, heads, total_q=n, total_kv=n, m=m)
+    assert lone(2500, (32, 8)) == lone(2816, (32, 8)) == HALF and lone(2817, (32, 8)) == lone(2500, (32, 8), None) == ROWS_256  # (704 workgroups of 128 rows)
+    assert lone(2944, (32, 32)) == HALF and lone(2945, (32, 32)) == lone(2944, (32, 32), None) == ROWS_256                      # (736)
+    assert lone(1400, (64, 8)) == ROWS_256 and lone(5000, (16, 2)) == HALF  # (several heads, up to 1536 rows: up to 576)
+    assert lone(6144, (14, 14)) == HALF and lone(6145, (14, 14)) == ROWS_256 and lone(6272, (13, 13)) == ROWS_128
+    assert lone(8300, (8, 1)) == lone(10752, (8, 1)) == ROWS_128 and lone(10753, (8, 1)) == lone(8300, (8, 1), None) == ROWS_256  # (672)
+    assert lone(1290, (40, 40)) == lone(1408, (36, 36)) == lone(1300, (40, 40), None) == HALF and lone(1409, (36, 36)) == ROWS_128
+    assert _route(1, 2500, (32, 8), total_q=2500, total_kv=2600, m=256) == ROWS_256 and _route(2, 1250, (32, 8), total_q=2500, total_kv=2500, m=256) != HALF

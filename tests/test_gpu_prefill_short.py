@@ -192,3 +192,10 @@ def test_short_prompts_in_three_stages_and_the_grids_orders(lsa, mode, V, what):
 def test_longer_prompts_with_16_positions_per_wave(lsa, mode, V, Hq, Hkv, lens):
     print("case", mode, V, Hq, Hkv, flush=True)
     _every_epilogue_on(SMALL_16, lsa, mode, V, 128, Hq, Hkv, lens, [0] * len(lens))
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(8, 1), (24, 24)])
+def test_lone_prompts_past_1280_rows(lsa, Hq, Hkv):
+    """The longest prompt that the kernel folds in place.  (The route that is asked for names no m: it is the 128-row one of the partial.)"""
+    print("case", Hq, Hkv, flush=True)
+    _every_epilogue_on(5, lsa, "in_place", "f16", 128, Hq, Hkv, [1472], [0])
