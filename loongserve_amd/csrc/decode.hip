@@ -1093,11 +1093,15 @@ constexpr int64_t kListedFromWorkgroups = 32768;  // launches of the plain grid 
 // list costs an even batch more than that (config 3, 16384 workgroups: 947 -> 962 us) and stays with the larger grids.
 constexpr int64_t kListedFromWorkgroupsCoarse = 8192;
 constexpr int64_t kListedCoarseTokens = 1024;
-// Equal shares from eight requests on wherever the plain shape would run, and for two to seven when the launch is large (waves of the plain
-// shape by the longest request): one request is even by itself and 1-3 % faster on the grids (65536 tokens, GQA 32/8: 50.8 us against
-// 52.6), a few long ones of one length 1 % (4 x 131072), a few ragged ones up to 13 % slower (4 of 1000 to 8000 tokens, MHA 32: 62 us
-// against 54; GQA 32/8, 1024 waves: 23.1 against 24.1).
-constexpr int64_t kSharesMinBatch = 8, kSharesMinWavesFew = 2048;
+// Equal shares from eight requests on wherever the plain shape would run, and for fewer, down to one, where the grid has more than a
+// workgroup per CU (1024 waves of 256 tokens): up to two, the CUs that hold two set its time, and a split of other sizes has as many.  Below that a few even
+// requests take 1.02 to 1.21 of the grid's time by shares.  Four and more KV heads, of the time of the grids, 180 launches: one request 0.73 to 0.99 (groups
+// below four, which keep the grid where it has nearly two workgroups per CU, to 1.05 there), two to seven of one length 0.83 to 1.08, of other lengths 0.63 to 1.06.
+//   (us: 1 x 35000 tokens 32/8 36 | 30, 1 x 66000 64/8 67 | 52; 3 x 14906 at most 32/8 32.3 | 24.9; 7 x 5387 at most 16/8 26.6 | 17.6; 2 x 24335 32/8 43.5 | 39.2)
+// Fewer than four KV heads, where a grid of the shape whose waves split a block stands against it, from more than 2048 waves on (four rounds of
+// two workgroups per CU) 0.57 to 1.10, in the mean 0.92, and with one KV head and four requests and more also in the first fourth of the third round 0.67 to
+// 1.03, 0.84 (8 requests, one of 33819 tokens, 16/1 27.5 | 18.4 us; three with one of 107373 23.6 | 31.8, not taken); in between one length loses up to 16 %.
+constexpr int64_t kSharesMinBatch = 8, kSharesMinWavesFew = 1025, kSharesMinWavesFewHeads = 2049;
 // Not where the rows of the partials' buffers hold less than half of the shares the chip has waves for: 256 requests of 256 tokens,
 // GQA 32/8, are one share (2.9 ms) or a grid (57 us).  And not in place of a grid that one round of workgroups, one per CU, walks,
 // if the rows hold fewer shares than the chip has waves for (24 requests of 1024 tokens, GQA 32/8, 73 shares: 30.1 us against 22.6; 33 of
@@ -1346,15 +1350,15 @@ __global__ __launch_bounds__(NT) void decode_stage2_kernel(Stage2Params p) {
 }
 
 // The merge behind decode_stage1_mfma_range_kernel: W waves per (request, head), 4 / W pairs per workgroup (heads of one
-// request).  Every wave counts the units in front of its request and in all and knows from them the first and the last
+// request; sixteen waves: one pair).  Every wave counts the units in front of its request and in all and knows from them the first and the last
 // share that reach into the request: their partials are consecutive rows.  Half a wave reads a row (16 bytes a lane), eight
 // rows and their log-sum-exps in flight per half wave.  Bound by its chain of dependent loads (the argument block, the lengths, the rows)
 // and, from a few thousand pairs on, by the workgroups' turn-over: with a whole workgroup of eight slices per pair, as in
 // decode_stage2_kernel, 128 requests with 32 heads took 10.2 us for one to three rows each.
 template <typename OT, int W>
-__global__ __launch_bounds__(256) void decode_merge_shares_kernel(Stage2Params p) {
+__global__ __launch_bounds__(W > 4 ? W * 64 : 256) void decode_merge_shares_kernel(Stage2Params p) {
   constexpr int D = 128, U = 8;
-  constexpr int PAIRS = 4 / W;
+  constexpr int PAIRS = W > 4 ? 1 : 4 / W;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t head_groups = ((uint32_t)p.heads + PAIRS - 1) / PAIRS;
   const int b = blockIdx.x / head_groups;
@@ -1432,8 +1436,21 @@ __global__ __launch_bounds__(256) void decode_merge_shares_kernel(Stage2Params p
     }
     __syncthreads();
     if (wave != 0) return;
+    if constexpr (W <= 4) {
 #pragma unroll
-    for (int w = 1; w < W; w++) join(sM[w], sL[w], sAcc[w][c]);
+      for (int w = 1; w < W; w++) join(sM[w], sL[w], sAcc[w][c]);
+    } else {  // (none of the sixteen waits for another)
+#pragma unroll
+      for (int w = 1; w < W; w++) M = fmaxf(M, sM[w]);
+      acc = f32x4{0.f, 0.f, 0.f, 0.f};
+      L = 0.f;
+#pragma unroll
+      for (int w = 0; w < W; w++) {
+        const float x = exp2_diff(sM[w] * kLog2e, M * kLog2e);
+        acc += sAcc[w][c] * x;
+        L += sL[w] * x;
+      }
+    }
   }
   if (half == 0 && live) {
     const int64_t out_row = (int64_t)b * p.heads + h;
@@ -1443,6 +1460,7 @@ __global__ __launch_bounds__(256) void decode_merge_shares_kernel(Stage2Params p
   }
 }
 
+constexpr uint32_t kWideMergePairs = 64;
 // What the fused call allows stage 1 to do beside it: merge its partials itself (JOIN), which leaves `done` set.
 struct JoinPlan {
   const lsattn_decode_stage2_args* s2;
@@ -1546,6 +1564,9 @@ static int launch_stage1(const lsattn_decode_stage1_args* a, hipStream_t st, Joi
   return check_launch();
 }
 
+// Waves of the plain shape up to which the shape whose waves split a block runs instead, on four and more KV heads.  513 to 576 waves 0.61 to 0.84 of the plain
+// shape where the lengths differ, 1.00 to 1.03 where they do not (24 requests of at most 592 tokens 32/8 16.8 -> 10.8 us); 577 to 640 0.68 to 0.96, 0.98 to 1.14, not taken.
+constexpr int64_t kSplitMaxWaves = 576;
 // Large launches: the matrix-pipe kernel, when its conditions hold (blocks a multiple of 32 tokens, enough waves to fill
 // the chip); lsattn_set_tuning forces the choice where the conditions allow it (tuning, tests).
 // What the fused call hands to stage 1 and on to the merge behind it.
@@ -1598,13 +1619,13 @@ template <typename T> static int launch_stage1_mfma(const lsattn_decode_stage1_a
   const int64_t wgs_x = (chunks + cw - 1) / cw, wgs_y = (p.tasks + tw - 1) / tw;
   if (wgs_x > 0x7fffffff || a->batch > 65535 || wgs_y > 65535) return LSATTN_OK;
   // Which shape, by the launch's size in waves of the plain shape (256 tokens x task x request; measured):
-  //   groups of four and more query heads per KV head: up to 512 waves (3072 on fewer than four KV heads, where the plain
+  //   groups of four and more query heads per KV head: up to kSplitMaxWaves waves (3072 on fewer than four KV heads, where the plain
   //     shape has no neighbouring heads to put side by side) the shape whose four waves split a block (a launch of 8 to 512
   //     plain waves runs 30-45 % shorter with it than with either other kernel), above that the plain shape;
   //   smaller groups (most of an MFMA's sixteen columns idle): the plain shape from 768 waves, below that the lane kernel.
   const int64_t waves = chunks * p.tasks * a->batch;
   const bool can_split = p.block_seq % (kMfmaWaves * kMfmaBatch) == 0 && nblk <= 0x7fffffff;
-  bool split_waves = group >= 4 && can_split && waves <= (p.tasks < 4 ? 3072 : 512);
+  bool split_waves = group >= 4 && can_split && waves <= (p.tasks < 4 ? 3072 : kSplitMaxWaves);
   bool use = !split_waves && waves >= (group >= 4 ? 513 : 768);
   const Tuning tn = tuning();  // (lsattn_set_tuning: tuning and tests)
   if (tn.decode_stage1 == LSATTN_DECODE_STAGE1_LANE) use = split_waves = false;
@@ -1625,8 +1646,10 @@ template <typename T> static int launch_stage1_mfma(const lsattn_decode_stage1_a
     if (!forced && tn.decode_stage1 != 0) return LSATTN_OK;
     // (waves of the plain shape at 256 tokens each, whatever the split asked for; the shape whose waves split a block keeps its launches)
     const int64_t waves256 = (shares->units * kMfmaBatch + 255) / 256 * p.tasks * a->batch;
-    const bool large = waves256 >= (group < 4 ? 768 : p.tasks < 4 ? 3073 : 513);
-    if (!forced && (!large || a->batch < 2 || (a->batch < kSharesMinBatch && waves256 < kSharesMinWavesFew))) return LSATTN_OK;
+    const bool large = waves256 >= (group < 4 ? 768 : p.tasks < 4 ? kSharesMinWavesFewHeads : kSplitMaxWaves + 1) ||
+                       (group >= 4 && p.tasks == 1 && a->batch >= 4 && waves256 > 4 * kCUs && waves256 <= 5 * kCUs);
+    const bool few = a->batch < kSharesMinBatch && waves256 < kSharesMinWavesFew, nearly_two = group < 4 && waves256 > 6 * kCUs && waves256 < 8 * kCUs;
+    if (!forced && (!large || few || (a->batch < 2 && (p.tasks < 4 || nearly_two)))) return LSATTN_OK;
     // Short contexts, whose rows hold too few shares (a longest request of up to 256 tokens one share, whatever the batch),
     // and grids of one round of workgroups, see kSharesOneRoundBatch.
     const int64_t wgs = wgs_x * wgs_y * a->batch;
@@ -1812,7 +1835,10 @@ template <typename OT> static int dispatch_stage2(const Stage2Params& p, int64_t
   if (p.max_shares > 0) {
     if (D != 128) return LSATTN_ERR_UNSUPPORTED;
     // four waves per pair while that keeps every pair resident at once (sixteen waves per CU)
-    if ((int64_t)grid.x <= 4 * kCUs) LSATTN_LAUNCH_KERNEL((decode_merge_shares_kernel<OT, 4>), grid, dim3(256), 0, st, p);
+    // (sixteen for the few pairs of one or two requests, or of few heads, which may have hundreds of rows each: one long request among short ones
+    // 0.84 to 1.03, in the mean 0.97, ragged ones 0.99, equal ones 1.00 to 1.01; with more pairs 0.99 to 1.17)
+    if (grid.x <= kWideMergePairs && p.max_shares >= 128) LSATTN_LAUNCH_KERNEL((decode_merge_shares_kernel<OT, 16>), grid, dim3(1024), 0, st, p);
+    else if ((int64_t)grid.x <= 4 * kCUs) LSATTN_LAUNCH_KERNEL((decode_merge_shares_kernel<OT, 4>), grid, dim3(256), 0, st, p);
     else LSATTN_LAUNCH_KERNEL((decode_merge_shares_kernel<OT, 1>), dim3((unsigned)(p.batch * ((p.heads + 3) / 4))), dim3(256), 0, st, p);
     return check_launch();
   }

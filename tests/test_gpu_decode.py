@@ -994,3 +994,30 @@ def test_one_launch_and_huge_values_that_weigh_nothing(lsa, dtype, huge, Hq, Hkv
     # (2^-10 of what the sums of values around 1 are held to)
     assert_o_close(o * 2.0 ** 10, o_ref * 2.0 ** 10, "o")
     assert_lse_close(l, l_ref, "lse")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Hq,Hkv,lens", [
+    (32, 8, [32769]), (32, 8, [33000]), (64, 8, [17000, 33]), (32, 32, [8193]),  # one request and two, merged by sixteen waves a pair (64 pairs)
+    (32, 4, [20000, 0, 17001]), (32, 8, [9000, 1, 33, 8999]),                    # more pairs, a request without tokens
+    (8, 1, [70000, 1, 300, 69999]), (16, 1, [33819] + [2000] * 7),               # one KV head, 1096 and 1064 waves
+    (4, 1, [131400, 500, 131072, 64]),                                           # ... and 2056
+    (32, 8, [592, 576] + [40] * 22, ), (32, 4, [36 * 256 - 100, 7, 2000, 1]),    # 576 waves: the shape whose waves split a block
+])
+def test_launches_of_a_few_workgroups_past_a_round(lsa, dtype, Hq, Hkv, lens):
+    """Few requests in equal shares, and the last launch that is split among a block's waves, as the library chooses."""
+    print("case", dtype, Hq, Hkv, lens[:4], flush=True)
+    B, D, BS = len(lens), 128, 256
+    q, kv, table, b_req, b_len = decode_case(321, B, Hq, Hkv, D, lens, sum(lens) + 500, dtype)
+    o_ref, l_ref = orc.decode_full(q, kv[:, :Hkv], kv[:, Hkv:], table, b_req, b_len)
+    kvd = kv.to(DEV)
+    mo = torch.full((max(lens) // BS + 1, B, Hq, D), float("nan"), device=DEV)
+    ml = torch.full(mo.shape[:3], float("nan"), device=DEV)
+    for _ in range(2):  # (the second call over what the first left in the buffers)
+        o, l = lsa.longserve_token_decode_attention_flash_decoding(q.to(DEV), table.to(DEV), b_req.to(DEV), b_len.to(DEV), mo, ml, B, max(lens), Hq, D,
+                                                                   kvd[:, :Hkv], kvd[:, Hkv:], BS)
+        torch.cuda.synchronize()
+        live = b_len > 0
+        assert_o_close(o.cpu()[live], o_ref[live], "o")
+        assert_lse_close(l.cpu()[live], l_ref[live], "lse")
+        assert bool((o.cpu()[~live] == 0).all()) and bool((l.cpu()[~live] == -math.inf).all())
