@@ -1021,3 +1021,25 @@ def test_launches_of_a_few_workgroups_past_a_round(lsa, dtype, Hq, Hkv, lens):
         assert_o_close(o.cpu()[live], o_ref[live], "o")
         assert_lse_close(l.cpu()[live], l_ref[live], "lse")
         assert bool((o.cpu()[~live] == 0).all()) and bool((l.cpu()[~live] == -math.inf).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Hq,Hkv,lens", [(32, 8, [32 * 256 + 1, 300, 0, 4000]), (16, 8, [48 * 256, 7, 2000, 12287]), (32, 32, [3072, 1, 3000, 257])])
+def test_both_stages_of_launches_just_past_a_workgroup_per_cu(lsa, dtype, Hq, Hkv, lens):
+    """1056 to 1536 waves, split among a block's waves: the stages apart, one partial per 256 tokens, in buffers that start as NaN."""
+    print("case", dtype, Hq, Hkv, lens, flush=True)
+    B, D, BS = len(lens), 128, 256
+    q, kv, table, b_req, b_len = decode_case(77, B, Hq, Hkv, D, lens, sum(lens) + 500, dtype)
+    o_ref, l_ref = orc.decode_full(q, kv[:, :Hkv], kv[:, Hkv:], table, b_req, b_len)
+    kvd = kv.to(DEV)
+    nblk = (max(lens) + BS - 1) // BS
+    mo, ml = torch.full((nblk, B, Hq, D), float("nan"), device=DEV), torch.full((nblk, B, Hq), float("nan"), device=DEV)
+    o, l = torch.empty(B, Hq, D, device=DEV), torch.empty(B, Hq, device=DEV)
+    lsa.longserve_flash_decode_stage1(q.to(DEV), kvd[:, :Hkv], kvd[:, Hkv:], table.to(DEV), b_req.to(DEV), b_len.to(DEV), max(lens), mo, ml, BS)
+    lsa.longserve_flash_decode_stage2(mo, ml, b_len.to(DEV), o, l, BS)
+    torch.cuda.synchronize()
+    written = torch.arange(nblk)[:, None] * BS < b_len[None, :]
+    assert torch.equal(~torch.isnan(ml.cpu()), written[:, :, None].expand(-1, -1, Hq))
+    live = b_len > 0
+    assert_o_close(o.cpu()[live], o_ref[live], "o")
+    assert_lse_close(l.cpu()[live], l_ref[live], "lse")
