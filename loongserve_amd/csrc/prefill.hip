@@ -1356,6 +1356,14 @@ static Shape choose_shape(const lsattn_prefill_args* a, bool dv, const Tuning& t
   // ... and where they are between three halves and seven quarters of a CU's and short (from there on the folded grid below): the split shape's second
   // round is one of a few too (36 to 48 heads, 1040 to 1400 rows: prompts 0.83 to 1.01, full steps 0.84 to 0.93; 32 heads, 1600 rows: 0.94 to 1.05, not taken).
   if (as_long && a->max_q_len <= 1408 && 2 * wgs128 > 3 * kCUs && 4 * wgs128 < 7 * kCUs) half = true;
+  // Ragged requests folded in place whose keys are no more than their rows (prompts, or a ring's steps), up to 2048 rows: the 256-row shape ends with the
+  // longest requests' workgroups alone on their CUs, the split shape in one round more.  From three halves of a workgroup per CU on (one where it
+  // would be the 256-row shape), over 45 launches: prompts of up to 1024 rows 0.84 of the others, 1536 0.93, 2048 0.97, full steps 0.93; 0.58 to 1.10 (133 launches: 0.92).
+  // Equal lengths 0.84 to 1.07, longer ragged ones 0.89 to 1.23: not taken.
+  //   (us: 20 of at most 840 tokens 8/1 52 | 37, 12 of at most 941 8/1 47 | 32, 5 of at most 854 32/8, full steps, 50 | 42)
+  if (a->batch > 1 && a->m && a->total_q_rows > 0 && a->total_kv_rows > 0 && a->total_kv_rows <= a->total_q_rows && a->max_q_len <= 2048 &&
+      a->total_q_rows * 10 <= (int64_t)a->batch * a->max_q_len * 9 && !a->o_b_start_loc && a->kv_cuts <= 1 && 2 * wgs128 >= (split ? 3 : 2) * kCUs)
+    half = true;
   if (tn.prefill_rows == LSATTN_PREFILL_ROWS_128) split = true, half = false;
   if (tn.prefill_rows == LSATTN_PREFILL_ROWS_256) split = false, half = false;
   if (tn.prefill_rows == LSATTN_PREFILL_ROWS_HALF) half = true;

@@ -534,3 +534,11 @@ def test_lone_prompts_of_a_few_workgroups_past_two_per_cu():
     assert lone(8300, (8, 1)) == lone(10752, (8, 1)) == ROWS_128 and lone(10753, (8, 1)) == lone(8300, (8, 1), None) == ROWS_256  # (672)
     assert lone(1290, (40, 40)) == lone(1408, (36, 36)) == lone(1300, (40, 40), None) == HALF and lone(1409, (36, 36)) == ROWS_128
     assert _route(1, 2500, (32, 8), total_q=2500, total_kv=2600, m=256) == ROWS_256 and _route(2, 1250, (32, 8), total_q=2500, total_kv=2500, m=256) != HALF
+
+
+def test_ragged_batches_folded_in_place_by_four_waves():
+    """Ragged requests of up to 2048 rows against as many keys, from a workgroup of 128 rows per CU on (three halves where it would be the split shape's)."""
+    step = lambda n, total, heads=(32, 8), m=256, **kw: _route(4, n, heads, total_q=total, total_kv=kw.pop("total_kv", total), m=m, **kw)
+    assert step(2048, 5000) == HALF and step(2049, 5000) == step(2048, 5000, m=None) == step(2048, 5000, total_kv=5001) == ROWS_256
+    assert step(2048, 7372) == HALF and step(2048, 7373) == ROWS_256  # (nine tenths of 8192)
+    assert step(1900, 2000, (8, 1)) == ROWS_128  # (1.0 per CU)
