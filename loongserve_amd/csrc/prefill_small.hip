@@ -104,7 +104,12 @@ constexpr int64_t kCUs = 256;
 constexpr int64_t kL2Bytes = 32 << 20;    // of the eight L2s together
 constexpr int64_t kBunchWorkgroups = 512; // workgroups of a bunch of requests of about equal, short lengths
 constexpr int64_t kShortMaxKeys = 1280;   // 128-wide heads: the keys of the longest request up to which this kernel may take a step,
-constexpr int64_t kLoneMaxKeys = 1472;    // of a lone prompt folded in place
+constexpr int64_t kLoneMaxKeys = 1472;    // of a lone prompt folded in place,
+constexpr int64_t kPartsMaxKeys = 2304, kPartsMaxKeysBf16 = 2048;  // and of one in up to a workgroup per CU, whose tiles two waves share
+// Two waves per wave's positions (KP = 2) from so many keys on: one workgroup per CU and less of 16 positions per wave, 128-wide heads, one wave each |
+// two (us, in place; 8/1 where nothing is said): 300 tokens 9.5 | 9.6, 32/32 9.1 | 9.5; 450 11.3 | 10.9, 32/32 11.8 | 11.7; 500 32/8 12.8 | 12.1; 600 13.6 | 12.7;
+// 900 17.6 | 15.7; 1280 22.6 | 19.4; a full step of a ring of 900 18.7 | 16.5.
+constexpr int64_t kPartsMinKeys = 512;
 constexpr int64_t kMaxIds = 65535;  // of the second or third index of a grid
 
 // s_waitcnt vmcnt(N) (expcnt / lgkmcnt fields left at their maximum)
@@ -132,8 +137,13 @@ template <int D, int WP, bool DV> constexpr int kResident = D == 128 ? (WP == 32
 // registers and are converted on the way.  WP: query positions per wave, 16 or 32.  (Products of 32 x 32 x 16, which take a tenth fewer
 // vector instructions, ran at 1.88 GHz where these run at 2.16: 8 ragged sequences of 64-wide heads 164 us against 161, 16 x 1024 tokens of
 // 128-wide ones 199 against 194.)
-template <typename T, int D, int MODE, bool DV, int WP>
-__global__ __launch_bounds__(kWaves * 64, (kResident<D, WP, DV>)) void prefill_small_kernel(SmallParams p) {
+// KP = 2: two waves share the positions of a wave and take the first and the second 32 keys of every tile (launches of up to a workgroup per CU, whose one
+// wave per SIMD issues an instruction every five cycles or so); their parts are joined in LDS.  A tile takes 0.75 us of a lone workgroup instead of 0.96, the join and the start
+// of twice the waves 1.1.
+template <typename T, int D, int MODE, bool DV, int WP, int KP = 1>
+__global__ __launch_bounds__(kWaves * KP * 64, (kResident<D, WP, DV>)) void prefill_small_kernel(SmallParams p) {
+  static_assert(KP == 1 || (KP == 2 && WP == 16 && D >= 32), "the parts of a tile of 64 keys, the columns that each of two waves finishes");
+  constexpr int NW = kWaves * KP;
   constexpr int QB = WP / 16;               // blocks of 16 positions per wave
   constexpr int KS = D >= 32 ? D / 32 : 1;  // contraction steps of Q K^T (32 elements each; D = 16 fills half of one)
   constexpr int NDB = D / 16;               // 16-wide blocks of the head
@@ -142,7 +152,7 @@ __global__ __launch_bounds__(kWaves * 64, (kResident<D, WP, DV>)) void prefill_s
   constexpr int RB = D * 2;                 // bytes per row in LDS
   constexpr int TB = TK * RB;               // bytes per tile
   constexpr int RPI = 64 / CPR;             // rows per load instruction (a wave's 64 lanes, 16 bytes each)
-  constexpr int NI = (TK + kWaves * RPI - 1) / (kWaves * RPI);  // load instructions per wave and tile
+  constexpr int NI = (TK + NW * RPI - 1) / (NW * RPI);  // load instructions per wave and tile
   constexpr int RPB = 256 / RB;             // rows that pass all 64 LDS banks once
   // NS stages of (K tile, V tile): the next tiles are written while the present one is read.  Rows are not padded (a load to
   // LDS writes 1 KB in a row); instead the 16-byte chunks of a row are XORed with a function of the row: K so that a
@@ -150,12 +160,14 @@ __global__ __launch_bounds__(kWaves * 64, (kResident<D, WP, DV>)) void prefill_s
   // each of eight rows (half a transposing read) cover the banks once.  Rows sixteen apart share their XOR.
   // (behind them, for the epilogue that folds into (o, m, l): 256 bytes per wave for the old m and l of its rows)
   constexpr int kStateOff = NS * 2 * TB;
-  __shared__ __attribute__((aligned(1024))) char lds[kStateOff + (MODE == 1 ? kWaves * 256 : 0)];
+  constexpr int kJoinOff = kStateOff + (MODE == 1 ? NW * 256 : 0);  // (KP = 2: the waves' maxima and sums)
+  __shared__ __attribute__((aligned(1024))) char lds[kJoinOff + (KP > 1 ? NW * 256 : 0)];
   auto swz_k = [](int row) { return (row / RPB) & (CPR - 1); };
   auto swz_v = [](int row) { return ((row / RPB) & (CPR / 2 - 1)) << 1; };
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;  // query column, lane group
+  const int rw = KP > 1 ? wave & (kWaves - 1) : wave, kp = KP > 1 ? wave / kWaves : 0;  // whose positions; which part of the keys
   // grid: (KV head, heads side by side), (tile from the last one down, request of a bunch), bunch of requests: the heaviest tiles of
   // all requests of a bunch start first, and with a multiple of eight KV heads the workgroups of one run on one XCD (ids are dealt round-robin)
   const int gq = (int)div_by(blockIdx.x, p.d_hkv), kvh = (int)blockIdx.x - gq * p.hkv;
@@ -172,8 +184,8 @@ __global__ __launch_bounds__(kWaves * 64, (kResident<D, WP, DV>)) void prefill_s
   asm volatile("" ::"s"(q_len), "s"(kv_len), "s"(qf), "s"(kf), "s"(q_start32), "s"(kv_start32), "s"(o_start32));
   if (m_wg >= q_len) return;  // (the whole workgroup: the loop below holds barriers)
   const int wph_shift = 2 - p.pack_shift;  // log2 of the waves per head
-  const int h = kvh * p.heads_per_kv + (gq << p.pack_shift) + (wave >> wph_shift);
-  const int m0 = m_wg + (wave & ((1 << wph_shift) - 1)) * WP;  // the wave's first position
+  const int h = kvh * p.heads_per_kv + (gq << p.pack_shift) + (rw >> wph_shift);
+  const int m0 = m_wg + (rw & ((1 << wph_shift) - 1)) * WP;  // the wave's first position
   const int64_t q_start = q_start32, kv_start = kv_start32, o_start = o_start32;
 
   // keys of this KV chunk visible to global query position qpos (ring_context_flashattention_nopad.py:156-159)
@@ -227,11 +239,11 @@ __global__ __launch_bounds__(kWaves * 64, (kResident<D, WP, DV>)) void prefill_s
   const char* vbase = (const char*)p.v + (kv_start * p.v_st + (int64_t)kvh * p.v_sh) * 2;
   // staging: instruction i of a wave carries rows (wave + 4 i) * RPI .. of the K tile and of the V tile.  Tiles that lie inside the
   // chunk take a scalar tile address and the lane's 32-bit offset, no vector arithmetic.
-  const bool stager = NI * kWaves * RPI == TK || wave * RPI < TK;  // (D = 16: two waves)
+  const bool stager = NI * NW * RPI == TK || wave * RPI < TK;  // (D = 16: two waves)
   const int st_row = wave * RPI + lane / CPR;
   const uint32_t k_row = (uint32_t)p.k_st * 2, v_row = (uint32_t)p.v_st * 2;  // (a tile's rows span less than 2^31 bytes)
   const uint32_t k_off = st_row * k_row + ((lane % CPR) ^ swz_k(st_row)) * 16, v_off = st_row * v_row + ((lane % CPR) ^ swz_v(st_row)) * 16;
-  constexpr int STEP = kWaves * RPI;  // rows between a wave's load instructions
+  constexpr int STEP = NW * RPI;  // rows between a wave's load instructions
   constexpr bool APART = !DV && NS > 2;  // K tiles are requested NS - 1 tiles ahead, V tiles that pass through registers one
   u32x4 vst[NI];
   // K and V of tile t (or one of them)
@@ -253,8 +265,8 @@ __global__ __launch_bounds__(kWaves * 64, (kResident<D, WP, DV>)) void prefill_s
         if (K) ko -= (uint32_t)back * k_row;
         if (V) vo -= (uint32_t)back * v_row;
       }
-      if (K) load_to_lds(dst + i * kWaves * 1024, kt, ko + (uint32_t)(i * STEP) * k_row);
-      if (V && DV) load_to_lds(dst + TB + i * kWaves * 1024, vt, vo + (uint32_t)(i * STEP) * v_row);
+      if (K) load_to_lds(dst + i * NW * 1024, kt, ko + (uint32_t)(i * STEP) * k_row);
+      if (V && DV) load_to_lds(dst + TB + i * NW * 1024, vt, vo + (uint32_t)(i * STEP) * v_row);
       if (V && !DV) vst[i] = *(const u32x4*)(vt + (vo + (uint32_t)(i * STEP) * v_row));
     }
   };
@@ -263,7 +275,7 @@ __global__ __launch_bounds__(kWaves * 64, (kResident<D, WP, DV>)) void prefill_s
   auto deposit_v = [&](int stage) __attribute__((always_inline)) {  // (bfloat16 V: the tile in the registers into LDS)
     if (!DV && stager) {
 #pragma unroll
-      for (int i = 0; i < NI; i++) *(u32x4*)(lds + stage * 2 * TB + TB + (wave + i * kWaves) * 1024 + lane * 16) = bf16_to_f16(vst[i]);
+      for (int i = 0; i < NI; i++) *(u32x4*)(lds + stage * 2 * TB + TB + (wave + i * NW) * 1024 + lane * 16) = bf16_to_f16(vst[i]);
     }
   };
   // transposing read: lane c of a 16-lane group points at row c >> 2, columns 4 (c & 3) .. + 3 of a 4 x 16 block and
@@ -324,10 +336,11 @@ __global__ __launch_bounds__(kWaves * 64, (kResident<D, WP, DV>)) void prefill_s
     } else {
       if (t + NS - 1 < nt) request(yes, yes, (S + NS - 1) % NS, t + NS - 1);
     }
-    if (t * TK < cnt_wave) load_ka(S * 2 * TB);
+    const int k_wave = 32 * kp, b_wave = k_wave * RB;  // (KP = 2) the wave's first key of the tile
+    if (t * TK + k_wave < cnt_wave) load_ka(S * 2 * TB + b_wave);
 #pragma unroll
-    for (int part = 0; part < TK / 32; part++) {
-      const int k0 = t * TK + 32 * part;
+    for (int part = 0; part < TK / 32 / KP; part++) {
+      const int k0 = t * TK + k_wave + 32 * part;
       if (k0 < cnt_wave) {  // (wave-uniform: else none of the wave's rows sees these keys)
         // S^T = K Q^T: s[qb][kb][j] = score of key k0 + 16 kb + 4 g + j for the lane's query of block qb; a K operand serves all blocks
         // (starting from named zeros: with the zero written into the first product the 128-wide kernel spills 22 registers)
@@ -389,7 +402,7 @@ __global__ __launch_bounds__(kWaves * 64, (kResident<D, WP, DV>)) void prefill_s
         __builtin_amdgcn_sched_barrier(0);
         u32x4 va[VR];  // V operand of block db in va[db % VR]
         auto load_va = [&](int db) __attribute__((always_inline)) {
-          const int at = vaddr_of(db) + S * 2 * TB + 32 * part * RB;
+          const int at = vaddr_of(db) + b_wave + S * 2 * TB + 32 * part * RB;
           const i16x4 xa = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_ptr)at);
           const i16x4 xb = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_ptr)(at + 16 * RB));
           const u32x2 wa = __builtin_bit_cast(u32x2, xa), wb = __builtin_bit_cast(u32x2, xb);
@@ -397,7 +410,7 @@ __global__ __launch_bounds__(kWaves * 64, (kResident<D, WP, DV>)) void prefill_s
         };
 #pragma unroll
         for (int db = 0; db < VR; db++) va[db] = load_va(db);
-        if (32 * (part + 1) < TK) load_ka(S * 2 * TB + 32 * (part + 1) * RB);
+        if (part + 1 < TK / 32 / KP) load_ka(S * 2 * TB + 32 * (part + 1) * RB);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int db = 0; db < NDB; db++) {
@@ -442,6 +455,36 @@ __global__ __launch_bounds__(kWaves * 64, (kResident<D, WP, DV>)) void prefill_s
   char* const o_lds = lds + wave * WP * RBO;
   if (MODE == 1 && nt == 0) wait_loads<0>();  // (else the loop has waited for the old m and l)
   if (TURNED) __syncthreads();                // (the last tile is done with)
+  // KP = 2: every wave leaves the half of O that the other finishes in LDS (the tiles are done with), its maximum and its sums, and joins the
+  // other's with its own half, EDB blocks that are oacc[0][0 .. EDB - 1] from here on, columns from col0.
+  constexpr int EDB = NDB / KP;
+  const int col0 = 16 * EDB * kp;
+  float lse_old = 0.f;  // (MODE 2)
+  if constexpr (KP > 1) {
+    static_assert(NW * EDB * 1024 <= kStateOff, "the tiles' LDS holds the halves");
+    if (MODE == 2) {  // (read before the wave that replaces it may write)
+      lse_old = p.lse[(o_start + (m0 + c < q_len ? m0 + c : m_wg)) * p.hq + h];
+      asm volatile("" ::"v"(lse_old));
+    }
+    const float l_wave = col_sum(l_run[0]);
+    const int other = wave ^ kWaves;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < EDB; i++) {
+      *(f32x4*)(lds + (wave * EDB + i) * 1024 + lane * 16) = kp ? oacc[0][i] : oacc[0][EDB + i];
+      if (kp) oacc[0][i] = oacc[0][EDB + i];
+    }
+    if (g == 0) *(f32x4*)(lds + kJoinOff + wave * 256 + c * 16) = f32x4{m_run[0], l_wave, l_pv[0][0], 0.f};
+    __syncthreads();
+    const f32x4 st = *(const f32x4*)(lds + kJoinOff + other * 256 + c * 16);
+    const float top = fmaxf(m_run[0], st[0]);
+    const float w0 = exp2_diff(m_run[0], top), w1 = exp2_diff(st[0], top);  // (0 for a part that saw no key)
+    l_run[0] = l_wave * w0 + st[1] * w1;
+    l_pv[0][0] = l_pv[0][0] * w0 + st[2] * w1;
+#pragma unroll
+    for (int i = 0; i < EDB; i++) oacc[0][i] = oacc[0][i] * w0 + *(const f32x4*)(lds + (other * EDB + i) * 1024 + lane * 16) * w1;
+    m_run[0] = top;
+  }
   if (m0 >= q_len) return;                    // (wave-uniform: a wave without positions; it only helped to stage)
   // (the lane's numbers are worked out again and not kept over the loop)
   const int lane_e = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), c_e = lane_e & 15, g_e = lane_e >> 4;
@@ -450,7 +493,7 @@ __global__ __launch_bounds__(kWaves * 64, (kResident<D, WP, DV>)) void prefill_s
 #pragma unroll
   for (int qb = 0; qb < QB; qb++) {
     const int mb = m0 + 16 * qb;
-    const float l_tot = col_sum(l_run[qb]);
+    const float l_tot = KP > 1 ? l_run[qb] : col_sum(l_run[qb]);
     // (0 exactly if the row saw no key.  A NaN score makes the sum NaN: it counts as a key, so that the row's outputs and its running
     // state become NaN, as they do in the reference, and no step before or after hides it)
     const bool seen = !(l_tot == 0.f);
@@ -466,11 +509,11 @@ __global__ __launch_bounds__(kWaves * 64, (kResident<D, WP, DV>)) void prefill_s
       factor[qb] = seen ? fix * (1.f / l_tot) : 0.f;
       if (here) {
         if (!TURNED) {
-          float* orow = (float*)p.o + tok * p.o_st + (int64_t)h * p.o_sh + 4 * g_e;
+          float* orow = (float*)p.o + tok * p.o_st + (int64_t)h * p.o_sh + col0 + 4 * g_e;
 #pragma unroll
-          for (int db = 0; db < NDB; db++) *(f32x4*)(orow + 16 * db) = oacc[qb][db] * factor[qb];
+          for (int db = 0; db < EDB; db++) *(f32x4*)(orow + 16 * db) = oacc[qb][db] * factor[qb];
         }
-        if (g_e == 0) p.lse[tok * p.hq + h] = seen ? (m_run[qb] + __builtin_amdgcn_logf(l_tot)) * kLn2 : -INFINITY;
+        if (g_e == 0 && kp == 0) p.lse[tok * p.hq + h] = seen ? (m_run[qb] + __builtin_amdgcn_logf(l_tot)) * kLn2 : -INFINITY;
       }
     }
     if (MODE == 1) {
@@ -483,20 +526,20 @@ __global__ __launch_bounds__(kWaves * 64, (kResident<D, WP, DV>)) void prefill_s
       const float w_new = exp2_diff(m_run[qb], M) * fix;
       const float L = w_old + l_tot * exp2_diff(m_run[qb], M);
       const float inv = 1.f / L;
-      uint16_t* orow = (uint16_t*)p.o + tok * p.o_st + (int64_t)h * p.o_sh + 4 * g_e;
-      u32x2 old[NDB];
+      uint16_t* orow = (uint16_t*)p.o + tok * p.o_st + (int64_t)h * p.o_sh + col0 + 4 * g_e;
+      u32x2 old[EDB];
 #pragma unroll
-      for (int db = 0; db < NDB; db++) old[db] = u32x2{0u, 0u};
+      for (int db = 0; db < EDB; db++) old[db] = u32x2{0u, 0u};
       // (a wave none of whose rows carries an earlier step's result, as in the first step of a ring and in a prefill on one GPU, does not
       // read o; w_old is NaN if an old sum or maximum is)
       if (__builtin_amdgcn_ballot_w64(w_old != 0.f) != 0) {
         if (w_old != 0.f) {
 #pragma unroll
-          for (int db = 0; db < NDB; db++) old[db] = *(const u32x2*)(orow + 16 * db);
+          for (int db = 0; db < EDB; db++) old[db] = *(const u32x2*)(orow + 16 * db);
         }
       }
 #pragma unroll
-      for (int db = 0; db < NDB; db++) {
+      for (int db = 0; db < EDB; db++) {
         float o0, o1, o2, o3;
         unpack2<T>(old[db][0], o0, o1);
         unpack2<T>(old[db][1], o2, o3);
@@ -507,7 +550,7 @@ __global__ __launch_bounds__(kWaves * 64, (kResident<D, WP, DV>)) void prefill_s
         else if (upd) *(u32x2*)(orow + 16 * db) = res;
       }
       rows |= (uint32_t)(__builtin_amdgcn_ballot_w64(upd) & 0xffffu) << 16 * qb;
-      if (upd && g_e == 0) {
+      if (upd && g_e == 0 && kp == 0) {
         p.m[tok * p.ml_st + (int64_t)h * p.ml_sh] = M;
         p.l[tok * p.ml_st + (int64_t)h * p.ml_sh] = L;
       }
@@ -515,7 +558,7 @@ __global__ __launch_bounds__(kWaves * 64, (kResident<D, WP, DV>)) void prefill_s
     if (MODE == 2) {
       // fold the step's partial into the running fp32 (O, LSE); a row that saw no key stays as it is
       const bool upd = here && seen;
-      const float a_old = p.lse[tok * p.hq + h] * kLog2e;
+      const float a_old = (KP > 1 ? lse_old : p.lse[tok * p.hq + h]) * kLog2e;
       float new_lse = 0.f;
       if (upd) {
         const float a_new = m_run[qb] + __builtin_amdgcn_logf(l_tot);
@@ -524,16 +567,16 @@ __global__ __launch_bounds__(kWaves * 64, (kResident<D, WP, DV>)) void prefill_s
         const float w_new = __builtin_amdgcn_exp2f(a_new - top);
         const float W = w_old + w_new;
         const float c_old = w_old / W, c_new = w_new / (W * l_tot) * fix;
-        float* orow = (float*)p.o + tok * p.o_st + (int64_t)h * p.o_sh + 4 * g_e;
+        float* orow = (float*)p.o + tok * p.o_st + (int64_t)h * p.o_sh + col0 + 4 * g_e;
 #pragma unroll
-        for (int db = 0; db < NDB; db++) {
+        for (int db = 0; db < EDB; db++) {
           // an empty row (lse = -inf) may hold anything: its old values are dropped, not multiplied by zero
           const f32x4 keep = w_old != 0.f ? *(const f32x4*)(orow + 16 * db) : f32x4{0.f, 0.f, 0.f, 0.f};
           *(f32x4*)(orow + 16 * db) = keep * c_old + oacc[qb][db] * c_new;
         }
         new_lse = (top + __builtin_amdgcn_logf(W)) * kLn2;
       }
-      if (upd && g_e == 0) p.lse[tok * p.hq + h] = new_lse;
+      if (upd && g_e == 0 && kp == 0) p.lse[tok * p.hq + h] = new_lse;
     }
   }
   if (TURNED) {
@@ -646,7 +689,7 @@ Order order_of(const lsattn_prefill_args* a, int pack_shift) {
   return {bunch, requests_take_turns(a, ids * bunch, tiles)};
 }
 
-template <typename T, int D, int MODE, bool DV, int WP> int launch_rows(SmallParams p, const lsattn_prefill_args* a, hipStream_t st) {
+template <typename T, int D, int MODE, bool DV, int WP, int KP = 1> int launch_rows(SmallParams p, const lsattn_prefill_args* a, hipStream_t st) {
   const int64_t rows_wg = (kWaves * WP) >> p.pack_shift;
   const Order order = WP == 32 ? order_of(a, p.pack_shift) : Order{p.batch, false};
   p.bunch = (int32_t)order.bunch;
@@ -656,12 +699,29 @@ template <typename T, int D, int MODE, bool DV, int WP> int launch_rows(SmallPar
   const unsigned bunches = (unsigned)((a->batch + p.bunch - 1) / p.bunch);
   for (int64_t tiles = (a->max_q_len + rows_wg - 1) / rows_wg; tiles > 0; tiles -= most) {
     p.last_tile = (int32_t)(tiles - 1);
-    LSATTN_LAUNCH_KERNEL((prefill_small_kernel<T, D, MODE, DV, WP>),
-                         dim3((unsigned)(p.hkv * p.group), (unsigned)((tiles < most ? tiles : most) * p.bunch), bunches), dim3(kWaves * 64), 0, st, p);
+    LSATTN_LAUNCH_KERNEL((prefill_small_kernel<T, D, MODE, DV, WP, KP>),
+                         dim3((unsigned)(p.hkv * p.group), (unsigned)((tiles < most ? tiles : most) * p.bunch), bunches), dim3(kWaves * KP * 64), 0, st, p);
     const int rc = check_launch();
     if (rc != LSATTN_OK) return rc;
   }
   return LSATTN_OK;
+}
+
+// The most keys a request can have, as far as the host can tell: what the K buffer holds beyond the query rows may all belong to one request, unless the
+// caller bounds the lengths.  kUnknownKeys: nothing is known.
+constexpr int64_t kUnknownKeys = INT64_MAX;
+int64_t longest_keys(const lsattn_prefill_args* a) {
+  int64_t longest = kUnknownKeys;
+  if (a->total_kv_rows > 0) {
+    longest = a->total_kv_rows;
+    if (a->total_q_rows > 0) {
+      const int64_t most = (int64_t)a->batch * a->max_q_len, rows = a->total_q_rows < most ? a->total_q_rows : most;
+      const int64_t beyond = a->total_kv_rows > rows ? a->total_kv_rows - rows : 0;
+      if (a->max_q_len + beyond < longest) longest = a->max_q_len + beyond;
+    }
+  }
+  if (a->max_kv_len > 0 && a->max_kv_len < longest) longest = a->max_kv_len;
+  return longest;
 }
 
 // 32 positions per wave serve twice the rows with each K and V operand read, 16 make twice as many, shorter waves: these from
@@ -678,7 +738,9 @@ template <typename T, int D, int MODE, bool DV> int launch(const SmallParams& p,
 
 template <typename T, int MODE, bool DV> int launch_128(const SmallParams& p, const lsattn_prefill_args* a, hipStream_t st) {
   switch (prefill_small_route(a)) {
-    case LSATTN_ROUTE_SMALL_16: return launch_rows<T, 128, MODE, DV, 16>(p, a, st);
+    case LSATTN_ROUTE_SMALL_16:
+      if (workgroups(a, pack_shift_of(a), 1) <= kCUs && longest_keys(a) >= kPartsMinKeys) return launch_rows<T, 128, MODE, DV, 16, 2>(p, a, st);
+      return launch_rows<T, 128, MODE, DV, 16>(p, a, st);
     default: return launch_rows<T, 128, MODE, DV, 32>(p, a, st);
   }
 }
@@ -720,9 +782,11 @@ template <typename T, bool DV> int launch_mode(const SmallParams& p, const lsatt
 // 100 stay below the figure in brackets), to so much of the time before this kernel, prompts, then full steps:
 //   up to 768 rows 0.79 (0.97), 0.91 (1.16)     769 to 1024 0.85 (0.99), 1.03 (1.25)     1025 to 1280 0.88 (1.02), 1.01 (1.12)
 // so the rule goes by the prompts up to 1024 rows and from there on takes what a ring's shards bear too; past 1280 that is one f16 prompt, up to
-// 1472 rows, in the in-place epilogue, with 16 positions: with one head per workgroup the third workgroup per CU, 0.78 to 0.91 and full steps 0.97 to 1.08
-// (1410 tokens 32/32 37.9 -> 31.3 us); up to one per CU 0.92 to 0.95 and 0.90 to 0.95.  (1536 rows 0.89 to 0.95 and 1.06 to 1.12, the partial 0.87 to 1.01 and
-// 1.06 to 1.12: not taken.)
+// 1472 rows, in the in-place epilogue, with 16 positions and one head per workgroup: the third workgroup per CU, 0.78 to 0.91 and full steps 0.97 to 1.08
+// (1410 tokens 32/32 37.9 -> 31.3 us; 1536 rows 0.89 to 0.95 and 1.06 to 1.12, the partial 0.87 to 1.01 and 1.06 to 1.12: not taken).
+//   One request folded in place in up to a workgroup per CU, where two waves share each tile: up to 2304 keys, bf16 2048, prompts, full steps and chunks
+// behind a context alike 0.77 to 0.98 of the other kernel (us: 8/1 1450 tokens 28.5 | 21.5, 2040 32.3 | 27.2, bf16 1100 25.5 | 20.3, 1850 33.0 | 29.8; 200 rows behind 1024 keys 32/8
+// 24.2 | 19.1, 300 behind 2000 36.0 | 31.2; past that f16 0.89 to 1.03, bf16 1.00 to 1.13).
 //   16 positions: up to three workgroups per CU (two and a half of a ragged batch; with one head per workgroup, which leaves each wave fewer
 // rows to mask, four and six), past 768 rows up to one, and the third, where workgroups of 128 rows would run a second round with a few of them (a ragged batch
 // only with one head per workgroup: a lone long request between short ones came to up to 1.6 of the other kernel's time).  Past 1024 rows
@@ -736,32 +800,23 @@ template <typename T, bool DV> int launch_mode(const SmallParams& p, const lsatt
 //   2 x 100, one behind 1900 30.6 | 31.8, 34.5 | 39.8      8 x 64, one behind 7500 79.8 | 108.8, 88 | 169      16 x 64, one behind 15000 145 | 264, 155 | 352
 // The host knows no lengths, only bounds: what total_kv_rows holds beyond the query rows may all belong to one request.
 int prefill_short_blocks(const lsattn_prefill_args* a) {
-  if (a->head_dim != 128 || a->kv_cuts > 1 || a->o_b_start_loc || a->max_q_len <= 0 || a->max_q_len > kLoneMaxKeys || a->batch <= 0 || a->batch > kMaxIds || a->num_kv_heads <= 0)
+  if (a->head_dim != 128 || a->kv_cuts > 1 || a->o_b_start_loc || a->max_q_len <= 0 || a->max_q_len > kPartsMaxKeys || a->batch <= 0 || a->batch > kMaxIds || a->num_kv_heads <= 0)
     return 0;
-  int64_t longest = kLoneMaxKeys + 1;
-  if (a->total_kv_rows > 0) {
-    longest = a->total_kv_rows;
-    if (a->total_q_rows > 0) {
-      const int64_t most = (int64_t)a->batch * a->max_q_len, rows = a->total_q_rows < most ? a->total_q_rows : most;
-      const int64_t beyond = a->total_kv_rows > rows ? a->total_kv_rows - rows : 0;
-      if (a->max_q_len + beyond < longest) longest = a->max_q_len + beyond;
-    }
-  }
-  if (a->max_kv_len > 0 && a->max_kv_len < longest) longest = a->max_kv_len;
-  if (longest > kLoneMaxKeys) return 0;
+  const int64_t longest = longest_keys(a);
+  if (longest > kPartsMaxKeys) return 0;
   const Tuning tn = tuning();
   if (tn.prefill_rows || tn.prefill_order || tn.prefill_pack) return 0;  // (choices among the 128-wide kernel's shapes)
   const int pack = pack_shift_of(a);
   const int64_t one = workgroups(a, pack, 1), two = workgroups(a, pack, 2);
   const bool f16 = a->dtype == LSATTN_F16, rag = ragged(a);
+  // (m: of the three steps only the in-place one has it)
+  if (a->batch == 1 && a->m && one <= kCUs && longest >= kPartsMinKeys && longest <= (f16 ? kPartsMaxKeys : kPartsMaxKeysBf16)) return 1;
+  if (longest > kShortMaxKeys || a->max_q_len > kShortMaxKeys)
+    return f16 && a->m && a->batch == 1 && a->max_q_len == longest && longest <= kLoneMaxKeys && pack == 0 && one > 2 * kCUs && one <= 3 * kCUs;
   if (a->max_q_len <= 768) return longest > 1024 ? 0 : 2 * one <= (pack ? rag ? 5 : 6 : rag ? 12 : 8) * kCUs ? 1 : 2;
-  if (longest > kShortMaxKeys || a->max_q_len > kShortMaxKeys) {
-    if (a->batch > 1 || a->max_q_len != longest) return 0;
-    return f16 && a->m && (one <= kCUs || (pack == 0 && one > 2 * kCUs && one <= 3 * kCUs));
-  }
   const bool past = longest > 1024;
   if (one <= kCUs) return !past || (f16 && a->batch == 1) ? 1 : 0;
-  // (m: of the three steps only the in-place one has it.  bf16 does not look at it: whether V is to be copied is asked before)
+  // (otherwise bf16 does not look at m: whether V is to be copied may be asked without it)
   if (one > 2 * kCUs && one <= 3 * kCUs && (past ? !rag && (f16 ? a->m != nullptr : pack == 0) : !rag || pack == 0)) return 1;
   if (past) return two > (rag ? 5 : 4) * kCUs && (rag || two <= 10 * kCUs) ? 2 : 0;
   return 2 * two >= (rag ? 7 : 6) * kCUs ? 2 : 0;

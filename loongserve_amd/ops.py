@@ -290,7 +290,7 @@ def context_attention_fwd(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first_token_
     is the reference's: one launch, no scratch.  (m, l) stay opaque: a step folded this way enters as (its LSE, 1).
 
     Keyword-only: max_kv_len also tells a batch of short chunks behind short contexts from one with a long context among them; up to
-    1280 keys a kernel of shorter workgroups may run (without it only where the rows of k and total_q_len, or the rows of k alone, prove as much).
+    1280 keys, for one request of few rows up to 2304, a kernel of shorter workgroups may run (without it only where the rows of k and total_q_len, or the rows of k alone, prove as much).
 
     Keyword-only, for batches that mix long and short requests: total_q_len, an upper bound of the sum of q_b_seq_len
     (q.shape[0] when q is packed and no two sequences share rows).  The launch is sized by max_q_b_seq_len times the batch

@@ -511,17 +511,20 @@ def test_prefill_route_names_a_kernel_for_every_step_and_none_for_others():
 
 
 def test_lone_prompts_past_1280_rows_fold_in_the_short_prompts_kernel():
-    """One f16 prompt of up to 1472 rows in the in-place epilogue, up to one workgroup of 64 rows per CU or, with a head each, in the third.
-    Not behind a context, against fewer keys, or beside another request."""
+    """One f16 prompt of up to 1472 rows in the in-place epilogue with a head per workgroup, in the third workgroup of 64 rows per CU; up to one per
+    CU, where two waves share a tile, any request of 512 to 2304 keys (bf16 2048).  Nothing else past 1280, or beside another request."""
     lone = lambda n, heads, kv=None, **kw: _route(1, n, heads, total_q=n, total_kv=kv or n, **kw)
+    bf16 = dict(dtype=1, v_is_f16=1, m=256)
     for n in (1281, 1410, 1472):
-        assert lone(n, (8, 1), m=256) == lone(n, (32, 32), m=256) == SMALL_16
-        assert lone(n, (32, 32)) == lone(n, (8, 1)) == ROWS_128 and lone(n, (8, 1), dtype=1, v_is_f16=1, m=256) == ROWS_128
-        assert lone(n, (32, 32), dtype=1, v_is_f16=1, m=256) == lone(n, (32, 8), m=256) == ROWS_128
+        assert lone(n, (32, 32), m=256) == SMALL_16 and lone(n, (32, 32)) == lone(n, (8, 1)) == ROWS_128
+        assert lone(n, (32, 32), **bf16) == lone(n, (32, 8), m=256) == ROWS_128
         assert lone(n, (32, 32), kv=n + 1, m=256) == lone(n, (32, 32), kv=1000, m=256) == ROWS_128
         assert _route(2, n, (32, 32), total_q=2 * n, total_kv=2 * n, m=256) not in (SMALL_16, SMALL_32)
-    assert lone(1473, (32, 32), m=256) == lone(1473, (8, 1), m=256) == ROWS_128
-    assert lone(1300, (20, 20), m=256) == ROWS_128  # (1.6 workgroups of 64 rows per CU)
+    assert lone(1473, (32, 32), m=256) == lone(1300, (20, 20), m=256) == ROWS_128  # (1.6 workgroups of 64 rows per CU)
+    assert lone(2048, (8, 1), m=256) == lone(2304, (4, 1), m=256) == SMALL_16 and lone(2049, (8, 1), m=256) == lone(2305, (4, 1), m=256) == ROWS_128
+    assert lone(1025, (8, 1), **bf16) == lone(2048, (8, 1), **bf16) == SMALL_16 and lone(2049, (4, 1), **bf16) == lone(1025, (8, 1), dtype=1, v_is_f16=1) == ROWS_128
+    assert lone(200, (32, 8), kv=1224, m=256) == lone(200, (32, 8), kv=2304, m=256) == SMALL_16
+    assert lone(200, (32, 8), kv=2305, m=256) == lone(200, (32, 8), kv=1224) == _route(2, 100, (32, 8), total_q=200, total_kv=1224, m=256) == ROWS_128
 
 
 def test_lone_prompts_of_a_few_workgroups_past_two_per_cu():

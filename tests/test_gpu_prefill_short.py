@@ -199,3 +199,39 @@ def test_lone_prompts_past_1280_rows(lsa, Hq, Hkv):
     """The longest prompt that the kernel folds in place.  (The route that is asked for names no m: it is the 128-row one of the partial.)"""
     print("case", Hq, Hkv, flush=True)
     _every_epilogue_on(5, lsa, "in_place", "f16", 128, Hq, Hkv, [1472], [0])
+
+
+@pytest.mark.parametrize("mode", ["partial", "accumulate", "in_place"])
+@pytest.mark.parametrize("V", ["f16", "bf16", "bf16 copied"])
+@pytest.mark.parametrize("Hq,Hkv,lens,ctx", [(8, 2, [545, 33, 512], [0, 0, 0]), (8, 1, [640, 1, 31], [0, 300, 0]), (20, 20, [768], [0]), (6, 3, [577, 64], [33, 100])])
+def test_two_waves_that_share_a_tile(lsa, mode, V, Hq, Hkv, lens, ctx):
+    """Up to a workgroup of 64 rows per CU from 512 keys on: one, two and four heads side by side, waves that see one part of a tile or none."""
+    print("case", mode, V, Hq, Hkv, lens, flush=True)
+    _every_epilogue_on(SMALL_16, lsa, mode, V, 128, Hq, Hkv, lens, ctx)
+
+
+@pytest.mark.parametrize("V", ["f16", "bf16 copied"])
+@pytest.mark.parametrize("Hq,Hkv,n,ctx", [(8, 1, 2048, 0), (4, 4, 1025, 0), (32, 8, 200, 1848), (12, 4, 77, 1300)])
+def test_lone_requests_whose_tiles_two_waves_share(lsa, V, Hq, Hkv, n, ctx):
+    """One request folded in place, past what other steps bring to the kernel (the route asked for here names no m: it is the 128-wide kernel's)."""
+    print("case", V, Hq, Hkv, n, ctx, flush=True)
+    _every_epilogue_on(SMALL_16 if n == 1025 and V == "f16" else 5, lsa, "in_place", V, 128, Hq, Hkv, [n], [ctx])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("key", [0, 31, 40, 575])
+def test_nan_keys_in_either_part_of_a_tile(lsa, dtype, key):
+    """A NaN in one K row of a prompt whose tiles two waves share: the rows that see it become NaN, the others stay."""
+    print("case", dtype, key, flush=True)
+    n, Hq, Hkv = 600, 8, 2
+    q, k, v = _dev(*(rand_t((n, h, 128), 91 + i, dtype) for i, h in enumerate((Hq, Hkv, Hkv))))
+    md = _dev(*meta([n]))
+    want, want_lse = lsa.prefill_attention_step(q, k, v, *md, *md, 1, n, total_q_len=n)
+    k[key, 1, 5] = float("nan")
+    got, lse = lsa.prefill_attention_step(q, k, v, *md, *md, 1, n, total_q_len=n)
+    hit = torch.zeros((n, Hq), dtype=torch.bool, device=DEV)
+    hit[key:, Hq // 2:] = True
+    assert torch.equal(got.isnan().all(-1), hit) and torch.equal(got.isnan().any(-1), hit) and torch.equal(lse.isnan(), hit)
+    # (a NaN makes a wave raise all its maxima, which moves its other rows by the rounding of their weights to fp16)
+    assert_o_close(got[~hit].cpu(), want[~hit].cpu(), "O")
+    assert_lse_close(lse[~hit].cpu(), want_lse[~hit].cpu(), "LSE")
