@@ -724,6 +724,18 @@ int64_t longest_keys(const lsattn_prefill_args* a) {
   return longest;
 }
 
+// Whether two waves share a wave's positions (KP = 2) in a launch of 64-wide heads with 16 positions per wave.  A wave has fewer products between its
+// waits here, so this gains with several workgroups on a CU too, the later the more there are.  Of the time of one wave each, over 270 launches (1 to 8 prompts of 150 to
+// 2500 tokens; 32/32, 32/8, 64/8, 16/16 and 8/1 heads, f16 and bf16, partials and in place), by the longest prompt:
+//   up to one per CU   below 300 1.01   300 to 450 0.97   to 600 0.93   to 800 0.90   to 1100 0.88   to 2500 0.84 (1700 tokens 32/8 bf16 27.4 -> 23.2 us)
+//   up to two          below 300 1.11   300 to 600 1.00   to 800 0.93   to 1100 0.90   to 2500 0.85      up to three   below 1100 1.02 to 1.15   to 1500 0.93   to 2500 0.89
+// and past that 0.99 to 1.21.
+bool parts_64(const lsattn_prefill_args* a) {
+  const int64_t one = workgroups(a, pack_shift_of(a), 1), longest = longest_keys(a);
+  if (one <= kCUs) return (longest == kUnknownKeys ? a->max_q_len : longest) >= 448;
+  return one <= 2 * kCUs ? a->max_q_len >= 640 : one <= 3 * kCUs && a->max_q_len >= 1152;
+}
+
 // 32 positions per wave serve twice the rows with each K and V operand read, 16 make twice as many, shorter waves: these from
 // three workgroups of the larger shape per CU down, where the launch is as long as its longest wave.  Measured at 64-wide heads
 // (32 | 16 positions, without the sum of the fp16 weights, which costs both 4 to 8 %): 256 workgroups 21.5 | 16.2 us, 512 24.9 | 20.4 and 40.3 | 32.6, 768 30.4 | 31.4, 1024 36.6 | 35.7 and
@@ -731,7 +743,10 @@ int64_t longest_keys(const lsattn_prefill_args* a) {
 template <typename T, int D, int MODE, bool DV> int launch(const SmallParams& p, const lsattn_prefill_args* a, hipStream_t st) {
   if (a->num_q_heads > 65535 || a->batch > 65535) return LSATTN_ERR_INVALID_ARG;
   switch (prefill_small_route(a)) {
-    case LSATTN_ROUTE_SMALL_16: return launch_rows<T, D, MODE, DV, 16>(p, a, st);
+    case LSATTN_ROUTE_SMALL_16:
+      if constexpr (D == 64)
+        if (parts_64(a)) return launch_rows<T, 64, MODE, DV, 16, 2>(p, a, st);
+      return launch_rows<T, D, MODE, DV, 16>(p, a, st);
     default: return launch_rows<T, D, MODE, DV, 32>(p, a, st);
   }
 }

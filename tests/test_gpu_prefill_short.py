@@ -235,3 +235,12 @@ def test_nan_keys_in_either_part_of_a_tile(lsa, dtype, key):
     # (a NaN makes a wave raise all its maxima, which moves its other rows by the rounding of their weights to fp16)
     assert_o_close(got[~hit].cpu(), want[~hit].cpu(), "O")
     assert_lse_close(lse[~hit].cpu(), want_lse[~hit].cpu(), "LSE")
+
+
+@pytest.mark.parametrize("mode", ["partial", "accumulate", "in_place"])
+@pytest.mark.parametrize("V", ["f16", "bf16", "bf16 copied"])
+@pytest.mark.parametrize("Hq,Hkv,lens,ctx", [(8, 2, [449, 33, 448], [0, 0, 0]), (4, 1, [50, 1], [0, 600]), (32, 16, [1000, 650], [0, 0]), (20, 20, [1153, 1], [0, 0])])
+def test_two_waves_that_share_a_tile_of_64_wide_heads(lsa, mode, V, Hq, Hkv, lens, ctx):
+    """One, two and three workgroups per CU, one, two and four heads side by side."""
+    print("case", mode, V, Hq, Hkv, lens, flush=True)
+    _every_epilogue_on(SMALL_16, lsa, mode, V, 64, Hq, Hkv, lens, ctx)
