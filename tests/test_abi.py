@@ -539,6 +539,16 @@ def test_lone_prompts_of_a_few_workgroups_past_two_per_cu():
     assert _route(1, 2500, (32, 8), total_q=2500, total_kv=2600, m=256) == ROWS_256 and _route(2, 1250, (32, 8), total_q=2500, total_kv=2500, m=256) != HALF
 
 
+def test_equal_prompts_fill_a_third_workgroup_per_cu():
+    """Equal f16 requests in place: 769 to 1024 rows from two workgroups of 32 positions per CU on, up to 1280 from 2.6 on, up to three."""
+    step = lambda b, n, heads, m=256, total=None, **kw: _route(b, n, heads, total_q=total or b * n, total_kv=total or b * n, m=m, **kw)
+    assert step(9, 1024, (8, 8)) == step(10, 769, (8, 8)) == SMALL_32 and step(8, 1024, (8, 8)) == ROWS_256  # (576, 560, 512)
+    assert step(9, 1280, (8, 8)) == SMALL_32 and step(8, 1280, (8, 8)) == ROWS_256  # (720, 640)
+    assert step(10, 1280, (8, 8)) != SMALL_32 and step(9, 1281, (8, 8)) != SMALL_32  # (800)
+    assert step(9, 1024, (8, 8), m=None) == step(9, 1024, (8, 8), dtype=1) == ROWS_256
+    assert step(9, 1024, (8, 8), total=8294) != SMALL_32  # (nine tenths of 9216)
+
+
 def test_ragged_batches_folded_in_place_by_four_waves():
     """Ragged requests of up to 2048 rows against as many keys, from a workgroup of 128 rows per CU on (three halves where it would be the split shape's)."""
     step = lambda n, total, heads=(32, 8), m=256, **kw: _route(4, n, heads, total_q=total, total_kv=kw.pop("total_kv", total), m=m, **kw)

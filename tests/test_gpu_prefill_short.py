@@ -218,6 +218,13 @@ def test_lone_requests_whose_tiles_two_waves_share(lsa, V, Hq, Hkv, n, ctx):
     _every_epilogue_on(SMALL_16 if n == 1025 and V == "f16" else 5, lsa, "in_place", V, 128, Hq, Hkv, [n], [ctx])
 
 
+@pytest.mark.parametrize("Hq,Hkv,lens", [(8, 8, [801] * 10), (8, 1, [1280] * 9), (18, 6, [1024] * 4)])
+def test_equal_prompts_in_place_with_a_third_workgroup_per_cu(lsa, Hq, Hkv, lens):
+    """Between two and three workgroups of 32 positions per CU (the route asked for here names no m: it is the 128-wide kernel's)."""
+    print("case", Hq, Hkv, lens, flush=True)
+    _every_epilogue_on(4, lsa, "in_place", "f16", 128, Hq, Hkv, lens, [0] * len(lens))
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("key", [0, 31, 40, 575])
 def test_nan_keys_in_either_part_of_a_tile(lsa, dtype, key):
