@@ -1654,6 +1654,10 @@ template <typename T> static int launch_stage1_mfma(const lsattn_decode_stage1_a
                        (group >= 4 && p.tasks == 1 && a->batch >= 4 && waves256 > 4 * kCUs && waves256 <= 5 * kCUs);
     const bool few = a->batch < kSharesMinBatch && waves256 < kSharesMinWavesFew, nearly_two = group < 4 && waves256 > 6 * kCUs && waves256 < 8 * kCUs;
     if (!forced && (!large || few || (a->batch < 2 && (p.tasks < 4 || nearly_two)))) return LSATTN_OK;
+    // bf16 launches that the lane kernel would take (in blocks as coarse as the split asked for they may be few waves): it multiplies V by fp32 weights, this
+    // kernel by two bf16 parts of them (error against 64 bits 4e-7 | 4.8e-6: two of 131870 tokens, 2/1 heads; one of 65936, 10/5).  So only the large ones.
+    const bool lane = std::is_same<T, BF16>::value && !use && !split_waves;
+    if (!forced && lane && (a->batch < 2 || (a->batch < kSharesMinBatch && waves256 < 8 * kCUs) || (group >= 4 && p.tasks < 4 && waves256 <= 12 * kCUs))) return LSATTN_OK;
     // Short contexts, whose rows hold too few shares (a longest request of up to 256 tokens one share, whatever the batch),
     // and grids of one round of workgroups, see kSharesOneRoundBatch.
     const int64_t wgs = wgs_x * wgs_y * a->batch;

@@ -1043,3 +1043,40 @@ def test_both_stages_of_launches_just_past_a_workgroup_per_cu(lsa, dtype, Hq, Hk
     live = b_len > 0
     assert_o_close(o.cpu()[live], o_ref[live], "o")
     assert_lse_close(l.cpu()[live], l_ref[live], "lse")
+
+
+def _against_64_bits(o, q, kv, table, b_req, lens, Hkv):
+    """Relative error of the decode result o against the same in 64 bits, over all requests and heads."""
+    off = norm = 0.0
+    for b, n in enumerate(lens):
+        rows = kv[table[b_req[b].long(), :n].long()]
+        for h in range(q.shape[1]):
+            kvh = h * Hkv // q.shape[1]
+            w = torch.softmax(rows[:, kvh].double() @ q[b, h].double() / math.sqrt(128), 0)
+            ref = w @ rows[:, Hkv + kvh].double()
+            off += float((o[b, h].double() - ref).square().sum())
+            norm += float(ref.square().sum())
+    return math.sqrt(off / norm)
+
+
+@pytest.mark.parametrize("Hq,Hkv,lens,BS", [(1, 1, [131870] * 2, 256), (3, 1, [87914, 87914, 300], 256), (2, 1, [65936] * 4, 256), (10, 5, [65936], 256),
+                                            (32, 32, [16384], 1024), (16, 4, [60000] * 2, 1056)])
+def test_long_contexts_in_bf16_keep_the_weights_in_full(lsa, Hq, Hkv, lens, BS):
+    """Few coarse blocks of contexts long enough for equal shares: the weights that multiply V stay fp32.  In two bf16 parts they have 16 bits, a rounding of
+    2^-17 / sqrt(3) = 4.4e-6 each, and the result's relative error is that of its weights; in full what is left are fp32's own roundings, below a tenth of that."""
+    print("case", Hq, Hkv, lens, BS, flush=True)
+    B, D = len(lens), 128
+    g = torch.Generator(device=DEV).manual_seed(5)
+    q = torch.empty(B, Hq, D, dtype=torch.bfloat16, device=DEV).normal_(0.0, 0.5, generator=g)
+    kv = torch.empty(sum(lens) + 100, 2 * Hkv, D, dtype=torch.bfloat16, device=DEV).normal_(0.0, 0.5, generator=g)
+    slots = torch.randperm(kv.shape[0], generator=g, device=DEV).int()
+    table, at = torch.zeros(B, max(lens), dtype=torch.int32, device=DEV), 0
+    for b, n in enumerate(lens):
+        table[b, :n] = slots[at:at + n]
+        at += n
+    b_len, b_req = torch.tensor(lens, dtype=torch.int32, device=DEV), torch.arange(B, dtype=torch.int32, device=DEV)
+    mo = torch.empty(max(lens) // BS + 1, B, Hq, D, device=DEV)
+    ml = torch.empty(mo.shape[:3], device=DEV)
+    o, _ = lsa.longserve_token_decode_attention_flash_decoding(q, table, b_req, b_len, mo, ml, B, max(lens), Hq, D, kv[:, :Hkv], kv[:, Hkv:], BS)
+    torch.cuda.synchronize()
+    assert _against_64_bits(o, q, kv, table, b_req, lens, Hkv) < 2.0 ** -19
