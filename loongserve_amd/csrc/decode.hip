@@ -1625,11 +1625,10 @@ template <typename T> static int launch_stage1_mfma(const lsattn_decode_stage1_a
   //   smaller groups (most of an MFMA's sixteen columns idle): the plain shape from 768 waves, below that the lane kernel.
   const int64_t waves = chunks * p.tasks * a->batch;
   const bool can_split = p.block_seq % (kMfmaWaves * kMfmaBatch) == 0 && nblk <= 0x7fffffff;
-  //   Of the plain shape's workgroups a few more than one per CU leave the CUs with two to set the time; the shape that splits a block has four
-  //     times as many.  1025 to 1536 waves on four and more KV heads, 40 launches of both stages at 256 tokens a block: one length 0.86 to 0.98 of the plain
-  //     shape's time, others 0.68 to 1.10, in the mean 0.86; from there to 2048 one length 0.97 to 1.10, not taken.  (The fused call deals these in equal shares.)
-  const bool past_round = can_split && p.tasks >= 4 && waves > 4 * kCUs && waves <= 6 * kCUs;
-  bool split_waves = past_round || (group >= 4 && can_split && waves <= (p.tasks < 4 ? 3072 : kSplitMaxWaves));
+  //   (A few more of the plain shape's workgroups than one per CU, 1025 to 1536 waves on four and more KV heads, split among a block's waves, 1200 launches of both stages
+  //     at 256 tokens a block: 0.53 to 1.0 of the time where the lengths differ and some CUs held two, but up to 1.23 where few enough workgroups found tokens, and 1.06 to 1.21 for one
+  //     request on 16 or 32 KV heads.  The host cannot tell them apart: not taken.)
+  bool split_waves = group >= 4 && can_split && waves <= (p.tasks < 4 ? 3072 : kSplitMaxWaves);
   bool use = !split_waves && waves >= (group >= 4 ? 513 : 768);
   const Tuning tn = tuning();  // (lsattn_set_tuning: tuning and tests)
   if (tn.decode_stage1 == LSATTN_DECODE_STAGE1_LANE) use = split_waves = false;

@@ -1080,3 +1080,28 @@ def test_long_contexts_in_bf16_keep_the_weights_in_full(lsa, Hq, Hkv, lens, BS):
     o, _ = lsa.longserve_token_decode_attention_flash_decoding(q, table, b_req, b_len, mo, ml, B, max(lens), Hq, D, kv[:, :Hkv], kv[:, Hkv:], BS)
     torch.cuda.synchronize()
     assert _against_64_bits(o, q, kv, table, b_req, lens, Hkv) < 2.0 ** -19
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Hq,Hkv,lens", [(16, 16, [3328, 900, 2000, 40, 2700]), (32, 32, [8448]), (32, 8, [33 * 256, 300, 0, 4000])])
+def test_stage1_just_past_a_workgroup_per_cu_runs_the_plain_shape(lsa, tuning, dtype, Hq, Hkv, lens):
+    """1040 to 1056 waves, where the shape whose waves split a block takes up to a fifth longer: the partials are the plain shape's, bit for bit."""
+    print("case", dtype, Hq, Hkv, lens, flush=True)
+    B, BS = len(lens), 256
+    q, kv, table, b_req, b_len = decode_case(78, B, Hq, Hkv, 128, lens, sum(lens) + 500, dtype)
+    qd, kvd, td, rd, ld = q.to(DEV), kv.to(DEV), table.to(DEV), b_req.to(DEV), b_len.to(DEV)
+    nblk = (max(lens) + BS - 1) // BS
+
+    def partials():
+        mo, ml = torch.zeros((nblk, B, Hq, 128), device=DEV), torch.zeros((nblk, B, Hq), device=DEV)
+        lsa.longserve_flash_decode_stage1(qd, kvd[:, :Hkv], kvd[:, Hkv:], td, rd, ld, max(lens), mo, ml, BS)
+        torch.cuda.synchronize()
+        return mo, ml
+
+    got = partials()
+    tuning(decode_stage1="mfma")
+    want = partials()
+    tuning(decode_stage1="split")
+    other = partials()
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    assert not torch.equal(other[0], want[0])  # (the two shapes can be told apart)
