@@ -1093,15 +1093,16 @@ constexpr int64_t kListedFromWorkgroups = 32768;  // launches of the plain grid 
 // list costs an even batch more than that (config 3, 16384 workgroups: 947 -> 962 us) and stays with the larger grids.
 constexpr int64_t kListedFromWorkgroupsCoarse = 8192;
 constexpr int64_t kListedCoarseTokens = 1024;
-// Equal shares from eight requests on wherever the plain shape would run, and for fewer, down to one, where the grid has more than a
-// workgroup per CU (1024 waves of 256 tokens): up to two, the CUs that hold two set its time, and a split of other sizes has as many.  Below that a few even
-// requests take 1.02 to 1.21 of the grid's time by shares.  Four and more KV heads, of the time of the grids, 180 launches: one request 0.73 to 0.99 (groups
-// below four, which keep the grid where it has nearly two workgroups per CU, to 1.05 there), two to seven of one length 0.83 to 1.08, of other lengths 0.63 to 1.06.
-//   (us: 1 x 35000 tokens 32/8 36 | 30, 1 x 66000 64/8 67 | 52; 3 x 14906 at most 32/8 32.3 | 24.9; 7 x 5387 at most 16/8 26.6 | 17.6; 2 x 24335 32/8 43.5 | 39.2)
+// Equal shares from eight requests on wherever the plain shape would run, and for fewer from 2048 waves of 256 tokens on, two workgroups per CU.  Of less than two,
+// where the CUs that hold two set the grid's time, those that gain whatever the lengths are (of the time of the grids, 3400 launches on four and more KV heads):
+//   two to seven requests, 1345 to 1536 waves: of one length 0.87 to 1.01, of others 0.58 to 0.97 (us, 32/8: 5 x 8860 40.0 | 38.1, 4 of at most 11264 31.4 | 24.5).  Below that one length gains more (0.81 to 0.95) but ragged ones
+//     of which few enough workgroups find tokens take up to 1.13 (6 of at most 6044 16/8 22.3 | 24.3), above it one length takes up to 1.09 (4 x 13569 8/8 42.5 | 44.8)
+//   one request from 1025 waves on 0.74 to 0.99 (35000 tokens 32/8 36 | 30, 66000 64/8 67 | 52), except where the grid has nearly two workgroups per CU, to 1.12 (groups below four
+//     from one and a half on), and there also nearly four, to 1.04
 // Fewer than four KV heads, where a grid of the shape whose waves split a block stands against it, from more than 2048 waves on (four rounds of
 // two workgroups per CU) 0.57 to 1.10, in the mean 0.92, and with one KV head and four requests and more also in the first fourth of the third round 0.67 to
 // 1.03, 0.84 (8 requests, one of 33819 tokens, 16/1 27.5 | 18.4 us; three with one of 107373 23.6 | 31.8, not taken); in between one length loses up to 16 %.
-constexpr int64_t kSharesMinBatch = 8, kSharesMinWavesFew = 1025, kSharesMinWavesFewHeads = 2049;
+constexpr int64_t kSharesMinBatch = 8, kSharesMinWavesFewHeads = 2049;
 // Not where the rows of the partials' buffers hold less than half of the shares the chip has waves for: 256 requests of 256 tokens,
 // GQA 32/8, are one share (2.9 ms) or a grid (57 us).  And not in place of a grid that one round of workgroups, one per CU, walks,
 // if the rows hold fewer shares than the chip has waves for (24 requests of 1024 tokens, GQA 32/8, 73 shares: 30.1 us against 22.6; 33 of
@@ -1651,8 +1652,10 @@ template <typename T> static int launch_stage1_mfma(const lsattn_decode_stage1_a
     const int64_t waves256 = (shares->units * kMfmaBatch + 255) / 256 * p.tasks * a->batch;
     const bool large = waves256 >= (group < 4 ? 768 : p.tasks < 4 ? kSharesMinWavesFewHeads : kSplitMaxWaves + 1) ||
                        (group >= 4 && p.tasks == 1 && a->batch >= 4 && waves256 > 4 * kCUs && waves256 <= 5 * kCUs);
-    const bool few = a->batch < kSharesMinBatch && waves256 < kSharesMinWavesFew, nearly_two = group < 4 && waves256 > 6 * kCUs && waves256 < 8 * kCUs;
-    if (!forced && (!large || few || (a->batch < 2 && (p.tasks < 4 || nearly_two)))) return LSATTN_OK;
+    const bool few = a->batch > 1 && a->batch < kSharesMinBatch && waves256 < 8 * kCUs && (4 * waves256 <= 21 * kCUs || waves256 > 6 * kCUs);
+    const bool nearly_two = waves256 > (group < 4 ? 6 : 7) * kCUs && waves256 <= 8 * kCUs, nearly_four = group < 4 && waves256 > 13 * kCUs && waves256 <= 16 * kCUs;
+    const bool one = a->batch < 2 && (p.tasks < 4 || waves256 <= 4 * kCUs || nearly_two || nearly_four);
+    if (!forced && (!large || few || one)) return LSATTN_OK;
     // bf16 launches that the lane kernel would take (in blocks as coarse as the split asked for they may be few waves): it multiplies V by fp32 weights, this
     // kernel by two bf16 parts of them (error against 64 bits 4e-7 | 4.8e-6: two of 131870 tokens, 2/1 heads; one of 65936, 10/5).  So only the large ones.
     const bool lane = std::is_same<T, BF16>::value && !use && !split_waves;

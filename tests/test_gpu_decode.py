@@ -1105,3 +1105,27 @@ def test_stage1_just_past_a_workgroup_per_cu_runs_the_plain_shape(lsa, tuning, d
     other = partials()
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
     assert not torch.equal(other[0], want[0])  # (the two shapes can be told apart)
+
+
+@pytest.mark.parametrize("Hq,Hkv,lens,shares", [
+    (16, 16, [10240] * 3, False), (32, 8, [8961, 300, 7000, 6453], False), (32, 8, [10752] * 4, False), (32, 8, [10753, 9000, 40, 10000], True), (32, 8, [12288] * 4, True), (32, 8, [12289] * 4, False),
+    (32, 8, [32768], False), (32, 8, [32769], True), (32, 8, [57344], True), (32, 8, [57345], False), (32, 8, [65537], True),
+    (16, 16, [24576], True), (16, 16, [24577], False), (16, 16, [32769], True), (16, 16, [53248], True), (16, 16, [53249], False), (16, 16, [65537], True)])
+def test_few_requests_in_equal_shares_where_these_are_no_slower(lsa, Hq, Hkv, lens, shares):
+    """A grid leaves one partial per block of a request; equal shares leave others.  On both sides of every line of the rule."""
+    from loongserve_amd.decoding import _fused_block_seq
+    print("case", Hq, Hkv, lens, flush=True)
+    B, D, BS = len(lens), 128, 256
+    q, kv, table, b_req, b_len = decode_case(322, B, Hq, Hkv, D, lens, sum(lens) + 500, torch.float16)
+    o_ref, l_ref = orc.decode_full(q, kv[:, :Hkv], kv[:, Hkv:], table, b_req, b_len)
+    kvd = kv.to(DEV)
+    mo = torch.full((max(lens) // BS + 1, B, Hq, D), float("nan"), device=DEV)
+    ml = torch.full(mo.shape[:3], float("nan"), device=DEV)
+    o, l = lsa.longserve_token_decode_attention_flash_decoding(q.to(DEV), table.to(DEV), b_req.to(DEV), b_len.to(DEV), mo, ml, B, max(lens), Hq, D,
+                                                               kvd[:, :Hkv], kvd[:, Hkv:], BS)
+    torch.cuda.synchronize()
+    assert_o_close(o, o_ref, "o")
+    assert_lse_close(l, l_ref, "lse")
+    split = _fused_block_seq(BS, B, max(lens), Hkv)
+    blocks = sum(-(-n // split) for n in lens) * Hq
+    assert (int((~ml.isnan()).sum()) != blocks) == shares
