@@ -1485,8 +1485,13 @@ static uint64_t next_arrivals() {
 // eight heads per task: 1 x 2048 8/1 10.5 | 9.6   1 x 3000 8/1, 96 rows, 11.1 | 10.8 (10.4 | 10.6, not taken)   1 x 8000 8/1, 256, 11.4 | 13.0 (not taken)
 // the lane kernel: 1 x 2048 32/32 10.6 | 9.5   10 x 400 24/8 14.0 | 13.1   4 x 5000 24/8, 60 rows, 640 workgroups, 24.8 | 25.4 (not taken)
 // sixteen heads: 1 x 1500 64/4, 96 rows in two turns, 12.0 | 12.8 (not taken).
+// Launches of more than a workgroup per CU, replayed from a graph (3000 launches): up to two per CU in blocks of up to 512 tokens and 64 rows 0.83 to 1.03; not taken: 65 to 128 rows (8 of at most 7935
+// 8/2 14.8 | 15.5), blocks of 1024 (40 x 10140 4/1 40.0 | 41.8), more workgroups (40 x 4608 8/2 36.7 | 42.6, 64 x 1535 8/2 24.5 | 28.0), and a request's only partial (400 x 768 8/1 35.7 | 42.6): partials are
+// stored through to memory, which the other workgroups' reads wait behind.  65 to 128 rows of few workgroups: eager 0.90 to 1.01, replayed 0.95 to 1.08 (3 of at most 8092 4/1 10.8 | 11.6).
 static bool join_takes(JoinPlan* join, Stage1Params& p, int64_t partials, int64_t heads, int64_t max_rows, int64_t workgroups) {
+  if (workgroups > kCUs && max_rows > 64) max_rows = 64;
   if (workgroups >= 2 * kCUs) max_rows /= 2;
+  if (partials < 2 || workgroups > 2 * kCUs || (workgroups > kCUs && p.block_seq > 512)) return false;
   if (!join || p.row_mul != 1 || partials > kJoinMaxPartials || heads > 8 || partials * heads > max_rows || (partials * p.blk_rows + heads) * 512 > 0x7fffffff) return false;
   join->done = true;
   p.o = join->s2->o;

@@ -1137,3 +1137,35 @@ def test_few_requests_in_equal_shares_where_these_are_no_slower(lsa, Hq, Hkv, le
 def test_few_kv_heads_in_equal_shares_where_these_are_no_slower(lsa, Hq, Hkv, lens, shares):
     """As above for fewer than four KV heads, against the shape whose waves split a block."""
     test_few_requests_in_equal_shares_where_these_are_no_slower(lsa, Hq, Hkv, lens, shares)
+
+
+@pytest.mark.parametrize("Hq,Hkv,lens,block,joined", [
+    (8, 1, [768] * 30, 1024, False), (8, 2, [770] * 64, 256, True), (8, 2, [513] * 86, 256, False),  # one partial; 512 and 516 workgroups
+    (8, 2, [4000] * 8, 256, True), (8, 2, [4097] * 8, 256, False), (4, 1, [8190] * 30, 1024, True), (4, 1, [8190] * 33, 1024, False), (4, 1, [4090] * 33, 512, True),  # 64 and 68 rows; 240 and 264 workgroups
+    (8, 4, [2000, 5], 128, True), (4, 4, [1500], 128, True), (8, 2, [1025, 0, 300], 128, True)])  # one and two heads of the lane kernel, four: several blocks per 256 tokens
+def test_partials_are_merged_in_their_launch_where_that_is_no_slower(lsa, Hq, Hkv, lens, block, joined):
+    """A graph of the fused call is one kernel or two, by the workgroups, the block and the partials, and either gives the result again and again."""
+    print("case", Hq, Hkv, lens[:2], len(lens), block, flush=True)
+    B, D = len(lens), 128
+    q, kv, table, b_req, b_len = decode_case(97, B, Hq, Hkv, D, lens, sum(lens) + 100, torch.float16)
+    o_ref, l_ref = orc.decode_full(q, kv[:, :Hkv], kv[:, Hkv:], table, b_req, b_len)
+    qd, kvd, td, rd, ld, rows = q.to(DEV), kv.to(DEV), table.to(DEV), b_req.to(DEV), b_len.to(DEV), (max(lens) + block - 1) // block
+    mo, ml = torch.full((rows, B, Hq, D), float("nan"), device=DEV), torch.full((rows, B, Hq), float("nan"), device=DEV)
+    o, l = torch.empty((B, Hq, D), device=DEV), torch.empty((B, Hq), device=DEV)
+
+    def call():
+        lsa.longserve_cuda_kernels.flash_decoding(mo, ml, qd, kvd[:, :Hkv], kvd[:, Hkv:], td, rd, ld, max(lens), o, l, block)
+
+    call()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        call()
+    assert (_kernel_nodes(graph) == 1) == joined
+    graph.instantiate()
+    for held in (0, -1, None):
+        if held is not None:
+            o.view(torch.int64).fill_(held)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_o_close(o, o_ref, "o")
+        assert_lse_close(l, l_ref, "lse")
