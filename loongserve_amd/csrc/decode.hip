@@ -1852,9 +1852,9 @@ template <typename OT> static int dispatch_stage2(const Stage2Params& p, int64_t
   if (p.max_shares > 0) {
     if (D != 128) return LSATTN_ERR_UNSUPPORTED;
     // four waves per pair while that keeps every pair resident at once (sixteen waves per CU)
-    // (sixteen for the few pairs of one or two requests, or of few heads, which may have hundreds of rows each: one long request among short ones
-    // 0.84 to 1.03, in the mean 0.97, ragged ones 0.99, equal ones 1.00 to 1.01; with more pairs 0.99 to 1.17)
-    if (grid.x <= kWideMergePairs && p.max_shares >= 128) LSATTN_LAUNCH_KERNEL((decode_merge_shares_kernel<OT, 16>), grid, dim3(1024), 0, st, p);
+    // (sixteen for the few pairs of one or two requests, which may have hundreds of rows each: both launches 0.84 to 1.03, in the mean 0.97 with one long
+    // request; with more pairs 0.99 to 1.17, and of more requests, whose rows are fewer, to 1.09: 16, one of 5120, 4/4 heads 15.3 | 16.7 us)
+    if (p.batch <= 2 && grid.x <= kWideMergePairs && p.max_shares >= 128) LSATTN_LAUNCH_KERNEL((decode_merge_shares_kernel<OT, 16>), grid, dim3(1024), 0, st, p);
     else if ((int64_t)grid.x <= 4 * kCUs) LSATTN_LAUNCH_KERNEL((decode_merge_shares_kernel<OT, 4>), grid, dim3(256), 0, st, p);
     else LSATTN_LAUNCH_KERNEL((decode_merge_shares_kernel<OT, 1>), dim3((unsigned)(p.batch * ((p.heads + 3) / 4))), dim3(256), 0, st, p);
     return check_launch();

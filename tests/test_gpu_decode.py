@@ -1169,3 +1169,43 @@ def test_partials_are_merged_in_their_launch_where_that_is_no_slower(lsa, Hq, Hk
         torch.cuda.synchronize()
         assert_o_close(o, o_ref, "o")
         assert_lse_close(l, l_ref, "lse")
+
+
+def _kernel_threads(graph):
+    """The threads per workgroup of a captured graph's kernels, in no order."""
+    import ctypes
+
+    class Params(ctypes.Structure):  # hipKernelNodeParams
+        _fields_ = [("block", ctypes.c_uint * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", ctypes.c_uint * 3),
+                    ("args", ctypes.c_void_p), ("lds", ctypes.c_uint)]
+
+    hip, n = ctypes.CDLL("libamdhip64.so"), ctypes.c_size_t(_kernel_nodes(graph))
+    nodes, found = (ctypes.c_void_p * n.value)(), []
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(int(graph.raw_cuda_graph())), nodes, ctypes.byref(n)) == 0
+    for node in nodes:
+        p = Params()
+        assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(p)) == 0
+        found.append(p.block[0] * p.block[1] * p.block[2])
+    return sorted(found)
+
+
+@pytest.mark.parametrize("Hq,Hkv,lens,threads", [(4, 4, [70000], 1024), (32, 8, [33000, 300], 1024), (8, 8, [5000] + [600] * 7, 256), (4, 4, [5120] + [300] * 15, 256)])
+def test_shares_of_many_requests_are_merged_by_four_waves(lsa, Hq, Hkv, lens, threads):
+    """Sixteen waves a (request, head) pair for one or two requests, whose rows are many; up to 64 pairs of more requests have few each."""
+    print("case", Hq, Hkv, lens[:2], flush=True)
+    B, D, BS = len(lens), 128, 256
+    q, kv, table, b_req, b_len = decode_case(323, B, Hq, Hkv, D, lens, sum(lens) + 500, torch.float16)
+    o_ref, l_ref = orc.decode_full(q, kv[:, :Hkv], kv[:, Hkv:], table, b_req, b_len)
+    qd, kvd, td, rd, ld = q.to(DEV), kv.to(DEV), table.to(DEV), b_req.to(DEV), b_len.to(DEV)
+    mo = torch.full((max(lens) // BS + 1, B, Hq, D), float("nan"), device=DEV)
+    ml = torch.full(mo.shape[:3], float("nan"), device=DEV)
+    o, l = torch.empty((B, Hq, D), device=DEV), torch.empty((B, Hq), device=DEV)
+    call = lambda: lsa.longserve_token_decode_attention_flash_decoding(qd, td, rd, ld, mo, ml, B, max(lens), Hq, D, kvd[:, :Hkv], kvd[:, Hkv:], BS, o, l)
+    call()
+    torch.cuda.synchronize()
+    assert_o_close(o, o_ref, "o")
+    assert_lse_close(l, l_ref, "lse")
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        call()
+    assert _kernel_threads(graph) == sorted([256, threads])
