@@ -1133,7 +1133,7 @@ def test_few_requests_in_equal_shares_where_these_are_no_slower(lsa, Hq, Hkv, le
 
 @pytest.mark.parametrize("Hq,Hkv,lens,shares", [
     (16, 1, [61952, 30000, 200, 5000, 100], False), (8, 1, [34000] + [700] * 7, False), (8, 1, [16640] + [700] * 15, True), (8, 1, [20480] + [9000] * 15, True), (8, 1, [20481] + [700] * 15, False),
-    (8, 1, [6400] + [50] * 83, True), (8, 1, [6144] + [50] * 95, True), (8, 1, [6145] + [50] * 95, False), (8, 1, [175360, 300, 7000], False), (12, 3, [64000, 4000, 6133], False)])
+    (8, 1, [6400] + [50] * 83, True), (8, 1, [6144] + [50] * 95, True), (8, 1, [6145] + [50] * 95, False), (8, 1, [175360, 300, 7000], False), (8, 1, [3000] + [50] * 99, True), (8, 1, [2800] + [50] * 100, False), (12, 3, [64000, 4000, 6133], False)])
 def test_few_kv_heads_in_equal_shares_where_these_are_no_slower(lsa, Hq, Hkv, lens, shares):
     """As above for fewer than four KV heads, against the shape whose waves split a block."""
     test_few_requests_in_equal_shares_where_these_are_no_slower(lsa, Hq, Hkv, lens, shares)
