@@ -1571,9 +1571,10 @@ static int launch_stage1(const lsattn_decode_stage1_args* a, hipStream_t st, Joi
   return check_launch();
 }
 
-// Waves of the plain shape up to which the shape whose waves split a block runs instead, on four and more KV heads.  513 to 576 waves 0.61 to 0.84 of the plain
-// shape where the lengths differ, 1.00 to 1.03 where they do not (24 requests of at most 592 tokens 32/8 16.8 -> 10.8 us); 577 to 640 0.68 to 0.96, 0.98 to 1.14, not taken.
-constexpr int64_t kSplitMaxWaves = 576;
+// Waves of the plain shape up to which the shape whose waves split a block runs instead, on four and more KV heads.  Of the plain shape's time, 1700 launches:
+// 513 to 544 waves 0.66 to 0.99 where the lengths differ, 0.94 to 1.02 where they do not (12 of at most 2716 16/4 20.0 | 16.7 us); 545 to 576 0.67 to 1.02, 0.99 to 1.09 (12 of 1281 32/8
+// 21.1 | 22.6), not taken.
+constexpr int64_t kSplitMaxWaves = 544;
 // Large launches: the matrix-pipe kernel, when its conditions hold (blocks a multiple of 32 tokens, enough waves to fill
 // the chip); lsattn_set_tuning forces the choice where the conditions allow it (tuning, tests).
 // What the fused call hands to stage 1 and on to the merge behind it.

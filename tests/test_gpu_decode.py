@@ -1209,3 +1209,21 @@ def test_shares_of_many_requests_are_merged_by_four_waves(lsa, Hq, Hkv, lens, th
     with torch.cuda.graph(graph):
         call()
     assert _kernel_threads(graph) == sorted([256, threads])
+
+
+@pytest.mark.parametrize("lens,shape", [([17408], "split"), ([17409], "mfma"), ([1281] * 12, "mfma"), ([4352, 7, 900, 3000], "split")])
+def test_stage1_is_split_among_a_blocks_waves_up_to_544_waves(lsa, tuning, lens, shape):
+    """On 32/8 heads: above that a batch of one length takes longer than in the plain shape.  The partials tell which of the two ran."""
+    print("case", lens[:2], flush=True)
+    B, BS = len(lens), 256
+    q, kv, table, b_req, b_len = decode_case(79, B, 32, 8, 128, lens, sum(lens) + 500, torch.float16)
+    qd, kvd, td, rd, ld = q.to(DEV), kv.to(DEV), table.to(DEV), b_req.to(DEV), b_len.to(DEV)
+    nblk = (max(lens) + BS - 1) // BS
+    got = {}
+    for how in (None, "split", "mfma"):
+        tuning(decode_stage1=how)
+        got[how] = torch.zeros((nblk, B, 32, 128), device=DEV)
+        ml = torch.zeros((nblk, B, 32), device=DEV)
+        lsa.longserve_flash_decode_stage1(qd, kvd[:, :8], kvd[:, 8:], td, rd, ld, max(lens), got[how], ml, BS)
+    torch.cuda.synchronize()
+    assert torch.equal(got[None], got[shape]) and not torch.equal(got["split"], got["mfma"])
