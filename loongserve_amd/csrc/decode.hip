@@ -1101,8 +1101,8 @@ constexpr int64_t kListedCoarseTokens = 1024;
 //     from one and a half on), and there also nearly four, to 1.04
 // Fewer than four KV heads, where a grid of the shape whose waves split a block stands against it, from more than 3072 waves on, and past whole rounds of that grid: one or two KV heads
 // and eight requests and more 2049 to 2304 waves 0.52 to 1.02, 0.95 in the mean (past that, or of fewer requests, to 1.13: 3 of at most 205825 16/1 39.2 | 44.1; three KV heads, which leave a
-// wave of a workgroup idle, to 1.12), with one KV head and sixteen to a hundred requests also 1025 to 1280, 0.51 to 1.02, 0.74
-// (fewer requests of different lengths to 1.28: 5 of at most 61952 16/1 23.4 | 30.0; four hundred of a block each to 1.19: 768 tokens 8/1 35.8 | 42.6); in between one length loses up to 16 %.
+// wave of a workgroup idle, to 1.12), with one KV head and 24 to a hundred requests also 1025 to 1280, 0.50 to 1.02, 0.74
+// (fewer requests of different lengths to 1.28: 5 of at most 61952 16/1 23.4 | 30.0, 16 of at most 16896 22.2 | 23.7; four hundred of a block each to 1.19: 768 tokens 8/1 35.8 | 42.6); in between one length loses up to 16 %.
 constexpr int64_t kSharesMinBatch = 8;
 // Not where the rows of the partials' buffers hold less than half of the shares the chip has waves for: 256 requests of 256 tokens,
 // GQA 32/8, are one share (2.9 ms) or a grid (57 us).  And not in place of a grid that one round of workgroups, one per CU, walks,
@@ -1658,11 +1658,13 @@ template <typename T> static int launch_stage1_mfma(const lsattn_decode_stage1_a
     // (waves of the plain shape at 256 tokens each, whatever the split asked for; the shape whose waves split a block keeps its launches)
     const int64_t waves256 = (shares->units * kMfmaBatch + 255) / 256 * p.tasks * a->batch;
     const bool past_rounds = group >= 4 && p.tasks < 3 && a->batch >= 8 && ((waves256 > 8 * kCUs && waves256 <= 9 * kCUs) ||
-                                                          (p.tasks == 1 && a->batch >= 16 && a->batch <= 100 && waves256 > 4 * kCUs && waves256 <= 5 * kCUs));
+                                                          (p.tasks == 1 && a->batch >= 24 && a->batch <= 100 && waves256 > 4 * kCUs && waves256 <= 5 * kCUs));
     const bool large = past_rounds || waves256 >= (group < 4 ? 768 : p.tasks < 4 ? 12 * kCUs + 1 : kSplitMaxWaves + 1);
     const bool few = a->batch > 1 && a->batch < kSharesMinBatch && waves256 < 8 * kCUs && (4 * waves256 <= 21 * kCUs || waves256 > 6 * kCUs);
-    const bool nearly_two = waves256 > (group < 4 ? 6 : 7) * kCUs && waves256 <= 8 * kCUs, nearly_four = group < 4 && waves256 > 13 * kCUs && waves256 <= 16 * kCUs;
-    const bool one = a->batch < 2 && (p.tasks < 4 || waves256 <= 4 * kCUs || nearly_two || nearly_four);
+    // (one request by the blocks it fills: a last block of a few tokens makes no round of its own, 1 x 32769 tokens 32/8 29.4 | 30.6)
+    const int64_t full = a->max_len_in_batch / 256 * p.tasks;
+    const bool nearly_two = full > (group < 4 ? 6 : 7) * kCUs && full <= 8 * kCUs, nearly_four = group < 4 && full > 13 * kCUs && full <= 16 * kCUs;
+    const bool one = a->batch < 2 && (p.tasks < 4 || full <= 4 * kCUs || nearly_two || nearly_four);
     if (!forced && (!large || few || one)) return LSATTN_OK;
     // bf16 launches that the lane kernel would take (in blocks as coarse as the split asked for they may be few waves): it multiplies V by fp32 weights, this
     // kernel by two bf16 parts of them (error against 64 bits 4e-7 | 4.8e-6: two of 131870 tokens, 2/1 heads; one of 65936, 10/5).  So only the large ones.

@@ -1109,8 +1109,8 @@ def test_stage1_just_past_a_workgroup_per_cu_runs_the_plain_shape(lsa, tuning, d
 
 @pytest.mark.parametrize("Hq,Hkv,lens,shares", [
     (16, 16, [10240] * 3, False), (32, 8, [8961, 300, 7000, 6453], False), (32, 8, [10752] * 4, False), (32, 8, [10753, 9000, 40, 10000], True), (32, 8, [12288] * 4, True), (32, 8, [12289] * 4, False),
-    (32, 8, [32768], False), (32, 8, [32769], True), (32, 8, [57344], True), (32, 8, [57345], False), (32, 8, [65537], True),
-    (16, 16, [24576], True), (16, 16, [24577], False), (16, 16, [32769], True), (16, 16, [53248], True), (16, 16, [53249], False), (16, 16, [65537], True)])
+    (32, 8, [32768], False), (32, 8, [33023], False), (32, 8, [33024], True), (32, 8, [57344], True), (32, 8, [57600], False), (32, 8, [65537], False), (32, 8, [65792], True),
+    (16, 16, [24576], True), (16, 16, [24832], False), (16, 16, [33024], True), (16, 16, [53248], True), (16, 16, [53504], False), (16, 16, [65792], True)])
 def test_few_requests_in_equal_shares_where_these_are_no_slower(lsa, Hq, Hkv, lens, shares):
     """A grid leaves one partial per block of a request; equal shares leave others.  On both sides of every line of the rule."""
     from loongserve_amd.decoding import _fused_block_seq
@@ -1132,7 +1132,7 @@ def test_few_requests_in_equal_shares_where_these_are_no_slower(lsa, Hq, Hkv, le
 
 
 @pytest.mark.parametrize("Hq,Hkv,lens,shares", [
-    (16, 1, [61952, 30000, 200, 5000, 100], False), (8, 1, [34000] + [700] * 7, False), (8, 1, [16640] + [700] * 15, True), (8, 1, [20480] + [9000] * 15, True), (8, 1, [20481] + [700] * 15, False),
+    (16, 1, [61952, 30000, 200, 5000, 100], False), (8, 1, [34000] + [700] * 7, False), (8, 1, [16640] + [700] * 15, False), (8, 1, [11264] + [700] * 23, True), (8, 1, [13568] + [5000] * 23, True), (8, 1, [13569] + [700] * 23, False),
     (8, 1, [6400] + [50] * 83, True), (8, 1, [6144] + [50] * 95, True), (8, 1, [6145] + [50] * 95, False), (8, 1, [175360, 300, 7000], False), (8, 1, [3000] + [50] * 99, True), (8, 1, [2800] + [50] * 100, False), (12, 3, [64000, 4000, 6133], False)])
 def test_few_kv_heads_in_equal_shares_where_these_are_no_slower(lsa, Hq, Hkv, lens, shares):
     """As above for fewer than four KV heads, against the shape whose waves split a block."""
