@@ -724,16 +724,24 @@ int64_t longest_keys(const lsattn_prefill_args* a) {
   return longest;
 }
 
-// Whether two waves share a wave's positions (KP = 2) in a launch of 64-wide heads with 16 positions per wave.  A wave has fewer products between its
-// waits here, so this gains with several workgroups on a CU too, the later the more there are.  Of the time of one wave each, over 270 launches (1 to 8 prompts of 150 to
+// Whether two waves share a wave's positions (KP = 2) in a launch with 16 positions per wave.  Up to a workgroup per CU, and with 64-wide heads, whose waves have fewer products
+// between their waits, up to three, the later the more there are.  Of the time of one wave each, 64 wide, over 270 launches (1 to 8 prompts of 150 to
 // 2500 tokens; 32/32, 32/8, 64/8, 16/16 and 8/1 heads, f16 and bf16, partials and in place), by the longest prompt:
 //   up to one per CU   below 300 1.01   300 to 450 0.97   to 600 0.93   to 800 0.90   to 1100 0.88   to 2500 0.84 (1700 tokens 32/8 bf16 27.4 -> 23.2 us)
 //   up to two          below 300 1.11   300 to 600 1.00   to 800 0.93   to 1100 0.90   to 2500 0.85      up to three   below 1100 1.02 to 1.15   to 1500 0.93   to 2500 0.89
-// and past that 0.99 to 1.21.
-bool parts_64(const lsattn_prefill_args* a) {
-  const int64_t one = workgroups(a, pack_shift_of(a), 1), longest = longest_keys(a);
-  if (one <= kCUs) return (longest == kUnknownKeys ? a->max_q_len : longest) >= 448;
-  return one <= 2 * kCUs ? a->max_q_len >= 640 : one <= 3 * kCUs && a->max_q_len >= 1152;
+// and past that 0.99 to 1.21.  Per CU as if all requests were as long as the longest: of ragged ones the workgroups without rows leave early and the long ones meet on
+// a few CUs, where twice the waves take up to 1.36 of the time (4, one of 742, full steps, 16/1 128 wide 39.6 | 45.4; 4 of at most 2075 8/8 64 wide 27.0 | 30.8); and of several requests by the
+// keys of the mean one, or of the longest prompt: what the K buffer holds beyond the rows was taken for one request's context (6 of at most 61 rows behind 87 keys 40/8 7.7 | 8.7).
+bool two_waves_share(const lsattn_prefill_args* a) {
+  const int64_t rows = (kWaves * 16) >> pack_shift_of(a);
+  const int64_t most = (int64_t)a->batch * ((a->max_q_len + rows - 1) / rows) * (a->num_q_heads >> pack_shift_of(a));
+  int64_t keys = longest_keys(a);
+  if (a->batch > 1 || keys == kUnknownKeys) {
+    const int64_t mean = a->total_kv_rows / a->batch, likely = mean > a->max_q_len ? mean : a->max_q_len;
+    if (likely < keys) keys = likely;
+  }
+  if (most <= kCUs) return keys >= (a->head_dim == 64 ? 448 : kPartsMinKeys);
+  return a->head_dim == 64 && (most <= 2 * kCUs ? a->max_q_len >= 640 : most <= 3 * kCUs && a->max_q_len >= 1152);
 }
 
 // 32 positions per wave serve twice the rows with each K and V operand read, 16 make twice as many, shorter waves: these from
@@ -745,7 +753,7 @@ template <typename T, int D, int MODE, bool DV> int launch(const SmallParams& p,
   switch (prefill_small_route(a)) {
     case LSATTN_ROUTE_SMALL_16:
       if constexpr (D == 64)
-        if (parts_64(a)) return launch_rows<T, 64, MODE, DV, 16, 2>(p, a, st);
+        if (two_waves_share(a)) return launch_rows<T, 64, MODE, DV, 16, 2>(p, a, st);
       return launch_rows<T, D, MODE, DV, 16>(p, a, st);
     default: return launch_rows<T, D, MODE, DV, 32>(p, a, st);
   }
@@ -754,7 +762,7 @@ template <typename T, int D, int MODE, bool DV> int launch(const SmallParams& p,
 template <typename T, int MODE, bool DV> int launch_128(const SmallParams& p, const lsattn_prefill_args* a, hipStream_t st) {
   switch (prefill_small_route(a)) {
     case LSATTN_ROUTE_SMALL_16:
-      if (workgroups(a, pack_shift_of(a), 1) <= kCUs && longest_keys(a) >= kPartsMinKeys) return launch_rows<T, 128, MODE, DV, 16, 2>(p, a, st);
+      if (two_waves_share(a)) return launch_rows<T, 128, MODE, DV, 16, 2>(p, a, st);
       return launch_rows<T, 128, MODE, DV, 16>(p, a, st);
     default: return launch_rows<T, 128, MODE, DV, 32>(p, a, st);
   }

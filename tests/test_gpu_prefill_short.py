@@ -251,3 +251,24 @@ def test_two_waves_that_share_a_tile_of_64_wide_heads(lsa, mode, V, Hq, Hkv, len
     """One, two and three workgroups per CU, one, two and four heads side by side."""
     print("case", mode, V, Hq, Hkv, lens, flush=True)
     _every_epilogue_on(SMALL_16, lsa, mode, V, 64, Hq, Hkv, lens, ctx)
+
+
+@pytest.mark.parametrize("D,Hq,Hkv,lens,klens", [(128, 16, 1, [742, 70, 69, 69], None), (64, 16, 16, [500, 33, 100, 64], None), (128, 40, 8, [61, 20, 8, 30, 7, 15], [148, 107, 95, 117, 94, 102])])
+def test_ragged_and_short_batches_run_one_wave_per_position(lsa, D, Hq, Hkv, lens, klens):
+    """Batches whose long request is counted as the only one, or as having all keys that the buffer holds beyond the rows: two waves share a tile only where a workgroup per CU is
+    enough if all were as long, and where the mean request has the keys.  Which kernel ran shows in the bits: without the bound on the rows,
+    or with one on the keys, the launch is one wave's without question."""
+    print("case", D, Hq, Hkv, lens, flush=True)
+    T, full = sum(lens), klens is None
+    klens = klens or lens
+    TK = sum(klens)
+    q, k, v = rand_t((T, Hq, D), 61), rand_t((TK, Hkv, D), 62), rand_t((TK, Hkv, D), 63)
+    qm, km = meta(lens, [0 if full else n - m for n, m in zip(klens, lens)]), meta(klens)
+    o_ref, lse_ref = orc.attn_step(q, k, v, *qm, *km, 1)
+    args = (*_dev(q, k, v), *_dev(*qm), *_dev(*km), 1, max(lens))
+    got = lsa.prefill_attention_step(*args, total_q_len=T)
+    sure = lsa.prefill_attention_step(*args) if full else lsa.prefill_attention_step(*args, total_q_len=T, max_kv_len=max(klens))
+    torch.cuda.synchronize()
+    assert_o_close(got[0], o_ref, "O")
+    assert_lse_close(got[1], lse_ref, "LSE")
+    assert torch.equal(got[0], sure[0]) and torch.equal(got[1], sure[1])
