@@ -1353,9 +1353,10 @@ static Shape choose_shape(const lsattn_prefill_args* a, bool dv, const Tuning& t
     if (a->max_q_len > 6144) split = split || (a->m && wgs128 <= 21 * kCUs / 8);
     else if (wgs128 <= (a->m && !several ? ph ? 22 : 23 : ph ? 18 : 22) * kCUs / 8) half = true;
   }
-  // ... and where they are between three halves and seven quarters of a CU's and short (from there on the folded grid below): the split shape's second
-  // round is one of a few too (36 to 48 heads, 1040 to 1400 rows: prompts 0.83 to 1.01, full steps 0.84 to 0.93; 32 heads, 1600 rows: 0.94 to 1.05, not taken).
-  if (as_long && a->max_q_len <= 1408 && 2 * wgs128 > 3 * kCUs && 4 * wgs128 < 7 * kCUs) half = true;
+  // ... and where they are between three halves and seven quarters of a CU's and short (from there on the folded grid below), with one head per workgroup: the split shape's
+  // second round is one of a few too (36 to 48 heads, 1040 to 1400 rows: prompts 0.83 to 1.01, full steps 0.84 to 0.93; 32 heads, 1600 rows: 0.94 to 1.05, not taken;
+  // heads side by side, prompts 0.86 to 0.91 of the 256-row shape but full steps 1.03 to 1.06, 800 rows 64/8 37.4 | 38.9: not taken).
+  if (as_long && ph == 0 && a->max_q_len <= 1408 && 2 * wgs128 > 3 * kCUs && 4 * wgs128 < 7 * kCUs) half = true;
   // Ragged requests folded in place whose keys are no more than their rows (prompts, or a ring's steps), up to 2048 rows: the 256-row shape ends with the
   // longest requests' workgroups alone on their CUs, the split shape in one round more.  From three halves of a workgroup per CU on (one where it
   // would be the 256-row shape), over 45 launches: prompts of up to 1024 rows 0.84 of the others, 1536 0.93, 2048 0.97, full steps 0.93; 0.58 to 1.10 (133 launches: 0.92).

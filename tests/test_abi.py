@@ -539,6 +539,13 @@ def test_lone_prompts_of_a_few_workgroups_past_two_per_cu():
     assert _route(1, 2500, (32, 8), total_q=2500, total_kv=2600, m=256) == ROWS_256 and _route(2, 1250, (32, 8), total_q=2500, total_kv=2500, m=256) != HALF
 
 
+def test_lone_prompts_of_heads_side_by_side_keep_256_rows():
+    """Between three halves and seven quarters of a 128-row workgroup per CU the four-wave shape takes one head per workgroup only."""
+    lone = lambda n, heads, m=256: _route(1, n, heads, total_q=n, total_kv=n, m=m)
+    assert lone(800, (64, 8)) == lone(800, (64, 8), None) == lone(863, (64, 8)) == ROWS_256
+    assert lone(1100, (44, 44)) == HALF
+
+
 def test_equal_prompts_fill_a_third_workgroup_per_cu():
     """Equal f16 requests in place: 769 to 1024 rows from two workgroups of 32 positions per CU on, up to 1280 from 2.6 on, up to three."""
     step = lambda b, n, heads, m=256, total=None, **kw: _route(b, n, heads, total_q=total or b * n, total_kv=total or b * n, m=m, **kw)
