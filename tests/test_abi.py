@@ -562,3 +562,14 @@ def test_ragged_batches_folded_in_place_by_four_waves():
     assert step(2048, 5000) == HALF and step(2049, 5000) == step(2048, 5000, m=None) == step(2048, 5000, total_kv=5001) == ROWS_256
     assert step(2048, 7372) == HALF and step(2048, 7373) == ROWS_256  # (nine tenths of 8192)
     assert step(1900, 2000, (8, 1)) == ROWS_128  # (1.0 per CU)
+
+
+def test_ragged_batches_of_few_workgroups_keep_their_shape():
+    """Folded in place by four waves from nine halves of a workgroup of 128 rows per CU on, of eight requests from three and of sixteen from one on; not in place of the split shape."""
+    step = lambda b, n, total, heads, m=256: _route(b, n, heads, total_q=total, total_kv=total, m=m)
+    assert step(4, 1973, 3262, (14, 2)) == step(5, 1704, 2399, (16, 16)) == ROWS_128        # (1.6 and 1.5 per CU, the split shape's)
+    assert step(2, 1523, 1713, (32, 32)) == step(3, 975, 1200, (32, 8)) == ROWS_256         # (1.8 and 1.3)
+    assert step(4, 2048, 4448, (32, 8)) == ROWS_256 and step(4, 2048, 4449, (32, 8)) == HALF  # (143 and 144 tiles of 32 rows)
+    assert step(8, 1500, 2784, (32, 8)) == ROWS_256 and step(8, 1500, 2785, (32, 8)) == HALF  # (95 and 96)
+    assert step(15, 1200, 2700, (32, 8)) == HALF and step(16, 900, 4000, (8, 1)) == step(20, 840, 5000, (8, 1)) == HALF  # (1.1 and 1.4)
+    assert step(15, 1200, 2400, (32, 8)) == ROWS_256                                        # (2.8)
