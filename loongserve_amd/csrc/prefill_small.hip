@@ -818,7 +818,7 @@ template <typename T, bool DV> int launch_mode(const SmallParams& p, const lsatt
 //   32 from there on: past 768 rows from three (ragged: three and a half) of its own per CU, past 1024 from four (five), where the other
 // kernel's four-wave shape has more than one round; equal prompts past 1024 rows in more than ten per CU are for that kernel's faster loop.
 //   Equal f16 requests in the in-place epilogue also fill the third workgroup of 32 positions per CU (workgroups of 128 rows split the launch into a full
-// round and a thin one there): 769 to 1024 rows in more than two per CU 0.61 to 0.95 of the other kernel's time, full steps 0.80 to 0.90; 1025 to 1280 in more than
+// round and a thin one there): 769 to 1024 rows in 33/16 per CU and more 0.58 to 1.01 of the other kernel's time, full steps 0.73 to 0.88 (in fewer prompts to 1.05, 5 x 832 16/1 30.8 | 32.3); 1025 to 1280 in more than
 // 2.6 0.75 to 0.87, full steps 0.83 to 0.96 (us: 11 x 929 8/1 62.3 | 40.4, 2 x 792 40/8 45.7 | 34.3, 9 x 1198 8/1 63.2 | 52.6, as a full step 9 x 1005 8/8 70.9 | 65.1; from 2 to 2.6 prompts up to 1.06; 1281 to 1408 up to 1.12, more than three per CU full steps to 1.22: not taken).
 // The keys: a chunk behind a context waits for its longest request, and a tile of a lone workgroup takes longer here (0.95 us against 0.56 in the
 // 128-row shape), so the longest request decides (whole call, 32/8 heads, the other kernel | this one with 16 positions, f16, then bf16):
@@ -844,7 +844,7 @@ int prefill_short_blocks(const lsattn_prefill_args* a) {
   if (one <= kCUs) return !past || (f16 && a->batch == 1) ? 1 : 0;
   // (otherwise bf16 does not look at m: whether V is to be copied may be asked without it)
   if (one > 2 * kCUs && one <= 3 * kCUs && (past ? !rag && (f16 ? a->m != nullptr : pack == 0) : !rag || pack == 0)) return 1;
-  if (f16 && a->m && a->batch > 1 && !rag && a->max_q_len == longest && two <= 3 * kCUs && 5 * two > (past ? 13 : 10) * kCUs) return 2;
+  if (f16 && a->m && a->batch > 1 && !rag && a->max_q_len == longest && two <= 3 * kCUs && (past ? 5 * two > 13 * kCUs : 16 * two >= 33 * kCUs)) return 2;
   if (past) return two > (rag ? 5 : 4) * kCUs && (rag || two <= 10 * kCUs) ? 2 : 0;
   return 2 * two >= (rag ? 7 : 6) * kCUs ? 2 : 0;
 }

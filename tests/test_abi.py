@@ -573,3 +573,10 @@ def test_ragged_batches_of_few_workgroups_keep_their_shape():
     assert step(8, 1500, 2784, (32, 8)) == ROWS_256 and step(8, 1500, 2785, (32, 8)) == HALF  # (95 and 96)
     assert step(15, 1200, 2700, (32, 8)) == HALF and step(16, 900, 4000, (8, 1)) == step(20, 840, 5000, (8, 1)) == HALF  # (1.1 and 1.4)
     assert step(15, 1200, 2400, (32, 8)) == ROWS_256                                        # (2.8)
+
+
+def test_equal_prompts_barely_past_two_workgroups_per_cu_keep_256_rows():
+    """Equal f16 requests in place fill a third workgroup of 32 positions per CU from 33/16 on."""
+    step = lambda b, n, heads: _route(b, n, heads, total_q=b * n, total_kv=b * n, m=256)
+    assert step(5, 832, (16, 1)) == ROWS_256 and step(5, 833, (16, 1)) == SMALL_32  # (26 and 27 tiles of 32 rows: 520 and 540 workgroups)
+    assert step(11, 1024, (6, 6)) == SMALL_32                                     # (528)
