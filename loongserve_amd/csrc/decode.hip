@@ -91,11 +91,21 @@ __device__ __forceinline__ void store_result(const Stage1Params& p, int64_t elem
   else if (p.o_dtype == LSATTN_F16) store4<F16>(p.o, elem, v);
   else store4<BF16>(p.o, elem, v);
 }
-// `seen`: what the word held when the workgroup (wave) started; n: partials, one of them each.
-__device__ __forceinline__ void start_arrivals(uint64_t* word, uint64_t seen, uint64_t start, int n) {
-  if (seen - start > (uint64_t)n) __hip_atomic_compare_exchange_strong(word, &seen, start, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// `seen`: what the word held when the workgroup (wave) started; n: partials, one of them each.  Returns what the word held when the start was put in, or `seen` if it is a count already;
+// nobody waits for it before arrive.
+__device__ __forceinline__ uint64_t start_arrivals(uint64_t* word, uint64_t seen, uint64_t start, int n) {
+  uint64_t held = seen;
+  if (seen - start > (uint64_t)n) __hip_atomic_compare_exchange_strong(word, &held, start, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return held;
 }
-__device__ __forceinline__ bool arrive(uint64_t* word, uint64_t start, int n) {  // (behind a wait for the stores of the partial)
+// Behind a wait for the stores of the partial.  If the word was neither what was seen nor a count of this launch, the start is put in over what it was then: once at most in memory
+// that nobody else writes, and never without end.
+constexpr int kStartTries = 64;
+__device__ __forceinline__ bool arrive(uint64_t* word, uint64_t seen, uint64_t held, uint64_t start, int n) {
+  for (int i = 0; i < kStartTries && held != seen && held - start > (uint64_t)n; i++) {
+    seen = held;
+    __hip_atomic_compare_exchange_strong(word, &held, start, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
   return __hip_atomic_fetch_add(word, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - start == (uint64_t)(n - 1);
 }
 // The merge of `n` <= kJoinMaxPartials partials of up to 16 query heads, by the four waves of a workgroup.
@@ -512,9 +522,9 @@ __global__ __launch_bounds__(NW * 64, JOIN ? (GT == 1 ? 4 : 3) : 1) void decode_
   if constexpr (JOIN) {
     __shared__ __attribute__((aligned(16))) char meet[16 + 8 * 32 * 16];
     if (wave == 0 && lane == 0) {
-      start_arrivals(word, seen, p.arrivals, arrivals);
+      const uint64_t held = start_arrivals(word, seen, p.arrivals, arrivals);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (wave 0 has stored the partials)
-      *(uint32_t*)meet = arrive(word, p.arrivals, arrivals);
+      *(uint32_t*)meet = arrive(word, seen, held, p.arrivals, arrivals);
     }
     __syncthreads();
     if (*(const uint32_t*)meet) join_partials(p, meet, lane, wave, b * p.hq + qh0, nh, b * p.req_rows + qh0, (int)nblk);
@@ -982,7 +992,8 @@ __device__ __forceinline__ void stage1_mfma_unit(const Stage1Params& p, char* ld
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (rows requested past the end land before the registers are given back)
-  if (JOIN && wave == 0 && lane == 0) start_arrivals(word, seen, p.arrivals, join_n);
+  uint64_t held = seen;
+  if (JOIN && wave == 0 && lane == 0) held = start_arrivals(word, seen, p.arrivals, join_n);
   if constexpr (WS) {
     // The four partials of the block meet in LDS (each wave's own 17.5 KB: its last batch's operands have been consumed);
     // every wave then finishes two of the eight d-blocks.  A wave without a batch of its own brings m = -inf, l = 0.
@@ -1037,7 +1048,7 @@ __device__ __forceinline__ void stage1_mfma_unit(const Stage1Params& p, char* ld
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's part of the partial is in memory
       __syncthreads();                                  // ... and so are the others'
       uint32_t* const last = (uint32_t*)lds;
-      if (wave == 0 && lane == 0) *last = arrive(word, p.arrivals, join_n);
+      if (wave == 0 && lane == 0) *last = arrive(word, seen, held, p.arrivals, join_n);
       __syncthreads();
       if (*last) join_partials(p, lds, lane, wave, b * p.hq + qh0, nh, b * p.req_rows + qh0, join_n);
     }

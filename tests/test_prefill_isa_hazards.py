@@ -466,3 +466,21 @@ def test_reference_counts_are_written_behind_a_wait_for_the_slot_states():
             assert labels[back.group(1)] <= waits[0] and barriers[0] < labels[back.group(1)], lines[i]
         else:
             assert i > barriers[0], lines[i]
+
+
+@pytest.mark.skipif(shutil.which(HIPCC) is None, reason="hipcc not available")
+def test_a_count_of_arrivals_that_was_not_started_is_tried_again():
+    """The kernels that merge their own partials put the launch's start into a word that may hold anything.  What the word held comes back from every
+    exchange, and a second one stands in a loop, so that a word that changed since it was first read is no reason to give up."""
+    kernels, name = {}, None
+    for raw in _decode_asm().split("\n"):
+        m = re.match(r"^(_ZN6lsattn\w+):", raw)
+        name = m.group(1) if m else None if raw.startswith(".Lfunc_end") else name
+        if name:
+            kernels.setdefault(name, []).append(raw)
+    kernels = {n: lines for n, lines in kernels.items() if any("global_atomic_cmpswap_x2" in ln for ln in lines)}
+    assert len(kernels) == 8, list(kernels)  # fp16 and bf16: the matrix-pipe kernel, the lane kernel with one, two and four heads
+    for name, lines in kernels.items():
+        tries = [i for i, ln in enumerate(lines) if "global_atomic_cmpswap_x2" in ln]
+        assert len(tries) == 2 and all(lines[i].rstrip().endswith("sc0") for i in tries), (name, [lines[i] for i in tries])
+        assert any(first < tries[1] <= last and last - first < 60 for first, last in _loops(lines)), name
