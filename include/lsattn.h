@@ -270,9 +270,10 @@ typedef struct lsattn_decode_stage2_args {
   int32_t o_dtype;         /* LSATTN_F16 / BF16 / F32  */
   int32_t o_is_apart;      /* read by the fused calls below.  1: neither o nor out_logexpsum shares memory with the pool's rows or the
                               table, so that short contexts may be one launch, which writes the result while others still read;
-                              0: not known (the call's two launches write it behind the last read).  2: as 1, and o lies in memory that
-                              the GPU of the launch has allocated (not the host's, not another GPU's) and nobody else uses during
-                              the call, so that workgroups may count in it with 64-bit atomics before the result is written there */
+                              0: not known (the call's two launches write it behind the last read).  2: as 1, and nobody else
+                              uses o during the call, so that workgroups may count in it with 64-bit atomics before the result is
+                              written there; they do where the runtime knows o as the current GPU's own memory (not the host's, managed
+                              or another GPU's: two launches) */
   float* out_logexpsum;    /* [batch, H] */
   const int32_t* b_seqlen; /* [batch]    */
   const float* mid_o;            /* [num_seq_blocks, batch, H, D] */

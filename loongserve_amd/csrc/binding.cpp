@@ -419,7 +419,7 @@ PyObject* token_decode_attention(PyObject*, PyObject* const* args, Py_ssize_t na
   d.s1.partials_by_request = d.s2.partials_by_request = by_request;
   d.s2.o_is_apart = (!out_in || (no_overlap(out, k) && no_overlap(out, v) && no_overlap(out, table))) &&
                     (!lse_in || (no_overlap(lse, k) && no_overlap(lse, v) && no_overlap(lse, table)));
-  if (d.s2.o_is_apart && out.device() == q->device()) d.s2.o_is_apart = 2;  // (a GPU tensor: memory of that GPU)
+  if (d.s2.o_is_apart && out.device() == q->device()) d.s2.o_is_apart = 2;  // (whose memory it is the library asks the runtime)
   if (const int rc = call(lib.decode_attention, &d.s1, &d.s2, stream())) return failed(rc, "lsattn_decode_attention");
   PyObject* o1 = out_in ? (Py_INCREF(py_out), py_out) : THPVariable_Wrap(out);
   PyObject* o2 = lse_in ? (Py_INCREF(py_lse), py_lse) : THPVariable_Wrap(lse);

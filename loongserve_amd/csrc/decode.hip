@@ -1499,11 +1499,23 @@ static uint64_t next_arrivals() {
 // Launches of more than a workgroup per CU, replayed from a graph (3000 launches): up to two per CU in blocks of up to 512 tokens and 64 rows 0.83 to 1.03; not taken: 65 to 128 rows (8 of at most 7935
 // 8/2 14.8 | 15.5), blocks of 1024 (40 x 10140 4/1 40.0 | 41.8), more workgroups (40 x 4608 8/2 36.7 | 42.6, 64 x 1535 8/2 24.5 | 28.0), and a request's only partial (400 x 768 8/1 35.7 | 42.6): partials are
 // stored through to memory, which the other workgroups' reads wait behind.  65 to 128 rows of few workgroups: eager 0.90 to 1.01, replayed 0.95 to 1.08 (3 of at most 8092 4/1 10.8 | 11.6).
+// Whether the runtime knows p as memory of the current GPU's own: not the host's, managed, or another GPU's, where the counts' 64-bit atomics at the scope of
+// one GPU are not sure to work.  (0.2 us, of launches that would merge only; a tensor labelled with this GPU may wrap any of them.)
+static bool is_memory_of_this_gpu(const void* p) {
+  hipPointerAttribute_t at = {};
+  int device = -1;
+  if (hipPointerGetAttributes(&at, p) != hipSuccess || hipGetDevice(&device) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return at.type == hipMemoryTypeDevice && !at.isManaged && at.device == device;
+}
 static bool join_takes(JoinPlan* join, Stage1Params& p, int64_t partials, int64_t heads, int64_t max_rows, int64_t workgroups) {
   if (workgroups > kCUs && max_rows > 64) max_rows = 64;
   if (workgroups >= 2 * kCUs) max_rows /= 2;
   if (partials < 2 || workgroups > 2 * kCUs || (workgroups > kCUs && p.block_seq > 512)) return false;
   if (!join || p.row_mul != 1 || partials > kJoinMaxPartials || heads > 8 || partials * heads > max_rows || (partials * p.blk_rows + heads) * 512 > 0x7fffffff) return false;
+  if (!is_memory_of_this_gpu(join->s2->o)) return false;
   join->done = true;
   p.o = join->s2->o;
   p.out_lse = join->s2->out_logexpsum;
@@ -1949,7 +1961,7 @@ extern "C" int lsattn_decode_attention(const lsattn_decode_stage1_args* s1, cons
       return decode_stage2(&a2, 0, stream, &shares);
     }
   }
-  // (the merge in stage 1's launch counts in o, which only memory of this GPU's own is sure to take; launches of forced shapes are two)
+  // (the merge in stage 1's launch counts in o, see is_memory_of_this_gpu; launches of forced shapes are two)
   JoinPlan join{s2};
   const Tuning tn = tuning();
   const bool may_join = s2->o_is_apart == 2 && tn.decode_stage1 == 0 && tn.decode_listed == 0 && validate_stage2(s2) == LSATTN_OK && (s2->o_dtype == LSATTN_F32 || s2->o_dtype == LSATTN_F16 || s2->o_dtype == LSATTN_BF16) &&

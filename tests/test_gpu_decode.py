@@ -1227,3 +1227,42 @@ def test_stage1_is_split_among_a_blocks_waves_up_to_544_waves(lsa, tuning, lens,
         lsa.longserve_flash_decode_stage1(qd, kvd[:, :8], kvd[:, 8:], td, rd, ld, max(lens), got[how], ml, BS)
     torch.cuda.synchronize()
     assert torch.equal(got[None], got[shape]) and not torch.equal(got["split"], got["mfma"])
+
+
+def _managed(shape):
+    """A float32 tensor of this GPU over managed memory, which is not freed."""
+    import ctypes
+    hip, ptr, n = ctypes.CDLL("libamdhip64.so"), ctypes.c_void_p(), math.prod(shape)
+    assert hip.hipMallocManaged(ctypes.byref(ptr), ctypes.c_size_t(4 * n), ctypes.c_uint(1)) == 0
+    t = torch.as_tensor(type("Held", (), {"__cuda_array_interface__": dict(shape=tuple(shape), typestr="<f4", data=(ptr.value, False), version=2)})(), device=DEV)
+    assert t.data_ptr() == ptr.value and t.is_cuda
+    return t
+
+
+@pytest.mark.parametrize("static", [False, True])
+def test_results_in_other_memory_than_the_gpus_own_take_two_launches(lsa, static):
+    """Workgroups count each other in the result only where the runtime knows it as the GPU's own memory; a tensor over managed memory is written behind
+    the last read, by two launches, whichever call it is handed to."""
+    lens, Hq, Hkv, D = [1500, 700], 32, 8, 128
+    q, kv, table, b_req, b_len = decode_case(98, 2, Hq, Hkv, D, lens, 3000, torch.float16)
+    o_ref, l_ref = orc.decode_full(q, kv[:, :Hkv], kv[:, Hkv:], table, b_req, b_len)
+    qd, kvd, td, rd, ld = q.to(DEV), kv.to(DEV), table.to(DEV), b_req.to(DEV), b_len.to(DEV)
+    mo, ml = torch.empty((6, 2, Hq, D), device=DEV), torch.empty((6, 2, Hq), device=DEV)
+    for o, kernels in ((torch.empty((2, Hq, D), device=DEV), 1), (_managed((2, Hq, D)), 2)):
+        l = torch.empty((2, Hq), device=DEV)
+
+        def call():
+            if static:
+                lsa.longserve_cuda_kernels.flash_decoding_static(qd, kvd[:, :Hkv], kvd[:, Hkv:], td, rd, ld, max(lens), o, l, 256)
+            else:
+                lsa.longserve_token_decode_attention_flash_decoding(qd, td, rd, ld, mo, ml, 2, max(lens), Hq, D, kvd[:, :Hkv], kvd[:, Hkv:], 256, o, l)
+
+        graph = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(graph):
+            call()
+        assert _kernel_nodes(graph) == kernels
+        o.fill_(float("nan"))
+        call()
+        torch.cuda.synchronize()
+        assert_o_close(o, o_ref, "o")
+        assert_lse_close(l, l_ref, "lse")
