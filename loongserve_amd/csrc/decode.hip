@@ -1916,7 +1916,7 @@ static int decode_stage2(const lsattn_decode_stage2_args* a, int64_t live_blocks
                  a->batch, a->num_heads, a->num_seq_blocks, a->block_seq,
                  a->partials_by_request ? a->num_heads : a->batch * a->num_heads,
                  a->partials_by_request ? a->num_seq_blocks * a->num_heads : a->num_heads, shares ? shares->units : 0,
-                 shares ? shares->max_shares : 0, kShareUnits, a->lead_rows};
+                 shares ? shares->max_shares : 0, kShareUnits, a->lead_rows < a->num_seq_blocks ? a->lead_rows : a->num_seq_blocks};
   dim3 grid((unsigned)(a->batch * a->num_heads));
   hipStream_t st = (hipStream_t)stream;
   switch (a->o_dtype) {

@@ -1266,3 +1266,19 @@ def test_results_in_other_memory_than_the_gpus_own_take_two_launches(lsa, static
         torch.cuda.synchronize()
         assert_o_close(o, o_ref, "o")
         assert_lse_close(l, l_ref, "lse")
+
+
+@pytest.mark.parametrize("lead", [7, 2 ** 62, 2 ** 63 - 1])
+def test_stage2_with_more_rows_of_peers_than_there_are(lsa, lead):
+    """Every row of the buffer is merged, whatever the length is, as for lead_rows of all its rows."""
+    print("case", lead, flush=True)
+    g = torch.Generator().manual_seed(3)
+    mo, ml = torch.randn(7, 3, 2, 128, generator=g).to(DEV), torch.randn(7, 3, 2, generator=g).to(DEV)
+    w = torch.softmax(ml.double(), 0)
+    want, want_lse = (w[..., None] * mo.double()).sum(0).float(), torch.logsumexp(ml.double(), 0).float()
+    for lens in ([0, 1, 5], [2 ** 31 - 1] * 3):
+        o, l = torch.zeros((3, 2, 128), device=DEV), torch.zeros((3, 2), device=DEV)
+        lsa.longserve_flash_decode_stage2(mo, ml, torch.tensor(lens, dtype=torch.int32, device=DEV), o, l, 1, lead)
+        torch.cuda.synchronize()
+        assert_o_close(o.cpu(), want.cpu(), "o")
+        assert_lse_close(l.cpu(), want_lse.cpu(), "lse", rel=1e-5)
