@@ -98,7 +98,7 @@ def _prefill_args(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first, kv_b_start_lo
                   peers: int, max_q_len: int, sm_scale: Optional[float], v_f16: Optional[torch.Tensor] = None,
                   v_f16_valid: bool = False, o_b_start_loc: Optional[torch.Tensor] = None,
                   cuts: Optional[Tuple[int, int, int]] = None, total_q_len: Optional[int] = None,
-                  max_kv_len: Optional[int] = None) -> _lib.PrefillArgs:
+                  max_kv_len: Optional[int] = None, state: Optional[Tuple[torch.Tensor, torch.Tensor]] = None) -> _lib.PrefillArgs:
     for t, n in ((q, "q"), (k, "k"), (v, "v"), (o, "o")):
         _dev(t, n)
         if t.dim() != 3:
@@ -150,6 +150,10 @@ def _prefill_args(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first, kv_b_start_lo
         a.total_q_rows = int(total_q_len)
     a.total_kv_rows = k.shape[0]
     a.max_kv_len = _keys_up_to(max_kv_len)
+    if state is not None:  # (in front of the question whether the kernel converts V: which kernel runs depends on m)
+        m, l = state
+        a.m, a.l = m.data_ptr(), l.data_ptr()
+        a.ml_stride_t, a.ml_stride_h = m.stride(0), m.stride(1)
     if q.dtype == torch.bfloat16 and (v_f16 is not None or (PRECONVERT_BF16_V and Lq == KERNEL_HEAD_DIM)):
         if v_f16_valid and (v_f16 is None or v_f16.dtype != torch.float16 or v_f16.shape != v.shape or v_f16.stride(2) != 1):
             raise ValueError("v_f16_valid needs v_f16, the float16 copy of v")
@@ -349,9 +353,7 @@ def _context_attention_checked(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first_t
         return
     a = _prefill_args(q, k, v, o, q_b_start_loc, q_b_seq_len, q_first_token_global_idx, kv_b_start_loc,
                       kv_b_seq_len, kv_first_token_global_idx, logical_sp_peers_num, max_q_b_seq_len,
-                      1.0 / (D ** 0.5), v_f16, v_f16_valid, total_q_len=total_q_len, max_kv_len=max_kv_len)
-    a.m, a.l = m.data_ptr(), l.data_ptr()
-    a.ml_stride_t, a.ml_stride_h = m.stride(0), m.stride(1)
+                      1.0 / (D ** 0.5), v_f16, v_f16_valid, total_q_len=total_q_len, max_kv_len=max_kv_len, state=(m, l))
     _lib.check(_lib.load().lsattn_prefill_step_merge(C.byref(a), _stream()), "lsattn_prefill_step_merge")
 
 

@@ -272,3 +272,25 @@ def test_ragged_and_short_batches_run_one_wave_per_position(lsa, D, Hq, Hkv, len
     assert_o_close(got[0], o_ref, "O")
     assert_lse_close(got[1], lse_ref, "LSE")
     assert torch.equal(got[0], sure[0]) and torch.equal(got[1], sure[1])
+
+
+@pytest.mark.parametrize("Hq,Hkv,n,ctx", [(8, 1, 1100, 0), (4, 4, 2048, 0), (32, 8, 200, 1848), (12, 4, 77, 1300)])
+def test_lone_bf16_requests_folded_in_place_are_not_copied(lsa, monkeypatch, Hq, Hkv, n, ctx):
+    """The kernel of short prompts converts the V of one request of up to 2048 keys itself, through the native pass and through the checked one (which a
+    bound given as a tensor takes): the same bits, and no fp16 copy of V."""
+    from loongserve_amd import ops
+    print("case", Hq, Hkv, n, ctx, flush=True)
+    q, k, v = rand_t((n, Hq, 128), 41, torch.bfloat16), rand_t((n + ctx, Hkv, 128), 42, torch.bfloat16), rand_t((n + ctx, Hkv, 128), 43, torch.bfloat16)
+    qm, km = meta([n], [ctx]), meta([n + ctx])
+    o_ref, lse_ref = orc.attn_step(q, k, v, *qm, *km, 1)
+    qd, kd, vd = _dev(q, k, v)
+    monkeypatch.setattr(ops, "_v_as_f16", lambda *a: pytest.fail("V is copied"))
+    got = []
+    for bound in (n + ctx, torch.tensor(n + ctx)):
+        o, m, l = torch.full_like(qd, 7.0), torch.full((n, Hq), float("-inf"), device=DEV), torch.zeros((n, Hq), device=DEV)
+        lsa.context_attention_fwd(qd, kd, vd, o, *_dev(*qm), *_dev(*km), 1, n, m, l, total_q_len=n, max_kv_len=bound)
+        torch.cuda.synchronize()
+        assert_inplace_o_close(o.cpu(), o_ref.to(torch.bfloat16), o_ref, "o")
+        assert_lse_close(orc.state_lse(m.cpu(), l.cpu()).float(), lse_ref, "state LSE")
+        got.append(o)
+    assert torch.equal(*got)
