@@ -580,3 +580,28 @@ def test_equal_prompts_barely_past_two_workgroups_per_cu_keep_256_rows():
     step = lambda b, n, heads: _route(b, n, heads, total_q=b * n, total_kv=b * n, m=256)
     assert step(5, 832, (16, 1)) == ROWS_256 and step(5, 833, (16, 1)) == SMALL_32  # (26 and 27 tiles of 32 rows: 520 and 540 workgroups)
     assert step(11, 1024, (6, 6)) == SMALL_32                                     # (528)
+
+
+def test_argument_blocks_in_the_documents_match_the_header():
+    """Every ctypes mirror that a document at the top of the tree shows has the fields, in order and type, of the block this package passes, its example names a value for each
+    of them, and the interface version beside it is the header's."""
+    import glob
+    from loongserve_amd import _lib
+    found = 0
+    for path in glob.glob(os.path.join(ROOT, "*.md")):
+        text = open(path).read()
+        for version in re.findall(r"lsattn_version\(\) == LSATTN_VERSION`? \((\d+)\)", text):
+            assert int(version) == _lib.LSATTN_VERSION, path
+        for name, body in re.findall(r"^class (\w+)\(C\.Structure\):.*?\n((?:    .*\n)+)", text, flags=re.M):
+            space = {"C": C}
+            exec("class %s(C.Structure):\n%s" % (name, body), space)
+            assert space[name]._fields_ == getattr(_lib, name)._fields_, (path, name)
+            calls = re.findall(r"= %s\((.*?)\)[ ]*(?:#.*)?\n(?=rc)" % name, text, flags=re.S)
+            for call in calls:
+                depth, args = 0, 1
+                for ch in call:
+                    depth += (ch in "([") - (ch in ")]")
+                    args += ch == "," and depth == 0
+                assert args == len(space[name]._fields_), (path, name, args)
+                found += 1
+    assert found >= 1
