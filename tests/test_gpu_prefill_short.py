@@ -294,3 +294,53 @@ def test_lone_bf16_requests_folded_in_place_are_not_copied(lsa, monkeypatch, Hq,
         assert_lse_close(orc.state_lse(m.cpu(), l.cpu()).float(), lse_ref, "state LSE")
         got.append(o)
     assert torch.equal(*got)
+
+
+ROWS_256, ROWS_128, HALF = 4, 5, 6  # LSATTN_ROUTE_* of include/lsattn.h
+
+
+def _in_place_on(route, lsa, V, Hq, Hkv, lens, ctx=None, full=False):
+    """Prompts (behind contexts) folded in place, then the same keys once more as a step that every row sees whole (full) or as before: the route asked for as the call takes it,
+    with its state, and the results against the oracle.  V: "f16" or "bf16"."""
+    from loongserve_amd import _lib, ops
+    dtype = torch.float16 if V == "f16" else torch.bfloat16
+    ctx = ctx or [0] * len(lens)
+    klens = [n + c for n, c in zip(lens, ctx)]
+    T, TK = sum(lens), sum(klens)
+    q, k, v = rand_t((T, Hq, 128), 31, dtype), rand_t((TK, Hkv, 128), 32, dtype), rand_t((TK, Hkv, 128), 33, dtype)
+    steps = [(meta(lens, ctx), meta(klens)), (meta(lens, [2 * n for n in klens] if full else ctx), meta(klens))]
+    qd, kd, vd = _dev(q, k, v)
+    o, m, l = torch.full((T, Hq, 128), 7.0, dtype=dtype, device=DEV), torch.full((T, Hq), float("-inf"), device=DEV), torch.zeros((T, Hq), device=DEV)
+    o_st, m_st, l_st = torch.zeros((T, Hq, 128), dtype=dtype), torch.full((T, Hq), float("-inf")), torch.zeros(T, Hq)
+    parts = []
+    for qm, km in steps:
+        a = ops._prefill_args(qd, kd, vd, o, *_dev(*qm), *_dev(*km), 1, max(lens), None, total_q_len=T, state=(m, l))
+        assert _lib.load().lsattn_prefill_route(C.byref(a)) == route
+        lsa.context_attention_fwd(qd, kd, vd, o, *_dev(*qm), *_dev(*km), 1, max(lens), m, l, total_q_len=T)
+        orc.context_attention_fwd(q, k, v, o_st, *qm, *km, 1, max(lens), m_st, l_st)
+        parts.append(orc.attn_step(q, k, v, *qm, *km, 1))
+    torch.cuda.synchronize()
+    lse = torch.logaddexp(parts[0][1], parts[1][1])
+    ref = sum(p[0] * (p[1] - lse).exp()[..., None] for p in parts)
+    assert_inplace_o_close(o.cpu(), o_st, ref, "o")
+    assert_lse_close(orc.state_lse(m.cpu(), l.cpu()).float(), lse, "state LSE")
+
+
+@pytest.mark.parametrize("V,Hq,Hkv,lens,ctx,route", [
+    ("f16", 8, 1, [1472], None, SMALL_16), ("f16", 24, 24, [1472], None, SMALL_16), ("f16", 8, 1, [2048], None, SMALL_16), ("bf16", 8, 1, [2048], None, SMALL_16),
+    ("bf16", 4, 4, [1025], None, SMALL_16), ("f16", 32, 8, [200], [1848], SMALL_16), ("bf16", 12, 4, [77], [1300], SMALL_16), ("f16", 4, 1, [2304], None, SMALL_16),
+    ("f16", 8, 8, [801] * 10, None, SMALL_32), ("f16", 8, 1, [1280] * 9, None, SMALL_32), ("f16", 18, 6, [1024] * 4, None, SMALL_32)])
+def test_short_prompts_kernel_folds_in_place(lsa, V, Hq, Hkv, lens, ctx, route):
+    print("case", V, Hq, Hkv, lens[:2], ctx, flush=True)
+    _in_place_on(route, lsa, V, Hq, Hkv, lens, ctx)
+
+
+@pytest.mark.parametrize("V", ["f16", "bf16"])
+@pytest.mark.parametrize("full", [False, True])
+@pytest.mark.parametrize("Hq,Hkv,lens,route", [
+    (32, 8, [2500], HALF), (44, 44, [1100], HALF), (8, 1, [8300], ROWS_128), (64, 8, [800], ROWS_256),             # lone prompts past whole rounds
+    (40, 8, [1600, 700, 1000, 95], HALF), (32, 8, [1400, 900, 33, 64, 1, 700, 800, 350, 555, 600], HALF), (8, 8, [900, 40, 300, 1] * 5, HALF),  # ragged: four, ten and twenty
+    (16, 16, [1704, 200, 200, 200, 95], ROWS_128), (32, 8, [975, 112, 113], ROWS_256)])
+def test_128_wide_kernels_shapes_fold_in_place(lsa, V, full, Hq, Hkv, lens, route):
+    print("case", V, full, Hq, Hkv, lens[:4], flush=True)
+    _in_place_on(route, lsa, V, Hq, Hkv, lens, full=full)
