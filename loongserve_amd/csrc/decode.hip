@@ -1689,9 +1689,10 @@ template <typename T> static int launch_stage1_mfma(const lsattn_decode_stage1_a
     const bool nearly_two = full > (group < 4 ? 6 : 7) * kCUs && full <= 8 * kCUs, nearly_four = group < 4 && full > 13 * kCUs && full <= 16 * kCUs;
     const bool one = a->batch < 2 && (p.tasks < 4 || full <= 4 * kCUs || nearly_two || nearly_four);
     if (!forced && (!large || few || one)) return LSATTN_OK;
-    // bf16 launches that the lane kernel would take (in blocks as coarse as the split asked for they may be few waves): it multiplies V by fp32 weights, this
-    // kernel by two bf16 parts of them (error against 64 bits 4e-7 | 4.8e-6: two of 131870 tokens, 2/1 heads; one of 65936, 10/5).  So only the large ones.
-    const bool lane = std::is_same<T, BF16>::value && !use && !split_waves;
+    // Launches that the lane kernel would take (in blocks as coarse as the split asked for they may be few waves): it multiplies V by fp32 weights where V is bf16, this kernel by two bf16
+    // parts of them (error against 64 bits 4e-7 | 4.8e-6: two of 131870 tokens, 2/1 heads; one of 65936, 10/5), and f16 weights round a little worse here (eight launches, in the mean
+    // 1.92e-4 | 2.01e-4).  So only the large ones.
+    const bool lane = !use && !split_waves;
     if (!forced && lane && (a->batch < 2 || (a->batch < kSharesMinBatch && waves256 < 8 * kCUs) || (group >= 4 && p.tasks < 4 && waves256 <= 12 * kCUs))) return LSATTN_OK;
     // Short contexts, whose rows hold too few shares (a longest request of up to 256 tokens one share, whatever the batch),
     // and grids of one round of workgroups, see kSharesOneRoundBatch.

@@ -1282,3 +1282,21 @@ def test_stage2_with_more_rows_of_peers_than_there_are(lsa, lead):
         torch.cuda.synchronize()
         assert_o_close(o.cpu(), want.cpu(), "o")
         assert_lse_close(l.cpu(), want_lse.cpu(), "lse", rel=1e-5)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Hq,Hkv,lens,BS", [(3, 1, [131870, 300], 256), (10, 5, [65936], 256), (16, 4, [60000, 7], 1056)])
+def test_long_contexts_of_few_coarse_blocks_run_the_lane_kernel(lsa, tuning, dtype, Hq, Hkv, lens, BS):
+    """Whose weights are rounded least: the bits are those of the forced choice."""
+    print("case", dtype, Hq, Hkv, lens, BS, flush=True)
+    B = len(lens)
+    q, kv, table, b_req, b_len = decode_case(80, B, Hq, Hkv, 128, lens, sum(lens) + 100, dtype)
+    qd, kvd, td, rd, ld = q.to(DEV), kv.to(DEV), table.to(DEV), b_req.to(DEV), b_len.to(DEV)
+    got = []
+    for how in (None, "lane"):
+        tuning(decode_stage1=how)
+        mo = torch.empty(max(lens) // BS + 1, B, Hq, 128, device=DEV)
+        ml = torch.empty(mo.shape[:3], device=DEV)
+        got.append(lsa.longserve_token_decode_attention_flash_decoding(qd, td, rd, ld, mo, ml, B, max(lens), Hq, 128, kvd[:, :Hkv], kvd[:, Hkv:], BS))
+    torch.cuda.synchronize()
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
