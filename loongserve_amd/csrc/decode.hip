@@ -1106,8 +1106,9 @@ constexpr int64_t kListedFromWorkgroupsCoarse = 8192;
 constexpr int64_t kListedCoarseTokens = 1024;
 // Equal shares from eight requests on wherever the plain shape would run, and for fewer from 2048 waves of 256 tokens on, two workgroups per CU.  Of less than two,
 // where the CUs that hold two set the grid's time, those that gain whatever the lengths are (of the time of the grids, 3400 launches on four and more KV heads):
-//   two to seven requests, 1345 to 1536 waves: of one length 0.87 to 1.01, of others 0.58 to 0.97 (us, 32/8: 5 x 8860 40.0 | 38.1, 4 of at most 11264 31.4 | 24.5).  Below that one length gains more (0.81 to 0.95) but ragged ones
-//     of which few enough workgroups find tokens take up to 1.13 (6 of at most 6044 16/8 22.3 | 24.3), above it one length takes up to 1.09 (4 x 13569 8/8 42.5 | 44.8)
+//   four to seven requests, 1345 to 1536 waves: of one length 0.87 to 1.01, of others 0.58 to 0.97 (us, 32/8: 5 x 8860 40.0 | 38.1, 4 of at most 11264 31.4 | 24.5).  Below that one length gains more (0.81 to 0.95)
+//     but ragged ones of which few enough workgroups find tokens take up to 1.13 (6 of at most 6044 16/8 22.3 | 24.3), as two or three do there (3 of at most 15516 24/8 22.6 | 24.9); above it one length takes up to
+//     1.09 (4 x 13569 8/8 42.5 | 44.8)
 //   one request from 1025 waves on 0.74 to 0.99 (35000 tokens 32/8 36 | 30, 66000 64/8 67 | 52), except where the grid has nearly two workgroups per CU, to 1.12 (groups below four
 //     from one and a half on), and there also nearly four, to 1.04
 // Fewer than four KV heads, where a grid of the shape whose waves split a block stands against it, from more than 3072 waves on, and past whole rounds of that grid: one or two KV heads
@@ -1683,7 +1684,7 @@ template <typename T> static int launch_stage1_mfma(const lsattn_decode_stage1_a
     const bool past_rounds = group >= 4 && p.tasks < 3 && a->batch >= 8 && ((waves256 > 8 * kCUs && waves256 <= 9 * kCUs) ||
                                                           (p.tasks == 1 && a->batch >= 24 && a->batch <= 100 && waves256 > 4 * kCUs && waves256 <= 5 * kCUs));
     const bool large = past_rounds || waves256 >= (group < 4 ? 768 : p.tasks < 4 ? 12 * kCUs + 1 : kSplitMaxWaves + 1);
-    const bool few = a->batch > 1 && a->batch < kSharesMinBatch && waves256 < 8 * kCUs && (4 * waves256 <= 21 * kCUs || waves256 > 6 * kCUs);
+    const bool few = a->batch > 1 && a->batch < kSharesMinBatch && waves256 < 8 * kCUs && (a->batch < 4 || 4 * waves256 <= 21 * kCUs || waves256 > 6 * kCUs);
     // (one request by the blocks it fills: a last block of a few tokens makes no round of its own, 1 x 32769 tokens 32/8 29.4 | 30.6)
     const int64_t full = a->max_len_in_batch / 256 * p.tasks;
     const bool nearly_two = full > (group < 4 ? 6 : 7) * kCUs && full <= 8 * kCUs, nearly_four = group < 4 && full > 13 * kCUs && full <= 16 * kCUs;

@@ -1108,7 +1108,7 @@ def test_stage1_just_past_a_workgroup_per_cu_runs_the_plain_shape(lsa, tuning, d
 
 
 @pytest.mark.parametrize("Hq,Hkv,lens,shares", [
-    (16, 16, [10240] * 3, False), (32, 8, [8961, 300, 7000, 6453], False), (32, 8, [10752] * 4, False), (32, 8, [10753, 9000, 40, 10000], True), (32, 8, [12288] * 4, True), (32, 8, [12289] * 4, False),
+    (16, 16, [10240] * 3, False), (32, 8, [8961, 300, 7000, 6453], False), (32, 8, [10752] * 4, False), (32, 8, [10753, 9000, 40, 10000], True), (32, 8, [12288] * 4, True), (32, 8, [12289] * 4, False), (32, 8, [15000, 300, 4000], False),
     (32, 8, [32768], False), (32, 8, [33023], False), (32, 8, [33024], True), (32, 8, [57344], True), (32, 8, [57600], False), (32, 8, [65537], False), (32, 8, [65792], True),
     (16, 16, [24576], True), (16, 16, [24832], False), (16, 16, [33024], True), (16, 16, [53248], True), (16, 16, [53504], False), (16, 16, [65792], True)])
 def test_few_requests_in_equal_shares_where_these_are_no_slower(lsa, Hq, Hkv, lens, shares):
