@@ -1358,12 +1358,12 @@ static Shape choose_shape(const lsattn_prefill_args* a, bool dv, const Tuning& t
   // heads side by side, prompts 0.86 to 0.91 of the 256-row shape but full steps 1.03 to 1.06, 800 rows 64/8 37.4 | 38.9: not taken).
   if (as_long && ph == 0 && a->max_q_len <= 1408 && 2 * wgs128 > 3 * kCUs && 4 * wgs128 < 7 * kCUs) half = true;
   // Ragged requests folded in place whose keys are no more than their rows (prompts, or a ring's steps), up to 2048 rows: the 256-row shape ends with the
-  // longest requests' workgroups alone on their CUs.  From nine halves of a workgroup per CU on, of eight requests and more from three on, of sixteen and more from
-  // one on 2000 launches took 0.56 to 1.10 of its time, 0.89 in the mean, eleven more than 1.02.  Fewer workgroups of fewer requests took full steps to 1.10 (2, one of 1523, 32/32 53.9 | 58.3)
+  // longest requests' workgroups alone on their CUs.  Of four requests and more from nine halves of a workgroup per CU on, of eight from three on, of sixteen from
+  // one on 3500 launches took 0.55 to 1.10 of its time, 0.89 in the mean, fifteen more than 1.02.  Fewer workgroups of fewer requests took full steps to 1.10 (2, one of 1523, 32/32 53.9 | 58.3)
   // and prompts to 1.06, and where the split shape would run prompts to 1.25 (4 of at most 1973 14/2 38.4 | 47.5): not taken, nor equal lengths (0.84 to 1.07) or longer ragged ones (0.89 to 1.23).
   //   (us: 20 of at most 807 tokens 8/1 42.9 | 27.7, 10 of at most 1724 12/12 68.3 | 55.2, 4 of at most 1611 40/8 79.3 | 66.0)
   const int64_t enough = a->batch >= 16 ? 2 * kCUs : a->batch >= 8 ? 6 * kCUs : 9 * kCUs;  // of half workgroups
-  if (!split && a->batch > 1 && a->m && a->total_q_rows > 0 && a->total_kv_rows > 0 && a->total_kv_rows <= a->total_q_rows && a->max_q_len <= 2048 &&
+  if (!split && a->batch > 3 && a->m && a->total_q_rows > 0 && a->total_kv_rows > 0 && a->total_kv_rows <= a->total_q_rows && a->max_q_len <= 2048 &&
       a->total_q_rows * 10 <= (int64_t)a->batch * a->max_q_len * 9 && !a->o_b_start_loc && a->kv_cuts <= 1 && 2 * wgs128 >= enough)
     half = true;
   if (tn.prefill_rows == LSATTN_PREFILL_ROWS_128) split = true, half = false;

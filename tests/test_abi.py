@@ -573,6 +573,7 @@ def test_ragged_batches_of_few_workgroups_keep_their_shape():
     assert step(8, 1500, 2784, (32, 8)) == ROWS_256 and step(8, 1500, 2785, (32, 8)) == HALF  # (95 and 96)
     assert step(15, 1200, 2700, (32, 8)) == HALF and step(16, 900, 4000, (8, 1)) == step(20, 840, 5000, (8, 1)) == HALF  # (1.1 and 1.4)
     assert step(15, 1200, 2400, (32, 8)) == ROWS_256                                        # (2.8)
+    assert step(3, 1959, 3000, (64, 8)) == step(2, 1959, 2565, (64, 8)) == ROWS_256         # (two and three requests: full steps 139 -> 147 us)
 
 
 def test_equal_prompts_barely_past_two_workgroups_per_cu_keep_256_rows():
