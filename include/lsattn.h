@@ -122,7 +122,7 @@ typedef struct lsattn_prefill_args {
   int32_t max_kv_len;
 } lsattn_prefill_args;
 
-/* Which kernel the step these arguments describe runs (by the numbers in the block and the tuning block; nothing is launched and
+/* Which kernel the step these arguments describe runs (by the numbers in the block, whether m is set, and the tuning block; nothing is launched and
  * no pointer followed).  Meant for tests and for reading profiles: the routes and where they change are the library's own. */
 enum {
   LSATTN_ROUTE_INVALID = 0,      /* no such step */
@@ -142,7 +142,8 @@ int lsattn_prefill_cut_count(int32_t batch, int32_t num_q_heads, int32_t num_kv_
 
 /* 1 if the step these arguments describe (v_is_f16 = 0) converts a bfloat16 V on its way into LDS at no cost, as the kernels
  * for head sizes below 128 and for batches of short prompts do; 0 if the caller should make an fp16 copy of V first
- * (lsattn_bf16_to_f16_rows).  Looks at the numbers in the block only, not through its pointers. */
+ * (lsattn_bf16_to_f16_rows).  Looks at the numbers in the block, and at whether m is set (ask with the block as the step will take it),
+ * not through its pointers. */
 int lsattn_prefill_converts_v(const lsattn_prefill_args* a);
 
 /* Partial of one step from the empty state: o = normalised fp32 output, lse = natural-log
