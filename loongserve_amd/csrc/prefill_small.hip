@@ -836,7 +836,7 @@ int prefill_short_blocks(const lsattn_prefill_args* a) {
   const int64_t one = workgroups(a, pack, 1), two = workgroups(a, pack, 2);
   const bool f16 = a->dtype == LSATTN_F16, rag = ragged(a);
   // (m: of the three steps only the in-place one has it)
-  if (a->batch == 1 && a->m && one <= kCUs && longest >= kPartsMinKeys && longest <= (f16 ? kPartsMaxKeys : kPartsMaxKeysBf16)) return 1;
+  if (a->batch == 1 && a->m && longest <= (f16 ? kPartsMaxKeys : kPartsMaxKeysBf16) && two_waves_share(a)) return 1;
   if (longest > kShortMaxKeys || a->max_q_len > kShortMaxKeys)
     return f16 && a->m && a->batch == 1 && a->max_q_len == longest && longest <= kLoneMaxKeys && pack == 0 && one > 2 * kCUs && one <= 3 * kCUs;
   if (a->max_q_len <= 768) return longest > 1024 ? 0 : 2 * one <= (pack ? rag ? 5 : 6 : rag ? 12 : 8) * kCUs ? 1 : 2;

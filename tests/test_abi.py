@@ -606,3 +606,10 @@ def test_argument_blocks_in_the_documents_match_the_header():
                 assert args == len(space[name]._fields_), (path, name, args)
                 found += 1
     assert found >= 1
+
+
+def test_lone_requests_of_few_rows_under_a_loose_bound_keep_their_shape():
+    """One request goes to the short prompts' kernel past 1280 keys for the two waves that share its tiles, which are counted by the bound on its rows."""
+    step = lambda n, total, kv: _route(1, n, (32, 8), total_q=total, total_kv=kv, m=256)
+    assert step(200, 200, 2000) == step(512, 200, 2000) == SMALL_16 and step(1400, 200, 2000) == ROWS_128  # (at most 13, 32 and 88 workgroups per head)
+    assert step(200, 200, 511) == SMALL_16
